@@ -13,6 +13,7 @@
 //   norm_sigmoid_gate    rms(o) * w * sigmoid(g)
 //   lightning_attn       S <- decay S + k v^T, o = S^T q: one workgroup per (sequence, head), the state in
 //                        registers (a column per lane quad), prompt portions and decode rows alike
+#include "chunk_rec.h"
 #include "common.h"
 #include "lin_launchers.h"
 
@@ -467,6 +468,14 @@ hipError_t launch_lightning_attn(const LightningArgs& a, RaggedRows r, hipStream
   if (a.heads < 1 || a.dim < 1 || a.dim > 128 || a.vdim < 1 || a.vdim > 256 || r.positions == nullptr ||
       r.state_slots == nullptr)
     return hipErrorInvalidValue;
+  if (!a.f32) {
+    ChunkLinearArgs c;
+    c.out = a.out, c.nq = nullptr, c.x = static_cast<const uint16_t*>(a.x), c.xstride = a.xstride;
+    c.qoff = a.qoff, c.koff = a.koff, c.voff = a.voff, c.silu = true, c.ab = nullptr, c.abw = 0, c.decay = a.decay;
+    c.state = a.state, c.n_state = nullptr;
+    c.heads = a.heads, c.groups = a.heads, c.dim = a.dim, c.vdim = a.vdim, c.qscale = 1.0f;
+    if (chunk_linear_takes(c, r.total_rows, r.num_seqs)) return launch_chunk_linear(c, r, s);
+  }
   if (a.dim <= 16) return launch_lightning_dp<4>(a, r, s);
   if (a.dim <= 32) return launch_lightning_dp<8>(a, r, s);
   if (a.dim <= 64) return launch_lightning_dp<16>(a, r, s);

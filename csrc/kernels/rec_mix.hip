@@ -16,6 +16,7 @@
 //   head_norm_gate            (o / (max(|n . q|, floor) + 1e-6), optional,) per-head RMS norm, weight, sigmoid or SiLU gate
 //   skip_gate_group_norm      (o + D x) * silu(z), RMS norm in equal parts of the row, weight
 //   pair_post_norm_residual   resid += mult * rms((rms(y1) w1 + rms(y2) w2) / 2) * (1 + w)
+#include "chunk_rec.h"
 #include "common.h"
 #include "lane_reduce.h"
 #include "rec_launchers.h"
@@ -899,6 +900,14 @@ hipError_t launch_gated_linear_attn(const GatedLinearArgs& a, RaggedRows r, hipS
       (a.z == nullptr && (a.ab == nullptr || a.abw < 2)) || (a.n_state != nullptr) != (a.nq != nullptr) ||
       (a.z != nullptr && (a.z_bias == nullptr || a.n_state != nullptr)))
     return hipErrorInvalidValue;
+  if (!a.f32 && a.z == nullptr) {
+    ChunkLinearArgs c;
+    c.out = a.out, c.nq = a.nq, c.x = static_cast<const uint16_t*>(a.x), c.xstride = a.xstride;
+    c.qoff = a.qoff, c.koff = a.koff, c.voff = a.voff, c.silu = false, c.ab = a.ab, c.abw = a.abw, c.decay = nullptr;
+    c.state = a.state, c.n_state = a.n_state;
+    c.heads = a.heads, c.groups = a.groups, c.dim = a.dim, c.vdim = a.vdim, c.qscale = a.qscale;
+    if (chunk_linear_takes(c, r.total_rows, r.num_seqs)) return launch_chunk_linear(c, r, s);
+  }
   if (a.dim <= 16) return launch_gla_dp<4, 1>(a, r, s);
   if (a.dim <= 32) return launch_gla_dp<8, 1>(a, r, s);
   if (a.dim <= 64) return launch_gla_dp<16, 1>(a, r, s);
