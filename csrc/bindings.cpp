@@ -7,6 +7,7 @@
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
 
+#include "bind_moe_gemm.h"
 #include "kernels/launchers.h"
 
 using torch::Tensor;
@@ -1036,6 +1037,10 @@ PYBIND11_MODULE(_C, m) {
   m.def("gather_blocks_rows", &gather_blocks_rows);
   m.def("topk_softmax", &topk_softmax);
   m.def("moe_align", &moe_align);
+  m.def("moe_gemm", [](Tensor out, Tensor x, Tensor w, Tensor offsets, std::optional<Tensor> sorted, int64_t topk,
+                       std::optional<Tensor> scale, int64_t act, double limit, double alpha) {
+    return moe_gemm_op(out, x, w, offsets, sorted, topk, scale, act, limit, alpha, cur_stream());
+  });
   m.def("moe_gather", &moe_gather);
   m.def("moe_combine", &moe_combine);
   m.def("gemm_decode", &gemm_decode);

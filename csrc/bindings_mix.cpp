@@ -5,6 +5,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 
+#include "bind_moe_gemm.h"
 #include "kernels/launchers.h"
 #include "kernels/mix_launchers.h"
 
@@ -532,6 +533,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("relu2_act", &relu2_act);
   m.def("route_grouped_topk", &route_grouped_topk);
   m.def("topk_grouped", &topk_grouped);
+  m.def("moe_gemm", [](Tensor out, Tensor x, Tensor w, Tensor offsets, OptTensor sorted, int64_t topk, OptTensor scale,
+                       int64_t act, double limit, double alpha) {
+    return moe_gemm_op(out, x, w, offsets, sorted, topk, scale, act, limit, alpha, cur_stream());
+  });
   m.def("rms_norm_ext", &rms_norm_ext);
   m.def("post_norm_residual", &post_norm_residual);
   m.def("gated_act", &gated_act);

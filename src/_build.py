@@ -26,7 +26,7 @@ EXT_SUFFIX = sysconfig.get_config_var("EXT_SUFFIX") or ".so"
 ARCH = os.environ.get("DIE_OFFLOAD_ARCH", "gfx950")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
-KERNELS = ["norm_act", "rope_cache", "attention", "sampling", "moe", "gemm_decode", "decode_step", "allreduce"]
+KERNELS = ["norm_act", "rope_cache", "attention", "sampling", "moe", "moe_gemm", "gemm_decode", "decode_step", "allreduce"]
 CONTRACT_ON = {"attention", "gemm_decode"}
 # hipcc only: keeps -O3 from forming packed fp32 instructions out of ordinary float code
 NO_PACKED_FP32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
@@ -97,7 +97,7 @@ def build_kernels(force: bool = False, jobs: int = 8, verbose: bool = False) -> 
     return out
 
 
-MIX_KERNELS = ["mix_ops", "latent_attn", "moe", "seq_mix", "sink_attn", "lin_mix", "rec_mix", "chunk_rec", "conv_mix"]
+MIX_KERNELS = ["mix_ops", "latent_attn", "moe", "moe_gemm", "seq_mix", "sink_attn", "lin_mix", "rec_mix", "chunk_rec", "conv_mix"]
 MIX_BINDINGS = ["bindings_mix", "bindings_seq", "bindings_lin", "bindings_rec", "bindings_conv"]
 
 

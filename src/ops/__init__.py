@@ -865,6 +865,11 @@ def moe_apply(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: torch.Ten
         out = torch.empty_like(x)
         kern.moe_combine(out, ys, pos, w)
         return out
+    if t > MOE_DECODE_MAX_T and grouped_experts(kern, x, w13, w2, offsets, sorted_idx, k, ys, MOE_SILU):
+        # prompt-sized steps: every expert's rows in two launches, offsets read on the device, rows gathered on the way
+        out = torch.empty_like(x)
+        kern.moe_combine(out, ys, pos, w)
+        return out if residual is None else residual_add_sumsq(residual, out, ssp)
     seg_tiles = _moe_decode_tiles(hdim, inter, MOE_DECODE_MAX_T)
     capturing = torch.cuda.is_current_stream_capturing()
     if (t >= MOE_LIBRARY_MIN_TOKENS or seg_tiles is None) and not capturing:
@@ -936,6 +941,6 @@ def _moe_down_wr(hdim: int, inter: int) -> int:
 
 
 # dtype-generic ops (bf16 / fp32 storage) of the src/_Cmix extension
-from .mix import (ACT_CLAMPED, ACT_SILU, gated_act, latent_attn, latent_kv_write, latent_qkv_prep,  # noqa: E402,F401
+from .mix import (ACT_CLAMPED, ACT_SILU, MOE_SILU, gated_act, grouped_experts, latent_attn, latent_kv_write, latent_qkv_prep,  # noqa: E402,F401
                   mix_available,
                   moe_input_scaled, post_norm_residual, rms_norm_ext, rope_inv_freq, route_sigmoid_topk)

@@ -196,6 +196,24 @@ def linear_f32(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.mm(x, w.t(), out_dtype=torch.float32)
 
 
+MOE_NONE, MOE_SILU, MOE_CLAMPED, MOE_GELU, MOE_RELU2 = range(5)   # activations of the grouped expert product (moe_gemm.h)
+_MOE_ACT = {ACT_SILU: MOE_SILU, ACT_CLAMPED: MOE_CLAMPED, ACT_GELU_TANH: MOE_GELU, ACT_RELU2: MOE_RELU2}
+
+
+def grouped_experts(kern, x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, offsets: torch.Tensor, sorted_idx: torch.Tensor,
+                    k: int, ys: torch.Tensor, act: int, limit: float = 0.0, alpha: float = 0.0,
+                    scale: Optional[torch.Tensor] = None) -> bool:
+    """Both products of every expert over its rows, two launches: ys[j] = W2 act(s W13 x[sorted_idx[j] / k]) for the rows j of the
+    expert-sorted order, s = scale by (token, slot). The expert offsets stay on the device. False, with nothing done, where the
+    sizes do not tile (bf16, widths in multiples of 256)."""
+    if x.dtype != torch.bfloat16 or w2.shape[2] % 64 or ys.shape[1] % 256:
+        return False
+    a = torch.empty(ys.shape[0], w2.shape[2], dtype=x.dtype, device=x.device)
+    if not kern.moe_gemm(a, x, w13, offsets, sorted_idx, k, scale, act, limit, alpha):
+        return False
+    return kern.moe_gemm(ys, a, w2, offsets, None, 1, None, MOE_NONE, 0.0, 0.0)
+
+
 # (token, expert) rows up to which the experts' weights are gathered per row for two batched GEMMs (no host
 # read, hipGraph-capturable: decode steps); above it each expert runs one library GEMM pair over its rows
 MOE_BMM_MAX_ROWS = 64
@@ -222,7 +240,6 @@ def moe_input_scaled(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: to
     e = w13.shape[0]
     x = x.contiguous()
     w = w.contiguous()
-    xs = torch.empty(n, h, dtype=x.dtype, device=x.device)
 
     def finish(ys, pos):
         if post_norm is not None:
@@ -246,6 +263,7 @@ def moe_input_scaled(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: to
             sorted_idx = torch.empty(n, dtype=torch.int32, device=x.device)
             pos = torch.empty(n, dtype=torch.int32, device=x.device)
             kern.moe_align(offsets, sorted_idx, pos, ids.reshape(-1).contiguous(), e)
+            xs = torch.empty(n, h, dtype=x.dtype, device=x.device)
             kern.gather_scaled(xs, x, sorted_idx, w, k)
             a = torch.empty(n, w13.shape[1] // 2, dtype=x.dtype, device=x.device)
             ys = torch.empty(n, h, dtype=x.dtype, device=x.device)
@@ -253,18 +271,22 @@ def moe_input_scaled(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: to
             ck.gemm_decode_grouped(a, xs, w13, offsets, 1, wr1, kc1, none, 1, t, 1)
             ck.gemm_decode_grouped(ys, a, w2, offsets, 0, wr2, kc2, none, 1, t, 1)
             return finish(ys, pos)
+    offsets = torch.empty(e + 1, dtype=torch.int32, device=x.device)
+    sorted_idx = torch.empty(n, dtype=torch.int32, device=x.device)
+    pos = torch.empty(n, dtype=torch.int32, device=x.device)
+    if n > MOE_BMM_MAX_ROWS:
+        kern.moe_align(offsets, sorted_idx, pos, ids.reshape(-1).contiguous(), e)
+        ys = torch.empty(n, h, dtype=x.dtype, device=x.device)
+        if grouped_experts(kern, x, w13, w2, offsets, sorted_idx, k, ys, MOE_SILU, scale=w):
+            return finish(ys, pos)
+    xs = torch.empty(n, h, dtype=x.dtype, device=x.device)
     if n <= MOE_BMM_MAX_ROWS or torch.cuda.is_current_stream_capturing():
         kern.gather_scaled(xs, x, None, w, k)
         sel = ids.reshape(-1).long()
         g = torch.bmm(w13.index_select(0, sel), xs.unsqueeze(2)).squeeze(2)
         ys = torch.bmm(w2.index_select(0, sel), gated_act(g, ACT_SILU).unsqueeze(2)).squeeze(2).contiguous()
         return finish(ys, None)
-    offsets = torch.empty(e + 1, dtype=torch.int32, device=x.device)
-    sorted_idx = torch.empty(n, dtype=torch.int32, device=x.device)
-    pos = torch.empty(n, dtype=torch.int32, device=x.device)
-    kern.moe_align(offsets, sorted_idx, pos, ids.reshape(-1).contiguous(), e)
     kern.gather_scaled(xs, x, sorted_idx, w, k)
-    ys = torch.empty(n, h, dtype=x.dtype, device=x.device)
     off = offsets.tolist()  # one host read per layer: the per-expert groups become library GEMMs
     for ei in range(e):
         a0, a1 = off[ei], off[ei + 1]
@@ -398,6 +420,15 @@ def moe_output_weighted(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w:
             ck.gemm_decode_grouped(ys, _expert_act(g, kind, limit, alpha), w2, offsets, 0, wr2, kc2,
                                    ops._NO_ROWS(x.device), 1, t, 1)
             return finish(ys, pos)
+    offsets = torch.empty(buckets + 1, dtype=torch.int32, device=x.device)
+    sorted_idx = torch.empty(n, dtype=torch.int32, device=x.device)
+    pos = torch.empty(n, dtype=torch.int32, device=x.device)
+    if n > MOE_BMM_MAX_ROWS:
+        # prompt-sized steps: rows sorted by expert (identity entries sort last and run nothing), all experts in two launches
+        kern.moe_align(offsets, sorted_idx, pos, ids.reshape(-1).contiguous(), buckets)
+        ys = torch.empty(n, h, dtype=x.dtype, device=x.device)
+        if grouped_experts(kern, x, w13, w2, offsets, sorted_idx, k, ys, _MOE_ACT[kind], limit, alpha):
+            return finish(ys, pos)
     if n <= MOE_BMM_MAX_ROWS or torch.cuda.is_current_stream_capturing():
         # decode-sized steps: the routed experts' weights gathered per row for two batched products (no host read,
         # hipGraph-capturable); an identity entry runs expert E - 1 and its product is ignored by the sum
@@ -406,15 +437,9 @@ def moe_output_weighted(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w:
         g = torch.bmm(w13.index_select(0, sel), xr).squeeze(2)
         ys = torch.bmm(w2.index_select(0, sel), _expert_act(g, kind, limit, alpha).unsqueeze(2)).squeeze(2).contiguous()
         return finish(ys, None)
-    # prompt-sized steps: rows sorted by expert (identity entries sort last and run nothing), one library GEMM pair
-    # per real expert over its rows
-    offsets = torch.empty(buckets + 1, dtype=torch.int32, device=x.device)
-    sorted_idx = torch.empty(n, dtype=torch.int32, device=x.device)
-    pos = torch.empty(n, dtype=torch.int32, device=x.device)
-    kern.moe_align(offsets, sorted_idx, pos, ids.reshape(-1).contiguous(), buckets)
+    # fp32, or widths that the grouped product does not tile: one library GEMM pair per real expert over its rows
     xs = torch.empty(n, h, dtype=x.dtype, device=x.device)
     kern.gather_scaled(xs, x, sorted_idx, None, k)
-    ys = torch.empty(n, h, dtype=x.dtype, device=x.device)
     off = offsets.tolist()  # one host read per layer: the per-expert groups become library GEMMs
     for ei in range(e):
         a0, a1 = off[ei], off[ei + 1]

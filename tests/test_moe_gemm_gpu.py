@@ -1,0 +1,107 @@
+"""The grouped expert product of prompt-sized steps (moe_gemm.hip) against the same product in float64.
+
+Results are rounded to bf16 once (2^-9 of each value); the fp32 sums of up to 1024 products add about 1024^0.5 * 2^-24 of their
+terms' size, which matters only beside cancelled values: 2^-8 of the value plus 2^-8 of the row's root mean square covers both, and
+is far below what one wrong row, column or stage moves."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from src.ops import mix
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(counts, K, ncols, gated, topk, seed=0):
+    """Rows sorted by expert with the given rows per expert; row j reads token sorted[j] / topk."""
+    g = torch.Generator().manual_seed(seed)
+    n, E = sum(counts), len(counts)
+    x = torch.randn(n // topk, K, generator=g).to(torch.bfloat16)
+    w = (torch.randn(E, ncols * (2 if gated else 1), K, generator=g) * K ** -0.5).to(torch.bfloat16)
+    offsets = torch.tensor([0] + list(counts)).cumsum(0).int()
+    return x, w, offsets, torch.randperm(n, generator=g).int(), torch.rand(n, generator=g) + 0.5
+
+
+def _want(x, w, offsets, idx, topk, act, scale, limit, alpha):
+    rows = x.double()[idx.long() // topk] if idx is not None else x.double()
+    out = []
+    for e in range(w.shape[0]):
+        a, b = int(offsets[e]), int(offsets[e + 1])
+        z = rows[a:b] @ w[e].double().t()
+        if scale is not None:
+            z = z * scale.double()[idx[a:b].long()][:, None]
+        if act in (mix.MOE_SILU, mix.MOE_CLAMPED, mix.MOE_GELU):
+            g, u = z.chunk(2, 1)
+            if act == mix.MOE_SILU:
+                z = F.silu(g) * u
+            elif act == mix.MOE_GELU:
+                z = F.gelu(g, approximate="tanh") * u
+            else:
+                g = g.clamp(max=limit)
+                z = g * torch.sigmoid(alpha * g) * (u.clamp(-limit, limit) + 1)
+        elif act == mix.MOE_RELU2:
+            z = torch.relu(z) ** 2
+        out.append(z)
+    return torch.cat(out)
+
+
+# rows per expert: none, one, around a 32-row piece, around a tile of 128 and of 192 - 256 rows, uneven heights
+COUNTS = [(0, 1, 31, 32), (33, 0, 95, 64), (129, 127, 0, 256), (257, 255, 193, 63), (700, 0, 0, 4)]
+
+
+@pytest.mark.parametrize("counts", COUNTS)
+@pytest.mark.parametrize("K,ncols,act", [(64, 256, mix.MOE_NONE), (128, 128, mix.MOE_SILU), (192, 256, mix.MOE_CLAMPED),
+                                         (1024, 512, mix.MOE_RELU2), (64, 384, mix.MOE_GELU)])
+def test_products(cuda, counts, K, ncols, act):
+    topk = 2 if sum(counts) % 2 == 0 else 1
+    x, w, offsets, idx, scale = _case(counts, K, ncols, act in (mix.MOE_SILU, mix.MOE_CLAMPED, mix.MOE_GELU), topk)
+    kern = mix._kern()
+    for rows, sc in ((idx, None), (idx, scale), (None, None)):
+        xs = x if rows is not None else x.repeat_interleave(topk, 0)
+        out = torch.full((sum(counts), ncols), 7.0, dtype=torch.bfloat16, device=cuda)
+        dev = [None if t is None else t.to(cuda) for t in (xs, w, offsets, rows, sc)]
+        assert kern.moe_gemm(out, *dev[:4], topk if rows is not None else 1, dev[4], act, 1.5, 1.7)
+        want = _want(xs, w, offsets, rows, topk, act, sc, 1.5, 1.7)
+        tol = 2.0 ** -8 * (want.abs() + want.square().mean(1, keepdim=True).sqrt())
+        bad = ((out.cpu().double() - want).abs() > tol).nonzero()
+        assert not len(bad), (len(bad), bad[:4].tolist())
+
+
+def test_extra_groups_are_left_alone(cuda):
+    """Rows behind the last expert (identity entries, other ranks' experts) are not written."""
+    x, w, offsets, idx, _ = _case((40, 60), 128, 256, False, 1)
+    out = torch.full((100, 256), 3.0, dtype=torch.bfloat16, device=cuda)
+    assert mix._kern().moe_gemm(out, x.to(cuda), w[:1].contiguous().to(cuda), offsets.to(cuda), idx.to(cuda), 1, None, mix.MOE_NONE, 0.0, 0.0)
+    assert (out[40:] == 3.0).all() and not (out[:40] == 3.0).all()
+
+
+def test_sizes_that_do_not_tile_are_left_to_the_caller(cuda):
+    x, w, offsets, idx, _ = _case((40, 60), 96, 256, False, 1)
+    out = torch.empty(100, 256, dtype=torch.bfloat16, device=cuda)
+    assert not mix._kern().moe_gemm(out, x.to(cuda), w.to(cuda), offsets.to(cuda), idx.to(cuda), 1, None, mix.MOE_NONE, 0.0, 0.0)
+
+
+@pytest.mark.parametrize("t,h,f,e,k", [(300, 256, 512, 4, 2), (300, 256, 320, 4, 2), (700, 512, 256, 6, 3)])
+def test_mixtures_of_prompt_steps(cuda, t, h, f, e, k):
+    """The three mixtures end to end, widths that the grouped product tiles and that it leaves (f = 320: not 256-wide columns)."""
+    g = torch.Generator().manual_seed(t + f)
+    bf = torch.bfloat16
+    x = torch.randn(t, h, generator=g).to(bf)
+    w13, w1, w2 = ((torch.randn(*s, generator=g) * 0.05).to(bf) for s in ((e, 2 * f, h), (e, f, h), (e, h, f)))
+    ids = torch.rand(t, e + 1, generator=g).argsort(1)[:, :k].int()   # e: an identity entry
+    w = torch.rand(t, k, generator=g)
+    real = ids.clamp(max=e - 1)
+    from src import ops
+    from src.ops import reference as ref
+
+    for name, got, want in (
+            ("scaled", lambda d: mix.moe_input_scaled(*d(x, w13, w2, w, real)), ref.moe_input_scaled(x, w13, w2, w, real, None)),
+            ("weighted", lambda d: mix.moe_output_weighted(*d(x, w13, w2, w, ids), mix.ACT_CLAMPED, 7.0, 1.7, n_route=e + 1),
+             ref.moe_output_weighted(x, w13, w2, w, ids, mix.ACT_CLAMPED, 7.0, 1.7, None, None)),
+            ("relu2", lambda d: mix.moe_output_weighted(*d(x, w1, w2, w, real), mix.ACT_RELU2, 0.0, 0.0),
+             ref.moe_output_weighted(x, w1, w2, w, real, mix.ACT_RELU2, 0.0, 0.0, None, None)),
+            ("mixtral", lambda d: ops.moe_apply(*d(x, w13, w2, w, real), e), ref.moe_experts(x, w13, w2, w, real))):
+        y = got(lambda *ts: [v.to(cuda) for v in ts]).float().cpu()
+        err = (y - want.float()).norm() / want.float().norm()
+        assert err < 1e-2, (name, err)   # two roundings to bf16 on either side
