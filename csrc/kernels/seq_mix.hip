@@ -9,9 +9,10 @@
 //   delta_prep          short conv + SiLU of q/k/v, unit q/k, beta (and the per-head decay) of the gated delta rule
 //   conv_state_update   the convolution's trailing inputs -> state
 //   gated_delta         the recurrence itself, one workgroup per (sequence, head), the state in registers (four
-//                       columns per group of 4 - 16 lanes)
+//                       columns per group of 4 - 16 lanes); prompt portions: chunk_delta.hip
 //   qkv_prep            projection bias or short conv, q/k norm, rotate-half rotary (optionally of the values too),
 //                       value norm / value mixing, paged cache write
+#include "chunk_delta.h"
 #include "common.h"
 #include "lane_reduce.h"
 #include "seq_launchers.h"
@@ -1173,6 +1174,7 @@ hipError_t launch_gated_delta(const GatedDeltaArgs& a, RaggedRows r, hipStream_t
   if (r.num_seqs == 0 || r.total_rows == 0) return hipSuccess;
   if (!delta_ok(a.sh) || !rows_ok(r) || (a.z != nullptr && (a.z_bias == nullptr || a.A_log == nullptr)))
     return hipErrorInvalidValue;
+  if (chunk_delta_takes(a, r.total_rows, r.num_seqs)) return launch_chunk_delta(a, r, s);
   if (a.sh.dim <= 16) return launch_gd<4, 1>(a, r, s);
   if (a.sh.dim <= 32) return launch_gd<8, 1>(a, r, s);
   if (a.sh.dim <= 64) return launch_gd<16, 1>(a, r, s);

@@ -1,0 +1,73 @@
+"""The gated delta rule of prompt portions: the chunked matrix-core kernel against the plain token-by-token form.
+
+Both sides hold state and results in fp32 and add in different orders. Keys are unit vectors and write strengths lie in (0, 1), so a
+token's rounding errors are not amplified by later ones: over a few hundred tokens 1e-4 of the largest value is some 1600 roundings
+of 2^-24, and far below what one dropped or doubled token moves. Results are rounded to bf16 (2^-8 relative, at most, where the two
+sides round to different neighbours)."""
+
+import pytest
+import torch
+
+from src.ops import seq
+
+pytestmark = pytest.mark.gpu
+LENS = [133, 1, 164, 17, 115, 97, 16]   # 77 rows a sequence: from 64 (16 with wider values) on the chunks take them
+PAST = [0, 5, 7, 0, 2, 0, 3]
+
+
+def _inputs(H, G, D, V, channel, lens=LENS, past=PAST):
+    T, S = sum(lens), len(lens)
+    unit = lambda x: x / x.norm(dim=-1, keepdim=True)
+    q, k = unit(torch.randn(T, G, D)) * D ** -0.5, unit(torch.randn(T, G, D) + 0.5)   # keys that overlap
+    qkv = torch.cat([q.reshape(T, -1), k.reshape(T, -1), torch.randn(T, H * V)], 1)
+    beta, g = torch.rand(T, H), torch.rand(T, H)
+    g[torch.rand(T, H) < 0.1] = 0.0      # states that are dropped
+    slab = torch.randn(T, H * (V + D) + 24).to(torch.bfloat16)
+    z = slab[:, H * V + 8: H * (V + D) + 8] if channel else None
+    extra = dict(z=z, z_bias=torch.randn(H * D) - 1, A_log=torch.randn(H)) if channel else {}
+    rag = (torch.cat([torch.arange(n) + p for n, p in zip(lens, past)]), torch.tensor([0] + lens).cumsum(0).int(),
+           torch.randperm(S + 1)[:S].int())
+    return qkv, beta if channel else torch.cat([beta, g], 1), slab[:, : H * V], torch.rand(V) + 0.5, torch.randn(S + 1, H, D, V), extra, rag
+
+
+def _run(args, dims, dev, **kw):
+    qkv, bg, gate, norm, state, extra, rag = args
+    slab = gate._base if gate._base is not None else gate
+    slab = slab.to(dev)
+    to = lambda t: t.to(dev) if t._base is None else slab.as_strided(t.shape, t.stride(), t.storage_offset())
+    state = state.clone().to(dev)
+    out = seq.gated_delta(to(qkv), to(bg), to(gate), to(norm), 1e-6, state, *dims, seq.Ragged(*(to(t) for t in rag)),
+                          **{k: to(t) for k, t in extra.items()}, **kw)
+    return out.cpu().float(), state.cpu()
+
+
+@pytest.mark.parametrize("channel", [False, True])
+@pytest.mark.parametrize("heads,groups,dim,vdim,sigmoid", [
+    (4, 2, 128, 128, False), (3, 3, 64, 64, True), (2, 1, 64, 256, False), (2, 2, 128, 64, True), (2, 1, 128, 256, True),
+    (3, 1, 64, 128, False)])
+def test_prompt_portions(cuda, heads, groups, dim, vdim, sigmoid, channel):
+    torch.manual_seed(heads + dim + vdim)
+    args, dims = _inputs(heads, groups, dim, vdim, channel), (heads, groups, dim, vdim)
+    want, st = _run(args, dims, "cpu", gate_sigmoid=sigmoid, mult=0.7)
+    got, st2 = _run(args, dims, cuda, gate_sigmoid=sigmoid, mult=0.7)
+    assert (st2 - st).abs().max() <= 1e-4 * st.abs().max()
+    assert ((got - want).abs() <= 2 ** -7 * want.abs() + 1e-4 * want.abs().max()).all()
+
+
+@pytest.mark.parametrize("what", ["k", "v", "beta", "decay"])
+def test_later_tokens_do_not_reach_earlier_rows(cuda, what):
+    """An infinite key or value or a NaN gate changes its own row and the later ones of its sequence, no others."""
+    torch.manual_seed(1)
+    H, D, V, at = 2, 64, 128, 99
+    args = _inputs(H, H, D, V, False, [80, 80, 80], [0, 0, 3])
+    want, _ = _run(args, (H, H, D, V), cuda)
+    if what in "kv":
+        args[0][at, (H * D if what == "k" else 2 * H * D) + 3] = float("inf")
+    else:
+        args[1][at, 0 if what == "beta" else H] = float("nan")
+    got, _ = _run(args, (H, H, D, V), cuda)
+    keep = torch.ones(240, dtype=torch.bool)
+    keep[at:160] = False
+    assert torch.equal(got[keep], want[keep])
+    assert torch.equal(got[at:160, V:], want[at:160, V:])
+    assert not torch.isfinite(got[at, :V]).all()
