@@ -34,10 +34,6 @@ constexpr int CT = 16;        // tokens of a chunk
 constexpr int TP = CT + 4;    // pitch of the 16-wide arrays (floats): 16-byte reads of 16 rows fall on different banks
 
 __device__ __forceinline__ f32x4_t mm(float a, float b, f32x4_t c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ float xor16_sum(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
 __device__ __forceinline__ float dpp_ror8(float x) {   // of lane ^ 8
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false));
 }
