@@ -471,16 +471,31 @@ template <int NW> hipError_t launch_mfma_ndb(const LatentAttnArgs& a, hipStream_
   return hipErrorInvalidValue;
 }
 
-// Prompt-sized steps at the common rotary widths (rot_dim = 16 * NROT, NROT = 0: no rotary part): the same algorithm with every wave's
-// query fragments held in registers (loaded straight from global memory, the rotary part rotated on the way;
-// no query tile in LDS, so the per-tile LDS traffic is the key tile alone) and the key tile double-buffered
-// (one barrier per tile: the next tile's registers are stored into the other buffer after this tile's MFMAs).
+// Prompt-sized steps at the common rotary widths (rot_dim = 16 * NROT, NROT = 0: no rotary part): the same algorithm with every
+// wave's query fragments in registers (loaded straight from global memory, the rotary part rotated on the way). A wave owns 16
+// rows: sums and queries take 64 + 36 registers at rank 256, so that 3 waves share a SIMD and one's softmax runs beside the others'
+// products. Key tiles come by DMA into two buffers of a workgroup of 4 waves, one barrier per tile. A tile of 32 rows by KCH 16-byte
+// pieces lies in LDS as the DMA writes it, without gaps; the pieces of a row are exchanged (XOR) so that 16 consecutive rows' reads
+// of one piece fall on all banks.
+// Bound by LDS reads (34 KB per wave and tile at 128 bytes a cycle: 120 us of the 253 below). 16 sequences of 1024 rows, 16 heads,
+// rank 256 + 32: 32 rows per wave, one wave per SIMD, tiles through registers, looked up piece by piece behind divisions: 518 us;
+// the same with DMA and the next tile's scores under the softmax 370; this 253 (570 TFLOP/s).
+template <int NDB, int NROT> struct RqTile {
+  static constexpr int KCH = 4 * NDB + 2 * NROT, NPF = (MKT * KCH + 255) / 256, BYTES = NPF * 4096;
+  static constexpr int G = KCH % 16 == 0 ? 16 : KCH % 8 == 0 ? 8 : KCH % 4 == 0 ? 4 : 2;   // rows r and r + 16 / G share banks
+  static __device__ __forceinline__ int swz(int row) { return row / (16 / G) % G; }
+  static constexpr int OP = 64 * NDB + 16;   // pitch of a result row in LDS
+  static constexpr int TABLE = 1024;         // block-table entries in LDS
+  static constexpr int LDS = 2 * BYTES + 4 * TABLE > 64 * OP ? 2 * BYTES + 4 * TABLE : 64 * OP;
+};
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(1))) const void global_cvoid;
+
 template <int NDB, int NROT>
-__global__ void __launch_bounds__(256) latent_attn_mfma_rq_kernel(LatentAttnArgs a, int KP) {
-  constexpr int NT = 256, NKK = 2 * NDB + NROT, KCH = 4 * NDB + 2 * NROT, NCH = MKT * KCH;
-  constexpr int NPF = (NCH + NT - 1) / NT;
-  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-  bf16_t* ks0 = reinterpret_cast<bf16_t*>(smem_raw);          // 2 x [MKT][KP]
+__global__ void __launch_bounds__(256, 3) latent_attn_mfma_rq_kernel(LatentAttnArgs a, uint32_t bs_mul, int bs_shift) {
+  using Z = RqTile<NDB, NROT>;
+  constexpr int KCH = Z::KCH, NPF = Z::NPF, NLAT = NDB, NK = NDB + NROT / 2;   // 32-wide steps of a row: latent, in all
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];   // two tiles, block-table entries; at the end the results
   // Workgroups are dealt to the 8 XCDs round-robin by their linear id, and each XCD has its own L2: renumber so
   // that XCD k runs a contiguous eighth of the (sequence-major) tile list — the row tiles of one sequence share
   // that sequence's cache rows in ONE L2 instead of streaming every sequence through all eight
@@ -489,225 +504,225 @@ __global__ void __launch_bounds__(256) latent_attn_mfma_rq_kernel(LatentAttnArgs
     const unsigned total = gridDim.x * gridDim.y, lin = blockIdx.x + gridDim.x * blockIdx.y;
     if (total % 8 == 0) {
       const unsigned nl = (lin % 8) * (total / 8) + lin / 8;
-      bx = (int)(nl % gridDim.x);
+      bx = (int)(gridDim.x - 1 - nl % gridDim.x);   // the tiles with the most keys first
       by = (int)(nl / gridDim.x);
     }
   }
-  const int s = by, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tid = threadIdx.x;
+  const int s = by, lane = threadIdx.x & 63, tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int H = a.heads;
   constexpr int R = 32 * NDB, Dk = R + 16 * NROT;
   const int q0 = a.cu_q ? a.cu_q[s] : s;
   const int nq = a.cu_q ? a.cu_q[s + 1] - q0 : 1;
-  const int nrows = nq * H, row0 = bx * 128;
+  const int nrows = nq * H, row0 = bx * 64;
   if (row0 >= nrows) return;
   const int ctx = a.ctx_lens[s];
-  const int last_row = min(row0 + 128, nrows) - 1;
+  const int last_row = min(row0 + 64, nrows) - 1;
   const int p_first = (int)a.positions[q0 + row0 / H], p_last = (int)a.positions[q0 + last_row / H];
   const int jlo = a.window > 0 ? max(0, p_first - a.window + 1) : 0;
   const int jhi = min(p_last, ctx - 1);
-  const bf16_t* qlat = reinterpret_cast<const bf16_t*>(a.q_lat);
-  const bf16_t* qrot = reinterpret_cast<const bf16_t*>(a.q_rot);
   const bf16_t* cache = reinterpret_cast<const bf16_t*>(a.cache);
-  const int qcol = lane & 31, hh = lane >> 5;
-  const int myrow = row0 + wave * 32 + qcol;
-  const bool rok = myrow < nrows;
-  const bool wave_live = row0 + wave * 32 < nrows;
-  const int64_t tq = rok ? q0 + myrow / H : 0;
+  const int li = lane & 15, lg = lane >> 4;
+
+  // Block-table entries of the workgroup's keys in LDS (TABLE at a time), so that a tile's loads depend on LDS reads alone
+  const int* bt = a.block_tables + (int64_t)s * a.bt_stride;
+  int* btl = reinterpret_cast<int*>(smem_raw + 2 * Z::BYTES);
+  auto block_of = [&](int j) { return a.block_size == 1 ? j : (int)(__umulhi((uint32_t)j, bs_mul) >> bs_shift); };
+  const int b_hi = block_of(max(jhi, 0));
+  int b_lo = block_of(jlo);
+  auto stage_table = [&]() {
+    for (int u = tid; u < Z::TABLE && b_lo + u <= b_hi; u += 256) btl[u] = bt[b_lo + u];
+    __syncthreads();
+  };
+  stage_table();
+  // tile rows by DMA: piece u of this thread is 16 bytes of key krow[u] (beyond the tile: of key 31, into the slack)
+  int krow[NPF], pcol[NPF];
+#pragma unroll
+  for (int u = 0; u < NPF; ++u) {
+    const int idx = tid + 256 * u, row = min(idx / KCH, MKT - 1);
+    krow[u] = row;
+    pcol[u] = 8 * (idx < MKT * KCH ? (idx - row * KCH) ^ Z::swz(row) : 0);
+  }
+  auto fetch = [&](int j0, int buf) {   // (keys beyond the last repeat it)
+    if (block_of(min(j0 + MKT - 1, jhi)) >= b_lo + Z::TABLE) {
+      __syncthreads();
+      b_lo = block_of(j0);
+      stage_table();
+    }
+#pragma unroll
+    for (int u = 0; u < NPF; ++u) {
+      const int j = min(j0 + krow[u], jhi), jb = block_of(j);
+      const bf16_t* src = cache + ((int64_t)btl[jb - b_lo] * a.block_size + (j - jb * a.block_size)) * Dk + pcol[u];
+      char* to = smem_raw + buf * Z::BYTES + (256 * u + 64 * wave) * 16;
+      __builtin_amdgcn_global_load_lds((global_cvoid*)src, (lds_void*)to, 16, 0, 0);
+    }
+  };
+  const int nt = jhi < jlo ? 0 : (jhi - jlo) / MKT + 1;
+  if (nt > 0) fetch(jlo, 0);
+
+  const int wrow = row0 + wave * 16, myrow = wrow + li;
+  const bool rok = myrow < nrows, wave_live = wrow < nrows, all_rows = wrow + 15 < nrows;
+  const int64_t tq = rok ? q0 + myrow / H : q0;
   const int hq = rok ? myrow % H : 0;
   const int64_t orow = (int64_t)hq * a.total_q + tq;
   const int prow = rok ? (int)a.positions[tq] : -1;
-  const int wrow_lo = row0 + wave * 32;
-  const bool all_rows = wrow_lo + 31 < nrows;
-  const int pw_min = wave_live ? (int)a.positions[q0 + wrow_lo / H] : 0;
-  const int pw_max = wave_live ? (int)a.positions[q0 + min(wrow_lo + 31, nrows - 1) / H] : 0;
-
-  // this lane's query fragments: qf[kk] = Q[row][16 kk + 8 hh .. + 8]
-  bf16x8_t qf[NKK];
+  const int pw_min = wave_live ? (int)a.positions[q0 + wrow / H] : 0;
+  const int pw_max = wave_live ? (int)a.positions[q0 + min(wrow + 15, nrows - 1) / H] : 0;
+  // this lane's query fragments: qf[k] = Q[row][32 k + 8 lg .. + 8]; an odd NROT leaves 16 columns, of which the lane has 4. (Rows
+  // beyond the last repeat the first; every load is unconditional, so that all are in flight together.)
+  bf16x8_t qf[NK > 0 ? NK : 1];
+  short4_t qt = {};
+  const bf16_t* qlat = reinterpret_cast<const bf16_t*>(a.q_lat) + orow * R;
 #pragma unroll
-  for (int kk = 0; kk < 2 * NDB; ++kk) {
-    uint4 v = make_uint4(0, 0, 0, 0);
-    if (rok) v = *reinterpret_cast<const uint4*>(qlat + orow * R + 16 * kk + 8 * hh);
-    qf[kk] = __builtin_bit_cast(bf16x8_t, v);
-  }
+  for (int k = 0; k < NLAT; ++k) qf[k] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(qlat + 32 * k + 8 * lg));
+  if constexpr (NROT > 0) {
+    constexpr int E = NROT % 2 == 0 ? 8 : 4, NS = (NROT + 1) / 2;
+    bf16_t qr[NS][E];
+    float fr[NS][E / 2];
+    const bf16_t* qp = reinterpret_cast<const bf16_t*>(a.q_rot) + tq * a.q_stride + (int64_t)hq * a.q_hstride + E * lg;
 #pragma unroll
-  for (int kr = 0; kr < NROT; ++kr) {
-    float f[8];
+    for (int k = 0; k < NS; ++k) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) f[e] = 0.f;
-    if (rok) {
-      const bf16_t* qp = qrot + tq * a.q_stride + (int64_t)hq * a.q_hstride + 16 * kr + 8 * hh;
+      for (int e = 0; e < E; ++e) qr[k][e] = qp[32 * k + e];
 #pragma unroll
-      for (int pr = 0; pr < 4; ++pr) {
-        const int i = (16 * kr + 8 * hh) / 2 + pr;
-        const float u = bf2f(qp[2 * pr]), w = bf2f(qp[2 * pr + 1]);
-        if (i < a.sh.rot_pairs) {
-          float sn, cs;
-          __sincosf((float)prow * a.sh.inv_freq[i], &sn, &cs);
-          f[2 * pr] = u * cs - w * sn;
-          f[2 * pr + 1] = w * cs + u * sn;
-        } else {
-          f[2 * pr] = u;
-          f[2 * pr + 1] = w;
-        }
-      }
+      for (int i = 0; i < E / 2; ++i)
+        fr[k][i] = a.sh.rot_pairs > 0 ? a.sh.inv_freq[min(16 * k + E / 2 * lg + i, a.sh.rot_pairs - 1)] : 0.f;
     }
-    qf[2 * NDB + kr] = __builtin_bit_cast(bf16x8_t, pack8(f));
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+      float f[8] = {};
+#pragma unroll
+      for (int i = 0; i < E / 2; ++i) {
+        const float u = bf2f(qr[k][2 * i]), w = bf2f(qr[k][2 * i + 1]);
+        float sn, cs;
+        __sincosf((float)prow * fr[k][i], &sn, &cs);
+        const bool turned = 16 * k + E / 2 * lg + i < a.sh.rot_pairs;
+        f[2 * i] = turned ? u * cs - w * sn : u;
+        f[2 * i + 1] = turned ? w * cs + u * sn : w;
+      }
+      const uint4 w = pack8(f);
+      if constexpr (E == 8)
+        qf[NLAT + k] = __builtin_bit_cast(bf16x8_t, w);
+      else
+        qt = __builtin_bit_cast(short4_t, make_uint2(w.x, w.y));
+    }
   }
 
   constexpr float LOG2E = 1.4426950408889634f;
   const float sl2 = a.scale * LOG2E;
   const bool has_sink = a.sink != nullptr && rok;
   float m = has_sink ? a.sink[hq] * LOG2E : -1e30f;
-  float l = has_sink ? 1.0f : 0.0f;
-  f32x16_t o[NDB];
+  float l = has_sink && lg == 0 ? 1.0f : 0.0f;   // (the sum of this lane's keys)
+  f32x4_t o[2 * NDB];
 #pragma unroll
-  for (int db = 0; db < NDB; ++db)
+  for (int db = 0; db < 2 * NDB; ++db) o[db] = f32x4_t{};
+  // K fragments: key li of 16, piece 4 k + lg; V fragments: keys 4 lg .. of either 16 (the order in which the weights lie in
+  // registers), columns 16 db ..
+  const int ksw = Z::swz(li), vrow = 4 * lg + (li >> 2), vsw = Z::swz(vrow);
+  const int kat = 16 * li * KCH, vat = 16 * vrow * KCH + 8 * (li & 1);
+  for (int i = 0; i < nt; ++i) {
+    const int j0 = jlo + i * MKT;
+    // tile i is in LDS for every wave, and every wave has left the other buffer
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(7 << 4);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (i + 1 < nt) fetch(j0 + MKT, (i + 1) & 1);
+    if (!wave_live) continue;
+    const char* ks = smem_raw + (i & 1) * Z::BYTES;
+    f32x4_t sc[2] = {};
 #pragma unroll
-    for (int r = 0; r < 16; ++r) o[db][r] = 0.f;
-
-  // the block-table entries of this workgroup's key range, staged in LDS: a key tile's loads then depend on an
-  // LDS read, not on a second global round trip
-  const int* bt = a.block_tables + (int64_t)s * a.bt_stride;
-  int* btl = reinterpret_cast<int*>(ks0 + 2 * MKT * KP);
-  const int b_lo = jlo / a.block_size, nbt = jhi / a.block_size - b_lo + 1;
-  const bool bt_lds = nbt <= BT_LDS_MAX;
-  if (bt_lds) {
-    for (int u = tid; u < nbt; u += NT) btl[u] = bt[b_lo + u];
-    __syncthreads();
-  }
-  uint4 pf[NPF];
-  auto fetch = [&](int j0) {
+    for (int k = 0; k < NK; ++k)
 #pragma unroll
-    for (int u = 0; u < NPF; ++u) {
-      const int idx = tid + u * NT;
-      const int k = idx / KCH, c = idx % KCH, j = j0 + k;
-      pf[u] = make_uint4(0, 0, 0, 0);
-      if (idx < NCH && j <= jhi) {
-        const int jb = j / a.block_size;
-        const int64_t blk = bt_lds ? btl[jb - b_lo] : bt[jb];
-        pf[u] = *reinterpret_cast<const uint4*>(cache + (blk * a.block_size + (j - jb * a.block_size)) * Dk + 8 * c);
+      for (int t = 0; t < 2; ++t) {
+        const uint4 w = *reinterpret_cast<const uint4*>(ks + kat + 256 * KCH * t + 16 * ((4 * k + lg) ^ ksw));
+        sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w), qf[k], sc[t], 0, 0, 0);
       }
-    }
-  };
-  auto stash = [&](bf16_t* ks) {
+    if constexpr (NROT % 2 != 0)
 #pragma unroll
-    for (int u = 0; u < NPF; ++u) {
-      const int idx = tid + u * NT;
-      if (idx < NCH) *reinterpret_cast<uint4*>(ks + (idx / KCH) * KP + 8 * (idx % KCH)) = pf[u];
-    }
-  };
-  fetch(jlo);
-  stash(ks0);
-  if (jlo + MKT <= jhi) fetch(jlo + MKT);
-  const int pitchB = KP * 2;
-  const int g16 = lane >> 4, i16 = lane & 15;
-  const int voff = (4 * hh + (i16 >> 2)) * pitchB + (16 * (g16 & 1) + 4 * (i16 & 3)) * 2;
-  int cur = 0;
-  for (int j0 = jlo; j0 <= jhi; j0 += MKT, cur ^= 1) {
-    __syncthreads();  // tile j0 is complete in buffer cur; every wave has left the other buffer
-    bf16_t* ks = ks0 + cur * (MKT * KP);
-    if (wave_live) {
-      f32x16_t sc;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) sc[r] = 0.f;
-      const bf16_t* ka = ks + qcol * KP + 8 * hh;
-#pragma unroll
-      for (int kk = 0; kk < NKK; ++kk) {
-        const bf16x8_t af = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(ka + 16 * kk));
-        sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, qf[kk], sc, 0, 0, 0);
+      for (int t = 0; t < 2; ++t) {
+        const uint2 w = *reinterpret_cast<const uint2*>(ks + kat + 256 * KCH * t + 16 * ((4 * NK + (lg >> 1)) ^ ksw) + 8 * (lg & 1));
+        sc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(short4_t, w), qt, sc[t], 0, 0, 0);
       }
-      float mx = -INFINITY;
-      // interior tiles (every key visible to every row of the wave) skip the per-score mask
-      if (all_rows && j0 + MKT - 1 <= min(pw_min, jhi) && (a.window <= 0 || pw_max - j0 < a.window)) {
+    // interior tiles (every key visible to every row of the wave) skip the per-score mask
+    float mx = -INFINITY;
+    const bool inner = all_rows && j0 + MKT - 1 <= min(pw_min, jhi) && (a.window <= 0 || pw_max - j0 < a.window);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          sc[r] *= sl2;
-          mx = fmaxf(mx, sc[r]);
-        }
-      } else {
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int j = j0 + (r & 3) + 8 * (r >> 2) + 4 * hh;
+      for (int e = 0; e < 4; ++e) sc[t][e] *= sl2;
+    if (!inner) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int j = j0 + 16 * t + 4 * lg + e;
           const bool valid = rok && j <= jhi && j <= prow && (a.window <= 0 || prow - j < a.window);
-          const float v = valid ? sc[r] * sl2 : -INFINITY;
-          sc[r] = v;
-          mx = fmaxf(mx, v);
+          sc[t][e] = valid ? sc[t][e] : -INFINITY;
         }
-      }
-      mx = xor32_max(mx);
-      const float mn = fmaxf(m, mx);
-      const float alpha = __builtin_amdgcn_exp2f(m - mn);
-      float sum = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float pe = __builtin_amdgcn_exp2f(sc[r] - mn);
-        sc[r] = pe;
-        sum += pe;
-      }
-      sum = xor32_sum(sum);
-      l = l * alpha + sum;
-      m = mn;
-      bf16x8_t pfr[2];
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        uint4 w;
-        w.x = pack2(sc[8 * s2 + 0], sc[8 * s2 + 1]);
-        w.y = pack2(sc[8 * s2 + 2], sc[8 * s2 + 3]);
-        w.z = pack2(sc[8 * s2 + 4], sc[8 * s2 + 5]);
-        w.w = pack2(sc[8 * s2 + 6], sc[8 * s2 + 7]);
-        pfr[s2] = __builtin_bit_cast(bf16x8_t, w);
-      }
-      const char* vbase = reinterpret_cast<const char*>(ks) + voff;
-      const bool rescale = __builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0;  // wave-uniform: most tiles keep the max
-#pragma unroll
-      for (int db = 0; db < NDB; ++db) {
-        if (rescale) {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) o[db][r] *= alpha;
-        }
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) {
-          const char* a0 = vbase + (16 * s2) * pitchB + 64 * db;
-          const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(a0));
-          const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(a0 + 8 * pitchB));
-          const short8_t a8 = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-          o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a8), pfr[s2], o[db], 0, 0, 0);
-        }
-      }
     }
-    if (j0 + MKT <= jhi) {
-      stash(ks0 + (cur ^ 1) * (MKT * KP));           // tile j0 + 32 (fetched one iteration ago) -> the other buffer
-      if (j0 + 2 * MKT <= jhi) fetch(j0 + 2 * MKT);  // in flight during the next tile's MFMAs
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) mx = fmaxf(mx, sc[t][e]);
+    mx = xor16_max(xor32_max(mx));
+    const float mn = fmaxf(m, mx);
+    float alpha = __builtin_amdgcn_exp2f(m - mn);
+    float sum = 0.f;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        sc[t][e] = __builtin_amdgcn_exp2f(sc[t][e] - mn);
+        sum += sc[t][e];
+      }
+    l = l * alpha + sum;
+    m = mn;
+    const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, make_uint4(pack2(sc[0][0], sc[0][1]), pack2(sc[0][2], sc[0][3]),
+                                                                pack2(sc[1][0], sc[1][1]), pack2(sc[1][2], sc[1][3])));
+    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {   // wave-uniform
+      asm volatile("" : "+v"(alpha));                        // (not multiplied ahead of the condition)
+#pragma unroll
+      for (int db = 0; db < 2 * NDB; ++db)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[db][e] *= alpha;
+    }
+#pragma unroll
+    for (int db = 0; db < 2 * NDB; ++db) {
+      const char* at = ks + vat + 16 * ((2 * db + (li >> 1 & 1)) ^ vsw);   // (rows r and r + 16 are exchanged alike)
+      const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)at);
+      const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(at + 256 * KCH));
+      const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, o[db], 0, 0, 0);
     }
   }
-  if (!rok) return;
+  // results through LDS (tiles and table are done with), so that whole rows are written 16 bytes a lane
+  __syncthreads();
+  l = xor16_sum(xor32_sum(l));
   const float inv = l > 0.f ? 1.0f / l : 0.f;
-  bf16_t* op = reinterpret_cast<bf16_t*>(a.out) + orow * R;
+  char* os = smem_raw + wave * 16 * Z::OP;
 #pragma unroll
-  for (int db = 0; db < NDB; ++db) {
+  for (int db = 0; db < 2 * NDB; ++db)
+    *reinterpret_cast<uint2*>(os + li * Z::OP + 32 * db + 8 * lg) = make_uint2(pack2(o[db][0] * inv, o[db][1] * inv), pack2(o[db][2] * inv, o[db][3] * inv));
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  constexpr int PR = R / 8, RPI = 64 / PR;   // pieces of a row, rows of an instruction
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      uint2 w;
-      w.x = pack2(o[db][4 * g + 0] * inv, o[db][4 * g + 1] * inv);
-      w.y = pack2(o[db][4 * g + 2] * inv, o[db][4 * g + 3] * inv);
-      *reinterpret_cast<uint2*>(op + 32 * db + 8 * g + 4 * hh) = w;
-    }
+  for (int u = 0; u < 16 / RPI; ++u) {
+    const int row = RPI * u + lane / PR;
+    const int64_t to = (int64_t)__shfl((int)orow, row, 64) * R + 8 * (lane % PR);
+    const uint4 w = *reinterpret_cast<const uint4*>(os + row * Z::OP + 16 * (lane % PR));
+    if (wrow + row < nrows) *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(a.out) + to) = w;
   }
 }
 
 template <int NDB, int NROT> hipError_t launch_mfma_rq(const LatentAttnArgs& a, hipStream_t s) {
-  static bool attr_set = false;
-  auto* fn = latent_attn_mfma_rq_kernel<NDB, NROT>;
-  const int kp = a.sh.rank + a.sh.rot_dim + 8;
-  const size_t lds = sizeof(bf16_t) * (size_t)2 * MKT * kp + sizeof(int) * BT_LDS_MAX;
-  if (!attr_set) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       64 * 1024);
-    if (e != hipSuccess) return e;
-    attr_set = true;
-  }
-  const dim3 grid((unsigned)(((int64_t)a.max_q * a.heads + 127) / 128), (unsigned)a.num_seqs);
-  hipLaunchKernelGGL(fn, grid, dim3(256), lds, s, a, kp);
+  // floor(j / block_size) = (j * bs_mul) >> (32 + bs_shift) for 31-bit j
+  int log = 1;
+  while ((int64_t)1 << log < a.block_size) ++log;
+  const uint32_t bs_mul = a.block_size == 1 ? 0 : (uint32_t)(((uint64_t)1 << (31 + log)) / a.block_size + 1);
+  const dim3 grid((unsigned)(((int64_t)a.max_q * a.heads + 63) / 64), (unsigned)a.num_seqs);
+  hipLaunchKernelGGL((latent_attn_mfma_rq_kernel<NDB, NROT>), grid, dim3(256), (RqTile<NDB, NROT>::LDS), s, a, bs_mul, log - 1);
   return hipGetLastError();
 }
 

@@ -1,0 +1,41 @@
+"""Latent attention of prompt-sized steps: the matrix-core kernel with its queries in registers against the fp32 FMA kernel, at
+remainders of its row and key tiles, every rotary width, page sizes that are no power of two and more pages than its table holds.
+
+The matrix-core side rounds softmax weights to bf16 (2^-9 of sum w |v|) and rotated queries (2^-9 of |q| in each of the rot_dim
+places: at most e = scale 2^-9 |q_rot| |k_rot| in a score, which moves weights by e^2e); both sides round results (2^-8 each)."""
+
+import pytest
+import torch
+
+from src import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rank,rot,heads,bs,window,past", [
+    (256, 32, 32, 16, 0, 0), (256, 64, 32, 24, 70, 100), (128, 16, 31, 1, 0, 1200), (64, 0, 32, 7, 0, 50), (256, 0, 33, 16, 33, 300),
+    (128, 64, 32, 16, 0, 33), (256, 16, 32, 1, 0, 1100), (64, 32, 32, 48, 200, 0)])
+def test_against_fma(cuda, rank, rot, heads, bs, window, past):
+    torch.manual_seed(rank + rot + heads)
+    S = 72   # with up to 64 tokens each: enough row tiles that the keys are not split
+    lens = [64, 1, 33, 2, 63, 31, 17, 48] * (S // 8)
+    pasts = [past + 5 * (s % 3) if past else 0 for s in range(S)]
+    T, need = sum(lens), [-(-(n + p) // bs) for n, p in zip(lens, pasts)]
+    pool = 1 + max(need) * 3
+    cache = torch.randn(pool, bs, rank + rot, device=cuda).to(torch.bfloat16)
+    bt = torch.randint(0, pool, (S, max(need)), device=cuda, dtype=torch.int32)
+    cu = torch.tensor([0] + lens, device=cuda).cumsum(0).int()
+    pos = torch.cat([torch.arange(n) + p for n, p in zip(lens, pasts)]).to(cuda)
+    ctx = torch.tensor([n + p for n, p in zip(lens, pasts)], device=cuda, dtype=torch.int32)
+    q_lat = torch.randn(heads, T, rank, device=cuda).to(torch.bfloat16)
+    q = torch.randn(T, heads * (rot + 6), device=cuda).to(torch.bfloat16)
+    inv, sink, scale = ops.rope_inv_freq(10000.0, max(rot, 2), cuda)[: rot // 2], torch.randn(heads, device=cuda) + 1, 0.08
+    args = (q_lat, q, 6, cache, bt, cu, ctx, pos, sink, 64, window, scale, rot, inv)
+    want, got = ops.latent_attn(*args, impl=1).float(), ops.latent_attn(*args, impl=2).float()
+    e = 0.0
+    if rot:
+        e = scale * 2 ** -9 * float(q.view(T, heads, -1)[..., 6:].float().norm(dim=-1).max() * cache[..., rank:].float().norm(dim=-1).max())
+    top = float(cache[..., :rank].float().abs().max())
+    assert ((got - want).abs() <= (2 ** -9 + 2 * e * 2.71828 ** (2 * e)) * top + 2 ** -7 * want.abs()).all()
+    # the bound above is for one key that has it all; over a row the roundings average out
+    assert ((got - want).norm() / want.norm()).item() < 2 ** -7
