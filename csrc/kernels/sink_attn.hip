@@ -630,6 +630,233 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 && NKC <= 16 && NDB <= 4 ? 2 
 }
 
 
+// Prompt-sized steps at the common widths (dim 64 or 128, vdim 64, 128 or 256), keys not split: the same algorithm with 16 rows per
+// wave and 16x16x32 products, so that the sums and queries take 32 + 16 registers at 128 + 128 and 4 waves share a SIMD: one's
+// softmax and waits run beside the others' products. A workgroup of 4 waves takes 64 rows; key tiles [K_g | V_g] come by DMA into two
+// buffers, one barrier per tile. A tile of 32 rows by KCH 16-byte pieces lies in LDS without gaps; the pieces of a row are exchanged
+// (XOR) so that 16 consecutive rows' reads of one piece fall on all banks.
+// Bound by the issue of vector instructions (110 per wave and tile beside 16 products). 16 ragged sequences of up to 1024 rows, 16 heads
+// in 4 groups of 128 + 128, a window of 512: 32 rows per wave (below), two waves per SIMD and tiles through registers took 110 us,
+// this takes 84; 16 sequences of 500, vdim 256: 222 -> 90. Where all keys of long sequences are seen the two come close (4 x 1500
+// rows, 32 heads: 153 and 148), as the other kernel reads LDS half as often.
+template <int NK, int NV> struct RowTile {
+  static constexpr int KCH = 4 * NK + 2 * NV, NPF = MKT * KCH / 256, BYTES = MKT * KCH * 16;
+  static constexpr int X = KCH % 16 == 0 ? 16 : 8;   // rows r and r + 16 / X share banks
+  static __device__ __forceinline__ int swz(int row) { return row / (16 / X) % X; }
+  static constexpr int OP = 32 * NV + 16;            // pitch of a result row in LDS
+  static constexpr int TABLE = 1024;                 // key rows in LDS
+  static constexpr int LDS = 2 * BYTES + 4 * TABLE > 64 * OP ? 2 * BYTES + 4 * TABLE : 64 * OP;
+};
+typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(1))) const void global_cvoid;
+
+template <int NK, int NV, bool SIG>
+__global__ void __launch_bounds__(256, NV <= 8 ? 4 : 3) sink_attn_rows_kernel(SinkAttnArgs a) {
+  using Z = RowTile<NK, NV>;
+  constexpr int KCH = Z::KCH, D = 32 * NK, DV = 16 * NV, roww = D + DV;
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];   // two tiles, key rows; at the end the results
+  int bx = blockIdx.x, by = blockIdx.y;
+  {
+    // XCD k takes a contiguous eighth of the sequence-major tile list, so one sequence's cache rows stay in one L2
+    const unsigned total = gridDim.x * gridDim.y, lin = blockIdx.x + gridDim.x * blockIdx.y;
+    if (total % 8 == 0) {
+      const unsigned nl = (lin % 8) * (total / 8) + lin / 8;
+      bx = (int)(nl % gridDim.x);
+      by = (int)(nl / gridDim.x);
+    }
+    bx = gridDim.x - 1 - bx;   // a sequence's last rows see the most keys: they start first
+  }
+  const int H = a.heads, G = a.kv_heads, QPG = H / G, s = by, g = blockIdx.z;
+  const int lane = threadIdx.x & 63, tid = threadIdx.x, li = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q0 = a.cu_q ? a.cu_q[s] : s;
+  const int nq = a.cu_q ? a.cu_q[s + 1] - q0 : 1;
+  const int nrows = nq * QPG, row0 = bx * 64;
+  if (row0 >= nrows) return;
+  const int last_row = min(row0 + 64, nrows) - 1;
+  const int p_first = (int)a.positions[q0 + row0 / QPG], p_last = (int)a.positions[q0 + last_row / QPG];
+  const int jlo = first_key(a, p_first), jhi = min(p_last, a.ctx_lens[s] - 1);
+  const int nt = jhi < jlo ? 0 : (jhi - jlo) / MKT + 1;
+
+  // cache rows of the workgroup's keys in LDS, TABLE keys at a time
+  const int* bt = a.block_tables + (int64_t)s * a.bt_stride;
+  int* rows = reinterpret_cast<int*>(smem_raw + 2 * Z::BYTES);
+  const int bs_shift = __builtin_ctz(a.block_size);   // a power of two (mfma_ok)
+  int jt = jlo;
+  auto stage_rows = [&]() {
+    for (int u = tid; u < Z::TABLE && jt + u <= jhi; u += 256)
+      rows[u] = ((bt[(jt + u) >> bs_shift] * G + g) << bs_shift) + ((jt + u) & (a.block_size - 1));
+    __syncthreads();
+  };
+  stage_rows();
+  // piece u of this thread: 16 bytes of key krow + u * 256 / KCH of the tile, or of the next one where a row ends
+  const bf16_t* cache = reinterpret_cast<const bf16_t*>(a.cache);
+  int krow[Z::NPF], pcol[Z::NPF];
+#pragma unroll
+  for (int u = 0; u < Z::NPF; ++u) {
+    const int idx = tid + 256 * u;
+    krow[u] = idx / KCH;
+    pcol[u] = 8 * ((idx % KCH) ^ Z::swz(krow[u]));
+  }
+  auto fetch = [&](int j0, int buf) {   // (keys beyond the last repeat it)
+    if (min(j0 + MKT - 1, jhi) - jt >= Z::TABLE) {
+      __syncthreads();
+      jt = j0;
+      stage_rows();
+    }
+    const int at = j0 - jt, end = jhi - jt;
+#pragma unroll
+    for (int u = 0; u < Z::NPF; ++u) {
+      const int row = rows[min(at + krow[u], end)];
+      char* to = smem_raw + buf * Z::BYTES + (256 * u + 64 * wave) * 16;
+      __builtin_amdgcn_global_load_lds((global_cvoid*)(cache + ((uint64_t)(uint32_t)row * roww + pcol[u])), (lds_void*)to, 16, 0, 0);
+    }
+  };
+  if (nt > 0) fetch(jlo, 0);
+
+  const int wrow = row0 + wave * 16, myrow = wrow + li;
+  const bool rok = myrow < nrows, wave_live = wrow < nrows, wave_full = wrow + 15 < nrows;
+  const int tq = q0 + (rok ? myrow / QPG : 0), myh = g * QPG + (rok ? myrow % QPG : 0);   // (rows beyond the last repeat the first)
+  const int64_t orow = (int64_t)tq * H + myh;
+  bf16x8_t qf[NK];
+#pragma unroll
+  for (int k = 0; k < NK; ++k)
+    qf[k] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(a.q) + orow * D + 32 * k + 8 * lg));
+  const int prow = rok ? (int)a.positions[tq] : -1;
+  const int jrow = first_key(a, max(prow, 0));
+  const unsigned seen = rok ? max(min(prow, jhi) - jrow + 1, 0) : 0;   // this row sees keys jrow .. jrow + seen - 1
+  // a tile is interior for a wave when every one of its 32 x 16 (key, row) pairs is visible: no masking then
+  const int pw_first = wave_live ? (int)a.positions[q0 + wrow / QPG] : 0;
+  const int pw_last = wave_live ? (int)a.positions[q0 + min(wrow + 15, nrows - 1) / QPG] : 0;
+  const int jw_first = first_key(a, pw_first), jw_last = first_key(a, pw_last);
+  constexpr float LOG2E = 1.4426950408889634f;
+  const float sl2 = a.scale * LOG2E;
+  const bool shaped = a.softcap > 0.f || a.slopes != nullptr;
+  const bool plain = !shaped && a.bias == nullptr && sl2 > 0.f;
+  const float capl2 = a.softcap * LOG2E, s2_over_cap = a.softcap > 0.f ? a.scale / a.softcap * 2.885390081777927f : 0.f;
+  const float slope2 = a.slopes != nullptr ? a.slopes[myh] * LOG2E : 0.f;
+  const float hb2 = SIG && a.head_bias != nullptr ? a.head_bias[myh] * LOG2E : 0.f;
+  const float* bias = a.bias ? a.bias + myh : nullptr;
+  const bool has_sink = !SIG && a.sink != nullptr && rok;
+  float m = has_sink ? a.sink[myh] * LOG2E : -1e30f;
+  float l = has_sink && lg == 0 ? 1.0f : 0.0f;   // (the sum of this lane's keys)
+  f32x4_t o[NV];
+#pragma unroll
+  for (int db = 0; db < NV; ++db) o[db] = f32x4_t{};
+  // K fragments: key li of 16, piece 4 k + lg; V fragments: keys 4 lg .. of either 16 (the order in which the weights lie in
+  // registers), columns 16 db ..
+  const int ksw = Z::swz(li), vrow = 4 * lg + (li >> 2), vsw = Z::swz(vrow);
+  const int kat = 16 * li * KCH, vat = 16 * vrow * KCH + 8 * (li & 1), vpc = 4 * NK + (li >> 1 & 1);
+  for (int i = 0; i < nt; ++i) {
+    const int j0 = jlo + i * MKT;
+    // tile i is in LDS for every wave, and every wave has left the other buffer
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(7 << 4);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (i + 1 < nt) fetch(j0 + MKT, (i + 1) & 1);
+    if (!wave_live || j0 > pw_last || j0 + MKT <= jw_first) continue;   // nothing of this tile is visible to the wave
+    const char* ks = smem_raw + (i & 1) * Z::BYTES;
+    f32x4_t sc[2] = {};
+#pragma unroll
+    for (int k = 0; k < NK; ++k)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const uint4 w = *reinterpret_cast<const uint4*>(ks + kat + 256 * KCH * t + 16 * ((4 * k + lg) ^ ksw));
+        sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, w), qf[k], sc[t], 0, 0, 0);
+      }
+    const bool interior = wave_full && j0 + MKT - 1 <= min(pw_first, jhi) && j0 >= jw_last;
+    float mul = 1.0f;   // sc * mul: scores in log2 units
+    if (plain) {
+      mul = sl2;
+    } else {
+      // capped scores: cap * tanh(s * scale / cap) = cap - 2 cap / (2^(2 x log2 e) + 1), one multiply-add of the reciprocal
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int n = prow - (j0 + 16 * t + 4 * lg + e);
+          float v = sc[t][e];
+          if (a.softcap > 0.f)
+            v = fmaf(-2.0f * capl2, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(v * s2_over_cap) + 1.0f), capl2);
+          else
+            v *= sl2;
+          v = fmaf(-slope2, (float)n, v);
+          if (bias != nullptr) v += bias[(int64_t)min(max(n, 0), a.bias_rows - 1) * H] * LOG2E;
+          sc[t][e] = v;
+        }
+    }
+    if (!interior) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sc[t][e] = (unsigned)(j0 + 16 * t + 4 * lg + e - jrow) < seen ? sc[t][e] : -INFINITY;
+    }
+    float alpha = 1.0f;
+    if constexpr (SIG) {   // 1 / (1 + 2^-(v + bias)); a masked score is -inf and weighs 0
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sc[t][e] = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(fmaf(-sc[t][e], mul, -hb2)));
+    } else {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mx = fmaxf(mx, sc[t][e]);
+      mx = xor16_max(xor32_max(mx * mul));
+      const float mn = mx > m + LAZY ? mx : m;
+      alpha = __builtin_amdgcn_exp2f(m - mn);   // v_exp_f32: arguments are <= 0 or -inf here
+      float sum = 0.f;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          sc[t][e] = __builtin_amdgcn_exp2f(fmaf(sc[t][e], mul, -mn));
+          sum += sc[t][e];
+        }
+      l = l * alpha + sum;
+      m = mn;
+    }
+    const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, make_uint4(pack2(sc[0][0], sc[0][1]), pack2(sc[0][2], sc[0][3]),
+                                                                pack2(sc[1][0], sc[1][1]), pack2(sc[1][2], sc[1][3])));
+    if (!SIG && __builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {   // wave-uniform
+      asm volatile("" : "+v"(alpha));                                // (not multiplied ahead of the condition)
+#pragma unroll
+      for (int db = 0; db < NV; ++db)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[db][e] *= alpha;
+    }
+#pragma unroll
+    for (int db = 0; db < NV; ++db) {
+      const char* at = ks + vat + 16 * ((2 * db + vpc) ^ vsw);   // (rows r and r + 16 are exchanged alike)
+      const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)at);
+      const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(at + 256 * KCH));
+      const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, o[db], 0, 0, 0);
+    }
+  }
+  // results through LDS (tiles and table are done with), so that whole rows are written 16 bytes a lane
+  __syncthreads();
+  l = xor16_sum(xor32_sum(l));
+  const float inv = SIG ? 1.0f : (l > 0.f ? 1.0f / l : 0.f);
+  char* os = smem_raw + wave * 16 * Z::OP;
+#pragma unroll
+  for (int db = 0; db < NV; ++db)
+    *reinterpret_cast<uint2*>(os + li * Z::OP + 32 * db + 8 * lg) = make_uint2(pack2(o[db][0] * inv, o[db][1] * inv), pack2(o[db][2] * inv, o[db][3] * inv));
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  constexpr int PR = DV / 8, RPI = 64 / PR;   // pieces of a row, rows of an instruction
+#pragma unroll
+  for (int u = 0; u < 16 / RPI; ++u) {
+    const int row = RPI * u + lane / PR;
+    const int64_t to = (int64_t)__shfl((int)orow, row, 64) * DV + 8 * (lane % PR);
+    const uint4 w = *reinterpret_cast<const uint4*>(os + row * Z::OP + 16 * (lane % PR));
+    if (wrow + row < nrows) *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(a.out) + to) = w;
+  }
+}
+
+
 // column c of an output row (token t, head h) after the optional turn and gate, from the row's raw columns o(c)
 template <typename F>
 __device__ __forceinline__ float gated_out(const SinkAttnArgs& a, int64_t t, int h, int c, F&& o) {
@@ -655,7 +882,7 @@ __device__ __forceinline__ float gated_out(const SinkAttnArgs& a, int64_t t, int
 //            64 / VL keys of a pass
 // The waves' sums meet in LDS, rescaled to one maximum. Bound by the loads in flight: 16 KB per wave, 3 waves per SIMD where 168
 // registers hold them (values are read after the keys' products free registers). Keys 128 at a time per workgroup, with barriers
-// between scores, softmax and values and shuffles for every sum, took 62 us of 73 (1.6 TB/s) where this takes 28 of 37: 32 sequences
+// between scores, softmax and values and shuffles for every sum, took 62 us of 73 (1.6 TB/s) where this takes 28 of 36: 32 sequences
 // of about 1500 keys, 16 heads in 4 groups, dim = vdim = 128; 64 sequences with 32 heads 194 -> 91 (4.3 TB/s).
 // Splits write unnormalised sums + (max, sum) to the workspace and
 // sink_attn_merge_kernel combines them.
@@ -905,6 +1132,7 @@ __global__ void __launch_bounds__(256, R < 8 && R * NKC * VL < 512 && NKC * VL <
 // (token, head).
 __global__ void __launch_bounds__(128) sink_attn_merge_kernel(SinkAttnArgs a) {
   __shared__ float wz[128];   // a split's weight 2^(m_z - m*) / sum (nsplit <= 128)
+  __shared__ int id[128], count[2];
   __shared__ float orow[256];
   const int64_t row = blockIdx.x, rows = (int64_t)a.heads * a.total_q;
   const int64_t t = row / a.heads;
@@ -919,19 +1147,38 @@ __global__ void __launch_bounds__(128) sink_attn_merge_kernel(SinkAttnArgs a) {
   mstar = fmaxf(red2[0], red2[1]);
   const float w = lz > 0.f ? exp2f(mz - mstar) : 0.f;
   float lsum = wave_sum(lz * w);
-  if ((threadIdx.x & 63) == 0) red2[2 + (threadIdx.x >> 6)] = lsum;
+  const bool holds = a.sigmoid ? lz > 0.f : w != 0.f;
+  const unsigned long long in = __ballot(holds);
+  if ((threadIdx.x & 63) == 0) {
+    red2[2 + (threadIdx.x >> 6)] = lsum;
+    count[threadIdx.x >> 6] = __popcll(in);
+  }
   __syncthreads();
   lsum = red2[2] + red2[3];
-  wz[z] = a.sigmoid ? (lz > 0.f ? 1.0f : 0.f) : (lsum > 0.f ? w / lsum : 0.f);
+  // the splits that hold keys, in order
+  const int n = a.sigmoid || lsum > 0.f ? count[0] + count[1] : 0;
+  if (holds) {
+    const int at = (z < 64 ? 0 : count[0]) + __popcll(in & ((1ull << (z & 63)) - 1));
+    wz[at] = a.sigmoid ? 1.0f : w / lsum;
+    id[at] = z;
+  }
   __syncthreads();
   for (int c = threadIdx.x; c < DV; c += 128) {
     float acc = 0.f;
-#pragma unroll 8
-    // loads in flight together: 7.6 -> 4.4 us for 16 splits of 512 rows (what an empty split has in the workspace is read, not used)
-    for (int k = 0; k < nsplit; ++k) {
-      const float wk = wz[k], x = a.ws_o[((int64_t)k * rows + row) * DV + c];
-      acc += wk != 0.f ? x * wk : 0.f;
-    }
+    int k0 = 0;
+    auto add = [&](auto count) {   // loads in flight together: 7.6 -> 4.4 us for 16 splits of 512 rows
+      constexpr int N = decltype(count)::value;
+      float x[N];
+#pragma unroll
+      for (int k = 0; k < N; ++k) x[k] = a.ws_o[((int64_t)id[k0 + k] * rows + row) * DV + c];
+#pragma unroll
+      for (int k = 0; k < N; ++k) acc += x[k] * wz[k0 + k];
+      k0 += N;
+    };
+    while (k0 + 8 <= n) add(IntC<8>{});
+    if (n & 4) add(IntC<4>{});
+    if (n & 2) add(IntC<2>{});
+    if (n & 1) add(IntC<1>{});
     orow[c] = acc;
   }
   if (a.out_inv_freq != nullptr) __syncthreads();   // (else every thread reads its own columns)
@@ -1022,6 +1269,23 @@ template <int NKC> hipError_t launch_decode_v(const SinkAttnArgs& a, hipStream_t
   return a.vdim <= 128 ? launch_decode_r<NKC, 16>(a, s) : launch_decode_r<NKC, 32>(a, s);
 }
 
+template <int NK, int NV> hipError_t launch_rows(const SinkAttnArgs& a, hipStream_t s) {
+  const int64_t rows = (int64_t)a.max_q * (a.heads / a.kv_heads);
+  const dim3 grid((unsigned)((rows + 63) / 64), (unsigned)a.num_seqs, (unsigned)a.kv_heads);
+  auto* fn = a.sigmoid ? sink_attn_rows_kernel<NK, NV, true> : sink_attn_rows_kernel<NK, NV, false>;
+  hipLaunchKernelGGL(fn, grid, dim3(256), (RowTile<NK, NV>::LDS), s, a);
+  return hipGetLastError();
+}
+template <int NK> hipError_t launch_rows_v(const SinkAttnArgs& a, hipStream_t s) {
+  if (a.vdim == 64) return launch_rows<NK, 4>(a, s);
+  return a.vdim == 128 ? launch_rows<NK, 8>(a, s) : launch_rows<NK, 16>(a, s);
+}
+// prompt-sized steps at the widths of sink_attn_rows_kernel, keys not split
+inline bool rows_takes(const SinkAttnArgs& a) {
+  return (a.ws_o == nullptr || a.nsplit <= 1) && a.max_q * (a.heads / a.kv_heads) > 32 && (a.dim == 64 || a.dim == 128) &&
+         (a.vdim == 64 || a.vdim == 128 || a.vdim == 256) && (int64_t)a.total_q * a.heads < (1ll << 31);
+}
+
 inline bool decode_ok(const SinkAttnArgs& a) {
   return !a.f32 && a.cu_q == nullptr && a.max_q == 1 && a.heads / a.kv_heads <= 8 && a.dim % 8 == 0 && a.dim <= 256 &&
          a.vdim % 8 == 0 && a.vdim <= 256 && (reinterpret_cast<uintptr_t>(a.q) & 15) == 0 &&
@@ -1056,6 +1320,7 @@ hipError_t launch_sink_attn(const SinkAttnArgs& a, hipStream_t s) {
   }
   if (sink_attn_uses_mfma(a)) {
     const int qpg = a.heads / a.kv_heads;
+    if (rows_takes(a)) return a.dim == 64 ? launch_rows_v<2>(a, s) : launch_rows_v<4>(a, s);
     return a.max_q * qpg <= 32 ? launch_mfma_nw<1>(a, s) : launch_mfma_nw<4>(a, s);
   }
   if (a.impl == 2) return hipErrorInvalidValue;

@@ -1,0 +1,52 @@
+"""Attention of prompt-sized steps: the 16-rows-per-wave matrix-core kernel against the fp32 FMA kernel, at remainders of its row and
+key tiles, in every score form, and over more keys than its row table holds. Weights are rounded to bf16 on the matrix-core side
+(2^-9 of sum w |v|), results on both (2^-8 each). The same inputs with the keys split go through the other kernel and the merge."""
+
+import pytest
+import torch
+
+from src.ops import seq
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("seqs", [2, 72])   # 2: split keys
+@pytest.mark.parametrize("dim,vdim,heads,groups,bs,style,past", [
+    (128, 128, 16, 4, 16, "", 0), (64, 64, 15, 5, 32, "sink", 70), (64, 128, 16, 4, 16, "cap", 5), (64, 256, 8, 2, 16, "bias", 33),
+    (128, 64, 8, 2, 8, "sigmoid", 60), (128, 256, 16, 4, 16, "window", 100), (128, 128, 12, 4, 1, "seg", 0), (128, 128, 16, 4, 4, "", 1300),
+    (128, 128, 16, 4, 16, "slopes", 200), (64, 64, 16, 4, 16, "sigmoid", 0)])
+def test_against_fma(cuda, dim, vdim, heads, groups, bs, style, past, seqs):
+    torch.manual_seed(dim + vdim + heads)
+    lens = ([130, 1, 33, 2, 63, 31, 127, 48] * 9)[:seqs]
+    pasts = [past + 7 * (s % 3) if past else 0 for s in range(seqs)]
+    T, need = sum(lens), [-(-(n + p) // bs) for n, p in zip(lens, pasts)]
+    pool = 1 + max(need) * 3
+    cache = torch.randn(pool, bs, groups * (dim + vdim), device=cuda).to(torch.bfloat16)
+    bt = torch.randint(0, pool, (seqs, max(need)), device=cuda, dtype=torch.int32)
+    cu = torch.tensor([0] + lens, device=cuda).cumsum(0).int()
+    pos = torch.cat([torch.arange(n) + p for n, p in zip(lens, pasts)]).to(cuda)
+    ctx = torch.tensor([n + p for n, p in zip(lens, pasts)], device=cuda, dtype=torch.int32)
+    q = torch.randn(T, heads * dim, device=cuda).to(torch.bfloat16)
+    f = lambda *s: torch.randn(*s, device=cuda)
+    sink, bias, window, kw = None, None, 0, {}
+    if style == "sink":
+        sink = f(heads) + 2
+    if style == "bias":
+        sink, bias = f(heads), f(40, heads)
+    if style == "cap":
+        kw = dict(softcap=5.0, slopes=torch.rand(heads, device=cuda) * 0.1)
+    if style == "slopes":
+        kw = dict(slopes=torch.rand(heads, device=cuda) * 0.1)
+    if style == "sigmoid":
+        kw = dict(sigmoid=True, head_bias=f(heads) - 3)
+    if style == "seg":
+        kw = dict(seg=100)
+    if style == "window":
+        window = 70
+    args = (q, cache, bt, cu, ctx, pos, sink, bias, max(lens), heads, groups, dim, vdim, window, dim ** -0.5)
+    want, got = seq.sink_attn(*args, impl=1, **kw).float(), seq.sink_attn(*args, impl=2, **kw).float()
+    mass = 1.0 if style != "sigmoid" else max(lens) + past + 14   # sigmoid weights do not sum to one
+    top = mass * float(cache.float().abs().max())
+    assert ((got - want).abs() <= 2 ** -8.5 * top + 2 ** -7 * want.abs()).all()
+    # the bound above is for one key that has it all; over a row the roundings average out
+    assert ((got - want).norm() / want.norm()).item() < 2 ** -7
