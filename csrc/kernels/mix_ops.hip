@@ -529,8 +529,64 @@ __global__ void __launch_bounds__(NT) topk_grouped_kernel(float* w_out, int* id_
   grouped_select(z + t * E, sc[wave], gopen[wave], E, K, count, keep, scale, w_out + t * K, id_out + t * K);
 }
 
+// softmax_select by one whole wave, E <= ROUTE_E_MAX, the same results to the bit: exponentials, scores and comparisons a lane each,
+// sums in the same order. sc [E] is LDS scratch.
+__device__ __forceinline__ void softmax_select_wave(const float* z, float* sc, const float* corr, int E, int K, float* w_out,
+                                                    int* id_out) {
+  constexpr int PL = ROUTE_E_MAX / 64;
+  const int lane = threadIdx.x & 63;
+  float mx = -INFINITY;
+  for (int e = lane; e < E; e += 64) mx = fmaxf(mx, z[e]);
+  mx = wave_max(mx);
+  for (int e = lane; e < E; e += 64) sc[e] = expf(z[e] - mx);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  float den = 0.f;
+  for (int e = 0; e < E; ++e) den += sc[e];
+  const float inv = 1.0f / den;
+  uint64_t key[PL];   // score + corr in an order that unsigned numbers keep, then the smaller index; 0: no candidate
+#pragma unroll
+  for (int i = 0; i < PL; ++i) {
+    const int e = lane + 64 * i;
+    key[i] = 0;
+    if (e < E) {
+      const float p = sc[e] * inv, v = p + (corr ? corr[e] : 0.f);
+      const uint32_t u = __float_as_uint(v + 0.0f);   // (-0 is 0)
+      if (v == v) key[i] = (uint64_t)(u & 0x80000000u ? ~u : u | 0x80000000u) << 32 | (uint32_t)(0x7fffffff - e);
+      sc[e] = p;
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  float sum = 0.f, w[PL];
+  int id[PL];
+  for (int k = 0; k < K; ++k) {
+    uint64_t best = 0;
+#pragma unroll
+    for (int i = 0; i < PL; ++i) best = key[i] > best ? key[i] : best;
+    best = wave_max_key(best);
+#pragma unroll
+    for (int i = 0; i < PL; ++i)
+      if (key[i] == best) key[i] = 0;
+    const int bi = key_index(best, E);
+    const float p = sc[bi];
+    sum += p;
+#pragma unroll
+    for (int i = 0; i < PL; ++i)   // choice k stays with lane k % 64
+      if (k == lane + 64 * i) w[i] = p, id[i] = bi;
+  }
+  const float rn = 1.0f / (sum + 1e-20f);
+#pragma unroll
+  for (int i = 0; i < PL; ++i)
+    if (lane + 64 * i < K) {
+      w_out[lane + 64 * i] = w[i] * rn;
+      id_out[lane + 64 * i] = id[i];
+    }
+}
+
 // One workgroup per token: wave v computes the logits of rows v, v + 4, ... of the router (E choices, then an
-// optional gate row); thread 0 selects.
+// optional gate row), four rows' loads in flight together; wave 0 selects. Bound by the latency of the loads and of the selection's
+// exchanges: 32 tokens, 10 choices of width 2048: 8.3 us (one row's loads at a time and one thread selecting: 9.9).
 __global__ void __launch_bounds__(NT) route_softmax_topk_kernel(float* w_out, int* id_out, float* gate_out,
                                                                const void* x, int64_t xstride, bool x_f32,
                                                                const void* wr, bool wr_f32, const float* corr, int H,
@@ -541,29 +597,39 @@ __global__ void __launch_bounds__(NT) route_softmax_topk_kernel(float* w_out, in
   const int rows = E + (gate_out ? 1 : 0);
   const bool vec = !x_f32 && !wr_f32 && H % 8 == 0 && xstride % 8 == 0 &&
                    (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(wr) & 15) == 0;
-  for (int e = wave; e < rows; e += NT / 64) {
-    float a = 0.f;
+  constexpr int WV = NT / 64, B = 4;
+  for (int e0 = wave; e0 < rows; e0 += B * WV) {
+    float a[B] = {};
     if (vec) {
       const uint4* xr = reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(x) + (int64_t)t * xstride);
-      const uint4* wp = reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(wr) + (int64_t)e * H);
+      const uint4* wp[B];   // (rows beyond the last repeat it)
+#pragma unroll
+      for (int b = 0; b < B; ++b) wp[b] = reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(wr) + (int64_t)min(e0 + WV * b, rows - 1) * H);
+#pragma unroll 4
       for (int c = lane; c < H / 8; c += 64) {
         float xf[8], wf[8];
         unpack8(xr[c], xf);
-        unpack8(wp[c], wf);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) a += xf[q] * wf[q];
+        for (int b = 0; b < B; ++b) {
+          unpack8(wp[b][c], wf);
+#pragma unroll
+          for (int q = 0; q < 8; ++q) a[b] += xf[q] * wf[q];
+        }
       }
     } else {
-      for (int c = lane; c < H; c += 64)
-        a += ldv(x, (int64_t)t * xstride + c, x_f32) * ldv(wr, (int64_t)e * H + c, wr_f32);
+      for (int b = 0; b < B; ++b)
+        for (int c = lane; c < H && e0 + WV * b < rows; c += 64)
+          a[b] += ldv(x, (int64_t)t * xstride + c, x_f32) * ldv(wr, (int64_t)(e0 + WV * b) * H + c, wr_f32);
     }
-    a = wave_sum(a);
-    if (lane == 0) z[e] = a;
+#pragma unroll
+    for (int b = 0; b < B; ++b) {
+      const float v = wave_sum(a[b]);
+      if (lane == 0 && e0 + WV * b < rows) z[e0 + WV * b] = v;
+    }
   }
   __syncthreads();
-  if (threadIdx.x != 0) return;
-  softmax_select(z, sc, corr, E, K, w_out + (int64_t)t * K, id_out + (int64_t)t * K);
-  if (gate_out) gate_out[t] = 1.0f / (1.0f + expf(-z[E]));
+  if (wave == 0) softmax_select_wave(z, sc, corr, E, K, w_out + (int64_t)t * K, id_out + (int64_t)t * K);
+  if (gate_out && threadIdx.x == 64) gate_out[t] = 1.0f / (1.0f + expf(-z[E]));
 }
 
 // Selection alone, from logits already computed (a library fp32 GEMM for prompt-sized steps): one thread per token,
