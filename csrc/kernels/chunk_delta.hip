@@ -16,8 +16,9 @@
 //
 // fp32 operands enter as three bf16 parts of 8 bits each (exact), of whose nine products the six largest are formed (the rest are
 // below 2^-25 of the whole): the fp32 matrix instructions run at the vector units' rate and in their place (7.2 us a chunk; these
-// 5.0). The state is rounded once per chunk instead of twice per token: against 64 bits its error (2-norm, 1 - 16 sequences of 8 -
-// 1024 tokens, 16 - 32 heads) is 0.4 - 1.3e-7, token by token 0.2 - 1.7e-7 and on average 10 % more.
+// 5.0). The state is rounded once per chunk instead of twice per token. Its error against 64 bits (2-norm, 1 - 16 sequences of 16 -
+// 1400 tokens, 16 - 32 heads, six seeds each) is 0.2 - 1.5e-7, token by token 0.2 - 1.7e-7 and 6 % more on average; decays per head
+// over one sequence come out even (1024 tokens: 2.24 and 2.18e-8, 300: 2.13 and 2.14e-8).
 //
 // Bound by the issue of vector and matrix instructions of the two waves per SIMD (LDS leaves one workgroup per compute unit):
 // per chunk 700 vector and 150 matrix instructions of a consuming wave beside 900 of a producing one, 11000 cycles. 16 sequences of
