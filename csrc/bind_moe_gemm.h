@@ -5,14 +5,17 @@
 
 #include "kernels/moe_gemm.h"
 
-// out [rows, ncols] (rows sorted by expert) = act(x[row] W_e^T): returns false, with nothing launched, where the sizes do not tile.
+// out [rows, ncols] (rows sorted by expert) = act(x[row] W_e^T): returns false, with nothing launched, where the sizes do not tile or
+// the weights are strided views (the library products that the caller has for such cases take any strides).
 inline bool moe_gemm_op(at::Tensor out, at::Tensor x, at::Tensor w, at::Tensor offsets, std::optional<at::Tensor> sorted, int64_t topk,
                         std::optional<at::Tensor> scale, int64_t act, double limit, double alpha, hipStream_t stream) {
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 &&
                   out.scalar_type() == at::kBFloat16 && w.is_cuda() && out.is_cuda(),
               "moe_gemm: bf16 device tensors");
-  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && w.dim() == 3 && w.is_contiguous() && out.dim() == 2 && out.is_contiguous() &&
-                  w.size(2) == x.size(1),
+  TORCH_CHECK(w.device() == x.device() && out.device() == x.device() && offsets.device() == x.device() &&
+                  (!sorted.has_value() || sorted->device() == x.device()) && (!scale.has_value() || scale->device() == x.device()),
+              "moe_gemm: one device");
+  TORCH_CHECK(x.dim() == 2 && x.stride(1) == 1 && w.dim() == 3 && out.dim() == 2 && out.is_contiguous() && w.size(2) == x.size(1),
               "moe_gemm: x [rows, K], w [E, N, K], out [rows, ncols]");
   TORCH_CHECK(act >= die::MOE_ACT_NONE && act <= die::MOE_ACT_RELU2, "moe_gemm: activation");
   const bool gated = act >= die::MOE_ACT_SILU && act <= die::MOE_ACT_GELU;
@@ -49,7 +52,7 @@ inline bool moe_gemm_op(at::Tensor out, at::Tensor x, at::Tensor w, at::Tensor o
   a.ncols = (int)out.size(1);
   a.K = (int)x.size(1);
   if (a.rows == 0) return true;
-  if (!die::moe_gemm_takes(a)) return false;
+  if (!w.is_contiguous() || !die::moe_gemm_takes(a)) return false;
   const hipError_t e = die::launch_moe_gemm(a, stream);
   TORCH_CHECK(e == hipSuccess, "moe_gemm: ", hipGetErrorString(e));
   return true;

@@ -205,8 +205,10 @@ def grouped_experts(kern, x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, 
                     scale: Optional[torch.Tensor] = None) -> bool:
     """Both products of every expert over its rows, two launches: ys[j] = W2 act(s W13 x[sorted_idx[j] / k]) for the rows j of the
     expert-sorted order, s = scale by (token, slot). The expert offsets stay on the device. False, with nothing done, where the
-    sizes do not tile (bf16, widths in multiples of 256)."""
+    sizes do not tile (bf16, widths in multiples of 256) or the weights are strided views."""
     if x.dtype != torch.bfloat16 or w2.shape[2] % 64 or ys.shape[1] % 256:
+        return False
+    if not (w13.is_contiguous() and w2.is_contiguous()) or w2.data_ptr() % 16:
         return False
     a = torch.empty(ys.shape[0], w2.shape[2], dtype=x.dtype, device=x.device)
     if not kern.moe_gemm(a, x, w13, offsets, sorted_idx, k, scale, act, limit, alpha):

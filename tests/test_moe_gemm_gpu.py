@@ -105,3 +105,32 @@ def test_mixtures_of_prompt_steps(cuda, t, h, f, e, k):
         y = got(lambda *ts: [v.to(cuda) for v in ts]).float().cpu()
         err = (y - want.float()).norm() / want.float().norm()
         assert err < 1e-2, (name, err)   # two roundings to bf16 on either side
+
+
+@pytest.mark.parametrize("stack", ["slice", "transposed"])
+def test_strided_weights_take_the_library(cuda, stack):
+    """Expert weights that are views (every other expert of a stack, a wider stack's columns, transposed storage) give the bits of the
+    library products on copies of them that the grouped product does not take either (an unaligned start)."""
+    from src import ops
+
+    g = torch.Generator().manual_seed(3)
+    t, h, f, e, k, bf = 300, 256, 512, 4, 2, torch.bfloat16
+    randn = lambda *s: (torch.randn(*s, generator=g) * 0.05).to(bf).to(cuda)
+    if stack == "slice":
+        w13, w1, w2 = randn(2 * e, 2 * f, h)[::2], randn(e, f, h + 64)[:, :, :h], randn(e, h + 8, f)[:, :h]
+    else:
+        w13, w1, w2 = (randn(e, h, n).transpose(1, 2) for n in (2 * f, f, f))
+        w2 = randn(e, f, h).transpose(1, 2)
+    assert not (w13.is_contiguous() or w1.is_contiguous() or w2.is_contiguous())
+
+    def off(v):   # the same values from an address that is no multiple of 16 bytes
+        return torch.empty(v.numel() + 1, dtype=bf, device=cuda)[1:].view(v.shape).copy_(v)
+
+    x, w = torch.randn(t, h, generator=g).to(bf).to(cuda), torch.rand(t, k, generator=g).to(cuda)
+    ids = torch.rand(t, e, generator=g).argsort(1)[:, :k].int().to(cuda)
+    for run in (lambda a, _, c: mix.moe_input_scaled(x, a, c, w, ids),
+                lambda a, _, c: mix.moe_output_weighted(x, a, c, w, ids, mix.ACT_CLAMPED, 7.0, 1.7),
+                lambda _, b, c: mix.moe_output_weighted(x, b, c, w, ids, mix.ACT_RELU2, 0.0, 0.0),
+                lambda a, _, c: ops.moe_apply(x, a, c, w, ids, e)):
+        got, want = run(w13, w1, w2).float(), run(off(w13), off(w1), off(w2)).float()
+        assert ((got - want).norm() / want.norm()).item() < 2 ** -9   # the library may take another kernel for other strides
