@@ -354,7 +354,8 @@ void qkv_prep(Tensor q_out, Tensor cache, Tensor q, Tensor k, OptTensor v, int64
   HIP_OK(die::launch_qkv_prep(a, cur_stream()));
 }
 
-void sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, OptTensor cu_q, Tensor ctx_lens,
+// returns the form that ran (sink_attn_form)
+const char* sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, OptTensor cu_q, Tensor ctx_lens,
                Tensor positions, OptTensor sink, OptTensor bias, int64_t max_q, int64_t heads, int64_t kv_heads,
                int64_t dim, int64_t vdim, int64_t window, double scale, int64_t impl, double softcap,
                OptTensor slopes, int64_t seg, OptTensor gate, OptTensor out_inv_freq, double gate_mult, bool sigmoid,
@@ -466,14 +467,14 @@ void sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, OptTenso
   a.ostride = out.stride(0);
   if (!gate.has_value()) {
     HIP_OK(die::launch_sink_attn(a, cur_stream()));
-    return;
+    return die::sink_attn_form(a);
   }
   if (die::sink_attn_fuses_gate(a)) {
     a.gate = gate->data_ptr();
     a.gstride = gate->stride(0);
     a.out_inv_freq = f32_ptr(out_inv_freq, vdim / 2, "out_inv_freq");
     HIP_OK(die::launch_sink_attn(a, cur_stream()));
-    return;
+    return die::sink_attn_form(a);
   }
   // the other forms write plain rows; the gate is a launch of its own
   Tensor raw = at::empty({T, heads * vdim}, q.options());
@@ -494,6 +495,7 @@ void sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, OptTenso
   g.heads = (int)heads;
   g.vdim = (int)vdim;
   HIP_OK(die::launch_rot_head_gate(g, cur_stream()));
+  return die::sink_attn_form(a);
 }
 
 }  // namespace

@@ -180,5 +180,8 @@ bool sink_attn_uses_mfma(const SinkAttnArgs& a);
 bool sink_attn_uses_decode(const SinkAttnArgs& a);
 // whether launch_sink_attn would apply the gate epilogue (nsplit already chosen)
 bool sink_attn_fuses_gate(const SinkAttnArgs& a);
+// the form that launch_sink_attn runs (nsplit already chosen): "decode", "rows" (16 rows per wave), "tiles" (32 rows per wave), "split"
+// (the same with the keys split) or "fma"
+const char* sink_attn_form(const SinkAttnArgs& a);
 
 }  // namespace die

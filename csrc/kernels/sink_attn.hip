@@ -637,8 +637,9 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 && NKC <= 16 && NDB <= 4 ? 2 
 // (XOR) so that 16 consecutive rows' reads of one piece fall on all banks.
 // Bound by the issue of vector instructions (110 per wave and tile beside 16 products). 16 ragged sequences of up to 1024 rows, 16 heads
 // in 4 groups of 128 + 128, a window of 512: 32 rows per wave (below), two waves per SIMD and tiles through registers took 110 us,
-// this takes 84; 16 sequences of 500, vdim 256: 222 -> 90. Where all keys of long sequences are seen the two come close (4 x 1500
-// rows, 32 heads: 153 and 148), as the other kernel reads LDS half as often.
+// this takes 84; 16 sequences of 500, vdim 256: 222 -> 90. Long sequences whose keys are all seen (the other kernel reads LDS half as
+// often there): 4 x 1500 rows of 32 heads 161 -> 149, 4 x 4096 of 16 558 -> 475, 1 x 16384 2582 -> 2501. With a bias per distance
+// (130 distances, a window of 1024) 16 x 1024 rows 160 -> 141, 4 x 4096 240 -> 228 (where every score looks its distance up: 182, 297).
 template <int NK, int NV> struct RowTile {
   static constexpr int KCH = 4 * NK + 2 * NV, NPF = MKT * KCH / 256, BYTES = MKT * KCH * 16;
   static constexpr int X = KCH % 16 == 0 ? 16 : 8;   // rows r and r + 16 / X share banks
@@ -737,6 +738,7 @@ __global__ void __launch_bounds__(256, NV <= 8 ? 4 : 3) sink_attn_rows_kernel(Si
   const float slope2 = a.slopes != nullptr ? a.slopes[myh] * LOG2E : 0.f;
   const float hb2 = SIG && a.head_bias != nullptr ? a.head_bias[myh] * LOG2E : 0.f;
   const float* bias = a.bias ? a.bias + myh : nullptr;
+  const float bias_far = bias ? bias[(int64_t)(a.bias_rows - 1) * H] * LOG2E : 0.f;
   const bool has_sink = !SIG && a.sink != nullptr && rok;
   float m = has_sink ? a.sink[myh] * LOG2E : -1e30f;
   float l = has_sink && lg == 0 ? 1.0f : 0.0f;   // (the sum of this lane's keys)
@@ -781,10 +783,24 @@ __global__ void __launch_bounds__(256, NV <= 8 ? 4 : 3) sink_attn_rows_kernel(Si
             v = fmaf(-2.0f * capl2, __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(v * s2_over_cap) + 1.0f), capl2);
           else
             v *= sl2;
-          v = fmaf(-slope2, (float)n, v);
-          if (bias != nullptr) v += bias[(int64_t)min(max(n, 0), a.bias_rows - 1) * H] * LOG2E;
-          sc[t][e] = v;
+          sc[t][e] = fmaf(-slope2, (float)n, v);
         }
+      if (bias != nullptr) {
+        // distances from bias_rows - 1 on share the table's last row: a lane whose keys all lie that far back looks nothing up
+        const int n0 = prow - (j0 + 4 * lg);   // of the lane's first key; the others are 1 .. 3 and 16 .. 19 nearer
+        if (n0 - 19 >= a.bias_rows - 1) {
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sc[t][e] += bias_far;
+        } else {
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              sc[t][e] += bias[(int64_t)min(max(n0 - 16 * t - e, 0), a.bias_rows - 1) * H] * LOG2E;
+        }
+      }
     }
     if (!interior) {
 #pragma unroll
@@ -1306,6 +1322,12 @@ bool sink_attn_uses_mfma(const SinkAttnArgs& a) { return a.impl != 1 && mfma_ok(
 bool sink_attn_uses_decode(const SinkAttnArgs& a) { return a.impl == 0 && decode_ok(a); }
 bool sink_attn_fuses_gate(const SinkAttnArgs& a) {
   return sink_attn_uses_decode(a) || (sink_attn_uses_mfma(a) && a.ws_o != nullptr && a.nsplit > 1);
+}
+
+const char* sink_attn_form(const SinkAttnArgs& a) {
+  if (sink_attn_uses_decode(a)) return "decode";
+  if (!sink_attn_uses_mfma(a)) return "fma";
+  return rows_takes(a) ? "rows" : a.ws_o != nullptr && a.nsplit > 1 ? "split" : "tiles";
 }
 
 hipError_t launch_sink_attn(const SinkAttnArgs& a, hipStream_t s) {

@@ -10,6 +10,20 @@ from src.ops import seq
 pytestmark = pytest.mark.gpu
 
 
+def _forms(monkeypatch):
+    """The forms that sink_attn's launches took, in a list that grows with every call."""
+    kern, forms = seq._kern(), []
+
+    class Spy:
+        def __getattr__(self, name):
+            if name != "sink_attn":
+                return getattr(kern, name)
+            return lambda *a: forms.append(kern.sink_attn(*a))
+
+    monkeypatch.setattr(seq, "_kern", lambda: Spy())
+    return forms
+
+
 @pytest.mark.parametrize("seqs", [2, 72])   # 2: split keys
 @pytest.mark.parametrize("dim,vdim,heads,groups,bs,style,past", [
     (128, 128, 16, 4, 16, "", 0), (64, 64, 15, 5, 32, "sink", 70), (64, 128, 16, 4, 16, "cap", 5), (64, 256, 8, 2, 16, "bias", 33),
@@ -49,4 +63,28 @@ def test_against_fma(cuda, dim, vdim, heads, groups, bs, style, past, seqs):
     top = mass * float(cache.float().abs().max())
     assert ((got - want).abs() <= 2 ** -8.5 * top + 2 ** -7 * want.abs()).all()
     # the bound above is for one key that has it all; over a row the roundings average out
+    assert ((got - want).norm() / want.norm()).item() < 2 ** -7
+
+
+@pytest.mark.parametrize("dim,vdim", [(128, 128), (64, 64), (64, 256)])
+@pytest.mark.parametrize("rows,style", [(1, ""), (2, "slopes"), (20, ""), (33, "cap"), (64, ""), (400, "")])
+def test_distance_bias_where_distances_end(cuda, monkeypatch, dim, vdim, rows, style):
+    """A bias per distance whose table ends within a lane's keys, at their first and last, and beyond all of them: keys so far back
+    that all share its last row are not looked up. Unsplit keys, the 16-rows-per-wave kernel."""
+    torch.manual_seed(rows + dim)
+    forms, heads, groups, bs, seqs = _forms(monkeypatch), 16, 4, 16, 72
+    lens = ([130, 1, 33, 2, 63, 31, 127, 48] * 9)[:seqs]
+    pasts, T, need = [11 * (s % 4) for s in range(seqs)], sum(lens), 12
+    cache = torch.randn(40, bs, groups * (dim + vdim), device=cuda).to(torch.bfloat16)
+    bt = torch.randint(0, 40, (seqs, need), device=cuda, dtype=torch.int32)
+    cu = torch.tensor([0] + lens, device=cuda).cumsum(0).int()
+    pos = torch.cat([torch.arange(n) + p for n, p in zip(lens, pasts)]).to(cuda)
+    ctx = torch.tensor([n + p for n, p in zip(lens, pasts)], device=cuda, dtype=torch.int32)
+    q = torch.randn(T, heads * dim, device=cuda).to(torch.bfloat16)
+    bias = torch.randn(rows, heads, device=cuda) * 2
+    kw = {"cap": dict(softcap=5.0), "slopes": dict(slopes=torch.rand(heads, device=cuda) * 0.1)}.get(style, {})
+    args = (q, cache, bt, cu, ctx, pos, None, bias, max(lens), heads, groups, dim, vdim, 0, dim ** -0.5)
+    want, got = seq.sink_attn(*args, impl=1, **kw).float(), seq.sink_attn(*args, impl=2, **kw).float()
+    assert forms == ["fma", "rows"]
+    assert ((got - want).abs() <= 2 ** -8.5 * float(cache.float().abs().max()) + 2 ** -7 * want.abs()).all()
     assert ((got - want).norm() / want.norm()).item() < 2 ** -7
