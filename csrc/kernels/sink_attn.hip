@@ -938,7 +938,7 @@ __global__ void __launch_bounds__(256, R < 8 && R * NKC * VL < 512 && NKC * VL <
   const int bs_shift = (a.block_size & (a.block_size - 1)) == 0 ? __builtin_ctz(a.block_size) : -1;
   // Every load is unconditional, so that all of them are in flight together: keys beyond the last repeat it (their weights are
   // zero), lanes beyond a row's width repeat its start (the query is zero there, the output columns are not used)
-  uint32_t rows[KT];   // cache row of key li of each 16
+  int64_t rows[KT];    // cache row of key li of each 16 (narrow rows: a cache of 2^32 of them fits the memory)
   int blk[KT];         // its block, asked for a trip ahead
   auto block_of = [&](int j) { return bs_shift >= 0 ? j >> bs_shift : j / a.block_size; };
   auto ask = [&](int j0) {
@@ -949,7 +949,7 @@ __global__ void __launch_bounds__(256, R < 8 && R * NKC * VL < 512 && NKC * VL <
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
       const int j = min(j0 + 16 * t + li, jhi);
-      rows[t] = (uint32_t)(blk[t] * G + g) * (uint32_t)a.block_size + (uint32_t)(j - block_of(j) * a.block_size);
+      rows[t] = ((int64_t)blk[t] * G + g) * a.block_size + (j - block_of(j) * a.block_size);
     }
   };
   bf16x8_t kq[KT][NKC];
@@ -957,7 +957,7 @@ __global__ void __launch_bounds__(256, R < 8 && R * NKC * VL < 512 && NKC * VL <
   auto load_keys = [&]() {
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
-      const bf16_t* row = cache + (uint64_t)rows[t] * roww;
+      const bf16_t* row = cache + rows[t] * roww;
 #pragma unroll
       for (int c = 0; c < NKC; ++c) {
         const int d = 32 * c + 8 * lg;
@@ -968,8 +968,8 @@ __global__ void __launch_bounds__(256, R < 8 && R * NKC * VL < 512 && NKC * VL <
   auto load_values = [&]() {
 #pragma unroll
     for (int u = 0; u < NPV; ++u) {
-      const uint32_t row = __shfl(rows[u * NV / 16], u * NV % 16 + vg, 64);
-      vq[u] = *reinterpret_cast<const uint4*>(cache + (uint64_t)row * roww + D + (8 * vl < DV ? 8 * vl : 0));
+      const int64_t row = __shfl((long long)rows[u * NV / 16], u * NV % 16 + vg, 64);
+      vq[u] = *reinterpret_cast<const uint4*>(cache + row * roww + D + (8 * vl < DV ? 8 * vl : 0));
     }
   };
   int j0 = jlo + KPT * wave;

@@ -48,3 +48,26 @@ def test_edges(cuda, dim, vdim, heads, groups, bs, style, width):
     want = seq.sink_attn(*args("cpu"), 1, heads, groups, dim, vdim, window, dim ** -0.5, **put("cpu")).float()
     got = seq.sink_attn(*args(cuda), 1, heads, groups, dim, vdim, window, dim ** -0.5, **put(cuda)).float().cpu()
     assert ((got - want).abs() <= 2 ** -7 * want.abs() + 1e-4 * want.abs().max()).all()
+
+
+def test_cache_of_more_rows_than_32_bits_count(cuda):
+    """The narrowest rows (8 + 8 values): blocks on either side of row 2^32 of one cache. Rows counted in 32 bits would be those of
+    the first blocks, which hold other values."""
+    bs, high = 16, 2 ** 28   # block 2^28 starts at row 2^32
+    if torch.cuda.mem_get_info()[0] < 160 * 2 ** 30:
+        pytest.skip("the cache takes 128 GiB")
+    torch.manual_seed(0)
+    heads, dim, vdim, ctx = 2, 8, 8, torch.tensor([90, 33], dtype=torch.int32)
+    small = torch.randn(16, bs, dim + vdim).to(torch.bfloat16)
+    big = torch.empty(high + 8, bs, dim + vdim, dtype=torch.bfloat16, device=cuda)
+    big[:8] = 9.0
+    big[high - 8:] = small.to(cuda)
+    near = torch.tensor([[7, 8, 15, 3, 10, 9], [12, 0, 8, 1, 2, 4]], dtype=torch.int32)
+    q = torch.randn(2, heads * dim).to(torch.bfloat16)
+    pos = ctx.long() - 1
+    want = seq.sink_attn(q, small, near, None, ctx, pos, None, None, 1, heads, 1, dim, vdim, 0, 0.35).float()
+    got = seq.sink_attn(q.to(cuda), big, (near + high - 8).to(cuda), None, ctx.to(cuda), pos.to(cuda), None, None, 1, heads, 1, dim, vdim,
+                        0, 0.35).float().cpu()
+    del big
+    torch.cuda.empty_cache()
+    assert ((got - want).abs() <= 2 ** -7 * want.abs() + 1e-4 * want.abs().max()).all()
