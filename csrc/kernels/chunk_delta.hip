@@ -1,6 +1,7 @@
 // The gated delta rule S <- diag(g_t) S, u_t = beta_t (v_t - S^T k_t), S <- S + k_t u_t^T, o_t = S^T q_t of prompt portions in
-// chunks of 16 tokens on the matrix cores (gfx950), normed and gated. Same results as the token-by-token kernel, with fp32 operands,
-// products and sums throughout.
+// chunks of 16 tokens on the matrix cores (gfx950), normed and gated. State, operands and sums are fp32, as in the token-by-token
+// kernel, in another order; decays, norm and gate are the same functions to the bit (hardware exponentials, a reciprocal and a
+// reciprocal root in norm and gate took 2 - 4 % less and rounded 12 of 262144 gated values to the other neighbour).
 //
 // With G_i = g_1 .. g_i (elementwise over the key channels) and, for j <= i, M_ij = sum_d k_i g_(j+1) .. g_i k_j and P_ij the same
 // with q_i, a chunk is
@@ -38,8 +39,18 @@ __device__ __forceinline__ f32x4_t mm(float a, float b, f32x4_t c) { return __bu
 __device__ __forceinline__ float dpp_ror8(float x) {   // of lane ^ 8
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false));
 }
+// the value of lane E of the own quad
+template <int E> __device__ __forceinline__ float of_quad(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), E * 0x55, 0xf, 0xf, true));
+}
+// n / (1 + e^-g), n = g or 1: the quotient by the reciprocal, corrected by its residual, which is the division's but for rare last
+// bits in half its instructions. Both sides are scaled, as the reciprocal of a divisor beyond 2^126 would be flushed; where e^-g
+// overflows or g is infinite there is no residual, and the quotient is exact without.
+__device__ __forceinline__ float gated(float n, float g) {
+  const float m = n * 0x1p-8f, d = fmaf(expf(-g), 0x1p-8f, 0x1p-8f), r = __builtin_amdgcn_rcpf(d), q = m * r;
+  return fabsf(g) < 88.7f ? fmaf(fmaf(-d, q, m), r, q) : q;
+}
 __device__ __forceinline__ f32x4_t ld4(const float* p) { return *reinterpret_cast<const f32x4_t*>(p); }
-__device__ __forceinline__ float sigm(float z) { return __builtin_amdgcn_rcpf(1.0f + exp_of<true>(-z)); }
 
 // x = h + m + l in bf16 parts, exact (8 bits each, rounded to nearest): pairs of values, packed
 __device__ __forceinline__ void split3(float x, float y, uint32_t (&p)[3]) {
@@ -377,16 +388,14 @@ __global__ void __launch_bounds__(64 * NC + 2 * D, 1) chunk_delta_kernel(GatedDe
     f32x4_t ss = {};
 #pragma unroll
     for (int w = 0; w < NC; ++w) ss += ld4(q + w * CT);
+    // (the four rows' factors by four lanes, one each)
+    const float own = (lane & 2) != 0 ? ((lane & 1) != 0 ? ss[3] : ss[2]) : ((lane & 1) != 0 ? ss[1] : ss[0]);
+    const float f = a.mult / sqrtf(own * (1.0f / V) + a.eps);
+    const float rs[4] = {of_quad<0>(f), of_quad<1>(f), of_quad<2>(f), of_quad<3>(f)};
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const float x = ss[e] * (1.0f / V) + a.eps, rr = __builtin_amdgcn_rsqf(x);
-      const float rs = a.mult * rr;
+    for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const float g = gd[c][e];
-        y[c][e] = o[c][e] * rs * nw[c] * (a.gate_sigmoid ? 1.0f : g) * sigm(g);
-      }
-    }
+      for (int c = 0; c < 2; ++c) y[c][e] = o[c][e] * rs[e] * nw[c] * gated(a.gate_sigmoid ? 1.0f : gd[c][e], gd[c][e]);
   };
   auto store = [&](int n) {
     bf16_t* to = reinterpret_cast<bf16_t*>(a.out) + (int64_t)(q0 + n * CT) * a.ostride + h * V;

@@ -71,3 +71,30 @@ def test_later_tokens_do_not_reach_earlier_rows(cuda, what):
     assert torch.equal(got[keep], want[keep])
     assert torch.equal(got[at:160, V:], want[at:160, V:])
     assert not torch.isfinite(got[at, :V]).all()
+
+
+@pytest.mark.parametrize("sigmoid", [False, True])
+@pytest.mark.parametrize("vdim", [64, 128, 256])
+def test_norm_and_gate_are_those_of_short_portions(cuda, vdim, sigmoid):
+    """Norm and gate of every bf16 value, to the bit as the token-by-token kernel gives them. Every token drops the state and writes one
+    value under a unit key, so that its row's result is that value exactly on either side; values of 8 bits, whose squares' sums are
+    exact in any order."""
+    torch.manual_seed(vdim)
+    H, D = 4, 64
+    gate = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    gate = gate[torch.isfinite(gate)]
+    gate = torch.cat([gate, gate[:65536 - gate.numel()]]).repeat(4)[torch.randperm(4 * 65536)].view(-1, H * vdim)
+    T = gate.shape[0]
+    eye = torch.eye(D)[torch.arange(T) % 8].repeat(1, H)
+    v = (torch.randn(T, H, 1).to(torch.bfloat16).float() * torch.ones(vdim)).view(T, -1)
+    qkv, bg = torch.cat([eye, eye, v], 1).to(cuda), torch.cat([torch.ones(T, H), torch.zeros(T, H)], 1).to(cuda)
+    norm = torch.rand(vdim, device=cuda) + 0.5
+
+    def run(rows):   # the same tokens as sequences of `rows`
+        S = T // rows
+        rag = seq.Ragged(torch.arange(rows).repeat(S).to(cuda), (torch.arange(S + 1) * rows).int().to(cuda), torch.arange(S).int().to(cuda))
+        return seq.gated_delta(qkv, bg, gate.to(cuda), norm, 1e-6, torch.zeros(S, H, D, vdim, device=cuda), H, H, D, vdim, rag,
+                               gate_sigmoid=sigmoid, mult=0.7)
+
+    chunks, tokens = run(256), run(8)   # in chunks, token by token
+    assert torch.equal(chunks, tokens), ((chunks != tokens).sum().item(), T * H * vdim)
