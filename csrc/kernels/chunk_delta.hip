@@ -17,9 +17,9 @@
 //
 // fp32 operands enter as three bf16 parts of 8 bits each (exact), of whose nine products the six largest are formed (the rest are
 // below 2^-25 of the whole): the fp32 matrix instructions run at the vector units' rate and in their place (7.2 us a chunk; these
-// 5.0). The state is rounded once per chunk instead of twice per token. Its error against 64 bits (2-norm, 1 - 16 sequences of 16 -
-// 1400 tokens, 16 - 32 heads, six seeds each) is 0.2 - 1.5e-7, token by token 0.2 - 1.7e-7 and 6 % more on average; decays per head
-// over one sequence come out even (1024 tokens: 2.24 and 2.18e-8, 300: 2.13 and 2.14e-8).
+// 5.0). Where a sum enters the state, lower parts are summed apart and added once, and of T the part below its diagonal is
+// multiplied; the state is rounded once per chunk instead of twice per token. Its error against 64 bits (2-norm; 1 - 16 sequences of
+// 32 - 1400 rows, 12 draws each) is 0.2 - 1.0e-7, 0.90 - 0.93 of that of the token-by-token kernel, decays per head and per channel.
 //
 // Bound by the issue of vector and matrix instructions of the two waves per SIMD (LDS leaves one workgroup per compute unit):
 // per chunk 700 vector and 150 matrix instructions of a consuming wave beside 900 of a producing one, 11000 cycles. 16 sequences of
@@ -325,7 +325,7 @@ __global__ void __launch_bounds__(64 * NC + 2 * D, 1) chunk_delta_kernel(GatedDe
         for (int r = 0; r < 4; ++r) t[r] = lg == b ? x[r] : lg > b ? z[r] : t[r];
       }
 #pragma unroll
-      for (int r = 0; r < 4; ++r) T[(4 * lg + r) * TP + li] = 4 * lg + r >= li ? t[r] : 0.f;
+      for (int r = 0; r < 4; ++r) T[(4 * lg + r) * TP + li] = 4 * lg + r > li ? t[r] : 0.f;   // (T - 1)
     };
     fetch_gates(0);
     fetch(0);
@@ -417,7 +417,7 @@ __global__ void __launch_bounds__(64 * NC + 2 * D, 1) chunk_delta_kernel(GatedDe
     const char* kd = sm + Z::kd + n % 3 * Z::SK;
     const float* end = reinterpret_cast<const float*>(kd + D * Z::DP) + 4 * lg;   // G_16, beta
     if (n > 0) norm(n - 1);   // (before the loop's first products: the two run side by side)
-    f32x4_t ks[2] = {}, qs[2] = {};
+    f32x4_t ks[2] = {}, qs[2] = {}, kl[2] = {};   // kl: the products of lower parts, so that ks is rounded once per 32 channels
     const char* xa = sm + n % 2 * Z::SX + li * Z::XP + 16 * lg;
 #pragma unroll
     for (int t = 0; t < ND; t += 2) {
@@ -439,7 +439,7 @@ __global__ void __launch_bounds__(64 * NC + 2 * D, 1) chunk_delta_kernel(GatedDe
         for (int i = 0; i < 3; ++i)   // all but the products below 2^-24 of the largest
 #pragma unroll
           for (int j = 0; i + j < 3; ++j) {
-            ks[c] = mm(kf[i], sf[j], ks[c]);
+            (i + j > 0 ? kl : ks)[c] = mm(kf[i], sf[j], (i + j > 0 ? kl : ks)[c]);
             qs[c] = mm(qf[i], sf[j], qs[c]);
           }
       }
@@ -452,7 +452,7 @@ __global__ void __launch_bounds__(64 * NC + 2 * D, 1) chunk_delta_kernel(GatedDe
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        R[c][e] = n * CT + 4 * lg + e < L ? beta[e] * (vv[c][e] - ks[c][e]) : 0.f;
+        R[c][e] = n * CT + 4 * lg + e < L ? beta[e] * (vv[c][e] - (ks[c][e] + kl[c][e])) : 0.f;
         gd[c][e] = gt[c][e];
       }
     if (n + 1 < nch) fetch(n + 1);
@@ -484,6 +484,8 @@ __global__ void __launch_bounds__(64 * NC + 2 * D, 1) chunk_delta_kernel(GatedDe
     for (int e = 0; e < 4; ++e)
 #pragma unroll
       for (int c = 0; c < 2; ++c) U[c] = mm(tf[e], R[c][e], U[c]);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) U[c] += R[c];
     take_out(U);
     bf16x8_t uf[2][3];   // (h, h), (m, m), (l, h): against (h, m), (h, m), (h, l) the same products as above and m m
     auto parts = [&]() {

@@ -98,3 +98,46 @@ def test_norm_and_gate_are_those_of_short_portions(cuda, vdim, sigmoid):
 
     chunks, tokens = run(256), run(8)   # in chunks, token by token
     assert torch.equal(chunks, tokens), ((chunks != tokens).sum().item(), T * H * vdim)
+
+
+@pytest.mark.parametrize("channel", [False, True])
+def test_state_is_no_further_from_64_bits_than_token_by_token(cuda, channel):
+    """Portions of 32 rows from an empty state, 12 draws: the 2-norm distance of the state from a float64 evaluation, in chunks and, the
+    same rows eight at a time, token by token. (0.92 of the other's, 1 % from draw to draw.)"""
+    S, L, H, D = 16, 32, 16, 128
+    T = S * L
+    unit = lambda x: x / x.norm(dim=-1, keepdim=True)
+    err = [0.0, 0.0]
+    for seed in range(12):
+        gen = torch.Generator(cuda).manual_seed(seed)
+        f = lambda *s: torch.randn(*s, device=cuda, generator=gen)
+        q, k, v, beta = unit(f(S, L, H, D)), unit(f(S, L, H, D)), f(S, L, H, D), torch.sigmoid(f(S, L, H))
+        A_log = 0.5 * f(H)
+        extra, bg = {}, beta
+        if channel:
+            z = (0.5 * f(S, L, H * D)).to(torch.bfloat16)
+            extra = dict(z_bias=0.7 * f(H * D) - 2.5, A_log=A_log)
+            sp = torch.nn.functional.softplus(z.double() + extra["z_bias"].double())
+            dec = torch.exp(-A_log.double().exp()[:, None] * sp.view(S, L, H, D))
+        else:
+            dec = torch.exp(-A_log.exp() * torch.nn.functional.softplus(0.7 * f(S, L, H) - 2.5))
+            bg, dec = torch.cat([beta, dec], -1), dec.double()[..., None].expand(S, L, H, D)
+        want = torch.zeros(S, H, D, D, dtype=torch.float64, device=cuda)
+        for t in range(L):
+            want *= dec[:, t, :, :, None]
+            kt = k[:, t].double()
+            u = beta[:, t, :, None].double() * (v[:, t].double() - (want * kt[..., None]).sum(2))
+            want += kt[..., None] * u[:, :, None]
+        qkv = torch.cat([x.reshape(S, L, -1) for x in (q, k, v)], 2)
+        gate, norm = torch.zeros(T, H * D, device=cuda, dtype=torch.bfloat16), torch.ones(D, device=cuda)
+        for n, rows in enumerate((L, 8)):
+            state = torch.zeros(S, H, D, D, device=cuda)
+            for a in range(0, L, rows):
+                cut = lambda x: x[:, a:a + rows].reshape(S * rows, -1).contiguous()
+                rag = seq.Ragged(torch.arange(a, a + rows, device=cuda).repeat(S), (torch.arange(S + 1, device=cuda) * rows).int(),
+                                 torch.arange(S, device=cuda).int())
+                if channel:
+                    extra["z"] = cut(z)
+                seq.gated_delta(cut(qkv), cut(bg), gate[: S * rows], norm, 1e-6, state, H, H, D, D, rag, **extra)
+            err[n] += ((state.double() - want).norm() / want.norm()).item() / 12
+    assert err[0] <= err[1] < 2e-7, err
