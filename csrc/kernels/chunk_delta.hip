@@ -104,7 +104,7 @@ __global__ void __launch_bounds__(64 * NC + 2 * D, 1) chunk_delta_kernel(GatedDe
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
   const int q0 = __builtin_amdgcn_readfirstlane(r.cu_q ? r.cu_q[s] : s);
   const int L = __builtin_amdgcn_readfirstlane(r.cu_q ? r.cu_q[s + 1] - q0 : 1);
-  if (L <= 0) return;
+  if (L <= 0 || L < a.cut) return;
   const int nch = (L + CT - 1) / CT;
 
   if (wave >= NC) {
@@ -561,11 +561,16 @@ template <int D> hipError_t launch_d(const GatedDeltaArgs& a, RaggedRows r, hipS
 
 }  // namespace
 
-bool chunk_delta_takes(const GatedDeltaArgs& a, int rows, int num_seqs) {
-  const int d = a.sh.dim, v = a.sh.vdim;
+int chunk_delta_cut(const GatedDeltaArgs& a, int rows, int num_seqs) {
+  const int d = a.sh.dim, v = a.sh.vdim, none = rows + 1;
   // offsets within a chunk are 32-bit
   const bool near = a.gstride < (1 << 26) && a.ostride < (1 << 26) && (a.z == nullptr || a.zstride < (1 << 26));
-  return !a.f32 && near && (d == 64 || d == 128) && (v == 64 || v == 128 || v == 256) && rows >= (v == 64 ? 64 : CT) * num_seqs;
+  if (a.f32 || !near || (d != 64 && d != 128) || (v != 64 && v != 128 && v != 256)) return none;
+  const int64_t wgs = (int64_t)a.sh.heads * num_seqs, cus = num_cus();
+  const bool many = v == 64 ? wgs > 2 * cus : d * v > 128 * 128 ? 2 * wgs > cus : v < 4 * d && wgs > cus;
+  const int64_t from = v == 64 ? 64 : CT, all = !many ? from : v != 64 ? 28 : wgs > 4 * cus ? 256 : 128;
+  if (rows >= all * num_seqs || (v != 64 && rows >= CT * num_seqs && rows < (CT + 1) * num_seqs)) return 0;
+  return rows >= from * num_seqs ? (int)all : none;
 }
 
 hipError_t launch_chunk_delta(const GatedDeltaArgs& a, RaggedRows r, hipStream_t s) {

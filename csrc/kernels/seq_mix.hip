@@ -655,7 +655,7 @@ __global__ void __launch_bounds__(M > 2 && NE == 1 ? 512 : 1024) gated_delta_ker
   const int kh = h / (H / G);
   const int q0 = r.cu_q ? r.cu_q[s] : s;
   const int L = r.cu_q ? r.cu_q[s + 1] - q0 : 1;
-  if (L <= 0) return;
+  if (L <= 0 || L >= a.cut) return;
   const bool fresh = r.positions[q0] <= 0;
   const bool live = j0 < dv;
   float* st = a.state + ((int64_t)r.state_slots[s] * H + h) * d * dv;
@@ -1170,11 +1170,16 @@ template <int LN, int M> static hipError_t launch_gd(const GatedDeltaArgs& a, Ra
   return vec ? launch_gd<LN, M, false, false, true>(a, r, s) : launch_gd<LN, M, false, false, false>(a, r, s);
 }
 
-hipError_t launch_gated_delta(const GatedDeltaArgs& a, RaggedRows r, hipStream_t s) {
+hipError_t launch_gated_delta(const GatedDeltaArgs& args, RaggedRows r, hipStream_t s) {
+  GatedDeltaArgs a = args;
   if (r.num_seqs == 0 || r.total_rows == 0) return hipSuccess;
   if (!delta_ok(a.sh) || !rows_ok(r) || (a.z != nullptr && (a.z_bias == nullptr || a.A_log == nullptr)))
     return hipErrorInvalidValue;
-  if (chunk_delta_takes(a, r.total_rows, r.num_seqs)) return launch_chunk_delta(a, r, s);
+  a.cut = chunk_delta_cut(a, r.total_rows, r.num_seqs);
+  if (a.cut <= r.total_rows) {
+    const hipError_t e = launch_chunk_delta(a, r, s);
+    if (e != hipSuccess || a.cut == 0) return e;
+  }
   if (a.sh.dim <= 16) return launch_gd<4, 1>(a, r, s);
   if (a.sh.dim <= 32) return launch_gd<8, 1>(a, r, s);
   if (a.sh.dim <= 64) return launch_gd<16, 1>(a, r, s);

@@ -141,3 +141,18 @@ def test_state_is_no_further_from_64_bits_than_token_by_token(cuda, channel):
                 seq.gated_delta(cut(qkv), cut(bg), gate[: S * rows], norm, 1e-6, state, H, H, D, D, rag, **extra)
             err[n] += ((state.double() - want).norm() / want.norm()).item() / 12
     assert err[0] <= err[1] < 2e-7, err
+
+
+@pytest.mark.parametrize("channel", [False, True])
+@pytest.mark.parametrize("vdim,short,long", [(128, [1, 9, 27], 28), (64, [64, 1, 127], 128)])
+def test_divided_steps(cuda, vdim, short, long, channel):
+    """A step of so many sequences that it is divided by their lengths: portions on either side of the cut, and none of a length."""
+    torch.manual_seed(vdim)
+    H, D = 8, 64
+    lens = short * 12 + [long, long + 33] * 6 + [short[-1]] * 20   # 68 sequences of 8 heads
+    args, dims = _inputs(H, 4, D, vdim, channel, lens, [3 * (i % 2) for i in range(len(lens))]), (H, 4, D, vdim)
+    assert long * len(lens) > sum(lens) >= (17 if vdim == 128 else 64) * len(lens)
+    want, st = _run(args, dims, "cpu")
+    got, st2 = _run(args, dims, cuda)
+    assert (st2 - st).abs().max() <= 1e-4 * st.abs().max()
+    assert ((got - want).abs() <= 2 ** -7 * want.abs() + 1e-4 * want.abs().max()).all()
