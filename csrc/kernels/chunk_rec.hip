@@ -75,7 +75,7 @@ template <typename T> __device__ __forceinline__ const T* at_bytes(const T* base
   return reinterpret_cast<const T*>(reinterpret_cast<const char*>(base) + off);
 }
 
-// bf16 silu(z) of 8 packed values, rounded to bf16
+// bf16 silu(z) of 8 packed values, rounded to bf16 (to the same bits as with expf, for every bf16 z)
 __device__ __forceinline__ uint4 silu8(uint4 w) {
   float f[8];
   unpack8(w, f);

@@ -87,3 +87,29 @@ def test_later_tokens_do_not_reach_earlier_rows(cuda, what):
     got = run(x, ab)
     assert torch.equal(got[: at + 9], want[: at + 9])
     assert not torch.isfinite(got[at + 9, :vdim]).all()
+
+
+def test_silu_is_that_of_short_portions(cuda):
+    """SiLU of every bf16 value as query, key and value, to the bit as the token-by-token kernel rounds it: with a decay of zero and one
+    channel that is not zero a row's result is one product of three rounded values, exactly."""
+    H, D, V = 4, 32, 128
+    x = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16)
+    x = x[(x.float().abs() < 1e30) & (x.float().abs() > 1e-30)]   # (products that neither overflow nor lose bits)
+    x = torch.cat([x, x])[:65536].to(cuda)
+    small, decay = (x.float() < 200) & (x.float() > -30) & (x.float().abs() > 1e-6), torch.zeros(H, device=cuda)
+
+    def run(qk, v, rows):   # qk [T, H]: channel 0 of q and k
+        T = v.shape[0]
+        row = torch.zeros(T, 2, H, D, dtype=torch.bfloat16, device=cuda)
+        row[..., 0] = qk[:, None]
+        S = T // rows
+        rag = seq.Ragged(torch.arange(rows, device=cuda).repeat(S), (torch.arange(S + 1, device=cuda) * rows).int(), torch.arange(S, device=cuda).int())
+        return lin.lightning_attn(torch.cat([row.view(T, -1), v], 1), 0, H * D, 2 * H * D, decay, torch.zeros(S, H, D, V, device=cuda), H, D, V, rag)
+
+    one = torch.full((65536 // V, H), 20.0, dtype=torch.bfloat16, device=cuda)   # its SiLU is 20
+    v = x.view(-1, V).repeat(1, H)[torch.arange(65536 // V, device=cuda)]
+    qk, unit = torch.where(small, x, 1.0).view(-1, H), torch.full((65536 // H, H * V), 20.0, dtype=torch.bfloat16, device=cuda)
+    for args in ((one, v), (qk, unit)):
+        chunks, tokens = run(*args, 64), run(*args, 4)   # (below 8 rows a sequence: token by token)
+        assert torch.isfinite(tokens).all()
+        assert torch.equal(chunks, tokens), ((chunks != tokens).sum().item(), tokens.numel())
