@@ -114,7 +114,7 @@ __global__ void __launch_bounds__(64 * (NW + 1), 2) chunk_linear_kernel(ChunkLin
   float* tab = reinterpret_cast<float*>(smem + BUF * sizeof(bf16_t)) + wave * 4 * CT;   // the wave's own
   const int q0 = __builtin_amdgcn_readfirstlane(r.cu_q ? r.cu_q[s] : s);
   const int L = __builtin_amdgcn_readfirstlane(r.cu_q ? r.cu_q[s + 1] - q0 : 1);
-  if (L <= 0) return;
+  if (L <= 0 || L < a.cut) return;
   const bool fresh = r.positions[q0] <= 0;
   const int H = a.heads, h0 = blockIdx.x * (NW / NV), g = h0 / (H / a.groups);
   const bool ones = wave == NW;                                  // the normaliser's column block (stages nothing)
@@ -393,11 +393,17 @@ template <int ND> hipError_t launch_silu(const ChunkLinearArgs& a, RaggedRows r,
 
 }  // namespace
 
-bool chunk_linear_takes(const ChunkLinearArgs& a, int rows, int num_seqs) {
+int chunk_linear_cut(const ChunkLinearArgs& a, int rows, int num_seqs) {
   const bool sizes = (a.dim == 32 || a.dim == 64 || a.dim == 128) && (a.vdim == 32 || a.vdim == 64 || a.vdim == 128);
   const bool aligned = a.xstride % 8 == 0 && a.qoff % 8 == 0 && a.koff % 8 == 0 && a.voff % 8 == 0 &&
                        (reinterpret_cast<uintptr_t>(a.x) & 15) == 0 && a.xstride < (1 << 25);   // (a chunk's offsets in 32 bits)
-  return sizes && aligned && rows >= CHUNK_LINEAR_MIN_ROWS * num_seqs;
+  const int64_t n = num_seqs, wgs = a.heads * n, cus = num_cus();
+  const bool norm = a.n_state != nullptr, many = wgs > 2 * cus;
+  const bool one = a.vdim == 32 && (norm || a.heads / a.groups % 4 != 0);   // one wave stages q, k and v (launch_nd)
+  const int64_t state = a.dim * a.vdim;
+  if (!sizes || !aligned || rows < 8 * n || (rows == 8 * n && (many || state < 128 * 128))) return rows + 1;
+  if (!a.silu && ((a.dim == 128 && one && rows < 24 * n) || (a.vdim == 4 * a.dim && many && rows < (norm ? 24 : 12) * n))) return rows + 1;
+  return norm && state > 64 * 64 && wgs * state > 2 * cus * 64 * 128 && rows <= 12 * n ? 13 : 0;
 }
 
 hipError_t launch_chunk_linear(const ChunkLinearArgs& a, RaggedRows r, hipStream_t s) {

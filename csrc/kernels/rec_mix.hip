@@ -444,7 +444,7 @@ __global__ void __launch_bounds__(512) gated_linear_attn_kernel(GatedLinearArgs 
   const int g = h / (H / a.groups);
   const int q0 = r.cu_q ? r.cu_q[s] : s;
   const int L = r.cu_q ? r.cu_q[s + 1] - q0 : 1;
-  if (L <= 0) return;
+  if (L <= 0 || L >= a.cut) return;
   const bool fresh = r.positions[q0] <= 0;
   const bool live = j0 < ncol;
   float* st = a.state + ((int64_t)r.state_slots[s] * H + h) * (int64_t)d * dv + v0;
@@ -894,7 +894,9 @@ hipError_t launch_exp_gate_scan(float* abe, const void* x, int64_t xstride, int 
   return hipGetLastError();
 }
 
-hipError_t launch_gated_linear_attn(const GatedLinearArgs& a, RaggedRows r, hipStream_t s) {
+hipError_t launch_gated_linear_attn(const GatedLinearArgs& args, RaggedRows r, hipStream_t s) {
+  GatedLinearArgs a = args;
+  a.cut = r.total_rows + 1;
   if (r.num_seqs == 0 || r.total_rows == 0) return hipSuccess;
   if (!rows_ok(r) || a.heads < 1 || a.groups < 1 || a.heads % a.groups || a.dim < 1 || a.dim > 256 || a.vdim < 1 ||
       (a.z == nullptr && (a.ab == nullptr || a.abw < 2)) || (a.n_state != nullptr) != (a.nq != nullptr) ||
@@ -906,7 +908,11 @@ hipError_t launch_gated_linear_attn(const GatedLinearArgs& a, RaggedRows r, hipS
     c.qoff = a.qoff, c.koff = a.koff, c.voff = a.voff, c.silu = false, c.ab = a.ab, c.abw = a.abw, c.decay = nullptr;
     c.state = a.state, c.n_state = a.n_state;
     c.heads = a.heads, c.groups = a.groups, c.dim = a.dim, c.vdim = a.vdim, c.qscale = a.qscale;
-    if (chunk_linear_takes(c, r.total_rows, r.num_seqs)) return launch_chunk_linear(c, r, s);
+    a.cut = c.cut = chunk_linear_cut(c, r.total_rows, r.num_seqs);
+    if (c.cut <= r.total_rows) {
+      const hipError_t e = launch_chunk_linear(c, r, s);
+      if (e != hipSuccess || c.cut == 0) return e;
+    }
   }
   if (a.dim <= 16) return launch_gla_dp<4, 1>(a, r, s);
   if (a.dim <= 32) return launch_gla_dp<8, 1>(a, r, s);

@@ -113,3 +113,24 @@ def test_silu_is_that_of_short_portions(cuda):
         chunks, tokens = run(*args, 64), run(*args, 4)   # (below 8 rows a sequence: token by token)
         assert torch.isfinite(tokens).all()
         assert torch.equal(chunks, tokens), ((chunks != tokens).sum().item(), tokens.numel())
+
+
+@pytest.mark.parametrize("dim,vdim", [(64, 128), (128, 128)])
+def test_divided_steps(cuda, dim, vdim):
+    """With a normaliser, so many sequences that the step is divided by their lengths: portions on either side of the cut."""
+    torch.manual_seed(dim)
+    lens, heads = [1] * 20 + [12] * 12 + [13] * 10 + [50] * 8 + [1] * 22, 8
+    T, S = sum(lens), len(lens)
+    assert 8 * S < T <= 12 * S and heads * S > 512
+    cu = torch.tensor([0] + lens).cumsum(0).int()
+    pos = torch.cat([torch.arange(n) + 3 * (i % 2) for i, n in enumerate(lens)])
+    rag = seq.Ragged(pos, cu, torch.randperm(S + 1)[:S].int())
+    x = torch.randn(T, heads * (2 * dim + vdim)).to(torch.bfloat16)
+    ab, state, nst = torch.rand(T, heads, 3), torch.randn(S + 1, heads, dim, vdim), torch.randn(S + 1, heads, dim)
+    gpu = [t.to(cuda) for t in (x, ab, state, nst)]
+    at = (0, heads * dim, 2 * heads * dim)
+    o, nq = rec.gated_linear_attn(x, *at, ab, state, nst, heads, heads, dim, vdim, 0.3, rag)
+    o2, nq2 = rec.gated_linear_attn(gpu[0], *at, *gpu[1:], heads, heads, dim, vdim, 0.3,
+                                    seq.Ragged(*(t.to(cuda) for t in (rag.positions, rag.cu_q, rag.state_slots))))
+    for got, want, name in ((o2, o, "results"), (gpu[2], state, "state"), (nq2, nq, "normaliser read-out"), (gpu[3], nst, "normaliser")):
+        _close(got, want, name)
