@@ -417,10 +417,10 @@ void combine_post_norm(Tensor resid, OptTensor act, Tensor ys, OptTensor pos, Op
                                        cur_stream()));
 }
 
-// out, q_lat [H, T, rank]; q [T, H * qh] whose head h keeps its rotary part at [h * qh + rot_off, + rot_dim)
-void latent_attn(Tensor out, Tensor q_lat, Tensor q, int64_t rot_off, Tensor cache, Tensor block_tables,
-                 OptTensor cu_q, Tensor ctx_lens, Tensor positions, OptTensor sink, int64_t max_q, int64_t window,
-                 double scale, int64_t rot_dim, Tensor inv_freq, int64_t impl) {
+// out, q_lat [H, T, rank]; q [T, H * qh] whose head h keeps its rotary part at [h * qh + rot_off, + rot_dim). Returns the form that ran.
+std::string latent_attn(Tensor out, Tensor q_lat, Tensor q, int64_t rot_off, Tensor cache, Tensor block_tables,
+                        OptTensor cu_q, Tensor ctx_lens, Tensor positions, OptTensor sink, int64_t max_q, int64_t window,
+                        double scale, int64_t rot_dim, Tensor inv_freq, int64_t impl) {
   const bool f = is_f32(q_lat, "q_lat");
   TORCH_CHECK(is_f32(out, "out") == f && is_f32(q, "q") == f && is_f32(cache, "cache") == f, "one dtype");
   TORCH_CHECK(q_lat.dim() == 3 && q_lat.is_contiguous() && out.is_contiguous() && out.sizes() == q_lat.sizes(),
@@ -500,6 +500,7 @@ void latent_attn(Tensor out, Tensor q_lat, Tensor q, int64_t rot_off, Tensor cac
     }
   }
   HIP_OK(die::launch_latent_attn(a, cur_stream()));
+  return die::latent_attn_form(a);
 }
 
 void moe_align(Tensor offsets, Tensor sorted, Tensor pos, Tensor ids, int64_t num_experts) {

@@ -726,11 +726,13 @@ template <int NDB, int NROT> hipError_t launch_mfma_rq(const LatentAttnArgs& a, 
   return hipGetLastError();
 }
 
-// the register-query kernel exists for rank in {64, 128, 256} x rot_dim in {0, 16, 32, 64}; unsplit steps only
+// the register-query kernel exists for rank in {64, 128, 256} x rot_dim in {0, 16, 32, 64}; unsplit steps only. It writes results
+// 16 bytes at a time and passes row numbers between lanes in 32 bits (the other kernel: 8 bytes, 64 bits).
 inline bool mfma_rq_ok(const LatentAttnArgs& a) {
   const int r = a.sh.rank, t = a.sh.rot_dim;
   return a.nsplit <= 1 && (int64_t)a.max_q * a.heads > 32 && (r == 64 || r == 128 || r == 256) &&
-         (t == 0 || t == 16 || t == 32 || t == 64);
+         (t == 0 || t == 16 || t == 32 || t == 64) && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0 &&
+         (int64_t)a.heads * a.total_q < (int64_t(1) << 31);
 }
 
 template <int NDB> hipError_t launch_mfma_rq_rot(const LatentAttnArgs& a, hipStream_t s) {
@@ -798,6 +800,11 @@ template <bool F32> hipError_t launch_bk(const LatentAttnArgs& a, hipStream_t s)
 }  // namespace
 
 bool latent_attn_uses_mfma(const LatentAttnArgs& a) { return a.impl != 1 && mfma_ok(a); }
+
+const char* latent_attn_form(const LatentAttnArgs& a) {
+  if (!latent_attn_uses_mfma(a)) return "fma";
+  return a.impl != 3 && mfma_rq_ok(a) ? "rows" : a.nsplit > 1 ? "split" : "tiles";
+}
 
 hipError_t launch_latent_attn(const LatentAttnArgs& a, hipStream_t s) {
   if (a.num_seqs == 0 || a.total_q == 0) return hipSuccess;

@@ -39,3 +39,28 @@ def test_against_fma(cuda, rank, rot, heads, bs, window, past):
     assert ((got - want).abs() <= (2 ** -9 + 2 * e * 2.71828 ** (2 * e)) * top + 2 ** -7 * want.abs()).all()
     # the bound above is for one key that has it all; over a row the roundings average out
     assert ((got - want).norm() / want.norm()).item() < 2 ** -7
+
+
+def test_results_at_any_8_bytes(cuda):
+    """Results that start at no multiple of 16 bytes go to the kernel that writes 8 at a time: the bits that it writes anywhere."""
+    from src.ops import mix
+
+    torch.manual_seed(3)
+    S, n, heads, rank, rot = 64, 40, 32, 64, 16
+    T, pages = S * n, 3
+    cache = torch.randn(S * pages, 16, rank + rot, device=cuda).to(torch.bfloat16)
+    bt = torch.randperm(S * pages, device=cuda).int().view(S, pages)
+    cu = (torch.arange(S + 1, device=cuda) * n).int()
+    pos, ctx = torch.arange(n, device=cuda).repeat(S), torch.full((S,), n, device=cuda, dtype=torch.int32)
+    q_lat, q = torch.randn(heads, T, rank, device=cuda).to(torch.bfloat16), torch.randn(T, heads * rot, device=cuda).to(torch.bfloat16)
+    room = torch.zeros(heads * T * rank + 8, device=cuda, dtype=torch.bfloat16)
+
+    def at(start, impl):
+        out = room[start:start + heads * T * rank].view(heads, T, rank)
+        form = mix._kern().latent_attn(out, q_lat, q, 0, cache, bt, cu, ctx, pos, None, n, 0, 0.1, rot, ops.rope_inv_freq(1e4, rot, cuda), impl)
+        return form, out.clone()
+
+    form, want = at(0, 3)
+    assert form == "tiles" and at(0, 0)[0] == "rows"
+    form, got = at(4, 0)
+    assert form == "tiles" and torch.equal(got, want)
