@@ -68,6 +68,25 @@ def test_products(cuda, counts, K, ncols, act):
         assert not len(bad), (len(bad), bad[:4].tolist())
 
 
+@pytest.mark.parametrize("act,kind", [(mix.MOE_SILU, mix.ACT_SILU), (mix.MOE_CLAMPED, mix.ACT_CLAMPED), (mix.MOE_GELU, mix.ACT_GELU_TANH)])
+def test_activations_are_those_of_the_separate_pass(cuda, act, kind):
+    """Rows with a single one: the sums are the weights themselves, exactly, and the results those of gated_act on the scaled fp32
+    values, rounded, to the bit (a million values, of which a coarser exponential rounds some dozens to the other neighbour)."""
+    g = torch.Generator().manual_seed(7)
+    n, ncols, K = 8192, 128, 64
+    x = torch.zeros(n, K)
+    at = torch.randint(0, K, (n,), generator=g)
+    x[torch.arange(n), at] = 1.0
+    w = (torch.randn(1, 2 * ncols, K, generator=g) * 3).to(torch.bfloat16)
+    scale = torch.rand(n, generator=g) + 0.5
+    want = mix.gated_act((w[0].float().t()[at] * scale[:, None]).to(cuda), kind, 7.0, 1.702).to(torch.bfloat16)
+    out = torch.empty(n, ncols, dtype=torch.bfloat16, device=cuda)
+    offsets = torch.tensor([0, n], dtype=torch.int32)
+    dev = [t.to(cuda) for t in (x.to(torch.bfloat16), w, offsets)]
+    assert mix._kern().moe_gemm(out, *dev, None, 1, scale.to(cuda), act, 7.0, 1.702)
+    assert torch.equal(out, want), (out != want).sum()
+
+
 def test_extra_groups_are_left_alone(cuda):
     """Rows behind the last expert (identity entries, other ranks' experts) are not written."""
     x, w, offsets, idx, _ = _case((40, 60), 128, 256, False, 1)
