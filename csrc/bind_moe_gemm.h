@@ -7,8 +7,9 @@
 
 // out [rows, ncols] (rows sorted by expert) = act(x[row] W_e^T): returns false, with nothing launched, where the sizes do not tile or
 // the weights are strided views (the library products that the caller has for such cases take any strides).
+// tile_rows: 0, or the rows of a tile (tests).
 inline bool moe_gemm_op(at::Tensor out, at::Tensor x, at::Tensor w, at::Tensor offsets, std::optional<at::Tensor> sorted, int64_t topk,
-                        std::optional<at::Tensor> scale, int64_t act, double limit, double alpha, hipStream_t stream) {
+                        std::optional<at::Tensor> scale, int64_t act, double limit, double alpha, int64_t tile_rows, hipStream_t stream) {
   TORCH_CHECK(x.is_cuda() && x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16 &&
                   out.scalar_type() == at::kBFloat16 && w.is_cuda() && out.is_cuda(),
               "moe_gemm: bf16 device tensors");
@@ -47,6 +48,7 @@ inline bool moe_gemm_op(at::Tensor out, at::Tensor x, at::Tensor w, at::Tensor o
   a.act = (int)act;
   a.limit = (float)limit;
   a.alpha = (float)alpha;
+  a.tile_rows = (int)tile_rows;
   a.experts = (int)w.size(0);
   a.rows = (int)out.size(0);
   a.ncols = (int)out.size(1);

@@ -1037,10 +1037,13 @@ PYBIND11_MODULE(_C, m) {
   m.def("gather_blocks_rows", &gather_blocks_rows);
   m.def("topk_softmax", &topk_softmax);
   m.def("moe_align", &moe_align);
-  m.def("moe_gemm", [](Tensor out, Tensor x, Tensor w, Tensor offsets, std::optional<Tensor> sorted, int64_t topk,
-                       std::optional<Tensor> scale, int64_t act, double limit, double alpha) {
-    return moe_gemm_op(out, x, w, offsets, sorted, topk, scale, act, limit, alpha, cur_stream());
-  });
+  m.def("moe_gemm",
+        [](Tensor out, Tensor x, Tensor w, Tensor offsets, std::optional<Tensor> sorted, int64_t topk, std::optional<Tensor> scale, int64_t act,
+           double limit, double alpha, int64_t tile_rows) {
+          return moe_gemm_op(out, x, w, offsets, sorted, topk, scale, act, limit, alpha, tile_rows, cur_stream());
+        },
+        py::arg("out"), py::arg("x"), py::arg("w"), py::arg("offsets"), py::arg("sorted"), py::arg("topk"), py::arg("scale"),
+        py::arg("act"), py::arg("limit"), py::arg("alpha"), py::arg("tile_rows") = 0);
   m.def("moe_gather", &moe_gather);
   m.def("moe_combine", &moe_combine);
   m.def("gemm_decode", &gemm_decode);

@@ -534,10 +534,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("relu2_act", &relu2_act);
   m.def("route_grouped_topk", &route_grouped_topk);
   m.def("topk_grouped", &topk_grouped);
-  m.def("moe_gemm", [](Tensor out, Tensor x, Tensor w, Tensor offsets, OptTensor sorted, int64_t topk, OptTensor scale,
-                       int64_t act, double limit, double alpha) {
-    return moe_gemm_op(out, x, w, offsets, sorted, topk, scale, act, limit, alpha, cur_stream());
-  });
+  m.def("moe_gemm",
+        [](Tensor out, Tensor x, Tensor w, Tensor offsets, OptTensor sorted, int64_t topk, OptTensor scale, int64_t act,
+           double limit, double alpha, int64_t tile_rows) {
+          return moe_gemm_op(out, x, w, offsets, sorted, topk, scale, act, limit, alpha, tile_rows, cur_stream());
+        },
+        py::arg("out"), py::arg("x"), py::arg("w"), py::arg("offsets"), py::arg("sorted"), py::arg("topk"), py::arg("scale"),
+        py::arg("act"), py::arg("limit"), py::arg("alpha"), py::arg("tile_rows") = 0);
   m.def("rms_norm_ext", &rms_norm_ext);
   m.def("post_norm_residual", &post_norm_residual);
   m.def("gated_act", &gated_act);

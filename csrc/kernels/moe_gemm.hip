@@ -239,7 +239,7 @@ int tile_height(const MoeGemmArgs& a, int cols) {
   return best;
 }
 template <int ACT> hipError_t launch_act(MoeGemmArgs a, hipStream_t s) {
-  a.tile_rows = tile_height(a, ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU ? BN / 2 : BN);
+  if (a.tile_rows == 0) a.tile_rows = tile_height(a, ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU ? BN / 2 : BN);
   return a.tile_rows > 128 ? launch_one<4, 64, 2, ACT>(a, s) : launch_one<2, 32, 3, ACT>(a, s);
 }
 
@@ -256,6 +256,7 @@ bool moe_gemm_takes(const MoeGemmArgs& a) {
 hipError_t launch_moe_gemm(const MoeGemmArgs& a, hipStream_t s) {
   if (a.rows == 0) return hipSuccess;
   if (a.rows < 0 || a.experts < 1 || a.topk < 1 || !moe_gemm_takes(a)) return hipErrorInvalidValue;
+  if (a.tile_rows != 0 && a.tile_rows != 128 && (a.tile_rows < 192 || a.tile_rows > 256 || a.tile_rows % 32 != 0)) return hipErrorInvalidValue;
   switch (a.act) {
     case MOE_ACT_NONE: return launch_act<MOE_ACT_NONE>(a, s);
     case MOE_ACT_SILU: return launch_act<MOE_ACT_SILU>(a, s);

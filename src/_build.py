@@ -61,7 +61,7 @@ def build_kernels(force: bool = False, jobs: int = 8, verbose: bool = False) -> 
     os.makedirs(OBJ, exist_ok=True)
     out = os.path.join(ROOT, "src", "_C" + EXT_SUFFIX)
     kdir = os.path.join(CSRC, "kernels")
-    hdrs = _headers(kdir)
+    hdrs = _headers(kdir) + _headers(CSRC)
     incs, torch_lib, abi = _torch_paths()
     jobs_list = []
     objs = []
@@ -109,7 +109,7 @@ def build_mix(force: bool = False, jobs: int = 8, verbose: bool = False) -> str:
     os.makedirs(odir, exist_ok=True)
     out = os.path.join(ROOT, "src", "_Cmix" + EXT_SUFFIX)
     kdir = os.path.join(CSRC, "kernels")
-    hdrs = _headers(kdir)
+    hdrs = _headers(kdir) + _headers(CSRC)
     incs, torch_lib, abi = _torch_paths()
     jobs_list, objs = [], []
     for k in MIX_KERNELS:

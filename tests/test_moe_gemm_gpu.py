@@ -46,8 +46,8 @@ def _want(x, w, offsets, idx, topk, act, scale, limit, alpha):
     return torch.cat(out)
 
 
-# rows per expert: none, one, around a 32-row piece, around a tile of 128 and of 192 - 256 rows, uneven heights
-COUNTS = [(0, 1, 31, 32), (33, 0, 95, 64), (129, 127, 0, 256), (257, 255, 193, 63), (700, 0, 0, 4)]
+# rows per expert: none, one, around a 32-row piece, around a tile of 128 and of 192 - 256 rows, uneven heights, an odd sum
+COUNTS = [(0, 1, 31, 32), (33, 0, 95, 64), (129, 127, 0, 256), (257, 255, 193, 63), (700, 0, 0, 4), (65, 0, 97, 3)]
 
 
 @pytest.mark.parametrize("counts", COUNTS)
@@ -85,6 +85,21 @@ def test_activations_are_those_of_the_separate_pass(cuda, act, kind):
     dev = [t.to(cuda) for t in (x.to(torch.bfloat16), w, offsets)]
     assert mix._kern().moe_gemm(out, *dev, None, 1, scale.to(cuda), act, 7.0, 1.702)
     assert torch.equal(out, want), (out != want).sum()
+
+
+@pytest.mark.parametrize("height", [128, 192, 224, 256])
+@pytest.mark.parametrize("K,ncols,act", [(64, 256, mix.MOE_NONE), (320, 128, mix.MOE_SILU)])
+def test_every_tile_height(cuda, height, K, ncols, act):
+    """The heights that large steps take, asked for: full tiles, last tiles of one row, around 32 rows and one short of full, several
+    tiles of an expert (two waves share a tile's 32-row pieces: 4 and 4, 4 and 3, 3 and 3, 2 and 2 of them, and all fewer)."""
+    counts = (height, height - 1, 1, 31, 33, height + 1, 2 * height + 33, 3 * height, 95, 161)
+    x, w, offsets, idx, scale = _case(counts, K, ncols, act != mix.MOE_NONE, 1, seed=height)
+    out = torch.full((sum(counts), ncols), 7.0, dtype=torch.bfloat16, device=cuda)
+    dev = [t.to(cuda) for t in (x, w, offsets, idx, scale)]
+    assert mix._kern().moe_gemm(out, *dev[:4], 1, dev[4], act, 1.5, 1.7, height)
+    want = _want(x, w, offsets, idx, 1, act, scale, 1.5, 1.7)
+    tol = 2.0 ** -8 * (want.abs() + want.square().mean(1, keepdim=True).sqrt())
+    assert ((out.cpu().double() - want).abs() <= tol).all()
 
 
 def test_extra_groups_are_left_alone(cuda):
