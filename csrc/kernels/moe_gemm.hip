@@ -11,11 +11,13 @@
 // activation runs on the fp32 accumulators (a wave holds gate and up of the same columns), which takes two passes over
 // [rows, 2 ff] out, and rounds once where the separate passes rounded twice.
 //
-// What bounds it at many rows: the L2's rate into LDS (10.7 TB/s over all CUs; without the matrix instructions the two products of
-// 4096 tokens through 8 experts of 4096 x 14336 take 2.75 of their 3.0 ms), at few the weights' rate from HBM. Both products and
-// their epilogues against one library pair per expert behind a host read of the offsets (us, before -> after): 4096 tokens of
-// that shape 3010 -> 3000, 300 tokens 913 -> 739; 8191 tokens, four of 16 experts of 2048 x 1024, 870 -> 453; 1000 of them 820 -> 97;
-// 2500 tokens, four of 32 experts of 4096 x 2048, 1594 -> 554.
+// What holds it up at many rows is its traffic into LDS (10.7 TB/s over all CUs; without the matrix instructions the two products of
+// 4096 tokens through 8 experts of 4096 x 14336 take 2.75 of their 3.0 ms): no limit of the chip, as 256 x rows are fetched also where
+// a tile holds fewer, and as with one workgroup per CU neither a tile's first stages nor its results pass beside another's products. At
+// few rows it is the weights' rate from HBM. Both products and their epilogues against one library pair per expert behind a host read
+// of the offsets (us, before -> after): 4096 tokens of that shape 2980 -> 2980, 1900 tokens 1628 -> 1340, 300 tokens 913 -> 729; 129 - 255
+// tokens, before by the decode kernel in segments of 128 rows, 767 - 808 -> 680 - 722; 8191 tokens, four of 16 experts of 2048 x 1024,
+// 870 -> 453; 1000 of them 820 -> 97; 2500 tokens, four of 32 experts of 4096 x 2048, 1594 -> 554.
 #include <math.h>
 
 #include "common.h"
@@ -30,6 +32,7 @@ typedef __attribute__((address_space(1))) const void global_cvoid;
 
 constexpr int BN = 256, TN = 2;                   // weight rows of a tile, 32-row W tiles per wave
 constexpr int WN = BN / (32 * TN), NW = 2 * WN;   // waves: 4 along the weight rows, 2 along the x rows
+constexpr int ANY_TALL = 0;                       // tile_rows: 192, 224 or 256, as the kernel finds
 
 // At most VM of the wave's LDS-DMA pieces outstanding and its LDS reads done. (The builtin, which the compiler's own waits take
 // into account: it would wait for all reads before the first use of any.)
@@ -68,9 +71,25 @@ __global__ void __launch_bounds__(64 * NW, MT == 4 ? 2 : 4) moe_gemm_kernel(MoeG
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   // ---- which tile: XCD i (blocks i, i + 8, ...) takes the i-th eighth of the tiles, whose neighbours share weights or x rows
-  const int NT = a.ncols / NO, R = a.tile_rows;
-  int total = 0;
-  for (int e = 0; e < a.experts; ++e) total += (a.offsets[e + 1] - a.offsets[e] + R - 1) / R;
+  const int NT = a.ncols / NO;
+  int R = a.tile_rows, total = 0;
+  if (MT == 4 && R == ANY_TALL) {   // (see tile_height)
+    int n[3] = {};
+    for (int e = 0; e < a.experts; ++e) {
+      const int m = a.offsets[e + 1] - a.offsets[e];
+      n[0] += (m + 191) / 192;
+      n[1] += (m + 223) / 224;
+      n[2] += (m + 255) / 256;
+    }
+    int least = 0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int cost = (n[i] * NT + a.cus - 1) / a.cus * (192 + 32 * i + 512);
+      if (i == 0 || cost < least) least = cost, R = 192 + 32 * i, total = n[i];
+    }
+  } else {
+    for (int e = 0; e < a.experts; ++e) total += (a.offsets[e + 1] - a.offsets[e] + R - 1) / R;
+  }
   total *= NT;
   const int per = (total + 7) / 8, t = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
   if ((int)(blockIdx.x >> 3) >= per || t >= total) return;
@@ -217,30 +236,23 @@ template <int MT, int BK, int NS, int ACT> hipError_t launch_one(const MoeGemmAr
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
   if (e != hipSuccess) return e;
   // at most one tile more per expert than its rows fill; blocks beyond the tiles that there are leave at once
-  const int64_t mts = a.rows / a.tile_rows + (a.experts < a.rows ? a.experts : a.rows);
+  const int64_t mts = a.rows / (a.tile_rows == ANY_TALL ? 192 : a.tile_rows) + (a.experts < a.rows ? a.experts : a.rows);
   const int64_t blocks = (mts * (a.ncols / NO) + 7) / 8 * 8;
   hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(64 * NW), smem, s, a);
   return hipGetLastError();
 }
 // Tile heights. Up to 96 rows per expert two workgroups per CU with tiles of 128 rows (75 rows per expert of 4096 x 14336: 739 us for
-// both products, with tall tiles 794); above, one workgroup per CU, and of 192, 224 and 256 rows the height whose rounds over the
-// CUs cost least, a tile's time being its rows plus what streams its weights. (Both products at 192 / 224 / 256 rows, us: 750 rows
-// per expert of 2048 x 2048 296 / 216 / 225, 1024 of 4096 x 14336 3054 / 3000 / 3088, 2048 of 2048 x 1024 480 / 453 / 471, 250 of
-// 4096 x 14336 1059 / 1056 / 1015.)
-int tile_height(const MoeGemmArgs& a, int cols) {
-  if (a.rows <= 96 * a.experts) return 128;
-  int best = 256;
-  double least = 1e30;
-  for (int h = 256; h >= 192; h -= 32) {
-    const double tiles = ((double)a.rows / (a.experts * h) + 0.5) * a.experts * (a.ncols / cols);
-    const double cost = ceil(tiles / num_cus()) * (h + 64);
-    if (cost < least) best = h, least = cost;
-  }
-  return best;
-}
+// both products, with tall tiles 794); above, one workgroup per CU and tiles of 192, 224 or 256 rows. Which of them depends on how the
+// experts' rows come out, so the kernel chooses from the offsets: the height whose rounds over the CUs cost least, a round being its
+// rows plus what goes with any height (weights, and x rows that are fetched either way). Over 660 steps (11 widths, 100 - 2048 rows per
+// expert: equal, random, skewed) that is within 0.2 % of the best height on average and 3 % at most; chosen from the average rows per
+// expert, with half a tile for the remainders, it was 4.7 % and 78 %. (Both products at 192 / 224 / 256 rows, us: 425 rows per expert
+// of 4096 x 14336 1768 / 1640 / 1276, 750 of 2048 x 2048 296 / 216 / 225, 1500 of 2048 x 1024 399 / 343 / 348.)
+int tile_height(const MoeGemmArgs& a) { return a.rows <= 96 * a.experts ? 128 : ANY_TALL; }
 template <int ACT> hipError_t launch_act(MoeGemmArgs a, hipStream_t s) {
-  if (a.tile_rows == 0) a.tile_rows = tile_height(a, ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU ? BN / 2 : BN);
-  return a.tile_rows > 128 ? launch_one<4, 64, 2, ACT>(a, s) : launch_one<2, 32, 3, ACT>(a, s);
+  if (a.tile_rows == 0) a.tile_rows = tile_height(a);
+  a.cus = num_cus();
+  return a.tile_rows != 128 ? launch_one<4, 64, 2, ACT>(a, s) : launch_one<2, 32, 3, ACT>(a, s);
 }
 
 }  // namespace

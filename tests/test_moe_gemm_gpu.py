@@ -102,6 +102,17 @@ def test_every_tile_height(cuda, height, K, ncols, act):
     assert ((out.cpu().double() - want).abs() <= tol).all()
 
 
+@pytest.mark.parametrize("counts", [(475,) * 4, (1024, 0, 3, 900, 511, 513), (97,) * 3 + (600,), (449, 448, 447, 1)])
+def test_chosen_heights(cuda, counts):
+    """The height that the kernel takes by itself: the same bits as with each of the heights (a row's sums do not depend on its tile)."""
+    x, w, offsets, idx, scale = _case(counts, 128, 1024, True, 1, seed=len(counts))
+    dev = [t.to(cuda) for t in (x, w, offsets, idx)]
+    outs = [torch.full((sum(counts), 1024), 7.0, dtype=torch.bfloat16, device=cuda) for _ in range(4)]
+    for out, height in zip(outs, (0, 192, 224, 256)):
+        assert mix._kern().moe_gemm(out, *dev, 1, scale.to(cuda), mix.MOE_SILU, 0.0, 0.0, height)
+    assert all(torch.equal(outs[0], o) for o in outs[1:])
+
+
 def test_extra_groups_are_left_alone(cuda):
     """Rows behind the last expert (identity entries, other ranks' experts) are not written."""
     x, w, offsets, idx, _ = _case((40, 60), 128, 256, False, 1)
