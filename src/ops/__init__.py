@@ -869,12 +869,12 @@ def moe_apply(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: torch.Ten
         # prompt-sized steps: every expert's rows in two launches, offsets read on the device, rows gathered on the way
         out = torch.empty_like(x)
         kern.moe_combine(out, ys, pos, w)
-        return out if residual is None else residual_add_sumsq(residual, out, ssp)
+        return out
     seg_tiles = _moe_decode_tiles(hdim, inter, MOE_DECODE_MAX_T)
     capturing = torch.cuda.is_current_stream_capturing()
     if (t >= MOE_LIBRARY_MIN_TOKENS or seg_tiles is None) and not capturing:
-        # prefill: the per-expert groups are thousands of rows — hipBLASLt GEMMs per expert at
-        # ~1.5 PF/s; costs one host read of the offsets per layer
+        # widths or strides that the grouped product leaves: hipBLASLt GEMMs per expert; costs one host read of the
+        # offsets per layer
         xs = torch.empty(t * k, hdim, dtype=x.dtype, device=x.device)
         kern.moe_gather(xs, x, sorted_idx, k)
         off = offsets.tolist()
@@ -884,8 +884,8 @@ def moe_apply(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: torch.Ten
                 act = silu_and_mul(torch.nn.functional.linear(xs[a0:a1], w13[ei]))
                 torch.nn.functional.linear(act, w2[ei], out=ys[a0:a1])
     else:
-        # between the decode path and the library path (and under graph capture): the expert-streaming
-        # grouped GEMM with each expert's rows cut into segments of <= 128 (offsets built on the device,
+        # the same below MOE_LIBRARY_MIN_TOKENS and under graph capture: the expert-streaming grouped GEMM
+        # with each expert's rows cut into segments of <= 128 (offsets built on the device,
         # no host read); an expert with r rows streams its weights ceil(r / 128) times
         if seg_tiles is None:
             raise ValueError(f"MoE shapes hidden={hdim} inter={inter} do not tile the grouped decode GEMM "

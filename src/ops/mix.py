@@ -200,15 +200,24 @@ MOE_NONE, MOE_SILU, MOE_CLAMPED, MOE_GELU, MOE_RELU2 = range(5)   # activations 
 _MOE_ACT = {ACT_SILU: MOE_SILU, ACT_CLAMPED: MOE_CLAMPED, ACT_GELU_TANH: MOE_GELU, ACT_RELU2: MOE_RELU2}
 
 
+# Rows per expert and elements of an expert's matrix from which a library GEMM pair per expert, behind a host read of the offsets,
+# is faster than the grouped product (eight experts of 4096 x 14336, us, library / grouped: 1024 rows 3019 / 3005, 1500 rows
+# 3985 / 4177, 2048 rows 5118 / 5600, 4096 rows 9735 / 11003; of 4096 x 2048, 2048 rows 1718 / 1774, 2500 rows 2171 / 2135)
+GROUPED_MAX_ROWS, GROUPED_ANY_ROWS_SIZE = 1280, 1 << 25
+
+
 def grouped_experts(kern, x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, offsets: torch.Tensor, sorted_idx: torch.Tensor,
                     k: int, ys: torch.Tensor, act: int, limit: float = 0.0, alpha: float = 0.0,
                     scale: Optional[torch.Tensor] = None) -> bool:
     """Both products of every expert over its rows, two launches: ys[j] = W2 act(s W13 x[sorted_idx[j] / k]) for the rows j of the
     expert-sorted order, s = scale by (token, slot). The expert offsets stay on the device. False, with nothing done, where the
-    sizes do not tile (bf16, widths in multiples of 256) or the weights are strided views."""
+    sizes do not tile (bf16, widths in multiples of 256), the weights are strided views or the library is faster."""
     if x.dtype != torch.bfloat16 or w2.shape[2] % 64 or ys.shape[1] % 256:
         return False
     if not (w13.is_contiguous() and w2.is_contiguous()) or w2.data_ptr() % 16:
+        return False
+    e, h, f = w2.shape
+    if h * f >= GROUPED_ANY_ROWS_SIZE and ys.shape[0] >= GROUPED_MAX_ROWS * e and not torch.cuda.is_current_stream_capturing():
         return False
     a = torch.empty(ys.shape[0], w2.shape[2], dtype=x.dtype, device=x.device)
     if not kern.moe_gemm(a, x, w13, offsets, sorted_idx, k, scale, act, limit, alpha):
@@ -217,7 +226,9 @@ def grouped_experts(kern, x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, 
 
 
 # (token, expert) rows up to which the experts' weights are gathered per row for two batched GEMMs (no host
-# read, hipGraph-capturable: decode steps); above it each expert runs one library GEMM pair over its rows
+# read, hipGraph-capturable: decode steps of widths that the expert-streaming product does not tile); above it the rows
+# sorted by expert run as one grouped product per matrix, or, in fp32, at widths that it does not tile and with strided
+# weights, one library GEMM pair per expert
 MOE_BMM_MAX_ROWS = 64
 
 

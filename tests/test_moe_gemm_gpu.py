@@ -179,3 +179,27 @@ def test_strided_weights_take_the_library(cuda, stack):
                 lambda a, _, c: ops.moe_apply(x, a, c, w, ids, e)):
         got, want = run(w13, w1, w2).float(), run(off(w13), off(w1), off(w2)).float()
         assert ((got - want).norm() / want.norm()).item() < 2 ** -9   # the library may take another kernel for other strides
+
+
+def test_many_rows_of_large_experts_take_the_library(cuda, monkeypatch):
+    """From GROUPED_MAX_ROWS rows per expert of a large matrix on the library products run (not where a graph is captured, which can't
+    read the offsets): the bits of a call whose weights the grouped product does not take (an unaligned start)."""
+    from src import ops
+
+    monkeypatch.setattr(mix, "GROUPED_ANY_ROWS_SIZE", 256 * 512)
+    monkeypatch.setattr(mix, "GROUPED_MAX_ROWS", 200)
+    g = torch.Generator().manual_seed(9)
+    h, f, e, k, bf = 256, 512, 3, 2, torch.bfloat16
+    w13, w2 = ((torch.randn(*s, generator=g) * 0.05).to(bf).to(cuda) for s in ((e, 2 * f, h), (e, h, f)))
+    off = lambda v: torch.empty(v.numel() + 1, dtype=bf, device=cuda)[1:].view(v.shape).copy_(v)
+    for t in (299, 300):   # one row short of it, there
+        x, w = torch.randn(t, h, generator=g).to(bf).to(cuda), torch.rand(t, k, generator=g).to(cuda)
+        ids = torch.rand(t, e, generator=g).argsort(1)[:, :k].int().to(cuda)
+        got, want = ops.moe_apply(x, w13, w2, w, ids, e), ops.moe_apply(x, off(w13), off(w2), w, ids, e)
+        assert torch.equal(got, want) == (t == 300)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops.moe_apply(x, w13, w2, w, ids, e)
+    for _ in range(3):
+        graph.replay()
+        assert ((out - want).float().norm() / want.float().norm()).item() < 1e-2
