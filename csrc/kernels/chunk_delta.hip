@@ -21,6 +21,9 @@
 // multiplied; the state is rounded once per chunk instead of twice per token. Its error against 64 bits (2-norm; 1 - 16 sequences of
 // 32 - 1400 rows, 12 draws each) is 0.2 - 1.0e-7, 0.90 - 0.93 of that of the token-by-token kernel, decays per head and per channel.
 //
+// An infinite key or value makes the rows from its token on and the state NaN (a part of an infinity is NaN), where token by token some
+// of them may stay infinite; earlier rows and other sequences are as they are.
+//
 // Bound by the issue of vector and matrix instructions of the two waves per SIMD (LDS leaves one workgroup per compute unit):
 // per chunk 700 vector and 150 matrix instructions of a consuming wave beside 900 of a producing one, 11000 cycles. 16 sequences of
 // 300 - 1000 rows, 16 heads, dim = vdim = 128, decays per channel: 914 -> 325 us; one sequence of 1024 rows: 874 -> 310 us.
@@ -105,6 +108,7 @@ __global__ void __launch_bounds__(64 * NC + 2 * D, 1) chunk_delta_kernel(GatedDe
   const int q0 = __builtin_amdgcn_readfirstlane(r.cu_q ? r.cu_q[s] : s);
   const int L = __builtin_amdgcn_readfirstlane(r.cu_q ? r.cu_q[s + 1] - q0 : 1);
   if (L <= 0 || L < a.cut) return;
+  if (a.cut > 0 && !divided(r.cu_q, r.num_seqs, r.total_rows, a.cut, a.longest)) return;
   const int nch = (L + CT - 1) / CT;
 
   if (wave >= NC) {
@@ -561,16 +565,21 @@ template <int D> hipError_t launch_d(const GatedDeltaArgs& a, RaggedRows r, hipS
 
 }  // namespace
 
-int chunk_delta_cut(const GatedDeltaArgs& a, int rows, int num_seqs) {
+void chunk_delta_cut(GatedDeltaArgs& a, int rows, int num_seqs) {
   const int d = a.sh.dim, v = a.sh.vdim, none = rows + 1;
   // offsets within a chunk are 32-bit
   const bool near = a.gstride < (1 << 26) && a.ostride < (1 << 26) && (a.z == nullptr || a.zstride < (1 << 26));
-  if (a.f32 || !near || (d != 64 && d != 128) || (v != 64 && v != 128 && v != 256)) return none;
+  a.cut = none;
+  if (a.f32 || !near || (d != 64 && d != 128) || (v != 64 && v != 128 && v != 256)) return;
   const int64_t wgs = (int64_t)a.sh.heads * num_seqs, cus = num_cus();
-  const bool many = v == 64 ? wgs > 2 * cus : d * v > 128 * 128 ? 2 * wgs > cus : v < 4 * d && wgs > cus;
-  const int64_t from = v == 64 ? 64 : CT, all = !many ? from : v != 64 ? 28 : wgs > 4 * cus ? 256 : 128;
-  if (rows >= all * num_seqs || (v != 64 && rows >= CT * num_seqs && rows < (CT + 1) * num_seqs)) return 0;
-  return rows >= from * num_seqs ? (int)all : none;
+  const bool many = v < 256 && wgs > 2 * cus;
+  const int64_t from = v == 64 ? 64 : CT, all = !many ? from : v == 128 ? 21 : wgs > 4 * cus ? 160 : 96;
+  if (rows >= all * num_seqs || (v != 64 && rows >= CT * num_seqs && rows < (CT + 1) * num_seqs)) {
+    a.cut = 0;
+  } else if (rows >= from * num_seqs) {
+    a.cut = v == 64 ? (int)all : 28;
+    a.longest = (int)(rows * (int64_t)a.sh.heads / (2 * cus)) + 30;
+  }
 }
 
 hipError_t launch_chunk_delta(const GatedDeltaArgs& a, RaggedRows r, hipStream_t s) {

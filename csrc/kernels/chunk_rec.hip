@@ -13,6 +13,9 @@
 // the token-by-token form. Distance from a 64-bit evaluation, 16 x 1024 tokens of the state-space shape: 1.2e-7 (results) and
 // 0.8e-7 (state), the token-by-token kernel 1.4e-7 and 1.1e-7.
 //
+// An infinite value or state makes the rows from its token on and the state NaN (a part of an infinity is NaN), where token by token some
+// of them may stay infinite; earlier rows and other sequences are as they are.
+//
 // What bounds it: the vector ALUs that cut fragments and weigh scores (about 1200 instructions per wave and chunk at dim 128
 // beside 62 matrix instructions), two waves per SIMD at 250 registers. Against the token-by-token kernels (bf16, us, before -> after):
 // 16 x 1024 tokens, 64 heads of 128 x 64 sharing q and k 794 -> 196 (2.3 TB/s of its inputs, results and states), 16 heads of
@@ -115,6 +118,7 @@ __global__ void __launch_bounds__(64 * (NW + 1), 2) chunk_linear_kernel(ChunkLin
   const int q0 = __builtin_amdgcn_readfirstlane(r.cu_q ? r.cu_q[s] : s);
   const int L = __builtin_amdgcn_readfirstlane(r.cu_q ? r.cu_q[s + 1] - q0 : 1);
   if (L <= 0 || L < a.cut) return;
+  if (a.cut > 0 && !divided(r.cu_q, r.num_seqs, r.total_rows, a.cut, a.longest)) return;
   const bool fresh = r.positions[q0] <= 0;
   const int H = a.heads, h0 = blockIdx.x * (NW / NV), g = h0 / (H / a.groups);
   const bool ones = wave == NW;                                  // the normaliser's column block (stages nothing)
@@ -393,7 +397,7 @@ template <int ND> hipError_t launch_silu(const ChunkLinearArgs& a, RaggedRows r,
 
 }  // namespace
 
-int chunk_linear_cut(const ChunkLinearArgs& a, int rows, int num_seqs) {
+void chunk_linear_cut(ChunkLinearArgs& a, int rows, int num_seqs) {
   const bool sizes = (a.dim == 32 || a.dim == 64 || a.dim == 128) && (a.vdim == 32 || a.vdim == 64 || a.vdim == 128);
   const bool aligned = a.xstride % 8 == 0 && a.qoff % 8 == 0 && a.koff % 8 == 0 && a.voff % 8 == 0 &&
                        (reinterpret_cast<uintptr_t>(a.x) & 15) == 0 && a.xstride < (1 << 25);   // (a chunk's offsets in 32 bits)
@@ -401,9 +405,12 @@ int chunk_linear_cut(const ChunkLinearArgs& a, int rows, int num_seqs) {
   const bool norm = a.n_state != nullptr, many = wgs > 2 * cus;
   const bool one = a.vdim == 32 && (norm || a.heads / a.groups % 4 != 0);   // one wave stages q, k and v (launch_nd)
   const int64_t state = a.dim * a.vdim;
-  if (!sizes || !aligned || rows < 8 * n || (rows == 8 * n && (many || state < 128 * 128))) return rows + 1;
-  if (!a.silu && ((a.dim == 128 && one && rows < 24 * n) || (a.vdim == 4 * a.dim && many && rows < (norm ? 24 : 12) * n))) return rows + 1;
-  return norm && state > 64 * 64 && wgs * state > 2 * cus * 64 * 128 && rows <= 12 * n ? 13 : 0;
+  a.cut = rows + 1;
+  if (!sizes || !aligned || rows < 8 * n || (rows == 8 * n && (many || state < 128 * 128))) return;
+  if (!a.silu && ((a.dim == 128 && one && rows < 24 * n) || (a.vdim == 4 * a.dim && many && rows < (norm ? 24 : 12) * n))) return;
+  const int64_t load = wgs * state / (64 * 128);   // in states of 64 x 128
+  a.cut = norm && state > 64 * 64 && load > 3 * cus && rows <= (load > 6 * cus ? 12 : 10) * n ? 13 : 0;
+  a.longest = (int)(rows * (int64_t)a.heads * 5 / (8 * cus)) + 8;
 }
 
 hipError_t launch_chunk_linear(const ChunkLinearArgs& a, RaggedRows r, hipStream_t s) {

@@ -72,6 +72,22 @@ __device__ __forceinline__ float xor16_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Whether a step of n portions (of cu[i + 1] - cu[i] rows, `total` in all) is divided between two kernels, those of `cut` rows and more
+// going to the other one: where one portion has `longest` rows or a quarter of all rows lie in portions of 2 * cut and more. (By whole
+// waves; the same answer in every wave that asks.)
+__device__ __forceinline__ bool divided(const int* cu, int n, int total, int cut, int longest) {
+  bool far = false;
+  int in_long = 0;
+  for (int i = threadIdx.x & 63; i < n; i += 64) {
+    const int rows = cu[i + 1] - cu[i];
+    far = far || rows >= longest;
+    in_long += rows >= 2 * cut ? rows : 0;
+  }
+#pragma unroll
+  for (int m = 1; m < 64; m *= 2) in_long += __shfl_xor(in_long, m, 64);
+  return __ballot(far) != 0 || in_long >= total - 3 * (total / 4);
+}
+
 // f(IntC<0>{}) ... f(IntC<N - 1>{}): a loop unrolled by the front end, so
 // register arrays indexed by the constant are split into VGPRs before any optimisation pass runs
 template <int I> struct IntC {

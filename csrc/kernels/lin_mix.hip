@@ -474,7 +474,7 @@ hipError_t launch_lightning_attn(const LightningArgs& a, RaggedRows r, hipStream
     c.qoff = a.qoff, c.koff = a.koff, c.voff = a.voff, c.silu = true, c.ab = nullptr, c.abw = 0, c.decay = a.decay;
     c.state = a.state, c.n_state = nullptr;
     c.heads = a.heads, c.groups = a.heads, c.dim = a.dim, c.vdim = a.vdim, c.qscale = 1.0f;
-    c.cut = chunk_linear_cut(c, r.total_rows, r.num_seqs);
+    chunk_linear_cut(c, r.total_rows, r.num_seqs);
     if (c.cut == 0) return launch_chunk_linear(c, r, s);   // (steps with a normaliser alone are divided)
   }
   if (a.dim <= 16) return launch_lightning_dp<4>(a, r, s);

@@ -92,7 +92,7 @@ struct GatedLinearArgs {
   float* n_state;          // [slots, H, dim] or nullptr
   int heads, groups, dim, vdim;
   float qscale;
-  int cut = 0;             // set by the launcher: sequences of fewer rows go token by token, the others in chunks
+  int cut = 0, longest = 0;   // set by the launcher: sequences of `cut` rows and more go in chunks, in divided steps (common.h)
 };
 // Per (sequence, head), token by token: S <- a S + b k v^T (with z: row i of S by its own a_i); o = S^T (q * qscale);
 // with n_state also

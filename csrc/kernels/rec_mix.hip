@@ -444,7 +444,8 @@ __global__ void __launch_bounds__(512) gated_linear_attn_kernel(GatedLinearArgs 
   const int g = h / (H / a.groups);
   const int q0 = r.cu_q ? r.cu_q[s] : s;
   const int L = r.cu_q ? r.cu_q[s + 1] - q0 : 1;
-  if (L <= 0 || L >= a.cut) return;
+  if (L <= 0) return;
+  if (!CD && L >= a.cut && divided(r.cu_q, r.num_seqs, r.total_rows, a.cut, a.longest)) return;   // (goes in chunks)
   const bool fresh = r.positions[q0] <= 0;
   const bool live = j0 < ncol;
   float* st = a.state + ((int64_t)r.state_slots[s] * H + h) * (int64_t)d * dv + v0;
@@ -908,7 +909,8 @@ hipError_t launch_gated_linear_attn(const GatedLinearArgs& args, RaggedRows r, h
     c.qoff = a.qoff, c.koff = a.koff, c.voff = a.voff, c.silu = false, c.ab = a.ab, c.abw = a.abw, c.decay = nullptr;
     c.state = a.state, c.n_state = a.n_state;
     c.heads = a.heads, c.groups = a.groups, c.dim = a.dim, c.vdim = a.vdim, c.qscale = a.qscale;
-    a.cut = c.cut = chunk_linear_cut(c, r.total_rows, r.num_seqs);
+    chunk_linear_cut(c, r.total_rows, r.num_seqs);
+    a.cut = c.cut, a.longest = c.longest;
     if (c.cut <= r.total_rows) {
       const hipError_t e = launch_chunk_linear(c, r, s);
       if (e != hipSuccess || c.cut == 0) return e;

@@ -92,7 +92,7 @@ struct GatedDeltaArgs {
   float eps, mult;
   float* state;           // [slots, heads, dim, vdim]
   DeltaShape sh;
-  int cut = 0;            // set by the launcher: sequences of fewer rows go token by token, the others in chunks
+  int cut = 0, longest = 0;   // set by the launcher: sequences of `cut` rows and more go in chunks, in divided steps (common.h)
 };
 // Per (sequence, head), token by token: S <- g S (g per head, or per row of S); u = beta (v - S^T k); S <- S + k u^T;
 // o = S^T q, with S [dim, vdim] fp32. out[t, h, :] = mult * o / rms(o) * norm_w * gate function(gate[t, h, :]).

@@ -655,7 +655,8 @@ __global__ void __launch_bounds__(M > 2 && NE == 1 ? 512 : 1024) gated_delta_ker
   const int kh = h / (H / G);
   const int q0 = r.cu_q ? r.cu_q[s] : s;
   const int L = r.cu_q ? r.cu_q[s + 1] - q0 : 1;
-  if (L <= 0 || L >= a.cut) return;
+  if (L <= 0) return;
+  if (L >= a.cut && divided(r.cu_q, r.num_seqs, r.total_rows, a.cut, a.longest)) return;   // (goes in chunks)
   const bool fresh = r.positions[q0] <= 0;
   const bool live = j0 < dv;
   float* st = a.state + ((int64_t)r.state_slots[s] * H + h) * d * dv;
@@ -1175,7 +1176,7 @@ hipError_t launch_gated_delta(const GatedDeltaArgs& args, RaggedRows r, hipStrea
   if (r.num_seqs == 0 || r.total_rows == 0) return hipSuccess;
   if (!delta_ok(a.sh) || !rows_ok(r) || (a.z != nullptr && (a.z_bias == nullptr || a.A_log == nullptr)))
     return hipErrorInvalidValue;
-  a.cut = chunk_delta_cut(a, r.total_rows, r.num_seqs);
+  chunk_delta_cut(a, r.total_rows, r.num_seqs);
   if (a.cut <= r.total_rows) {
     const hipError_t e = launch_chunk_delta(a, r, s);
     if (e != hipSuccess || a.cut == 0) return e;

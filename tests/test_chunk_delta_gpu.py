@@ -144,14 +144,16 @@ def test_state_is_no_further_from_64_bits_than_token_by_token(cuda, channel):
 
 
 @pytest.mark.parametrize("channel", [False, True])
-@pytest.mark.parametrize("vdim,short,long", [(128, [1, 9, 27], 28), (64, [64, 1, 127], 128)])
-def test_divided_steps(cuda, vdim, short, long, channel):
-    """A step of so many sequences that it is divided by their lengths: portions on either side of the cut, and none of a length."""
+@pytest.mark.parametrize("vdim,short,fill,long", [(128, [1, 9, 27], 20, 28), (64, [64, 1, 95], 70, 96)])
+@pytest.mark.parametrize("more", [33, 0])
+def test_divided_steps(cuda, vdim, short, fill, long, channel, more):
+    """A step of so many sequences that it may be divided by their lengths: portions on either side of the cut, some of them long enough
+    for it or none."""
     torch.manual_seed(vdim)
     H, D = 8, 64
-    lens = short * 12 + [long, long + 33] * 6 + [short[-1]] * 20   # 68 sequences of 8 heads
+    lens = short * 12 + [long, long + more] * 6 + [fill] * 22   # 70 sequences of 8 heads
     args, dims = _inputs(H, 4, D, vdim, channel, lens, [3 * (i % 2) for i in range(len(lens))]), (H, 4, D, vdim)
-    assert long * len(lens) > sum(lens) >= (17 if vdim == 128 else 64) * len(lens)
+    assert (21 if vdim == 128 else 96) * len(lens) > sum(lens) >= (17 if vdim == 128 else 64) * len(lens)
     want, st = _run(args, dims, "cpu")
     got, st2 = _run(args, dims, cuda)
     assert (st2 - st).abs().max() <= 1e-4 * st.abs().max()

@@ -115,13 +115,15 @@ def test_silu_is_that_of_short_portions(cuda):
         assert torch.equal(chunks, tokens), ((chunks != tokens).sum().item(), tokens.numel())
 
 
+# portions on either side of the cut of 13 rows: a quarter of the rows in long ones, a long one alone (both divided), no long ones (not)
+@pytest.mark.parametrize("lens", [[1] * 20 + [12] * 12 + [13] * 10 + [50] * 8 + [1] * 22, [8] * 70 + [13, 90], [8] * 60 + [13] * 6 + [14] * 6])
 @pytest.mark.parametrize("dim,vdim", [(64, 128), (128, 128)])
-def test_divided_steps(cuda, dim, vdim):
-    """With a normaliser, so many sequences that the step is divided by their lengths: portions on either side of the cut."""
+def test_divided_steps(cuda, dim, vdim, lens):
+    """With a normaliser, so many sequences that the step may be divided by their lengths."""
     torch.manual_seed(dim)
-    lens, heads = [1] * 20 + [12] * 12 + [13] * 10 + [50] * 8 + [1] * 22, 8
+    heads = 16
     T, S = sum(lens), len(lens)
-    assert 8 * S < T <= 12 * S and heads * S > 512
+    assert 8 * S < T <= 10 * S and heads * S > 768
     cu = torch.tensor([0] + lens).cumsum(0).int()
     pos = torch.cat([torch.arange(n) + 3 * (i % 2) for i, n in enumerate(lens)])
     rag = seq.Ragged(pos, cu, torch.randperm(S + 1)[:S].int())
