@@ -46,13 +46,6 @@ __device__ __forceinline__ float dpp_ror8(float x) {   // of lane ^ 8
 template <int E> __device__ __forceinline__ float of_quad(float x) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), E * 0x55, 0xf, 0xf, true));
 }
-// n / (1 + e^-g), n = g or 1: the quotient by the reciprocal, corrected by its residual, which is the division's but for rare last
-// bits in half its instructions. Both sides are scaled, as the reciprocal of a divisor beyond 2^126 would be flushed; where e^-g
-// overflows or g is infinite there is no residual, and the quotient is exact without.
-__device__ __forceinline__ float gated(float n, float g) {
-  const float m = n * 0x1p-8f, d = fmaf(expf(-g), 0x1p-8f, 0x1p-8f), r = __builtin_amdgcn_rcpf(d), q = m * r;
-  return fabsf(g) < 88.7f ? fmaf(fmaf(-d, q, m), r, q) : q;
-}
 __device__ __forceinline__ f32x4_t ld4(const float* p) { return *reinterpret_cast<const f32x4_t*>(p); }
 
 // x = h + m + l in bf16 parts, exact (8 bits each, rounded to nearest): pairs of values, packed

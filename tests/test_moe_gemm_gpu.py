@@ -71,7 +71,7 @@ def test_products(cuda, counts, K, ncols, act):
 @pytest.mark.parametrize("act,kind", [(mix.MOE_SILU, mix.ACT_SILU), (mix.MOE_CLAMPED, mix.ACT_CLAMPED), (mix.MOE_GELU, mix.ACT_GELU_TANH)])
 def test_activations_are_those_of_the_separate_pass(cuda, act, kind):
     """Rows with a single one: the sums are the weights themselves, exactly, and the results those of gated_act on the scaled fp32
-    values, rounded, to the bit (a million values, of which a coarser exponential rounds some dozens to the other neighbour)."""
+    values, rounded, to the bf16 value (a million of them, of which a coarser exponential rounds some dozens to the other neighbour)."""
     g = torch.Generator().manual_seed(7)
     n, ncols, K = 8192, 128, 64
     x = torch.zeros(n, K)
