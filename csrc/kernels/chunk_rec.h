@@ -20,7 +20,7 @@ struct ChunkLinearArgs {
   float* n_state;          // [slots, H, dim] or nullptr
   int heads, groups, dim, vdim;
   float qscale;
-  int cut, longest;        // (chunk_linear_cut) cut > 0: sequences of so many rows, in divided steps (common.h)
+  int cut = 0, longest = 0;   // (chunk_linear_cut) cut > 0: sequences of so many rows, in divided steps (common.h)
 };
 
 // Sets cut, the rows from which a sequence of this step goes in chunks: 0 for all of them, more than `rows` for none; in between (with a
