@@ -1,24 +1,28 @@
 // out[j] = act(x[row(j)] W_e^T) over rows sorted by expert, one launch for all experts (gfx950, bf16 in and out, fp32 sums).
 //
-// A workgroup of 8 waves owns a tile of 256 weight rows (gated activations: 128 gate rows and the 128 matching up rows) and BM of
-// one expert's rows; which ones it finds from the offsets on the device, so nothing waits for the host. Both operands stream
-// through a ring of LDS stages, filled by LDS-DMA (global_load_lds, 16 bytes per lane): W rows as they stand, x rows
-// gathered through the sorted order on the way, so there is no gather pass. The LDS image is lane-linear; 16-byte pieces are
-// XOR-ed by row, which makes the 32x32x16 fragment reads (32 rows, one piece per lane) conflict-free.
+// A tile is 256 weight rows (gated activations: 128 gate rows and the 128 matching up rows) by up to 256 of one expert's rows. One
+// workgroup of 8 waves per CU goes from tile to tile; which ones it finds from the offsets on the device, so nothing waits for the host.
+// Both operands stream through LDS, filled by LDS-DMA (global_load_lds, 16 bytes per lane): W rows as they stand, x rows gathered
+// through the sorted order on the way, so there is no gather pass. A unit is the W or the x rows of a stage of 64 K (whole 128-byte
+// lines); five units fit, so that while one stage is read the next and half of the one behind it are on their way, and while a tile's
+// results are formed and stored the first units of the next tile. The LDS image is lane-linear; 16-byte pieces are XOR-ed by row,
+// which makes the 32x32x16 fragment reads (32 rows, one piece per lane) conflict-free.
 //
-// Per stage a wave runs steps of 2 x MT matrix instructions, 16 deep. Fragments are read one step ahead, between the matrix
-// instructions; the stage's one barrier stands before its last step, whose fragments are in registers by then. The
-// activation runs on the fp32 accumulators (a wave holds gate and up of the same columns), which takes two passes over
-// [rows, 2 ff] out, and rounds once where the separate passes rounded twice.
+// The waves are two groups, one wave of each per SIMD, half a stage apart: while one group's 16 matrix instructions run, the other
+// reads its next fragments and issues its fetches, and a barrier exchanges them. (Both waves of a SIMD reading and multiplying at their
+// own pace left the matrix cores waiting for fragments: a stage took 2500 - 2900 cycles, now 2000 - 2500 of 2048.) The activation runs
+// on the fp32 accumulators (a wave holds gate and up of the same columns), which takes two passes over [rows, 2 ff] out, and rounds
+// once where the separate passes rounded twice.
 //
-// What holds it up at many rows is its traffic into LDS (10.7 TB/s over all CUs; without the matrix instructions the two products of
-// 4096 tokens through 8 experts of 4096 x 14336 take 2.75 of their 3.0 ms): no limit of the chip, as 256 x rows are fetched also where
-// a tile holds fewer, and as with one workgroup per CU neither a tile's first stages nor its results pass beside another's products. At
-// few rows it is the weights' rate from HBM. Both products and their epilogues against one library pair per expert behind a host read
-// of the offsets (us, before -> after): 4096 tokens of that shape 2980 -> 2980, 1900 tokens 1628 -> 1340, 300 tokens 913 -> 729; 129 - 255
-// tokens, before by the decode kernel in segments of 128 rows, 767 - 808 -> 680 - 722; 8191 tokens, four of 16 experts of 2048 x 1024,
-// 870 -> 453; 1000 of them 820 -> 97; 2500 tokens, four of 32 experts of 4096 x 2048, 1594 -> 554.
+// What holds it up at many rows: LDS, which per stage reads 192 KB and takes 64 KB in (2048 cycles, as long as the products), and the
+// clock, which the products pull down to 1.6 - 1.8 GHz. (One wave per SIMD with 128 x 128 products reads a third less and ran 4096 x
+// 14336 up to 5 % faster, 2048-wide experts up to 15 % slower, as nothing runs beside its epilogues.) At few rows it is the weights' rate from
+// HBM. Each product alone, before (a barrier per stage, one tile per workgroup) -> now, us: 4096 tokens, two of 8 experts of 4096 x 14336:
+// 1880 -> 1700 and 1050 -> 920; 1000 of them 637 -> 569 and 357 -> 290; 8191 tokens, four of 16 experts of 2048 x 1024: 174 -> 140 and 172 -> 144;
+// 450 of them 38 -> 25 and 26 -> 19; 3000 tokens, four of 32 experts of 4096 x 2048: 252 -> 210 and 290 -> 223.
 #include <math.h>
+
+#include <algorithm>
 
 #include "common.h"
 #include "moe_gemm.h"
@@ -30,21 +34,31 @@ namespace {
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) const void global_cvoid;
 
-constexpr int BN = 256, TN = 2;                   // weight rows of a tile, 32-row W tiles per wave
+constexpr int BN = 256, BM = 256, TN = 2;         // weight rows and x rows of a tile, 32-row W tiles per wave
 constexpr int WN = BN / (32 * TN), NW = 2 * WN;   // waves: 4 along the weight rows, 2 along the x rows
-constexpr int ANY_TALL = 0;                       // tile_rows: 192, 224 or 256, as the kernel finds
+constexpr int BK = 64, ROWB = 2 * BK;             // K of a stage, bytes of a stage's row
+constexpr int UNIT = BN * ROWB, NU = 5;           // a stage's W or x rows in LDS; places of the ring
+constexpr int PC = UNIT / 1024 / NW;              // 1-KiB pieces (8 rows) of a unit per wave
+static_assert(NU * UNIT <= 160 * 1024, "LDS of a compute unit");
 
-// At most VM of the wave's LDS-DMA pieces outstanding and its LDS reads done. (The builtin, which the compiler's own waits take
-// into account: it would wait for all reads before the first use of any.)
-template <int VM> __device__ __forceinline__ void wait_for() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt((VM & 15) | (VM >> 4) << 14 | 7 << 4);
-  asm volatile("" ::: "memory");
+__device__ __forceinline__ void fence() { asm volatile("" ::: "memory"); }
+// at most VM of the wave's LDS-DMA pieces and stores outstanding / its LDS reads done
+template <int VM> __device__ __forceinline__ void wait_vm() {
+  fence();
+  __builtin_amdgcn_s_waitcnt((VM & 15) | (VM >> 4) << 14 | 7 << 4 | 15 << 8);
+  fence();
 }
-template <int VM> __device__ __forceinline__ void wait_barrier() {
-  wait_for<VM>();
+__device__ __forceinline__ void wait_lds() {
+  fence();
+  __builtin_amdgcn_s_waitcnt(15 | 3 << 14 | 7 << 4);
+  fence();
+}
+__device__ __forceinline__ void barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  fence();
   __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
+  fence();
+  __builtin_amdgcn_sched_barrier(0);
 }
 
 // The functions of gated_act, to the same bf16 values. (__expf has twice the largest error and takes, of the 2955 us of 4096 tokens through
@@ -57,203 +71,292 @@ template <int ACT> __device__ __forceinline__ float gate(float g, float u, float
   return gated(g, alpha * g) * (u + 1.0f);
 }
 
-// MT: 32-row x tiles per wave (BM = 64 MT rows per workgroup); BK: K of a stage (32 or 64); NS: stages of the ring
-// (their products, if the expert's rows end there, are left out: a wave's time goes with its share of the tile's 32-row pieces)
-template <int MT, int BK, int NS, int ACT>
-__global__ void __launch_bounds__(64 * NW, MT == 4 ? 2 : 4) moe_gemm_kernel(MoeGemmArgs a) {
+// inclusive sums over the lanes of a wave
+template <int CTRL> __device__ __forceinline__ int from_before(int x) { return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, false); }
+__device__ __forceinline__ int scan64(int x, int lane) {
+  x += from_before<0x111>(x);
+  x += from_before<0x112>(x);
+  x += from_before<0x114>(x);
+  x += from_before<0x118>(x);
+  const int a = __builtin_amdgcn_readlane(x, 15), b = __builtin_amdgcn_readlane(x, 31), c = __builtin_amdgcn_readlane(x, 47);
+  return x + (lane >= 16 ? a : 0) + (lane >= 32 ? b : 0) + (lane >= 48 ? c : 0);
+}
+
+struct Tile {
+  int e, n0, r0, M;   // expert, first output column, first of M rows
+};
+// The tiles of the launch, found from the offsets by every wave (lane i looks at experts i, i + 64, ...). Tiles of an expert are as even
+// as 32-row pieces allow, at most R rows. XCD i (blocks i, i + 8, ...) takes the i-th eighth of the list, whose neighbours share
+// weights or x rows; its CUs take turns. What is left for less than a turn of all of them is cut into `parts` by rows.
+//
+// R and parts are those that cost least. A tile's time goes with 128 + its rows (2048 K, all CUs busy: 256 rows 66 us, 192 46, 128 36,
+// 64 26); of the whole, 0.7 go with the turns of the CU that has most and 0.3 with the mean of all, as CUs that rest leave the others a
+// higher clock. Over 43 products (200 - 16000 tokens of 5 expert sizes, random routing) that is within 1.8 % of the best R and parts on average;
+// the same R without parts 4.9 %, 256 rows without parts 14 %. (Candidates are weighed by a lane each: one after the other they took 5 us.)
+struct Plan {
+  int R = 0, per = 0, count = 0, full = 0, parts = 1;   // count: tiles of the own XCD
+  int NT, cpx;
+  const MoeGemmArgs& a;
+  int lane;
+  __device__ __forceinline__ Plan(const MoeGemmArgs& args, int nt, int lane_) : NT(nt), a(args), lane(lane_) {
+    constexpr int NH = 5;   // heights 256, 224, .. 128: lanes 4 i + log2(parts)
+    int n = 1, filled = 0;  // tiles of the lane's height; rows in whole 32-row pieces
+    for (int b = 0; b < a.experts; b += 64) {
+      const int m = a.offsets[min(b + lane + 1, a.experts)] - a.offsets[min(b + lane, a.experts)];
+      filled += 32 * __builtin_amdgcn_readlane(scan64((m + 31) / 32, lane), 63);
+#pragma unroll
+      for (int i = 0; i < NH; ++i) {
+        const int k = __builtin_amdgcn_readlane(scan64((m + 255 - 32 * i) / (256 - 32 * i), lane), 63);
+        n = lane / 4 == i ? (b == 0 ? k : n + k) : n;
+      }
+    }
+    cpx = max(a.cus / 8, 1);
+    const int h = 256 - 32 * min(lane / 4, NH - 1), c = 1 << (lane & 3), p = (n * NT + 7) / 8, turns = p / cpx, rem = p - turns * cpx;
+    const float mean = (float)filled / (float)n, whole = 128.f + mean, cut = 128.f + fmaxf(mean / (float)c, 32.f);
+    float cost = 0.7f * ((float)turns * whole + (float)((rem * c + cpx - 1) / cpx) * cut) +
+                 0.3f * ((float)turns * whole + (float)(rem * c) / (float)cpx * cut);
+    const bool out = lane >= 4 * NH || (lane & 3) == 3 || (a.tile_rows != 0 && (a.tile_rows != h || c > 1));
+    cost = out ? __builtin_inff() : cost;
+    float least = cost;
+#pragma unroll
+    for (int d = 1; d < 32; d *= 2) least = fminf(least, __shfl_xor(least, d, 64));
+    const int best = __builtin_amdgcn_readfirstlane(__builtin_ctzll(__builtin_amdgcn_ballot_w64(cost == least) | 1ull << 63));
+    R = __builtin_amdgcn_readlane(h, best);
+    parts = __builtin_amdgcn_readlane(c, best);
+    per = __builtin_amdgcn_readlane(p, best);
+    const int total = __builtin_amdgcn_readlane(n * NT, best);
+    full = per / cpx * cpx;
+    count = min(max(total - (int)(blockIdx.x & 7) * per, 0), per);
+  }
+  // the block's first job from job j on
+  __device__ __forceinline__ bool find(int& j, Tile& t) const {
+    for (;; j += cpx) {
+      if (j >= min(full, count) + max(count - full, 0) * parts) return false;
+      int tile = (int)(blockIdx.x & 7) * per + j, part = 0, cut = 1;
+      if (j >= full) {
+        tile += (j - full) / parts - (j - full);
+        part = (j - full) % parts;
+        cut = parts;
+      }
+      int o0, o1, before, b = 0;
+      uint64_t beyond;
+      for (;; b += 64) {
+        o0 = a.offsets[min(b + lane, a.experts)], o1 = a.offsets[min(b + lane + 1, a.experts)];
+        const int own = (o1 - o0 + R - 1) / R * NT, upto = scan64(own, lane);
+        beyond = __builtin_amdgcn_ballot_w64(upto > tile);
+        before = upto - own;
+        if (beyond != 0 || b + 64 >= a.experts) break;
+        tile -= __builtin_amdgcn_readlane(upto, 63);
+      }
+      if (beyond == 0) return false;
+      const int l = __builtin_ctzll(beyond);
+      tile -= __builtin_amdgcn_readlane(before, l);
+      t.e = b + l;
+      t.r0 = __builtin_amdgcn_readlane(o0, l);
+      t.M = __builtin_amdgcn_readlane(o1, l) - t.r0;
+      // up to 8 x tiles go over all weight tiles together, so that an XCD's CUs share both
+      const int mts = (t.M + R - 1) / R, rows = ((t.M + mts - 1) / mts + 31) / 32 * 32;
+      const int groups = (mts + 7) / 8, gs = (mts + groups - 1) / groups, g = tile / (gs * NT), gm = min(gs, mts - g * gs);
+      tile -= g * gs * NT;
+      const int h = (rows / 32 + cut - 1) / cut * 32, m0 = (g * gs + tile % gm) * rows + part * h;
+      t.n0 = tile / gm;
+      t.M = min(min(t.M - m0, rows - part * h), h);
+      t.r0 += m0;
+      if (t.M > 0) return true;
+    }
+  }
+};
+
+template <int ACT>
+__global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
-  constexpr int BM = 64 * MT;
   constexpr bool GATED = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU;
   constexpr int NO = GATED ? BN / 2 : BN;           // output columns of a tile
-  constexpr int ROWB = 2 * BK, CPR = BK / 8, RPP = 64 / CPR;        // bytes and 16-byte chunks of a stage's row, rows per 1-KiB piece
-  constexpr int STAGE = (BN + BM) * ROWB, PW = BN / RPP / NW, PX = BM / RPP / NW, PER = PW + PX;   // pieces per wave and stage
-  constexpr int SUB = BK / 16;                                      // steps of one matrix instruction's depth
-  static_assert(PW * NW * RPP == BN && PX * NW * RPP == BM, "whole pieces per wave");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-
-  // ---- which tile: XCD i (blocks i, i + 8, ...) takes the i-th eighth of the tiles, whose neighbours share weights or x rows
-  const int NT = a.ncols / NO;
-  int R = a.tile_rows, total = 0;
-  if (MT == 4 && R == ANY_TALL) {   // (see tile_height)
-    int n[3] = {};
-    for (int e = 0; e < a.experts; ++e) {
-      const int m = a.offsets[e + 1] - a.offsets[e];
-      n[0] += (m + 191) / 192;
-      n[1] += (m + 223) / 224;
-      n[2] += (m + 255) / 256;
-    }
-    int least = 0;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      const int cost = (n[i] * NT + a.cus - 1) / a.cus * (192 + 32 * i + 512);
-      if (i == 0 || cost < least) least = cost, R = 192 + 32 * i, total = n[i];
-    }
-  } else {
-    for (int e = 0; e < a.experts; ++e) total += (a.offsets[e + 1] - a.offsets[e] + R - 1) / R;
-  }
-  total *= NT;
-  const int per = (total + 7) / 8, t = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-  if ((int)(blockIdx.x >> 3) >= per || t >= total) return;
-  int e = 0, r0 = 0, M = 0, tile = t;
-  for (;; ++e) {
-    r0 = a.offsets[e];
-    M = a.offsets[e + 1] - r0;
-    const int n = (M + R - 1) / R * NT;
-    if (tile < n) break;
-    tile -= n;
-  }
-  const int mts = (M + R - 1) / R, rows = ((M + mts - 1) / mts + 31) / 32 * 32;     // tiles of even heights
-  const int n0 = tile / mts * NO, m0 = tile % mts * rows;                           // x tiles of one weight tile side by side
-  r0 += m0;
-  M = min(M - m0, rows);
-
-  // ---- the wave's pieces: RPP rows each, chunk c of row r at place c ^ swz(r)
-  auto swz = [](int r) { return BK == 64 ? r >> 1 & 7 : r >> 2 & 3; };
-  const char* wbase = reinterpret_cast<const char*>(a.w) + (int64_t)e * (GATED ? 2 : 1) * a.ncols * a.K * 2;
-  const char* xbase = reinterpret_cast<const char*>(a.x);
-  uint32_t off[PER];
-#pragma unroll
-  for (int p = 0; p < PER; ++p) {
-    const int r = RPP * (wave + NW * (p < PW ? p : p - PW)) + lane / CPR;   // row of the W or the x part
-    const int col = 16 * (lane % CPR ^ swz(r));
-    if (p < PW) {   // 32 TN rows per wave column: with a gate the gate rows, then the matching up rows
-      const int wr = GATED ? (r & 16 * TN ? a.ncols : 0) + n0 + r / (32 * TN) * (16 * TN) + r % (16 * TN) : n0 + r;
-      off[p] = (uint32_t)wr * (uint32_t)(a.K * 2) + col;
-    } else {
-      const int j = r0 + min(r, M - 1);
-      off[p] = (uint32_t)(a.sorted != nullptr ? a.sorted[j] / a.topk : j) * (uint32_t)(a.ldx * 2) + col;
-    }
-  }
-  const int nst = a.K / BK;
-  auto issue = [&](int s) {
-    char* st = smem + s % NS * STAGE;
-    const int64_t k = (int64_t)min(s, nst - 1) * ROWB;
-#pragma unroll
-    for (int p = 0; p < PER; ++p) {
-      const char* src = (p < PW ? wbase : xbase) + k + off[p];
-      char* to = st + (p < PW ? wave + NW * p : BN / RPP + wave + NW * (p - PW)) * 1024;
-      __builtin_amdgcn_global_load_lds((global_cvoid*)src, (lds_void*)to, 16, 0, 0);
-    }
-  };
-
   const int wn = wave % WN, wm = wave / WN, fr = lane & 31, hi = lane >> 5;
-  // a fragment of step kk: 32 rows from `row`, chunk 2 kk + hi of each
-  auto load = [&](int s, int kk, int row) {
-    const char* p = smem + s % NS * STAGE + (row + fr) * ROWB + 16 * ((2 * kk + hi) ^ swz(fr));
-    return __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(p));
-  };
-  f32x16_t acc[TN][MT] = {};
+  const int nst = a.K / BK;
+
+  const Plan plan(a, a.ncols / NO, lane);
+  int job = (int)(blockIdx.x >> 3);
+  Tile t, next;
+  if (!plan.find(job, t)) return;
+
+  // ---- the wave's pieces of a unit: 8 rows each, 16-byte chunk c of row r at place c ^ swz(r)
+  auto swz = [](int r) { return r >> 1 & 7; };
+  const char *wbase, *xbase = reinterpret_cast<const char*>(a.x);
+  uint32_t woff[PC], xoff[PC];
+  int xr[PC];
+  auto rows_of = [&](const Tile& u) {   // the x rows of the wave's pieces
 #pragma unroll
-  for (int p = 0; p < NS; ++p) issue(p);
-  // (past the last stage the last one is fetched again, into a place that nothing reads any more: no branch stands between the
-  // fragments' reads and their use, so every wait is for what is needed only)
-  auto run = [&](auto count) {
-    constexpr int MC = decltype(count)::value, MX = MC > 0 ? MC : 1, NF = MC > 0 ? TN + MC : 0;
-    bf16x8_t wf[2][TN], xf[2][MX];   // [parity of the step][tile]
-    auto frag = [&](int s, int kk, int i) {   // those of W, then the x tiles
-      if (i < TN)
-        wf[kk & 1][i] = load(s, kk, 32 * (TN * wn + i));
-      else
-        xf[kk & 1][i - TN] = load(s, kk, BN + 32 * (2 * (i - TN) + wm));
-    };
-    // The products of step kk. The next step's fragments (stage s, step next; next < 0: none) are read behind the first two pairs, so
-    // that their latency passes under the rest, and `then` follows the third.
-    auto step = [&](int kk, int s, int next, auto&& then) {
-      static_for<MX>([&](auto mi) {
-        constexpr int m = decltype(mi)::value;
-        if constexpr (m < MC) {
+    for (int p = 0; p < PC; ++p) xr[p] = u.r0 + min(8 * (wave + NW * p) + lane / 8, u.M - 1);
+    if (a.sorted != nullptr) {
 #pragma unroll
-          for (int n = 0; n < TN; ++n)
-            acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[kk & 1][n], xf[kk & 1][m], acc[n][m], 0, 0, 0);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        if (next >= 0) {
-#pragma unroll
-          for (int i = 0; i < NF; ++i)
-            if (m == (MX > 1 && i >= (NF + 1) / 2 ? 1 : 0)) frag(s, next, i);
-        }
-        if constexpr (m == (MX > 2 ? 2 : MX - 1)) then();
-        __builtin_amdgcn_sched_barrier(0);
-      });
-    };
-    wait_barrier<(NS - 1) * PER>();
-#pragma unroll
-    for (int i = 0; i < NF; ++i) frag(0, 0, i);
-#pragma unroll 1
-    for (int s = 0; s + 1 < nst; ++s) {
-      static_for<SUB - 1>([&](auto ki) {
-        wait_for<63>();   // the step's fragments, read during the last one's products
-        step(decltype(ki)::value, s, decltype(ki)::value + 1, [] {});
-      });
-      // stage s + 1 has landed when only the stages behind it are outstanding; behind the barrier every wave has read all of stage s,
-      // whose place in the ring stage s + NS takes
-      wait_barrier<(NS - 2) * PER>();
-      step(SUB - 1, s + 1, 0, [&] { issue(s + NS); });
+      for (int p = 0; p < PC; ++p) xr[p] = a.sorted[xr[p]];
     }
-    static_for<SUB>([&](auto ki) {
-      constexpr int kk = decltype(ki)::value;
-      wait_for<63>();
-      step(kk, nst - 1, kk + 1 < SUB ? kk + 1 : -1, [] {});
-    });
   };
-  const int mc = ((M + 31) / 32 + 1 - wm) / 2;   // the wave's 32-row pieces of x: wm, wm + 2, ...
-  if constexpr (MT == 4) {
-    if (mc == 4) run(IntC<4>{});
-    if (mc == 3) run(IntC<3>{});
-  }
-  if (mc == 2) run(IntC<2>{});
-  if (mc == 1) run(IntC<1>{});
-  if (mc == 0) run(IntC<0>{});
-  wait_for<0>();   // no LDS-DMA outlives the workgroup
+  auto offsets_of = [&](const Tile& u) {
+    wbase = reinterpret_cast<const char*>(a.w) + (int64_t)u.e * (GATED ? 2 : 1) * a.ncols * a.K * 2;
+#pragma unroll
+    for (int p = 0; p < PC; ++p) {
+      const int r = 8 * (wave + NW * p) + lane / 8, col = 16 * (lane % 8 ^ swz(r));
+      // 32 TN rows per wave column: with a gate the gate rows, then the matching up rows
+      const int wr = GATED ? (r & 16 * TN ? a.ncols : 0) + u.n0 * NO + r / (32 * TN) * (16 * TN) + r % (16 * TN) : u.n0 * NO + r;
+      woff[p] = (uint32_t)wr * (uint32_t)(a.K * 2) + col;
+      const uint32_t row = a.sorted != nullptr && a.topk > 1 ? (uint32_t)xr[p] / (uint32_t)a.topk : (uint32_t)xr[p];
+      xoff[p] = row * (uint32_t)(a.ldx * 2) + col;
+    }
+  };
+  auto issue_w = [&](int s, int slot) {
+#pragma unroll
+    for (int p = 0; p < PC; ++p)
+      __builtin_amdgcn_global_load_lds((global_cvoid*)(wbase + (int64_t)s * ROWB + woff[p]),
+                                       (lds_void*)(smem + slot * UNIT + (wave + NW * p) * 1024), 16, 0, 0);
+  };
+  auto issue_x = [&](int s, int slot, int pieces) {
+#pragma unroll
+    for (int p = 0; p < PC; ++p)
+      if (p < pieces)
+        __builtin_amdgcn_global_load_lds((global_cvoid*)(xbase + (int64_t)s * ROWB + xoff[p]),
+                                         (lds_void*)(smem + slot * UNIT + (wave + NW * p) * 1024), 16, 0, 0);
+  };
+  auto begin = [&](const Tile& u) {   // the first units of a tile, into places 0, 1, 2
+    offsets_of(u);
+    issue_w(0, 0);
+    issue_x(0, 1, (u.M + 63) / 64);
+    if (nst > 1) issue_w(1, 2);
+  };
+  int lo[BK / 16];   // a fragment of 32 rows: the lane's place at step kk
+#pragma unroll
+  for (int kk = 0; kk < BK / 16; ++kk) lo[kk] = fr * ROWB + 16 * ((2 * kk + hi) ^ swz(fr));
 
-  // ---- results: x row in the lane, weight rows 8 g + 4 hi + 0 .. 3 of a 32-row tile in the registers
+  rows_of(t);
+  begin(t);
+  for (;;) {
+    job += plan.cpx;
+    const bool more = plan.find(job, next);
+    if (more) rows_of(next);
+    const int nx = (t.M + 63) / 64, mc = ((t.M + 31) / 32 + 1 - wm) / 2;   // 64-row pieces of x that are fetched; the wave's 32-row pieces
+    auto run = [&](auto mc_) {
+    constexpr int MC = decltype(mc_)::value, MX = MC > 0 ? MC : 1;
+    f32x16_t acc[TN][MX] = {};
+    bf16x8_t wf[2][TN], xf[2][MX];
+    auto products = [&] {
+      __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    const int row = 32 * (2 * m + wm) + fr;
-    const float sc = a.scale != nullptr ? a.scale[a.sorted != nullptr ? a.sorted[r0 + min(row, M - 1)] : r0 + min(row, M - 1)] : 1.0f;
-    uint16_t* op = a.out + (int64_t)(r0 + row) * a.ncols + n0 + (GATED ? 16 : 32) * TN * wn + 4 * hi;
+      for (int k = 0; k < 2; ++k)
 #pragma unroll
-    for (int n = 0; n < (GATED ? TN / 2 : TN); ++n)
+        for (int m = 0; m < MC; ++m)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        float y[4];
+          for (int n = 0; n < TN; ++n) acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[k][n], xf[k][m], acc[n][m], 0, 0, 0);
+      __builtin_amdgcn_s_setprio(0);
+    };
+      auto load = [&](int ws, int xs, auto half) {   // fragments of half a stage
+        const char* wp = smem + ws * UNIT + 32 * TN * wn * ROWB;
+        const char* xp = smem + xs * UNIT + 32 * wm * ROWB;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if constexpr (GATED)
-            y[i] = gate<ACT>(acc[n][m][4 * g + i] * sc, acc[TN / 2 + n][m][4 * g + i] * sc, a.limit, a.alpha);
-          else
-            y[i] = acc[n][m][4 * g + i] * sc;
-          if constexpr (ACT == MOE_ACT_RELU2) y[i] = fmaxf(y[i], 0.f) * fmaxf(y[i], 0.f);
+        for (int k = 0; k < 2; ++k) {
+          const int l = lo[2 * decltype(half)::value + k];
+#pragma unroll
+          for (int n = 0; n < TN; ++n) wf[k][n] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(wp + 32 * n * ROWB + l));
+#pragma unroll
+          for (int m = 0; m < MC; ++m)
+            xf[k][m] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(xp + 64 * m * ROWB + l));
         }
-        if (row < M) *reinterpret_cast<uint2*>(op + 32 * n + 8 * g) = make_uint2(pack2(y[0], y[1]), pack2(y[2], y[3]));
+      };
+      wait_vm<0>();
+      barrier();
+      if (wm == 1) barrier();
+      int ws = 0, xs = 1;
+#pragma unroll 1
+      for (int s = 1; s < nst; ++s) {   // stage s - 1
+        int sx = xs + 2, sw = ws + 4;   // places of x(s), W(s + 1): those that stage s - 2 has left
+        sx = sx >= NU ? sx - NU : sx;
+        sw = sw >= NU ? sw - NU : sw;
+        load(ws, xs, IntC<0>{});
+        issue_x(s, sx, nx);
+        wait_lds();
+        barrier();
+        products();
+        barrier();
+        load(ws, xs, IntC<1>{});
+        const bool ahead = s + 1 < nst;
+        if (ahead) issue_w(s + 1, sw);
+        if (wm == 1) {   // stage s is there
+          if (ahead) wait_vm<PC>(); else wait_vm<0>();
+        }
+        wait_lds();
+        barrier();
+        products();
+        if (wm == 0) {
+          if (ahead) wait_vm<PC>(); else wait_vm<0>();
+        }
+        barrier();
+        ws += 2;
+        ws = ws >= NU ? ws - NU : ws;
+        xs = sx;
       }
+      load(ws, xs, IntC<0>{});
+      wait_lds();
+      barrier();
+      products();
+      barrier();
+      load(ws, xs, IntC<1>{});
+      wait_lds();
+      barrier();
+      if (wm == 1 && more) begin(next);   // (no wave reads this tile's units any more)
+      products();
+      barrier();
+      if (wm == 0 && more) begin(next);
+
+    // ---- results: x row in the lane, weight rows 8 g + 4 hi + 0 .. 3 of a 32-row tile in the registers; lanes 32 apart exchange
+    // halves of neighbouring g, so that each stores 8 columns
+#pragma unroll
+    for (int m = 0; m < MC; ++m) {
+      const int row = 32 * (2 * m + wm) + fr, rr = t.r0 + min(row, t.M - 1);
+      const float sc = a.scale != nullptr ? a.scale[a.sorted != nullptr ? a.sorted[rr] : rr] : 1.0f;
+      uint16_t* op = a.out + (int64_t)rr * a.ncols + t.n0 * NO + (GATED ? 16 : 32) * TN * wn + 8 * hi;
+#pragma unroll
+      for (int n = 0; n < (GATED ? TN / 2 : TN); ++n)
+#pragma unroll
+        for (int g = 0; g < 4; g += 2) {
+          uint32_t p[2][2];
+#pragma unroll
+          for (int q = 0; q < 2; ++q) {
+            float y[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              if constexpr (GATED)
+                y[i] = gate<ACT>(acc[n][m][4 * (g + q) + i] * sc, acc[TN / 2 + n][m][4 * (g + q) + i] * sc, a.limit, a.alpha);
+              else
+                y[i] = acc[n][m][4 * (g + q) + i] * sc;
+              if constexpr (ACT == MOE_ACT_RELU2) y[i] = fmaxf(y[i], 0.f) * fmaxf(y[i], 0.f);
+            }
+            p[q][0] = pack2(y[0], y[1]), p[q][1] = pack2(y[2], y[3]);
+          }
+          const auto u = __builtin_amdgcn_permlane32_swap(p[0][0], p[1][0], false, false);
+          const auto v = __builtin_amdgcn_permlane32_swap(p[0][1], p[1][1], false, false);
+          if (row < t.M) *reinterpret_cast<uint4*>(op + 32 * n + 8 * g) = make_uint4(u[0], v[0], u[1], v[1]);
+        }
+    }
+    };
+    if (mc == 4) run(IntC<4>{});
+    else if (mc == 3) run(IntC<3>{});
+    else if (mc == 2) run(IntC<2>{});
+    else if (mc == 1) run(IntC<1>{});
+    else run(IntC<0>{});
+    if (wm == 0) barrier();   // (the second waves' last products)
+    if (!more) return;
+    t = next;
   }
 }
 
-template <int MT, int BK, int NS, int ACT> hipError_t launch_one(const MoeGemmArgs& a, hipStream_t s) {
-  constexpr int BM = 64 * MT, NO = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU ? BN / 2 : BN;
-  constexpr size_t smem = (size_t)NS * (BN + BM) * 2 * BK;
-  auto* fn = moe_gemm_kernel<MT, BK, NS, ACT>;
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-  if (e != hipSuccess) return e;
-  // at most one tile more per expert than its rows fill; blocks beyond the tiles that there are leave at once
-  const int64_t mts = a.rows / (a.tile_rows == ANY_TALL ? 192 : a.tile_rows) + (a.experts < a.rows ? a.experts : a.rows);
-  const int64_t blocks = (mts * (a.ncols / NO) + 7) / 8 * 8;
-  hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(64 * NW), smem, s, a);
-  return hipGetLastError();
-}
-// Tile heights. Up to 96 rows per expert two workgroups per CU with tiles of 128 rows (75 rows per expert of 4096 x 14336: 739 us for
-// both products, with tall tiles 794); above, one workgroup per CU and tiles of 192, 224 or 256 rows. Which of them depends on how the
-// experts' rows come out, so the kernel chooses from the offsets: the height whose rounds over the CUs cost least, a round being its
-// rows plus what goes with any height (weights, and x rows that are fetched either way). Over 660 steps (11 widths, 100 - 2048 rows per
-// expert: equal, random, skewed) that is within 0.2 % of the best height on average and 3 % at most; chosen from the average rows per
-// expert, with half a tile for the remainders, it was 4.7 % and 78 %. (Both products at 192 / 224 / 256 rows, us: 425 rows per expert
-// of 4096 x 14336 1768 / 1640 / 1276, 750 of 2048 x 2048 296 / 216 / 225, 1500 of 2048 x 1024 399 / 343 / 348.)
-int tile_height(const MoeGemmArgs& a) { return a.rows <= 96 * a.experts ? 128 : ANY_TALL; }
 template <int ACT> hipError_t launch_act(MoeGemmArgs a, hipStream_t s) {
-  if (a.tile_rows == 0) a.tile_rows = tile_height(a);
+  auto* fn = moe_gemm_kernel<ACT>;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, NU * UNIT);
+  if (e != hipSuccess) return e;
   a.cus = num_cus();
-  return a.tile_rows != 128 ? launch_one<4, 64, 2, ACT>(a, s) : launch_one<2, 32, 3, ACT>(a, s);
+  hipLaunchKernelGGL(fn, dim3(8 * std::max(a.cus / 8, 1)), dim3(64 * NW), NU * UNIT, s, a);
+  return hipGetLastError();
 }
 
 }  // namespace

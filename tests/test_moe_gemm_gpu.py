@@ -113,6 +113,22 @@ def test_chosen_heights(cuda, counts):
     assert all(torch.equal(outs[0], o) for o in outs[1:])
 
 
+@pytest.mark.parametrize("counts,K,ncols,act", [
+    ((2300, 40, 0, 1900), 64, 512, mix.MOE_NONE),              # more than 8 tiles of an expert share a weight tile
+    ((5, 0, 64) * 30, 128, 256, mix.MOE_RELU2),                # more experts than lanes, no full turn of the compute units
+    ((300,) * 16, 192, 1024, mix.MOE_SILU),                    # a rest that is cut by rows
+    ((2100, 2050, 1990, 2060), 64, 1280, mix.MOE_NONE),        # full turns and a rest; one stage: its successor is another tile's
+])
+def test_tiles_and_turns(cuda, counts, K, ncols, act):
+    x, w, offsets, idx, scale = _case(counts, K, ncols, act == mix.MOE_SILU, 1, seed=K)
+    out = torch.full((sum(counts), ncols), 7.0, dtype=torch.bfloat16, device=cuda)
+    dev = [t.to(cuda) for t in (x, w, offsets, idx, scale)]
+    assert mix._kern().moe_gemm(out, *dev[:4], 1, dev[4], act, 1.5, 1.7)
+    want = _want(x, w, offsets, idx, 1, act, scale, 1.5, 1.7)
+    tol = 2.0 ** -8 * (want.abs() + want.square().mean(1, keepdim=True).sqrt())
+    assert ((out.cpu().double() - want).abs() <= tol).all()
+
+
 def test_extra_groups_are_left_alone(cuda):
     """Rows behind the last expert (identity entries, other ranks' experts) are not written."""
     x, w, offsets, idx, _ = _case((40, 60), 128, 256, False, 1)
