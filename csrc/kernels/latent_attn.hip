@@ -471,19 +471,33 @@ template <int NW> hipError_t launch_mfma_ndb(const LatentAttnArgs& a, hipStream_
   return hipErrorInvalidValue;
 }
 
+// The row tile and sequence of a workgroup, of a grid (tiles, sequences). Workgroups go to the 8 XCDs, which have an L2 each, in turn: sequence
+// s is XCD s % 8's, so that its cache rows are in one L2 and long and short sequences are spread; numbers that are no multiple of 8
+// are dealt tile by tile. A sequence's last tiles see the most keys and start first.
+__device__ __forceinline__ void tile_of(int& bx, int& s) {
+  const unsigned nx = gridDim.x, lin = blockIdx.x + nx * blockIdx.y, j = lin / 8;
+  const bool whole = gridDim.y % 8 == 0;
+  s = (int)(whole ? lin % 8 + 8 * (j / nx) : blockIdx.y);
+  bx = (int)(nx - 1 - (whole ? j % nx : blockIdx.x));
+}
+
 // Prompt-sized steps at the common rotary widths (rot_dim = 16 * NROT, NROT = 0: no rotary part): the same algorithm with every
 // wave's query fragments in registers (loaded straight from global memory, the rotary part rotated on the way). A wave owns 16
 // rows: sums and queries take 64 + 36 registers at rank 256, so that 3 waves share a SIMD and one's softmax runs beside the others'
 // products. Key tiles come by DMA into two buffers of a workgroup of 4 waves, one barrier per tile. A tile of 32 rows by KCH 16-byte
 // pieces lies in LDS as the DMA writes it, without gaps; the pieces of a row are exchanged (XOR) so that 16 consecutive rows' reads
-// of one piece fall on all banks.
+// of one piece fall on all banks, and so do the transposed reads of 8 rows by two pieces (the number is rotated for those: by the plain
+// row number pairs of rows shared banks, a quarter of the kernel's cycles).
 // Bound by LDS reads (34 KB per wave and tile at 128 bytes a cycle: 120 us of the 253 below). 16 sequences of 1024 rows, 16 heads,
 // rank 256 + 32: 32 rows per wave, one wave per SIMD, tiles through registers, looked up piece by piece behind divisions: 518 us;
 // the same with DMA and the next tile's scores under the softmax 370; this 253 (570 TFLOP/s).
 template <int NDB, int NROT> struct RqTile {
   static constexpr int KCH = 4 * NDB + 2 * NROT, NPF = (MKT * KCH + 255) / 256, BYTES = NPF * 4096;
   static constexpr int G = KCH % 16 == 0 ? 16 : KCH % 8 == 0 ? 8 : KCH % 4 == 0 ? 4 : 2;   // rows r and r + 16 / G share banks
-  static __device__ __forceinline__ int swz(int row) { return row / (16 / G) % G; }
+  static __device__ __forceinline__ int swz(int row) {
+    const int i = row / (16 / G) % G;
+    return (2 * i & (G - 1)) | i / (G / 2);
+  }
   static constexpr int OP = 64 * NDB + 16;   // pitch of a result row in LDS
   static constexpr int TABLE = 1024;         // block-table entries in LDS
   static constexpr int LDS = 2 * BYTES + 4 * TABLE > 64 * OP ? 2 * BYTES + 4 * TABLE : 64 * OP;
@@ -496,18 +510,8 @@ __global__ void __launch_bounds__(256, 3) latent_attn_mfma_rq_kernel(LatentAttnA
   using Z = RqTile<NDB, NROT>;
   constexpr int KCH = Z::KCH, NPF = Z::NPF, NLAT = NDB, NK = NDB + NROT / 2;   // 32-wide steps of a row: latent, in all
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];   // two tiles, block-table entries; at the end the results
-  // Workgroups are dealt to the 8 XCDs round-robin by their linear id, and each XCD has its own L2: renumber so
-  // that XCD k runs a contiguous eighth of the (sequence-major) tile list — the row tiles of one sequence share
-  // that sequence's cache rows in ONE L2 instead of streaming every sequence through all eight
-  int bx = blockIdx.x, by = blockIdx.y;
-  {
-    const unsigned total = gridDim.x * gridDim.y, lin = blockIdx.x + gridDim.x * blockIdx.y;
-    if (total % 8 == 0) {
-      const unsigned nl = (lin % 8) * (total / 8) + lin / 8;
-      bx = (int)(gridDim.x - 1 - nl % gridDim.x);   // the tiles with the most keys first
-      by = (int)(nl / gridDim.x);
-    }
-  }
+  int bx, by;
+  tile_of(bx, by);
   const int s = by, lane = threadIdx.x & 63, tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int H = a.heads;
@@ -549,12 +553,17 @@ __global__ void __launch_bounds__(256, 3) latent_attn_mfma_rq_kernel(LatentAttnA
       b_lo = block_of(j0);
       stage_table();
     }
+    uint32_t row[NPF];   // (as many cache rows as a device holds)
 #pragma unroll
     for (int u = 0; u < NPF; ++u) {
       const int j = min(j0 + krow[u], jhi), jb = block_of(j);
-      const bf16_t* src = cache + ((int64_t)btl[jb - b_lo] * a.block_size + (j - jb * a.block_size)) * Dk + pcol[u];
+      row[u] = (uint32_t)btl[jb - b_lo] * (uint32_t)a.block_size + (uint32_t)(j - jb * a.block_size);
+    }
+    __builtin_amdgcn_sched_barrier(0);   // (all lookups, then the loads: they would go in turns, each waited for)
+#pragma unroll
+    for (int u = 0; u < NPF; ++u) {
       char* to = smem_raw + buf * Z::BYTES + (256 * u + 64 * wave) * 16;
-      __builtin_amdgcn_global_load_lds((global_cvoid*)src, (lds_void*)to, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((global_cvoid*)(cache + ((uint64_t)row[u] * Dk + pcol[u])), (lds_void*)to, 16, 0, 0);
     }
   };
   const int nt = jhi < jlo ? 0 : (jhi - jlo) / MKT + 1;
@@ -620,6 +629,8 @@ __global__ void __launch_bounds__(256, 3) latent_attn_mfma_rq_kernel(LatentAttnA
   // registers), columns 16 db ..
   const int ksw = Z::swz(li), vrow = 4 * lg + (li >> 2), vsw = Z::swz(vrow);
   const int kat = 16 * li * KCH, vat = 16 * vrow * KCH + 8 * (li & 1);
+  // The queries are here. (Without this the compiler waits for them in the loop, behind the next tile's DMA and so for that too.)
+  __builtin_amdgcn_s_waitcnt(15 << 8 | 7 << 4);
   for (int i = 0; i < nt; ++i) {
     const int j0 = jlo + i * MKT;
     // tile i is in LDS for every wave, and every wave has left the other buffer
@@ -716,6 +727,247 @@ __global__ void __launch_bounds__(256, 3) latent_attn_mfma_rq_kernel(LatentAttnA
   }
 }
 
+// The same with 32 rows per wave and 32x32x16 products, for steps of few row tiles (launch_rows): a fragment that is read from LDS serves 32
+// rows, and the next ones are read ahead of a group's products. Two waves share 32 rows: both form the scores and weights, each its half
+// of the value columns, so that sums and queries take 64 + 72 registers at rank 256 and two waves share a SIMD. (Whole rows
+// per wave spill with two waves per SIMD; with one its sums move between the two kinds of registers: 337 us of 16 x 1024 rows against 324.)
+template <int NDB, int NROT> struct LatentTile {
+  static constexpr int KCH = 4 * NDB + 2 * NROT, NPF = (32 * KCH + 255) / 256, BYTES = NPF * 256 * 16;
+  static constexpr int X = KCH % 16 == 0 ? 16 : KCH % 8 == 0 ? 8 : KCH % 4 == 0 ? 4 : 2;   // pieces that change places
+  static __device__ __forceinline__ int swz(int row) {
+    return X == 16 ? (row & 3) << 2 | (row >> 2 & 3) : X == 8 ? (row >> 1 & 1) << 2 | (row >> 2 & 3) : row / (16 / X) % X;
+  }
+  static constexpr int HC = 2, ROWS = 128 / HC;   // waves that share rows, each with its value columns; rows of a workgroup
+  static constexpr int TABLE = 1024;                            // key rows in LDS
+  static constexpr int LDS = 2 * BYTES + 4 * TABLE;
+};
+
+template <int NDB, int NROT>
+__global__ void __launch_bounds__(256, 2) latent_attn_wide_kernel(LatentAttnArgs a, uint32_t bs_mul, int bs_shift) {
+  using Z = LatentTile<NDB, NROT>;
+  constexpr int HC = Z::HC, NO = NDB / HC;   // 32-column blocks of a wave
+  constexpr int KCH = Z::KCH, NPF = Z::NPF, KT = 32, NLAT = 2 * NDB, NK = NLAT + NROT;   // 16-wide steps of a row: latent, in all
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];   // two tiles, key rows
+  int bx, by;
+  tile_of(bx, by);
+  const int s = by, lane = threadIdx.x & 63, tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int H = a.heads;
+  constexpr int R = 32 * NDB, Dk = R + 16 * NROT;
+  const int q0 = a.cu_q ? a.cu_q[s] : s;
+  const int nq = a.cu_q ? a.cu_q[s + 1] - q0 : 1;
+  const int nrows = nq * H, row0 = bx * Z::ROWS;
+  if (row0 >= nrows) return;
+  const int ctx = a.ctx_lens[s];
+  const int last_row = min(row0 + Z::ROWS, nrows) - 1;
+  const int p_first = (int)a.positions[q0 + row0 / H], p_last = (int)a.positions[q0 + last_row / H];
+  const int jlo = a.window > 0 ? max(0, p_first - a.window + 1) : 0;
+  const int jhi = min(p_last, ctx - 1);
+  const bf16_t* cache = reinterpret_cast<const bf16_t*>(a.cache);
+  const int li = lane & 31, hi = lane >> 5;
+
+  // cache rows of the workgroup's keys in LDS, TABLE keys at a time
+  const int* bt = a.block_tables + (int64_t)s * a.bt_stride;
+  int* rows = reinterpret_cast<int*>(smem_raw + 2 * Z::BYTES);
+  int jt = jlo;
+  auto stage_rows = [&]() {
+    for (int u = tid; u < Z::TABLE && jt + u <= jhi; u += 256) {
+      const int jb = a.block_size == 1 ? jt + u : (int)(__umulhi((uint32_t)(jt + u), bs_mul) >> bs_shift);
+      rows[u] = (int)((uint32_t)bt[jb] * (uint32_t)a.block_size + (uint32_t)(jt + u - jb * a.block_size));
+    }
+    __syncthreads();
+  };
+  stage_rows();
+  // tile rows by DMA: piece u of this thread is 16 bytes of key krow[u] (beyond the tile: of its last key, into the slack)
+  int krow[NPF], pcol[NPF];
+#pragma unroll
+  for (int u = 0; u < NPF; ++u) {
+    const int idx = tid + 256 * u, row = min(idx / KCH, KT - 1);
+    krow[u] = row;
+    pcol[u] = 8 * (idx < KT * KCH ? (idx - row * KCH) ^ Z::swz(row) : 0);
+  }
+  auto fetch = [&](int j0, int buf) {   // (keys beyond the last repeat it)
+    if (min(j0 + KT - 1, jhi) - jt >= Z::TABLE) {
+      __syncthreads();
+      jt = j0;
+      stage_rows();
+    }
+    const int at = j0 - jt, end = jhi - jt;
+    int row[NPF];
+#pragma unroll
+    for (int u = 0; u < NPF; ++u) row[u] = rows[min(at + krow[u], end)];
+    __builtin_amdgcn_sched_barrier(0);   // (all lookups, then the loads: they would go in turns, each waited for)
+#pragma unroll
+    for (int u = 0; u < NPF; ++u) {
+      char* to = smem_raw + buf * Z::BYTES + (256 * u + 64 * wave) * 16;
+      __builtin_amdgcn_global_load_lds((global_cvoid*)(cache + ((uint64_t)(uint32_t)row[u] * Dk + pcol[u])), (lds_void*)to, 16, 0, 0);
+    }
+  };
+  const int nt = jhi < jlo ? 0 : (jhi - jlo) / KT + 1;
+  if (nt > 0) fetch(jlo, 0);
+
+  const int wrow = row0 + wave / HC * 32, myrow = wrow + li;
+  const bool rok = myrow < nrows, wave_live = wrow < nrows, all_rows = wrow + 31 < nrows;
+  const int64_t tq = rok ? q0 + myrow / H : q0;
+  const int hq = rok ? myrow % H : 0;
+  const int64_t orow = (int64_t)hq * a.total_q + tq;
+  const int prow = rok ? (int)a.positions[tq] : -1;
+  const int pw_min = wave_live ? (int)a.positions[q0 + wrow / H] : 0;
+  const int pw_max = wave_live ? (int)a.positions[q0 + min(wrow + 31, nrows - 1) / H] : 0;
+  // this lane's query fragments: qf[k] = Q[row][16 k + 8 hi .. + 8]. (Rows beyond the last repeat the first; every load is
+  // unconditional, so that all are in flight together.)
+  bf16x8_t qf[NK];
+  const bf16_t* qlat = reinterpret_cast<const bf16_t*>(a.q_lat) + orow * R;
+#pragma unroll
+  for (int k = 0; k < NLAT; ++k) qf[k] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(qlat + 16 * k + 8 * hi));
+  if constexpr (NROT > 0) {
+    bf16_t qr[NROT][8];
+    float fr[NROT][4];
+    const bf16_t* qp = reinterpret_cast<const bf16_t*>(a.q_rot) + tq * a.q_stride + (int64_t)hq * a.q_hstride + 8 * hi;
+#pragma unroll
+    for (int k = 0; k < NROT; ++k) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) qr[k][e] = qp[16 * k + e];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) fr[k][i] = a.sh.rot_pairs > 0 ? a.sh.inv_freq[min(8 * k + 4 * hi + i, a.sh.rot_pairs - 1)] : 0.f;
+    }
+#pragma unroll
+    for (int k = 0; k < NROT; ++k) {
+      float f[8];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float u = bf2f(qr[k][2 * i]), w = bf2f(qr[k][2 * i + 1]);
+        float sn, cs;
+        __sincosf((float)prow * fr[k][i], &sn, &cs);
+        const bool turned = 8 * k + 4 * hi + i < a.sh.rot_pairs;
+        f[2 * i] = turned ? u * cs - w * sn : u;
+        f[2 * i + 1] = turned ? w * cs + u * sn : w;
+      }
+      qf[NLAT + k] = __builtin_bit_cast(bf16x8_t, pack8(f));
+    }
+  }
+
+  constexpr float LOG2E = 1.4426950408889634f;
+  const float sl2 = a.scale * LOG2E;
+  const bool has_sink = a.sink != nullptr && rok;
+  float m = has_sink ? a.sink[hq] * LOG2E : -1e30f;
+  float l = has_sink && hi == 0 ? 1.0f : 0.0f;   // (the sum of this lane's keys)
+  f32x16_t o[NO];
+#pragma unroll
+  for (int db = 0; db < NO; ++db) o[db] = f32x16_t{};
+  // K fragments: key li of 32, piece 2 k + hi; V fragments: keys 4 hi .. and 8 + 4 hi .. of 16 (the order in which the weights lie
+  // in registers), columns 32 db ..
+  const int ksw = Z::swz(li), vrow = 4 * hi + (lane & 15) / 4, vsw = Z::swz(vrow), vsw8 = Z::swz(vrow + 8);
+  const int kat = 16 * li * KCH, vat = 16 * vrow * KCH + 8 * (lane & 1), vpc = 4 * NO * (wave % HC) + 2 * (lane >> 4 & 1) + (lane >> 1 & 1);
+  // The queries are here. (Without this the compiler waits for them in the loop, behind the next tile's DMA and so for that too.)
+  __builtin_amdgcn_s_waitcnt(15 << 8 | 7 << 4);
+  for (int i = 0; i < nt; ++i) {
+    const int j0 = jlo + i * KT;
+    // tile i is in LDS for every wave, and every wave has left the other buffer
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(7 << 4);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (i + 1 < nt) fetch(j0 + KT, (i + 1) & 1);
+    const char* ks = smem_raw + (i & 1) * Z::BYTES;
+    f32x16_t sc = {};
+    constexpr int KG = NK % 2 == 0 ? 2 : 1, NG = NK / KG;   // fragments of KG steps ahead
+    static_assert(NG * KG == NK, "whole groups");
+    bf16x8_t kf[2][KG];
+    auto read_k = [&](int g) {
+#pragma unroll
+      for (int k = 0; k < KG; ++k)
+        kf[g & 1][k] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(ks + kat + 16 * ((2 * (KG * g + k) + hi) ^ ksw)));
+    };
+    read_k(0);
+#pragma unroll
+    for (int g = 0; g < NG; ++g) {
+      if (g + 1 < NG) read_k(g + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < KG; ++k) sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[g & 1][k], qf[KG * g + k], sc, 0, 0, 0);
+    }
+    // interior tiles (every key visible to every row of the wave) skip the per-score mask
+    const bool inner = all_rows && j0 + KT - 1 <= min(pw_min, jhi) && (a.window <= 0 || pw_max - j0 < a.window);
+    if (!inner) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int j = j0 + 8 * (e / 4) + 4 * hi + e % 4;
+        const bool valid = rok && j <= jhi && j <= prow && (a.window <= 0 || prow - j < a.window);
+        sc[e] = valid ? sc[e] : -INFINITY;
+      }
+    }
+    float mx = sc[0];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sc[e]);
+    const float mn = fmaxf(m, xor32_max(mx) * sl2);
+    if (__builtin_amdgcn_ballot_w64(mn != m) != 0) {   // wave-uniform
+      const float alpha = __builtin_amdgcn_exp2f(m - mn);
+      l *= alpha;
+#pragma unroll
+      for (int db = 0; db < NO; ++db)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[db][e] *= alpha;
+      m = mn;
+    }
+    float sum[2] = {};
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      sc[e] = __builtin_amdgcn_exp2f(fmaf(sc[e], sl2, -m));
+      sum[e & 1] += sc[e];
+    }
+    l += sum[0] + sum[1];
+    // 16 keys and VG column blocks a group, fragments of the next group ahead
+    constexpr int VG = NO < 2 ? NO : 2, NV = 2 * NO / VG;
+    bf16x8_t vf[2][VG];
+    auto read_v = [&](int g) {
+      const int u = g / (NO / VG), d0 = g % (NO / VG) * VG;
+#pragma unroll
+      for (int d = 0; d < VG; ++d) {
+        const char* at = ks + vat + 256 * KCH * u;
+        const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(at + 16 * ((4 * (d0 + d) + vpc) ^ vsw)));
+        const short4_t up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(at + 128 * KCH + 16 * ((4 * (d0 + d) + vpc) ^ vsw8)));
+        vf[g & 1][d] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
+      }
+    };
+    read_v(0);
+#pragma unroll
+    for (int g = 0; g < NV; ++g) {
+      const int u = g / (NO / VG), d0 = g % (NO / VG) * VG, e = 8 * (u & 1);
+      const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, make_uint4(pack2(sc[e], sc[e + 1]), pack2(sc[e + 2], sc[e + 3]),
+                                                                  pack2(sc[e + 4], sc[e + 5]), pack2(sc[e + 6], sc[e + 7])));
+      if (g + 1 < NV) read_v(g + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int d = 0; d < VG; ++d) o[d0 + d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[g & 1][d], pf, o[d0 + d], 0, 0, 0);
+    }
+  }
+  // results: a row's columns 32 db + 8 q + 4 hi .. in the registers; lanes 32 apart exchange halves, so that each stores 8 columns
+  l = xor32_sum(l);
+  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  bf16_t* op = reinterpret_cast<bf16_t*>(a.out) + orow * R + 32 * NO * (wave % HC) + 8 * hi;
+#pragma unroll
+  for (int db = 0; db < NO; ++db)
+#pragma unroll
+    for (int q = 0; q < 16; q += 8) {
+      const auto x = __builtin_amdgcn_permlane32_swap(pack2(o[db][q] * inv, o[db][q + 1] * inv), pack2(o[db][q + 4] * inv, o[db][q + 5] * inv), false, false);
+      const auto y = __builtin_amdgcn_permlane32_swap(pack2(o[db][q + 2] * inv, o[db][q + 3] * inv), pack2(o[db][q + 6] * inv, o[db][q + 7] * inv), false, false);
+      if (rok) *reinterpret_cast<uint4*>(op + 32 * db + 2 * q) = make_uint4(x[0], y[0], x[1], y[1]);
+    }
+}
+
+template <int NDB, int NROT> hipError_t launch_wide(const LatentAttnArgs& a, hipStream_t s) {
+  int log = 1;
+  while ((int64_t)1 << log < a.block_size) ++log;
+  const uint32_t bs_mul = a.block_size == 1 ? 0 : (uint32_t)(((uint64_t)1 << (31 + log)) / a.block_size + 1);
+  const dim3 grid((unsigned)(((int64_t)a.max_q * a.heads + LatentTile<NDB, NROT>::ROWS - 1) / LatentTile<NDB, NROT>::ROWS), (unsigned)a.num_seqs);
+  auto* fn = latent_attn_wide_kernel<NDB, NROT>;
+  constexpr int lds = LatentTile<NDB, NROT>::LDS;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, grid, dim3(256), lds, s, a, bs_mul, log - 1);
+  return hipGetLastError();
+}
 template <int NDB, int NROT> hipError_t launch_mfma_rq(const LatentAttnArgs& a, hipStream_t s) {
   // floor(j / block_size) = (j * bs_mul) >> (32 + bs_shift) for 31-bit j
   int log = 1;
@@ -728,19 +980,27 @@ template <int NDB, int NROT> hipError_t launch_mfma_rq(const LatentAttnArgs& a, 
 
 // the register-query kernel exists for rank in {64, 128, 256} x rot_dim in {0, 16, 32, 64}; unsplit steps only. It writes results
 // 16 bytes at a time and passes row numbers between lanes in 32 bits (the other kernel: 8 bytes, 64 bits).
-inline bool mfma_rq_ok(const LatentAttnArgs& a) {
+inline bool mfma_rq_fits(const LatentAttnArgs& a) {
   const int r = a.sh.rank, t = a.sh.rot_dim;
-  return a.nsplit <= 1 && (int64_t)a.max_q * a.heads > 32 && (r == 64 || r == 128 || r == 256) &&
+  return (int64_t)a.max_q * a.heads > 32 && (r == 64 || r == 128 || r == 256) &&
          (t == 0 || t == 16 || t == 32 || t == 64) && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0 &&
          (int64_t)a.heads * a.total_q < (int64_t(1) << 31);
 }
 
+// A workgroup has 64 rows in either kernel. Up to two of them per CU go with 32 rows per wave (whose maxima are taken before the scale: a
+// positive one), more with 16, of which three workgroups share a CU and which start faster, for few keys too. 16 / 32 rows per wave, rank 256 + 32, us: 1 x 300 rows of 16 heads
+// 23.5 / 17.9, 1 x 1500 behind 400 118 / 78, 8 x 128 14.4 / 12.8; 32 x 30 9.7 / 10.8; 8 x 500 behind 100 50 / 54, 16 x 1024 309 / 324.
+template <int NDB, int NROT> hipError_t launch_rows(const LatentAttnArgs& a, hipStream_t s) {
+  const int64_t wgs = ((int64_t)a.max_q * a.heads + 63) / 64 * a.num_seqs;
+  const int64_t keys = (int64_t)a.bt_stride * a.block_size;
+  return wgs <= 2 * (int64_t)num_cus() && keys >= 96 && a.scale > 0.f ? launch_wide<NDB, NROT>(a, s) : launch_mfma_rq<NDB, NROT>(a, s);
+}
 template <int NDB> hipError_t launch_mfma_rq_rot(const LatentAttnArgs& a, hipStream_t s) {
   switch (a.sh.rot_dim) {
-    case 0: return launch_mfma_rq<NDB, 0>(a, s);   // no rotary part: latents without positions
-    case 16: return launch_mfma_rq<NDB, 1>(a, s);
-    case 32: return launch_mfma_rq<NDB, 2>(a, s);
-    case 64: return launch_mfma_rq<NDB, 4>(a, s);
+    case 0: return launch_rows<NDB, 0>(a, s);   // no rotary part: latents without positions
+    case 16: return launch_rows<NDB, 1>(a, s);
+    case 32: return launch_rows<NDB, 2>(a, s);
+    case 64: return launch_rows<NDB, 4>(a, s);
   }
   return hipErrorInvalidValue;
 }
@@ -755,7 +1015,7 @@ hipError_t launch_mfma_rq_any(const LatentAttnArgs& a, hipStream_t s) {
 }
 
 hipError_t launch_mfma_any(const LatentAttnArgs& a, hipStream_t s) {
-  if (a.impl != 3 && mfma_rq_ok(a)) return launch_mfma_rq_any(a, s);
+  if (a.impl != 3 && a.nsplit <= 1 && mfma_rq_fits(a)) return launch_mfma_rq_any(a, s);
   // one wave per workgroup when a sequence brings at most 32 rows (decode steps): small LDS, many workgroups
   return (int64_t)a.max_q * a.heads <= 32 ? launch_mfma_ndb<1>(a, s) : launch_mfma_ndb<4>(a, s);
 }
@@ -800,10 +1060,11 @@ template <bool F32> hipError_t launch_bk(const LatentAttnArgs& a, hipStream_t s)
 }  // namespace
 
 bool latent_attn_uses_mfma(const LatentAttnArgs& a) { return a.impl != 1 && mfma_ok(a); }
+bool latent_attn_fits_rows(const LatentAttnArgs& a) { return latent_attn_uses_mfma(a) && a.impl != 3 && mfma_rq_fits(a); }
 
 const char* latent_attn_form(const LatentAttnArgs& a) {
   if (!latent_attn_uses_mfma(a)) return "fma";
-  return a.impl != 3 && mfma_rq_ok(a) ? "rows" : a.nsplit > 1 ? "split" : "tiles";
+  return a.impl != 3 && a.nsplit <= 1 && mfma_rq_fits(a) ? "rows" : a.nsplit > 1 ? "split" : "tiles";
 }
 
 hipError_t launch_latent_attn(const LatentAttnArgs& a, hipStream_t s) {

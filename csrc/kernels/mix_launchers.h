@@ -127,6 +127,8 @@ hipError_t launch_latent_attn(const LatentAttnArgs& a, hipStream_t s);
 // whether launch_latent_attn would run the matrix-core kernel for these arguments (the split workspace is only
 // used by it)
 bool latent_attn_uses_mfma(const LatentAttnArgs& a);
+// whether the kernel for prompt-sized steps would run if the keys are not split
+bool latent_attn_fits_rows(const LatentAttnArgs& a);
 // the kernel that launch_latent_attn runs: "rows" (matrix cores, queries in registers), "tiles" (queries in LDS), "split" (the same,
 // keys split and merged), "fma"
 const char* latent_attn_form(const LatentAttnArgs& a);

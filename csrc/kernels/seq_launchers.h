@@ -176,6 +176,8 @@ struct SinkAttnArgs {
 };
 hipError_t launch_sink_attn(const SinkAttnArgs& a, hipStream_t s);
 bool sink_attn_uses_mfma(const SinkAttnArgs& a);
+// whether the kernel for prompt-sized steps would run if the keys are not split
+bool sink_attn_fits_rows(const SinkAttnArgs& a);
 // whether launch_sink_attn would run the decode-step kernel (impl 0, one bf16 query token per sequence); it splits
 // the keys in multiples of 128
 bool sink_attn_uses_decode(const SinkAttnArgs& a);

@@ -14,6 +14,8 @@
 // of the H / G query heads of ONE key/value head), stages tiles of BK keys and values once in LDS as fp32 (odd row
 // stride) and shares them between its rows. Lanes split (key, slice of dim) for the scores, value columns for the
 // weighted sum. The matrix-core form for bf16 follows it below.
+#include <algorithm>
+
 #include "common.h"
 #include "seq_launchers.h"
 
@@ -630,20 +632,45 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 && NKC <= 16 && NDB <= 4 ? 2 
 }
 
 
+// The row tile, sequence and key/value head of a workgroup, of a grid (tiles, sequences, heads). A pair of sequence and head has its own
+// cache rows. Workgroups go to the 8 XCDs, which have an L2 each, in turn: pair u is XCD u % 8's, so that its cache rows are in one L2
+// and long and short sequences are spread (an eighth of the list for each XCD left it with neighbours of a sorted batch: 16 sequences of 519 -
+// 1000 tokens behind 150 - 300, 4 heads: 165 us, now 131). Pairs that are no multiple of 8 are dealt tile by tile. Last tiles see the most keys
+// and start first, those of all pairs together.
+__device__ __forceinline__ void tile_of(int G, int& bx, int& s, int& g) {
+  const unsigned nx = gridDim.x, pairs = gridDim.y * gridDim.z, lin = blockIdx.x + nx * (blockIdx.y + gridDim.y * blockIdx.z);
+  unsigned u, t;
+  if (pairs % 8 == 0) {
+    const unsigned own = pairs / 8, j = lin / 8;
+    t = j / own;
+    u = lin % 8 + 8 * (j % own);
+  } else {
+    t = lin / pairs;
+    u = lin % pairs;
+  }
+  bx = (int)(nx - 1 - t);
+  s = (int)(u / (unsigned)G);
+  g = (int)(u % (unsigned)G);
+}
+
 // Prompt-sized steps at the common widths (dim 64 or 128, vdim 64, 128 or 256), keys not split: the same algorithm with 16 rows per
 // wave and 16x16x32 products, so that the sums and queries take 32 + 16 registers at 128 + 128 and 4 waves share a SIMD: one's
 // softmax and waits run beside the others' products. A workgroup of 4 waves takes 64 rows; key tiles [K_g | V_g] come by DMA into two
 // buffers, one barrier per tile. A tile of 32 rows by KCH 16-byte pieces lies in LDS without gaps; the pieces of a row are exchanged
-// (XOR) so that 16 consecutive rows' reads of one piece fall on all banks.
+// (XOR) so that 16 consecutive rows' reads of one piece fall on all banks, and the transposed reads of 8 rows by two pieces (a rotated row number:
+// by the plain one pairs of rows shared banks).
 // Bound by the issue of vector instructions (110 per wave and tile beside 16 products). 16 ragged sequences of up to 1024 rows, 16 heads
-// in 4 groups of 128 + 128, a window of 512: 32 rows per wave (below), two waves per SIMD and tiles through registers took 110 us,
-// this takes 84; 16 sequences of 500, vdim 256: 222 -> 90. Long sequences whose keys are all seen (the other kernel reads LDS half as
+// in 4 groups of 128 + 128, a window of 512: 32 rows per wave (above), two waves per SIMD and tiles through registers took 110 us,
+// this takes 82 (99 before tile_of and the two waits named below); 16 sequences of 500, vdim 256: 222 -> 90. Long sequences whose keys are all seen (the other kernel reads LDS half as
 // often there): 4 x 1500 rows of 32 heads 161 -> 149, 4 x 4096 of 16 558 -> 475, 1 x 16384 2582 -> 2501. With a bias per distance
 // (130 distances, a window of 1024) 16 x 1024 rows 160 -> 141, 4 x 4096 240 -> 228 (where every score looks its distance up: 182, 297).
 template <int NK, int NV> struct RowTile {
   static constexpr int KCH = 4 * NK + 2 * NV, NPF = MKT * KCH / 256, BYTES = MKT * KCH * 16;
   static constexpr int X = KCH % 16 == 0 ? 16 : 8;   // rows r and r + 16 / X share banks
-  static __device__ __forceinline__ int swz(int row) { return row / (16 / X) % X; }
+  static __device__ __forceinline__ int swz(int row) {
+    const int i = row / (16 / X) % X;
+    return (2 * i & (X - 1)) | i / (X / 2);
+  }
   static constexpr int OP = 32 * NV + 16;            // pitch of a result row in LDS
   static constexpr int TABLE = 1024;                 // key rows in LDS
   static constexpr int LDS = 2 * BYTES + 4 * TABLE > 64 * OP ? 2 * BYTES + 4 * TABLE : 64 * OP;
@@ -656,18 +683,9 @@ __global__ void __launch_bounds__(256, NV <= 8 ? 4 : 3) sink_attn_rows_kernel(Si
   using Z = RowTile<NK, NV>;
   constexpr int KCH = Z::KCH, D = 32 * NK, DV = 16 * NV, roww = D + DV;
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];   // two tiles, key rows; at the end the results
-  int bx = blockIdx.x, by = blockIdx.y;
-  {
-    // XCD k takes a contiguous eighth of the sequence-major tile list, so one sequence's cache rows stay in one L2
-    const unsigned total = gridDim.x * gridDim.y, lin = blockIdx.x + gridDim.x * blockIdx.y;
-    if (total % 8 == 0) {
-      const unsigned nl = (lin % 8) * (total / 8) + lin / 8;
-      bx = (int)(nl % gridDim.x);
-      by = (int)(nl / gridDim.x);
-    }
-    bx = gridDim.x - 1 - bx;   // a sequence's last rows see the most keys: they start first
-  }
-  const int H = a.heads, G = a.kv_heads, QPG = H / G, s = by, g = blockIdx.z;
+  const int H = a.heads, G = a.kv_heads, QPG = H / G;
+  int bx, s, g;
+  tile_of(G, bx, s, g);
   const int lane = threadIdx.x & 63, tid = threadIdx.x, li = lane & 15, lg = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int q0 = a.cu_q ? a.cu_q[s] : s;
@@ -706,11 +724,14 @@ __global__ void __launch_bounds__(256, NV <= 8 ? 4 : 3) sink_attn_rows_kernel(Si
       stage_rows();
     }
     const int at = j0 - jt, end = jhi - jt;
+    int row[Z::NPF];
+#pragma unroll
+    for (int u = 0; u < Z::NPF; ++u) row[u] = rows[min(at + krow[u], end)];
+    __builtin_amdgcn_sched_barrier(0);   // (all lookups, then the loads: they would go in turns, each waited for)
 #pragma unroll
     for (int u = 0; u < Z::NPF; ++u) {
-      const int row = rows[min(at + krow[u], end)];
       char* to = smem_raw + buf * Z::BYTES + (256 * u + 64 * wave) * 16;
-      __builtin_amdgcn_global_load_lds((global_cvoid*)(cache + ((uint64_t)(uint32_t)row * roww + pcol[u])), (lds_void*)to, 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((global_cvoid*)(cache + ((uint64_t)(uint32_t)row[u] * roww + pcol[u])), (lds_void*)to, 16, 0, 0);
     }
   };
   if (nt > 0) fetch(jlo, 0);
@@ -749,6 +770,8 @@ __global__ void __launch_bounds__(256, NV <= 8 ? 4 : 3) sink_attn_rows_kernel(Si
   // registers), columns 16 db ..
   const int ksw = Z::swz(li), vrow = 4 * lg + (li >> 2), vsw = Z::swz(vrow);
   const int kat = 16 * li * KCH, vat = 16 * vrow * KCH + 8 * (li & 1), vpc = 4 * NK + (li >> 1 & 1);
+  // The queries are here. (Without this the compiler waits for them in the loop, behind the next tile's DMA and so for that too.)
+  __builtin_amdgcn_s_waitcnt(15 << 8 | 7 << 4);
   for (int i = 0; i < nt; ++i) {
     const int j0 = jlo + i * MKT;
     // tile i is in LDS for every wave, and every wave has left the other buffer
@@ -872,6 +895,216 @@ __global__ void __launch_bounds__(256, NV <= 8 ? 4 : 3) sink_attn_rows_kernel(Si
   }
 }
 
+
+// The same with 32 rows per wave and 32x32x16 products, for steps of many rows: a fragment of keys or values that is read from LDS
+// serves 32 rows, and a lane holds one row's scores of half the tile, so that maxima and sums cross lanes once. 4 waves take 128 rows,
+// two workgroups share a CU. Key tiles of 64 (vdim 256: 32). Pieces of a row are exchanged (XOR) by the row's low bits, rotated: 16
+// consecutive rows' reads of one piece, and the transposed reads of 4 rows by four neighbouring pieces, fall on all banks.
+// Plain scores of a positive scale only (wide_takes). Bound by vector and matrix instructions of two waves per SIMD, which run in turns
+// more than side by side (30 % and 42 % of the cycles): figures at wide_takes.
+template <int NK, int NVB> struct WideTile {
+  static constexpr int KT = NVB > 4 ? 32 : 64;                    // keys of a tile
+  static constexpr int KCH = 4 * NK + 4 * NVB, NPF = KT * KCH / 256, BYTES = KT * KCH * 16;
+  static constexpr int X = KCH % 16 == 0 && NVB <= 4 ? 16 : 8;    // pieces that change places
+  static __device__ __forceinline__ int swz(int row) { 
+    return X == 16 ? (row & 3) << 2 | (row >> 2 & 3) : KCH % 16 == 8 ? (row >> 1 & 1) << 2 | (row >> 2 & 3) : (row & 3) << 1 | (row >> 2 & 1);
+  }
+  static constexpr int TABLE = 1024;                              // key rows in LDS
+  static constexpr int LDS = 2 * BYTES + 4 * TABLE;
+};
+
+template <int NK, int NVB, bool SIG>
+__global__ void __launch_bounds__(256, 2) sink_attn_wide_kernel(SinkAttnArgs a) {
+  using Z = WideTile<NK, NVB>;
+  constexpr int KCH = Z::KCH, KT = Z::KT, NT = KT / 32, D = 32 * NK, DV = 32 * NVB, roww = D + DV;
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];   // two tiles, key rows
+  const int H = a.heads, G = a.kv_heads, QPG = H / G;
+  int bx, s, g;
+  tile_of(G, bx, s, g);
+  const int lane = threadIdx.x & 63, tid = threadIdx.x, li = lane & 31, hi = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q0 = a.cu_q ? a.cu_q[s] : s;
+  const int nq = a.cu_q ? a.cu_q[s + 1] - q0 : 1;
+  const int nrows = nq * QPG, row0 = bx * 128;
+  if (row0 >= nrows) return;
+  const int last_row = min(row0 + 128, nrows) - 1;
+  const int p_first = (int)a.positions[q0 + row0 / QPG], p_last = (int)a.positions[q0 + last_row / QPG];
+  const int jlo = first_key(a, p_first), jhi = min(p_last, a.ctx_lens[s] - 1);
+  const int nt = jhi < jlo ? 0 : (jhi - jlo) / KT + 1;
+
+  // cache rows of the workgroup's keys in LDS, TABLE keys at a time
+  const int* bt = a.block_tables + (int64_t)s * a.bt_stride;
+  int* rows = reinterpret_cast<int*>(smem_raw + 2 * Z::BYTES);
+  const int bs_shift = __builtin_ctz(a.block_size);   // a power of two (mfma_ok)
+  int jt = jlo;
+  auto stage_rows = [&]() {
+    for (int u = tid; u < Z::TABLE && jt + u <= jhi; u += 256)
+      rows[u] = ((bt[(jt + u) >> bs_shift] * G + g) << bs_shift) + ((jt + u) & (a.block_size - 1));
+    __syncthreads();
+  };
+  stage_rows();
+  // piece u of this thread: 16 bytes of key krow[u] of the tile
+  const bf16_t* cache = reinterpret_cast<const bf16_t*>(a.cache);
+  int krow[Z::NPF], pcol[Z::NPF];
+#pragma unroll
+  for (int u = 0; u < Z::NPF; ++u) {
+    const int idx = tid + 256 * u;
+    krow[u] = idx / KCH;
+    pcol[u] = 8 * ((idx % KCH) ^ Z::swz(krow[u]));
+  }
+  auto fetch = [&](int j0, int buf) {   // (keys beyond the last repeat it)
+    if (min(j0 + KT - 1, jhi) - jt >= Z::TABLE) {
+      __syncthreads();
+      jt = j0;
+      stage_rows();
+    }
+    const int at = j0 - jt, end = jhi - jt;
+    int row[Z::NPF];
+#pragma unroll
+    for (int u = 0; u < Z::NPF; ++u) row[u] = rows[min(at + krow[u], end)];
+    __builtin_amdgcn_sched_barrier(0);   // (all lookups, then the loads)
+#pragma unroll
+    for (int u = 0; u < Z::NPF; ++u) {
+      char* to = smem_raw + buf * Z::BYTES + (256 * u + 64 * wave) * 16;
+      __builtin_amdgcn_global_load_lds((global_cvoid*)(cache + ((uint64_t)(uint32_t)row[u] * roww + pcol[u])), (lds_void*)to, 16, 0, 0);
+    }
+  };
+  if (nt > 0) fetch(jlo, 0);
+
+  const int wrow = row0 + wave * 32, myrow = wrow + li;
+  const bool rok = myrow < nrows, wave_live = wrow < nrows, wave_full = wrow + 31 < nrows;
+  const int tq = q0 + (rok ? myrow / QPG : 0), myh = g * QPG + (rok ? myrow % QPG : 0);   // (rows beyond the last repeat the first)
+  const int64_t orow = (int64_t)tq * H + myh;
+  bf16x8_t qf[2 * NK];
+#pragma unroll
+  for (int k = 0; k < 2 * NK; ++k)
+    qf[k] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(a.q) + orow * D + 16 * k + 8 * hi));
+  const int prow = rok ? (int)a.positions[tq] : -1;
+  const int jrow = first_key(a, max(prow, 0));
+  const unsigned seen = rok ? max(min(prow, jhi) - jrow + 1, 0) : 0;   // this row sees keys jrow .. jrow + seen - 1
+  // a tile is interior for a wave when every one of its (key, row) pairs is visible: no masking then
+  const int pw_first = wave_live ? (int)a.positions[q0 + wrow / QPG] : 0;
+  const int pw_last = wave_live ? (int)a.positions[q0 + min(wrow + 31, nrows - 1) / QPG] : 0;
+  const int jw_first = first_key(a, pw_first), jw_last = first_key(a, pw_last);
+  constexpr float LOG2E = 1.4426950408889634f;
+  const float sl2 = a.scale * LOG2E;
+  const float hb2 = SIG && a.head_bias != nullptr ? a.head_bias[myh] * LOG2E : 0.f;
+  const bool has_sink = !SIG && a.sink != nullptr && rok;
+  float m = has_sink ? a.sink[myh] * LOG2E : -1e30f;
+  float l = has_sink && hi == 0 ? 1.0f : 0.0f;   // (the sum of this lane's keys)
+  f32x16_t o[NVB];
+#pragma unroll
+  for (int db = 0; db < NVB; ++db) o[db] = f32x16_t{};
+  // K fragments: key li of 32, piece 2 k + hi; V fragments: keys 4 hi .. and 8 + 4 hi .. of 16 (the order in which the weights lie
+  // in registers), columns 32 db ..
+  const int ksw = Z::swz(li), vrow = 4 * hi + (lane & 15) / 4, vsw = Z::swz(vrow), vsw8 = Z::swz(vrow + 8);
+  const int kat = 16 * li * KCH, vat = 16 * vrow * KCH + 8 * (lane & 1), vpc = 4 * NK + 2 * (lane >> 4 & 1) + (lane >> 1 & 1);
+  __builtin_amdgcn_s_waitcnt(15 << 8 | 7 << 4);
+  for (int i = 0; i < nt; ++i) {
+    const int j0 = jlo + i * KT;
+    // tile i is in LDS for every wave, and every wave has left the other buffer
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(7 << 4);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (i + 1 < nt) fetch(j0 + KT, (i + 1) & 1);
+    if (!wave_live || j0 > pw_last || j0 + KT <= jw_first) continue;   // nothing of this tile is visible to the wave
+    const char* ks = smem_raw + (i & 1) * Z::BYTES;
+    f32x16_t sc[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) sc[t] = f32x16_t{};
+    // fragments of NT x KG products ahead
+    constexpr int KG = 2, NG = 2 * NK / KG;
+    bf16x8_t kf[2][KG][NT];
+    auto read_k = [&](int gk) {
+#pragma unroll
+      for (int k = 0; k < KG; ++k)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          kf[gk & 1][k][t] = __builtin_bit_cast(
+              bf16x8_t, *reinterpret_cast<const uint4*>(ks + kat + 512 * KCH * t + 16 * ((2 * (KG * gk + k) + hi) ^ ksw)));
+    };
+    read_k(0);
+#pragma unroll
+    for (int gk = 0; gk < NG; ++gk) {
+      if (gk + 1 < NG) read_k(gk + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < KG; ++k)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          sc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[gk & 1][k][t], qf[KG * gk + k], sc[t], 0, 0, 0);
+    }
+    // score e of block t: key j0 + 32 t + 8 (e / 4) + 4 hi + e % 4
+    const bool interior = wave_full && j0 + KT - 1 <= min(pw_first, jhi) && j0 >= jw_last;
+    if (!interior) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          sc[t][e] = (unsigned)(j0 + 32 * t + 8 * (e / 4) + 4 * hi + e % 4 - jrow) < seen ? sc[t][e] : -INFINITY;
+    }
+    if constexpr (SIG) {   // 1 / (1 + 2^-(v + bias)); a masked score is -inf and weighs 0
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sc[t][e] = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(fmaf(-sc[t][e], sl2, -hb2)));
+    } else {
+      float mx = sc[0][0];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sc[t][e]);
+      mx = xor32_max(mx * sl2);
+      const float mn = mx > m + LAZY ? mx : m;
+      if (__builtin_amdgcn_ballot_w64(mn != m) != 0) {   // wave-uniform
+        const float alpha = __builtin_amdgcn_exp2f(m - mn);
+        l *= alpha;
+#pragma unroll
+        for (int db = 0; db < NVB; ++db)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) o[db][e] *= alpha;
+        m = mn;
+      }
+      float sum[2] = {};
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          sc[t][e] = __builtin_amdgcn_exp2f(fmaf(sc[t][e], sl2, -m));   // v_exp_f32: arguments are at most LAZY, or -inf
+          sum[e & 1] += sc[t][e];
+        }
+      l += sum[0] + sum[1];
+    }
+#pragma unroll
+    for (int u = 0; u < 2 * NT; ++u) {   // 16 keys each
+      const f32x16_t& c = sc[u / 2];
+      const int e = 8 * (u & 1);
+      const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, make_uint4(pack2(c[e], c[e + 1]), pack2(c[e + 2], c[e + 3]), pack2(c[e + 4], c[e + 5]),
+                                                                  pack2(c[e + 6], c[e + 7])));
+#pragma unroll
+      for (int db = 0; db < NVB; ++db) {
+        const char* at = ks + vat + 256 * KCH * u;
+        const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(at + 16 * ((4 * db + vpc) ^ vsw)));
+        const short4_t up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(at + 128 * KCH + 16 * ((4 * db + vpc) ^ vsw8)));
+        const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
+        o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, pf, o[db], 0, 0, 0);
+      }
+    }
+  }
+  // results: a row's columns 32 db + 8 q + 4 hi .. in the registers; lanes 32 apart exchange halves, so that each stores 8 columns
+  l = xor32_sum(l);
+  const float inv = SIG ? 1.0f : (l > 0.f ? 1.0f / l : 0.f);
+  bf16_t* op = reinterpret_cast<bf16_t*>(a.out) + orow * DV + 8 * hi;
+#pragma unroll
+  for (int db = 0; db < NVB; ++db)
+#pragma unroll
+    for (int q = 0; q < 16; q += 8) {
+      const auto x = __builtin_amdgcn_permlane32_swap(pack2(o[db][q] * inv, o[db][q + 1] * inv), pack2(o[db][q + 4] * inv, o[db][q + 5] * inv), false, false);
+      const auto y = __builtin_amdgcn_permlane32_swap(pack2(o[db][q + 2] * inv, o[db][q + 3] * inv), pack2(o[db][q + 6] * inv, o[db][q + 7] * inv), false, false);
+      if (rok) *reinterpret_cast<uint4*>(op + 32 * db + 2 * q) = make_uint4(x[0], y[0], x[1], y[1]);
+    }
+}
 
 // column c of an output row (token t, head h) after the optional turn and gate, from the row's raw columns o(c)
 template <typename F>
@@ -1293,14 +1526,42 @@ template <int NK, int NV> hipError_t launch_rows(const SinkAttnArgs& a, hipStrea
   hipLaunchKernelGGL(fn, grid, dim3(256), (RowTile<NK, NV>::LDS), s, a);
   return hipGetLastError();
 }
+template <int NK, int NVB> hipError_t launch_wide(const SinkAttnArgs& a, hipStream_t s) {
+  using Z = WideTile<NK, NVB>;
+  const int64_t rows = (int64_t)a.max_q * (a.heads / a.kv_heads);
+  const dim3 grid((unsigned)((rows + 127) / 128), (unsigned)a.num_seqs, (unsigned)a.kv_heads);
+  auto* fn = a.sigmoid ? sink_attn_wide_kernel<NK, NVB, true> : sink_attn_wide_kernel<NK, NVB, false>;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, Z::LDS);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, grid, dim3(256), Z::LDS, s, a);
+  return hipGetLastError();
+}
+template <int NK> hipError_t launch_wide_v(const SinkAttnArgs& a, hipStream_t s) {
+  if (a.vdim == 64) return launch_wide<NK, 2>(a, s);
+  return a.vdim == 128 ? launch_wide<NK, 4>(a, s) : launch_wide<NK, 8>(a, s);
+}
 template <int NK> hipError_t launch_rows_v(const SinkAttnArgs& a, hipStream_t s) {
   if (a.vdim == 64) return launch_rows<NK, 4>(a, s);
   return a.vdim == 128 ? launch_rows<NK, 8>(a, s) : launch_rows<NK, 16>(a, s);
 }
-// prompt-sized steps at the widths of sink_attn_rows_kernel, keys not split
-inline bool rows_takes(const SinkAttnArgs& a) {
-  return (a.ws_o == nullptr || a.nsplit <= 1) && a.max_q * (a.heads / a.kv_heads) > 32 && (a.dim == 64 || a.dim == 128) &&
-         (a.vdim == 64 || a.vdim == 128 || a.vdim == 256) && (int64_t)a.total_q * a.heads < (1ll << 31);
+// prompt-sized steps at the widths of sink_attn_rows_kernel
+inline bool rows_fits(const SinkAttnArgs& a) {
+  return a.max_q * (a.heads / a.kv_heads) > 32 && (a.dim == 64 || a.dim == 128) && (a.vdim == 64 || a.vdim == 128 || a.vdim == 256) &&
+         (int64_t)a.total_q * a.heads < (1ll << 31);
+}
+// and keys not split
+inline bool rows_takes(const SinkAttnArgs& a) { return (a.ws_o == nullptr || a.nsplit <= 1) && rows_fits(a); }
+
+// Of these, those that go 128 rows per workgroup: where that still gives every CU two workgroups twice over, and long keys (a workgroup's
+// start is the same for 64 rows). Scores with caps, slopes or a bias are bound by vector instructions, of which four waves per SIMD
+// issue more than two. 64 / 128 rows, us: 16 x 1000 behind 300, 16 heads 132 / 110, vdim 256 187 / 160, window of 512 89 / 80; 4 x 1000 of 32
+// heads 57 / 54; 2 x 1000 37 / 38; 16 x 250 23.0 / 24.3; capped 16 x 500 of 32 heads 121 / 135.
+inline bool wide_takes(const SinkAttnArgs& a) {
+  const int64_t rows = (int64_t)a.max_q * (a.heads / a.kv_heads), wgs = (rows + 127) / 128 * a.num_seqs * a.kv_heads;
+  int64_t keys = (int64_t)a.bt_stride * a.block_size;
+  if (a.window > 0) keys = std::min<int64_t>(keys, (int64_t)a.window + a.max_q);
+  if (a.seg > 0) keys = std::min<int64_t>(keys, (int64_t)a.seg + a.max_q);
+  return a.softcap <= 0.f && a.slopes == nullptr && a.bias == nullptr && a.scale > 0.f && wgs >= 4 * (int64_t)num_cus() && keys >= 512;
 }
 
 inline bool decode_ok(const SinkAttnArgs& a) {
@@ -1319,6 +1580,7 @@ inline bool mfma_ok(const SinkAttnArgs& a) {
 }  // namespace
 
 bool sink_attn_uses_mfma(const SinkAttnArgs& a) { return a.impl != 1 && mfma_ok(a); }
+bool sink_attn_fits_rows(const SinkAttnArgs& a) { return sink_attn_uses_mfma(a) && rows_fits(a); }
 bool sink_attn_uses_decode(const SinkAttnArgs& a) { return a.impl == 0 && decode_ok(a); }
 bool sink_attn_fuses_gate(const SinkAttnArgs& a) {
   return sink_attn_uses_decode(a) || (sink_attn_uses_mfma(a) && a.ws_o != nullptr && a.nsplit > 1);
@@ -1343,6 +1605,7 @@ hipError_t launch_sink_attn(const SinkAttnArgs& a, hipStream_t s) {
   }
   if (sink_attn_uses_mfma(a)) {
     const int qpg = a.heads / a.kv_heads;
+    if (rows_takes(a) && wide_takes(a)) return a.dim == 64 ? launch_wide_v<2>(a, s) : launch_wide_v<4>(a, s);
     if (rows_takes(a)) return a.dim == 64 ? launch_rows_v<2>(a, s) : launch_rows_v<4>(a, s);
     return a.max_q * qpg <= 32 ? launch_mfma_nw<1>(a, s) : launch_mfma_nw<4>(a, s);
   }

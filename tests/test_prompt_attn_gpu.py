@@ -90,3 +90,36 @@ def test_distance_bias_where_distances_end(cuda, monkeypatch, dim, vdim, rows, s
     assert forms == ["fma", "rows"]
     assert ((got - want).abs() <= 2 ** -8.5 * float(cache.float().abs().max()) + 2 ** -7 * want.abs()).all()
     assert ((got - want).norm() / want.norm()).item() < 2 ** -7
+
+
+def _ragged(cuda, lens, pasts, bs, groups, dim, vdim, heads):
+    T, need = sum(lens), max(-(-(n + p) // bs) for n, p in zip(lens, pasts))
+    cache = torch.randn(1 + 3 * need, bs, groups * (dim + vdim), device=cuda).to(torch.bfloat16)
+    bt = torch.randint(0, 1 + 3 * need, (len(lens), need), device=cuda, dtype=torch.int32)
+    cu = torch.tensor([0] + lens, device=cuda).cumsum(0).int()
+    pos = torch.cat([torch.arange(n) + p for n, p in zip(lens, pasts)]).to(cuda)
+    ctx = torch.tensor([n + p for n, p in zip(lens, pasts)], device=cuda, dtype=torch.int32)
+    return torch.randn(T, heads * dim, device=cuda).to(torch.bfloat16), cache, bt, cu, ctx, pos
+
+
+@pytest.mark.parametrize("dim,vdim,heads,groups,bs,style", [
+    (128, 128, 16, 4, 16, ""), (64, 64, 20, 5, 4, "sink"), (64, 128, 16, 4, 16, "window"), (128, 64, 16, 4, 8, "sigmoid"), (64, 256, 12, 4, 16, ""),
+    (128, 256, 16, 4, 1, "sink"), (128, 128, 12, 4, 16, "seg")])
+def test_many_rows_of_long_keys(cuda, monkeypatch, dim, vdim, heads, groups, bs, style):
+    """128 rows per workgroup: four of them per compute unit, tiles of 64 keys (vdim 256: 32), row counts around 32 and 128, pairs of
+    sequence and head that are and are not a multiple of 8."""
+    torch.manual_seed(dim + vdim + heads)
+    forms = _forms(monkeypatch)
+    lens = ([200, 8, 33, 1, 65, 32, 129, 190] * 11)[:88 if style else 81]
+    data = _ragged(cuda, lens, [520 + 7 * (s % 9) for s in range(len(lens))], bs, groups, dim, vdim, heads)
+    sink, kw = (torch.randn(heads, device=cuda) if style == "sink" else None), {}
+    if style == "sigmoid":
+        kw = dict(sigmoid=True, head_bias=torch.randn(heads, device=cuda) - 5)
+    if style == "seg":
+        kw = dict(seg=512)
+    args = (*data, sink, None, max(lens), heads, groups, dim, vdim, 400 if style == "window" else 0, dim ** -0.5)
+    want, got = seq.sink_attn(*args, impl=1, **kw).float(), seq.sink_attn(*args, **kw).float()
+    assert forms == ["fma", "rows"]
+    mass = 1.0 if style != "sigmoid" else 20.0   # of the sigmoid weights
+    assert ((got - want).abs() <= 2 ** -8.5 * mass * float(data[1].float().abs().max()) + 2 ** -7 * want.abs()).all()
+    assert ((got - want).norm() / want.norm()).item() < 2 ** -7
