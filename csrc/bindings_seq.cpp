@@ -7,6 +7,7 @@
 
 #include "kernels/conv_launchers.h"
 #include "kernels/seq_launchers.h"
+#include "split_rule.h"
 
 using at::Tensor;
 using OptTensor = c10::optional<Tensor>;
@@ -442,11 +443,17 @@ const char* sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, O
     ns = std::min<int64_t>({(int64_t)128, std::max<int64_t>(1, 2048 / std::max<int64_t>(1, wgs)), (bound + 127) / 128});
     if (ns > 1) a.chunk = (int)((((bound + ns - 1) / ns) + 127) / 128 * 128);
   } else if (die::sink_attn_uses_mfma(a)) {
-    // few row tiles: split the keys over workgroups until about 2048 are in flight
-    const int64_t qpg = heads / kv_heads;
-    const int64_t rows_wg = max_q * qpg <= 32 ? 32 : 128;
-    const int64_t tiles = S * kv_heads * ((max_q * qpg + rows_wg - 1) / rows_wg);
+    // few row tiles: split the keys over workgroups until about 2048 are in flight, or less where that is estimated to be faster (a gate
+    // is applied to the merged fp32 rows, without splits to rounded ones: such steps keep their splits)
+    const int64_t qpg = heads / kv_heads, rows = max_q * qpg;
+    const int64_t rows_wg = rows <= 32 ? 32 : 128;
+    const int64_t tiles = S * kv_heads * ((rows + rows_wg - 1) / rows_wg);
     ns = std::min<int64_t>({(int64_t)16, 2048 / std::max<int64_t>(1, tiles), (bound + 63) / 64});
+    if (ns > 1 && a.impl == 0 && !gate.has_value() && die::sink_attn_fits_rows(a)) {
+      const bool broad = vdim > 128;
+      const SplitTimes t = {broad ? 1.2 : 0.85, broad ? 3.0 : 4.0, 10.0, broad ? 1.9 : 1.1, 2.0};
+      ns = best_splits(t, ns, bound, S * kv_heads * ((rows + 63) / 64), tiles, at::cuda::getCurrentDeviceProperties()->multiProcessorCount, T * heads * vdim * 4);
+    }
     if (ns > 1) a.chunk = (int)((((bound + ns - 1) / ns) + 31) / 32 * 32);
   }
   if (ns > 1) {

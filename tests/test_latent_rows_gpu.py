@@ -41,6 +41,36 @@ def test_against_fma(cuda, rank, rot, heads, bs, window, past):
     assert ((got - want).norm() / want.norm()).item() < 2 ** -7
 
 
+@pytest.mark.parametrize("rank,rot,heads,bs,window,lens,past", [
+    (256, 32, 16, 16, 0, (130, 97), 0), (256, 64, 16, 24, 70, (40, 1, 33, 64), 300), (128, 16, 33, 1, 0, (31, 12), 1200), (64, 0, 20, 7, 33, (60,) * 8, 50),
+    (256, 0, 5, 16, 0, (100, 64, 7), 40), (256, 16, 32, 16, 0, (16,) * 8, 90)])
+def test_few_row_tiles(cuda, rank, rot, heads, bs, window, lens, past):
+    """32 rows per wave, two waves to a row's value columns: steps of up to two workgroups per compute unit, unsplit."""
+    from src.ops import mix
+
+    torch.manual_seed(rank + rot + heads)
+    S, T, need = len(lens), sum(lens), -(-(max(lens) + past) // bs)
+    cache = torch.randn(1 + 3 * need, bs, rank + rot, device=cuda).to(torch.bfloat16)
+    bt = torch.randint(0, 1 + 3 * need, (S, need), device=cuda, dtype=torch.int32)
+    cu = torch.tensor([0, *lens], device=cuda).cumsum(0).int()
+    pos = torch.cat([torch.arange(n) + past for n in lens]).to(cuda)
+    ctx = torch.tensor([n + past for n in lens], device=cuda, dtype=torch.int32)
+    q_lat = torch.randn(heads, T, rank, device=cuda).to(torch.bfloat16)
+    q = torch.randn(T, heads * (rot + 6), device=cuda).to(torch.bfloat16)
+    inv, sink, scale = ops.rope_inv_freq(10000.0, max(rot, 2), cuda)[: rot // 2], torch.randn(heads, device=cuda) + 1, 0.08
+    got = torch.empty_like(q_lat)
+    tail = (cache, bt, cu, ctx, pos, sink, max(lens), window, scale, rot, inv)
+    form = mix._kern().latent_attn(got, q_lat, q, 6, *tail, 0)
+    assert form == "rows" or past >= 1000
+    want = ops.latent_attn(q_lat, q, 6, *tail, impl=1).float()
+    e = 0.0
+    if rot:
+        e = scale * 2 ** -9 * float(q.view(T, heads, -1)[..., 6:].float().norm(dim=-1).max() * cache[..., rank:].float().norm(dim=-1).max())
+    top = float(cache[..., :rank].float().abs().max())
+    assert ((got.float() - want).abs() <= (2 ** -9 + 2 * e * 2.71828 ** (2 * e)) * top + 2 ** -7 * want.abs()).all()
+    assert ((got.float() - want).norm() / want.norm()).item() < 2 ** -7
+
+
 def test_results_at_any_8_bytes(cuda):
     """Results that start at no multiple of 16 bytes go to the kernel that writes 8 at a time: the bits that it writes anywhere."""
     from src.ops import mix

@@ -123,3 +123,14 @@ def test_many_rows_of_long_keys(cuda, monkeypatch, dim, vdim, heads, groups, bs,
     mass = 1.0 if style != "sigmoid" else 20.0   # of the sigmoid weights
     assert ((got - want).abs() <= 2 ** -8.5 * mass * float(data[1].float().abs().max()) + 2 ** -7 * want.abs()).all()
     assert ((got - want).norm() / want.norm()).item() < 2 ** -7
+
+
+@pytest.mark.parametrize("seqs,rows,past,form", [(2, 300, 0, "rows"), (8, 128, 0, "rows"), (1, 64, 30, "rows"), (1, 20, 5000, "split"), (3, 9, 1000, "split")])
+def test_keys_are_split_behind_few_rows_only(cuda, monkeypatch, seqs, rows, past, form):
+    torch.manual_seed(rows)
+    forms = _forms(monkeypatch)
+    data = _ragged(cuda, [rows - s for s in range(seqs)], [past] * seqs, 16, 4, 128, 128, 16)
+    args = (*data, None, None, rows, 16, 4, 128, 128, 0, 128 ** -0.5)
+    want, got = seq.sink_attn(*args, impl=1).float(), seq.sink_attn(*args).float()
+    assert forms == ["fma", form]
+    assert ((got - want).norm() / want.norm()).item() < 2 ** -7
