@@ -488,9 +488,9 @@ void moe_combine(Tensor out, Tensor ys, Tensor pos, Tensor w) {
   CHK_DTYPE(pos, at::kInt);
   CHK_DTYPE(w, at::kFloat);
   const int64_t T = out.size(0), K = w.size(1);
-  TORCH_CHECK(w.size(0) == T && pos.numel() == T * K && ys.size(0) == T * K && ys.size(1) == out.size(1),
-              "moe_combine shapes");
-  HIP_OK(die::launch_moe_combine(bf(out), bf(ys), pos.data_ptr<int>(), w.data_ptr<float>(), (int)T, (int)K,
+  TORCH_CHECK(w.size(0) == T && (pos.numel() == T * K || pos.numel() == 0) && ys.size(0) == T * K && ys.size(1) == out.size(1),
+              "moe_combine shapes");   // (no pos: rows in pair order)
+  HIP_OK(die::launch_moe_combine(bf(out), bf(ys), pos.numel() == 0 ? nullptr : pos.data_ptr<int>(), w.data_ptr<float>(), (int)T, (int)K,
                                   (int)out.size(1), cur_stream()));
 }
 
@@ -527,10 +527,10 @@ void moe_combine_residual(Tensor ssp, Tensor resid, Tensor ys, Tensor pos, Tenso
   CHK_DTYPE(w, at::kFloat);
   check_rows(resid, "resid");
   const int64_t T = resid.size(0), H = resid.size(1), K = w.size(1);
-  TORCH_CHECK(w.size(0) == T && pos.numel() == T * K && ys.size(0) == T * K && ys.size(1) == H && ssp.numel() >= T,
-              "moe_combine_residual shapes");
+  TORCH_CHECK(w.size(0) == T && (pos.numel() == T * K || pos.numel() == 0) && ys.size(0) == T * K && ys.size(1) == H && ssp.numel() >= T,
+              "moe_combine_residual shapes");   // (no pos: rows in pair order)
   HIP_OK(die::launch_moe_combine_residual(ssp.data_ptr<float>(), bf(resid), resid.stride(0), bf(ys),
-                                           pos.data_ptr<int>(), w.data_ptr<float>(), (int)T, (int)K, (int)H,
+                                           pos.numel() == 0 ? nullptr : pos.data_ptr<int>(), w.data_ptr<float>(), (int)T, (int)K, (int)H,
                                            cur_stream()));
 }
 
@@ -764,6 +764,32 @@ void gemm_decode_grouped(Tensor y, Tensor x, Tensor w, Tensor offsets, int64_t m
   HIP_OK(die::launch_gemm_decode(y.data_ptr(), y.stride(0), bf(x), x.stride(0), bf(w),
                                   (int)std::min<int64_t>(y.size(0), max_rows), (int)N, (int)K, (int)mode, (int)wr,
                                   (int)kc, 1, true, fz, cur_stream()));
+}
+
+// Expert products of a decode step from its routing (launchers.h): y [n, N], x [n / k or n, K] (pair i reads row i / k), w [E, N or 2 N, K],
+// ids [n] int32. False, with nothing launched, where there is no (wr, kc) tile of these sizes.
+bool gemm_decode_ids(Tensor y, Tensor x, Tensor w, Tensor ids, int64_t k, int64_t max_rows, int64_t act, double limit, double alpha, int64_t wr, int64_t kc) {
+  CHK_CUDA(x);
+  CHK_BF16(x);
+  CHK_BF16(w);
+  CHK_BF16(y);
+  CHK_CONTIG(w);
+  check_rows(x, "x");
+  check_rows(y, "y");
+  CHK_DTYPE(ids, at::kInt);
+  CHK_CONTIG(ids);
+  TORCH_CHECK(ids.device() == x.device() && w.device() == x.device() && y.device() == x.device(), "gemm_decode_ids: one device");
+  const bool gate = act >= die::MOE_ACT_SILU && act <= die::MOE_ACT_GELU;
+  TORCH_CHECK(act >= die::MOE_ACT_NONE && act <= die::MOE_ACT_RELU2, "gemm_decode_ids: activation");
+  TORCH_CHECK(w.dim() == 3 && w.size(2) == x.size(1) && w.size(1) == y.size(1) * (gate ? 2 : 1), "w [E, N or 2 N, K]");
+  TORCH_CHECK(k >= 1 && ids.numel() == y.size(0) && x.size(0) * k == y.size(0), "one row of y per id, one of x per k");
+  TORCH_CHECK(max_rows >= 1 && max_rows <= 128, "1 <= max_rows <= 128");
+  const hipError_t e = die::launch_gemm_decode_ids(y.data_ptr(), y.stride(0), bf(x), x.stride(0), bf(w), ids.data_ptr<int>(), (int)ids.numel(), (int)k,
+                                                   (int)max_rows, (int)w.size(0), (int)y.size(1), (int)x.size(1), (int)act, (float)limit, (float)alpha,
+                                                   (int)wr, (int)kc, cur_stream());
+  if (e == hipErrorInvalidValue) return false;
+  HIP_OK(e);
+  return true;
 }
 
 // Decode-step input advance (decode_step.hip), for multi-step decode windows.
@@ -1061,6 +1087,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("moe_route", &moe_route);
   m.def("moe_combine_residual", &moe_combine_residual);
   m.def("gemm_decode_grouped", &gemm_decode_grouped);
+  m.def("gemm_decode_ids", &gemm_decode_ids);
   m.def("fused_add_rms_norm_slab", &fused_add_rms_norm_slab);
   m.def("rope_and_cache_slab", &rope_and_cache_slab);
   m.def("car_alloc", &car_alloc, py::arg("bytes"), py::arg("uncached") = true);

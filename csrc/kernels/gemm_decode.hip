@@ -33,6 +33,7 @@
 #include "car_common.h"
 #include "common.h"
 #include "launchers.h"
+#include "moe_gemm.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -52,6 +53,15 @@ typedef __attribute__((ext_vector_type(4))) float f4;
 template <int AUX = 0>
 __device__ __forceinline__ void glds16(const void* src, char* lds_wave_base) {
   __builtin_amdgcn_global_load_lds((global_cvoid*)src, (lds_void*)lds_wave_base, 16, 0, AUX);
+}
+
+// the gates of the grouped product (moe_gemm.hip)
+template <int ACT> __device__ __forceinline__ float moe_gate(float g, float u, float limit, float alpha) {
+  if constexpr (ACT == MOE_ACT_SILU) return gated(g, g) * u;
+  if constexpr (ACT == MOE_ACT_GELU) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) * u;
+  g = fminf(g, limit);
+  u = fminf(fmaxf(u, -limit), limit);
+  return gated(g, alpha * g) * (u + 1.0f);
 }
 
 template <int N>
@@ -159,14 +169,17 @@ __device__ __forceinline__ uint32_t car_tile_exchange(f4 (&own)[EPT], const Gemm
 // KC = K elements per ring slot. XR = activation rows staged per chunk.
 // NT: weight pieces are loaded non-temporal (aux = 2): each weight byte is read once per step by one CU,
 // so it should not displace the activations / KV in L2 and MALL (MI355X_MICROARCH.md "nt-weights").
-template <int WR, int EPI, int S, bool NT, int KC, int XR, int SKC = 0>
+// EPI 5: gated activation of any kind of fz.act over W = [gate; up] rows, EPI 7: bf16 XW^T or its squared ReLU; both for the rows
+// `list` of the step's (token, slot) pairs (gemm_decode_ids_kernel): X row list[m] / fz.grp_k, Y row list[m].
+template <int WR, int EPI, int S, bool NT, int KC, int XR, int SKC = 0, class FZ = GemmDecodeFuse>
 __device__ __forceinline__ void gd_body(char* smem, void* Yv, int64_t ldy, const bf16_t* __restrict__ X, int64_t ldx,
                                         const bf16_t* __restrict__ W, int M, int N_out, int K,
-                                        const GemmDecodeFuse& fz, const int bx, const int by, const int ny) {
+                                        const FZ& fz, const int bx, const int by, const int ny, const int* list = nullptr) {
+  constexpr bool IDS = EPI == 5 || EPI == 7;
   constexpr int ROWB = KC * 2;                 // bytes per image row
   constexpr int CPR = KC / 8;                  // 16-byte chunks per row
   constexpr int RPP = 64 / CPR;                // rows per 1-KiB DMA piece
-  constexpr bool SILU = EPI == 1 || EPI == 4 || EPI == 6;
+  constexpr bool SILU = EPI == 1 || EPI == 4 || EPI == 6 || EPI == 5;
   constexpr int NO = SILU ? WR / 2 : WR;       // output columns per workgroup
   constexpr int SLOT = (WR + XR) * ROWB;       // bytes per ring slot
   constexpr int INSTR = (WR + XR) / RPP;       // 1-KiB DMA pieces per chunk
@@ -184,7 +197,9 @@ __device__ __forceinline__ void gd_body(char* smem, void* Yv, int64_t ldy, const
   static_assert(S * SLOT <= 160 * 1024, "ring exceeds LDS");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int r0 = 0;
-  if (fz.grp_off != nullptr) {
+  if constexpr (IDS) {
+    W += (int64_t)blockIdx.z * fz.grp_wstride;
+  } else if (fz.grp_off != nullptr) {
     // grouped (MoE) form: blockIdx.z = group; its rows of X/Y are [off[e], off[e+1]) of the
     // token-sorted activations, its weights those of expert e / grp_div (an expert with more rows than
     // the image is split into grp_div segments). Empty groups cost nothing.
@@ -221,7 +236,10 @@ __device__ __forceinline__ void gd_body(char* smem, void* Yv, int64_t ldy, const
       base = W + (int64_t)grow * K;
     } else {
       const int xr = min(row - WR, M - 1);
-      base = fz.grp_rows != nullptr ? X + (int64_t)(fz.grp_rows[r0 + xr] / fz.grp_k) * ldx : X + (int64_t)xr * ldx;
+      if constexpr (IDS)
+        base = X + (int64_t)(list[xr] / fz.grp_k) * ldx;
+      else
+        base = fz.grp_rows != nullptr ? X + (int64_t)(fz.grp_rows[r0 + xr] / fz.grp_k) * ldx : X + (int64_t)xr * ldx;
     }
     src[p] = base + k0 + lch * 8;
     if (row < WR && fz.tiled) {
@@ -329,6 +347,31 @@ __device__ __forceinline__ void gd_body(char* smem, void* Yv, int64_t ldy, const
       }
   __syncthreads();
   char* escr = smem + NRED * RR * WR * 4;  // epilogue scratch after the partials
+  if constexpr (IDS) {   // rows of 16-byte pieces, CPW lanes each
+    constexpr int CPW = NO / 8;
+    for (int m = tid / CPW; m < M; m += NTH / CPW) {
+      const int q = tid % CPW;
+      float v[8] = {}, u[8] = {};
+#pragma unroll
+      for (int w = 0; w < NRED; ++w)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          v[c] += red[(w * RR + m) * WR + 8 * q + c];
+          if (SILU) u[c] += red[(w * RR + m) * WR + NO + 8 * q + c];
+        }
+#pragma unroll
+      for (int c = 0; c < 8; ++c) {
+        if constexpr (SILU)
+          v[c] = fz.act == MOE_ACT_SILU ? moe_gate<MOE_ACT_SILU>(v[c], u[c], fz.limit, fz.alpha)
+                 : fz.act == MOE_ACT_GELU ? moe_gate<MOE_ACT_GELU>(v[c], u[c], fz.limit, fz.alpha)
+                                          : moe_gate<MOE_ACT_CLAMPED>(v[c], u[c], fz.limit, fz.alpha);
+        else if (fz.act == MOE_ACT_RELU2)
+          v[c] = fmaxf(v[c], 0.f) * fmaxf(v[c], 0.f);
+      }
+      *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(Yv) + (int64_t)list[m] * ldy + n0 + 8 * q) = pack8(v);
+    }
+    return;
+  }
   if constexpr (EPI == 3) {
     // split-K partial -> last arriver: h += sum of partials in slice order (bf16), per-tile row sums of squares.
     // Every thread owns EPT float4 groups (row m, columns j..j+3); its own workgroup's partial stays in
@@ -816,6 +859,120 @@ hipError_t launch_gemm_decode(void* Y, int64_t ldy, const bf16_t* X, int64_t ldx
   GD_TILE(64, 32)
   GD_TILE(128, 32)
 #undef GD_TILE
+  return hipErrorInvalidValue;
+}
+
+// ---- expert products of a decode step straight from its routing: no launch sorts the rows
+struct MoeDecodeFuse : GemmDecodeFuse {
+  const int* ids;      // [n] expert of every (token, slot) pair
+  int n, act;
+  float limit, alpha;
+};
+constexpr int IDS_MAX_ROWS = 128;
+// LDS of the kernel: the deepest ring of its images of 16 .. XR rows, then every wave's list
+constexpr size_t ids_ring(int wr, int xr, int kc) {
+  size_t most = 0;
+  for (int r = 16; r <= xr; r *= 2)
+    if (gd_valid(wr, r, kc) && gd_lds(wr, r, kc, ring_slots(wr, r, kc)) > most) most = gd_lds(wr, r, kc, ring_slots(wr, r, kc));
+  return most;
+}
+
+// blockIdx.z: the expert. Its rows are the pairs that name it, in order: every wave lists them for itself (a workgroup has
+// 100 KB and more of weights to read; a launch that sorts the pairs took 4.6 us). The activation image is the smallest that
+// holds them, not one for all rows of the step: it is read with every chunk of K and takes its part of the ring. Bound by the weights'
+// stream. Both products of 8 experts of 2048 x 2048, clamped gate, two of 10 choices (us; separate sort and activation, image of the
+// step's rows -> this): 32 tokens 33.8 + 18.1 + 9.5 -> 31.7 + 14.7, 128 tokens 55.9 + 27.3 + 9.5 -> 33.3 + 18.4; 32 experts of 4096 x 2048, four of them,
+// 64 tokens 149 + 157 -> 95 + 100 (4.6 TB/s).
+template <int WR, int EPI, int KC, int XR>
+__global__ void __launch_bounds__(NTH) gemm_decode_ids_kernel(void* __restrict__ Y, int64_t ldy, const bf16_t* __restrict__ X, int64_t ldx,
+                                                              const bf16_t* __restrict__ W, int N_out, int K, MoeDecodeFuse fz) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, e = blockIdx.z;
+  int* list = reinterpret_cast<int*>(smem + ids_ring(WR, XR, KC)) + wave * IDS_MAX_ROWS;
+  int M = 0;
+  for (int b0 = 0; b0 < fz.n; b0 += 256) {
+    int id[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int j = b0 + 64 * i + lane;
+      id[i] = j < fz.n ? fz.ids[j] : -1;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint64_t named = __builtin_amdgcn_ballot_w64(id[i] == e);
+      const int at = M + __builtin_amdgcn_mbcnt_hi((uint32_t)(named >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)named, 0));
+      if (id[i] == e && at < IDS_MAX_ROWS) list[at] = b0 + 64 * i + lane;
+      M += __builtin_popcountll(named);
+    }
+  }
+  M = min(M, XR);
+  if (M == 0) return;
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  auto run = [&](auto xr) {
+    constexpr int R = decltype(xr)::value;
+    if constexpr (R <= XR && gd_valid(WR, R, KC))
+      gd_body<WR, EPI, ring_slots(WR, R, KC), true, KC, R, 0, MoeDecodeFuse>(smem, Y, ldy, X, ldx, W, M, N_out, K, fz, blockIdx.x, 0, 1, list);
+  };
+  if (M <= 16 && gd_valid(WR, 16, KC)) run(IntC<16>{});
+  else if (M <= 32 && gd_valid(WR, 32, KC)) run(IntC<32>{});
+  else if (M <= 64 && gd_valid(WR, 64, KC)) run(IntC<64>{});
+  else run(IntC<128>{});
+}
+
+template <int WR, int EPI, int KC, int XR>
+static hipError_t launch_ids_xr(void* Y, int64_t ldy, const bf16_t* X, int64_t ldx, const bf16_t* W, int N, int K, const MoeDecodeFuse& fz,
+                                hipStream_t s) {
+  if constexpr (!gd_valid(WR, XR, KC)) {
+    return hipErrorInvalidValue;
+  } else {
+    constexpr size_t lds = ids_ring(WR, XR, KC) + 4 * IDS_MAX_ROWS * sizeof(int);
+    static_assert(lds <= 160 * 1024, "LDS of a compute unit");
+    auto* fn = gemm_decode_ids_kernel<WR, EPI, KC, XR>;
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(fn, dim3(N / (EPI == 5 ? WR / 2 : WR), 1, fz.grp_n), dim3(NTH), lds, s, Y, ldy, X, ldx, W, N, K, fz);
+    return hipGetLastError();
+  }
+}
+template <int WR, int EPI, int KC>
+static hipError_t launch_ids(void* Y, int64_t ldy, const bf16_t* X, int64_t ldx, const bf16_t* W, int M, int N, int K, const MoeDecodeFuse& fz,
+                             hipStream_t s) {
+  if (N % (EPI == 5 ? WR / 2 : WR) || K % KC) return hipErrorInvalidValue;
+  if (M <= 32) return launch_ids_xr<WR, EPI, KC, 32>(Y, ldy, X, ldx, W, N, K, fz, s);
+  if (M <= 64) return launch_ids_xr<WR, EPI, KC, 64>(Y, ldy, X, ldx, W, N, K, fz, s);
+  return launch_ids_xr<WR, EPI, KC, 128>(Y, ldy, X, ldx, W, N, K, fz, s);
+}
+
+hipError_t launch_gemm_decode_ids(void* Y, int64_t ldy, const bf16_t* X, int64_t ldx, const bf16_t* W, const int* ids, int n, int k, int max_rows,
+                                  int experts, int N, int K, int act, float limit, float alpha, int wr, int kc, hipStream_t s) {
+  if (n <= 0 || experts <= 0) return hipSuccess;
+  const bool gate = act >= MOE_ACT_SILU && act <= MOE_ACT_GELU;
+  if (k < 1 || max_rows < 1 || max_rows > IDS_MAX_ROWS || act < MOE_ACT_NONE || act > MOE_ACT_RELU2 ||
+      ((reinterpret_cast<uintptr_t>(Y) | reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(W) | (uintptr_t)(ldy * 2) | (uintptr_t)(ldx * 2)) & 15))
+    return hipErrorInvalidValue;
+  MoeDecodeFuse fz;
+  fz.grp_wstride = (int64_t)(gate ? 2 : 1) * N * K;
+  fz.grp_n = experts;
+  fz.grp_k = k;
+  fz.ids = ids;
+  fz.n = n;
+  fz.act = act;
+  fz.limit = limit;
+  fz.alpha = alpha;
+#define GD_IDS(WR, KC) \
+  if (wr == WR && kc == KC) \
+    return gate ? launch_ids<WR, 5, KC>(Y, ldy, X, ldx, W, max_rows, N, K, fz, s) : launch_ids<WR, 7, KC>(Y, ldy, X, ldx, W, max_rows, N, K, fz, s);
+  GD_IDS(32, 128)
+  GD_IDS(64, 128)
+  GD_IDS(128, 128)
+  GD_IDS(32, 256)
+  GD_IDS(64, 256)
+  GD_IDS(64, 64)
+  GD_IDS(128, 64)
+  GD_IDS(64, 32)
+  GD_IDS(128, 32)
+#undef GD_IDS
   return hipErrorInvalidValue;
 }
 

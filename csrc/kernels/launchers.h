@@ -175,6 +175,10 @@ struct GemmDecodeFuse {
 hipError_t launch_gemm_decode(void* Y, int64_t ldy, const bf16_t* X, int64_t ldx, const bf16_t* W, int M, int N,
                               int K, int mode, int wr, int kc, int sk, bool nt, const GemmDecodeFuse& fz,
                               hipStream_t s);
+// Expert products of a decode step from its routing: Y row i = act(X row i / k of W_ids[i]^T) for the pairs i < n with ids[i] < experts (others
+// are not written); no expert has more than max_rows (<= 128) of them. W [experts][N or 2 N][K]; act of moe_gemm.h; rows at 16-byte addresses.
+hipError_t launch_gemm_decode_ids(void* Y, int64_t ldy, const bf16_t* X, int64_t ldx, const bf16_t* W, const int* ids, int n, int k, int max_rows,
+                                  int experts, int N, int K, int act, float limit, float alpha, int wr, int kc, hipStream_t s);
 // consumers of fp32 split-K slabs [sk][rows][width]
 hipError_t launch_fused_add_rms_norm_slab(bf16_t* out, const float* slab, int sk, bf16_t* residual, const bf16_t* w,
                                           float eps, int rows, int hidden, int64_t out_stride, hipStream_t s);

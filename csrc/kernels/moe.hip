@@ -6,7 +6,7 @@
 //   moe_gather    — x_sorted[j] = x[sorted[j] / K]   (16-byte row copies);
 //   (the expert GEMMs themselves run on the expert-streaming grouped decode GEMM,
 //    gemm_decode.hip, or per expert on hipBLASLt for large prefills: src/ops moe_apply);
-//   moe_combine   — out[t] = sum_k w[t,k] * y_sorted[pos[t*K+k]].
+//   moe_combine   — out[t] = sum_k w[t,k] * y_sorted[pos[t*K+k]] (without pos: rows in pair order).
 #include "common.h"
 #include "launchers.h"
 
@@ -185,7 +185,7 @@ __global__ void __launch_bounds__(256) moe_combine_kernel(bf16_t* __restrict__ o
     for (int k = 0; k < K; ++k) {
       const float wk = w[(int64_t)t * K + k];
       float y[8];
-      unpack8(reinterpret_cast<const uint4*>(ys + (int64_t)pos[t * K + k] * H)[c], y);
+      unpack8(reinterpret_cast<const uint4*>(ys + (int64_t)(pos != nullptr ? pos[t * K + k] : t * K + k) * H)[c], y);
 #pragma unroll
       for (int q = 0; q < 8; ++q) acc[q] += wk * y[q];
     }
@@ -210,7 +210,7 @@ __global__ void __launch_bounds__(256) moe_combine_residual_kernel(float* __rest
     for (int k = 0; k < K; ++k) {
       const float wk = w[(int64_t)t * K + k];
       float y[8];
-      unpack8(reinterpret_cast<const uint4*>(ys + (int64_t)pos[t * K + k] * H)[c], y);
+      unpack8(reinterpret_cast<const uint4*>(ys + (int64_t)(pos != nullptr ? pos[t * K + k] : t * K + k) * H)[c], y);
 #pragma unroll
       for (int q = 0; q < 8; ++q) acc[q] += wk * y[q];
     }

@@ -845,6 +845,15 @@ def moe_apply(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: torch.Ten
     inter = w13.shape[1] // 2
     ids = ids.to(torch.int32).contiguous()
     w = w.float().contiguous()
+    if MOE_IDS_MIN_T <= t <= MOE_DECODE_MAX_T:
+        ys = (torch.zeros if groups > e else torch.empty)(t * k, hdim, dtype=x.dtype, device=x.device)
+        if decode_experts(kern, x.contiguous(), w13, w2, ids, k, t, MOE_SILU, ys=ys) is not None:
+            if residual is not None:
+                kern.moe_combine_residual(ssp, residual, ys, _NO_ROWS(x.device), w)
+                return residual
+            out = torch.empty_like(x, memory_format=torch.contiguous_format)
+            kern.moe_combine(out, ys, _NO_ROWS(x.device), w)
+            return out
     offsets, sorted_idx, pos = moe_align(ids, groups)
     # rows of the extra groups are never computed: zero them so that weight 0 x row stays 0
     ys = (torch.zeros if groups > e else torch.empty)(t * k, hdim, dtype=x.dtype, device=x.device)
@@ -906,6 +915,9 @@ def moe_apply(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: torch.Ten
 
 
 MOE_LIBRARY_MIN_TOKENS = 256
+# Tokens from which decode steps take the products of unsorted rows, whose activation image goes with an expert's rows instead of the step's
+# (eight experts of 4096 x 14336, both products, us, sorted / unsorted: 32 tokens 459 / 470 without the sort's 5, 128 tokens 732 / 536)
+MOE_IDS_MIN_T = 33
 _NO_ROWS_CACHE: dict = {}
 
 
@@ -941,6 +953,6 @@ def _moe_down_wr(hdim: int, inter: int) -> int:
 
 
 # dtype-generic ops (bf16 / fp32 storage) of the src/_Cmix extension
-from .mix import (ACT_CLAMPED, ACT_SILU, MOE_SILU, gated_act, grouped_experts, latent_attn, latent_kv_write, latent_qkv_prep,  # noqa: E402,F401
+from .mix import (ACT_CLAMPED, ACT_SILU, MOE_SILU, decode_experts, gated_act, grouped_experts, latent_attn, latent_kv_write, latent_qkv_prep,  # noqa: E402,F401
                   mix_available,
                   moe_input_scaled, post_norm_residual, rms_norm_ext, rope_inv_freq, route_sigmoid_topk)

@@ -225,6 +225,45 @@ def grouped_experts(kern, x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, 
     return kern.moe_gemm(ys, a, w2, offsets, None, 1, None, MOE_NONE, 0.0, 0.0)
 
 
+def _ids_tile(n: int, k: int, gate: bool, t: int, pairs: int) -> Optional[Tuple[int, int]]:
+    """(weight rows of a workgroup, K of a ring slot) of the expert products of a decode step, or None where none divides N
+    and K. 64 x 256: of 9 tiles the best or within 3 % for 2 - 64 tokens (8 experts of 2048 x 2048 at 32 tokens, us, gated / plain
+    product: 32 x 128 36.9 / 18.3, 64 x 128 33.2 / 15.9, 64 x 256 31.7 / 14.7, 128 x 128 30.0 / 17.3); above 64 rows its activation image
+    leaves no ring. Where 64 rows give less than a workgroup to every second compute unit, 32 (2 pairs: 9.0 / 7.5)."""
+    wide = ((64, 256), (64, 128)) if t <= 64 else ((64, 128), (64, 64))
+    narrow = ((32, 256), (32, 128)) if t <= 64 else ((32, 128),)
+    few = pairs * (n // (32 if gate else 64)) <= 128
+    for wr, kc in narrow + wide if few else wide + narrow:
+        if k % kc == 0 and n % (wr // 2 if gate else wr) == 0:
+            return wr, kc
+    return None
+
+
+def decode_experts(ck, x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: torch.Tensor, k: int, t: int, act: int,
+                   limit: float = 0.0, alpha: float = 0.0, ys: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """The experts of a decode step of t <= 128 tokens in two launches: row i of the result (``ys``, or new) is
+    W2 act(W13 x[i / k]) of expert ids[i], for the (token, slot) pairs i whose id is an expert's; other rows are not
+    written. Every workgroup lists its expert's rows from ``ids``, so nothing sorts them. None, with nothing done, where the
+    sizes do not tile or the operands are not contiguous at 16-byte addresses."""
+    e, h, f = w2.shape
+    gate = MOE_SILU <= act <= MOE_GELU
+    n = t * ids.shape[-1]
+    if x.dtype != torch.bfloat16 or t > 128 or not (w13.is_contiguous() and w2.is_contiguous() and x.is_contiguous()):
+        return None
+    if any(m.data_ptr() % 16 for m in (x, w13, w2)) or (ys is not None and ys.data_ptr() % 16):
+        return None
+    one, two = _ids_tile(f, h, gate, t, min(n, e * t)), _ids_tile(h, f, False, t, min(n, e * t))
+    if one is None or two is None:
+        return None
+    flat = ids.reshape(-1).contiguous()
+    a = torch.empty(n, f, dtype=x.dtype, device=x.device)
+    ys = torch.empty(n, h, dtype=x.dtype, device=x.device) if ys is None else ys
+    if not ck.gemm_decode_ids(a, x, w13, flat, k, t, act, limit, alpha, *one):
+        return None
+    assert ck.gemm_decode_ids(ys, a, w2, flat, 1, t, MOE_NONE, 0.0, 0.0, *two)
+    return ys
+
+
 # (token, expert) rows up to which the experts' weights are gathered per row for two batched GEMMs (no host
 # read, hipGraph-capturable: decode steps of widths that the expert-streaming product does not tile); above it the rows
 # sorted by expert run as one grouped product per matrix, or, in fp32, at widths that it does not tile and with strided
@@ -264,10 +303,16 @@ def moe_input_scaled(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: to
         return out
 
     if x.dtype == torch.bfloat16 and t <= 128:
-        # decode-sized steps: the framework's expert-streaming grouped GEMM (every routed expert's weights
-        # streamed once, SiLU * up fused; no host read, hipGraph-capturable) on the scaled, expert-sorted rows
+        # decode-sized steps: the framework's expert-streaming products (every routed expert's weights
+        # streamed once, SiLU * up fused; no host read, hipGraph-capturable) on the scaled rows, unsorted where they tile
         from src import ops
 
+        if ops.native_available() and ids.dtype == torch.int32 and n > 0:
+            xs = torch.empty(n, h, dtype=x.dtype, device=x.device)
+            kern.gather_scaled(xs, x, None, w, k)
+            ys = decode_experts(ops._kern(), xs, w13, w2, ids, 1, t, MOE_SILU)
+            if ys is not None:
+                return finish(ys, None)
         tiles = ops._moe_decode_tiles(h, w13.shape[1] // 2, t) if ops.native_available() else None
         if tiles is not None:
             ck = ops._kern()
@@ -407,11 +452,15 @@ def moe_output_weighted(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w:
         return finish(torch.empty(0, h, dtype=x.dtype, device=x.device), None)
     buckets = max(e, int(n_route))
     if x.dtype == torch.bfloat16 and t <= 128:
-        # decode-sized steps: the framework's expert-streaming grouped GEMM (every routed expert's weights streamed
-        # once; rows gathered in expert-sorted order by the kernel; no host read, hipGraph-capturable). Identity
-        # entries sort behind the last real expert and run nothing.
+        # decode-sized steps: the framework's expert-streaming products (every routed expert's weights streamed
+        # once; no host read, hipGraph-capturable), of unsorted rows where they tile, else gathered in expert-sorted order. Identity
+        # entries run nothing (sorted, they come behind the last real expert).
         from src import ops
 
+        if ops.native_available() and ids.dtype == torch.int32 and n > 0 and kind in _MOE_ACT:
+            ys = decode_experts(ops._kern(), x, w13, w2, ids, k, t, _MOE_ACT[kind], limit, alpha)
+            if ys is not None:
+                return finish(ys, None)
         tiles = None
         if ops.native_available() and h % 32 == 0 and w2.shape[2] % 32 == 0:
             try:
