@@ -450,8 +450,8 @@ const char* sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, O
     const int64_t tiles = S * kv_heads * ((rows + rows_wg - 1) / rows_wg);
     ns = std::min<int64_t>({(int64_t)16, 2048 / std::max<int64_t>(1, tiles), (bound + 63) / 64});
     if (ns > 1 && a.impl == 0 && !gate.has_value() && die::sink_attn_fits_rows(a)) {
-      const bool broad = vdim > 128;
-      const SplitTimes t = {broad ? 1.2 : 0.85, broad ? 3.0 : 4.0, 10.0, broad ? 1.9 : 1.1, 2.0};
+      const bool broad = vdim > 128, shaped = a.softcap > 0.f || a.slopes != nullptr || a.bias != nullptr;
+      const SplitTimes t = {broad ? (shaped ? 1.5 : 1.2) : (shaped ? 1.1 : 0.85), broad ? 3.0 : 4.0, 10.0, broad ? 1.9 : 1.1, 2.0};
       ns = best_splits(t, ns, bound, S * kv_heads * ((rows + 63) / 64), tiles, at::cuda::getCurrentDeviceProperties()->multiProcessorCount, T * heads * vdim * 4);
     }
     if (ns > 1) a.chunk = (int)((((bound + ns - 1) / ns) + 31) / 32 * 32);

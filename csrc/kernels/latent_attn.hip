@@ -731,6 +731,8 @@ __global__ void __launch_bounds__(256, 3) latent_attn_mfma_rq_kernel(LatentAttnA
 // rows, and the next ones are read ahead of a group's products. Two waves share 32 rows: both form the scores and weights, each its half
 // of the value columns, so that sums and queries take 64 + 72 registers at rank 256 and two waves share a SIMD. (Whole rows
 // per wave spill with two waves per SIMD; with one its sums move between the two kinds of registers: 337 us of 16 x 1024 rows against 324.)
+// The weights enter the products in two bf16 parts: split keys, which such steps had before, round relative to every split's own
+// largest weight, and whole keys with rounded weights were up to 4 % further from 64 bits.
 template <int NDB, int NROT> struct LatentTile {
   static constexpr int KCH = 4 * NDB + 2 * NROT, NPF = (32 * KCH + 255) / 256, BYTES = NPF * 256 * 16;
   static constexpr int X = KCH % 16 == 0 ? 16 : KCH % 8 == 0 ? 8 : KCH % 4 == 0 ? 4 : 2;   // pieces that change places
@@ -936,8 +938,13 @@ __global__ void __launch_bounds__(256, 2) latent_attn_wide_kernel(LatentAttnArgs
       const int u = g / (NO / VG), d0 = g % (NO / VG) * VG, e = 8 * (u & 1);
       const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, make_uint4(pack2(sc[e], sc[e + 1]), pack2(sc[e + 2], sc[e + 3]),
                                                                   pack2(sc[e + 4], sc[e + 5]), pack2(sc[e + 6], sc[e + 7])));
+      const uint4 h = __builtin_bit_cast(uint4, pf);
+      auto rest = [&](int i, uint32_t b) { return pack2(sc[e + i] - __uint_as_float(b << 16), sc[e + i + 1] - __uint_as_float(b & 0xffff0000u)); };
+      const bf16x8_t pl = __builtin_bit_cast(bf16x8_t, make_uint4(rest(0, h.x), rest(2, h.y), rest(4, h.z), rest(6, h.w)));
       if (g + 1 < NV) read_v(g + 1);
       __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int d = 0; d < VG; ++d) o[d0 + d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[g & 1][d], pl, o[d0 + d], 0, 0, 0);
 #pragma unroll
       for (int d = 0; d < VG; ++d) o[d0 + d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[g & 1][d], pf, o[d0 + d], 0, 0, 0);
     }
@@ -993,7 +1000,7 @@ inline bool mfma_rq_fits(const LatentAttnArgs& a) {
 template <int NDB, int NROT> hipError_t launch_rows(const LatentAttnArgs& a, hipStream_t s) {
   const int64_t wgs = ((int64_t)a.max_q * a.heads + 63) / 64 * a.num_seqs;
   const int64_t keys = (int64_t)a.bt_stride * a.block_size;
-  return wgs <= 2 * (int64_t)num_cus() && keys >= 96 && a.scale > 0.f ? launch_wide<NDB, NROT>(a, s) : launch_mfma_rq<NDB, NROT>(a, s);
+  return wgs <= 2 * (int64_t)num_cus() && keys > 64 && a.scale > 0.f ? launch_wide<NDB, NROT>(a, s) : launch_mfma_rq<NDB, NROT>(a, s);
 }
 template <int NDB> hipError_t launch_mfma_rq_rot(const LatentAttnArgs& a, hipStream_t s) {
   switch (a.sh.rot_dim) {

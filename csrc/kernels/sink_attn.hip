@@ -678,7 +678,7 @@ template <int NK, int NV> struct RowTile {
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) const void global_cvoid;
 
-template <int NK, int NV, bool SIG>
+template <int NK, int NV, bool SIG, bool FINE>
 __global__ void __launch_bounds__(256, NV <= 8 ? 4 : 3) sink_attn_rows_kernel(SinkAttnArgs a) {
   using Z = RowTile<NK, NV>;
   constexpr int KCH = Z::KCH, D = 32 * NK, DV = 16 * NV, roww = D + DV;
@@ -859,6 +859,13 @@ __global__ void __launch_bounds__(256, NV <= 8 ? 4 : 3) sink_attn_rows_kernel(Si
     }
     const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, make_uint4(pack2(sc[0][0], sc[0][1]), pack2(sc[0][2], sc[0][3]),
                                                                 pack2(sc[1][0], sc[1][1]), pack2(sc[1][2], sc[1][3])));
+    bf16x8_t pl = {};   // what the rounding left
+    if constexpr (FINE) {
+      const uint4 h = __builtin_bit_cast(uint4, pf);
+      auto rest = [](float x, float y, uint32_t b) { return pack2(x - __uint_as_float(b << 16), y - __uint_as_float(b & 0xffff0000u)); };
+      pl = __builtin_bit_cast(bf16x8_t, make_uint4(rest(sc[0][0], sc[0][1], h.x), rest(sc[0][2], sc[0][3], h.y), rest(sc[1][0], sc[1][1], h.z),
+                                                   rest(sc[1][2], sc[1][3], h.w)));
+    }
     if (!SIG && __builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {   // wave-uniform
       asm volatile("" : "+v"(alpha));                                // (not multiplied ahead of the condition)
 #pragma unroll
@@ -873,6 +880,7 @@ __global__ void __launch_bounds__(256, NV <= 8 ? 4 : 3) sink_attn_rows_kernel(Si
       const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(at + 256 * KCH));
       const bf16x8_t vf = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
       o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf, o[db], 0, 0, 0);
+      if constexpr (FINE) o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pl, o[db], 0, 0, 0);
     }
   }
   // results through LDS (tiles and table are done with), so that whole rows are written 16 bytes a lane
@@ -1519,10 +1527,21 @@ template <int NKC> hipError_t launch_decode_v(const SinkAttnArgs& a, hipStream_t
   return a.vdim <= 128 ? launch_decode_r<NKC, 16>(a, s) : launch_decode_r<NKC, 32>(a, s);
 }
 
+// cached keys of a sequence that a step can see
+inline int64_t keys_of(const SinkAttnArgs& a) {
+  int64_t keys = (int64_t)a.bt_stride * a.block_size;
+  if (a.window > 0) keys = std::min<int64_t>(keys, (int64_t)a.window + a.max_q);
+  return a.seg > 0 ? std::min<int64_t>(keys, (int64_t)a.seg + a.max_q) : keys;
+}
+// FINE: the weights enter the products in two bf16 parts, for steps of up to four row tiles of 128 per CU over more than one of 64 keys. The
+// kernel with split keys, which ran them before, rounds relative to every split's own largest weight, which is then exact: whole
+// keys with rounded weights are up to 6 % further from 64 bits (5 x 77 rows behind 300: 2.18e-3, whole 2.31e-3, in two parts 1.66e-3).
 template <int NK, int NV> hipError_t launch_rows(const SinkAttnArgs& a, hipStream_t s) {
   const int64_t rows = (int64_t)a.max_q * (a.heads / a.kv_heads);
+  const bool fine = (rows + 127) / 128 * a.num_seqs * a.kv_heads <= 4 * (int64_t)num_cus() && keys_of(a) > 64;
   const dim3 grid((unsigned)((rows + 63) / 64), (unsigned)a.num_seqs, (unsigned)a.kv_heads);
-  auto* fn = a.sigmoid ? sink_attn_rows_kernel<NK, NV, true> : sink_attn_rows_kernel<NK, NV, false>;
+  auto* fn = a.sigmoid ? (fine ? sink_attn_rows_kernel<NK, NV, true, true> : sink_attn_rows_kernel<NK, NV, true, false>)
+                       : (fine ? sink_attn_rows_kernel<NK, NV, false, true> : sink_attn_rows_kernel<NK, NV, false, false>);
   hipLaunchKernelGGL(fn, grid, dim3(256), (RowTile<NK, NV>::LDS), s, a);
   return hipGetLastError();
 }
@@ -1558,10 +1577,7 @@ inline bool rows_takes(const SinkAttnArgs& a) { return (a.ws_o == nullptr || a.n
 // heads 57 / 54; 2 x 1000 37 / 38; 16 x 250 23.0 / 24.3; capped 16 x 500 of 32 heads 121 / 135.
 inline bool wide_takes(const SinkAttnArgs& a) {
   const int64_t rows = (int64_t)a.max_q * (a.heads / a.kv_heads), wgs = (rows + 127) / 128 * a.num_seqs * a.kv_heads;
-  int64_t keys = (int64_t)a.bt_stride * a.block_size;
-  if (a.window > 0) keys = std::min<int64_t>(keys, (int64_t)a.window + a.max_q);
-  if (a.seg > 0) keys = std::min<int64_t>(keys, (int64_t)a.seg + a.max_q);
-  return a.softcap <= 0.f && a.slopes == nullptr && a.bias == nullptr && a.scale > 0.f && wgs >= 4 * (int64_t)num_cus() && keys >= 512;
+  return a.softcap <= 0.f && a.slopes == nullptr && a.bias == nullptr && a.scale > 0.f && wgs > 4 * (int64_t)num_cus() && keys_of(a) >= 512;
 }
 
 inline bool decode_ok(const SinkAttnArgs& a) {
