@@ -94,3 +94,25 @@ def test_results_at_any_8_bytes(cuda):
     assert form == "tiles" and at(0, 0)[0] == "rows"
     form, got = at(4, 0)
     assert form == "tiles" and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("lens,window", [((64, 1, 33, 2, 63, 31, 17, 48) * 8 + (5, 64, 9), 0), ((200, 333, 1, 140, 257, 90, 310, 16, 128), 70)])
+def test_sequences_not_in_eights(cuda, lens, window):
+    """The row tiles of a number of sequences that is no multiple of 8 are dealt in another order: every row once, the longest sequence's too."""
+    torch.manual_seed(len(lens))
+    rank, rot, heads, bs, scale = 256, 32, 32, 16, 0.08
+    S, T, need = len(lens), sum(lens), -(-max(lens) // bs)
+    cache = torch.randn(1 + 3 * need, bs, rank + rot, device=cuda).to(torch.bfloat16)
+    bt = torch.randint(0, 1 + 3 * need, (S, need), device=cuda, dtype=torch.int32)
+    cu = torch.tensor([0, *lens], device=cuda).cumsum(0).int()
+    pos = torch.cat([torch.arange(n) for n in lens]).to(cuda)
+    ctx = torch.tensor(lens, device=cuda, dtype=torch.int32)
+    q_lat = torch.randn(heads, T, rank, device=cuda).to(torch.bfloat16)
+    q = torch.randn(T, heads * (rot + 6), device=cuda).to(torch.bfloat16)
+    inv, sink = ops.rope_inv_freq(10000.0, rot, cuda)[: rot // 2], torch.randn(heads, device=cuda) + 1
+    args = (q_lat, q, 6, cache, bt, cu, ctx, pos, sink, max(lens), window, scale, rot, inv)
+    want, got = ops.latent_attn(*args, impl=1).float(), ops.latent_attn(*args).float()
+    e = scale * 2 ** -9 * float(q.view(T, heads, -1)[..., 6:].float().norm(dim=-1).max() * cache[..., rank:].float().norm(dim=-1).max())
+    top = float(cache[..., :rank].float().abs().max())
+    assert ((got - want).abs() <= (2 ** -9 + 2 * e * 2.71828 ** (2 * e)) * top + 2 ** -7 * want.abs()).all()
+    assert ((got - want).norm() / want.norm()).item() < 2 ** -7
