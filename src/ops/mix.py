@@ -201,9 +201,10 @@ _MOE_ACT = {ACT_SILU: MOE_SILU, ACT_CLAMPED: MOE_CLAMPED, ACT_GELU_TANH: MOE_GEL
 
 
 # Rows per expert and elements of an expert's matrix from which a library GEMM pair per expert, behind a host read of the offsets,
-# is faster than the grouped product (eight experts of 4096 x 14336, us, library / grouped: 1024 rows 3019 / 3005, 1500 rows
-# 3985 / 4177, 2048 rows 5118 / 5600, 4096 rows 9735 / 11003; of 4096 x 2048, 2048 rows 1718 / 1774, 2500 rows 2171 / 2135)
-GROUPED_MAX_ROWS, GROUPED_ANY_ROWS_SIZE = 1280, 1 << 25
+# is faster than the grouped product (eight experts, us, library / grouped; 4096 x 14336: 1024 rows 3131 / 2907, 1280 rows 3663 / 3470,
+# 1500 rows 3910 / 3799, 2048 rows 5332 / 5469, 4096 rows 10262 / 10633; smaller experts never: 4096 x 4096, 2048 rows 1745 / 1609,
+# 4096 rows 3491 / 3145; 4096 x 2048, 8192 rows 3378 / 3200; 2048 x 2048, 4096 rows 1088 / 906)
+GROUPED_MAX_ROWS, GROUPED_ANY_ROWS_SIZE = 1792, 1 << 25
 
 
 def grouped_experts(kern, x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, offsets: torch.Tensor, sorted_idx: torch.Tensor,
