@@ -491,9 +491,10 @@ __device__ __forceinline__ void tile_of(int& bx, int& s) {
 // pieces lies in LDS as the DMA writes it, without gaps; the pieces of a row are exchanged (XOR) so that 16 consecutive rows' reads
 // of one piece fall on all banks, and so do the transposed reads of 8 rows by two pieces (the number is rotated for those: by the plain
 // row number pairs of rows shared banks, a quarter of the kernel's cycles).
-// Bound by LDS reads (34 KB per wave and tile at 128 bytes a cycle: 120 us of the 253 below). 16 sequences of 1024 rows, 16 heads,
+// Bound by LDS reads (34 KB per wave and tile at 128 bytes a cycle: 120 us of the 246 below). 16 sequences of 1024 rows, 16 heads,
 // rank 256 + 32: 32 rows per wave, one wave per SIMD, tiles through registers, looked up piece by piece behind divisions: 518 us;
-// the same with DMA and the next tile's scores under the softmax 370; this 253 (570 TFLOP/s).
+// the same with DMA and the next tile's scores under the softmax 370; this 246 (585 TFLOP/s; 250 with the queries
+// loaded behind the first tile, where 24 - 100 rows of 20 and more sequences took 3 % longer too).
 template <int NDB, int NROT> struct RqTile {
   static constexpr int KCH = 4 * NDB + 2 * NROT, NPF = (MKT * KCH + 255) / 256, BYTES = NPF * 4096;
   static constexpr int G = KCH % 16 == 0 ? 16 : KCH % 8 == 0 ? 8 : KCH % 4 == 0 ? 4 : 2;   // rows r and r + 16 / G share banks
@@ -530,6 +531,36 @@ __global__ void __launch_bounds__(256, 3) latent_attn_mfma_rq_kernel(LatentAttnA
   const int jhi = min(p_last, ctx - 1);
   const bf16_t* cache = reinterpret_cast<const bf16_t*>(a.cache);
   const int li = lane & 15, lg = lane >> 4;
+
+  const int wrow = row0 + wave * 16, myrow = wrow + li;
+  const bool rok = myrow < nrows, wave_live = wrow < nrows, all_rows = wrow + 15 < nrows;
+  const int64_t tq = rok ? q0 + myrow / H : q0;
+  const int hq = rok ? myrow % H : 0;
+  const int64_t orow = (int64_t)hq * a.total_q + tq;
+  const int prow = rok ? (int)a.positions[tq] : -1;
+  const int pw_min = wave_live ? (int)a.positions[q0 + wrow / H] : 0;
+  const int pw_max = wave_live ? (int)a.positions[q0 + min(wrow + 15, nrows - 1) / H] : 0;
+  // this lane's query fragments: qf[k] = Q[row][32 k + 8 lg .. + 8]; an odd NROT leaves 16 columns, of which the lane has 4. (Rows
+  // beyond the last repeat the first; every load is unconditional, so that all are in flight together, and beside the table's.)
+  bf16x8_t qf[NK > 0 ? NK : 1];
+  short4_t qt = {};
+  const bf16_t* qlat = reinterpret_cast<const bf16_t*>(a.q_lat) + orow * R;
+#pragma unroll
+  for (int k = 0; k < NLAT; ++k) qf[k] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(qlat + 32 * k + 8 * lg));
+  constexpr int E = NROT % 2 == 0 ? 8 : 4, NS = (NROT + 1) / 2;
+  bf16_t qr[NS > 0 ? NS : 1][E];
+  float fr[NS > 0 ? NS : 1][E / 2];
+  if constexpr (NROT > 0) {
+    const bf16_t* qp = reinterpret_cast<const bf16_t*>(a.q_rot) + tq * a.q_stride + (int64_t)hq * a.q_hstride + E * lg;
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+#pragma unroll
+      for (int e = 0; e < E; ++e) qr[k][e] = qp[32 * k + e];
+#pragma unroll
+      for (int i = 0; i < E / 2; ++i)
+        fr[k][i] = a.sh.rot_pairs > 0 ? a.sh.inv_freq[min(16 * k + E / 2 * lg + i, a.sh.rot_pairs - 1)] : 0.f;
+    }
+  }
 
   // Block-table entries of the workgroup's keys in LDS (TABLE at a time), so that a tile's loads depend on LDS reads alone
   const int* bt = a.block_tables + (int64_t)s * a.bt_stride;
@@ -572,34 +603,7 @@ __global__ void __launch_bounds__(256, 3) latent_attn_mfma_rq_kernel(LatentAttnA
   const int nt = jhi < jlo ? 0 : (jhi - jlo) / MKT + 1;
   if (nt > 0) fetch(jlo, 0);
 
-  const int wrow = row0 + wave * 16, myrow = wrow + li;
-  const bool rok = myrow < nrows, wave_live = wrow < nrows, all_rows = wrow + 15 < nrows;
-  const int64_t tq = rok ? q0 + myrow / H : q0;
-  const int hq = rok ? myrow % H : 0;
-  const int64_t orow = (int64_t)hq * a.total_q + tq;
-  const int prow = rok ? (int)a.positions[tq] : -1;
-  const int pw_min = wave_live ? (int)a.positions[q0 + wrow / H] : 0;
-  const int pw_max = wave_live ? (int)a.positions[q0 + min(wrow + 15, nrows - 1) / H] : 0;
-  // this lane's query fragments: qf[k] = Q[row][32 k + 8 lg .. + 8]; an odd NROT leaves 16 columns, of which the lane has 4. (Rows
-  // beyond the last repeat the first; every load is unconditional, so that all are in flight together.)
-  bf16x8_t qf[NK > 0 ? NK : 1];
-  short4_t qt = {};
-  const bf16_t* qlat = reinterpret_cast<const bf16_t*>(a.q_lat) + orow * R;
-#pragma unroll
-  for (int k = 0; k < NLAT; ++k) qf[k] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(qlat + 32 * k + 8 * lg));
   if constexpr (NROT > 0) {
-    constexpr int E = NROT % 2 == 0 ? 8 : 4, NS = (NROT + 1) / 2;
-    bf16_t qr[NS][E];
-    float fr[NS][E / 2];
-    const bf16_t* qp = reinterpret_cast<const bf16_t*>(a.q_rot) + tq * a.q_stride + (int64_t)hq * a.q_hstride + E * lg;
-#pragma unroll
-    for (int k = 0; k < NS; ++k) {
-#pragma unroll
-      for (int e = 0; e < E; ++e) qr[k][e] = qp[32 * k + e];
-#pragma unroll
-      for (int i = 0; i < E / 2; ++i)
-        fr[k][i] = a.sh.rot_pairs > 0 ? a.sh.inv_freq[min(16 * k + E / 2 * lg + i, a.sh.rot_pairs - 1)] : 0.f;
-    }
 #pragma unroll
     for (int k = 0; k < NS; ++k) {
       float f[8] = {};
