@@ -15,9 +15,12 @@ struct SplitTimes {
 // read fp32 results of every row; chosen only to have 2048 workgroups in flight they took 1.5 - 5 times as long as no split
 // (attention over 8 x 500 rows, 16 heads of 128 + 128: 80 us in 8 splits, 22 in one kernel; 16 x 250 of 32 heads: 112 / 23). They stay for few
 // rows behind many keys (16 rows behind 8000: 29 / 220) and are halved in between (1000 behind 2000: 16 splits 87, 4 63, none 78).
-inline int64_t best_splits(const SplitTimes& t, int64_t most, int64_t keys, int64_t one_wgs, int64_t split_wgs, int64_t cus, int64_t split_bytes) {
+// `one_keys`: the keys that a row tile of the kernel without splits walks, fewer than `keys` where a window follows the rows (1500 rows with a
+// window of 1024, capped scores: 89 us in the two splits that the whole portion's keys would call for, 51 in one kernel).
+inline int64_t best_splits(const SplitTimes& t, int64_t most, int64_t keys, int64_t one_keys, int64_t one_wgs, int64_t split_wgs, int64_t cus,
+                           int64_t split_bytes) {
   const double tiles = (double)keys / 32.0, c = (double)cus;
-  double least = 4.0 + t.one_tile * tiles * std::max(1.0, (double)one_wgs / (t.one_resident * c));
+  double least = 4.0 + t.one_tile * (double)one_keys / 32.0 * std::max(1.0, (double)one_wgs / (t.one_resident * c));
   int64_t best = 1;
   for (int64_t n = most; n > 1; n /= 2) {
     const double turns = std::max(1.0, (double)(split_wgs * n) / (t.split_resident * c));

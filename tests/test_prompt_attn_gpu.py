@@ -134,3 +134,14 @@ def test_keys_are_split_behind_few_rows_only(cuda, monkeypatch, seqs, rows, past
     want, got = seq.sink_attn(*args, impl=1).float(), seq.sink_attn(*args).float()
     assert forms == ["fma", form]
     assert ((got - want).norm() / want.norm()).item() < 2 ** -7
+
+
+@pytest.mark.parametrize("rows,past,cap,vdim,form", [(700, 900, 0.0, 128, "rows"), (700, 900, 30.0, 256, "rows"), (40, 4000, 30.0, 128, "split")])
+def test_a_window_bounds_the_keys_that_splits_are_weighed_by(cuda, monkeypatch, rows, past, cap, vdim, form):
+    torch.manual_seed(rows)
+    forms = _forms(monkeypatch)
+    data = _ragged(cuda, [rows], [past], 16, 4, 128, vdim, 16)
+    args, kw = (*data, None, None, rows, 16, 4, 128, vdim, 500 if rows > 64 else 2000, 128 ** -0.5), {"softcap": cap} if cap else {}
+    want, got = seq.sink_attn(*args, impl=1, **kw).float(), seq.sink_attn(*args, **kw).float()
+    assert forms == ["fma", form]
+    assert ((got - want).norm() / want.norm()).item() < 2 ** -7
