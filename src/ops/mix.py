@@ -261,7 +261,8 @@ def decode_experts(ck, x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids
     ys = torch.empty(n, h, dtype=x.dtype, device=x.device) if ys is None else ys
     if not ck.gemm_decode_ids(a, x, w13, flat, k, t, act, limit, alpha, *one):
         return None
-    assert ck.gemm_decode_ids(ys, a, w2, flat, 1, t, MOE_NONE, 0.0, 0.0, *two)
+    if not ck.gemm_decode_ids(ys, a, w2, flat, 1, t, MOE_NONE, 0.0, 0.0, *two):
+        raise RuntimeError(f"experts of a decode step: no {two} tile for {h} x {f} at {t} tokens")
     return ys
 
 
