@@ -845,19 +845,17 @@ def moe_apply(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: torch.Ten
     inter = w13.shape[1] // 2
     ids = ids.to(torch.int32).contiguous()
     w = w.float().contiguous()
-    if MOE_IDS_MIN_T <= t <= MOE_DECODE_MAX_T:
-        ys = (torch.zeros if groups > e else torch.empty)(t * k, hdim, dtype=x.dtype, device=x.device)
-        if decode_experts(kern, x.contiguous(), w13, w2, ids, k, t, MOE_SILU, ys=ys) is not None:
-            if residual is not None:
-                kern.moe_combine_residual(ssp, residual, ys, _NO_ROWS(x.device), w)
-                return residual
-            out = torch.empty_like(x, memory_format=torch.contiguous_format)
-            kern.moe_combine(out, ys, _NO_ROWS(x.device), w)
-            return out
-    offsets, sorted_idx, pos = moe_align(ids, groups)
+    x = x.contiguous()
     # rows of the extra groups are never computed: zero them so that weight 0 x row stays 0
     ys = (torch.zeros if groups > e else torch.empty)(t * k, hdim, dtype=x.dtype, device=x.device)
-    x = x.contiguous()
+    if MOE_IDS_MIN_T <= t <= MOE_DECODE_MAX_T and decode_experts(kern, x, w13, w2, ids, k, t, MOE_SILU, ys=ys) is not None:
+        if residual is not None:
+            kern.moe_combine_residual(ssp, residual, ys, _NO_ROWS(x.device), w)
+            return residual
+        out = torch.empty_like(x)
+        kern.moe_combine(out, ys, _NO_ROWS(x.device), w)
+        return out
+    offsets, sorted_idx, pos = moe_align(ids, groups)
     tiles = _moe_decode_tiles(hdim, inter, t)
     if tiles is not None and t <= MOE_DECODE_MAX_T:
         # decode: every expert's weights streamed once by the weight-streaming kernel, its routed

@@ -240,22 +240,30 @@ def _ids_tile(n: int, k: int, gate: bool, t: int, pairs: int) -> Optional[Tuple[
     return None
 
 
+def decode_tiles(w13: torch.Tensor, w2: torch.Tensor, t: int, n: int, act: int, *rows: torch.Tensor) -> Optional[Tuple[Tuple[int, int], Tuple[int, int]]]:
+    """The :func:`_ids_tile` of both products of :func:`decode_experts` for n (token, slot) pairs of t tokens, or None where the sizes do
+    not tile or a matrix (or ``rows``, activations that exist already) is not contiguous at a 16-byte address."""
+    e, h, f = w2.shape
+    if t > 128 or any(not m.is_contiguous() or m.data_ptr() % 16 for m in (w13, w2, *rows)):
+        return None
+    one, two = _ids_tile(f, h, MOE_SILU <= act <= MOE_GELU, t, min(n, e * t)), _ids_tile(h, f, False, t, min(n, e * t))
+    return None if one is None or two is None else (one, two)
+
+
 def decode_experts(ck, x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, ids: torch.Tensor, k: int, t: int, act: int,
                    limit: float = 0.0, alpha: float = 0.0, ys: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """The experts of a decode step of t <= 128 tokens in two launches: row i of the result (``ys``, or new) is
     W2 act(W13 x[i / k]) of expert ids[i], for the (token, slot) pairs i whose id is an expert's; other rows are not
-    written. Every workgroup lists its expert's rows from ``ids``, so nothing sorts them. None, with nothing done, where the
-    sizes do not tile or the operands are not contiguous at 16-byte addresses."""
+    written. Every workgroup lists its expert's rows from ``ids``, so nothing sorts them. None, with nothing done, where
+    :func:`decode_tiles` has no tiles."""
     e, h, f = w2.shape
-    gate = MOE_SILU <= act <= MOE_GELU
     n = t * ids.shape[-1]
-    if x.dtype != torch.bfloat16 or t > 128 or not (w13.is_contiguous() and w2.is_contiguous() and x.is_contiguous()):
+    if x.dtype != torch.bfloat16:
         return None
-    if any(m.data_ptr() % 16 for m in (x, w13, w2)) or (ys is not None and ys.data_ptr() % 16):
+    tiles = decode_tiles(w13, w2, t, n, act, *((x,) if ys is None else (x, ys)))
+    if tiles is None:
         return None
-    one, two = _ids_tile(f, h, gate, t, min(n, e * t)), _ids_tile(h, f, False, t, min(n, e * t))
-    if one is None or two is None:
-        return None
+    one, two = tiles
     flat = ids.reshape(-1).contiguous()
     a = torch.empty(n, f, dtype=x.dtype, device=x.device)
     ys = torch.empty(n, h, dtype=x.dtype, device=x.device) if ys is None else ys
@@ -309,7 +317,7 @@ def moe_input_scaled(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: to
         # streamed once, SiLU * up fused; no host read, hipGraph-capturable) on the scaled rows, unsorted where they tile
         from src import ops
 
-        if ops.native_available() and ids.dtype == torch.int32 and n > 0:
+        if ops.native_available() and ids.dtype == torch.int32 and n > 0 and decode_tiles(w13, w2, t, n, MOE_SILU) is not None:
             xs = torch.empty(n, h, dtype=x.dtype, device=x.device)
             kern.gather_scaled(xs, x, None, w, k)
             ys = decode_experts(ops._kern(), xs, w13, w2, ids, 1, t, MOE_SILU)

@@ -89,3 +89,32 @@ def test_mixtures(cuda, t, H, ff, E, k, n_route):
     assert ((got.cpu().double() - want).norm() / want.norm()).item() < 2 ** -7
     got = ops.moe_apply(*dev(x, w13, w2, w, real), E)
     assert ((got.cpu().double() - plain).norm() / plain.norm()).item() < 2 ** -7
+
+
+@pytest.mark.parametrize("t", [3, 40, 100])
+@pytest.mark.parametrize("H,ff", [(512, 256), (320, 96)])
+def test_rows_and_results_are_formed_once(cuda, monkeypatch, t, H, ff):
+    """Whether or not the widths tile, the rows are gathered once and one buffer takes the experts' results."""
+    E, k, bf = 4, 2, torch.bfloat16
+    x, w13, w2 = (torch.randn(*s, device=cuda).to(bf) for s in ((t, H), (E, 2 * ff, H), (E, H, ff)))
+    w, ids = torch.rand(t, k, device=cuda), torch.randint(0, E, (t, k), device=cuda, dtype=torch.int32)
+
+    class Counting:
+        gathers = 0
+
+        def __init__(self, kern):
+            self.kern = kern
+
+        def __getattr__(self, name):
+            Counting.gathers += name == "gather_scaled"
+            return getattr(self.kern, name)
+
+    kern = Counting(mix._kern())
+    monkeypatch.setattr(mix, "_kern", lambda: kern)
+    mix.moe_input_scaled(x, w13, w2, w, ids)
+    assert Counting.gathers == 1
+    made = []
+    zeros = torch.zeros
+    monkeypatch.setattr(torch, "zeros", lambda *a, **kw: (made.append(a), zeros(*a, **kw))[1])
+    ops.moe_apply(x, w13, w2, w, ids, E + 1)
+    assert made.count((t * k, H)) == 1
