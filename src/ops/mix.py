@@ -317,13 +317,19 @@ def moe_input_scaled(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: to
         # streamed once, SiLU * up fused; no host read, hipGraph-capturable) on the scaled rows, unsorted where they tile
         from src import ops
 
-        if ops.native_available() and ids.dtype == torch.int32 and n > 0 and decode_tiles(w13, w2, t, n, MOE_SILU) is not None:
+        tiles = ops._moe_decode_tiles(h, w13.shape[1] // 2, t) if ops.native_available() else None
+        # The sorted form has the activation in its first product too, and so only the sort to lose. It keeps few tokens of large experts whose
+        # gate's halves of weight rows are a multiple of 4 KiB long: its tiles of 32 rows read such weights faster than the unsorted form's
+        # of 64 (8 experts, us, sorted / unsorted: 4096 x 4096, 2 tokens 80 / 83, 8 tokens 140 / 160, 32 tokens 159 / 175; 4096 x 2048, 8 tokens 90 / 94,
+        # 32 tokens 97 / 103; their first product of 6144 x 2048 alone 74 / 80; but 4096 x 1024 59 / 59 and 64 / 63, 2048 x 2048 60 / 56 and 68 / 61,
+        # 3072 x 2048 70 / 67 and 83 / 76).
+        sort = tiles is not None and tiles[0][0] <= 32 and h >= 4096 and h % 2048 == 0 and w2.shape[2] >= 2048 and t <= 32 and n >= 4
+        if ops.native_available() and ids.dtype == torch.int32 and n > 0 and not sort and decode_tiles(w13, w2, t, n, MOE_SILU) is not None:
             xs = torch.empty(n, h, dtype=x.dtype, device=x.device)
             kern.gather_scaled(xs, x, None, w, k)
             ys = decode_experts(ops._kern(), xs, w13, w2, ids, 1, t, MOE_SILU)
             if ys is not None:
                 return finish(ys, None)
-        tiles = ops._moe_decode_tiles(h, w13.shape[1] // 2, t) if ops.native_available() else None
         if tiles is not None:
             ck = ops._kern()
             (wr1, kc1), (wr2, kc2) = tiles

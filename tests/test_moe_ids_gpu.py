@@ -118,3 +118,33 @@ def test_rows_and_results_are_formed_once(cuda, monkeypatch, t, H, ff):
     monkeypatch.setattr(torch, "zeros", lambda *a, **kw: (made.append(a), zeros(*a, **kw))[1])
     ops.moe_apply(x, w13, w2, w, ids, E + 1)
     assert made.count((t * k, H)) == 1
+
+
+@pytest.mark.parametrize("H,ff,t,form", [(4096, 2048, 1, "ids"), (4096, 2048, 2, "grouped"), (4096, 2048, 32, "grouped"), (4096, 2048, 33, "ids"),
+                                         (6144, 2048, 8, "grouped"), (4096, 1024, 8, "ids"), (2048, 2048, 32, "ids"), (5120, 2048, 8, "ids")])
+def test_scaled_mixtures_whose_sorted_form_is_faster_keep_it(cuda, monkeypatch, H, ff, t, form):
+    """Large gated experts with weight rows of a multiple of 4 KiB, 2 to 32 tokens: sorted rows, tiles of 32 weight rows."""
+    E, k, bf, ran = 3, 2, torch.bfloat16, []
+    g = torch.Generator(device=cuda).manual_seed(H + t)
+    x, w13, w2 = (torch.randn(*s, generator=g, device=cuda).to(bf) for s in ((t, H), (E, 2 * ff, H), (E, H, ff)))
+    w13, w2 = w13 * 2.0 ** -6, w2 * 2.0 ** -6
+    w, ids = torch.rand(t, k, generator=g, device=cuda) + 0.1, torch.rand(t, E, generator=g, device=cuda).argsort(1)[:, :k].int().contiguous()
+
+    class Recording:
+        def __init__(self, kern):
+            self.kern = kern
+
+        def __getattr__(self, name):
+            ran.append(name)
+            return getattr(self.kern, name)
+
+    kern = Recording(ops._kern())
+    monkeypatch.setattr(ops, "_kern", lambda: kern)
+    got = mix.moe_input_scaled(x, w13, w2, w, ids)
+    assert ran == [f"gemm_decode_{form}"] * 2
+    want = torch.zeros(t, H, dtype=torch.float64, device=cuda)
+    for e in range(E):
+        for j in range(k):
+            rows = (ids[:, j] == e).nonzero().flatten()
+            want[rows] += _act((x[rows].double() * w[rows, j:j + 1].double()) @ w13[e].double().T, mix.MOE_SILU) @ w2[e].double().T
+    assert ((got.double() - want).norm() / want.norm()).item() < 2 ** -7
