@@ -237,6 +237,10 @@ template <bool F32> hipError_t launch_fma(const SinkAttnArgs& a, hipStream_t s) 
 constexpr int MKT = 32;
 constexpr int BT_LDS_MAX = 2048;
 constexpr float LAZY = 8.0f;
+// Weights that enter the products in two bf16 parts are taken 1 + 2^-8 times, and the sums divided by that: the second part is then positive
+// wherever the weight is (a rounding leaves up to 2^-9 of it, of either sign), so that an infinite value stays what it is: zero times it
+// would be NaN, and a negative part of the other sign. (From weights of 2^-124 on; the part is no bf16 number below.)
+constexpr float OVER = 1.0f + 0x1p-8f;
 // keys per stage; whether the queries live in registers (else in LDS)
 template <int NW, int NKC> constexpr int stage_keys() { return NW == 4 && NKC <= 16 ? 64 : MKT; }
 template <int NDB, int NW, int NKC> constexpr bool q_in_regs() { return NKC <= 16 && (NW == 4 || NDB <= 4); }
@@ -859,10 +863,10 @@ __global__ void __launch_bounds__(256, NV <= 8 ? 4 : 3) sink_attn_rows_kernel(Si
     }
     const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, make_uint4(pack2(sc[0][0], sc[0][1]), pack2(sc[0][2], sc[0][3]),
                                                                 pack2(sc[1][0], sc[1][1]), pack2(sc[1][2], sc[1][3])));
-    bf16x8_t pl = {};   // what the rounding left
+    bf16x8_t pl = {};   // what the rounding left, and 2^-8 of the weight (OVER)
     if constexpr (FINE) {
       const uint4 h = __builtin_bit_cast(uint4, pf);
-      auto rest = [](float x, float y, uint32_t b) { return pack2(x - __uint_as_float(b << 16), y - __uint_as_float(b & 0xffff0000u)); };
+      auto rest = [](float x, float y, uint32_t b) { return pack2(fmaf(x, OVER, -__uint_as_float(b << 16)), fmaf(y, OVER, -__uint_as_float(b & 0xffff0000u))); };
       pl = __builtin_bit_cast(bf16x8_t, make_uint4(rest(sc[0][0], sc[0][1], h.x), rest(sc[0][2], sc[0][3], h.y), rest(sc[1][0], sc[1][1], h.z),
                                                    rest(sc[1][2], sc[1][3], h.w)));
     }
@@ -886,7 +890,8 @@ __global__ void __launch_bounds__(256, NV <= 8 ? 4 : 3) sink_attn_rows_kernel(Si
   // results through LDS (tiles and table are done with), so that whole rows are written 16 bytes a lane
   __syncthreads();
   l = xor16_sum(xor32_sum(l));
-  const float inv = SIG ? 1.0f : (l > 0.f ? 1.0f / l : 0.f);
+  if constexpr (FINE) l *= OVER;
+  const float inv = SIG ? (FINE ? 1.0f / OVER : 1.0f) : (l > 0.f ? 1.0f / l : 0.f);
   char* os = smem_raw + wave * 16 * Z::OP;
 #pragma unroll
   for (int db = 0; db < NV; ++db)

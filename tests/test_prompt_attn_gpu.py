@@ -145,3 +145,29 @@ def test_a_window_bounds_the_keys_that_splits_are_weighed_by(cuda, monkeypatch, 
     want, got = seq.sink_attn(*args, impl=1, **kw).float(), seq.sink_attn(*args, **kw).float()
     assert forms == ["fma", form]
     assert ((got - want).norm() / want.norm()).item() < 2 ** -7
+
+
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (64, 256), (128, 128)])
+@pytest.mark.parametrize("style", ["", "sink", "sigmoid", "capped"])
+def test_infinite_values_stay_infinite(cuda, monkeypatch, dim, vdim, style):
+    """A value of either infinity at a key that every row sees, where weights go in two parts: the same infinity, and the other columns as
+    they are without it."""
+    torch.manual_seed(dim + vdim)
+    forms, heads, groups, bs = _forms(monkeypatch), 16, 4, 16
+    q, cache, bt, cu, ctx, pos = _ragged(cuda, [150, 77, 99], [0, 30, 8], bs, groups, dim, vdim, heads)
+    bt = torch.arange(bt.numel(), device=cuda, dtype=torch.int32).view_as(bt)
+    cache = torch.randn(bt.numel(), bs, groups * (dim + vdim), device=cuda).to(torch.bfloat16)
+    sink, kw = (torch.randn(heads, device=cuda) if style == "sink" else None), {}
+    if style == "sigmoid":
+        kw = dict(sigmoid=True, head_bias=torch.randn(heads, device=cuda) - 5)
+    if style == "capped":
+        kw = dict(softcap=20.0)
+    tail = (bt, cu, ctx, pos, sink, None, 150, heads, groups, dim, vdim, 0, dim ** -0.5)
+    plain = seq.sink_attn(q, cache, *tail, **kw).view(-1, heads, vdim)
+    first = cache.view(-1, groups, bs, dim + vdim)[:, :, 0]   # of every block; of block bt[s, 0] the sequence's token 0
+    first[bt[:, 0].long(), :, dim + 3], first[bt[:, 0].long(), :, dim + 40] = float("inf"), float("-inf")
+    got = seq.sink_attn(q, cache, *tail, **kw).view(-1, heads, vdim)
+    assert forms == ["rows", "rows"]
+    assert (got[:, :, 3] == float("inf")).all() and (got[:, :, 40] == float("-inf")).all()
+    rest = [c for c in range(vdim) if c not in (3, 40)]
+    assert torch.equal(got[:, :, rest], plain[:, :, rest])
