@@ -458,8 +458,10 @@ const char* sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, O
       int64_t seen = bound;   // of a row tile: what it sees before its first row, its rows' tokens, a part of a key tile
       if (window > 0) seen = std::min<int64_t>(seen, window + 64 / qpg + 31);
       if (seg > 0) seen = std::min<int64_t>(seen, seg + 64 / qpg + 31);
-      ns = best_splits(t, ns, bound, seen, S * kv_heads * ((rows + 63) / 64), tiles, at::cuda::getCurrentDeviceProperties()->multiProcessorCount,
+      const int64_t most = ns;
+      ns = best_splits(t, most, bound, seen, S * kv_heads * ((rows + 63) / 64), tiles, at::cuda::getCurrentDeviceProperties()->multiProcessorCount,
                        T * heads * vdim * 4);
+      a.fine = ns < most;   // (a split rounds relative to its own largest weight: fewer of them were up to 5 % further from 64 bits)
     }
     if (ns > 1) a.chunk = (int)((((bound + ns - 1) / ns) + 31) / 32 * 32);
   }

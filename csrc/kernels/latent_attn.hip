@@ -182,8 +182,14 @@ constexpr int MKT = 32;
 constexpr int BT_LDS_MAX = 2048;  // block-table entries staged per workgroup (else read from global memory)
 typedef __attribute__((address_space(3))) short4_t lds_short4;
 typedef __attribute__((ext_vector_type(8))) short short8_t;
+// What the rounding of the weights x, y to b left. (Zero and negative as well: an infinite latent column makes its key's score infinite or NaN,
+// and so its weight 0 or NaN, before any of it counts.)
+__device__ __forceinline__ uint32_t rest2(float x, float y, uint32_t b) {
+  return pack2(x - __uint_as_float(b << 16), y - __uint_as_float(b & 0xffff0000u));
+}
 
-template <int NDB, int NW>
+// FINE: the weights enter the products in two bf16 parts (LatentAttnArgs::fine)
+template <int NDB, int NW, bool FINE>
 __global__ void __launch_bounds__(64 * NW) latent_attn_mfma_kernel(LatentAttnArgs a, int KP) {
   constexpr int ROWS = 32 * NW, NT = 64 * NW;
   constexpr int NPF = (MKT * (4 * NDB + 16) + NT - 1) / NT;  // 16-byte chunks of a key tile per thread (rot_dim <= 128)
@@ -348,7 +354,7 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_mfma_kernel(LatentAttnArg
     sum = xor32_sum(sum);
     l = l * alpha + sum;
     m = mn;
-    bf16x8_t pfr[2];
+    bf16x8_t pfr[2], plr[2];
 #pragma unroll
     for (int s2 = 0; s2 < 2; ++s2) {
       uint4 w;
@@ -357,6 +363,10 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_mfma_kernel(LatentAttnArg
       w.z = pack2(sc[8 * s2 + 4], sc[8 * s2 + 5]);
       w.w = pack2(sc[8 * s2 + 6], sc[8 * s2 + 7]);
       pfr[s2] = __builtin_bit_cast(bf16x8_t, w);
+      if constexpr (FINE) {
+        auto rest = [&](int r, uint32_t b) { return rest2(sc[8 * s2 + r], sc[8 * s2 + r + 1], b); };
+        plr[s2] = __builtin_bit_cast(bf16x8_t, make_uint4(rest(0, w.x), rest(2, w.y), rest(4, w.z), rest(6, w.w)));
+      }
     }
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
@@ -371,6 +381,7 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_mfma_kernel(LatentAttnArg
         const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(a0 + 8 * pitchB));
         const short8_t a8 = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
         o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a8), pfr[s2], o[db], 0, 0, 0);
+        if constexpr (FINE) o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a8), plr[s2], o[db], 0, 0, 0);
       }
     }
   }
@@ -430,14 +441,17 @@ inline size_t mfma_lds_bytes(int kp, int nw) {
 }
 
 template <int NDB, int NW> hipError_t launch_mfma(const LatentAttnArgs& a, hipStream_t s) {
-  static bool attr_set = false;
-  auto* fn = latent_attn_mfma_kernel<NDB, NW>;
+  static bool attr_set[2] = {};
+  auto* fn = latent_attn_mfma_kernel<NDB, NW, false>;
+  if constexpr (NW == 4 && (NDB == 2 || NDB == 4 || NDB == 8))
+    if (a.fine) fn = latent_attn_mfma_kernel<NDB, NW, true>;
   const int kp = a.sh.rank + a.sh.rot_dim + 8;
-  if (!attr_set) {
+  bool& set = attr_set[fn != latent_attn_mfma_kernel<NDB, NW, false>];
+  if (!set) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        144 * 1024);
     if (e != hipSuccess) return e;
-    attr_set = true;
+    set = true;
   }
   const dim3 grid((unsigned)(((int64_t)a.max_q * a.heads + 32 * NW - 1) / (32 * NW)), (unsigned)a.num_seqs,
                   (unsigned)max(1, a.nsplit));
@@ -946,7 +960,7 @@ __global__ void __launch_bounds__(256, 2) latent_attn_wide_kernel(LatentAttnArgs
       const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, make_uint4(pack2(sc[e], sc[e + 1]), pack2(sc[e + 2], sc[e + 3]),
                                                                   pack2(sc[e + 4], sc[e + 5]), pack2(sc[e + 6], sc[e + 7])));
       const uint4 h = __builtin_bit_cast(uint4, pf);
-      auto rest = [&](int i, uint32_t b) { return pack2(sc[e + i] - __uint_as_float(b << 16), sc[e + i + 1] - __uint_as_float(b & 0xffff0000u)); };
+      auto rest = [&](int i, uint32_t b) { return rest2(sc[e + i], sc[e + i + 1], b); };
       const bf16x8_t pl = __builtin_bit_cast(bf16x8_t, make_uint4(rest(0, h.x), rest(2, h.y), rest(4, h.z), rest(6, h.w)));
       if (g + 1 < NV) read_v(g + 1);
       __builtin_amdgcn_sched_barrier(0);

@@ -120,6 +120,7 @@ struct LatentAttnArgs {
   float* ws_o;
   float* ws_ml;
   int nsplit, chunk;
+  bool fine = false;      // split keys of prompt steps (latent_attn_fits_rows): weights in two bf16 parts
   int impl;               // 0: matrix cores where they apply, else the FMA form; 1: FMA form; 2: matrix cores or fail;
                           // 3: as 2, but never the register-query variant (A/B)
 };

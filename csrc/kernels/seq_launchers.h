@@ -165,6 +165,7 @@ struct SinkAttnArgs {
   float* ws_o;
   float* ws_ml;
   int nsplit, chunk;
+  bool fine = false;      // split keys of prompt steps (sink_attn_fits_rows), softmax: weights in two bf16 parts, as in steps without splits
   // epilogue of the decode-step and the split-key forms (sink_attn_fuses_gate): with gate [T, H] (bf16, row stride gstride)
   // head h's output, turned by -positions[t] * out_inv_freq[i] over pairs (i, i + vdim / 2) if out_inv_freq is given, times
   // gate_mult * sigmoid(gate[t, h]). These forms write rows of stride ostride; the others contiguous rows and no gate.

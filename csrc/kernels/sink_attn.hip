@@ -241,13 +241,18 @@ constexpr float LAZY = 8.0f;
 // wherever the weight is (a rounding leaves up to 2^-9 of it, of either sign), so that an infinite value stays what it is: zero times it
 // would be NaN, and a negative part of the other sign. (From weights of 2^-124 on; the part is no bf16 number below.)
 constexpr float OVER = 1.0f + 0x1p-8f;
+// second parts of the weights x, y, whose first ones are in b
+__device__ __forceinline__ uint32_t rest2(float x, float y, uint32_t b) {
+  return pack2(fmaf(x, OVER, -__uint_as_float(b << 16)), fmaf(y, OVER, -__uint_as_float(b & 0xffff0000u)));
+}
 // keys per stage; whether the queries live in registers (else in LDS)
 template <int NW, int NKC> constexpr int stage_keys() { return NW == 4 && NKC <= 16 ? 64 : MKT; }
 template <int NDB, int NW, int NKC> constexpr bool q_in_regs() { return NKC <= 16 && (NW == 4 || NDB <= 4); }
 typedef __attribute__((address_space(3))) short4_t lds_short4;
 typedef __attribute__((ext_vector_type(8))) short short8_t;
 
-template <int NDB, int NW, int NKC, bool SIG>
+// FINE: the weights enter the products in two bf16 parts (SinkAttnArgs::fine)
+template <int NDB, int NW, int NKC, bool SIG, bool FINE>
 __global__ void __launch_bounds__(64 * NW, NW == 4 && NKC <= 16 && NDB <= 4 ? 2 : 1) sink_attn_mfma_kernel(SinkAttnArgs a, int KP, int QP, int QR, int BTC,
                                                                 float* ws_o, float* ws_ml, int nsplit, int chunk) {
   constexpr int ROWS = 32 * NW, NT = 64 * NW, STG = stage_keys<NW, NKC>();
@@ -548,7 +553,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 && NKC <= 16 && NDB <= 4 ? 2 
         l = l * alpha + sum;
         m = mn;
       }
-      bf16x8_t pfr[2];
+      bf16x8_t pfr[2], plr[2];
 #pragma unroll
       for (int s2 = 0; s2 < 2; ++s2) {
         uint4 w;
@@ -557,6 +562,10 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 && NKC <= 16 && NDB <= 4 ? 2 
         w.z = pack2(sc[8 * s2 + 4], sc[8 * s2 + 5]);
         w.w = pack2(sc[8 * s2 + 6], sc[8 * s2 + 7]);
         pfr[s2] = __builtin_bit_cast(bf16x8_t, w);
+        if constexpr (FINE) {
+          auto rest = [&](int r, uint32_t b) { return rest2(sc[8 * s2 + r], sc[8 * s2 + r + 1], b); };
+          plr[s2] = __builtin_bit_cast(bf16x8_t, make_uint4(rest(0, w.x), rest(2, w.y), rest(4, w.z), rest(6, w.w)));
+        }
       }
 #pragma unroll
       for (int db = 0; db < NDB; ++db) {
@@ -571,10 +580,12 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 && NKC <= 16 && NDB <= 4 ? 2 
           const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(a0 + 8 * pitchB));
           const short8_t a8 = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
           o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a8), pfr[s2], o[db], 0, 0, 0);
+          if constexpr (FINE) o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a8), plr[s2], o[db], 0, 0, 0);
         }
       }
     }
   }
+  if constexpr (FINE) l *= OVER;
   if (NW > 1 && nsplit <= 1) {
     // whole rows of 16-byte pieces through LDS: straight from the accumulators every store would touch 32 rows
     const float inv = SIG ? 1.0f : (l > 0.f ? 1.0f / l : 0.f);
@@ -866,9 +877,8 @@ __global__ void __launch_bounds__(256, NV <= 8 ? 4 : 3) sink_attn_rows_kernel(Si
     bf16x8_t pl = {};   // what the rounding left, and 2^-8 of the weight (OVER)
     if constexpr (FINE) {
       const uint4 h = __builtin_bit_cast(uint4, pf);
-      auto rest = [](float x, float y, uint32_t b) { return pack2(fmaf(x, OVER, -__uint_as_float(b << 16)), fmaf(y, OVER, -__uint_as_float(b & 0xffff0000u))); };
-      pl = __builtin_bit_cast(bf16x8_t, make_uint4(rest(sc[0][0], sc[0][1], h.x), rest(sc[0][2], sc[0][3], h.y), rest(sc[1][0], sc[1][1], h.z),
-                                                   rest(sc[1][2], sc[1][3], h.w)));
+      pl = __builtin_bit_cast(bf16x8_t, make_uint4(rest2(sc[0][0], sc[0][1], h.x), rest2(sc[0][2], sc[0][3], h.y), rest2(sc[1][0], sc[1][1], h.z),
+                                                   rest2(sc[1][2], sc[1][3], h.w)));
     }
     if (!SIG && __builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {   // wave-uniform
       asm volatile("" : "+v"(alpha));                                // (not multiplied ahead of the condition)
@@ -1450,7 +1460,9 @@ __global__ void __launch_bounds__(128) sink_attn_merge_kernel(SinkAttnArgs a) {
 }
 
 template <int NDB, int NW, int NKC, bool SIG> hipError_t launch_mfma(const SinkAttnArgs& a, hipStream_t s) {
-  auto* fn = sink_attn_mfma_kernel<NDB, NW, NKC, SIG>;
+  auto* fn = sink_attn_mfma_kernel<NDB, NW, NKC, SIG, false>;
+  if constexpr (!SIG && NW == 4 && NKC <= 16 && (NDB == 2 || NDB == 4 || NDB == 8))
+    if (a.fine) fn = sink_attn_mfma_kernel<NDB, NW, NKC, SIG, true>;
   const int kp = a.dim + 32 * NDB + 8, qp = a.dim + 8;
   const int qpg0 = a.heads / a.kv_heads;
   const int qr = q_in_regs<NDB, NW, NKC>() ? 0 : (NW == 1 ? min(32, a.max_q * qpg0 + 1) : 32 * NW);
@@ -1460,12 +1472,13 @@ template <int NDB, int NW, int NKC, bool SIG> hipError_t launch_mfma(const SinkA
   const size_t lds = sizeof(bf16_t) * ((size_t)qr * qp + (size_t)(2 * stage_keys<NW, NKC>() + 1) * kp) + sizeof(int) * btc;
   if (lds > 150 * 1024) return hipErrorInvalidValue;
   if (lds > 48 * 1024) {  // only then: the limit is raised per function, and a raised limit is not free
-    static size_t raised = 0;
-    if (lds > raised) {
+    static size_t raised[2] = {};
+    size_t& own = raised[fn != sink_attn_mfma_kernel<NDB, NW, NKC, SIG, false>];
+    if (lds > own) {
       hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
                                          (int)lds);
       if (e != hipSuccess) return e;
-      raised = lds;
+      own = lds;
     }
   }
   const int qpg = a.heads / a.kv_heads;

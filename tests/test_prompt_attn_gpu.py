@@ -171,3 +171,23 @@ def test_infinite_values_stay_infinite(cuda, monkeypatch, dim, vdim, style):
     assert (got[:, :, 3] == float("inf")).all() and (got[:, :, 40] == float("-inf")).all()
     rest = [c for c in range(vdim) if c not in (3, 40)]
     assert torch.equal(got[:, :, rest], plain[:, :, rest])
+
+
+@pytest.mark.parametrize("style,vdim", [("", 128), ("sink", 64), ("capped", 128), ("bias", 256), ("sigmoid", 128)])
+def test_fewer_splits_are_no_further_from_64_bits(cuda, monkeypatch, style, vdim):
+    """Steps whose keys the rule cuts into fewer splits than there could be: their weights go in two bf16 parts (softmax), so that the results
+    are no further from float64 than with all splits, which impl 2 takes. (1 % for the roundings of the results themselves.)"""
+    torch.manual_seed(vdim)
+    heads, groups, dim = 16, 4, 128 if vdim > 64 else 64
+    q, cache, bt, cu, ctx, pos = _ragged(cuda, [150, 140, 133], [1500, 1400, 1333], 16, groups, dim, vdim, heads)
+    sink, bias = (torch.randn(heads, device=cuda) if style == "sink" else None), (torch.randn(64, heads, device=cuda) if style == "bias" else None)
+    kw = dict(softcap=20.0) if style == "capped" else dict(sigmoid=True, head_bias=torch.randn(heads, device=cuda) - 5) if style == "sigmoid" else {}
+    call = lambda impl: seq.sink_attn(q, cache, bt, cu, ctx, pos, sink, bias, 150, heads, groups, dim, vdim, 0, dim ** -0.5, impl, **kw)
+    forms = _forms(monkeypatch)
+    got, all_splits = call(0), call(2)
+    assert forms == ["split", "split"]
+    cpu = lambda x: x if x is None else x.cpu()
+    want = seq.sink_attn(*(cpu(x) for x in (q.float(), cache.float(), bt, cu, ctx, pos, sink, bias)), 150, heads, groups, dim, vdim, 0, dim ** -0.5,
+                         **{k: cpu(v) if torch.is_tensor(v) else v for k, v in kw.items()})
+    error = lambda x: ((x.cpu().double() - want.double()).norm() / want.double().norm()).item()
+    assert error(got) <= 1.01 * error(all_splits)
