@@ -490,7 +490,9 @@ std::string latent_attn(Tensor out, Tensor q_lat, Tensor q, int64_t rot_off, Ten
     if (ns > 1 && a.impl == 0 && die::latent_attn_fits_rows(a)) {
       const int64_t seen = window > 0 ? std::min<int64_t>(bound, window + (H + 63) / H + 31) : bound;   // of a tile of 64 rows
       const int64_t most = ns;
-      ns = best_splits({1.3, 2.0, 14.0, 3.5, 1.0}, most, bound, seen, S * ((max_q * H + 63) / 64), tiles, at::cuda::getCurrentDeviceProperties()->multiProcessorCount, T * H * rank * 4);
+      // (times fitted to 524 random steps of rank 256 + 32 in 1 to 16 splits)
+      ns = best_splits({0.9, 1.16, 2.2, 13.9, 3.25, 1.3}, most, bound, seen, S * ((max_q * H + 63) / 64), tiles,
+                       at::cuda::getCurrentDeviceProperties()->multiProcessorCount, T * H * rank * 4);
       a.fine = ns < most;   // (a split rounds relative to its own largest weight)
     }
     if (ns > 1) {

@@ -451,10 +451,9 @@ const char* sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, O
     ns = std::min<int64_t>({(int64_t)16, 2048 / std::max<int64_t>(1, tiles), (bound + 63) / 64});
     if (ns > 1 && a.impl == 0 && !gate.has_value() && die::sink_attn_fits_rows(a)) {
       const bool broad = vdim > 128, shaped = a.softcap > 0.f || a.slopes != nullptr || a.bias != nullptr;
-      // (over 16 shapes each of full, windowed, capped and biased scores at both widths, 1 to 16 splits measured: the choice is within 0.8 % of
-      // the best in the mean, 28 % at worst)
-      const SplitTimes t = broad ? SplitTimes{shaped ? 1.7 : 1.2, 3.0, 10.0, shaped ? 2.8 : 1.9, 2.0}
-                                 : SplitTimes{shaped ? 1.3 : 0.85, 4.0, 10.0, shaped ? 1.8 : 1.1, 2.0};
+      // (fitted to the times of 1978 random steps, six kinds of scores, in 1 to 16 splits)
+      const SplitTimes t = broad ? (shaped ? SplitTimes{5.0, 2.33, 3.5, 11.2, 4.14, 1.0} : SplitTimes{3.2, 1.93, 3.7, 4.4, 5.32, 2.8})
+                                 : (shaped ? SplitTimes{8.9, 2.51, 2.5, 13.7, 5.93, 2.0} : SplitTimes{4.5, 1.23, 2.1, 7.6, 2.82, 2.8});
       int64_t seen = bound;   // of a row tile: what it sees before its first row, its rows' tokens, a part of a key tile
       if (window > 0) seen = std::min<int64_t>(seen, window + 64 / qpg + 31);
       if (seg > 0) seen = std::min<int64_t>(seen, seg + 64 / qpg + 31);

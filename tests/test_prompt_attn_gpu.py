@@ -125,7 +125,8 @@ def test_many_rows_of_long_keys(cuda, monkeypatch, dim, vdim, heads, groups, bs,
     assert ((got - want).norm() / want.norm()).item() < 2 ** -7
 
 
-@pytest.mark.parametrize("seqs,rows,past,form", [(2, 300, 0, "rows"), (8, 128, 0, "rows"), (1, 64, 30, "rows"), (1, 20, 5000, "split"), (3, 9, 1000, "split")])
+@pytest.mark.parametrize("seqs,rows,past,form", [(2, 300, 0, "rows"), (8, 128, 0, "rows"), (1, 64, 30, "rows"), (1, 20, 5000, "split"), (3, 9, 1000, "split"),
+                                                 (2, 22, 304, "split"), (1, 20, 300, "split")])
 def test_keys_are_split_behind_few_rows_only(cuda, monkeypatch, seqs, rows, past, form):
     torch.manual_seed(rows)
     forms = _forms(monkeypatch)
