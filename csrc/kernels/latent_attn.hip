@@ -485,17 +485,27 @@ template <int NW> hipError_t launch_mfma_ndb(const LatentAttnArgs& a, hipStream_
   return hipErrorInvalidValue;
 }
 
-// The row tile and sequence of a workgroup, of a grid (tiles, sequences). Workgroups go to the 8 XCDs, which have an L2 each, in turn. Numbers
-// of sequences that are multiples of 8: sequence s is XCD s % 8's, one after the other, so that its cache rows are in one L2 and long and
-// short sequences are spread; its last tiles see the most keys and start first (all sequences' last tiles first, and so more
-// sequences in an L2 at a time: 32 of 250 ragged rows, 32 heads 76 -> 90 us; 16 of 1024 203 -> 230). Other numbers share every L2
-// anyhow: there the last tiles of all sequences start first, which leaves the short ones for the end and gives each CU one of every
-// kind (one sequence after the other, equal lengths, 16 heads: 12 of 500 73 -> 55, 7 of 1000 129 -> 105, 12 of 182 22.9 -> 22.1).
-__device__ __forceinline__ void tile_of(int& bx, int& s) {
+// The first row and the sequence of a workgroup, of a grid (tiles of ROWS rows, sequences); false where the sequence has no such tile. A sequence's
+// last tiles see the most keys and start first. Workgroups go to the 8 XCDs, which have an L2 each, in turn. Numbers of
+// sequences that are multiples of 8: sequence s is XCD s % 8's, one after the other, so that its cache rows are in one L2 (all
+// sequences' last tiles first, and so more sequences in an L2 at a time: 32 of 250 ragged rows, 32 heads 76 -> 90 us; 16 of 1024
+// 203 -> 230). Other numbers share every L2 anyhow: there the last tiles of all sequences start first, which leaves the short ones for
+// the end and gives each CU one of every kind (one sequence after the other, equal lengths, 16 heads: 12 of 500 73 -> 55, 7 of
+// 1000 129 -> 105, 12 of 182 22.9 -> 22.1). So do up to 3 sequences of unequal lengths per XCD, each of them over all XCDs: an XCD's own would
+// hold 1.3 - 1.5 times the mean work (24 of 101 - 200 rows, 16 heads 47.7 -> 38.7, 16 of 251 - 500, 32 heads 151 -> 120, 8 of 351 - 700 80 -> 73).
+template <int ROWS> __device__ __forceinline__ bool tile_of(const LatentAttnArgs& a, int& s, int& row0) {
   const unsigned nx = gridDim.x, n = gridDim.y, lin = blockIdx.x + nx * blockIdx.y;
-  const bool whole = n % 8 == 0;
-  s = (int)(whole ? lin % 8 + 8 * (lin / 8 / nx) : lin % n);
-  bx = (int)(nx - 1 - (whole ? lin / 8 % nx : lin / n));
+  unsigned t;   // from the sequence's last tile
+  if (n % 8 == 0 && (n >= 32 || a.total_q == (int64_t)a.max_q * n)) {
+    t = lin / 8 % nx;
+    s = (int)(lin % 8 + 8 * (lin / 8 / nx));
+  } else {
+    t = lin / n;
+    s = (int)(n % 8 == 0 ? (lin % n + t) % n : lin % n);
+  }
+  const int rows = (a.cu_q ? a.cu_q[s + 1] - a.cu_q[s] : 1) * a.heads;
+  row0 = ((rows + ROWS - 1) / ROWS - 1 - (int)t) * ROWS;
+  return row0 >= 0;
 }
 
 // Prompt-sized steps at the common rotary widths (rot_dim = 16 * NROT, NROT = 0: no rotary part): the same algorithm with every
@@ -528,16 +538,15 @@ __global__ void __launch_bounds__(256, 3) latent_attn_mfma_rq_kernel(LatentAttnA
   using Z = RqTile<NDB, NROT>;
   constexpr int KCH = Z::KCH, NPF = Z::NPF, NLAT = NDB, NK = NDB + NROT / 2;   // 32-wide steps of a row: latent, in all
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];   // two tiles, block-table entries; at the end the results
-  int bx, by;
-  tile_of(bx, by);
-  const int s = by, lane = threadIdx.x & 63, tid = threadIdx.x;
+  int s, row0;
+  if (!tile_of<64>(a, s, row0)) return;
+  const int lane = threadIdx.x & 63, tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int H = a.heads;
   constexpr int R = 32 * NDB, Dk = R + 16 * NROT;
   const int q0 = a.cu_q ? a.cu_q[s] : s;
   const int nq = a.cu_q ? a.cu_q[s + 1] - q0 : 1;
-  const int nrows = nq * H, row0 = bx * 64;
-  if (row0 >= nrows) return;
+  const int nrows = nq * H;
   const int ctx = a.ctx_lens[s];
   const int last_row = min(row0 + 64, nrows) - 1;
   const int p_first = (int)a.positions[q0 + row0 / H], p_last = (int)a.positions[q0 + last_row / H];
@@ -771,16 +780,15 @@ __global__ void __launch_bounds__(256, 2) latent_attn_wide_kernel(LatentAttnArgs
   constexpr int HC = Z::HC, NO = NDB / HC;   // 32-column blocks of a wave
   constexpr int KCH = Z::KCH, NPF = Z::NPF, KT = 32, NLAT = 2 * NDB, NK = NLAT + NROT;   // 16-wide steps of a row: latent, in all
   extern __shared__ __attribute__((aligned(16))) char smem_raw[];   // two tiles, key rows
-  int bx, by;
-  tile_of(bx, by);
-  const int s = by, lane = threadIdx.x & 63, tid = threadIdx.x;
+  int s, row0;
+  if (!tile_of<Z::ROWS>(a, s, row0)) return;
+  const int lane = threadIdx.x & 63, tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int H = a.heads;
   constexpr int R = 32 * NDB, Dk = R + 16 * NROT;
   const int q0 = a.cu_q ? a.cu_q[s] : s;
   const int nq = a.cu_q ? a.cu_q[s + 1] - q0 : 1;
-  const int nrows = nq * H, row0 = bx * Z::ROWS;
-  if (row0 >= nrows) return;
+  const int nrows = nq * H;
   const int ctx = a.ctx_lens[s];
   const int last_row = min(row0 + Z::ROWS, nrows) - 1;
   const int p_first = (int)a.positions[q0 + row0 / H], p_last = (int)a.positions[q0 + last_row / H];

@@ -96,9 +96,11 @@ def test_results_at_any_8_bytes(cuda):
     assert form == "tiles" and torch.equal(got, want)
 
 
-@pytest.mark.parametrize("lens,window", [((64, 1, 33, 2, 63, 31, 17, 48) * 8 + (5, 64, 9), 0), ((200, 333, 1, 140, 257, 90, 310, 16, 128), 70)])
+@pytest.mark.parametrize("lens,window", [((64, 1, 33, 2, 63, 31, 17, 48) * 8 + (5, 64, 9), 0), ((200, 333, 1, 140, 257, 90, 310, 16, 128), 70),
+                                         ((70, 2, 55, 64, 9, 33, 70, 41) * 2, 0), ((199, 101, 1, 160, 177, 200, 140, 33) * 3, 0), ((5, 64, 1, 17, 32, 40, 63, 2) * 4, 0)])
 def test_sequences_not_in_eights(cuda, lens, window):
-    """The row tiles of a number of sequences that is no multiple of 8 are dealt in another order: every row once, the longest sequence's too."""
+    """The row tiles of a number of sequences that is no multiple of 8, or a small one of unequal lengths, are dealt in another order: every
+    row once, the longest sequence's too."""
     torch.manual_seed(len(lens))
     rank, rot, heads, bs, scale = 256, 32, 32, 16, 0.08
     S, T, need = len(lens), sum(lens), -(-max(lens) // bs)
