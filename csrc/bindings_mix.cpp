@@ -448,6 +448,7 @@ std::string latent_attn(Tensor out, Tensor q_lat, Tensor q, int64_t rot_off, Ten
   a.cache = cache.data_ptr();
   a.block_tables = block_tables.data_ptr<int>();
   a.bt_stride = (int)block_tables.stride(0);
+  a.bt_cols = (int)block_tables.size(1);
   a.cu_q = nullptr;
   if (cu_q.has_value()) {
     check_i(*cu_q, at::kInt, "cu_q");

@@ -391,6 +391,7 @@ const char* sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, O
   a.cache = cache.data_ptr();
   a.block_tables = block_tables.data_ptr<int>();
   a.bt_stride = (int)block_tables.stride(0);
+  a.bt_cols = (int)block_tables.size(1);
   a.cu_q = nullptr;
   if (cu_q.has_value()) {
     check_c(*cu_q, at::kInt, "cu_q");

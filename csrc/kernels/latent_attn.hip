@@ -1028,7 +1028,7 @@ inline bool mfma_rq_fits(const LatentAttnArgs& a) {
 // 23.5 / 17.9, 1 x 1500 behind 400 118 / 78, 8 x 128 14.4 / 12.8; 32 x 30 9.7 / 10.8; 8 x 500 behind 100 50 / 54, 16 x 1024 309 / 324.
 template <int NDB, int NROT> hipError_t launch_rows(const LatentAttnArgs& a, hipStream_t s) {
   const int64_t wgs = ((int64_t)a.max_q * a.heads + 63) / 64 * a.num_seqs;
-  const int64_t keys = (int64_t)a.bt_stride * a.block_size;
+  const int64_t keys = (int64_t)a.bt_cols * a.block_size;
   return wgs <= 2 * (int64_t)num_cus() && keys > 64 && a.scale > 0.f ? launch_wide<NDB, NROT>(a, s) : launch_mfma_rq<NDB, NROT>(a, s);
 }
 template <int NDB> hipError_t launch_mfma_rq_rot(const LatentAttnArgs& a, hipStream_t s) {

@@ -104,7 +104,7 @@ struct LatentAttnArgs {
   int64_t q_stride, q_hstride;
   const void* cache;      // [num_blocks, block_size, rank + rot_dim]
   const int* block_tables;
-  int bt_stride;
+  int bt_stride, bt_cols; // of a row of the tables: to the next one, entries that the step may use
   const int* cu_q;        // [S + 1] first row of each sequence (nullptr: one row per sequence)
   const int* ctx_lens;    // [S] keys after this step
   const int64_t* positions;

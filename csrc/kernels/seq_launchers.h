@@ -141,7 +141,7 @@ struct SinkAttnArgs {
   const void* q;          // [T, H * dim]
   const void* cache;      // [num_blocks][G][block_size][K: dim | V: vdim]
   const int* block_tables;
-  int bt_stride;
+  int bt_stride, bt_cols; // of a row of the tables: to the next one, entries that the step may use
   const int* cu_q;        // nullptr: one row per sequence
   const int* ctx_lens;    // [S] keys after this step
   const int64_t* positions;

@@ -1547,7 +1547,7 @@ template <int NKC> hipError_t launch_decode_v(const SinkAttnArgs& a, hipStream_t
 
 // cached keys of a sequence that a step can see
 inline int64_t keys_of(const SinkAttnArgs& a) {
-  int64_t keys = (int64_t)a.bt_stride * a.block_size;
+  int64_t keys = (int64_t)a.bt_cols * a.block_size;
   if (a.window > 0) keys = std::min<int64_t>(keys, (int64_t)a.window + a.max_q);
   return a.seg > 0 ? std::min<int64_t>(keys, (int64_t)a.seg + a.max_q) : keys;
 }

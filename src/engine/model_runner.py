@@ -273,7 +273,7 @@ class ModelRunner:
         self._h2d(t, n, with_cu=True)
         max_q = max(c.length for c in chunks)
         self._sync_step(self.KIND_PREFILL, t, n, max_q, nd)
-        ids = self._exec_prefill(t, n, max_q, nd, greedy, kv_hook=kv_hook)
+        ids = self._exec_prefill(t, n, max_q, nd, greedy, kv_hook=kv_hook, max_ctx=max(c.start + c.length for c in chunks))
         res: List[Optional[int]] = [None] * n
         if nd:
             vals = self._to_host(ids, nd)
@@ -313,7 +313,8 @@ class ModelRunner:
         else:
             meta = AttnMetadata(is_prefill=True, slot_mapping=self.d_slots[:t], block_tables=self.d_bt[:n],
                                 ctx_lens=self.d_ctx[:n], cu_q=self.d_cu[: n + 1],
-                                max_q_len=max(c.length for c in chunks), state_slots=self._state_slots(n))
+                                max_q_len=max(c.length for c in chunks), max_ctx=max(c.start + c.length for c in chunks),
+                                state_slots=self._state_slots(n))
         hidden = self.model.forward(self.d_ids[:t], self.d_pos[:t], meta, self.pool.tensor)
         if not rows:
             if self.is_cuda:
@@ -323,11 +324,11 @@ class ModelRunner:
         logits = self.model.compute_logits(hidden.index_select(0, sel)).float()
         return logits.cpu()
 
-    def _exec_prefill(self, t: int, n: int, max_q: int, nd: int, greedy: bool, kv_hook=None) -> Optional[torch.Tensor]:
+    def _exec_prefill(self, t: int, n: int, max_q: int, nd: int, greedy: bool, kv_hook=None, max_ctx: int = 0) -> Optional[torch.Tensor]:
         # the last layer runs only for the sampled rows (CausalLM._last_layer_kept_rows; DIE_PRUNE_LAST=0: all)
         keep = self.d_last[:nd] if self.prune_last else None
         meta = AttnMetadata(is_prefill=True, slot_mapping=self.d_slots[:t], block_tables=self.d_bt[:n],
-                            ctx_lens=self.d_ctx[:n], cu_q=self.d_cu[: n + 1], max_q_len=max_q, kv_hook=kv_hook,
+                            ctx_lens=self.d_ctx[:n], cu_q=self.d_cu[: n + 1], max_q_len=max_q, max_ctx=max_ctx, kv_hook=kv_hook,
                             keep_rows=keep, state_slots=self._state_slots(n))
         hidden = self.model.forward(self.d_ids[:t], self.d_pos[:t], meta, self.pool.tensor)
         if not nd:

@@ -279,7 +279,7 @@ class LatentAttentionMixer:
             cq = mix.rms_norm_ext(p[:, :nq], self.dq_norm, eps)
         q = mix.linear(cq, self.uq)
         q_lat = torch.bmm(q.view(t, s.heads, s.dim + s.rot_dim)[:, :, : s.dim].transpose(0, 1), self.uk)
-        o_lat = mix.latent_attn(q_lat, q, s.dim, cache, meta.block_tables, meta.cu_q if meta.is_prefill else None,
+        o_lat = mix.latent_attn(q_lat, q, s.dim, cache, meta.step_tables(cache.shape[1]), meta.cu_q if meta.is_prefill else None,
                                 meta.ctx_lens, positions, self.sink, meta.max_q_len if meta.is_prefill else 1,
                                 s.window, s.scale, s.rot_dim, self.inv_freq)
         o = torch.bmm(o_lat, self.uv_t)                                    # [H, T, vdim]

@@ -429,7 +429,7 @@ class SinkAttentionMixer:
                           rag=rag if s.conv else None, rot_gain=self.rot_gain, v_inv_freq=self.v_inv_freq)
         if s.conv:
             rec.conv_tail_update(state["qkv_conv"], p[:, : s.channels], rag)
-        return seq.sink_attn(qr, cache, meta.block_tables, meta.cu_q if meta.is_prefill else None, meta.ctx_lens,
+        return seq.sink_attn(qr, cache, meta.step_tables(cache.shape[1]), meta.cu_q if meta.is_prefill else None, meta.ctx_lens,
                              positions, self.sink, self.bias, meta.max_q_len if meta.is_prefill else 1, s.heads,
                              s.kv_heads, s.dim, s.vdim, s.window, s.scale, softcap=s.softcap, slopes=self.slopes, seg=s.seg,
                              gate=gate, out_inv_freq=self.v_inv_freq if gate is not None else None, gate_mult=mult, out=out,

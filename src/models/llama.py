@@ -43,7 +43,7 @@ class AttnMetadata:
     ctx_lens: torch.Tensor          # [S] int32 (KV length after this step)
     cu_q: Optional[torch.Tensor] = None    # [S+1] int32 (prefill)
     max_q_len: int = 1
-    max_ctx: int = 0                # decode grid bound (static under hipGraph)
+    max_ctx: int = 0                # decode grid bound (static under hipGraph); prompt steps: their longest context (0: not known)
     part_o: Optional[torch.Tensor] = None
     part_ml: Optional[torch.Tensor] = None
     attn_cnt: Optional[torch.Tensor] = None  # decode attention merge tickets (int32, zeroed once)
@@ -59,6 +59,14 @@ class AttnMetadata:
     # models with per-sequence state besides the cache (recurrent layers, the previous token): the state slot of
     # every sequence of the step, [S] int32 (padded rows of a captured decode step: the pool's spare slot)
     state_slots: Optional[torch.Tensor] = None
+
+    def step_tables(self, block_size: int) -> torch.Tensor:
+        """The block tables as wide as the step's longest context where that is known (prompt steps): attention that takes their width for
+        the keys there can be splits keys, and chooses its kernels, by what the step holds and not by the longest sequence that the
+        model may have (rows keep their stride). Decode steps keep the whole width, which a captured graph holds."""
+        if not self.is_prefill or self.max_ctx <= 0:
+            return self.block_tables
+        return self.block_tables[:, : -(-self.max_ctx // block_size)]
 
 
 class LayerWeights:
