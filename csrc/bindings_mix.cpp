@@ -418,7 +418,8 @@ void combine_post_norm(Tensor resid, OptTensor act, Tensor ys, OptTensor pos, Op
                                        cur_stream()));
 }
 
-// out, q_lat [H, T, rank]; q [T, H * qh] whose head h keeps its rotary part at [h * qh + rot_off, + rot_dim). Returns the form that ran.
+// out, q_lat [H, T, rank]; q [T, H * qh] whose head h keeps its rotary part at [h * qh + rot_off, + rot_dim). Returns the form that ran, or its kernel.
+template <bool KERNEL>
 std::string latent_attn(Tensor out, Tensor q_lat, Tensor q, int64_t rot_off, Tensor cache, Tensor block_tables,
                         OptTensor cu_q, Tensor ctx_lens, Tensor positions, OptTensor sink, int64_t max_q, int64_t window,
                         double scale, int64_t rot_dim, Tensor inv_freq, int64_t impl) {
@@ -510,7 +511,7 @@ std::string latent_attn(Tensor out, Tensor q_lat, Tensor q, int64_t rot_off, Ten
     }
   }
   HIP_OK(die::launch_latent_attn(a, cur_stream()));
-  return die::latent_attn_form(a);
+  return KERNEL ? die::latent_attn_kernel(a) : die::latent_attn_form(a);
 }
 
 void moe_align(Tensor offsets, Tensor sorted, Tensor pos, Tensor ids, int64_t num_experts) {
@@ -560,7 +561,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gather_scaled", &gather_scaled);
   m.def("combine_sum", &combine_sum);
   m.def("latent_kv_write", &latent_kv_write);
-  m.def("latent_attn", &latent_attn);
+  m.def("latent_attn", &latent_attn<false>);
+  m.def("latent_attn_named", &latent_attn<true>);   // tests
   m.def("latent_qkv_prep", &latent_qkv_prep);
   m.def("combine_post_norm", &combine_post_norm);
   m.def("moe_align", &moe_align);

@@ -355,7 +355,8 @@ void qkv_prep(Tensor q_out, Tensor cache, Tensor q, Tensor k, OptTensor v, int64
   HIP_OK(die::launch_qkv_prep(a, cur_stream()));
 }
 
-// returns the form that ran (sink_attn_form)
+// returns the form that ran (sink_attn_form), or its kernel (sink_attn_kernel)
+template <bool KERNEL>
 const char* sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, OptTensor cu_q, Tensor ctx_lens,
                Tensor positions, OptTensor sink, OptTensor bias, int64_t max_q, int64_t heads, int64_t kv_heads,
                int64_t dim, int64_t vdim, int64_t window, double scale, int64_t impl, double softcap,
@@ -483,14 +484,14 @@ const char* sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, O
   a.ostride = out.stride(0);
   if (!gate.has_value()) {
     HIP_OK(die::launch_sink_attn(a, cur_stream()));
-    return die::sink_attn_form(a);
+    return KERNEL ? die::sink_attn_kernel(a) : die::sink_attn_form(a);
   }
   if (die::sink_attn_fuses_gate(a)) {
     a.gate = gate->data_ptr();
     a.gstride = gate->stride(0);
     a.out_inv_freq = f32_ptr(out_inv_freq, vdim / 2, "out_inv_freq");
     HIP_OK(die::launch_sink_attn(a, cur_stream()));
-    return die::sink_attn_form(a);
+    return KERNEL ? die::sink_attn_kernel(a) : die::sink_attn_form(a);
   }
   // the other forms write plain rows; the gate is a launch of its own
   Tensor raw = at::empty({T, heads * vdim}, q.options());
@@ -511,7 +512,7 @@ const char* sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, O
   g.heads = (int)heads;
   g.vdim = (int)vdim;
   HIP_OK(die::launch_rot_head_gate(g, cur_stream()));
-  return die::sink_attn_form(a);
+  return KERNEL ? die::sink_attn_kernel(a) : die::sink_attn_form(a);
 }
 
 }  // namespace
@@ -525,5 +526,6 @@ void register_seq_ops(pybind11::module& m) {
   m.def("conv_state_update", &conv_state_update);
   m.def("gated_delta", &gated_delta);
   m.def("qkv_prep", &qkv_prep);
-  m.def("sink_attn", &sink_attn);
+  m.def("sink_attn", &sink_attn<false>);
+  m.def("sink_attn_named", &sink_attn<true>);   // tests
 }

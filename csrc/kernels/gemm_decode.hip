@@ -33,7 +33,7 @@
 #include "car_common.h"
 #include "common.h"
 #include "launchers.h"
-#include "moe_gemm.h"
+#include "moe_gate.h"
 
 #include <algorithm>
 #include <cstdlib>
@@ -53,15 +53,6 @@ typedef __attribute__((ext_vector_type(4))) float f4;
 template <int AUX = 0>
 __device__ __forceinline__ void glds16(const void* src, char* lds_wave_base) {
   __builtin_amdgcn_global_load_lds((global_cvoid*)src, (lds_void*)lds_wave_base, 16, 0, AUX);
-}
-
-// the gates of the grouped product (moe_gemm.hip)
-template <int ACT> __device__ __forceinline__ float moe_gate(float g, float u, float limit, float alpha) {
-  if constexpr (ACT == MOE_ACT_SILU) return gated(g, g) * u;
-  if constexpr (ACT == MOE_ACT_GELU) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) * u;
-  g = fminf(g, limit);
-  u = fminf(fmaxf(u, -limit), limit);
-  return gated(g, alpha * g) * (u + 1.0f);
 }
 
 template <int N>

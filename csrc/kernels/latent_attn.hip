@@ -1026,10 +1026,12 @@ inline bool mfma_rq_fits(const LatentAttnArgs& a) {
 // A workgroup has 64 rows in either kernel. Up to two of them per CU go with 32 rows per wave (whose maxima are taken before the scale: a
 // positive one), more with 16, of which three workgroups share a CU and which start faster, for few keys too. 16 / 32 rows per wave, rank 256 + 32, us: 1 x 300 rows of 16 heads
 // 23.5 / 17.9, 1 x 1500 behind 400 118 / 78, 8 x 128 14.4 / 12.8; 32 x 30 9.7 / 10.8; 8 x 500 behind 100 50 / 54, 16 x 1024 309 / 324.
+inline bool wide_takes(const LatentAttnArgs& a) {
+  const int64_t wgs = ((int64_t)a.max_q * a.heads + 63) / 64 * a.num_seqs, keys = (int64_t)a.bt_cols * a.block_size;
+  return wgs <= 2 * (int64_t)num_cus() && keys > 64 && a.scale > 0.f;
+}
 template <int NDB, int NROT> hipError_t launch_rows(const LatentAttnArgs& a, hipStream_t s) {
-  const int64_t wgs = ((int64_t)a.max_q * a.heads + 63) / 64 * a.num_seqs;
-  const int64_t keys = (int64_t)a.bt_cols * a.block_size;
-  return wgs <= 2 * (int64_t)num_cus() && keys > 64 && a.scale > 0.f ? launch_wide<NDB, NROT>(a, s) : launch_mfma_rq<NDB, NROT>(a, s);
+  return wide_takes(a) ? launch_wide<NDB, NROT>(a, s) : launch_mfma_rq<NDB, NROT>(a, s);
 }
 template <int NDB> hipError_t launch_mfma_rq_rot(const LatentAttnArgs& a, hipStream_t s) {
   switch (a.sh.rot_dim) {
@@ -1101,6 +1103,12 @@ bool latent_attn_fits_rows(const LatentAttnArgs& a) { return latent_attn_uses_mf
 const char* latent_attn_form(const LatentAttnArgs& a) {
   if (!latent_attn_uses_mfma(a)) return "fma";
   return a.impl != 3 && a.nsplit <= 1 && mfma_rq_fits(a) ? "rows" : a.nsplit > 1 ? "split" : "tiles";
+}
+
+const char* latent_attn_kernel(const LatentAttnArgs& a) {
+  const char* form = latent_attn_form(a);
+  if (form[0] == 'r' && wide_takes(a)) return "wide";
+  return form[0] == 's' && a.fine ? "fine split" : form;
 }
 
 hipError_t launch_latent_attn(const LatentAttnArgs& a, hipStream_t s) {

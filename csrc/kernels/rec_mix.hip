@@ -883,8 +883,8 @@ hipError_t launch_selective_scan(const SelectiveScanArgs& a, RaggedRows r, hipSt
     // reads and exponentials that 8 or 4 states per lane shorten (1 x 1024 tokens of 4096 channels 485 us, in 2 / 4 lanes 398 / 381; 4 x 500
     // 246, 201 / 190; 16 x 1024 497, 464 / 587; 32 x 100 69, 75 / 99)
     const int64_t waves = ((int64_t)a.I * r.num_seqs + 63) / 64, simds = 4 * (int64_t)num_cus();
-    if (a.N > 8 && 2 * waves <= simds) return launch_scan_one<4, 4>(a, r, s);
-    if (a.N > 8 && waves <= simds) return launch_scan_one<8, 2>(a, r, s);
+    if (2 * waves <= simds) return launch_scan_one<4, 4>(a, r, s);
+    if (waves <= simds) return launch_scan_one<8, 2>(a, r, s);
     return launch_scan_one<16, 1>(a, r, s);
   }
   if (a.N <= 32) return launch_scan_one<16, 2>(a, r, s);

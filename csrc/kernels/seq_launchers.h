@@ -187,5 +187,8 @@ bool sink_attn_fuses_gate(const SinkAttnArgs& a);
 // the form that launch_sink_attn runs (nsplit already chosen): "decode", "rows" (16 rows per wave), "tiles" (32 rows per wave), "split"
 // (the same with the keys split) or "fma"
 const char* sink_attn_form(const SinkAttnArgs& a);
+// its kernel, of the forms that have several: "wide" (128 rows per workgroup), "rows" and "fine rows" (64, weights in one or two parts),
+// "split" and "fine split"
+const char* sink_attn_kernel(const SinkAttnArgs& a);
 
 }  // namespace die

@@ -1554,9 +1554,11 @@ inline int64_t keys_of(const SinkAttnArgs& a) {
 // FINE: the weights enter the products in two bf16 parts, for steps of up to four row tiles of 128 per CU over more than one of 64 keys. The
 // kernel with split keys, which ran them before, rounds relative to every split's own largest weight, which is then exact: whole
 // keys with rounded weights are up to 6 % further from 64 bits (5 x 77 rows behind 300: 2.18e-3, whole 2.31e-3, in two parts 1.66e-3).
+inline int64_t wide_tiles(const SinkAttnArgs& a) { return ((int64_t)a.max_q * (a.heads / a.kv_heads) + 127) / 128 * a.num_seqs * a.kv_heads; }
+inline bool fine_takes(const SinkAttnArgs& a) { return wide_tiles(a) <= 4 * (int64_t)num_cus() && keys_of(a) > 64; }
 template <int NK, int NV> hipError_t launch_rows(const SinkAttnArgs& a, hipStream_t s) {
   const int64_t rows = (int64_t)a.max_q * (a.heads / a.kv_heads);
-  const bool fine = (rows + 127) / 128 * a.num_seqs * a.kv_heads <= 4 * (int64_t)num_cus() && keys_of(a) > 64;
+  const bool fine = fine_takes(a);
   const dim3 grid((unsigned)((rows + 63) / 64), (unsigned)a.num_seqs, (unsigned)a.kv_heads);
   auto* fn = a.sigmoid ? (fine ? sink_attn_rows_kernel<NK, NV, true, true> : sink_attn_rows_kernel<NK, NV, true, false>)
                        : (fine ? sink_attn_rows_kernel<NK, NV, false, true> : sink_attn_rows_kernel<NK, NV, false, false>);
@@ -1589,13 +1591,13 @@ inline bool rows_fits(const SinkAttnArgs& a) {
 // and keys not split
 inline bool rows_takes(const SinkAttnArgs& a) { return (a.ws_o == nullptr || a.nsplit <= 1) && rows_fits(a); }
 
-// Of these, those that go 128 rows per workgroup: where that still gives every CU two workgroups twice over, and long keys (a workgroup's
-// start is the same for 64 rows). Scores with caps, slopes or a bias are bound by vector instructions, of which four waves per SIMD
+// Of these, those that go 128 rows per workgroup: more than four tiles per CU and long keys (a workgroup's start is the same for 64 rows). Fewer tiles
+// keep 64 rows also where 128 are faster: their keys were split before, and their weights go in two bf16 parts (fine_takes), which the wide
+// kernel has no registers for. Scores with caps, slopes or a bias are bound by vector instructions, of which four waves per SIMD
 // issue more than two. 64 / 128 rows, us: 16 x 1000 behind 300, 16 heads 132 / 110, vdim 256 187 / 160, window of 512 89 / 80; 4 x 1000 of 32
-// heads 57 / 54; 2 x 1000 37 / 38; 16 x 250 23.0 / 24.3; capped 16 x 500 of 32 heads 121 / 135.
+// heads (4 tiles per CU) 57 / 54; 2 x 1000 37 / 38; 16 x 250 23.0 / 24.3; capped 16 x 500 of 32 heads 121 / 135.
 inline bool wide_takes(const SinkAttnArgs& a) {
-  const int64_t rows = (int64_t)a.max_q * (a.heads / a.kv_heads), wgs = (rows + 127) / 128 * a.num_seqs * a.kv_heads;
-  return a.softcap <= 0.f && a.slopes == nullptr && a.bias == nullptr && a.scale > 0.f && wgs > 4 * (int64_t)num_cus() && keys_of(a) >= 512;
+  return a.softcap <= 0.f && a.slopes == nullptr && a.bias == nullptr && a.scale > 0.f && wide_tiles(a) > 4 * (int64_t)num_cus() && keys_of(a) >= 512;
 }
 
 inline bool decode_ok(const SinkAttnArgs& a) {
@@ -1624,6 +1626,12 @@ const char* sink_attn_form(const SinkAttnArgs& a) {
   if (sink_attn_uses_decode(a)) return "decode";
   if (!sink_attn_uses_mfma(a)) return "fma";
   return rows_takes(a) ? "rows" : a.ws_o != nullptr && a.nsplit > 1 ? "split" : "tiles";
+}
+
+const char* sink_attn_kernel(const SinkAttnArgs& a) {
+  if (sink_attn_uses_decode(a) || !sink_attn_uses_mfma(a)) return sink_attn_form(a);
+  if (rows_takes(a)) return wide_takes(a) ? "wide" : fine_takes(a) ? "fine rows" : "rows";
+  return a.ws_o != nullptr && a.nsplit > 1 && a.fine && !a.sigmoid ? "fine split" : sink_attn_form(a);
 }
 
 hipError_t launch_sink_attn(const SinkAttnArgs& a, hipStream_t s) {

@@ -60,8 +60,36 @@ def test_few_row_tiles(cuda, rank, rot, heads, bs, window, lens, past):
     inv, sink, scale = ops.rope_inv_freq(10000.0, max(rot, 2), cuda)[: rot // 2], torch.randn(heads, device=cuda) + 1, 0.08
     got = torch.empty_like(q_lat)
     tail = (cache, bt, cu, ctx, pos, sink, max(lens), window, scale, rot, inv)
-    form = mix._kern().latent_attn(got, q_lat, q, 6, *tail, 0)
-    assert form == "rows" or past >= 1000
+    form = mix._kern().latent_attn_named(got, q_lat, q, 6, *tail, 0)
+    assert form == ("split" if past >= 1000 else "wide")   # (few rows behind that many keys)
+    want = ops.latent_attn(q_lat, q, 6, *tail, impl=1).float()
+    e = 0.0
+    if rot:
+        e = scale * 2 ** -9 * float(q.view(T, heads, -1)[..., 6:].float().norm(dim=-1).max() * cache[..., rank:].float().norm(dim=-1).max())
+    top = float(cache[..., :rank].float().abs().max())
+    assert ((got.float() - want).abs() <= (2 ** -9 + 2 * e * 2.71828 ** (2 * e)) * top + 2 ** -7 * want.abs()).all()
+    assert ((got.float() - want).norm() / want.norm()).item() < 2 ** -7
+
+
+@pytest.mark.parametrize("rank,rot,heads,bs,lens,past,kernel", [
+    (256, 32, 16, 1, (1300,), 0, "wide"), (256, 16, 16, 24, (1300,), 0, "wide"), (64, 0, 12, 16, (700, 600), 700, "wide"), (128, 64, 16, 7, (1100,), 60, "wide"),
+    (256, 32, 16, 1, (1100, 1100), 0, "rows")])
+def test_row_table_is_filled_again(cuda, rank, rot, heads, bs, lens, past, kernel):
+    """More visible keys than the 1024 entries that a workgroup's table holds, at page sizes of 1 and others."""
+    from src.ops import mix
+
+    torch.manual_seed(rank + rot + bs)
+    S, T, need = len(lens), sum(lens), -(-(max(lens) + past) // bs)
+    cache = torch.randn(1 + 2 * need, bs, rank + rot, device=cuda).to(torch.bfloat16)
+    bt = torch.randint(0, 1 + 2 * need, (S, need), device=cuda, dtype=torch.int32)
+    cu = torch.tensor([0, *lens], device=cuda).cumsum(0).int()
+    pos = torch.cat([torch.arange(n) + past for n in lens]).to(cuda)
+    ctx = torch.tensor([n + past for n in lens], device=cuda, dtype=torch.int32)
+    q_lat, q = torch.randn(heads, T, rank, device=cuda).to(torch.bfloat16), torch.randn(T, heads * (rot + 6), device=cuda).to(torch.bfloat16)
+    inv, sink, scale = ops.rope_inv_freq(10000.0, max(rot, 2), cuda)[: rot // 2], torch.randn(heads, device=cuda) + 1, 0.08
+    got = torch.empty_like(q_lat)
+    tail = (cache, bt, cu, ctx, pos, sink, max(lens), 0, scale, rot, inv)
+    assert mix._kern().latent_attn_named(got, q_lat, q, 6, *tail, 0) == kernel
     want = ops.latent_attn(q_lat, q, 6, *tail, impl=1).float()
     e = 0.0
     if rot:

@@ -87,11 +87,11 @@ def test_activations_are_those_of_the_separate_pass(cuda, act, kind):
     assert torch.equal(out, want), (out != want).sum()
 
 
-@pytest.mark.parametrize("height", [128, 192, 224, 256])
+@pytest.mark.parametrize("height", [128, 160, 192, 224, 256])
 @pytest.mark.parametrize("K,ncols,act", [(64, 256, mix.MOE_NONE), (320, 128, mix.MOE_SILU)])
 def test_every_tile_height(cuda, height, K, ncols, act):
     """The heights that large steps take, asked for: full tiles, last tiles of one row, around 32 rows and one short of full, several
-    tiles of an expert (two waves share a tile's 32-row pieces: 4 and 4, 4 and 3, 3 and 3, 2 and 2 of them, and all fewer)."""
+    tiles of an expert (two waves share a tile's 32-row pieces: 4 and 4, 4 and 3, 3 and 3, 3 and 2, 2 and 2 of them, and all fewer)."""
     counts = (height, height - 1, 1, 31, 33, height + 1, 2 * height + 33, 3 * height, 95, 161)
     x, w, offsets, idx, scale = _case(counts, K, ncols, act != mix.MOE_NONE, 1, seed=height)
     out = torch.full((sum(counts), ncols), 7.0, dtype=torch.bfloat16, device=cuda)
@@ -107,8 +107,8 @@ def test_chosen_heights(cuda, counts):
     """The height that the kernel takes by itself: the same bits as with each of the heights (a row's sums do not depend on its tile)."""
     x, w, offsets, idx, scale = _case(counts, 128, 1024, True, 1, seed=len(counts))
     dev = [t.to(cuda) for t in (x, w, offsets, idx)]
-    outs = [torch.full((sum(counts), 1024), 7.0, dtype=torch.bfloat16, device=cuda) for _ in range(4)]
-    for out, height in zip(outs, (0, 192, 224, 256)):
+    outs = [torch.full((sum(counts), 1024), 7.0, dtype=torch.bfloat16, device=cuda) for _ in range(6)]
+    for out, height in zip(outs, (0, 128, 160, 192, 224, 256)):
         assert mix._kern().moe_gemm(out, *dev, 1, scale.to(cuda), mix.MOE_SILU, 0.0, 0.0, height)
     assert all(torch.equal(outs[0], o) for o in outs[1:])
 

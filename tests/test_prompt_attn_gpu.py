@@ -24,6 +24,20 @@ def _forms(monkeypatch):
     return forms
 
 
+def _kernels(monkeypatch):
+    """The same with the kernels of the forms that have several."""
+    kern, names = seq._kern(), []
+
+    class Spy:
+        def __getattr__(self, name):
+            if name != "sink_attn":
+                return getattr(kern, name)
+            return lambda *a: names.append(kern.sink_attn_named(*a))
+
+    monkeypatch.setattr(seq, "_kern", lambda: Spy())
+    return names
+
+
 @pytest.mark.parametrize("seqs", [2, 72])   # 2: the keys are split, and the 32-rows-per-wave kernel runs; 72: enough row tiles without
 @pytest.mark.parametrize("dim,vdim,heads,groups,bs,style,past", [
     (128, 128, 16, 4, 16, "", 0), (64, 64, 15, 5, 32, "sink", 70), (64, 128, 16, 4, 16, "cap", 5), (64, 256, 16, 4, 16, "bias", 33), (128, 128, 16, 4, 16, "bias", 0),
@@ -109,7 +123,7 @@ def test_many_rows_of_long_keys(cuda, monkeypatch, dim, vdim, heads, groups, bs,
     """128 rows per workgroup: four of them per compute unit, tiles of 64 keys (vdim 256: 32), row counts around 32 and 128, pairs of
     sequence and head that are and are not a multiple of 8."""
     torch.manual_seed(dim + vdim + heads)
-    forms = _forms(monkeypatch)
+    forms = _kernels(monkeypatch)
     lens = ([200, 8, 33, 1, 65, 32, 129, 190] * 11)[:88 if style else 81]
     data = _ragged(cuda, lens, [520 + 7 * (s % 9) for s in range(len(lens))], bs, groups, dim, vdim, heads)
     sink, kw = (torch.randn(heads, device=cuda) if style == "sink" else None), {}
@@ -119,7 +133,7 @@ def test_many_rows_of_long_keys(cuda, monkeypatch, dim, vdim, heads, groups, bs,
         kw = dict(seg=512)
     args = (*data, sink, None, max(lens), heads, groups, dim, vdim, 400 if style == "window" else 0, dim ** -0.5)
     want, got = seq.sink_attn(*args, impl=1, **kw).float(), seq.sink_attn(*args, **kw).float()
-    assert forms == ["fma", "rows"]
+    assert forms == ["fma", "wide"]
     mass = 1.0 if style != "sigmoid" else 20.0   # of the sigmoid weights
     assert ((got - want).abs() <= 2 ** -8.5 * mass * float(data[1].float().abs().max()) + 2 ** -7 * want.abs()).all()
     assert ((got - want).norm() / want.norm()).item() < 2 ** -7
@@ -192,3 +206,50 @@ def test_fewer_splits_are_no_further_from_64_bits(cuda, monkeypatch, style, vdim
                          **{k: cpu(v) if torch.is_tensor(v) else v for k, v in kw.items()})
     error = lambda x: ((x.cpu().double() - want.double()).norm() / want.double().norm()).item()
     assert error(got) <= 1.01 * error(all_splits)
+
+
+@pytest.mark.parametrize("kernel,dim,vdim,style,seqs,past", [
+    ("wide", 128, 128, "", 76, 1150), ("wide", 64, 256, "sink", 76, 1060), ("wide", 64, 64, "sigmoid", 76, 2200), ("rows", 128, 128, "cap", 72, 1150),
+    ("rows", 64, 64, "bias", 72, 2200), ("rows", 64, 256, "slopes", 72, 1100), ("fine rows", 128, 128, "", 50, 1300), ("fine rows", 64, 128, "sigmoid", 50, 1300),
+    ("fine rows", 128, 256, "sink", 40, 1100)])
+def test_row_table_is_filled_again(cuda, monkeypatch, kernel, dim, vdim, style, seqs, past):
+    """More visible keys than the 1024 rows that a workgroup's table of cache rows holds, for every kernel that has one."""
+    torch.manual_seed(dim + vdim + seqs)
+    names, heads, groups = _kernels(monkeypatch), 16, 4
+    data = _ragged(cuda, ([130, 1, 33, 2, 63, 31, 127, 48] * 10)[:seqs], [past + 7 * (s % 3) for s in range(seqs)], 16, groups, dim, vdim, heads)
+    f = lambda *s: torch.randn(*s, device=cuda)
+    sink, bias, kw = (f(heads) if style == "sink" else None), (f(40, heads) if style == "bias" else None), {}
+    if style == "cap":
+        kw = dict(softcap=5.0, slopes=torch.rand(heads, device=cuda) * 0.01)
+    if style == "slopes":
+        kw = dict(slopes=torch.rand(heads, device=cuda) * 0.01)
+    if style == "sigmoid":
+        kw = dict(sigmoid=True, head_bias=f(heads) - 5)
+    args = (*data, sink, bias, 130, heads, groups, dim, vdim, 0, dim ** -0.5)
+    want, got = seq.sink_attn(*args, impl=1, **kw).float(), seq.sink_attn(*args, **kw).float()
+    assert names == ["fma", kernel]
+    mass = 1.0 if style != "sigmoid" else 40.0   # of the sigmoid weights
+    assert ((got - want).abs() <= 2 ** -8.5 * mass * float(data[1].float().abs().max()) + 2 ** -7 * want.abs()).all()
+    assert ((got - want).norm() / want.norm()).item() < 2 ** -7
+
+
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (64, 128), (64, 256), (128, 64), (128, 128), (128, 256)])
+@pytest.mark.parametrize("style", ["sigmoid", "sink", "bias", "cap", "window"])
+def test_weights_in_two_parts(cuda, monkeypatch, dim, vdim, style):
+    """Every width and kind of scores of the steps whose weights go in two bf16 parts. The weights' own rounding is gone (2^-17 of sum w |v|
+    is left), so results are within their one rounding, 2^-9, of the fp32 kernel's before its rounding: 2^-8 of both, and 2^-12 for sums of cancelled values."""
+    torch.manual_seed(dim + vdim)
+    names, heads, groups = _kernels(monkeypatch), 16, 4
+    data = _ragged(cuda, [150, 1, 77, 33], [0, 40, 21, 64], 16, groups, dim, vdim, heads)
+    f = lambda *s: torch.randn(*s, device=cuda)
+    sink, bias, window, kw = (f(heads) if style == "sink" else None), (f(40, heads) if style == "bias" else None), 50 if style == "window" else 0, {}
+    if style == "cap":
+        kw = dict(softcap=5.0, slopes=torch.rand(heads, device=cuda) * 0.1)
+    if style == "sigmoid":
+        kw = dict(sigmoid=True, head_bias=f(heads) - 3)
+    args = (*data, sink, bias, 150, heads, groups, dim, vdim, window, dim ** -0.5)
+    want, got = seq.sink_attn(*args, impl=1, **kw).float(), seq.sink_attn(*args, **kw).float()
+    assert names == ["fma", "fine rows"]
+    mass = 1.0 if style != "sigmoid" else 150.0   # of the sigmoid weights
+    assert ((got - want).abs() <= 2 ** -12 * mass * float(data[1].float().abs().max()) + 2 ** -7 * want.abs()).all()
+    assert ((got - want).norm() / want.norm()).item() < 2 ** -8
