@@ -482,7 +482,7 @@ std::string latent_attn(Tensor out, Tensor q_lat, Tensor q, int64_t rot_off, Ten
   Tensor ws_o, ws_ml;
   if (die::latent_attn_uses_mfma(a)) {
     // few row tiles (decode steps): split the keys over workgroups until about 256 are in flight. The key range
-    // is bounded by the window, else by the block table's width (under a captured graph: the model length;
+    // is bounded by the window, else by the block table's width (a prompt step's: its longest context; under a captured graph: the model length;
     // splits beyond a sequence's keys exit at once)
     const int64_t rows_wg = max_q * H <= 32 ? 32 : 128;
     const int64_t tiles = S * ((max_q * H + rows_wg - 1) / rows_wg);

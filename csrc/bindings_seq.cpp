@@ -432,8 +432,8 @@ const char* sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, O
   a.nsplit = 1;
   a.chunk = 0;
   Tensor ws_o, ws_ml;
-  // The key range is bounded by the window, else by the block table's width (under a captured graph: the model
-  // length; splits beyond a sequence's keys exit at once)
+  // The key range is bounded by the window, else by the block table's width (a prompt step's: its longest context; under a captured
+  // graph: the model length; splits beyond a sequence's keys exit at once)
   int64_t bound = block_tables.size(1) * cache.size(1);
   if (window > 0) bound = std::min<int64_t>(bound, window + max_q);
   if (seg > 0) bound = std::min<int64_t>(bound, seg + max_q);

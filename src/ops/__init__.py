@@ -914,7 +914,9 @@ def moe_apply(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: torch.Ten
 
 MOE_LIBRARY_MIN_TOKENS = 256
 # Tokens from which decode steps take the products of unsorted rows, whose activation image goes with an expert's rows instead of the step's
-# (eight experts of 4096 x 14336, both products, us, sorted / unsorted: 32 tokens 459 / 470 without the sort's 5, 128 tokens 732 / 536)
+# (eight experts of 4096 x 14336, both products, us, sorted / unsorted: 32 tokens 459 / 470 without the sort's 5, 128 tokens 732 / 536). The line is
+# drawn for such experts and holds for every width: eight of 2048 x 2048 would gain from 1 token on (whole input-scaled mixture, whose sorted
+# form is the same: 8 tokens 60 / 56, 32 tokens 68 / 61).
 MOE_IDS_MIN_T = 33
 _NO_ROWS_CACHE: dict = {}
 

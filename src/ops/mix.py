@@ -230,7 +230,9 @@ def _ids_tile(n: int, k: int, gate: bool, t: int, pairs: int) -> Optional[Tuple[
     """(weight rows of a workgroup, K of a ring slot) of the expert products of a decode step, or None where none divides N
     and K. 64 x 256: of 9 tiles the best or within 3 % for 2 - 64 tokens (8 experts of 2048 x 2048 at 32 tokens, us, gated / plain
     product: 32 x 128 36.9 / 18.3, 64 x 128 33.2 / 15.9, 64 x 256 31.7 / 14.7, 128 x 128 30.0 / 17.3); above 64 rows its activation image
-    leaves no ring. Where 64 rows give less than a workgroup to every second compute unit, 32 (2 pairs: 9.0 / 7.5)."""
+    leaves no ring. Where 64 rows give less than a workgroup to every second compute unit, 32 (2 pairs: 9.0 / 7.5). K that is no multiple
+    of 128 has a tile above 64 tokens only; up to 64 it keeps the sorted products, though 64 x 64 would be faster there too (8 experts of 2048 x
+    1472, 32 tokens, output-weighted: 59 sorted, 49)."""
     wide = ((64, 256), (64, 128)) if t <= 64 else ((64, 128), (64, 64))
     narrow = ((32, 256), (32, 128)) if t <= 64 else ((32, 128),)
     few = pairs * (n // (32 if gate else 64)) <= 128
