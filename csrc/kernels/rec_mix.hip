@@ -7,7 +7,7 @@
 //                             the per-head (decay, step size) of a scalar-decay state-space layer
 //   conv_tail_update          the convolution's trailing inputs -> state
 //   selective_scan            S[c, :] <- exp(d A[c, :]) S[c, :] + d x B; y = S[c, :] . C + D x; y * silu(z): a
-//                             channel's states in the registers of 1 - 4 lanes for the whole step
+//                             channel's states in the registers of 1 - 4 lanes for the whole step (9 - 16 states: selective_scan.hip)
 //   exp_gate_scan             log-space input / forget gates under a running maximum: a wave-wide scan over tokens
 //   gated_linear_attn         S <- a S + b k v^T, o = S^T q: one workgroup per (sequence, head, block of columns), the
 //                             state in registers (four columns per group of 4 - 16 lanes); the normaliser n <- a n + b k with its
@@ -20,6 +20,7 @@
 #include "common.h"
 #include "lane_reduce.h"
 #include "rec_launchers.h"
+#include "selective_scan.h"
 
 namespace die {
 
@@ -878,15 +879,7 @@ hipError_t launch_selective_scan(const SelectiveScanArgs& a, RaggedRows r, hipSt
   if (!rows_ok(r) || a.I < 1 || a.N < 1 || a.N > 256) return hipErrorInvalidValue;
   if (a.N <= 4) return launch_scan_one<4, 1>(a, r, s);
   if (a.N <= 8) return launch_scan_one<8, 1>(a, r, s);
-  if (a.N <= 16) {
-    // a channel's states over more lanes where the channels do not fill the SIMDs with a wave each: a token is a chain of
-    // reads and exponentials that 8 or 4 states per lane shorten (1 x 1024 tokens of 4096 channels 485 us, in 2 / 4 lanes 398 / 381; 4 x 500
-    // 246, 201 / 190; 16 x 1024 497, 464 / 587; 32 x 100 69, 75 / 99)
-    const int64_t waves = ((int64_t)a.I * r.num_seqs + 63) / 64, simds = 4 * (int64_t)num_cus();
-    if (2 * waves <= simds) return launch_scan_one<4, 4>(a, r, s);
-    if (waves <= simds) return launch_scan_one<8, 2>(a, r, s);
-    return launch_scan_one<16, 1>(a, r, s);
-  }
+  if (a.N <= 16) return launch_scan_lanes(a, r, s);
   if (a.N <= 32) return launch_scan_one<16, 2>(a, r, s);
   if (a.N <= 64) return launch_scan_one<16, 4>(a, r, s);
   if (a.N <= 128) return launch_scan_one<32, 4>(a, r, s);
