@@ -249,7 +249,11 @@ void gated_delta(Tensor out, Tensor qkv32, Tensor bg, Tensor gate, Tensor norm_w
   a.eps = (float)eps;
   a.mult = (float)mult;
   a.state = state.data_ptr<float>();
-  HIP_OK(die::launch_gated_delta(a, ragged(T, positions, cu_q, state_slots), cur_stream()));
+  const die::RaggedRows rag = ragged(T, positions, cu_q, state_slots);
+  const int64_t n = die::gated_delta_work(a, rag.total_rows, rag.num_seqs);
+  const Tensor work = n > 0 ? at::empty({n}, qkv32.options()) : Tensor();
+  a.work = n > 0 ? work.data_ptr<float>() : nullptr;
+  HIP_OK(die::launch_gated_delta(a, rag, cur_stream()));
 }
 
 // q [T, H * dim], k [T, G * dim], v [T, G * vdim]: column slices of ONE projection output

@@ -25,6 +25,8 @@ namespace die {
 // sequences of 80 / 96 / 112 rows: 88 / 104 / 120 token by token, 91 / 103 / 116 in chunks), with more than four 160 (128 sequences of
 // 128 / 160 rows: 238 / 292, in chunks 253 / 301).
 void chunk_delta_cut(GatedDeltaArgs& a, int rows, int num_seqs);
+// floats of scratch (GatedDeltaArgs::work) that the step needs: 0 where no sequence goes in chunks
+int64_t chunk_delta_work(GatedDeltaArgs a, int rows, int num_seqs);
 hipError_t launch_chunk_delta(const GatedDeltaArgs& a, RaggedRows r, hipStream_t s);
 
 }  // namespace die

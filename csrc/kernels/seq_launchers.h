@@ -92,8 +92,10 @@ struct GatedDeltaArgs {
   float eps, mult;
   float* state;           // [slots, heads, dim, vdim]
   DeltaShape sh;
+  float* work;            // scratch of gated_delta_work floats, nullptr for none
   int cut = 0, longest = 0;   // set by the launcher: sequences of `cut` rows and more go in chunks, in divided steps (common.h)
 };
+int64_t gated_delta_work(const GatedDeltaArgs& a, int rows, int num_seqs);
 // Per (sequence, head), token by token: S <- g S (g per head, or per row of S); u = beta (v - S^T k); S <- S + k u^T;
 // o = S^T q, with S [dim, vdim] fp32. out[t, h, :] = mult * o / rms(o) * norm_w * gate function(gate[t, h, :]).
 hipError_t launch_gated_delta(const GatedDeltaArgs& a, RaggedRows r, hipStream_t s);

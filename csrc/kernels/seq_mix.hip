@@ -1171,6 +1171,10 @@ template <int LN, int M> static hipError_t launch_gd(const GatedDeltaArgs& a, Ra
   return vec ? launch_gd<LN, M, false, false, true>(a, r, s) : launch_gd<LN, M, false, false, false>(a, r, s);
 }
 
+int64_t gated_delta_work(const GatedDeltaArgs& a, int rows, int num_seqs) {
+  return num_seqs > 0 && rows > 0 ? chunk_delta_work(a, rows, num_seqs) : 0;
+}
+
 hipError_t launch_gated_delta(const GatedDeltaArgs& args, RaggedRows r, hipStream_t s) {
   GatedDeltaArgs a = args;
   if (r.num_seqs == 0 || r.total_rows == 0) return hipSuccess;
@@ -1178,6 +1182,7 @@ hipError_t launch_gated_delta(const GatedDeltaArgs& args, RaggedRows r, hipStrea
     return hipErrorInvalidValue;
   chunk_delta_cut(a, r.total_rows, r.num_seqs);
   if (a.cut <= r.total_rows) {
+    if (a.work == nullptr) return hipErrorInvalidValue;
     const hipError_t e = launch_chunk_delta(a, r, s);
     if (e != hipSuccess || a.cut == 0) return e;
   }
