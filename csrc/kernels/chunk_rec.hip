@@ -16,11 +16,13 @@
 // An infinite value or state makes the rows from its token on and the state NaN (a part of an infinity is NaN), where token by token some
 // of them may stay infinite; earlier rows and other sequences are as they are.
 //
-// What bounds it: the vector ALUs that cut fragments and weigh scores (about 1200 instructions per wave and chunk at dim 128
-// beside 62 matrix instructions), two waves per SIMD at 250 registers. Against the token-by-token kernels (bf16, us, before -> after):
-// 16 x 1024 tokens, 64 heads of 128 x 64 sharing q and k 794 -> 196 (2.3 TB/s of its inputs, results and states), 16 heads of
-// 128 x 128 with SiLU 1050 -> 203; 16 x 1000, 32 heads of 64 x 128 with normaliser 589 -> 220; one sequence of 1024, 64 heads
-// 410 -> 122.
+// What bounds it: instruction issue. A wave takes some 950 vector and 62 matrix instructions per chunk at dim 128 (cutting fragments, weighing
+// scores), a SIMD issues one per 4.5 - 5 cycles in all, and two waves per SIMD at 230 registers hide the rest. Against the token-by-token
+// kernels (bf16, us, before -> after): 16 x 1024 tokens, 64 heads of 128 x 64 sharing q and k 794 -> 189 (2.4 TB/s of its inputs, results and
+// states), 16 heads of 128 x 128 with SiLU 1050 -> 154; 16 x 1000, 32 heads of 64 x 128 with normaliser 589 -> 220; one sequence of 1024, 64
+// heads 410 -> 102. Of these, decays chosen where they are used and not where they are loaded (which waited for all loads of the chunk), rows
+// of whole chunks stored without a condition each, and parts cut beside the products before them: 197 -> 189, 200 -> 154, 121 -> 102. (Remainders by
+// the dot product with -1, one instruction for two: no gain, with the normaliser 3 % slower.)
 #include "common.h"
 #include "lane_reduce.h"
 #include "chunk_rec.h"
@@ -152,13 +154,8 @@ __global__ void __launch_bounds__(64 * (NW + 1), 2) chunk_linear_kernel(ChunkLin
       for (int u = 0; u < PV; ++u)
         pf[PQ + u] = *reinterpret_cast<const uint4*>(at_bytes(x, 2 * (min(u * RV + rv, last) * (uint32_t)a.xstride + cv)));
     }
-    const bool in = li <= last;
-    if (a.ab != nullptr) {
-      const float* p = a.ab + ((int64_t)(q0 + t0 + min(li, last)) * H + h) * a.abw;
-      pa = in ? p[0] : 1.0f, pb = in ? p[1] : 0.0f;
-    } else {
-      pa = in ? a.decay[h] : 1.0f, pb = in ? 1.0f : 0.0f;
-    }
+    const float* p = a.ab != nullptr ? a.ab + ((int64_t)(q0 + t0 + min(li, last)) * H + h) * a.abw : a.decay + h;
+    pa = p[0], pb = p[a.ab != nullptr ? 1 : 0];   // (as they are: a choice here would wait for all of these loads)
   };
   auto stash = [&] {
     if (ones) return;
@@ -184,7 +181,8 @@ __global__ void __launch_bounds__(64 * (NW + 1), 2) chunk_linear_kernel(ChunkLin
   const int trow = 4 * hi + (lane & 15) / 4, tcol = 16 * (lane >> 4 & 1) + 4 * (lane & 3);   // of the transposed reads
   for (int t0 = 0; t0 < L; t0 += CT) {
     const bf16_t* b = buf;
-    const float av = pa, bv = pb;
+    const bool in = li < L - t0;
+    const float av = in ? pa : 1.0f, bv = in ? (a.ab != nullptr ? pb : 1.0f) : 0.0f;
     int G = li >> 2, rr = li & 3;              // the own token's quad and place in it
     asm volatile("" : "+v"(G), "+v"(rr));      // (else some 80 masks are kept over the loop, in spilled scalar registers)
     const bool more = t0 + CT < L;
@@ -238,21 +236,26 @@ __global__ void __launch_bounds__(64 * (NW + 1), 2) chunk_linear_kernel(ChunkLin
     f32x16_t sc = {}, o = {};
     const bf16_t* qr = b + li * KP + 4 * hi;
     const bf16_t* kr = b + CT * KP + li * KP + 4 * hi;
+    // 16 channels at a time, the next ones' parts cut beside the products of the current ones: a wave's instructions issue in order
+    bf16x8_t qf[2], kf1[2], sf[2][3];
+    auto rows_of = [&](int t) { qf[t & 1] = row_frag(qr + 16 * t), kf1[t & 1] = row_frag(kr + 16 * t); };
+    auto cut = [&](int t) {
+      float x[8];
 #pragma unroll
-    for (int m = 0; m < ND; ++m)
+      for (int e = 0; e < 8; ++e) x[e] = S[t / 2][8 * (t & 1) + e];
+      split3(x, sf[t & 1]);
+    };
+    rows_of(0);
+    cut(0);
 #pragma unroll
-      for (int k2 = 0; k2 < 2; ++k2) {
-        const bf16x8_t qf = row_frag(qr + 32 * m + 16 * k2);
-        sc = mm(row_frag(kr + 32 * m + 16 * k2), qf, sc);
-        float x[8];
-        bf16x8_t f[3];
+    for (int t = 0; t < 2 * ND; ++t) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (t + 1 < 2 * ND) rows_of(t + 1), cut(t + 1);
+      sc = mm(kf1[t & 1], qf[t & 1], sc);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) x[e] = S[m][8 * k2 + e];
-        split3(x, f);
-#pragma unroll
-        for (int p = 2; p >= 0; --p) o = mm(qf, f[p], o);
-        __builtin_amdgcn_sched_barrier(0);   // one step's operands at a time: hoisted together they would spill
-      }
+      for (int p = 2; p >= 0; --p) o = mm(qf[t & 1], sf[t & 1][p], o);
+    }
+    __builtin_amdgcn_sched_barrier(0);
     // ---- weights, then P V
     const char* vb = reinterpret_cast<const char*>(b + 2 * CT * KP + 32 * (ones ? 0 : wave)) + trow * (2 * VP) + 2 * tcol;
     bf16x8_t vf[2];
@@ -317,39 +320,54 @@ __global__ void __launch_bounds__(64 * (NW + 1), 2) chunk_linear_kernel(ChunkLin
     }
     // ---- results: row i in the registers, the wave's columns in its lanes
     const int nb = L - t0;
-    const uint32_t hv = ones ? H : H * V, at = 4 * (4 * hi * hv + (ones ? 0 : li));
+    const uint32_t hv = ones ? H : H * V;
+    uint32_t at = 4 * (4 * hi * hv + (ones ? 0 : li));
+    asm volatile("" : "+v"(at));   // (else the rows' offsets are kept over the loop, in registers that spill)
     float* op = ones ? a.nq + (int64_t)(q0 + t0) * H + h : a.out + ((int64_t)(q0 + t0) * H + h) * V + col;
     const bool mine = !ones || li == 0;
+    if (nb >= CT && !ones) {   // (a condition per row costs as much as the row)
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+      for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (mine && 8 * u + 4 * hi + e < nb) *at_bytes(op, at + 4 * (8 * u + e) * hv) = o[4 * u + e] * a.qscale;
-    // ---- the state
+        for (int e = 0; e < 4; ++e) *at_bytes(op + (int64_t)(8 * u + e) * hv, at) = o[4 * u + e] * a.qscale;
+    } else {
 #pragma unroll
-    for (int m = 0; m < ND; ++m)
+      for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) S[m][e] *= all;
+        for (int e = 0; e < 4; ++e)
+          if (mine && 8 * u + 4 * hi + e < nb) *at_bytes(op, at + 4 * (8 * u + e) * hv) = o[4 * u + e] * a.qscale;
+    }
+    // ---- the state: its scaling and the values' parts beside the products
     const char* kb = reinterpret_cast<const char*>(b + CT * KP) + trow * (2 * KP) + 2 * tcol;
-#pragma unroll
-    for (int k2 = 0; k2 < 2; ++k2) {
+    bf16x8_t wf[2][3], kf[2];
+    auto weigh = [&](int k2) {
       const float4 ta = *reinterpret_cast<const float4*>(tab + CT + 16 * k2 + 4 * hi);
       const float4 tb = *reinterpret_cast<const float4*>(tab + CT + 16 * k2 + 8 + 4 * hi);
       const float tt[8] = {ta.x, ta.y, ta.z, ta.w, tb.x, tb.y, tb.z, tb.w};
       float x[8];
-      bf16x8_t f[3];
       unpack8(__builtin_bit_cast(uint4, vf[k2]), x);
 #pragma unroll
       for (int e = 0; e < 8; ++e) x[e] *= tt[e];
-      split3(x, f);
+      split3(x, wf[k2]);
+    };
+    auto fade = [&](int m) {
 #pragma unroll
-      for (int m = 0; m < ND; ++m) {
-        const bf16x8_t kf = col_frag(kb + 16 * k2 * (2 * KP) + 64 * m, 2 * KP);
+      for (int e = 0; e < 16; ++e) S[m][e] *= all;
+    };
+    auto cols_of = [&](int t) { kf[t & 1] = col_frag(kb + 16 * (t / ND) * (2 * KP) + 64 * (t % ND), 2 * KP); };
+    cols_of(0);
+    weigh(0);
+    fade(0);
 #pragma unroll
-        for (int p = 2; p >= 0; --p) S[m] = mm(kf, f[p], S[m]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+    for (int t = 0; t < 2 * ND; ++t) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (t + 1 < 2 * ND) cols_of(t + 1);
+      if (t + 1 < ND) fade(t + 1);
+      if (t == ND - 1) weigh(1);
+#pragma unroll
+      for (int p = 2; p >= 0; --p) S[t % ND] = mm(kf[t & 1], wf[t / ND][p], S[t % ND]);
     }
+    __builtin_amdgcn_sched_barrier(0);
     if (more) {
       __syncthreads();   // every wave is done with this chunk
       stash();
