@@ -9,13 +9,14 @@
 //   selective_scan            S[c, :] <- exp(d A[c, :]) S[c, :] + d x B; y = S[c, :] . C + D x; y * silu(z): a
 //                             channel's states in the registers of 1 - 4 lanes for the whole step (9 - 16 states: selective_scan.hip)
 //   exp_gate_scan             log-space input / forget gates under a running maximum: a wave-wide scan over tokens
-//   gated_linear_attn         S <- a S + b k v^T, o = S^T q: one workgroup per (sequence, head, block of columns), the
+//   gated_linear_attn         S <- a S + b k v^T, o = S^T q (prompt portions: chunk_rec.hip, chunk_channel.hip): one workgroup per (sequence, head, block of columns), the
 //                             state in registers (four columns per group of 4 - 16 lanes); the normaliser n <- a n + b k with its
 //                             read-out n . q rides on the first wave; optionally a decay per row of S,
 //                             sigmoid(z)^(1/tau), computed while a trip is staged
 //   head_norm_gate            (o / (max(|n . q|, floor) + 1e-6), optional,) per-head RMS norm, weight, sigmoid or SiLU gate
 //   skip_gate_group_norm      (o + D x) * silu(z), RMS norm in equal parts of the row, weight
 //   pair_post_norm_residual   resid += mult * rms((rms(y1) w1 + rms(y2) w2) / 2) * (1 + w)
+#include "chunk_channel.h"
 #include "chunk_rec.h"
 #include "common.h"
 #include "lane_reduce.h"
@@ -917,6 +918,7 @@ hipError_t launch_gated_linear_attn(const GatedLinearArgs& args, RaggedRows r, h
       if (e != hipSuccess || c.cut == 0) return e;
     }
   }
+  if (chunk_channel_fits(a, r.total_rows, r.num_seqs)) return launch_chunk_channel(a, r, s);
   if (a.dim <= 16) return launch_gla_dp<4, 1>(a, r, s);
   if (a.dim <= 32) return launch_gla_dp<8, 1>(a, r, s);
   if (a.dim <= 64) return launch_gla_dp<16, 1>(a, r, s);

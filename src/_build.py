@@ -97,7 +97,7 @@ def build_kernels(force: bool = False, jobs: int = 8, verbose: bool = False) -> 
     return out
 
 
-MIX_KERNELS = ["mix_ops", "latent_attn", "moe", "moe_gemm", "seq_mix", "sink_attn", "lin_mix", "rec_mix", "selective_scan", "chunk_rec", "chunk_delta", "conv_mix"]
+MIX_KERNELS = ["mix_ops", "latent_attn", "moe", "moe_gemm", "seq_mix", "sink_attn", "lin_mix", "rec_mix", "selective_scan", "chunk_rec", "chunk_delta", "chunk_channel", "conv_mix"]
 MIX_BINDINGS = ["bindings_mix", "bindings_seq", "bindings_lin", "bindings_rec", "bindings_conv"]
 
 

@@ -1,0 +1,81 @@
+"""Linear attention with a decay per key channel: prompt portions in chunks on the matrix cores against a float64 evaluation.
+
+Both sides hold the same bf16 inputs. The kernel's decays come from the hardware's exponential and logarithm, some 2^-22 of an exponent of
+at most 1 per token; over a few hundred tokens a state's terms are off by 1e-5 of their size at most, and results by as much of their root
+mean square. A dropped or doubled token moves them by 1e-2 and more."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from src.ops import rec, seq
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(lens, past, H, G, D, V, pad=0):
+    T, S = sum(lens), len(lens)
+    x = torch.randn(T, 2 * G * D + H * V + pad).bfloat16()[:, pad:]
+    z, zb = torch.randn(T, H * D + pad).bfloat16()[:, pad:], torch.randn(H * D) + 1
+    z[torch.rand(T, H * D) < 0.02] = -300.0   # channels that are dropped
+    state, slots = torch.randn(S + 1, H, D, V) * 0.3, torch.randperm(S + 1)[:S].int()
+    pos = torch.cat([torch.arange(n) + p for n, p in zip(lens, past)])
+    return x, z, zb, state, slots, pos, torch.tensor([0] + lens).cumsum(0).int()
+
+
+def _run(cuda, args, H, G, D, V, scale=0.3, tau=16.0):
+    x, z, zb, state, slots, pos, cu = args
+    pad = x.stride(0) - x.shape[1]
+    wide = lambda t: F.pad(t, (pad, 0)).to(cuda)[:, pad:]
+    st = state.to(cuda)
+    o, _ = rec.gated_linear_attn(wide(x), 0, G * D, 2 * G * D, None, st, None, H, G, D, V, scale, seq.Ragged(pos.to(cuda), cu.to(cuda), slots.to(cuda)),
+                                 z=wide(z), z_bias=zb.to(cuda), tau=tau)
+    return o.cpu(), st.cpu()
+
+
+def _exact(args, H, G, D, V, scale=0.3, tau=16.0):
+    x, z, zb, state, slots, pos, cu = args
+    T = x.shape[0]
+    q, k = (x[:, i * G * D:(i + 1) * G * D].double().view(T, G, D).repeat_interleave(H // G, 1) for i in (0, 1))
+    v = x[:, 2 * G * D:].double().view(T, H, V)
+    dec = torch.exp(F.logsigmoid(z.double() + zb.double()) / tau).view(T, H, D)
+    out, st = torch.empty(T, H, V, dtype=torch.float64), state.double()
+    for s in range(len(slots)):
+        S = st[slots[s]] if pos[cu[s]] > 0 else torch.zeros(H, D, V, dtype=torch.float64)
+        for t in range(int(cu[s]), int(cu[s + 1])):
+            S = dec[t][:, :, None] * S + k[t][:, :, None] * v[t][:, None, :]
+            out[t] = (S * (q[t] * scale)[:, :, None]).sum(1)
+        st[slots[s]] = S
+    return out.reshape(T, H * V), st
+
+
+@pytest.mark.parametrize("H,G,D,V,pad", [(4, 4, 64, 128, 0), (3, 1, 64, 64, 1), (2, 2, 64, 256, 3), (2, 1, 128, 128, 0), (4, 2, 128, 64, 1)])
+@pytest.mark.parametrize("lens,past", [([16], [0]), ([17, 1, 64, 33], [0, 4, 9, 0]), ([48, 15, 130], [2, 0, 0])])
+def test_portions(cuda, H, G, D, V, pad, lens, past):
+    torch.manual_seed(sum(lens) + D + V)
+    args = _inputs(lens, past, H, G, D, V, pad)
+    want, ws = _exact(args, H, G, D, V)
+    got, st = _run(cuda, args, H, G, D, V)
+    assert (got.double() - want).abs().max() <= 1e-5 * want.square().mean().sqrt() + 1e-5 * want.abs().max()
+    assert (st.double() - ws).abs().max() <= 1e-5 * ws.abs().max()
+
+
+@pytest.mark.parametrize("what", ["k", "v", "z"])
+def test_later_tokens_do_not_reach_earlier_rows(cuda, what):
+    """An infinite key or value or a NaN decay changes its own row and the later ones of its sequence, no others."""
+    torch.manual_seed(3)
+    H, D, V, at = 2, 64, 128, 60
+    args = _inputs([40, 40, 41], [0, 0, 7], H, H, D, V)
+    want, ws = _run(cuda, args, H, H, D, V)
+    if what == "z":
+        args[1][at, 5] = float("nan")
+    else:
+        args[0][at, H * D + 5 if what == "k" else 2 * H * D + 5] = float("inf")
+    got, st = _run(cuda, args, H, H, D, V)
+    keep = torch.ones(121, dtype=torch.bool)
+    keep[at:80] = False
+    assert torch.equal(got[keep], want[keep])
+    assert torch.equal(got[at:80, V:], want[at:80, V:])
+    assert not torch.isfinite(got[at:80, 5]).any()
+    slot = int(args[4][1])
+    assert torch.equal(st[[i for i in range(4) if i != slot]], ws[[i for i in range(4) if i != slot]]) and not torch.isfinite(st[slot, 0, :, 5]).all()
