@@ -489,7 +489,10 @@ std::string latent_attn(Tensor out, Tensor q_lat, Tensor q, int64_t rot_off, Ten
     int64_t bound = block_tables.size(1) * cache.size(1);
     if (window > 0) bound = std::min<int64_t>(bound, window + max_q);
     int64_t ns = std::min<int64_t>({(int64_t)16, 512 / std::max<int64_t>(1, tiles), (bound + 63) / 64});
-    if (ns > 1 && a.impl == 0 && die::latent_attn_fits_rows(a)) {
+    if (die::latent_attn_decodes(a)) {
+      // one workgroup per compute unit: twice as many write twice the partial results (32 sequences of 750 - 1500 keys, 16 heads 12.2 + 4.7 us, 14.3 + 5.9)
+      ns = std::min<int64_t>({(int64_t)16, at::cuda::getCurrentDeviceProperties()->multiProcessorCount / std::max<int64_t>(1, S * ((H + 15) / 16)), (bound + 127) / 128});
+    } else if (ns > 1 && a.impl == 0 && die::latent_attn_fits_rows(a)) {
       const int64_t seen = window > 0 ? std::min<int64_t>(bound, window + (H + 63) / H + 31) : bound;   // of a tile of 64 rows
       const int64_t most = ns;
       // (times fitted to 524 random steps of rank 256 + 32 in 1 to 16 splits)
@@ -499,7 +502,7 @@ std::string latent_attn(Tensor out, Tensor q_lat, Tensor q, int64_t rot_off, Ten
     }
     if (ns > 1) {
       a.chunk = (int)((((bound + ns - 1) / ns) + 31) / 32 * 32);
-      a.nsplit = (int)((bound + a.chunk - 1) / a.chunk);
+      a.nsplit = die::latent_attn_decodes(a) ? (int)ns : (int)((bound + a.chunk - 1) / a.chunk);
       if (a.nsplit > 1) {
         ws_o = at::empty({a.nsplit, H * T, rank}, q_lat.options().dtype(at::kFloat));
         ws_ml = at::empty({a.nsplit, H * T, 2}, q_lat.options().dtype(at::kFloat));

@@ -414,25 +414,244 @@ __global__ void __launch_bounds__(64 * NW) latent_attn_mfma_kernel(LatentAttnArg
   }
 }
 
-// out[row] = sum_z O_z 2^(m_z - m*) / sum_z l_z 2^(m_z - m*), m* = max_z m_z (running maxima in log2 units).
+// out[row] = sum_z O_z 2^(m_z - m*) / sum_z l_z 2^(m_z - m*), m* = max_z m_z (running maxima in log2 units). One wave per row, 4 columns per
+// lane and pass; the weights of 64 splits at a time on its lanes, so that the splits' rows are loaded together (with one after the other
+// behind its weight 16 splits of 512 rows took 10.6 us).
 __global__ void __launch_bounds__(256) latent_attn_merge_kernel(bf16_t* out, const float* ws_o, const float* ws_ml,
                                                                 int nsplit, int64_t rows, int R) {
-  const int64_t row = blockIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
   float mstar = -1e30f;
-  for (int z = 0; z < nsplit; ++z) mstar = fmaxf(mstar, ws_ml[((int64_t)z * rows + row) * 2]);
+  for (int z = lane; z < nsplit; z += 64) mstar = fmaxf(mstar, ws_ml[((int64_t)z * rows + row) * 2]);
+  mstar = wave_max(mstar);
   float lsum = 0.f;
-  for (int z = 0; z < nsplit; ++z) {
-    const float lz = ws_ml[((int64_t)z * rows + row) * 2 + 1];
-    if (lz > 0.f) lsum += lz * exp2f(ws_ml[((int64_t)z * rows + row) * 2] - mstar);
+  for (int z0 = 0; z0 < nsplit; z0 += 64) {
+    const int z = min(z0 + lane, nsplit - 1);
+    const float2 ml = *reinterpret_cast<const float2*>(ws_ml + ((int64_t)z * rows + row) * 2);
+    lsum += z0 + lane < nsplit && ml.y > 0.f ? ml.y * exp2f(ml.x - mstar) : 0.f;
   }
+  lsum = wave_sum(lsum);
   const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
-  for (int c = threadIdx.x; c < R; c += 256) {
-    float acc = 0.f;
-    for (int z = 0; z < nsplit; ++z) {
-      const float lz = ws_ml[((int64_t)z * rows + row) * 2 + 1];
-      if (lz > 0.f) acc += ws_o[((int64_t)z * rows + row) * R + c] * exp2f(ws_ml[((int64_t)z * rows + row) * 2] - mstar);
+  for (int c0 = 0; c0 < R; c0 += 256) {
+    const int c = c0 + 4 * lane;
+    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int z0 = 0; z0 < nsplit; z0 += 64) {
+      const int zl = min(z0 + lane, nsplit - 1);
+      const float2 ml = *reinterpret_cast<const float2*>(ws_ml + ((int64_t)zl * rows + row) * 2);
+      const float wl = z0 + lane < nsplit && ml.y > 0.f ? exp2f(ml.x - mstar) : 0.f;
+      const uint64_t full = __ballot(wl != 0.f);
+      if (full == 0) continue;
+      const int some = __builtin_ctzll(full), n = 64 - __builtin_clzll(full);
+      if (c < R) {
+#pragma unroll 8
+        for (int z = 0; z < n; ++z) {   // (an empty split's row is not written: another's is read, and counts nothing)
+          const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(wl), z));
+          const float4 o = *reinterpret_cast<const float4*>(ws_o + ((int64_t)(z0 + (w != 0.f ? z : some)) * rows + row) * R + c);
+          acc.x = fmaf(o.x, w, acc.x), acc.y = fmaf(o.y, w, acc.y), acc.z = fmaf(o.z, w, acc.z), acc.w = fmaf(o.w, w, acc.w);
+        }
+      }
     }
-    out[row * R + c] = f2bf(acc * inv);
+    if (c < R) *reinterpret_cast<uint2*>(out + row * R + c) = make_uint2(pack2(acc.x * inv, acc.y * inv), pack2(acc.z * inv, acc.w * inv));
+  }
+}
+inline hipError_t launch_merge(const LatentAttnArgs& a, hipStream_t s) {
+  const int64_t rows = (int64_t)a.heads * a.total_q;
+  hipLaunchKernelGGL(latent_attn_merge_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, s, reinterpret_cast<bf16_t*>(a.out), a.ws_o, a.ws_ml,
+                     a.nsplit, rows, a.sh.rank);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------------------------------
+// Decode steps (one row per sequence): 16 heads of a sequence per workgroup, keys in tiles of 32 over its waves and, with nsplit > 1, over
+// several workgroups: wave w of all of them takes tiles w, w + waves, .., so that every wave has work whatever the sequence's length. A wave
+// loads a tile's rows straight into operands of the scores (key = lane % 16, all loads in flight together, the table's entries a tile
+// ahead), writes their latent columns to LDS for the weighted sum's transposed reads, and has the next tile's rows loaded during softmax and
+// sum. Waves share no barrier before the end, where their sums are brought to one maximum and added. Against one wave per workgroup that staged
+// tiles in LDS for both products, by divisions at run time (rank 256 + 32, main kernel + merge, us): 32 sequences of 750 - 1500 keys, 16 heads
+// 36 + 10 -> 12 + 4.7 (21 MB of rows: 4 at the copy rate, latency of three tiles), 64 of 1000 - 2000, 32 heads 87 + 9 -> 24 + 4 (4.0 TB/s with L2), 3 of
+// 600 24 + 8 -> 9 + 4, 58 of 10 17 -> 8.
+template <int NDB, int NROT> struct DecodeTile {
+  static constexpr int R = 32 * NDB, NK = NDB + (NROT + 1) / 2, DK = R + 16 * NROT;   // latent columns, 32-wide steps of a row, its width
+  static constexpr int PB = 2 * R + 32;                                               // pitch in LDS, bytes: 4 rows on different banks
+  static constexpr int OP = R + 4;                                                    // pitch of a head's sums (floats)
+  static constexpr int wave = 32 * PB > 64 * OP ? 32 * PB : 64 * OP;
+  static constexpr int total = 4 * wave + 4 * 16 * 2 * 4;
+};
+template <int NDB, int NROT>
+__global__ void __launch_bounds__(256, 2) latent_attn_decode_kernel(LatentAttnArgs a, int hblocks) {
+  using Z = DecodeTile<NDB, NROT>;
+  constexpr int R = Z::R, NK = Z::NK, ND = R / 16;
+  extern __shared__ __attribute__((aligned(16))) char dsm[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, lg = lane >> 4;
+  // a sequence's blocks of heads read the same rows: they go to one XCD (workgroups are dealt to the 8 XCDs in turn), one after the other
+  const int ns = max(1, a.nsplit), u = blockIdx.x / (8 * hblocks) * 8 + blockIdx.x % 8, hb = blockIdx.x / 8 % hblocks;
+  if (u >= a.num_seqs * ns) return;
+  const int s = u / ns, z = u % ns, H = a.heads, T = a.total_q;
+  const int h0 = 16 * hb, h = min(h0 + li, H - 1);
+  const int p = (int)a.positions[s], ctx = a.ctx_lens[s];
+  const int jlo = a.window > 0 ? max(0, p - a.window + 1) : 0, jhi = min(p, ctx - 1);
+  float* const ml = reinterpret_cast<float*>(dsm + 4 * Z::wave);   // [4][16][2]: maximum, sum of every wave
+  const int64_t rows_all = (int64_t)H * T;
+  if (jlo + 128 * z > jhi) {   // an empty split: it only reports that it holds nothing
+    if (ns > 1 && tid < min(16, H - h0)) {
+      float* w = a.ws_ml + ((int64_t)z * rows_all + (int64_t)(h0 + tid) * T + s) * 2;
+      w[0] = -1e30f, w[1] = 0.f;
+    }
+    if (ns > 1) return;
+  }
+  const bf16_t* cache = reinterpret_cast<const bf16_t*>(a.cache);
+  const int* bt = a.block_tables + (int64_t)s * a.bt_stride;
+  const int bs_shift = (a.block_size & (a.block_size - 1)) == 0 ? __builtin_ctz(a.block_size) : -1;
+  auto block_of = [&](int j) { return bs_shift >= 0 ? j >> bs_shift : j / a.block_size; };
+  int blk[2];          // block of key 16 t + li of the tile that is loaded next
+  bf16x8_t kf[2][NK];
+  auto ask = [&](int j0) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) blk[t] = bt[block_of(min(j0 + 16 * t + li, jhi))];   // (keys beyond the last repeat it: their weights are zero)
+  };
+  auto load = [&](int j0) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int j = min(j0 + 16 * t + li, jhi);
+      const bf16_t* row = cache + ((int64_t)blk[t] * a.block_size + (j - block_of(j) * a.block_size)) * Z::DK + 8 * lg;
+#pragma unroll
+      for (int c = 0; c < NK; ++c)
+        kf[t][c] = *reinterpret_cast<const bf16x8_t*>(row + (NROT == 1 && c == NDB && lg >= 2 ? 0 : 32 * c));
+    }
+  };
+  const int step = 128 * ns;
+  int j0 = jlo + 32 * (4 * z + wave);
+  const bool any = j0 <= jhi;
+  if (any) {
+    ask(j0);
+    load(j0);
+    ask(j0 + step);
+  }
+  // queries: the latent part as it lies, the rotary part turned in fp32
+  bf16x8_t qf[NK];
+  const bool mine = h0 + li < H;
+  {
+    const bf16_t* ql = reinterpret_cast<const bf16_t*>(a.q_lat) + ((int64_t)h * T + s) * R + 8 * lg;
+#pragma unroll
+    for (int c = 0; c < NDB; ++c) {
+      const uint4 w = *reinterpret_cast<const uint4*>(ql + 32 * c);
+      qf[c] = __builtin_bit_cast(bf16x8_t, mine ? w : make_uint4(0, 0, 0, 0));
+    }
+    const bf16_t* qr = reinterpret_cast<const bf16_t*>(a.q_rot) + (int64_t)s * a.q_stride + (int64_t)h * a.q_hstride;
+#pragma unroll
+    for (int c = NDB; c < NK; ++c) {
+      uint32_t w[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int i = 16 * (c - NDB) + 4 * lg + e;   // pair of dims 2 i, 2 i + 1
+        const bool in = mine && 2 * i < a.sh.rot_dim;
+        const float x = in ? bf2f(qr[2 * i]) : 0.f, y = in ? bf2f(qr[2 * i + 1]) : 0.f;
+        float sn = 0.f, cs = 1.0f;
+        if (in && i < a.sh.rot_pairs) __sincosf((float)p * a.sh.inv_freq[i], &sn, &cs);
+        w[e] = pack2(x * cs - y * sn, y * cs + x * sn);
+      }
+      qf[c] = __builtin_bit_cast(bf16x8_t, make_uint4(w[0], w[1], w[2], w[3]));
+    }
+  }
+  constexpr float LOG2E = 1.4426950408889634f;
+  const float sl2 = a.scale * LOG2E;
+  const bool has_sink = a.sink != nullptr && z == 0 && wave == 0;
+  float m = has_sink ? a.sink[h] * LOG2E : -1e30f, l = has_sink && lg == 0 ? 1.0f : 0.0f;
+  f32x4_t o[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d) o[d] = f32x4_t{};
+  char* const mem = dsm + wave * Z::wave;
+  char* const wr = mem + li * Z::PB + 16 * lg;
+  const char* const rd = mem + (4 * lg + (li >> 2)) * Z::PB + 8 * (li & 3);
+  for (; j0 <= jhi; j0 += step) {
+    f32x4_t sc[2] = {};
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int c = 0; c < NK; ++c) {
+        bf16x8_t k = kf[t][c];
+        if (NROT == 1 && c == NDB && lg >= 2) k = bf16x8_t{};
+        sc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k, qf[c], sc[t], 0, 0, 0);
+      }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int c = 0; c < NDB; ++c) *reinterpret_cast<bf16x8_t*>(wr + 16 * t * Z::PB + 64 * c) = kf[t][c];
+    if (j0 + step <= jhi) {
+      load(j0 + step);
+      ask(j0 + 2 * step);
+    }
+    float top = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float x = j0 + 16 * t + 4 * lg + e <= jhi ? sc[t][e] * sl2 : -INFINITY;
+        sc[t][e] = x;
+        top = fmaxf(top, x);
+      }
+    const float mn = fmaxf(m, xor16_max(xor32_max(top)));
+    const float alpha = exp2f(m - mn);
+    l *= alpha;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        sc[t][e] = exp2f(sc[t][e] - mn);
+        l += sc[t][e];
+      }
+    m = mn;
+    const bf16x8_t pf = __builtin_bit_cast(
+        bf16x8_t, make_uint4(pack2(sc[0][0], sc[0][1]), pack2(sc[0][2], sc[0][3]), pack2(sc[1][0], sc[1][1]), pack2(sc[1][2], sc[1][3])));
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    if (__ballot(alpha != 1.0f) != 0) {
+#pragma unroll
+      for (int d = 0; d < ND; ++d) o[d] *= alpha;
+    }
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(rd + 32 * d));
+      const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(rd + 16 * Z::PB + 32 * d));
+      const short8_t v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, v), pf, o[d], 0, 0, 0);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the tile is read before the next one replaces it
+    __builtin_amdgcn_wave_barrier();
+  }
+  // one maximum for the waves, then the sum of their results
+  l = xor16_sum(xor32_sum(l));
+  if (lane < 16) ml[(wave * 16 + lane) * 2] = m, ml[(wave * 16 + lane) * 2 + 1] = l;
+  __syncthreads();
+  float mt = ml[2 * li];
+#pragma unroll
+  for (int w = 1; w < 4; ++w) mt = fmaxf(mt, ml[(16 * w + li) * 2]);
+  const float f = exp2f(m - mt);
+  float* const mo = reinterpret_cast<float*>(mem) + li * Z::OP + 4 * lg;   // (the wave's own part: its tiles are done)
+#pragma unroll
+  for (int d = 0; d < ND; ++d) *reinterpret_cast<f32x4_t*>(mo + 16 * d) = o[d] * f;
+  __syncthreads();
+  for (int e = tid; e < 16 * R / 4; e += 256) {
+    const int hd = e / (R / 4), c = 4 * (e % (R / 4));
+    if (h0 + hd >= H) break;
+    f32x4_t v = {};
+    float mx = ml[2 * hd], lt = 0.f;
+#pragma unroll
+    for (int w = 1; w < 4; ++w) mx = fmaxf(mx, ml[(16 * w + hd) * 2]);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      v += *reinterpret_cast<const f32x4_t*>(dsm + w * Z::wave + 4 * (hd * Z::OP + c));
+      lt += ml[(16 * w + hd) * 2 + 1] * exp2f(ml[(16 * w + hd) * 2] - mx);
+    }
+    const int64_t row = (int64_t)(h0 + hd) * T + s;
+    if (ns > 1) {
+      *reinterpret_cast<f32x4_t*>(a.ws_o + ((int64_t)z * rows_all + row) * R + c) = v;
+      if (c == 0) *reinterpret_cast<float2*>(a.ws_ml + ((int64_t)z * rows_all + row) * 2) = make_float2(mx, lt);
+    } else {
+      const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+      *reinterpret_cast<uint2*>(reinterpret_cast<bf16_t*>(a.out) + row * R + c) = make_uint2(pack2(v[0] * inv, v[1] * inv), pack2(v[2] * inv, v[3] * inv));
+    }
   }
 }
 
@@ -458,10 +677,7 @@ template <int NDB, int NW> hipError_t launch_mfma(const LatentAttnArgs& a, hipSt
   hipLaunchKernelGGL(fn, grid, dim3(64 * NW), mfma_lds_bytes(kp, NW), s, a, kp);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || a.nsplit <= 1) return e;
-  hipLaunchKernelGGL(latent_attn_merge_kernel, dim3((unsigned)((int64_t)a.heads * a.total_q)), dim3(256), 0, s,
-                     reinterpret_cast<bf16_t*>(a.out), a.ws_o, a.ws_ml, a.nsplit, (int64_t)a.heads * a.total_q,
-                     a.sh.rank);
-  return hipGetLastError();
+  return launch_merge(a, s);
 }
 
 inline bool mfma_ok(const LatentAttnArgs& a) {
@@ -469,6 +685,31 @@ inline bool mfma_ok(const LatentAttnArgs& a) {
   return !a.f32 && r % 32 == 0 && r <= 256 && a.sh.rot_dim % 16 == 0 && a.sh.rot_dim <= 128 &&
          (reinterpret_cast<uintptr_t>(a.q_lat) & 15) == 0 && (reinterpret_cast<uintptr_t>(a.cache) & 15) == 0 &&
          (reinterpret_cast<uintptr_t>(a.out) & 7) == 0;
+}
+
+// decode steps of the usual row widths
+inline bool decode_fits(const LatentAttnArgs& a) {
+  const int r = a.sh.rank, d = a.sh.rot_dim;
+  return a.impl == 0 && a.cu_q == nullptr && a.max_q == 1 && mfma_ok(a) && (r == 64 || r == 128 || r == 256) && (d == 0 || d == 16 || d == 32 || d == 64);
+}
+template <int NDB, int NROT> hipError_t launch_decode(const LatentAttnArgs& a, hipStream_t s) {
+  const auto fn = latent_attn_decode_kernel<NDB, NROT>;
+  constexpr int smem = DecodeTile<NDB, NROT>::total;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+  if (e != hipSuccess) return e;
+  const int hb = (a.heads + 15) / 16;
+  const int64_t units = (int64_t)a.num_seqs * max(1, a.nsplit);
+  hipLaunchKernelGGL(fn, dim3((unsigned)((units + 7) / 8 * 8 * hb)), dim3(256), smem, s, a, hb);
+  if (a.nsplit <= 1) return hipGetLastError();
+  const hipError_t e2 = hipGetLastError();
+  return e2 != hipSuccess ? e2 : launch_merge(a, s);
+}
+template <int NDB> hipError_t launch_decode_rot(const LatentAttnArgs& a, hipStream_t s) {
+  if (a.sh.rot_dim == 0) return launch_decode<NDB, 0>(a, s);
+  return a.sh.rot_dim == 16 ? launch_decode<NDB, 1>(a, s) : a.sh.rot_dim == 32 ? launch_decode<NDB, 2>(a, s) : launch_decode<NDB, 4>(a, s);
+}
+hipError_t launch_decode_any(const LatentAttnArgs& a, hipStream_t s) {
+  return a.sh.rank == 64 ? launch_decode_rot<2>(a, s) : a.sh.rank == 128 ? launch_decode_rot<4>(a, s) : launch_decode_rot<8>(a, s);
 }
 
 template <int NW> hipError_t launch_mfma_ndb(const LatentAttnArgs& a, hipStream_t s) {
@@ -1053,6 +1294,7 @@ hipError_t launch_mfma_rq_any(const LatentAttnArgs& a, hipStream_t s) {
 }
 
 hipError_t launch_mfma_any(const LatentAttnArgs& a, hipStream_t s) {
+  if (decode_fits(a)) return launch_decode_any(a, s);
   if (a.impl != 3 && a.nsplit <= 1 && mfma_rq_fits(a)) return launch_mfma_rq_any(a, s);
   // one wave per workgroup when a sequence brings at most 32 rows (decode steps): small LDS, many workgroups
   return (int64_t)a.max_q * a.heads <= 32 ? launch_mfma_ndb<1>(a, s) : launch_mfma_ndb<4>(a, s);
@@ -1098,6 +1340,7 @@ template <bool F32> hipError_t launch_bk(const LatentAttnArgs& a, hipStream_t s)
 }  // namespace
 
 bool latent_attn_uses_mfma(const LatentAttnArgs& a) { return a.impl != 1 && mfma_ok(a); }
+bool latent_attn_decodes(const LatentAttnArgs& a) { return decode_fits(a); }
 bool latent_attn_fits_rows(const LatentAttnArgs& a) { return latent_attn_uses_mfma(a) && a.impl != 3 && mfma_rq_fits(a); }
 
 const char* latent_attn_form(const LatentAttnArgs& a) {
@@ -1106,6 +1349,7 @@ const char* latent_attn_form(const LatentAttnArgs& a) {
 }
 
 const char* latent_attn_kernel(const LatentAttnArgs& a) {
+  if (decode_fits(a)) return "decode";
   const char* form = latent_attn_form(a);
   if (form[0] == 'r' && wide_takes(a)) return "wide";
   return form[0] == 's' && a.fine ? "fine split" : form;

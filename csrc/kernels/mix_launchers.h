@@ -128,6 +128,8 @@ hipError_t launch_latent_attn(const LatentAttnArgs& a, hipStream_t s);
 // whether launch_latent_attn would run the matrix-core kernel for these arguments (the split workspace is only
 // used by it)
 bool latent_attn_uses_mfma(const LatentAttnArgs& a);
+// whether the kernel for decode steps would run (keys then split in tiles of 32 dealt out in turn, not in chunks)
+bool latent_attn_decodes(const LatentAttnArgs& a);
 // whether the kernel for prompt-sized steps would run if the keys are not split
 bool latent_attn_fits_rows(const LatentAttnArgs& a);
 // the kernel that launch_latent_attn runs: "rows" (matrix cores, queries in registers), "tiles" (queries in LDS), "split" (the same,
