@@ -443,11 +443,14 @@ const char* sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, O
   if (seg > 0) bound = std::min<int64_t>(bound, seg + max_q);
   int64_t ns = 1;
   if (die::sink_attn_uses_decode(a)) {
-    // decode steps: a workgroup per (sequence, key/value head, split); trips of 128 keys, splits until about 2048
-    // workgroups are in flight
-    const int64_t wgs = S * kv_heads;
-    ns = std::min<int64_t>({(int64_t)128, std::max<int64_t>(1, 2048 / std::max<int64_t>(1, wgs)), (bound + 127) / 128});
-    if (ns > 1) a.chunk = (int)((((bound + ns - 1) / ns) + 127) / 128 * 128);
+    // decode steps: a workgroup per (sequence, key/value head, split), which take trips of 128 keys in turn. Two workgroups per compute unit hold
+    // enough loads in flight; more splits write and merge more partial results (32 sequences of 1000 - 2000 keys, 4 groups of 128 + 128: 16
+    // splits 32.0 us, 4 27.6; 64 of 8 groups 42, one split and no merge 33). A little more than one or two workgroups per compute unit would leave
+    // most of them waiting for a few: those are cut finer (40 sequences of 8 groups in 1 / 2 / 5 splits 50.2 / 52.3 / 47.7, 68 in 1 / 3 54.7 / 50.8).
+    const int64_t wgs = std::max<int64_t>(1, S * kv_heads), cus = at::cuda::getCurrentDeviceProperties()->multiProcessorCount;
+    ns = wgs > cus && 3 * wgs <= 4 * cus ? 5 : wgs > 2 * cus && 3 * wgs <= 7 * cus ? 3 : std::max<int64_t>(1, 2 * cus / wgs);
+    ns = std::min<int64_t>({(int64_t)128, ns, (bound + 127) / 128});
+    a.nsplit = (int)ns;
   } else if (die::sink_attn_uses_mfma(a)) {
     // few row tiles: split the keys over workgroups until about 2048 are in flight, or less where that is estimated to be faster (a gate
     // is applied to the merged fp32 rows, without splits to rounded ones: such steps keep their splits)
@@ -471,7 +474,7 @@ const char* sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, O
     if (ns > 1) a.chunk = (int)((((bound + ns - 1) / ns) + 31) / 32 * 32);
   }
   if (ns > 1) {
-    a.nsplit = (int)((bound + a.chunk - 1) / a.chunk);
+    if (a.chunk > 0) a.nsplit = (int)((bound + a.chunk - 1) / a.chunk);
     if (a.nsplit > 1) {
       ws_o = at::empty({a.nsplit, T * heads, vdim}, q.options().dtype(at::kFloat));
       ws_ml = at::empty({a.nsplit, T * heads, 2}, q.options().dtype(at::kFloat));

@@ -1154,13 +1154,13 @@ __device__ __forceinline__ float gated_out(const SinkAttnArgs& a, int64_t t, int
 //            64 / VL keys of a pass
 // The waves' sums meet in LDS, rescaled to one maximum. Bound by the loads in flight: 16 KB per wave, 3 waves per SIMD where 168
 // registers hold them (values are read after the keys' products free registers). Keys 128 at a time per workgroup, with barriers
-// between scores, softmax and values and shuffles for every sum, took 62 us of 73 (1.6 TB/s) where this takes 28 of 36: 32 sequences
-// of about 1500 keys, 16 heads in 4 groups, dim = vdim = 128; 64 sequences with 32 heads 194 -> 91 (4.3 TB/s).
+// between scores, softmax and values and shuffles for every sum, took 62 us of 73 (1.6 TB/s) where this takes 24 of 33: 32 sequences
+// of about 1500 keys, 16 heads in 4 groups, dim = vdim = 128 (4.1 TB/s; in 16 splits of 128 keys, one trip each, 28 of 39); 64 sequences with 32
+// heads 194 -> 91.
 // Splits write unnormalised sums + (max, sum) to the workspace and
 // sink_attn_merge_kernel combines them.
 template <int R, int NKC, int VL, int KT, bool SIG>
-__global__ void __launch_bounds__(256, R < 8 && R * NKC * VL < 512 && NKC * VL < 256 ? 3 : 2) sink_attn_decode_kernel(SinkAttnArgs a, float* ws_o, float* ws_ml, int nsplit,
-                                                              int chunk) {
+__global__ void __launch_bounds__(256, R < 8 && R * NKC * VL < 512 && NKC * VL < 256 ? 3 : 2) sink_attn_decode_kernel(SinkAttnArgs a, float* ws_o, float* ws_ml, int nsplit) {
   constexpr int KPT = 16 * KT, NV = 64 / VL, NPV = KPT / NV, WK = KPT + 1;
   extern __shared__ __attribute__((aligned(16))) float dsm[];
   const int z = blockIdx.x, s = blockIdx.y, g = blockIdx.z, tid = threadIdx.x, lane = tid & 63;
@@ -1171,15 +1171,11 @@ __global__ void __launch_bounds__(256, R < 8 && R * NKC * VL < 512 && NKC * VL <
   const int H = a.heads, G = a.kv_heads, QPG = H / G, D = a.dim, DV = a.vdim, roww = D + DV;
   const int p = (int)a.positions[s];
   const int ctx = a.ctx_lens[s];
-  int jlo = first_key(a, p);
-  int jhi = min(p, ctx - 1);
-  if (nsplit > 1) {
-    jlo += z * chunk;
-    jhi = min(jhi, jlo + chunk - 1);
-  }
+  // wave w of all splits takes trips w, w + waves, ..: each has its share of the keys that are there, however many the table has room for
+  const int jlo = first_key(a, p), jhi = min(p, ctx - 1), step = 4 * KPT * nsplit;
   const int64_t wrows = (int64_t)a.total_q * H;
-  if (jlo > jhi) {   // an empty split: it only reports that it holds nothing
-    if (nsplit > 1 && tid < QPG) {
+  if (jlo + 4 * KPT * z > jhi && nsplit > 1) {   // an empty split: it only reports that it holds nothing
+    if (tid < QPG) {
       const int64_t orow = (int64_t)s * H + g * QPG + tid;
       ws_ml[((int64_t)z * wrows + orow) * 2] = -1e30f;
       ws_ml[((int64_t)z * wrows + orow) * 2 + 1] = 0.f;
@@ -1228,13 +1224,13 @@ __global__ void __launch_bounds__(256, R < 8 && R * NKC * VL < 512 && NKC * VL <
       vq[u] = *reinterpret_cast<const uint4*>(cache + row * roww + D + (8 * vl < DV ? 8 * vl : 0));
     }
   };
-  int j0 = jlo + KPT * wave;
+  int j0 = jlo + KPT * (4 * z + wave);
   if (j0 <= jhi) {
     ask(j0);
     find(j0);
     load_keys();
     load_values();
-    ask(j0 + 4 * KPT);
+    ask(j0 + step);
   }
   bf16x8_t qf[NKC];
   const bool mine = li < QPG;
@@ -1256,7 +1252,7 @@ __global__ void __launch_bounds__(256, R < 8 && R * NKC * VL < 512 && NKC * VL <
     for (int e = 0; e < 8; ++e) acc[r][e] = 0.f;
   const float qk_scale = a.softcap > 0.f ? a.scale / a.softcap : a.scale * LOG2E;
 
-  for (; j0 <= jhi; j0 += 4 * KPT) {
+  for (; j0 <= jhi; j0 += step) {
     f32x4_t d[KT];
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
@@ -1264,11 +1260,11 @@ __global__ void __launch_bounds__(256, R < 8 && R * NKC * VL < 512 && NKC * VL <
 #pragma unroll
       for (int c = 0; c < NKC; ++c) d[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kq[t][c], qf[c], d[t], 0, 0, 0);
     }
-    const bool more = j0 + 4 * KPT <= jhi;
+    const bool more = j0 + step <= jhi;
     if (more) {
-      find(j0 + 4 * KPT);
+      find(j0 + step);
       load_keys();
-      ask(j0 + 8 * KPT);
+      ask(j0 + 2 * step);
     }
     float top = -INFINITY;
 #pragma unroll
@@ -1523,7 +1519,7 @@ template <int R, int NKC, int VL, bool SIG> hipError_t launch_decode_one(const S
   auto* fn = sink_attn_decode_kernel<R, NKC, VL, KT, SIG>;
   const size_t lds = sizeof(float) * ((size_t)4 * (16 * KT + 1) * R + 8 * R + (size_t)4 * R * a.vdim);   // at most 37 KB
   const int nsplit = a.ws_o != nullptr ? max(1, a.nsplit) : 1;
-  hipLaunchKernelGGL(fn, dim3(nsplit, a.num_seqs, a.kv_heads), dim3(256), lds, s, a, a.ws_o, a.ws_ml, nsplit, a.chunk);
+  hipLaunchKernelGGL(fn, dim3(nsplit, a.num_seqs, a.kv_heads), dim3(256), lds, s, a, a.ws_o, a.ws_ml, nsplit);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || nsplit <= 1) return e;
   hipLaunchKernelGGL(sink_attn_merge_kernel, dim3((unsigned)((int64_t)a.heads * a.total_q)), dim3(128), 0, s, a);
