@@ -229,34 +229,55 @@ template <int KIND> hipError_t launch_act1(void* out, const void* z, bool f32, i
 
 constexpr int ROUTE_E_MAX = 256;
 
-// One workgroup per token: wave v computes the logits of experts v, v + 4, ...; thread 0 selects.
-__global__ void __launch_bounds__(NT) route_sigmoid_topk_kernel(float* w_out, int* id_out, const void* x,
-                                                               int64_t xstride, bool x_f32, const void* wr,
-                                                               bool wr_f32, int H, int E, int K) {
-  __shared__ float z[ROUTE_E_MAX];
-  const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  // 16-byte loads where both rows allow them (bf16 x and router: 8 elements per lane and trip, independent trips)
-  const bool vec = !x_f32 && !wr_f32 && H % 8 == 0 && xstride % 8 == 0 &&
-                   (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(wr) & 15) == 0;
-  for (int e = wave; e < E; e += NT / 64) {
+// Routers of decode steps: one workgroup of RNT threads per token, z [rows] its logits, a row of the router a wave at a time. A step has few
+// tokens, so this is bound by the latency of its loads, to rows that no L2 holds yet: 16 waves, each with 4096 columns in flight. us before (4 waves,
+// loads of one or four rows at a time as the compiler left them) and now: 40 tokens, 32 experts of width 4096 31 / 8.6, 32 tokens, 10 of 2048
+// 6.9 / 5.0, 1 token, 8 of 2048 4.7 / 4.4. A logit is the sum of a lane's columns in turn, then of the lanes.
+constexpr int RNT = 1024;
+__device__ __forceinline__ void router_logits(float* z, const void* x, int64_t x0, bool x_f32, const void* wr, bool wr_f32, int H, int rows,
+                                              bool vec) {
+  constexpr int U = 8;
+  const int lane = threadIdx.x & 63, n8 = H / 8;
+  for (int e = threadIdx.x >> 6; e < rows; e += RNT / 64) {
     float a = 0.f;
     if (vec) {
-      const uint4* xr = reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(x) + (int64_t)t * xstride);
+      const uint4* xr = reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(x) + x0);
       const uint4* wp = reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(wr) + (int64_t)e * H);
-      for (int c = lane; c < H / 8; c += 64) {
-        float xf[8], wf[8];
-        unpack8(xr[c], xf);
-        unpack8(wp[c], wf);
+      for (int c0 = lane; c0 < n8; c0 += 64 * U) {
+        uint4 xv[U], wv[U];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) a += xf[q] * wf[q];
+        for (int u = 0; u < U; ++u) {   // (columns past the last repeat it)
+          const int c = min(c0 + 64 * u, n8 - 1);
+          xv[u] = xr[c];
+          wv[u] = wp[c];
+        }
+        asm volatile("" ::: "memory");   // (all loads before the first condition)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (c0 + 64 * u >= n8) break;
+          float xf[8], wf[8];
+          unpack8(xv[u], xf);
+          unpack8(wv[u], wf);
+#pragma unroll
+          for (int q = 0; q < 8; ++q) a += xf[q] * wf[q];
+        }
       }
     } else {
-      for (int c = lane; c < H; c += 64)
-        a += ldv(x, (int64_t)t * xstride + c, x_f32) * ldv(wr, (int64_t)e * H + c, wr_f32);
+      for (int c = lane; c < H; c += 64) a += ldv(x, x0 + c, x_f32) * ldv(wr, (int64_t)e * H + c, wr_f32);
     }
     a = wave_sum(a);
     if (lane == 0) z[e] = a;
   }
+}
+
+// thread 0 selects
+__global__ void __launch_bounds__(RNT) route_sigmoid_topk_kernel(float* w_out, int* id_out, const void* x,
+                                                               int64_t xstride, bool x_f32, const void* wr,
+                                                               bool wr_f32, int H, int E, int K) {
+  __shared__ float z[ROUTE_E_MAX];
+  const int t = blockIdx.x;
+  const bool vec = !x_f32 && !wr_f32 && H % 8 == 0 && xstride % 8 == 0 && aligned16(x) && aligned16(wr);
+  router_logits(z, x, (int64_t)t * xstride, x_f32, wr, wr_f32, H, E, vec);
   __syncthreads();
   if (threadIdx.x != 0) return;
   for (int k = 0; k < K; ++k) {
@@ -391,9 +412,8 @@ __device__ __forceinline__ void softmax_select(const float* z, float* sc, const 
   for (int k = 0; k < K; ++k) w_out[k] *= rn;
 }
 
-// ---- softmax scores with group-limited choice: one wave selects, GE experts per lane
+// ---- softmax scores with group-limited choice: one wave selects, up to 8 experts per lane
 constexpr int GROUP_E_MAX = 512;
-constexpr int GE = GROUP_E_MAX / 64;
 
 // the larger of all lanes' keys (every lane receives it)
 __device__ __forceinline__ uint64_t wave_max_key(uint64_t k) {
@@ -404,22 +424,49 @@ __device__ __forceinline__ uint64_t wave_max_key(uint64_t k) {
   }
   return k;
 }
-// scores are >= 0, so their bits are ordered; the smaller index wins a tie; 0: no candidate
-__device__ __forceinline__ uint64_t score_key(float s, int i) {
-  return ((uint64_t)__float_as_uint(s) << 32) | (uint32_t)(0x7fffffff - i);
-}
 __device__ __forceinline__ int key_index(uint64_t k, int n) { return k == 0 ? 0 : min(0x7fffffff - (int)(uint32_t)k, n - 1); }
 
+// the largest of all lanes' numbers, on the VALU (DPP operands; each step leaves the maximum of a longer run in its last lane)
+template <int CTRL> __device__ __forceinline__ uint32_t max_before(uint32_t x) {
+  return max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, false));
+}
+__device__ __forceinline__ uint32_t wave_max_bits(uint32_t x) {
+  x = max_before<0x118>(max_before<0x114>(max_before<0x112>(max_before<0x111>(x))));
+  return max(max((uint32_t)__builtin_amdgcn_readlane((int)x, 15), (uint32_t)__builtin_amdgcn_readlane((int)x, 31)),
+             max((uint32_t)__builtin_amdgcn_readlane((int)x, 47), (uint32_t)__builtin_amdgcn_readlane((int)x, 63)));
+}
+// scores are >= 0, so their bits are ordered; + 1: 0 is no candidate
+__device__ __forceinline__ uint32_t score_bits(float s) { return min(__float_as_uint(s), 0xfffffffeu) + 1u; }
+// The largest of keys 64 i + lane, the smallest index on ties, is taken out of them: its index (0 without a candidate), its key in `best`.
+template <int PL> __device__ __forceinline__ int take_best(uint32_t (&key)[PL], int lane, uint32_t& best) {
+  uint32_t m = key[0];
+#pragma unroll
+  for (int i = 1; i < PL; ++i) m = max(m, key[i]);
+  best = wave_max_bits(m);
+  int at = 0;
+#pragma unroll
+  for (int i = PL - 1; i >= 0; --i) {
+    const uint64_t owners = __ballot(key[i] == best);
+    at = owners ? 64 * i + __builtin_ctzll(owners) : at;
+  }
+  at = best == 0 ? 0 : at;
+#pragma unroll
+  for (int i = 0; i < PL; ++i) key[i] = at == lane + 64 * i ? 0 : key[i];
+  return at;
+}
+
 // z [E] -> s = softmax(z); of `count` equal groups of neighbouring experts the `keep` with the largest single scores stay
-// open; the K largest open scores are chosen, w = scale * s. Called by one whole wave; sc [E] and gopen [count] are LDS
-// scratch of this wave.
+// open; the K largest open scores are chosen, w = scale * s. Called by one whole wave, with PL experts a lane; sc [E] and gopen [count]
+// are LDS scratch of this wave. Bound by instructions issued: maxima on the VALU (as exchanges of 64-bit keys through LDS, and with the
+// 8 places of 512 experts for any number of them, 8191 tokens of 16 experts took 17.5 us, now 6.9).
+template <int PL>
 __device__ __forceinline__ void grouped_select(const float* z, float* sc, int* gopen, int E, int K, int count, int keep,
                                                float scale, float* w_out, int* id_out) {
   const int lane = threadIdx.x & 63, per = E / count;
-  float v[GE];
+  float v[PL];
   float mx = -INFINITY;
 #pragma unroll
-  for (int i = 0; i < GE; ++i) {
+  for (int i = 0; i < PL; ++i) {
     const int e = lane + 64 * i;
     v[i] = e < E ? z[e] : -INFINITY;
     mx = fmaxf(mx, v[i]);
@@ -427,106 +474,85 @@ __device__ __forceinline__ void grouped_select(const float* z, float* sc, int* g
   mx = wave_max(mx);
   float den = 0.f;
 #pragma unroll
-  for (int i = 0; i < GE; ++i) {
+  for (int i = 0; i < PL; ++i) {
     v[i] = lane + 64 * i < E ? expf(v[i] - mx) : 0.f;
     den += v[i];
   }
   const float inv = 1.0f / wave_sum(den);
 #pragma unroll
-  for (int i = 0; i < GE; ++i) {
+  for (int i = 0; i < PL; ++i) {
     v[i] *= inv;
     if (lane + 64 * i < E) sc[lane + 64 * i] = v[i];
   }
   if (keep < count) {
     __threadfence_block();   // one wave: its LDS writes are in order, the fence keeps the compiler from moving the reads
-    uint64_t gk[GE];
+    uint32_t gk[PL];
 #pragma unroll
-    for (int i = 0; i < GE; ++i) {
+    for (int i = 0; i < PL; ++i) {
       const int g = lane + 64 * i;
       gk[i] = 0;
       if (g < count) {
         float best = 0.f;
         for (int e = 0; e < per; ++e) best = fmaxf(best, sc[g * per + e]);
-        gk[i] = score_key(best, g);
+        gk[i] = score_bits(best);
         gopen[g] = 0;
       }
     }
     for (int r = 0; r < keep; ++r) {
-      uint64_t k = 0;
-#pragma unroll
-      for (int i = 0; i < GE; ++i) k = gk[i] > k ? gk[i] : k;
-      k = wave_max_key(k);
-      if (k == 0) break;
-#pragma unroll
-      for (int i = 0; i < GE; ++i)
-        if (gk[i] == k) {   // (keys hold the index: one owner)
-          gk[i] = 0;
-          gopen[key_index(k, count)] = 1;
-        }
+      uint32_t best;
+      const int g = take_best<PL>(gk, lane, best);
+      if (best == 0) break;
+      if (lane == 0) gopen[g] = 1;
     }
     __threadfence_block();
   }
-  uint64_t ek[GE];
+  uint32_t ek[PL];
 #pragma unroll
-  for (int i = 0; i < GE; ++i) {
+  for (int i = 0; i < PL; ++i) {
     const int e = lane + 64 * i;
-    ek[i] = e < E && (keep >= count || gopen[e / per]) ? score_key(v[i], e) : 0;
+    ek[i] = e < E && (keep >= count || gopen[e / per]) ? score_bits(v[i]) : 0;
   }
+  float w[PL];
+  int id[PL];
   for (int r = 0; r < K; ++r) {
-    uint64_t k = 0;
+    uint32_t best;
+    const int e = take_best<PL>(ek, lane, best);
 #pragma unroll
-    for (int i = 0; i < GE; ++i) k = ek[i] > k ? ek[i] : k;
-    k = wave_max_key(k);
-#pragma unroll
-    for (int i = 0; i < GE; ++i)
-      if (ek[i] == k) ek[i] = 0;
-    if (lane == 0) {
-      w_out[r] = k == 0 ? 0.f : scale * __uint_as_float((uint32_t)(k >> 32));
-      id_out[r] = key_index(k, E);
-    }
+    for (int i = 0; i < PL; ++i)   // choice r stays with lane r % 64
+      if (r == lane + 64 * i) w[i] = best == 0 ? 0.f : scale * __uint_as_float(best - 1), id[i] = e;
   }
+#pragma unroll
+  for (int i = 0; i < PL; ++i)
+    if (lane + 64 * i < K) {
+      w_out[lane + 64 * i] = w[i];
+      id_out[lane + 64 * i] = id[i];
+    }
 }
 
-// One workgroup per token: wave v computes the logits of experts v, v + 4, ...; wave 0 selects.
-__global__ void __launch_bounds__(NT) route_grouped_topk_kernel(float* w_out, int* id_out, const void* x, int64_t xstride,
+// wave 0 selects
+template <int PL>
+__global__ void __launch_bounds__(RNT) route_grouped_topk_kernel(float* w_out, int* id_out, const void* x, int64_t xstride,
                                                                bool x_f32, const void* wr, bool wr_f32, int H, int E,
                                                                int K, int count, int keep, float scale) {
-  __shared__ float z[GROUP_E_MAX], sc[GROUP_E_MAX];
-  __shared__ int gopen[GROUP_E_MAX];
+  __shared__ float z[GROUP_E_MAX], sc[64 * PL];
+  __shared__ int gopen[64 * PL];
   const int64_t t = blockIdx.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const bool vec = !x_f32 && !wr_f32 && H % 8 == 0 && xstride % 8 == 0 && aligned16(x) && aligned16(wr);
-  for (int e = wave; e < E; e += NT / 64) {
-    float a = 0.f;
-    if (vec) {
-      const uint4* xr = reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(x) + t * xstride);
-      const uint4* wp = reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(wr) + (int64_t)e * H);
-      for (int c = lane; c < H / 8; c += 64) {
-        float xf[8], wf[8];
-        unpack8(xr[c], xf);
-        unpack8(wp[c], wf);
-#pragma unroll
-        for (int q = 0; q < 8; ++q) a += xf[q] * wf[q];
-      }
-    } else {
-      for (int c = lane; c < H; c += 64) a += ldv(x, t * xstride + c, x_f32) * ldv(wr, (int64_t)e * H + c, wr_f32);
-    }
-    a = wave_sum(a);
-    if (lane == 0) z[e] = a;
-  }
+  router_logits(z, x, t * xstride, x_f32, wr, wr_f32, H, E, vec);
   __syncthreads();
-  if (wave == 0) grouped_select(z, sc, gopen, E, K, count, keep, scale, w_out + t * K, id_out + t * K);
+  if (threadIdx.x < 64) grouped_select<PL>(z, sc, gopen, E, K, count, keep, scale, w_out + t * K, id_out + t * K);
 }
 
 // Selection alone, from fp32 logits z [T, E] computed elsewhere: one wave per token.
+template <int PL>
 __global__ void __launch_bounds__(NT) topk_grouped_kernel(float* w_out, int* id_out, const float* z, int T, int E, int K,
                                                          int count, int keep, float scale) {
-  __shared__ float sc[NT / 64][GROUP_E_MAX];
-  __shared__ int gopen[NT / 64][GROUP_E_MAX];
+  __shared__ float sc[NT / 64][64 * PL];
+  __shared__ int gopen[NT / 64][64 * PL];
   const int wave = threadIdx.x >> 6;
   const int64_t t = (int64_t)blockIdx.x * (NT / 64) + wave;
   if (t >= T) return;
-  grouped_select(z + t * E, sc[wave], gopen[wave], E, K, count, keep, scale, w_out + t * K, id_out + t * K);
+  grouped_select<PL>(z + t * E, sc[wave], gopen[wave], E, K, count, keep, scale, w_out + t * K, id_out + t * K);
 }
 
 // softmax_select by one whole wave, E <= ROUTE_E_MAX, the same results to the bit: exponentials, scores and comparisons a lane each,
@@ -584,51 +610,18 @@ __device__ __forceinline__ void softmax_select_wave(const float* z, float* sc, c
     }
 }
 
-// One workgroup per token: wave v computes the logits of rows v, v + 4, ... of the router (E choices, then an
-// optional gate row), four rows' loads in flight together; wave 0 selects. Bound by the latency of the loads and of the selection's
-// exchanges: 32 tokens, 10 choices of width 2048: 8.3 us (one row's loads at a time and one thread selecting: 9.9).
-__global__ void __launch_bounds__(NT) route_softmax_topk_kernel(float* w_out, int* id_out, float* gate_out,
+// the logits of E choices, then of an optional gate row; wave 0 selects
+__global__ void __launch_bounds__(RNT) route_softmax_topk_kernel(float* w_out, int* id_out, float* gate_out,
                                                                const void* x, int64_t xstride, bool x_f32,
                                                                const void* wr, bool wr_f32, const float* corr, int H,
                                                                int E, int K) {
   __shared__ float z[ROUTE_E_MAX + 1];
   __shared__ float sc[ROUTE_E_MAX];
-  const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int rows = E + (gate_out ? 1 : 0);
-  const bool vec = !x_f32 && !wr_f32 && H % 8 == 0 && xstride % 8 == 0 &&
-                   (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(wr) & 15) == 0;
-  constexpr int WV = NT / 64, B = 4;
-  for (int e0 = wave; e0 < rows; e0 += B * WV) {
-    float a[B] = {};
-    if (vec) {
-      const uint4* xr = reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(x) + (int64_t)t * xstride);
-      const uint4* wp[B];   // (rows beyond the last repeat it)
-#pragma unroll
-      for (int b = 0; b < B; ++b) wp[b] = reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(wr) + (int64_t)min(e0 + WV * b, rows - 1) * H);
-#pragma unroll 4
-      for (int c = lane; c < H / 8; c += 64) {
-        float xf[8], wf[8];
-        unpack8(xr[c], xf);
-#pragma unroll
-        for (int b = 0; b < B; ++b) {
-          unpack8(wp[b][c], wf);
-#pragma unroll
-          for (int q = 0; q < 8; ++q) a[b] += xf[q] * wf[q];
-        }
-      }
-    } else {
-      for (int b = 0; b < B; ++b)
-        for (int c = lane; c < H && e0 + WV * b < rows; c += 64)
-          a[b] += ldv(x, (int64_t)t * xstride + c, x_f32) * ldv(wr, (int64_t)(e0 + WV * b) * H + c, wr_f32);
-    }
-#pragma unroll
-    for (int b = 0; b < B; ++b) {
-      const float v = wave_sum(a[b]);
-      if (lane == 0 && e0 + WV * b < rows) z[e0 + WV * b] = v;
-    }
-  }
+  const int t = blockIdx.x;
+  const bool vec = !x_f32 && !wr_f32 && H % 8 == 0 && xstride % 8 == 0 && aligned16(x) && aligned16(wr);
+  router_logits(z, x, (int64_t)t * xstride, x_f32, wr, wr_f32, H, E + (gate_out ? 1 : 0), vec);
   __syncthreads();
-  if (wave == 0) softmax_select_wave(z, sc, corr, E, K, w_out + (int64_t)t * K, id_out + (int64_t)t * K);
+  if (threadIdx.x < 64) softmax_select_wave(z, sc, corr, E, K, w_out + (int64_t)t * K, id_out + (int64_t)t * K);
   if (gate_out && threadIdx.x == 64) gate_out[t] = 1.0f / (1.0f + expf(-z[E]));
 }
 
@@ -949,7 +942,7 @@ hipError_t launch_route_sigmoid_topk(float* w, int* ids, const void* x, int64_t 
                                      bool wr_f32, int T, int H, int E, int K, hipStream_t s) {
   if (T == 0) return hipSuccess;
   if (E < 1 || E > ROUTE_E_MAX || K < 1 || K > E) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(route_sigmoid_topk_kernel, dim3(T), dim3(NT), 0, s, w, ids, x, xstride, x_f32, wr, wr_f32, H, E,
+  hipLaunchKernelGGL(route_sigmoid_topk_kernel, dim3(T), dim3(RNT), 0, s, w, ids, x, xstride, x_f32, wr, wr_f32, H, E,
                      K);
   return hipGetLastError();
 }
@@ -966,7 +959,7 @@ hipError_t launch_route_softmax_topk(float* w, int* ids, float* gate, const void
                                      hipStream_t s) {
   if (T == 0) return hipSuccess;
   if (E < 1 || E > ROUTE_E_MAX || K < 1 || K > E) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(route_softmax_topk_kernel, dim3(T), dim3(NT), 0, s, w, ids, gate, x, xstride, x_f32, wr, wr_f32,
+  hipLaunchKernelGGL(route_softmax_topk_kernel, dim3(T), dim3(RNT), 0, s, w, ids, gate, x, xstride, x_f32, wr, wr_f32,
                      corr, H, E, K);
   return hipGetLastError();
 }
@@ -981,8 +974,10 @@ hipError_t launch_route_grouped_topk(float* w, int* ids, const void* x, int64_t 
                                      hipStream_t s) {
   if (T == 0) return hipSuccess;
   if (!groups_ok(E, K, count, keep)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(route_grouped_topk_kernel, dim3(T), dim3(NT), 0, s, w, ids, x, xstride, x_f32, wr, wr_f32, H, E, K,
-                     count, keep, scale);
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(T), dim3(RNT), 0, s, w, ids, x, xstride, x_f32, wr, wr_f32, H, E, K, count, keep, scale);
+  };
+  E <= 64 ? launch(route_grouped_topk_kernel<1>) : E <= 256 ? launch(route_grouped_topk_kernel<4>) : launch(route_grouped_topk_kernel<GROUP_E_MAX / 64>);
   return hipGetLastError();
 }
 
@@ -990,8 +985,10 @@ hipError_t launch_topk_grouped(float* w, int* ids, const float* z, int T, int E,
                                hipStream_t s) {
   if (T == 0) return hipSuccess;
   if (!groups_ok(E, K, count, keep)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(topk_grouped_kernel, dim3((T + NT / 64 - 1) / (NT / 64)), dim3(NT), 0, s, w, ids, z, T, E, K, count,
-                     keep, scale);
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((T + NT / 64 - 1) / (NT / 64)), dim3(NT), 0, s, w, ids, z, T, E, K, count, keep, scale);
+  };
+  E <= 64 ? launch(topk_grouped_kernel<1>) : E <= 256 ? launch(topk_grouped_kernel<4>) : launch(topk_grouped_kernel<GROUP_E_MAX / 64>);
   return hipGetLastError();
 }
 

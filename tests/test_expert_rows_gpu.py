@@ -1,0 +1,62 @@
+"""Rows of the experts: the pairs put in order of their experts, at the edges of the kernels (2048 pairs less 8 per expert, 4096, 12288 and
+32768 in one reading), and the group-limited choice, at the edges of the experts a lane holds (64, 256, 512) and with ties."""
+
+import pytest
+import torch
+
+from src import ops
+from src.ops import mix
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,E", [(0, 3), (1, 1), (63, 10), (511, 8), (512, 256), (513, 64), (1920, 16), (1921, 16), (3, 256), (4097, 31), (8191, 2), (8193, 65), (20001, 256), (12289, 12), (32768, 64), (40000, 5)])
+@pytest.mark.parametrize("kern", ["main", "mix"])
+@pytest.mark.parametrize("lean", [1, 6])
+def test_align(cuda, n, E, kern, lean):
+    """Whatever the experts' shares (lean 6: most pairs to the first ones). With many pairs those of an expert ascend."""
+    torch.manual_seed(n + E)
+    ids = (torch.rand(n, device=cuda) ** lean * E).int().clamp_(max=E - 1)
+    off, at, pos = (torch.full((s,), -7, dtype=torch.int32, device=cuda) for s in (E + 1, n, n))
+    (ops if kern == "main" else mix)._kern().moe_align(off, at, pos, ids, E)
+    want = torch.sort(ids.long(), stable=True).indices
+    assert torch.equal(pos.long()[at.long()], torch.arange(n, device=cuda)) and torch.equal(ids[at.long()], ids[want])
+    assert n + 8 * E <= 2048 or torch.equal(at.long(), want)
+    assert off.tolist() == [0, *torch.bincount(ids.long(), minlength=E).cumsum(0).tolist()]
+
+
+@pytest.mark.parametrize("E,k,groups,keep", [(1, 1, 1, 1), (10, 3, 5, 2), (63, 63, 1, 1), (64, 6, 4, 2), (64, 8, 64, 8), (65, 5, 13, 3), (256, 8, 8, 4),
+                                             (257, 70, 1, 1), (512, 300, 4, 3), (512, 9, 512, 9)])
+def test_grouped_choice(cuda, E, k, groups, keep):
+    """Logits in steps of 1/4 (equal ones have equal scores, others differ by more than rounding). A score's error is that of its
+    exponential (a few 2^-24) and of the sum, whose longest chain is E / 64 + 6 terms: less than 2^-19 of it."""
+    torch.manual_seed(E + k)
+    z = (torch.randn(300, E) * 8).round() / 4
+    best = z.view(300, groups, -1).amax(-1)
+    shut = torch.ones(300, groups, dtype=torch.bool).scatter_(1, torch.sort(best, descending=True, stable=True).indices[:, :keep], False)
+    ranked = z.masked_fill(shut.repeat_interleave(E // groups, 1), float("-inf"))   # (scores are in the order of their logits)
+    want_i = torch.sort(ranked, descending=True, stable=True).indices[:, :k]
+    want_w = 2.5 * torch.softmax(z.double(), 1).gather(1, want_i)
+    eye = torch.eye(E, device=cuda)
+    for a, b in ((0, 300), (0, 256), (256, 300)):    # selection alone, fused
+        w, i = mix.route_grouped_topk(z[a:b].to(cuda), eye, k, groups, keep, 2.5)
+        assert torch.equal(i.cpu().long(), want_i[a:b])
+        assert ((w.cpu().double() - want_w[a:b]).abs() <= 2.0 ** -19 * want_w[a:b]).all()
+
+
+@pytest.mark.parametrize("H", [8, 520, 2056, 4096])
+@pytest.mark.parametrize("E", [1, 3, 16, 17, 40])
+def test_logits_of_rows_beyond_a_turn(cuda, H, E):
+    """Four rows a wave at a time, four waves: the rows past the last are no one's."""
+    torch.manual_seed(H + E)
+    x, r = torch.randn(5, H, device=cuda).bfloat16(), torch.randn(E, H, device=cuda).bfloat16() / H ** 0.5
+    z = x.double() @ r.double().t()
+    w, i = mix.route_grouped_topk(x, r, E)
+    s = torch.softmax(z, 1).gather(1, i.long())
+    # a logit's fp32 sum: H / 64 + 6 additions in a row of 2^-24 of the terms' sum
+    e = (H / 64 + 8) * 2.0 ** -24 * float((x.double().abs() @ r.double().abs().t()).max()) + 2.0 ** -20
+    assert i.long().sort(1).values.equal(torch.arange(E, device=cuda).expand(5, E)) and ((w.double() - s).abs() <= 3 * e * s).all()
+    w, i = mix.route_sigmoid_topk(x, r, E)
+    assert i.long().sort(1).values.equal(torch.arange(E, device=cuda).expand(5, E))
+    s = torch.sigmoid(z).gather(1, i.long())
+    assert ((w.double() - s).abs() <= 3 * e * s).all()
