@@ -234,9 +234,9 @@ constexpr int ROUTE_E_MAX = 256;
 // loads of one or four rows at a time as the compiler left them) and now: 40 tokens, 32 experts of width 4096 31 / 8.6, 32 tokens, 10 of 2048
 // 6.9 / 5.0, 1 token, 8 of 2048 4.7 / 4.4. A logit is the sum of a lane's columns in turn, then of the lanes.
 constexpr int RNT = 1024;
+template <int U>
 __device__ __forceinline__ void router_logits(float* z, const void* x, int64_t x0, bool x_f32, const void* wr, bool wr_f32, int H, int rows,
                                               bool vec) {
-  constexpr int U = 8;
   const int lane = threadIdx.x & 63, n8 = H / 8;
   for (int e = threadIdx.x >> 6; e < rows; e += RNT / 64) {
     float a = 0.f;
@@ -270,32 +270,86 @@ __device__ __forceinline__ void router_logits(float* z, const void* x, int64_t x
   }
 }
 
-// thread 0 selects
+__device__ __forceinline__ void router_logits(float* z, const void* x, int64_t x0, bool x_f32, const void* wr, bool wr_f32, int H, int rows,
+                                              bool vec) {
+  if (H <= 1024)
+    router_logits<2>(z, x, x0, x_f32, wr, wr_f32, H, rows, vec);
+  else
+    router_logits<8>(z, x, x0, x_f32, wr, wr_f32, H, rows, vec);
+}
+
+// the largest of all lanes' numbers, on the VALU (DPP operands; each step leaves the maximum of a longer run in its last lane)
+template <int CTRL> __device__ __forceinline__ uint32_t max_before(uint32_t x) {
+  return max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, false));
+}
+__device__ __forceinline__ uint32_t wave_max_bits(uint32_t x) {
+  x = max_before<0x118>(max_before<0x114>(max_before<0x112>(max_before<0x111>(x))));
+  return max(max((uint32_t)__builtin_amdgcn_readlane((int)x, 15), (uint32_t)__builtin_amdgcn_readlane((int)x, 31)),
+             max((uint32_t)__builtin_amdgcn_readlane((int)x, 47), (uint32_t)__builtin_amdgcn_readlane((int)x, 63)));
+}
+// scores are >= 0, so their bits are ordered; + 1: 0 is no candidate
+__device__ __forceinline__ uint32_t score_bits(float s) { return min(__float_as_uint(s), 0xfffffffeu) + 1u; }
+// any number but NaN in an order that unsigned numbers keep, 0: no candidate
+__device__ __forceinline__ uint32_t order_bits(float v) {
+  const uint32_t u = __float_as_uint(v + 0.0f);   // (-0 is 0)
+  return v == v ? (u & 0x80000000u ? ~u : u | 0x80000000u) : 0;
+}
+// The largest of keys 64 i + lane, the smallest index on ties, is taken out of them: its index (0 without a candidate), its key in `best`.
+template <int PL> __device__ __forceinline__ int take_best(uint32_t (&key)[PL], int lane, uint32_t& best) {
+  uint32_t m = key[0];
+#pragma unroll
+  for (int i = 1; i < PL; ++i) m = max(m, key[i]);
+  best = wave_max_bits(m);
+  int at = 0;
+#pragma unroll
+  for (int i = PL - 1; i >= 0; --i) {
+    const uint64_t owners = __ballot(key[i] == best);
+    at = owners ? 64 * i + __builtin_ctzll(owners) : at;
+  }
+  at = best == 0 ? 0 : at;
+#pragma unroll
+  for (int i = 0; i < PL; ++i) key[i] = at == lane + 64 * i ? 0 : key[i];
+  return at;
+}
+
+// The K largest of a token's logits z [E], lowest index on ties, and their sigmoids, by a whole wave with PL experts a lane. NaN is no
+// candidate, -inf only if LOWEST; without one expert 0 is chosen with a logit of 0.
+template <int PL, bool LOWEST>
+__device__ __forceinline__ void sigmoid_select(const float* z, int E, int K, float* w_out, int* id_out) {
+  const int lane = threadIdx.x & 63;
+  uint32_t key[PL];
+#pragma unroll
+  for (int i = 0; i < PL; ++i) {
+    const int e = lane + 64 * i;
+    const float v = e < E ? z[e] : NAN;
+    key[i] = LOWEST || v != -INFINITY ? order_bits(v) : 0;
+  }
+  float w[PL];
+  int id[PL];
+  for (int k = 0; k < K; ++k) {
+    uint32_t best;
+    const int e = take_best<PL>(key, lane, best);
+#pragma unroll
+    for (int i = 0; i < PL; ++i)   // choice k stays with lane k % 64
+      if (k == lane + 64 * i) w[i] = best == 0 ? 0.f : z[e], id[i] = e;
+  }
+#pragma unroll
+  for (int i = 0; i < PL; ++i)
+    if (lane + 64 * i < K) {
+      w_out[lane + 64 * i] = 1.0f / (1.0f + expf(-w[i]));
+      id_out[lane + 64 * i] = id[i];
+    }
+}
+
 __global__ void __launch_bounds__(RNT) route_sigmoid_topk_kernel(float* w_out, int* id_out, const void* x,
                                                                int64_t xstride, bool x_f32, const void* wr,
                                                                bool wr_f32, int H, int E, int K) {
   __shared__ float z[ROUTE_E_MAX];
-  const int t = blockIdx.x;
+  const int64_t t = blockIdx.x;
   const bool vec = !x_f32 && !wr_f32 && H % 8 == 0 && xstride % 8 == 0 && aligned16(x) && aligned16(wr);
-  router_logits(z, x, (int64_t)t * xstride, x_f32, wr, wr_f32, H, E, vec);
+  router_logits(z, x, t * xstride, x_f32, wr, wr_f32, H, E, vec);
   __syncthreads();
-  if (threadIdx.x != 0) return;
-  for (int k = 0; k < K; ++k) {
-    int bi = -1;
-    float bv = 0.f;
-    for (int e = 0; e < E; ++e) {
-      const float v = z[e];
-      if (v != v || v == -INFINITY) continue;  // taken (marked below) or unusable
-      if (bi < 0 || v > bv) {
-        bv = v;
-        bi = e;
-      }
-    }
-    if (bi < 0) bi = 0;
-    w_out[(int64_t)t * K + k] = 1.0f / (1.0f + expf(-bv));
-    id_out[(int64_t)t * K + k] = bi;
-    z[bi] = -INFINITY;
-  }
+  if (threadIdx.x < 64) sigmoid_select<ROUTE_E_MAX / 64, false>(z, E, K, w_out + t * K, id_out + t * K);
 }
 
 // Selection alone, from logits already computed (a library fp32 GEMM for prompt-sized steps): one thread per token.
@@ -415,46 +469,6 @@ __device__ __forceinline__ void softmax_select(const float* z, float* sc, const 
 // ---- softmax scores with group-limited choice: one wave selects, up to 8 experts per lane
 constexpr int GROUP_E_MAX = 512;
 
-// the larger of all lanes' keys (every lane receives it)
-__device__ __forceinline__ uint64_t wave_max_key(uint64_t k) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const uint64_t other = ((uint64_t)(uint32_t)__shfl_xor((int)(k >> 32), o, 64) << 32) | (uint32_t)__shfl_xor((int)(uint32_t)k, o, 64);
-    k = other > k ? other : k;
-  }
-  return k;
-}
-__device__ __forceinline__ int key_index(uint64_t k, int n) { return k == 0 ? 0 : min(0x7fffffff - (int)(uint32_t)k, n - 1); }
-
-// the largest of all lanes' numbers, on the VALU (DPP operands; each step leaves the maximum of a longer run in its last lane)
-template <int CTRL> __device__ __forceinline__ uint32_t max_before(uint32_t x) {
-  return max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xf, 0xf, false));
-}
-__device__ __forceinline__ uint32_t wave_max_bits(uint32_t x) {
-  x = max_before<0x118>(max_before<0x114>(max_before<0x112>(max_before<0x111>(x))));
-  return max(max((uint32_t)__builtin_amdgcn_readlane((int)x, 15), (uint32_t)__builtin_amdgcn_readlane((int)x, 31)),
-             max((uint32_t)__builtin_amdgcn_readlane((int)x, 47), (uint32_t)__builtin_amdgcn_readlane((int)x, 63)));
-}
-// scores are >= 0, so their bits are ordered; + 1: 0 is no candidate
-__device__ __forceinline__ uint32_t score_bits(float s) { return min(__float_as_uint(s), 0xfffffffeu) + 1u; }
-// The largest of keys 64 i + lane, the smallest index on ties, is taken out of them: its index (0 without a candidate), its key in `best`.
-template <int PL> __device__ __forceinline__ int take_best(uint32_t (&key)[PL], int lane, uint32_t& best) {
-  uint32_t m = key[0];
-#pragma unroll
-  for (int i = 1; i < PL; ++i) m = max(m, key[i]);
-  best = wave_max_bits(m);
-  int at = 0;
-#pragma unroll
-  for (int i = PL - 1; i >= 0; --i) {
-    const uint64_t owners = __ballot(key[i] == best);
-    at = owners ? 64 * i + __builtin_ctzll(owners) : at;
-  }
-  at = best == 0 ? 0 : at;
-#pragma unroll
-  for (int i = 0; i < PL; ++i) key[i] = at == lane + 64 * i ? 0 : key[i];
-  return at;
-}
-
 // z [E] -> s = softmax(z); of `count` equal groups of neighbouring experts the `keep` with the largest single scores stay
 // open; the K largest open scores are chosen, w = scale * s. Called by one whole wave, with PL experts a lane; sc [E] and gopen [count]
 // are LDS scratch of this wave. Bound by instructions issued: maxima on the VALU (as exchanges of 64-bit keys through LDS, and with the
@@ -555,11 +569,11 @@ __global__ void __launch_bounds__(NT) topk_grouped_kernel(float* w_out, int* id_
   grouped_select<PL>(z + t * E, sc[wave], gopen[wave], E, K, count, keep, scale, w_out + t * K, id_out + t * K);
 }
 
-// softmax_select by one whole wave, E <= ROUTE_E_MAX, the same results to the bit: exponentials, scores and comparisons a lane each,
+// softmax_select by one whole wave with PL experts a lane, the same results to the bit: exponentials, scores and comparisons a lane each,
 // sums in the same order. sc [E] is LDS scratch.
+template <int PL>
 __device__ __forceinline__ void softmax_select_wave(const float* z, float* sc, const float* corr, int E, int K, float* w_out,
                                                     int* id_out) {
-  constexpr int PL = ROUTE_E_MAX / 64;
   const int lane = threadIdx.x & 63;
   float mx = -INFINITY;
   for (int e = lane; e < E; e += 64) mx = fmaxf(mx, z[e]);
@@ -570,15 +584,14 @@ __device__ __forceinline__ void softmax_select_wave(const float* z, float* sc, c
   float den = 0.f;
   for (int e = 0; e < E; ++e) den += sc[e];
   const float inv = 1.0f / den;
-  uint64_t key[PL];   // score + corr in an order that unsigned numbers keep, then the smaller index; 0: no candidate
+  uint32_t key[PL];
 #pragma unroll
   for (int i = 0; i < PL; ++i) {
     const int e = lane + 64 * i;
     key[i] = 0;
     if (e < E) {
-      const float p = sc[e] * inv, v = p + (corr ? corr[e] : 0.f);
-      const uint32_t u = __float_as_uint(v + 0.0f);   // (-0 is 0)
-      if (v == v) key[i] = (uint64_t)(u & 0x80000000u ? ~u : u | 0x80000000u) << 32 | (uint32_t)(0x7fffffff - e);
+      const float p = sc[e] * inv;
+      key[i] = order_bits(p + (corr ? corr[e] : 0.f));
       sc[e] = p;
     }
   }
@@ -587,19 +600,13 @@ __device__ __forceinline__ void softmax_select_wave(const float* z, float* sc, c
   float sum = 0.f, w[PL];
   int id[PL];
   for (int k = 0; k < K; ++k) {
-    uint64_t best = 0;
-#pragma unroll
-    for (int i = 0; i < PL; ++i) best = key[i] > best ? key[i] : best;
-    best = wave_max_key(best);
-#pragma unroll
-    for (int i = 0; i < PL; ++i)
-      if (key[i] == best) key[i] = 0;
-    const int bi = key_index(best, E);
-    const float p = sc[bi];
+    uint32_t best;
+    const int e = take_best<PL>(key, lane, best);
+    const float p = sc[e];
     sum += p;
 #pragma unroll
     for (int i = 0; i < PL; ++i)   // choice k stays with lane k % 64
-      if (k == lane + 64 * i) w[i] = p, id[i] = bi;
+      if (k == lane + 64 * i) w[i] = p, id[i] = e;
   }
   const float rn = 1.0f / (sum + 1e-20f);
 #pragma unroll
@@ -621,8 +628,113 @@ __global__ void __launch_bounds__(RNT) route_softmax_topk_kernel(float* w_out, i
   const bool vec = !x_f32 && !wr_f32 && H % 8 == 0 && xstride % 8 == 0 && aligned16(x) && aligned16(wr);
   router_logits(z, x, (int64_t)t * xstride, x_f32, wr, wr_f32, H, E + (gate_out ? 1 : 0), vec);
   __syncthreads();
-  if (threadIdx.x < 64) softmax_select_wave(z, sc, corr, E, K, w_out + (int64_t)t * K, id_out + (int64_t)t * K);
+  if (threadIdx.x < 64) softmax_select_wave<ROUTE_E_MAX / 64>(z, sc, corr, E, K, w_out + (int64_t)t * K, id_out + (int64_t)t * K);
   if (gate_out && threadIdx.x == 64) gate_out[t] = 1.0f / (1.0f + expf(-z[E]));
+}
+
+// ---- routers of prompt-sized steps, bf16 tokens and router of up to 64 rows (a gate's included), width a multiple of 64
+enum { ROUTE_SIGMOID, ROUTE_SOFTMAX, ROUTE_GROUPED };
+struct RouteRows {
+  float* w;
+  int* ids;
+  float* gate;
+  const bf16_t *x, *wr;
+  int64_t xstride;
+  const float* corr;
+  int T, H, E, K, count, keep;
+  float scale;
+};
+// A workgroup's 16 MT tokens by 16 NT rows of the router on the matrix cores. Its 8 waves share the width in blocks of 64 columns (a cache line
+// of every row), the waves' parts are added in fp32 and a wave selects for every eighth token. Bound by the latency of the loads, U blocks of
+// a wave in flight, and on from 8000 tokens by their bytes. Loaded as the product takes them (neighbouring lanes of different rows, 16 bytes each)
+// operands came at 17 bytes a cycle; so they turn in LDS (600 tokens of width 2048, 16 choices 6.6 -> 4.9 us, 1200 of 4096, 32 choices 13.7 -> 8.0).
+// us as a library product and a selection of its own (for sigmoid and softmax scores an fp32 product, behind a pass that widens the tokens) and so:
+//   sigmoid, 8 choices, 600 tokens of 2048 18.5 -> 4.9, 8191 38 -> 6.8, 8192 of 4096 60 -> 14; softmax 19 -> 5.8, 39 -> 8.0, 60 -> 15;
+//   groups of 16 experts 9.2 -> 5.7, 16.8 -> 8.3, 21 -> 15. Errors against 64 bits (sigmoid, 8191 tokens): 1.4e-6 at most, now 7.2e-7.
+template <int KIND, int NT, int MT>
+__global__ void __launch_bounds__(512) route_rows_kernel(const RouteRows a) {
+  constexpr int WV = 8, F = MT + NT, U = F <= 3 ? 4 : 2, TOK = 16 * MT, P = 16 * NT + 1;
+  __shared__ union {
+    u32x4_t turn[WV][F][2][64];
+    float part[WV][TOK][P];
+  } lds;
+  __shared__ float z[TOK][P];
+  __shared__ float sc[WV][64];
+  __shared__ int gopen[WV][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+  const int64_t t0 = (int64_t)blockIdx.x * TOK;
+  const int nb = a.H / 64, rows = a.E + (a.gate ? 1 : 0);
+  // Eight lanes load the 128 bytes of a row's block, eight rows at a time; a lane of the product holds another row each. In between 16-byte
+  // pieces of a row change places by its number's half, so that no eight rows read the same banks.
+  const bf16_t* from[F][2];   // (tokens and rows past the last repeat it)
+#pragma unroll
+  for (int f = 0; f < F; ++f)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int row = 16 * (f < MT ? f : f - MT) + 8 * h + (lane >> 3), piece = (lane & 7) ^ ((lane >> 4) & 3);
+      from[f][h] = (f < MT ? a.x + min(t0 + row, (int64_t)a.T - 1) * a.xstride : a.wr + (int64_t)min(row, rows - 1) * a.H) + 8 * piece;
+    }
+  const int at = (r & 7) * 8, swap = (r >> 1) & 3;
+  f32x4_t acc[MT][NT] = {};
+  for (int b0 = wave; b0 < nb; b0 += WV * U) {
+    u32x4_t v[U][F][2];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {   // (blocks past the last repeat it)
+      const int c = 64 * min(b0 + WV * u, nb - 1);
+#pragma unroll
+      for (int f = 0; f < F; ++f)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) v[u][f][h] = *reinterpret_cast<const u32x4_t*>(from[f][h] + c);
+    }
+    asm volatile("" ::: "memory");   // (all loads before the first condition)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (b0 + WV * u >= nb) break;
+#pragma unroll
+      for (int f = 0; f < F; ++f)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) lds.turn[wave][f][h][lane] = v[u][f][h];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // (LDS keeps a wave's order)
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        bf16x8_t op[F];
+#pragma unroll
+        for (int f = 0; f < F; ++f) op[f] = __builtin_bit_cast(bf16x8_t, lds.turn[wave][f][r >> 3][at + ((4 * k + g) ^ swap)]);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int n = 0; n < NT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(op[m], op[MT + n], acc[m][n], 0, 0, 0);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) lds.part[wave][16 * m + 4 * g + i][16 * n + r] = acc[m][n][i];
+  __syncthreads();
+  for (int i = threadIdx.x; i < TOK * 16 * NT; i += 64 * WV) {
+    const int t = i / (16 * NT), e = i % (16 * NT);
+    float v = 0.f;
+#pragma unroll
+    for (int k = 0; k < WV; ++k) v += lds.part[k][t][e];
+    z[t][e] = v;
+  }
+  __syncthreads();
+  for (int i = wave; i < TOK && t0 + i < a.T; i += WV) {
+    const int64_t t = t0 + i;
+    float* w = a.w + t * a.K;
+    int* ids = a.ids + t * a.K;
+    if constexpr (KIND == ROUTE_SIGMOID) sigmoid_select<1, true>(z[i], a.E, a.K, w, ids);
+    if constexpr (KIND == ROUTE_SOFTMAX) softmax_select_wave<1>(z[i], sc[wave], a.corr, a.E, a.K, w, ids);
+    if constexpr (KIND == ROUTE_GROUPED) grouped_select<1>(z[i], sc[wave], gopen[wave], a.E, a.K, a.count, a.keep, a.scale, w, ids);
+    if (KIND == ROUTE_SOFTMAX && a.gate && lane == 0) a.gate[t] = 1.0f / (1.0f + expf(-z[i][a.E]));
+  }
 }
 
 // Selection alone, from logits already computed (a library fp32 GEMM for prompt-sized steps): one thread per token,
@@ -938,10 +1050,30 @@ hipError_t launch_relu2_act(void* out, const void* z, bool f32, int64_t n, hipSt
   return launch_act1<ACT1_RELU2>(out, z, f32, n, s);
 }
 
+// Decode-sized steps (up to 256 tokens) go token by token where a wave has one row of the router, else in rows: us by token / in rows, 16 choices,
+// 64 tokens of width 4096 5.5 / 6.0, 16 of 2048 5.4 / 5.6, 1 of 8192 7.1 / 8.3 (1 of 2048 4.7 / 3.8); 32 choices 7.8 / 7.7, 7.1 / 5.4, 10.9 / 10.3.
+static bool route_in_rows(const void* x, int64_t xstride, bool x_f32, const void* wr, bool wr_f32, int T, int H, int rows) {
+  return (T > 256 || rows > RNT / 64) && !x_f32 && !wr_f32 && rows <= 64 && H % 64 == 0 && xstride % 8 == 0 &&
+         ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(wr)) & 15) == 0;
+}
+// 32 tokens share what is read of a router of more than 32 rows once 16 of them fill the CUs (4100 tokens of width 2048 13.3 -> 11.0 us, 2500 7.8
+// -> 10.4); with fewer rows they cost more than that gives (8192 tokens of 4096, 16 rows: 13.7 -> 18.0).
+template <int KIND> static hipError_t launch_route_rows(const RouteRows& a, hipStream_t s) {
+  const int rows = a.E + (a.gate ? 1 : 0);
+  const auto launch = [&](auto kernel, int tokens) { hipLaunchKernelGGL(kernel, dim3((a.T + tokens - 1) / tokens), dim3(512), 0, s, a); };
+  rows <= 16   ? launch(route_rows_kernel<KIND, 1, 1>, 16)
+  : rows <= 32 ? launch(route_rows_kernel<KIND, 2, 1>, 16)
+  : a.T <= 4096 ? launch(route_rows_kernel<KIND, 4, 1>, 16)
+                : launch(route_rows_kernel<KIND, 4, 2>, 32);
+  return hipGetLastError();
+}
+
 hipError_t launch_route_sigmoid_topk(float* w, int* ids, const void* x, int64_t xstride, bool x_f32, const void* wr,
                                      bool wr_f32, int T, int H, int E, int K, hipStream_t s) {
   if (T == 0) return hipSuccess;
   if (E < 1 || E > ROUTE_E_MAX || K < 1 || K > E) return hipErrorInvalidValue;
+  if (route_in_rows(x, xstride, x_f32, wr, wr_f32, T, H, E))
+    return launch_route_rows<ROUTE_SIGMOID>({w, ids, nullptr, static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(wr), xstride, nullptr, T, H, E, K, 1, 1, 1.f}, s);
   hipLaunchKernelGGL(route_sigmoid_topk_kernel, dim3(T), dim3(RNT), 0, s, w, ids, x, xstride, x_f32, wr, wr_f32, H, E,
                      K);
   return hipGetLastError();
@@ -959,6 +1091,8 @@ hipError_t launch_route_softmax_topk(float* w, int* ids, float* gate, const void
                                      hipStream_t s) {
   if (T == 0) return hipSuccess;
   if (E < 1 || E > ROUTE_E_MAX || K < 1 || K > E) return hipErrorInvalidValue;
+  if (route_in_rows(x, xstride, x_f32, wr, wr_f32, T, H, E + (gate ? 1 : 0)))
+    return launch_route_rows<ROUTE_SOFTMAX>({w, ids, gate, static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(wr), xstride, corr, T, H, E, K, 1, 1, 1.f}, s);
   hipLaunchKernelGGL(route_softmax_topk_kernel, dim3(T), dim3(RNT), 0, s, w, ids, gate, x, xstride, x_f32, wr, wr_f32,
                      corr, H, E, K);
   return hipGetLastError();
@@ -974,6 +1108,8 @@ hipError_t launch_route_grouped_topk(float* w, int* ids, const void* x, int64_t 
                                      hipStream_t s) {
   if (T == 0) return hipSuccess;
   if (!groups_ok(E, K, count, keep)) return hipErrorInvalidValue;
+  if (route_in_rows(x, xstride, x_f32, wr, wr_f32, T, H, E))
+    return launch_route_rows<ROUTE_GROUPED>({w, ids, nullptr, static_cast<const bf16_t*>(x), static_cast<const bf16_t*>(wr), xstride, nullptr, T, H, E, K, count, keep, scale}, s);
   const auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, dim3(T), dim3(RNT), 0, s, w, ids, x, xstride, x_f32, wr, wr_f32, H, E, K, count, keep, scale);
   };

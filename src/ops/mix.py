@@ -140,6 +140,15 @@ def embed_norm(ids: torch.Tensor, embed: torch.Tensor, w: Optional[torch.Tensor]
 ROUTE_FUSED_MAX_T = 256  # up to here one fused launch computes the logits and selects (decode-sized steps)
 
 
+def _route_fused(x: torch.Tensor, router: torch.Tensor, rows: int) -> bool:
+    """Logits and choice in one launch: decode-sized steps, and prompts with bf16 factors, up to 64 ``rows`` of the router and a width that
+    the matrix-core kernel takes (figures beside it). Other prompts take a library product and a selection kernel."""
+    if x.shape[0] <= ROUTE_FUSED_MAX_T:
+        return True
+    return (x.dtype == router.dtype == torch.bfloat16 and rows <= 64 and x.shape[1] % 64 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and router.is_contiguous() and (x.data_ptr() | router.data_ptr()) % 16 == 0)
+
+
 def route_sigmoid_topk(x: torch.Tensor, router: torch.Tensor, k: int) -> Tuple[torch.Tensor, torch.Tensor]:
     """(w [T, k] fp32, ids [T, k] int32): the k experts with the largest sigmoid(x . router[e]) (fp32 logits) and
     those scores, not renormalised."""
@@ -148,8 +157,8 @@ def route_sigmoid_topk(x: torch.Tensor, router: torch.Tensor, k: int) -> Tuple[t
     t = x.shape[0]
     w = torch.empty(t, k, dtype=torch.float32, device=x.device)
     ids = torch.empty(t, k, dtype=torch.int32, device=x.device)
-    if t > ROUTE_FUSED_MAX_T:
-        # prompt-sized steps: the logits as one true-fp32 library GEMM, then the selection kernel
+    if not _route_fused(x, router, router.shape[0]):
+        # the logits as one true-fp32 library GEMM, then the selection kernel
         _kern().topk_sigmoid(w, ids, F.linear(x.float(), router.float()))
     else:
         _kern().route_sigmoid_topk(w, ids, x, router.contiguous())
@@ -387,8 +396,8 @@ def route_softmax_topk(x: torch.Tensor, router: torch.Tensor, k: int, n_route: i
     w = torch.empty(t, k, dtype=torch.float32, device=x.device)
     ids = torch.empty(t, k, dtype=torch.int32, device=x.device)
     gate = torch.empty(t, dtype=torch.float32, device=x.device) if gate_row else None
-    if t > ROUTE_FUSED_MAX_T:
-        # prompt-sized steps: the logits as one true-fp32 library GEMM, then the selection kernel
+    if not _route_fused(x, router, rows):
+        # the logits as one true-fp32 library GEMM, then the selection kernel
         _kern().topk_softmax_corrected(w, ids, gate, F.linear(x.float(), router[:rows].float()), n_route, correction)
     else:
         _kern().route_softmax_topk(w, ids, gate, x, router.contiguous(), n_route, correction)
@@ -406,8 +415,10 @@ def route_grouped_topk(x: torch.Tensor, router: torch.Tensor, k: int, groups: in
     t = x.shape[0]
     w = torch.empty(t, k, dtype=torch.float32, device=x.device)
     ids = torch.empty(t, k, dtype=torch.int32, device=x.device)
-    if t > ROUTE_FUSED_MAX_T:
-        # prompt-sized steps: the logits as one library GEMM with fp32 results (bf16 factors multiply exactly), then the
+    e = router.shape[0]
+    # (many tokens and choices are a bf16 product's own kind of work: 16384 x 2048 by 64 27 us, in rows 29; 8192 by 64 18.5 / 14.5)
+    if not _route_fused(x, router, e) or (t > 8192 and e > 32):
+        # the logits as one library GEMM with fp32 results (bf16 factors multiply exactly), then the
         # selection kernel
         z = F.linear(x, router) if x.dtype == torch.float32 else torch.mm(x, router.t(), out_dtype=torch.float32)
         _kern().topk_grouped(w, ids, z, groups, keep, float(scale))

@@ -60,3 +60,57 @@ def test_logits_of_rows_beyond_a_turn(cuda, H, E):
     assert i.long().sort(1).values.equal(torch.arange(E, device=cuda).expand(5, E))
     s = torch.sigmoid(z).gather(1, i.long())
     assert ((w.double() - s).abs() <= 3 * e * s).all()
+
+
+@pytest.mark.parametrize("T,H", [(1, 64), (40, 576), (257, 64), (300, 576), (271, 2048), (513, 4160), (4097, 64), (4130, 128)])
+@pytest.mark.parametrize("E,k,groups,keep", [(1, 1, 1, 1), (16, 3, 4, 2), (17, 17, 1, 1), (31, 2, 1, 1), (32, 4, 8, 4), (33, 6, 11, 2), (63, 5, 7, 3), (64, 8, 8, 2)])
+def test_prompts_in_rows(cuda, T, H, E, k, groups, keep):
+    """Tokens and a router of small whole numbers: logits exact in fp32 in any order of their sum, and full of ties. A score's error is that of
+    its exponential (a few 2^-24) and of a sum of at most 64 terms one after the other: less than 2^-17 of it."""
+    torch.manual_seed(T + H + E)
+    wide = torch.randint(-2, 3, (T, H + 8), device=cuda).bfloat16()
+    x, r = wide[:, :H], torch.randint(-2, 3, (E + 1, H), device=cuda).bfloat16()
+    z = (x.double() @ r.double().t() / 64).cpu()     # (a 64th: scores stay apart from 0 and 1)
+    x = x * 0.125
+    x = torch.cat([x, x[:, :8]], 1)[:, :H]           # rows that are no neighbours
+    r = r * 0.125
+
+    def check(w, i, score, ranked):
+        want = torch.sort(ranked, descending=True, stable=True).indices[:, :k]
+        assert torch.equal(i.cpu().long(), want)
+        s = score.gather(1, want)
+        assert ((w.cpu().double() - s).abs() <= 2.0 ** -17 * s).all()
+
+    z, zg = z[:, :E], z[:, E]
+    w, i = mix.route_sigmoid_topk(x, r[:E], k)
+    check(w, i, torch.sigmoid(z), z)
+    best = z.view(T, groups, -1).amax(-1)
+    shut = torch.ones(T, groups, dtype=torch.bool).scatter_(1, torch.sort(best, descending=True, stable=True).indices[:, :keep], False)
+    w, i = mix.route_grouped_topk(x, r[:E], k, groups, keep, 2.5)
+    check(w, i, 2.5 * torch.softmax(z, 1), z.masked_fill(shut.repeat_interleave(E // groups, 1), float("-inf")))
+    for gated in (False, True):
+        w, i, g = mix.route_softmax_topk(x, r, k, E, None, gated)
+        s = torch.softmax(z, 1)
+        top = torch.sort(z, descending=True, stable=True).indices[:, :k]
+        check(w, i, s / s.gather(1, top).sum(1, keepdim=True), z)
+        assert g is None if not gated else torch.allclose(g.cpu().double(), torch.sigmoid(zg), rtol=2.0 ** -17, atol=0)
+
+
+@pytest.mark.parametrize("name", ["route_sigmoid_topk", "route_softmax_topk", "route_grouped_topk"])
+def test_rows_that_go_to_the_library(cuda, name):
+    """Tokens at no multiple of 16 bytes, a router that is not contiguous, fp32 factors, 65 choices, a width of no whole blocks: the same answers."""
+    torch.manual_seed(7)
+    T, H, E = 300, 192, 20
+    x, r = torch.randint(-2, 3, (T, H), device=cuda).bfloat16() / 8, torch.randint(-2, 3, (65, H), device=cuda).bfloat16() / 8
+
+    def go(x, r):
+        return (mix.route_softmax_topk(x, r, 3, r.shape[0]) if "softmax" in name else getattr(mix, name)(x, r, 3))[:2]
+
+    odd = torch.empty(T * H + 1, device=cuda, dtype=torch.bfloat16)[1:].view(T, H).copy_(x)
+    w, i = go(x, r[:E])
+    for a, b in ((odd, r[:E]), (x, r[:E].t().contiguous().t()), (x.float(), r[:E].float())):
+        v, j = go(a, b)
+        assert torch.equal(i, j) and torch.allclose(w, v, rtol=2.0 ** -17, atol=0)
+    for a, b in ((x, r), (x[:, :100].contiguous(), r[:E, :100].contiguous())):
+        (v, j), (u, k) = go(a, b), go(a.float(), b.float())
+        assert torch.equal(j, k) and torch.allclose(u, v, rtol=2.0 ** -17, atol=0)
