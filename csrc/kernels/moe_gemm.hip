@@ -74,7 +74,15 @@ __device__ __forceinline__ int scan64(int x, int lane) {
 
 struct Tile {
   int e, n0, r0, M;   // expert, first output column, first of M rows
+  int turn;           // the stage of K that it starts with
 };
+// Weight rows are K apart, mostly a power of two: tiles that go through K in step ask the same few memory channels for their pieces. So
+// each starts at a K of its own, spread by the golden ratio, and goes round. Experts of one tile of rows, us in step / so, at 64 rows each: 32 of
+// 4096 x 2048 132 / 107 and 135 / 109, 8 gated ones of 4096 x 4096 135 / 109, of 2048 x 2048 43 / 39. Experts of more tiles stay in step, as these
+// share the weights through L2 (4096 x 4096, 1000 rows each: in step 523, from places of their own 548), and so do launches that leave more than
+// half of the CUs idle (16 of 2048 x 1024, 256 rows: 33.0 / 34.6).
+__device__ __forceinline__ int first_stage(int n, int nst) { return (int)((uint64_t)((uint32_t)n * 2654435769u) * (uint32_t)nst >> 32); }
+__device__ __forceinline__ int stage_of(int s, int turn, int nst) { return s + turn >= nst ? s + turn - nst : s + turn; }
 // The tiles of the launch, found from the offsets by every wave (lane i looks at experts i, i + 64, ...). Tiles of an expert are as even
 // as 32-row pieces allow, at most R rows. XCD i (blocks i, i + 8, ...) takes the i-th eighth of the list, whose neighbours share
 // weights or x rows; its CUs take turns. What is left for less than a turn of all of them is cut into `parts` by rows.
@@ -150,6 +158,7 @@ struct Plan {
       tile -= g * gs * NT;
       const int h = (rows / 32 + cut - 1) / cut * 32, m0 = (g * gs + tile % gm) * rows + part * h;
       t.n0 = tile / gm;
+      t.turn = mts == 1 ? first_stage(t.e * NT + t.n0, a.K / BK) : 0;   // (used where the launch asks for it)
       t.M = min(min(t.M - m0, rows - part * h), h);
       t.r0 += m0;
       if (t.M > 0) return true;
@@ -157,7 +166,35 @@ struct Plan {
   }
 };
 
-template <int ACT>
+// A lane's results of 32 TN weight rows: z(n, i) is register i of the n-th 32-row tile (weight rows 8 g + 4 hi + 0 .. 3 of it for i = 4 g ..).
+// Lanes 32 apart exchange halves of neighbouring g, so that each stores 8 columns at `op`, its own 8 hi columns on.
+template <int ACT, class Z> __device__ __forceinline__ void store_row(Z z, uint16_t* op, bool in, const MoeGemmArgs& a) {
+  constexpr bool GATED = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU;
+#pragma unroll
+  for (int n = 0; n < (GATED ? TN / 2 : TN); ++n)
+#pragma unroll
+    for (int g = 0; g < 4; g += 2) {
+      uint32_t p[2][2];
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        float y[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (GATED)
+            y[i] = moe_gate<ACT>(z(n, 4 * (g + q) + i), z(TN / 2 + n, 4 * (g + q) + i), a.limit, a.alpha);
+          else
+            y[i] = z(n, 4 * (g + q) + i);
+          if constexpr (ACT == MOE_ACT_RELU2) y[i] = fmaxf(y[i], 0.f) * fmaxf(y[i], 0.f);
+        }
+        p[q][0] = pack2(y[0], y[1]), p[q][1] = pack2(y[2], y[3]);
+      }
+      const auto u = __builtin_amdgcn_permlane32_swap(p[0][0], p[1][0], false, false);
+      const auto v = __builtin_amdgcn_permlane32_swap(p[0][1], p[1][1], false, false);
+      if (in) *reinterpret_cast<uint4*>(op + 32 * n + 8 * g) = make_uint4(u[0], v[0], u[1], v[1]);
+    }
+}
+
+template <int ACT, bool TURN>
 __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   constexpr bool GATED = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU;
@@ -184,7 +221,9 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
       for (int p = 0; p < PC; ++p) xr[p] = a.sorted[xr[p]];
     }
   };
+  int turn = 0;
   auto offsets_of = [&](const Tile& u) {
+    turn = TURN ? u.turn : 0;
     wbase = reinterpret_cast<const char*>(a.w) + (int64_t)u.e * (GATED ? 2 : 1) * a.ncols * a.K * 2;
 #pragma unroll
     for (int p = 0; p < PC; ++p) {
@@ -197,12 +236,14 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
     }
   };
   auto issue_w = [&](int s, int slot) {
+    if constexpr (TURN) s = stage_of(s, turn, nst);
 #pragma unroll
     for (int p = 0; p < PC; ++p)
       __builtin_amdgcn_global_load_lds((global_cvoid*)(wbase + (int64_t)s * ROWB + woff[p]),
                                        (lds_void*)(smem + slot * UNIT + (wave + NW * p) * 1024), 16, 0, 0);
   };
   auto issue_x = [&](int s, int slot, int pieces) {
+    if constexpr (TURN) s = stage_of(s, turn, nst);
 #pragma unroll
     for (int p = 0; p < PC; ++p)
       if (p < pieces)
@@ -298,35 +339,13 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
       barrier();
       if (wm == 0 && more) begin(next);
 
-    // ---- results: x row in the lane, weight rows 8 g + 4 hi + 0 .. 3 of a 32-row tile in the registers; lanes 32 apart exchange
-    // halves of neighbouring g, so that each stores 8 columns
+    // ---- results: x row in the lane, weight rows in the registers
 #pragma unroll
     for (int m = 0; m < MC; ++m) {
       const int row = 32 * (2 * m + wm) + fr, rr = t.r0 + min(row, t.M - 1);
       const float sc = a.scale != nullptr ? a.scale[a.sorted != nullptr ? a.sorted[rr] : rr] : 1.0f;
       uint16_t* op = a.out + (int64_t)rr * a.ncols + t.n0 * NO + (GATED ? 16 : 32) * TN * wn + 8 * hi;
-#pragma unroll
-      for (int n = 0; n < (GATED ? TN / 2 : TN); ++n)
-#pragma unroll
-        for (int g = 0; g < 4; g += 2) {
-          uint32_t p[2][2];
-#pragma unroll
-          for (int q = 0; q < 2; ++q) {
-            float y[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-              if constexpr (GATED)
-                y[i] = moe_gate<ACT>(acc[n][m][4 * (g + q) + i] * sc, acc[TN / 2 + n][m][4 * (g + q) + i] * sc, a.limit, a.alpha);
-              else
-                y[i] = acc[n][m][4 * (g + q) + i] * sc;
-              if constexpr (ACT == MOE_ACT_RELU2) y[i] = fmaxf(y[i], 0.f) * fmaxf(y[i], 0.f);
-            }
-            p[q][0] = pack2(y[0], y[1]), p[q][1] = pack2(y[2], y[3]);
-          }
-          const auto u = __builtin_amdgcn_permlane32_swap(p[0][0], p[1][0], false, false);
-          const auto v = __builtin_amdgcn_permlane32_swap(p[0][1], p[1][1], false, false);
-          if (row < t.M) *reinterpret_cast<uint4*>(op + 32 * n + 8 * g) = make_uint4(u[0], v[0], u[1], v[1]);
-        }
+      store_row<ACT>([&](int n, int i) __attribute__((always_inline)) { return acc[n][m][i] * sc; }, op, row < t.M, a);
     }
     };
     if (mc == 4) run(IntC<4>{});
@@ -340,11 +359,202 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
   }
 }
 
+// ---- few tiles: 64 weight rows (with a gate 32 and the 32 matching ones) by up to 256 rows, one tile per workgroup
+// Where tiles of 256 weight rows leave compute units idle, these are four times as many, and what is left to bound them is the weights'
+// rate from HBM and the x rows' from L2. A stage is 64 K of both operands, the same LDS image as above; as many stages as LDS holds are on
+// their way, one barrier each. The waves are groups along K of a stage (2, up to 64 rows 4), whose sums meet in LDS at the end, so
+// that two waves per SIMD have work and each reads 64 weight rows by 32 or 64 x rows. PAIR: half the LDS and tiles of up to 128 rows, two workgroups
+// per CU, for the steps that have two tiles per CU (one's beginning and end beside the other's products).
+// us, tiles of 256 weight rows / these, at 32, 64, 128 and 192 rows per expert:
+//   16 experts of 2048 x 1024, 256 tiles    29 29 30 32 / 15 18 24 27       PAIR  15 19 28 28
+//   8 of 2048 x 2048, 256 tiles             28 29 30 30 / 15 17 24 26       PAIR  15 18 28 28
+//   16 of 1024 x 2048, 512 tiles            19 20 23 25 / 18 20 28 31       PAIR  15 17 26 32
+//   8 gated of 2048 x 2048, 512             40 39 42 46 / 34 37 50 56       PAIR  32 34 57 55
+//   8 of 4096 x 4096, 512                   68 67 73 80 / 57 63 88 99       PAIR  55 61 108 106
+//   8 of 14336 x 4096, 512                  233 224 248 272 / 175 213 307 402   PAIR 178 213 451 491 (80 rows 230 of 229)
+//   32 of 4096 x 2048, 1024                 102 107 126 144 / 109 126 171 199   PAIR 108 122 185 212
+// So steps of up to a tile per CU take them up to 192 rows per expert on average (more than 256 are two tiles), of up to two PAIR up to 80.
+constexpr int FN = 32 * TN, FUNIT = FN * ROWB;   // weight rows of a tile, bytes of 64 rows of a stage
+
+constexpr int few_lds(bool pair) { return (pair ? 80 : 160) * 1024; }
+
+template <int ACT, bool PAIR>
+__global__ void __launch_bounds__(64 * NW, (PAIR ? 4 : 2)) moe_gemm_few_kernel(MoeGemmArgs a) {
+  extern __shared__ __attribute__((aligned(1024))) char smem[];
+  constexpr bool GATED = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU;
+  constexpr int NO = GATED ? FN / 2 : FN, FM = PAIR ? 128 : 256, LDS = few_lds(PAIR);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 31, hi = lane >> 5;
+  const int nst = a.K / BK, NT = a.ncols / NO;
+
+  // ---- the workgroup's tile: XCD i (blocks i, i + 8, ..) takes the i-th eighth of the list, whose neighbours share x rows or weights
+  int total = 0;
+  for (int b = 0; b < a.experts; b += 64) {
+    const int m = a.offsets[min(b + lane + 1, a.experts)] - a.offsets[min(b + lane, a.experts)];
+    total += __builtin_amdgcn_readlane(scan64((m + FM - 1) / FM * NT, lane), 63);
+  }
+  const int per = (total + 7) / 8;
+  int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per || tile >= total) return;
+  Tile t;
+  for (int b = 0;; b += 64) {
+    const int o0 = a.offsets[min(b + lane, a.experts)], o1 = a.offsets[min(b + lane + 1, a.experts)];
+    const int own = (o1 - o0 + FM - 1) / FM * NT, upto = scan64(own, lane);
+    const uint64_t beyond = __builtin_amdgcn_ballot_w64(upto > tile);
+    if (beyond == 0) {   // (there is one: tile < total)
+      tile -= __builtin_amdgcn_readlane(upto, 63);
+      continue;
+    }
+    const int l = __builtin_ctzll(beyond);
+    tile -= __builtin_amdgcn_readlane(upto - own, l);
+    t.e = b + l;
+    t.r0 = __builtin_amdgcn_readlane(o0, l);
+    t.M = __builtin_amdgcn_readlane(o1, l) - t.r0;
+    break;
+  }
+  {
+    const int mts = (t.M + FM - 1) / FM, rows = ((t.M + mts - 1) / mts + 31) / 32 * 32, m0 = tile % mts * rows;
+    t.n0 = tile / mts;
+    t.M = min(t.M - m0, rows);
+    t.r0 += m0;
+    if (t.M <= 0) return;
+  }
+
+  t.turn = first_stage(t.e * NT + t.n0, nst);
+  auto run = [&](auto mx_) __attribute__((always_inline)) {
+    constexpr int MX = decltype(mx_)::value;             // 64-row pieces of x
+    constexpr int SLOT = FUNIT * (1 + MX), D = LDS / SLOT < 8 ? LDS / SLOT : 8;   // a stage in LDS, stages that it holds
+    constexpr int MW = MX == 1 ? 2 : 4, KG = NW / MW;    // waves along the x rows, along K
+    constexpr int MT = 2 * MX > MW ? 2 : 1, KS = BK / 16 / KG;   // 32-row tiles and 16-K steps of a wave
+    const int wm = wave % MW, kg = wave / MW;
+    // ---- the wave's pieces of a stage: 8 rows each, 16-byte chunk c of row r at place c ^ (r >> 1 & 7)
+    const int r8 = 8 * wave + lane / 8, col = 16 * (lane % 8 ^ (r8 >> 1 & 7));
+    const char* wp = reinterpret_cast<const char*>(a.w) + ((int64_t)t.e * (GATED ? 2 : 1) * a.ncols + t.n0 * NO +
+                                                            (GATED ? (r8 & 32 ? a.ncols : 0) + r8 % 32 : r8)) * a.K * 2 + col;
+    const char* xp[MX];
+#pragma unroll
+    for (int p = 0; p < MX; ++p) {
+      int row = t.r0 + min(r8 + 64 * p, t.M - 1);
+      if (a.sorted != nullptr) row = a.topk > 1 ? a.sorted[row] / a.topk : a.sorted[row];
+      xp[p] = reinterpret_cast<const char*>(a.x) + (int64_t)row * a.ldx * 2 + col;
+    }
+    auto issue = [&](int s, int slot) __attribute__((always_inline)) {
+      s = stage_of(s, t.turn, nst);
+      __builtin_amdgcn_global_load_lds((global_cvoid*)(wp + (int64_t)s * ROWB), (lds_void*)(smem + slot * SLOT + wave * 1024), 16, 0, 0);
+#pragma unroll
+      for (int p = 0; p < MX; ++p)
+        __builtin_amdgcn_global_load_lds((global_cvoid*)(xp[p] + (int64_t)s * ROWB),
+                                         (lds_void*)(smem + slot * SLOT + FUNIT * (1 + p) + wave * 1024), 16, 0, 0);
+    };
+    int lo[KS];   // a fragment of 32 rows: the lane's place at step kk
+#pragma unroll
+    for (int kk = 0; kk < KS; ++kk) lo[kk] = fr * ROWB + 16 * ((2 * (KS * kg + kk) + hi) ^ (fr >> 1 & 7));
+    f32x16_t acc[TN][MT] = {};
+#pragma unroll
+    for (int s = 0; s < D - 1; ++s)
+      if (s < nst) issue(s, s);
+    int slot = 0;
+#pragma unroll 1
+    for (int s = 0; s < nst; ++s) {
+      // stage s is there once no more than the stages behind it are on their way
+      const int behind = min(D - 2, nst - 1 - s);
+      if (behind == D - 2) wait_vm<(D - 2) * (1 + MX)>();
+      else if (D > 7 && behind == 5) wait_vm<5 * (1 + MX)>();
+      else if (D > 6 && behind == 4) wait_vm<4 * (1 + MX)>();
+      else if (D > 5 && behind == 3) wait_vm<3 * (1 + MX)>();
+      else if (D > 4 && behind == 2) wait_vm<2 * (1 + MX)>();
+      else if (behind == 1) wait_vm<1 + MX>();
+      else wait_vm<0>();
+      wait_lds();   // (the reads of stage s - 1, whose place is filled next)
+      barrier();
+      if (s + D - 1 < nst) issue(s + D - 1, slot == 0 ? D - 1 : slot - 1);
+      const char* wl = smem + slot * SLOT;
+      bf16x8_t wf[KS][TN], xf[KS][MT];
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk) {
+#pragma unroll
+        for (int n = 0; n < TN; ++n) wf[kk][n] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(wl + 32 * n * ROWB + lo[kk]));
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          xf[kk][m] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(wl + FUNIT + 32 * min(wm + MW * m, 2 * MX - 1) * ROWB + lo[kk]));
+      }
+#pragma unroll
+      for (int kk = 0; kk < KS; ++kk)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int n = 0; n < TN; ++n) acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[kk][n], xf[kk][m], acc[n][m], 0, 0, 0);
+      slot = slot == D - 1 ? 0 : slot + 1;
+    }
+    // ---- the groups' sums, the first group's last
+    wait_lds();
+    barrier();
+    float* sums = reinterpret_cast<float*>(smem);
+    static_assert((KG - 1) * MW * MT * TN * 16 * 256 <= LDS, "LDS of a compute unit");
+    auto place = [&](int g, int m, int n, int i) __attribute__((always_inline)) { return ((((g - 1) * MW + wm) * MT + m) * TN + n) * 1024 + 64 * i + lane; };
+    if (kg > 0) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < TN; ++n)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) sums[place(kg, m, n, i)] = acc[n][m][i];
+    }
+    wait_lds();
+    barrier();
+    if (kg > 0) return;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+#pragma unroll
+      for (int g = 1; g < KG; ++g)
+#pragma unroll
+        for (int n = 0; n < TN; ++n)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[n][m][i] += sums[place(g, m, n, i)];
+      const int row = 32 * (wm + MW * m) + fr, rr = t.r0 + min(row, t.M - 1);
+      const float sc = a.scale != nullptr ? a.scale[a.sorted != nullptr ? a.sorted[rr] : rr] : 1.0f;
+      uint16_t* op = a.out + (int64_t)rr * a.ncols + t.n0 * NO + 8 * hi;
+      store_row<ACT>([&](int n, int i) __attribute__((always_inline)) { return acc[n][m][i] * sc; }, op, row < t.M, a);
+    }
+  };
+  const int mx = (t.M + 63) / 64;
+  if (mx == 1) run(IntC<1>{});
+  else if (PAIR || mx == 2) run(IntC<2>{});
+  else if constexpr (!PAIR) {
+    if (mx == 3) run(IntC<3>{});
+    else run(IntC<4>{});
+  }
+}
+
+// `tile_rows` of the small tiles, one or two workgroups per CU; what a step takes
+enum { ROWS_WHOLE = 0, ROWS_FEW = 64, ROWS_PAIR = 32 };
+inline int few_tiles(const MoeGemmArgs& a) {
+  const int no = a.act >= MOE_ACT_SILU && a.act <= MOE_ACT_GELU ? FN / 2 : FN;
+  const int64_t tiles = (int64_t)std::min(a.experts, a.rows) * (a.ncols / no);   // of experts of up to 256 rows
+  if (tiles <= a.cus && a.rows <= 192 * (int64_t)a.experts) return ROWS_FEW;
+  return tiles <= 2 * a.cus && a.rows <= 80 * (int64_t)a.experts ? ROWS_PAIR : ROWS_WHOLE;
+}
+
+template <int ACT, bool PAIR> hipError_t launch_few(const MoeGemmArgs& a, hipStream_t s) {
+  auto* fn = moe_gemm_few_kernel<ACT, PAIR>;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, few_lds(PAIR));
+  if (e != hipSuccess) return e;
+  constexpr int NO = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU ? FN / 2 : FN;
+  const int64_t tiles = ((int64_t)std::min(a.experts, a.rows) + a.rows / (PAIR ? 128 : 256)) * (a.ncols / NO);   // at most
+  hipLaunchKernelGGL(fn, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(64 * NW), few_lds(PAIR), s, a);
+  return hipGetLastError();
+}
+
 template <int ACT> hipError_t launch_act(MoeGemmArgs a, hipStream_t s) {
-  auto* fn = moe_gemm_kernel<ACT>;
+  a.cus = num_cus();
+  const int few = a.tile_rows != 0 ? a.tile_rows : few_tiles(a);
+  if (few == ROWS_FEW) return launch_few<ACT, false>(a, s);
+  if (few == ROWS_PAIR) return launch_few<ACT, true>(a, s);
+  // (at most one row tile per expert on average: the places cost 0.6 % where they are all the first, 8 of 4096 x 14336, 1024 rows each)
+  constexpr int NO = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU ? BN / 2 : BN;
+  const bool turn = a.rows <= (int64_t)BM * a.experts && 2 * (int64_t)a.experts * (a.ncols / NO) >= a.cus;
+  auto* fn = turn ? moe_gemm_kernel<ACT, true> : moe_gemm_kernel<ACT, false>;
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, NU * UNIT);
   if (e != hipSuccess) return e;
-  a.cus = num_cus();
   hipLaunchKernelGGL(fn, dim3(8 * std::max(a.cus / 8, 1)), dim3(64 * NW), NU * UNIT, s, a);
   return hipGetLastError();
 }
@@ -362,7 +572,7 @@ bool moe_gemm_takes(const MoeGemmArgs& a) {
 hipError_t launch_moe_gemm(const MoeGemmArgs& a, hipStream_t s) {
   if (a.rows == 0) return hipSuccess;
   if (a.rows < 0 || a.experts < 1 || a.topk < 1 || !moe_gemm_takes(a)) return hipErrorInvalidValue;
-  if (a.tile_rows != 0 && (a.tile_rows < 128 || a.tile_rows > 256 || a.tile_rows % 32 != 0)) return hipErrorInvalidValue;
+  if (a.tile_rows != 0 && a.tile_rows != ROWS_FEW && a.tile_rows != ROWS_PAIR && (a.tile_rows < 128 || a.tile_rows > 256 || a.tile_rows % 32 != 0)) return hipErrorInvalidValue;
   switch (a.act) {
     case MOE_ACT_NONE: return launch_act<MOE_ACT_NONE>(a, s);
     case MOE_ACT_SILU: return launch_act<MOE_ACT_SILU>(a, s);

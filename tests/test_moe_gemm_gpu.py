@@ -219,3 +219,35 @@ def test_many_rows_of_large_experts_take_the_library(cuda, monkeypatch):
     for _ in range(3):
         graph.replay()
         assert ((out - want).float().norm() / want.float().norm()).item() < 1e-2
+
+
+@pytest.mark.parametrize("tile", [32, 64])   # two workgroups per compute unit, one
+@pytest.mark.parametrize("counts", [(0, 1, 63, 64, 65), (31, 0, 127, 128, 129, 192), (193, 255, 0, 256, 257), (513, 700, 2)])
+@pytest.mark.parametrize("K,ncols,act", [(64, 256, mix.MOE_NONE), (256, 128, mix.MOE_SILU), (448, 256, mix.MOE_CLAMPED), (512, 512, mix.MOE_RELU2),
+                                         (1088, 384, mix.MOE_GELU), (4096, 256, mix.MOE_NONE)])
+def test_small_tiles(cuda, tile, counts, K, ncols, act):
+    """Tiles of 64 weight rows: heights around 64-row pieces, fewer and more stages than LDS holds of each."""
+    topk = 2 if sum(counts) % 2 == 0 else 1
+    x, w, offsets, idx, scale = _case(counts, K, ncols, act in (mix.MOE_SILU, mix.MOE_CLAMPED, mix.MOE_GELU), topk)
+    for rows, sc in ((idx, None), (idx, scale), (None, None)):
+        if rows is None and topk > 1:
+            continue
+        out = torch.full((sum(counts), ncols), float("nan"), dtype=torch.bfloat16, device=cuda)
+        dev = [t.to(cuda) if t is not None else None for t in (x, w, offsets, rows, sc)]
+        assert mix._kern().moe_gemm(out, *dev[:4], topk if rows is not None else 1, dev[4], act, 1.5, 1.7, tile)
+        want = _want(x, w, offsets, rows, topk, act, sc, 1.5, 1.7)
+        tol = 2.0 ** -8 * (want.abs() + want.square().mean(1, keepdim=True).sqrt())
+        assert ((out.cpu().double() - want).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("tile,K,ncols,act", [(256, 448, 512, mix.MOE_NONE), (128, 64, 256, mix.MOE_SILU), (160, 1088, 256, mix.MOE_CLAMPED), (0, 640, 512, mix.MOE_RELU2)])
+def test_tiles_that_start_within_k(cuda, tile, K, ncols, act):
+    """Enough weight tiles that each starts at a stage of its own, beside experts of several row tiles, which start at the first."""
+    counts = [3, 0, 1, 300] * 16 + [40] * 8
+    x, w, offsets, idx, scale = _case(counts, K, ncols, act in (mix.MOE_SILU, mix.MOE_CLAMPED), 2)
+    out = torch.full((sum(counts), ncols), float("nan"), dtype=torch.bfloat16, device=cuda)
+    dev = [t.to(cuda) for t in (x, w, offsets, idx, scale)]
+    assert mix._kern().moe_gemm(out, *dev[:4], 2, dev[4], act, 1.5, 1.7, tile)
+    want = _want(x, w, offsets, idx, 2, act, scale, 1.5, 1.7)
+    tol = 2.0 ** -8 * (want.abs() + want.square().mean(1, keepdim=True).sqrt())
+    assert ((out.cpu().double() - want).abs() <= tol).all()
