@@ -140,7 +140,8 @@ hipError_t launch_moe_route(float* w, int* ids, const bf16_t* x, int64_t ldx, co
   return hipGetLastError();
 }
 
-// Few pairs and experts, one workgroup. offsets[E+1]; sorted[j] = flat (t*K+k) index; pos[flat] = j.
+// Few pairs and experts, one workgroup. offsets[E+1]; sorted[j] = flat (t*K+k) index; pos[flat] = j. An id outside
+// [0, E) is in no expert's rows.
 __global__ void __launch_bounds__(1024) moe_align_few_kernel(int* __restrict__ offsets, int* __restrict__ sorted,
                                                          int* __restrict__ pos, const int* __restrict__ ids, int n,
                                                          int E) {
@@ -148,7 +149,8 @@ __global__ void __launch_bounds__(1024) moe_align_few_kernel(int* __restrict__ o
   __shared__ int cur[256];
   for (int e = threadIdx.x; e < E; e += blockDim.x) cnt[e] = 0;
   __syncthreads();
-  for (int i = threadIdx.x; i < n; i += blockDim.x) atomicAdd(&cnt[ids[i]], 1);
+  for (int i = threadIdx.x; i < n; i += blockDim.x)
+    if ((unsigned)ids[i] < (unsigned)E) atomicAdd(&cnt[ids[i]], 1);
   __syncthreads();
   if (threadIdx.x == 0) {
     int acc = 0;
@@ -161,14 +163,14 @@ __global__ void __launch_bounds__(1024) moe_align_few_kernel(int* __restrict__ o
   }
   __syncthreads();
   for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    if ((unsigned)ids[i] >= (unsigned)E) continue;
     const int j = atomicAdd(&cur[ids[i]], 1);
     sorted[j] = i;
     pos[i] = j;
   }
 }
 
-// More pairs: one workgroup per expert; the same, and a pair's place in `sorted` ascends within its expert. An id outside [0, E) is in no
-// expert's rows. Every workgroup reads all ids, counts those of lower experts and of its own, and writes its own rows, whose places are
+// More pairs: one workgroup per expert; the same, and a pair's place in `sorted` ascends within its expert. Every workgroup reads all ids, counts those of lower experts and of its own, and writes its own rows, whose places are
 // neighbours: the one workgroup was bound by its scattered stores and by LDS atomics. This is bound by the first reading of the ids, which
 // no L2 holds, and by a CU's instructions, five per id and wave. us, few / this: 32764 pairs of 16 experts 24.0 / 9.0, 8192 of 8 6.9 / 5.3,
 // 5040 of 32 6.8 / 5.6, 4160 of 8 5.6 / 5.5, 1172 of 10 2.6 / 3.8 (lines of results that several XCDs share); with a launch's 5 us, 1024 of

@@ -216,6 +216,25 @@ _MOE_ACT = {ACT_SILU: MOE_SILU, ACT_CLAMPED: MOE_CLAMPED, ACT_GELU_TANH: MOE_GEL
 GROUPED_MAX_ROWS, GROUPED_ANY_ROWS_SIZE = 1792, 1 << 25
 
 
+DECODE_EXPERTS_MAX_T = 128   # tokens of a decode step whose experts stream through the decode products
+# From so many on the grouped product of prompts takes them instead, where the experts together have many weights and a matrix is not of the largest. us,
+# decode products / grouped, 64, 96 and 128 tokens: scaled mixture of 8 experts of 2048 x 2048 59 66 69 / 53 53 53, weighted one 56 62 63 / 54 54 54,
+# 16 of 2048 x 1024 44 50 53 / 46 46 47, 32 of 4096 x 2048 213 232 234 / 218 219 221; 80 and 128 tokens of 32 of 1024 x 1024 54 55 / 45 46; but 8 of
+# 2048 x 1024 29.2 32.8 / 29.9 30.5, 8 of 1024 x 1024 20 24 / 24 25, 32 of 512 x 256 14 14 / 18 18, 8 gated ones of 4096 x 4096 (96 and 128) 175 179 / 177 178.
+GROUPED_EXPERTS_MIN_T, GROUPED_MIN_WEIGHTS, GROUPED_MAX_MATRIX = 65, 1 << 25, 1 << 23
+
+
+def grouped_decode(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, act: int, buckets: int) -> bool:
+    """Whether a step of up to DECODE_EXPERTS_MAX_T tokens takes :func:`grouped_experts`: by its size, and only where both matrices tile and pairs
+    of so many ``buckets`` can be put in their order."""
+    e, h, f = w2.shape
+    if x.shape[0] < GROUPED_EXPERTS_MIN_T or e * h * f < GROUPED_MIN_WEIGHTS or h * f > GROUPED_MAX_MATRIX:
+        return False
+    return (x.dtype == w13.dtype == w2.dtype == torch.bfloat16 and h % 256 == 0 and f % (128 if MOE_SILU <= act <= MOE_GELU else 256) == 0
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and w13.is_contiguous() and w2.is_contiguous()
+            and (x.data_ptr() | w13.data_ptr() | w2.data_ptr()) % 16 == 0 and buckets <= 256)
+
+
 def grouped_experts(kern, x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, offsets: torch.Tensor, sorted_idx: torch.Tensor,
                     k: int, ys: torch.Tensor, act: int, limit: float = 0.0, alpha: float = 0.0,
                     scale: Optional[torch.Tensor] = None) -> bool:
@@ -323,7 +342,7 @@ def moe_input_scaled(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: to
         kern.combine_sum(out, ys, pos, extra, k)
         return out
 
-    if x.dtype == torch.bfloat16 and t <= 128:
+    if x.dtype == torch.bfloat16 and t <= DECODE_EXPERTS_MAX_T and not grouped_decode(x, w13, w2, MOE_SILU, e):
         # decode-sized steps: the framework's expert-streaming products (every routed expert's weights
         # streamed once, SiLU * up fused; no host read, hipGraph-capturable) on the scaled rows, unsorted where they tile
         from src import ops
@@ -480,7 +499,8 @@ def moe_output_weighted(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w:
     if e == 0:
         return finish(torch.empty(0, h, dtype=x.dtype, device=x.device), None)
     buckets = max(e, int(n_route))
-    if x.dtype == torch.bfloat16 and t <= 128:
+    if x.dtype == torch.bfloat16 and t <= DECODE_EXPERTS_MAX_T and not (
+            kind in _MOE_ACT and grouped_decode(x, w13, w2, _MOE_ACT[kind], buckets)):
         # decode-sized steps: the framework's expert-streaming products (every routed expert's weights streamed
         # once; no host read, hipGraph-capturable), of unsorted rows where they tile, else gathered in expert-sorted order. Identity
         # entries run nothing (sorted, they come behind the last real expert).

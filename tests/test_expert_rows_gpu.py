@@ -114,3 +114,51 @@ def test_rows_that_go_to_the_library(cuda, name):
     for a, b in ((x, r), (x[:, :100].contiguous(), r[:E, :100].contiguous())):
         (v, j), (u, k) = go(a, b), go(a.float(), b.float())
         assert torch.equal(j, k) and torch.allclose(u, v, rtol=2.0 ** -17, atol=0)
+
+
+@pytest.mark.parametrize("n,E", [(100, 4), (3000, 16)])
+def test_align_leaves_out_what_is_no_expert(cuda, n, E):
+    torch.manual_seed(n)
+    ids = torch.randint(-1, E + 2, (n,), device=cuda, dtype=torch.int32)
+    off, at, pos = (torch.full((s,), -7, dtype=torch.int32, device=cuda) for s in (E + 1, n, n))
+    mix._kern().moe_align(off, at, pos, ids, E)
+    real = (ids >= 0) & (ids < E)
+    m = int(real.sum())
+    assert off.tolist() == [0, *torch.bincount(ids[real].long(), minlength=E).cumsum(0).tolist()]
+    assert (at[m:] == -7).all() and (pos[~real] == -7).all() and torch.equal(at[pos[real].long()].long(), real.nonzero().flatten())
+    assert torch.equal(ids[at[:m].long()], ids[real].sort().values)
+
+
+@pytest.mark.parametrize("E,h,f,k,kind", [(64, 1024, 512, 2, mix.ACT_CLAMPED), (129, 512, 512, 3, mix.ACT_RELU2), (64, 1024, 576, 2, mix.ACT_SILU)])
+def test_experts_of_65_tokens_and_more(cuda, E, h, f, k, kind):
+    """Large decode steps go through the grouped product where it tiles (f = 576 it does not), eagerly and replayed: the same as 64 tokens at a time,
+    up to rounding. A hidden value is rounded once on one side, on the other with f = 576 three times, of which the gate's may count double (|g| up
+    to 3): 2^-9 3^-0.5 (1 + 1 + 4 + 1)^0.5 = 1.5 * 2^-9 root mean square; where both choices are one expert it adds up, 2^0.5 of a result's; 4.5
+    sigma (of 10^5 results) are 4.9 * 2^-8. The k experts' results are rounded themselves, 2^-9 each, with weights up to 1.25: 2^-8 k of the
+    value and 1.3 * 2^-8 of the root mean square."""
+    torch.manual_seed(E + h)
+    T, wide = 128, 2 if kind != mix.ACT_RELU2 else 1
+    x = torch.randn(T, h, device=cuda).bfloat16()
+    w13, w2 = torch.randn(E, wide * f, h, device=cuda).bfloat16() / h ** 0.5, torch.randn(E, h, f, device=cuda).bfloat16() / f ** 0.5
+    ids = torch.randint(0, E + 2, (T, k), device=cuda, dtype=torch.int32)
+    w = torch.rand(T, k, device=cuda) + 0.25
+
+    def weighted(a, b):
+        return mix.moe_output_weighted(x[a:b], w13, w2, w[a:b], ids[a:b], kind, 1.5, 1.7, E + 2)
+
+    def scaled(a, b):
+        return mix.moe_input_scaled(x[a:b], w13, w2, torch.ones_like(w[a:b]), ids[a:b] % E)
+
+    for step in (weighted, scaled) if wide == 2 else (weighted,):
+        want = torch.cat([step(0, 64), step(64, T)])
+        tol = 2.0 ** -8 * (k * want.abs() + 6.2 * want.square().mean(1, keepdim=True).sqrt())
+        for b in (65, 97, T):
+            assert ((step(0, b) - want[:b]).abs() <= tol[:b]).all()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            out = step(0, T)
+        for _ in range(3):
+            out.zero_()
+            g.replay()
+            assert ((out - want).abs() <= tol).all()
+            torch.cuda.synchronize()
