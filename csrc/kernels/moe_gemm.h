@@ -22,7 +22,7 @@ struct MoeGemmArgs {
   int act;
   float limit, alpha;
   int experts, rows, ncols, K;
-  int tile_rows;           // rows of a tile at most: 128, 160, 192, 224 or 256; 64, 32: the small tiles; 0: as the step's rows tile best
+  int tile_rows;           // rows of a tile at most: 128, 160, 192, 224 or 256; 64, 96: tiles of 64, 128 weight rows; 0: as the step's rows tile best
   int cus;                 // set by the launcher: compute units of the device
 };
 // whether launch_moe_gemm takes these sizes: K a multiple of 64, ncols of 256 (gated: 128), 16-byte aligned rows, offsets of rows

@@ -359,30 +359,32 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
   }
 }
 
-// ---- few tiles: 64 weight rows (with a gate 32 and the 32 matching ones) by up to 256 rows, one tile per workgroup
-// Where tiles of 256 weight rows leave compute units idle, these are four times as many, and what is left to bound them is the weights'
-// rate from HBM and the x rows' from L2. A stage is 64 K of both operands, the same LDS image as above; as many stages as LDS holds are on
-// their way, one barrier each. The waves are groups along K of a stage (2, up to 64 rows 4), whose sums meet in LDS at the end, so
-// that two waves per SIMD have work and each reads 64 weight rows by 32 or 64 x rows. PAIR: half the LDS and tiles of up to 128 rows, two workgroups
-// per CU, for the steps that have two tiles per CU (one's beginning and end beside the other's products).
-// us, tiles of 256 weight rows / these, at 32, 64, 128 and 192 rows per expert:
-//   16 experts of 2048 x 1024, 256 tiles    29 29 30 32 / 15 18 24 27       PAIR  15 19 28 28
-//   8 of 2048 x 2048, 256 tiles             28 29 30 30 / 15 17 24 26       PAIR  15 18 28 28
-//   16 of 1024 x 2048, 512 tiles            19 20 23 25 / 18 20 28 31       PAIR  15 17 26 32
-//   8 gated of 2048 x 2048, 512             40 39 42 46 / 34 37 50 56       PAIR  32 34 57 55
-//   8 of 4096 x 4096, 512                   68 67 73 80 / 57 63 88 99       PAIR  55 61 108 106
-//   8 of 14336 x 4096, 512                  233 224 248 272 / 175 213 307 402   PAIR 178 213 451 491 (80 rows 230 of 229)
-//   32 of 4096 x 2048, 1024                 102 107 126 144 / 109 126 171 199   PAIR 108 122 185 212
-// So steps of up to a tile per CU take them up to 192 rows per expert on average (more than 256 are two tiles), of up to two PAIR up to 80.
+// ---- few tiles: 64 NB weight rows (with a gate 32 NB and the 32 NB matching ones) by up to 256 rows, one tile per workgroup
+// Where tiles of 256 weight rows leave compute units idle, these are four times or twice as many, and what is left to bound them is the weights'
+// rate from HBM and, with many rows, LDS (x rows are read once per 64 weight rows). A stage is 64 K of both operands, the same LDS image as above; as many
+// stages as LDS holds are on their way, one barrier each. The waves are 2 or 4 along the x rows, NB along the weight rows, and what is left (2 or 4)
+// groups along K of a stage, whose sums meet in LDS at the end: two waves per SIMD have work, and a wave that has more x rows reads less.
+// us, tiles of 256 weight rows / 64 / 128, at 32, 64, 96, 128 and 160 rows per expert:
+//   16 experts of 2048 x 1024, 256 tiles of 64     29 29 30 30 31 / 15 18 19 24 25        / 18 23 24 30 31
+//   8 of 2048 x 2048, 256                          28 29 30 30 30 / 15 17 18 23 24        / 17 22 24 30 30
+//   16 of 1024 x 2048, 512                         19 20 20 23 24 / 18 22 24 29 31        / 15 17 17 21 21
+//   8 gated of 2048 x 2048, 512                    40 39 40 42 43 / 34 40 44 51 53        / 29 32 33 38 39
+//   8 of 4096 x 4096, 512                          68 67 70 73 77 / 57 64 71 84 90        / 51 54 56 63 69
+//   8 of 14336 x 4096, 512                         233 224 237 248 263 / 170 210 241 285 331   / 166 181 206 239 270
+//   32 of 4096 x 2048, 1024                        102 107 115 125 134 / 109 126 141 163 177   / 100 108 112 132 147
+//   8 gated of 4096 x 14336, 3584                  352 361 373 402 429 / 363 452 495 575 614   / 323 361 379 457 485
+// So steps of up to a tile of 64 per CU take these up to 192 rows per expert on average (27 of 32 us; from 257 rows they are two tiles), of up to two
+// those of 128 rows up to 144; larger ones up to 40. (Two workgroups per CU, each with half the LDS and tiles of 64 by up to 128 rows: 15 17 19 27 for
+// the third, 55 61 68 108 for the fifth.)
 constexpr int FN = 32 * TN, FUNIT = FN * ROWB;   // weight rows of a tile, bytes of 64 rows of a stage
 
-constexpr int few_lds(bool pair) { return (pair ? 80 : 160) * 1024; }
+constexpr int FEW_LDS = 160 * 1024;
 
-template <int ACT, bool PAIR>
-__global__ void __launch_bounds__(64 * NW, (PAIR ? 4 : 2)) moe_gemm_few_kernel(MoeGemmArgs a) {
+template <int ACT, int NB>
+__global__ void __launch_bounds__(64 * NW, 2) moe_gemm_few_kernel(MoeGemmArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   constexpr bool GATED = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU;
-  constexpr int NO = GATED ? FN / 2 : FN, FM = PAIR ? 128 : 256, LDS = few_lds(PAIR);
+  constexpr int NO = (GATED ? FN / 2 : FN) * NB;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 31, hi = lane >> 5;
   const int nst = a.K / BK, NT = a.ncols / NO;
 
@@ -390,7 +392,7 @@ __global__ void __launch_bounds__(64 * NW, (PAIR ? 4 : 2)) moe_gemm_few_kernel(M
   int total = 0;
   for (int b = 0; b < a.experts; b += 64) {
     const int m = a.offsets[min(b + lane + 1, a.experts)] - a.offsets[min(b + lane, a.experts)];
-    total += __builtin_amdgcn_readlane(scan64((m + FM - 1) / FM * NT, lane), 63);
+    total += __builtin_amdgcn_readlane(scan64((m + BM - 1) / BM * NT, lane), 63);
   }
   const int per = (total + 7) / 8;
   int tile = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
@@ -398,7 +400,7 @@ __global__ void __launch_bounds__(64 * NW, (PAIR ? 4 : 2)) moe_gemm_few_kernel(M
   Tile t;
   for (int b = 0;; b += 64) {
     const int o0 = a.offsets[min(b + lane, a.experts)], o1 = a.offsets[min(b + lane + 1, a.experts)];
-    const int own = (o1 - o0 + FM - 1) / FM * NT, upto = scan64(own, lane);
+    const int own = (o1 - o0 + BM - 1) / BM * NT, upto = scan64(own, lane);
     const uint64_t beyond = __builtin_amdgcn_ballot_w64(upto > tile);
     if (beyond == 0) {   // (there is one: tile < total)
       tile -= __builtin_amdgcn_readlane(upto, 63);
@@ -412,7 +414,7 @@ __global__ void __launch_bounds__(64 * NW, (PAIR ? 4 : 2)) moe_gemm_few_kernel(M
     break;
   }
   {
-    const int mts = (t.M + FM - 1) / FM, rows = ((t.M + mts - 1) / mts + 31) / 32 * 32, m0 = tile % mts * rows;
+    const int mts = (t.M + BM - 1) / BM, rows = ((t.M + mts - 1) / mts + 31) / 32 * 32, m0 = tile % mts * rows;
     t.n0 = tile / mts;
     t.M = min(t.M - m0, rows);
     t.r0 += m0;
@@ -422,14 +424,17 @@ __global__ void __launch_bounds__(64 * NW, (PAIR ? 4 : 2)) moe_gemm_few_kernel(M
   t.turn = first_stage(t.e * NT + t.n0, nst);
   auto run = [&](auto mx_) __attribute__((always_inline)) {
     constexpr int MX = decltype(mx_)::value;             // 64-row pieces of x
-    constexpr int SLOT = FUNIT * (1 + MX), D = LDS / SLOT < 8 ? LDS / SLOT : 8;   // a stage in LDS, stages that it holds
-    constexpr int MW = MX == 1 ? 2 : 4, KG = NW / MW;    // waves along the x rows, along K
-    constexpr int MT = 2 * MX > MW ? 2 : 1, KS = BK / 16 / KG;   // 32-row tiles and 16-K steps of a wave
-    const int wm = wave % MW, kg = wave / MW;
+    constexpr int SLOT = FUNIT * (NB + MX), D = FEW_LDS / SLOT < 8 ? FEW_LDS / SLOT : 8;   // a stage in LDS, stages that it holds
+    constexpr int MW = NB == 1 && MX % 2 == 0 ? 4 : 2, KG = NW / MW / NB;   // waves along the x rows, along K
+    constexpr int MT = 2 * MX / MW, KS = BK / 16 / KG;   // 32-row tiles and 16-K steps of a wave
+    const int wm = wave % MW, wn = wave / MW % NB, kg = wave / (MW * NB);
     // ---- the wave's pieces of a stage: 8 rows each, 16-byte chunk c of row r at place c ^ (r >> 1 & 7)
     const int r8 = 8 * wave + lane / 8, col = 16 * (lane % 8 ^ (r8 >> 1 & 7));
-    const char* wp = reinterpret_cast<const char*>(a.w) + ((int64_t)t.e * (GATED ? 2 : 1) * a.ncols + t.n0 * NO +
-                                                            (GATED ? (r8 & 32 ? a.ncols : 0) + r8 % 32 : r8)) * a.K * 2 + col;
+    const char* wp[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+      wp[b] = reinterpret_cast<const char*>(a.w) + ((int64_t)t.e * (GATED ? 2 : 1) * a.ncols + t.n0 * NO + b * (NO / NB) +
+                                                     (GATED ? (r8 & 32 ? a.ncols : 0) + r8 % 32 : r8)) * a.K * 2 + col;
     const char* xp[MX];
 #pragma unroll
     for (int p = 0; p < MX; ++p) {
@@ -439,11 +444,13 @@ __global__ void __launch_bounds__(64 * NW, (PAIR ? 4 : 2)) moe_gemm_few_kernel(M
     }
     auto issue = [&](int s, int slot) __attribute__((always_inline)) {
       s = stage_of(s, t.turn, nst);
-      __builtin_amdgcn_global_load_lds((global_cvoid*)(wp + (int64_t)s * ROWB), (lds_void*)(smem + slot * SLOT + wave * 1024), 16, 0, 0);
+#pragma unroll
+      for (int b = 0; b < NB; ++b)
+        __builtin_amdgcn_global_load_lds((global_cvoid*)(wp[b] + (int64_t)s * ROWB), (lds_void*)(smem + slot * SLOT + FUNIT * b + wave * 1024), 16, 0, 0);
 #pragma unroll
       for (int p = 0; p < MX; ++p)
         __builtin_amdgcn_global_load_lds((global_cvoid*)(xp[p] + (int64_t)s * ROWB),
-                                         (lds_void*)(smem + slot * SLOT + FUNIT * (1 + p) + wave * 1024), 16, 0, 0);
+                                         (lds_void*)(smem + slot * SLOT + FUNIT * (NB + p) + wave * 1024), 16, 0, 0);
     };
     int lo[KS];   // a fragment of 32 rows: the lane's place at step kk
 #pragma unroll
@@ -457,12 +464,12 @@ __global__ void __launch_bounds__(64 * NW, (PAIR ? 4 : 2)) moe_gemm_few_kernel(M
     for (int s = 0; s < nst; ++s) {
       // stage s is there once no more than the stages behind it are on their way
       const int behind = min(D - 2, nst - 1 - s);
-      if (behind == D - 2) wait_vm<(D - 2) * (1 + MX)>();
-      else if (D > 7 && behind == 5) wait_vm<5 * (1 + MX)>();
-      else if (D > 6 && behind == 4) wait_vm<4 * (1 + MX)>();
-      else if (D > 5 && behind == 3) wait_vm<3 * (1 + MX)>();
-      else if (D > 4 && behind == 2) wait_vm<2 * (1 + MX)>();
-      else if (behind == 1) wait_vm<1 + MX>();
+      if (behind == D - 2) wait_vm<(D - 2) * (NB + MX)>();
+      else if (D > 7 && behind == 5) wait_vm<5 * (NB + MX)>();
+      else if (D > 6 && behind == 4) wait_vm<4 * (NB + MX)>();
+      else if (D > 5 && behind == 3) wait_vm<3 * (NB + MX)>();
+      else if (D > 4 && behind == 2) wait_vm<2 * (NB + MX)>();
+      else if (D > 3 && behind == 1) wait_vm<NB + MX>();
       else wait_vm<0>();
       wait_lds();   // (the reads of stage s - 1, whose place is filled next)
       barrier();
@@ -472,10 +479,10 @@ __global__ void __launch_bounds__(64 * NW, (PAIR ? 4 : 2)) moe_gemm_few_kernel(M
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk) {
 #pragma unroll
-        for (int n = 0; n < TN; ++n) wf[kk][n] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(wl + 32 * n * ROWB + lo[kk]));
+        for (int n = 0; n < TN; ++n) wf[kk][n] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(wl + FUNIT * wn + 32 * n * ROWB + lo[kk]));
 #pragma unroll
         for (int m = 0; m < MT; ++m)
-          xf[kk][m] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(wl + FUNIT + 32 * min(wm + MW * m, 2 * MX - 1) * ROWB + lo[kk]));
+          xf[kk][m] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(wl + FUNIT * NB + 32 * (wm + MW * m) * ROWB + lo[kk]));
       }
 #pragma unroll
       for (int kk = 0; kk < KS; ++kk)
@@ -489,8 +496,8 @@ __global__ void __launch_bounds__(64 * NW, (PAIR ? 4 : 2)) moe_gemm_few_kernel(M
     wait_lds();
     barrier();
     float* sums = reinterpret_cast<float*>(smem);
-    static_assert((KG - 1) * MW * MT * TN * 16 * 256 <= LDS, "LDS of a compute unit");
-    auto place = [&](int g, int m, int n, int i) __attribute__((always_inline)) { return ((((g - 1) * MW + wm) * MT + m) * TN + n) * 1024 + 64 * i + lane; };
+    static_assert((KG - 1) * MW * NB * MT * TN * 16 * 256 <= FEW_LDS, "LDS of a compute unit");
+    auto place = [&](int g, int m, int n, int i) __attribute__((always_inline)) { return (((((g - 1) * NB + wn) * MW + wm) * MT + m) * TN + n) * 1024 + 64 * i + lane; };
     if (kg > 0) {
 #pragma unroll
       for (int m = 0; m < MT; ++m)
@@ -512,43 +519,41 @@ __global__ void __launch_bounds__(64 * NW, (PAIR ? 4 : 2)) moe_gemm_few_kernel(M
           for (int i = 0; i < 16; ++i) acc[n][m][i] += sums[place(g, m, n, i)];
       const int row = 32 * (wm + MW * m) + fr, rr = t.r0 + min(row, t.M - 1);
       const float sc = a.scale != nullptr ? a.scale[a.sorted != nullptr ? a.sorted[rr] : rr] : 1.0f;
-      uint16_t* op = a.out + (int64_t)rr * a.ncols + t.n0 * NO + 8 * hi;
+      uint16_t* op = a.out + (int64_t)rr * a.ncols + t.n0 * NO + wn * (NO / NB) + 8 * hi;
       store_row<ACT>([&](int n, int i) __attribute__((always_inline)) { return acc[n][m][i] * sc; }, op, row < t.M, a);
     }
   };
   const int mx = (t.M + 63) / 64;
   if (mx == 1) run(IntC<1>{});
-  else if (PAIR || mx == 2) run(IntC<2>{});
-  else if constexpr (!PAIR) {
-    if (mx == 3) run(IntC<3>{});
-    else run(IntC<4>{});
-  }
+  else if (mx == 2) run(IntC<2>{});
+  else if (mx == 3) run(IntC<3>{});
+  else run(IntC<4>{});
 }
 
-// `tile_rows` of the small tiles, one or two workgroups per CU; what a step takes
-enum { ROWS_WHOLE = 0, ROWS_FEW = 64, ROWS_PAIR = 32 };
+// `tile_rows` of the tiles of 64 and 128 weight rows; what a step takes
+enum { ROWS_WHOLE = 0, ROWS_64 = 64, ROWS_128 = 96 };
 inline int few_tiles(const MoeGemmArgs& a) {
   const int no = a.act >= MOE_ACT_SILU && a.act <= MOE_ACT_GELU ? FN / 2 : FN;
   const int64_t tiles = (int64_t)std::min(a.experts, a.rows) * (a.ncols / no);   // of experts of up to 256 rows
-  if (tiles <= a.cus && a.rows <= 192 * (int64_t)a.experts) return ROWS_FEW;
-  return tiles <= 2 * a.cus && a.rows <= 80 * (int64_t)a.experts ? ROWS_PAIR : ROWS_WHOLE;
+  if (tiles <= a.cus && a.rows <= 192 * (int64_t)a.experts) return ROWS_64;
+  return a.rows <= (tiles <= 2 * a.cus ? 144 : 40) * (int64_t)a.experts ? ROWS_128 : ROWS_WHOLE;
 }
 
-template <int ACT, bool PAIR> hipError_t launch_few(const MoeGemmArgs& a, hipStream_t s) {
-  auto* fn = moe_gemm_few_kernel<ACT, PAIR>;
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, few_lds(PAIR));
+template <int ACT, int NB> hipError_t launch_few(const MoeGemmArgs& a, hipStream_t s) {
+  auto* fn = moe_gemm_few_kernel<ACT, NB>;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, FEW_LDS);
   if (e != hipSuccess) return e;
-  constexpr int NO = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU ? FN / 2 : FN;
-  const int64_t tiles = ((int64_t)std::min(a.experts, a.rows) + a.rows / (PAIR ? 128 : 256)) * (a.ncols / NO);   // at most
-  hipLaunchKernelGGL(fn, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(64 * NW), few_lds(PAIR), s, a);
+  constexpr int NO = (ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU ? FN / 2 : FN) * NB;
+  const int64_t tiles = ((int64_t)std::min(a.experts, a.rows) + a.rows / BM) * (a.ncols / NO);   // at most
+  hipLaunchKernelGGL(fn, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(64 * NW), FEW_LDS, s, a);
   return hipGetLastError();
 }
 
 template <int ACT> hipError_t launch_act(MoeGemmArgs a, hipStream_t s) {
   a.cus = num_cus();
   const int few = a.tile_rows != 0 ? a.tile_rows : few_tiles(a);
-  if (few == ROWS_FEW) return launch_few<ACT, false>(a, s);
-  if (few == ROWS_PAIR) return launch_few<ACT, true>(a, s);
+  if (few == ROWS_64) return launch_few<ACT, 1>(a, s);
+  if (few == ROWS_128) return launch_few<ACT, 2>(a, s);
   // (at most one row tile per expert on average: the places cost 0.6 % where they are all the first, 8 of 4096 x 14336, 1024 rows each)
   constexpr int NO = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU ? BN / 2 : BN;
   const bool turn = a.rows <= (int64_t)BM * a.experts && 2 * (int64_t)a.experts * (a.ncols / NO) >= a.cus;
@@ -572,7 +577,7 @@ bool moe_gemm_takes(const MoeGemmArgs& a) {
 hipError_t launch_moe_gemm(const MoeGemmArgs& a, hipStream_t s) {
   if (a.rows == 0) return hipSuccess;
   if (a.rows < 0 || a.experts < 1 || a.topk < 1 || !moe_gemm_takes(a)) return hipErrorInvalidValue;
-  if (a.tile_rows != 0 && a.tile_rows != ROWS_FEW && a.tile_rows != ROWS_PAIR && (a.tile_rows < 128 || a.tile_rows > 256 || a.tile_rows % 32 != 0)) return hipErrorInvalidValue;
+  if (a.tile_rows != 0 && a.tile_rows != ROWS_64 && a.tile_rows != ROWS_128 && (a.tile_rows < 128 || a.tile_rows > 256 || a.tile_rows % 32 != 0)) return hipErrorInvalidValue;
   switch (a.act) {
     case MOE_ACT_NONE: return launch_act<MOE_ACT_NONE>(a, s);
     case MOE_ACT_SILU: return launch_act<MOE_ACT_SILU>(a, s);

@@ -221,12 +221,12 @@ def test_many_rows_of_large_experts_take_the_library(cuda, monkeypatch):
         assert ((out - want).float().norm() / want.float().norm()).item() < 1e-2
 
 
-@pytest.mark.parametrize("tile", [32, 64])   # two workgroups per compute unit, one
+@pytest.mark.parametrize("tile", [64, 96])   # 64, 128 weight rows
 @pytest.mark.parametrize("counts", [(0, 1, 63, 64, 65), (31, 0, 127, 128, 129, 192), (193, 255, 0, 256, 257), (513, 700, 2)])
 @pytest.mark.parametrize("K,ncols,act", [(64, 256, mix.MOE_NONE), (256, 128, mix.MOE_SILU), (448, 256, mix.MOE_CLAMPED), (512, 512, mix.MOE_RELU2),
                                          (1088, 384, mix.MOE_GELU), (4096, 256, mix.MOE_NONE)])
 def test_small_tiles(cuda, tile, counts, K, ncols, act):
-    """Tiles of 64 weight rows: heights around 64-row pieces, fewer and more stages than LDS holds of each."""
+    """Tiles of 64 and 128 weight rows: heights around 64-row pieces, fewer and more stages than LDS holds of each."""
     topk = 2 if sum(counts) % 2 == 0 else 1
     x, w, offsets, idx, scale = _case(counts, K, ncols, act in (mix.MOE_SILU, mix.MOE_CLAMPED, mix.MOE_GELU), topk)
     for rows, sc in ((idx, None), (idx, scale), (None, None)):
