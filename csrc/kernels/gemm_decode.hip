@@ -167,6 +167,7 @@ __device__ __forceinline__ void gd_body(char* smem, void* Yv, int64_t ldy, const
                                         const bf16_t* __restrict__ W, int M, int N_out, int K,
                                         const FZ& fz, const int bx, const int by, const int ny, const int* list = nullptr) {
   constexpr bool IDS = EPI == 5 || EPI == 7;
+  constexpr bool TURNS = IDS || ((EPI == 0 || EPI == 1) && SKC == 0);   // (0, 1: of sorted rows too; the others are dense)
   constexpr int ROWB = KC * 2;                 // bytes per image row
   constexpr int CPR = KC / 8;                  // 16-byte chunks per row
   constexpr int RPP = 64 / CPR;                // rows per 1-KiB DMA piece
@@ -241,8 +242,15 @@ __device__ __forceinline__ void gd_body(char* smem, void* Yv, int64_t ldy, const
     isw[p] = row < WR;
   }
   const int64_t wstep = fz.tiled ? (int64_t)(WR / RPP) * 512 : KC;  // W elements per K-chunk
+  // Experts' weights: tiles that go through K in step ask few memory channels for rows that are a power of two apart, so each starts at a chunk
+  // of its own, spread by the golden ratio, and goes round. us of a layer, in step / so: 8 gated experts of 4096 x 14336, 40 tokens 478 / 445; 8 of 4096 x
+  // 4096 173 / 139; 32 of 4096 x 2048 213 / 187; 8 of 2048 x 2048, 32 tokens 56 / 51. One matrix that all tiles read (dense layers) is faster in
+  // step: Llama decode, 1 request 517 / 572, 32 requests 623 / 661.
+  int turn = 0;
+  if (IDS || (TURNS && fz.grp_off != nullptr)) turn = (int)((uint64_t)((blockIdx.z * gridDim.x + bx) * 2654435769u) * (uint32_t)nch >> 32);
   auto issue = [&](int c) {
     char* slot = smem + (c % S) * SLOT;
+    if constexpr (TURNS) c = c + turn >= nch ? c + turn - nch : c + turn;
 #pragma unroll
     for (int p = 0; p < PER_WAVE; ++p) {
       // a piece is all-weight or all-activation rows: wave-uniform branch
@@ -873,7 +881,7 @@ constexpr size_t ids_ring(int wr, int xr, int kc) {
 // holds them, not one for all rows of the step: it is read with every chunk of K and takes its part of the ring. Bound by the weights'
 // stream. Both products of 8 experts of 2048 x 2048, clamped gate, two of 10 choices (us; separate sort and activation, image of the
 // step's rows -> this): 32 tokens 33.8 + 18.1 + 9.5 -> 31.7 + 14.7, 128 tokens 55.9 + 27.3 + 9.5 -> 33.3 + 18.4; 32 experts of 4096 x 2048, four of them,
-// 64 tokens 149 + 157 -> 95 + 100 (4.6 TB/s).
+// 64 tokens 149 + 157 -> 95 + 100 (4.6 TB/s; with places of K of their own 189 of 213 for the layer).
 template <int WR, int EPI, int KC, int XR>
 __global__ void __launch_bounds__(NTH) gemm_decode_ids_kernel(void* __restrict__ Y, int64_t ldy, const bf16_t* __restrict__ X, int64_t ldx,
                                                               const bf16_t* __restrict__ W, int N_out, int K, MoeDecodeFuse fz) {

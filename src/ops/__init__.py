@@ -848,7 +848,8 @@ def moe_apply(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: torch.Ten
     x = x.contiguous()
     # rows of the extra groups are never computed: zero them so that weight 0 x row stays 0
     ys = (torch.zeros if groups > e else torch.empty)(t * k, hdim, dtype=x.dtype, device=x.device)
-    if MOE_IDS_MIN_T <= t <= MOE_DECODE_MAX_T and decode_experts(kern, x, w13, w2, ids, k, t, MOE_SILU, ys=ys) is not None:
+    # (eight experts of 4096 x 14336, us, sorted / unsorted: 1 token 153 / 130, 8 tokens 466 / 436, 32 tokens 479 / 442)
+    if t <= MOE_DECODE_MAX_T and decode_experts(kern, x, w13, w2, ids, k, t, MOE_SILU, ys=ys) is not None:
         if residual is not None:
             kern.moe_combine_residual(ssp, residual, ys, _NO_ROWS(x.device), w)
             return residual
@@ -913,11 +914,6 @@ def moe_apply(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: torch.Ten
 
 
 MOE_LIBRARY_MIN_TOKENS = 256
-# Tokens from which decode steps take the products of unsorted rows, whose activation image goes with an expert's rows instead of the step's
-# (eight experts of 4096 x 14336, both products, us, sorted / unsorted: 32 tokens 459 / 470 without the sort's 5, 128 tokens 732 / 536). The line is
-# drawn for such experts and holds for every width: eight of 2048 x 2048 would gain from 1 token on (whole input-scaled mixture, whose sorted
-# form is the same: 8 tokens 60 / 56, 32 tokens 68 / 61).
-MOE_IDS_MIN_T = 33
 _NO_ROWS_CACHE: dict = {}
 
 

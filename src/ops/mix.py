@@ -218,10 +218,10 @@ GROUPED_MAX_ROWS, GROUPED_ANY_ROWS_SIZE = 1792, 1 << 25
 
 DECODE_EXPERTS_MAX_T = 128   # tokens of a decode step whose experts stream through the decode products
 # From so many on the grouped product of prompts takes them instead, where the experts together have many weights and a matrix is not of the largest. us,
-# decode products / grouped, 64, 96 and 128 tokens: scaled mixture of 8 experts of 2048 x 2048 59 66 69 / 53 53 53, weighted one 56 62 63 / 54 54 54,
-# 16 of 2048 x 1024 44 50 53 / 46 46 47, 32 of 4096 x 2048 213 232 234 / 218 219 221; 80 and 128 tokens of 32 of 1024 x 1024 54 55 / 45 46; but 8 of
-# 2048 x 1024 29.2 32.8 / 29.9 30.5, 8 of 1024 x 1024 20 24 / 24 25, 32 of 512 x 256 14 14 / 18 18, 8 gated ones of 4096 x 4096 (96 and 128) 175 179 / 177 178.
-GROUPED_EXPERTS_MIN_T, GROUPED_MIN_WEIGHTS, GROUPED_MAX_MATRIX = 65, 1 << 25, 1 << 23
+# decode products / grouped, 65, 96 and 128 tokens: scaled mixture of 8 experts of 2048 x 2048 60 62 67 / 52 53 52, weighted one 57 58 62 / 52 53 53,
+# 16 of 2048 x 1024 46 47 52 / 45 45 45; 80 and 128 tokens of 32 of 1024 x 1024 54 56 / 46 47, 32 of 2048 x 2048 158 161 / 155 161; but 8 of 2048 x
+# 1024 29.2 32.8 / 29.9 30.5, 8 of 1024 x 1024 20 24 / 24 25, 32 of 512 x 256 14 14 / 18 18, 32 of 4096 x 2048 (65, 96 and 128) 202 209 215 / 221 222 223.
+GROUPED_EXPERTS_MIN_T, GROUPED_MIN_WEIGHTS, GROUPED_MAX_MATRIX = 65, 1 << 25, 1 << 22
 
 
 def grouped_decode(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, act: int, buckets: int) -> bool:
@@ -348,11 +348,10 @@ def moe_input_scaled(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: to
         from src import ops
 
         tiles = ops._moe_decode_tiles(h, w13.shape[1] // 2, t) if ops.native_available() else None
-        # The sorted form has the activation in its first product too, and so only the sort to lose. It keeps few tokens of large experts whose
-        # gate's halves of weight rows are a multiple of 4 KiB long: its tiles of 32 rows read such weights faster than the unsorted form's
-        # of 64 (8 experts, us, sorted / unsorted: 4096 x 4096, 2 tokens 80 / 83, 8 tokens 140 / 160, 32 tokens 159 / 175; 4096 x 2048, 8 tokens 90 / 94,
-        # 32 tokens 97 / 103; their first product of 6144 x 2048 alone 74 / 80; but 4096 x 1024 59 / 59 and 64 / 63, 2048 x 2048 60 / 56 and 68 / 61,
-        # 3072 x 2048 70 / 67 and 83 / 76).
+        # The sorted form has the activation in its first product too, and so only the sort to lose. Few tokens of large experts whose gate's halves of
+        # weight rows are a multiple of 4 KiB long keep it: its tiles of 32 rows read such weights faster than the unsorted form's of 64 while both went through K
+        # in step (8 experts of 4096 x 4096, us, sorted / unsorted, 2 tokens 80 / 83, 8 tokens 140 / 160, 32 tokens 159 / 175). With places of K of their
+        # own they are within 7 %: 12 tokens 145 / 140, 24 tokens 150 / 141.
         sort = tiles is not None and tiles[0][0] <= 32 and h >= 4096 and h % 2048 == 0 and w2.shape[2] >= 2048 and t <= 32 and n >= 4
         if ops.native_available() and ids.dtype == torch.int32 and n > 0 and not sort and decode_tiles(w13, w2, t, n, MOE_SILU) is not None:
             xs = torch.empty(n, h, dtype=x.dtype, device=x.device)
