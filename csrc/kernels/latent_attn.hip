@@ -471,6 +471,7 @@ inline hipError_t launch_merge(const LatentAttnArgs& a, hipStream_t s) {
 // tiles in LDS for both products, by divisions at run time (rank 256 + 32, main kernel + merge, us): 32 sequences of 750 - 1500 keys, 16 heads
 // 36 + 10 -> 12 + 4.7 (21 MB of rows: 4 at the copy rate, latency of three tiles), 64 of 1000 - 2000, 32 heads 87 + 9 -> 24 + 4 (4.0 TB/s with L2), 3 of
 // 600 24 + 8 -> 9 + 4, 58 of 10 17 -> 8.
+// FINE: the weights enter the products in two bf16 parts (more than 32 heads: launch_decode).
 template <int NDB, int NROT> struct DecodeTile {
   static constexpr int R = 32 * NDB, NK = NDB + (NROT + 1) / 2, DK = R + 16 * NROT;   // latent columns, 32-wide steps of a row, its width
   static constexpr int PB = 2 * R + 32;                                               // pitch in LDS, bytes: 4 rows on different banks
@@ -478,7 +479,7 @@ template <int NDB, int NROT> struct DecodeTile {
   static constexpr int wave = 32 * PB > 64 * OP ? 32 * PB : 64 * OP;
   static constexpr int total = 4 * wave + 4 * 16 * 2 * 4;
 };
-template <int NDB, int NROT>
+template <int NDB, int NROT, bool FINE>
 __global__ void __launch_bounds__(256, 2) latent_attn_decode_kernel(LatentAttnArgs a, int hblocks) {
   using Z = DecodeTile<NDB, NROT>;
   constexpr int R = Z::R, NK = Z::NK, ND = R / 16;
@@ -602,8 +603,12 @@ __global__ void __launch_bounds__(256, 2) latent_attn_decode_kernel(LatentAttnAr
         l += sc[t][e];
       }
     m = mn;
-    const bf16x8_t pf = __builtin_bit_cast(
-        bf16x8_t, make_uint4(pack2(sc[0][0], sc[0][1]), pack2(sc[0][2], sc[0][3]), pack2(sc[1][0], sc[1][1]), pack2(sc[1][2], sc[1][3])));
+    const uint4 hp = make_uint4(pack2(sc[0][0], sc[0][1]), pack2(sc[0][2], sc[0][3]), pack2(sc[1][0], sc[1][1]), pack2(sc[1][2], sc[1][3]));
+    const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, hp);
+    bf16x8_t pl;
+    if constexpr (FINE)
+      pl = __builtin_bit_cast(bf16x8_t, make_uint4(rest2(sc[0][0], sc[0][1], hp.x), rest2(sc[0][2], sc[0][3], hp.y), rest2(sc[1][0], sc[1][1], hp.z),
+                                                   rest2(sc[1][2], sc[1][3], hp.w)));
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     if (__ballot(alpha != 1.0f) != 0) {
@@ -615,6 +620,7 @@ __global__ void __launch_bounds__(256, 2) latent_attn_decode_kernel(LatentAttnAr
       const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(rd + 32 * d));
       const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(rd + 16 * Z::PB + 32 * d));
       const short8_t v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+      if constexpr (FINE) o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, v), pl, o[d], 0, 0, 0);
       o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, v), pf, o[d], 0, 0, 0);
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // the tile is read before the next one replaces it
@@ -692,8 +698,11 @@ inline bool decode_fits(const LatentAttnArgs& a) {
   const int r = a.sh.rank, d = a.sh.rot_dim;
   return a.impl == 0 && a.cu_q == nullptr && a.max_q == 1 && mfma_ok(a) && (r == 64 || r == 128 || r == 256) && (d == 0 || d == 16 || d == 32 || d == 64);
 }
+// Two bf16 parts of the weights for more than 32 heads: such steps went through latent_attn_wide_kernel or FINE splits, which have them, and in one
+// part were up to 10 % further from 64 bits (in two, 40, 64 and 128 heads, 1.0001 of those kernels; 2 - 8 % of the time). Up to 32 heads the
+// kernels before had one part, and more splits: 0.988 of their distance in one.
 template <int NDB, int NROT> hipError_t launch_decode(const LatentAttnArgs& a, hipStream_t s) {
-  const auto fn = latent_attn_decode_kernel<NDB, NROT>;
+  const auto fn = a.heads > 32 ? latent_attn_decode_kernel<NDB, NROT, true> : latent_attn_decode_kernel<NDB, NROT, false>;
   constexpr int smem = DecodeTile<NDB, NROT>::total;
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
   if (e != hipSuccess) return e;
@@ -1296,7 +1305,7 @@ hipError_t launch_mfma_rq_any(const LatentAttnArgs& a, hipStream_t s) {
 hipError_t launch_mfma_any(const LatentAttnArgs& a, hipStream_t s) {
   if (decode_fits(a)) return launch_decode_any(a, s);
   if (a.impl != 3 && a.nsplit <= 1 && mfma_rq_fits(a)) return launch_mfma_rq_any(a, s);
-  // one wave per workgroup when a sequence brings at most 32 rows (decode steps): small LDS, many workgroups
+  // one wave per workgroup when a sequence brings at most 32 rows (decode steps of other widths): small LDS, many workgroups
   return (int64_t)a.max_q * a.heads <= 32 ? launch_mfma_ndb<1>(a, s) : launch_mfma_ndb<4>(a, s);
 }
 
