@@ -313,16 +313,15 @@ template <int PL> __device__ __forceinline__ int take_best(uint32_t (&key)[PL], 
 }
 
 // The K largest of a token's logits z [E], lowest index on ties, and their sigmoids, by a whole wave with PL experts a lane. NaN is no
-// candidate, -inf only if LOWEST; without one expert 0 is chosen with a logit of 0.
-template <int PL, bool LOWEST>
+// candidate (-inf is one, of weight 0); without one expert 0 is chosen with a logit of 0.
+template <int PL>
 __device__ __forceinline__ void sigmoid_select(const float* z, int E, int K, float* w_out, int* id_out) {
   const int lane = threadIdx.x & 63;
   uint32_t key[PL];
 #pragma unroll
   for (int i = 0; i < PL; ++i) {
     const int e = lane + 64 * i;
-    const float v = e < E ? z[e] : NAN;
-    key[i] = LOWEST || v != -INFINITY ? order_bits(v) : 0;
+    key[i] = e < E ? order_bits(z[e]) : 0;
   }
   float w[PL];
   int id[PL];
@@ -349,7 +348,7 @@ __global__ void __launch_bounds__(RNT) route_sigmoid_topk_kernel(float* w_out, i
   const bool vec = !x_f32 && !wr_f32 && H % 8 == 0 && xstride % 8 == 0 && aligned16(x) && aligned16(wr);
   router_logits(z, x, t * xstride, x_f32, wr, wr_f32, H, E, vec);
   __syncthreads();
-  if (threadIdx.x < 64) sigmoid_select<ROUTE_E_MAX / 64, false>(z, E, K, w_out + t * K, id_out + t * K);
+  if (threadIdx.x < 64) sigmoid_select<ROUTE_E_MAX / 64>(z, E, K, w_out + t * K, id_out + t * K);
 }
 
 // Selection alone, from logits already computed (a library fp32 GEMM for prompt-sized steps): one thread per token.
@@ -730,7 +729,7 @@ __global__ void __launch_bounds__(512) route_rows_kernel(const RouteRows a) {
     const int64_t t = t0 + i;
     float* w = a.w + t * a.K;
     int* ids = a.ids + t * a.K;
-    if constexpr (KIND == ROUTE_SIGMOID) sigmoid_select<1, true>(z[i], a.E, a.K, w, ids);
+    if constexpr (KIND == ROUTE_SIGMOID) sigmoid_select<1>(z[i], a.E, a.K, w, ids);
     if constexpr (KIND == ROUTE_SOFTMAX) softmax_select_wave<1>(z[i], sc[wave], a.corr, a.E, a.K, w, ids);
     if constexpr (KIND == ROUTE_GROUPED) grouped_select<1>(z[i], sc[wave], gopen[wave], a.E, a.K, a.count, a.keep, a.scale, w, ids);
     if (KIND == ROUTE_SOFTMAX && a.gate && lane == 0) a.gate[t] = 1.0f / (1.0f + expf(-z[i][a.E]));

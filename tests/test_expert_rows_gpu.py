@@ -116,6 +116,22 @@ def test_rows_that_go_to_the_library(cuda, name):
         assert torch.equal(j, k) and torch.allclose(u, v, rtol=2.0 ** -17, atol=0)
 
 
+@pytest.mark.parametrize("T", [5, 300])
+@pytest.mark.parametrize("E", [8, 16, 20, 64, 70])
+def test_sigmoid_choice_of_infinite_and_nan_logits(cuda, E, T):
+    """Whichever kernel forms the logits: -inf is the smallest of them, each its own choice with weight 0; NaN is none."""
+    torch.manual_seed(E + T)
+    x, r = torch.randint(1, 4, (T, 128)).bfloat16(), torch.randint(-2, 3, (E, 128)).bfloat16() / 32
+    r[2, 5] = r[5, 100] = r[E - 1, 0] = float("-inf")
+    w, i = mix.route_sigmoid_topk(x.to(cuda), r.to(cuda), E)
+    v, j = mix.route_sigmoid_topk(x, r, E)
+    assert torch.equal(i.cpu(), j) and torch.allclose(w.cpu(), v, rtol=2.0 ** -17, atol=0) and (w[:, -3:] == 0).all()
+    r[3, 7] = float("nan")
+    w, i = mix.route_sigmoid_topk(x.to(cuda), r.to(cuda), E - 1)
+    keep = j != 3
+    assert torch.equal(i.cpu(), j[keep].view(T, E - 1)) and torch.allclose(w.cpu(), v[keep].view(T, E - 1), rtol=2.0 ** -17, atol=0)
+
+
 @pytest.mark.parametrize("n,E", [(100, 4), (3000, 16)])
 def test_align_leaves_out_what_is_no_expert(cuda, n, E):
     torch.manual_seed(n)
