@@ -348,11 +348,13 @@ def moe_input_scaled(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: to
         from src import ops
 
         tiles = ops._moe_decode_tiles(h, w13.shape[1] // 2, t) if ops.native_available() else None
-        # The sorted form has the activation in its first product too, and so only the sort to lose. Few tokens of large experts whose gate's halves of
-        # weight rows are a multiple of 4 KiB long keep it: its tiles of 32 rows read such weights faster than the unsorted form's of 64 while both went through K
-        # in step (8 experts of 4096 x 4096, us, sorted / unsorted, 2 tokens 80 / 83, 8 tokens 140 / 160, 32 tokens 159 / 175). With places of K of their
-        # own they are within 7 %: 12 tokens 145 / 140, 24 tokens 150 / 141.
-        sort = tiles is not None and tiles[0][0] <= 32 and h >= 4096 and h % 2048 == 0 and w2.shape[2] >= 2048 and t <= 32 and n >= 4
+        # The sorted form has the activation in its first product too, and so only the sort to lose. Its tiles of 32 weight rows keep few tokens of experts
+        # of 2048 to 4095 columns at widths of 4096 and more, in 2048s (us, sorted / unsorted, 2, 4, 8 and 32 tokens: 8 experts of 4096 x 2048 46 65
+        # 81 87 / 44 69 84 92, 32 of them, four of a token's, 88 128 200 280 / 89 134 211 295, 8 of 8192 x 2048 81 112 143 152 / 81 118 142 151; 6144 x 2048
+        # would lose them, 68 92 110 124 / 63 92 103 116). From 4096 columns on the tiles of 64 are as fast or faster: 4096 x 4096 68 104 135 148 /
+        # 67 103 133 141, 8192 x 4096 133 194 255 269 / 130 188 251 264, 4096 x 8192 113 179 245 260 / 113 179 243 261, 4096 x 14336 178 299 413
+        # 450 / 182 306 419 452.
+        sort = tiles is not None and tiles[0][0] <= 32 and h >= 4096 and h % 2048 == 0 and 2048 <= w2.shape[2] < 4096 and t <= 32 and n >= 4
         if ops.native_available() and ids.dtype == torch.int32 and n > 0 and not sort and decode_tiles(w13, w2, t, n, MOE_SILU) is not None:
             xs = torch.empty(n, h, dtype=x.dtype, device=x.device)
             kern.gather_scaled(xs, x, None, w, k)

@@ -121,9 +121,9 @@ def test_rows_and_results_are_formed_once(cuda, monkeypatch, t, H, ff):
 
 
 @pytest.mark.parametrize("H,ff,t,form", [(4096, 2048, 1, "ids"), (4096, 2048, 2, "grouped"), (4096, 2048, 32, "grouped"), (4096, 2048, 33, "ids"),
-                                         (6144, 2048, 8, "grouped"), (4096, 1024, 8, "ids"), (2048, 2048, 32, "ids"), (5120, 2048, 8, "ids")])
+                                         (6144, 2048, 8, "grouped"), (4096, 1024, 8, "ids"), (2048, 2048, 32, "ids"), (5120, 2048, 8, "ids"), (4096, 4096, 2, "ids"), (4096, 4096, 32, "ids")])
 def test_scaled_mixtures_whose_sorted_form_is_faster_keep_it(cuda, monkeypatch, H, ff, t, form):
-    """Large gated experts with weight rows of a multiple of 4 KiB, 2 to 32 tokens: sorted rows, tiles of 32 weight rows."""
+    """Large gated experts with weight rows of a multiple of 4 KiB and fewer than 4096 columns, 2 to 32 tokens: sorted rows, tiles of 32 weight rows."""
     E, k, bf, ran = 3, 2, torch.bfloat16, []
     g = torch.Generator(device=cuda).manual_seed(H + t)
     x, w13, w2 = (torch.randn(*s, generator=g, device=cuda).to(bf) for s in ((t, H), (E, 2 * ff, H), (E, H, ff)))
