@@ -207,7 +207,7 @@ void conv_state_update(Tensor conv_state, Tensor x, int64_t heads, int64_t kv_he
 
 void gated_delta(Tensor out, Tensor qkv32, Tensor bg, Tensor gate, Tensor norm_w, double eps, Tensor state,
                  int64_t heads, int64_t kv_heads, int64_t dim, int64_t vdim, Tensor positions, OptTensor cu_q,
-                 Tensor state_slots, OptTensor z, OptTensor z_bias, OptTensor A_log, bool gate_sigmoid, double mult) {
+                 Tensor state_slots, OptTensor z, OptTensor z_bias, OptTensor A_log, bool gate_sigmoid, double mult, int64_t max_rows) {
   die::GatedDeltaArgs a;
   a.sh = delta_shape(heads, kv_heads, dim, vdim, 1);
   const int64_t C = a.sh.channels();
@@ -249,7 +249,8 @@ void gated_delta(Tensor out, Tensor qkv32, Tensor bg, Tensor gate, Tensor norm_w
   a.eps = (float)eps;
   a.mult = (float)mult;
   a.state = state.data_ptr<float>();
-  const die::RaggedRows rag = ragged(T, positions, cu_q, state_slots);
+  die::RaggedRows rag = ragged(T, positions, cu_q, state_slots);
+  rag.max_rows = (int)max_rows;
   const int64_t n = die::gated_delta_work(a, rag.total_rows, rag.num_seqs);
   const Tensor work = n > 0 ? at::empty({n}, qkv32.options()) : Tensor();
   a.work = n > 0 ? work.data_ptr<float>() : nullptr;
@@ -531,7 +532,9 @@ void register_seq_ops(pybind11::module& m) {
   m.def("poly_norm_act", &poly_norm_act);
   m.def("delta_prep", &delta_prep);
   m.def("conv_state_update", &conv_state_update);
-  m.def("gated_delta", &gated_delta);
+  m.def("gated_delta", &gated_delta, py::arg("out"), py::arg("qkv32"), py::arg("bg"), py::arg("gate"), py::arg("norm_w"), py::arg("eps"),
+        py::arg("state"), py::arg("heads"), py::arg("kv_heads"), py::arg("dim"), py::arg("vdim"), py::arg("positions"), py::arg("cu_q"),
+        py::arg("state_slots"), py::arg("z"), py::arg("z_bias"), py::arg("A_log"), py::arg("gate_sigmoid"), py::arg("mult"), py::arg("max_rows") = 0);
   m.def("qkv_prep", &qkv_prep);
   m.def("sink_attn", &sink_attn<false>);
   m.def("sink_attn_named", &sink_attn<true>);   // tests

@@ -679,13 +679,15 @@ template <int D, int V, bool CD> hipError_t launch_one(const GatedDeltaArgs& a, 
   constexpr size_t smem = Lds<D, V>::total;
   const auto fn = chunk_delta_kernel<D, V, CD>;
   // Where portions have a chunk on average, pairs are formed inside, two chunks ahead: the launch of its own, which longer portions gain from,
-  // takes longer than they do (16 tokens of 1 / 16 sequences, 16 heads of 128 x 128: 13.7 / 19.2 us with it, 11.4 / 15.5 without), and with one
-  // workgroup per compute unit two chunks do not pay for it either (16 x 22: 23.4 / 21.5). Nor do divided steps of narrow values, in which there
-  // may be nothing for either kernel. (128 x 256 leaves no LDS for it: 16 tokens 17.2 -> 18.0.)
+  // takes longer than they do (16 tokens of 1 / 16 / 64 sequences, 16 heads of 128 x 128: 12.5 / 19.4 / 59 us with it, 10.6 / 15.9 / 54 without; only
+  // many of 64 x 128 are faster with it, 128 of 16 tokens 68 / 73), and with one workgroup per compute unit two chunks do not pay for it either (16 x
+  // 22: 22.2 / 21.2). An average hides long portions, whose chain is up to twice as long with pairs inside (1000 tokens beside 63 rows of a token, 64 x
+  // 128, 191 / 314; before there were two forms 267): where the longest is known to have more than two chunks, the launch of its own is taken.
   constexpr size_t own = 4 * PairLds<D>::total, most = smem + own <= 160 * 1024 ? smem + own : smem;
   const int64_t wgs = (int64_t)a.sh.heads * r.num_seqs, cus = num_cus();
-  const bool few = r.total_rows <= (CT + 1) * r.num_seqs || (wgs <= cus && 2 * wgs > cus && r.total_rows <= 2 * CT * r.num_seqs);
-  const bool inside = most > smem && (few || (V == 64 && a.cut > 0));
+  const bool few = r.total_rows <= (CT + 1) * r.num_seqs ? D != 64 || V != 128 || wgs <= 2 * cus
+                                                         : wgs <= cus && 2 * wgs > cus && r.total_rows <= 2 * CT * r.num_seqs;
+  const bool inside = most > smem && few && r.max_rows <= 2 * CT;
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
   if (e != hipSuccess) return e;
   if (!inside)
@@ -711,12 +713,14 @@ void chunk_delta_cut(GatedDeltaArgs& a, int rows, int num_seqs) {
   a.cut = none;
   if (a.f32 || !near || (d != 64 && d != 128) || (v != 64 && v != 128 && v != 256)) return;
   const int64_t wgs = (int64_t)a.sh.heads * num_seqs, cus = num_cus();
-  const bool many = v < 256 && wgs > 2 * cus;
-  const int64_t from = v == 64 ? 64 : CT, all = !many ? from : v == 128 ? 21 : wgs > 4 * cus ? 160 : 96;
-  if (rows >= all * num_seqs || (v != 64 && rows >= CT * num_seqs && rows < (CT + 1) * num_seqs)) {
+  // rows of a sequence on average: up to 1, 2, 4 workgroups per compute unit, more
+  static constexpr int FROM[2][3][4] = {{{9, 9, 20, 24}, {9, CT, CT, CT}, {9, 9, 9, 9}}, {{9, 36, 56, 96}, {9, 14, CT, CT}, {9, 10, 10, 10}}};
+  const int64_t from = FROM[d / 128][v / 128][wgs <= cus ? 0 : wgs <= 2 * cus ? 1 : wgs <= 4 * cus ? 2 : 3];
+  const int64_t all = v == 128 && wgs > 2 * cus ? 21 : from;
+  if (rows >= all * num_seqs || (rows >= from * num_seqs && rows < (CT + 1) * num_seqs)) {
     a.cut = 0;
   } else if (rows >= from * num_seqs) {
-    a.cut = v == 64 ? (int)all : 28;
+    a.cut = 28;
     a.longest = (int)(rows * (int64_t)a.sh.heads / (2 * cus)) + 30;
   }
 }

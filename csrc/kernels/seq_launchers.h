@@ -22,6 +22,7 @@ struct RaggedRows {
   const int64_t* positions;   // [T]
   const int* state_slots;     // [S]
   int num_seqs, total_rows;
+  int max_rows = 0;           // of a sequence, 0: not known
 };
 
 // streams[t, s, :] (fp32, s < S) = embed[ids[t]] * scale + bigram[row(t)] for all s. row(t) = buckets at

@@ -780,7 +780,7 @@ class FekolornLM:
         if self.seq_state is None or getattr(meta, "state_slots", None) is None:
             raise RuntimeError("Fekolorn needs per-sequence state slots (LLMEngine provides them)")
         a, st, eps = self.arch, self.seq_state, self.arch.rms_eps
-        rag = seq.Ragged(positions, meta.cu_q if meta.is_prefill else None, meta.state_slots)
+        rag = seq.Ragged(positions, meta.cu_q if meta.is_prefill else None, meta.state_slots, meta.max_q_len if meta.is_prefill else 1)
         xs = seq.embed_hash(input_ids, self.embed, self.bigram, rag, st.prev_tok, a.embed_scale, a.bigram_buckets,
                             a.bigram_mul_prev, a.bigram_mul_cur, self.S)
         if self.bigram is not None:

@@ -588,7 +588,7 @@ class RerozenLM:
         if self.seq_state is None or getattr(meta, "state_slots", None) is None:
             raise RuntimeError("Rerozen needs per-sequence state slots (LLMEngine provides them)")
         a, st, eps, dt = self.arch, self.seq_state.layers, self.arch.rms_eps, self.dtype
-        rag = seq.Ragged(positions, meta.cu_q if meta.is_prefill else None, meta.state_slots)
+        rag = seq.Ragged(positions, meta.cu_q if meta.is_prefill else None, meta.state_slots, meta.max_q_len if meta.is_prefill else 1)
         max_q = meta.max_q_len if meta.is_prefill else 1
         x, _ = rec.embed_scaled(input_ids, self.embed, a.embed_scale, copy=False)
         y = spare = None

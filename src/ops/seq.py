@@ -37,6 +37,7 @@ class Ragged:
     positions: torch.Tensor            # [T] int64
     cu_q: Optional[torch.Tensor]       # [S + 1] int32 or None (one row per sequence)
     state_slots: torch.Tensor          # [S] int32
+    max_rows: int = 0                  # rows of the longest sequence (0: not known), for the choice between kernels only
 
     def spans(self, rows: int) -> List[Tuple[int, int, int]]:
         """(first row, rows, slot) per sequence — host-side, CPU path only."""
@@ -215,7 +216,7 @@ def gated_delta(qkv32: torch.Tensor, bg: torch.Tensor, gate: torch.Tensor, norm_
         out = torch.empty(T, heads * vdim, dtype=gate.dtype, device=gate.device)
     if gate.is_cuda:
         _kern().gated_delta(out, qkv32, bg, gate, norm_w, eps, state, heads, kv_heads, dim, vdim, rag.positions,
-                            rag.cu_q, rag.state_slots, z, z_bias, A_log, bool(gate_sigmoid), float(mult))
+                            rag.cu_q, rag.state_slots, z, z_bias, A_log, bool(gate_sigmoid), float(mult), rag.max_rows)
         return out
     G, rep = kv_heads, heads // kv_heads
     q = qkv32[:, : G * dim].view(T, G, dim).repeat_interleave(rep, 1)
