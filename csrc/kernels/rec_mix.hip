@@ -875,12 +875,24 @@ hipError_t launch_conv_tail_update(float* conv_state, const void* x, int64_t xst
   return hipGetLastError();
 }
 
+// 9 - 16 states: whether a channel goes to one lane (rows of tokens formed by every lane for itself) and not to 4 or 16 that share what depends on
+// the token (selective_scan.hip). The shared form costs a wave more instructions beside its states' own and is faster while waves are few; so many waves of
+// one lane per channel on each SIMD are enough for the other, by the rows of a portion on average: below 17 reading and writing the states counts most, and 4
+// lanes load padding with 9 - 12 of them. us, shared / one lane: 128 sequences of 2 rows, 8192 channels of 12 states 47 / 32, of 16 47 / 53; of 5
+// rows of 9 55 / 43; 64 x 40 of 8192 of 16 110 / 97; 128 x 40 of 4096 of 12 107 / 90. Over 2736 steps of 2 - 400 rows and 1.5 - 24 waves it is 0.5 % from the
+// better form in the mean.
+static bool scan_on_one_lane(const SelectiveScanArgs& a, const RaggedRows& r) {
+  static constexpr int BRIEF[8] = {4, 8, 16, 3, 64, 64, 64, 64}, MIDDLE[8] = {7, 7, 7, 7, 12, 12, 12, 7}, LONG[8] = {7, 7, 7, 7, 8, 8, 8, 7};
+  const int64_t waves = (int64_t)a.I * r.num_seqs / 64, simds = 4 * (int64_t)num_cus(), n = r.num_seqs;
+  return r.cu_q != nullptr && waves >= (r.total_rows < 17 * n ? BRIEF : r.total_rows < 32 * n ? MIDDLE : LONG)[a.N - 9] * simds;
+}
+
 hipError_t launch_selective_scan(const SelectiveScanArgs& a, RaggedRows r, hipStream_t s) {
   if (r.num_seqs == 0 || r.total_rows == 0) return hipSuccess;
   if (!rows_ok(r) || a.I < 1 || a.N < 1 || a.N > 256) return hipErrorInvalidValue;
   if (a.N <= 4) return launch_scan_one<4, 1>(a, r, s);
   if (a.N <= 8) return launch_scan_one<8, 1>(a, r, s);
-  if (a.N <= 16) return launch_scan_lanes(a, r, s);
+  if (a.N <= 16) return scan_on_one_lane(a, r) ? launch_scan_one<16, 1>(a, r, s) : launch_scan_lanes(a, r, s);
   if (a.N <= 32) return launch_scan_one<16, 2>(a, r, s);
   if (a.N <= 64) return launch_scan_one<16, 4>(a, r, s);
   if (a.N <= 128) return launch_scan_one<32, 4>(a, r, s);

@@ -1,5 +1,5 @@
-"""The selective scan of 9 - 16 states per channel over several trips of 16 tokens (4 and 16 lanes per channel) and one row per sequence,
-with rows inside wider tensors, against float64.
+"""The selective scan of 9 - 16 states per channel over several trips of 16 tokens (4 and 16 lanes per channel; one, where waves of channels fill the SIMDs)
+and one row per sequence, with rows inside wider tensors, against float64.
 
 bf16 steps use the hardware's exponential and reciprocal (a few 2^-22) and round the result once (2^-9 of it); fp32 steps are
 within some 2^-20 of the sums' terms, 1e-5 of the result's root mean square."""
@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
-@pytest.mark.parametrize("lens,I,N", [([16, 1, 50, 33], 70, 16), ([32, 15, 64], 8500, 16), ([17, 48], 4096, 11), ([47], 40, 9), ([1] * 5, 1030, 16), ([1] * 3, 65, 10)])
+@pytest.mark.parametrize("lens,I,N", [([16, 1, 50, 33], 70, 16), ([32, 15, 64], 8500, 16), ([17, 48], 4096, 11), ([47], 40, 9), ([1] * 5, 1030, 16), ([1] * 3, 65, 10),
+                                      ([3, 20, 1, 17] * 6, 8500, 12), ([21, 20, 33] * 16, 8500, 16), ([2] * 32, 8500, 9)])
 def test_trips_and_steps(cuda, lens, I, N, dt):
     g = torch.Generator().manual_seed(I + N)
     S, T = len(lens), sum(lens)
