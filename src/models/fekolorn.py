@@ -154,6 +154,12 @@ class ParallelSpec:
                 "right_scale": self.right_scale}
 
 
+def delta_scratch_bytes(mixer: Any, tokens: int) -> int:
+    """What a layer's delta rule allocates in a step of ``tokens`` rows besides its results (0 without one)."""
+    m = getattr(mixer, "right", mixer)
+    return seq.gated_delta_work_bytes(tokens, m.heads) if isinstance(m, GatedDeltaSpec) else 0
+
+
 @dataclass(frozen=True)
 class PolyMlpSpec:
     ff: int
@@ -769,7 +775,8 @@ class FekolornLM:
             if l.mlp is not None:
                 w = max(w, 3 * l.mlp.ff)
             widest = max(widest, w)
-        return tokens * (4 * self.S * a.hidden_size + 8 * a.hidden_size + 4 * widest) + (1 << 30)
+        scratch = max((delta_scratch_bytes(l.mixer, tokens) for l in a.layers), default=0)
+        return tokens * (4 * self.S * a.hidden_size + 8 * a.hidden_size + 4 * widest) + scratch + (1 << 30)
 
     # ----------------------------------------------------------------- forward
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor, meta, kv_pool,

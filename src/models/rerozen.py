@@ -37,7 +37,7 @@ from typing import Any, Dict, List, Optional, Tuple
 import torch
 
 from src.models.datatar import MIXERS, LayerRowPool
-from src.models.fekolorn import GatedDeltaSpec, SeqStatePool, SinkAttentionMixer, SinkAttnSpec
+from src.models.fekolorn import GatedDeltaSpec, SeqStatePool, SinkAttentionMixer, SinkAttnSpec, delta_scratch_bytes
 from src.ops import conv, mix, rec, seq
 from src.parallel.tp import TPContext
 
@@ -577,7 +577,8 @@ class RerozenLM:
         for l, lw in zip(a.layers, self.layers):
             m = lw.mix
             widest = max(widest, 4 * (m.w_in.shape[0] + m.w_low.shape[0] + m.w_o.shape[1]), 3 * l.ff)
-        return tokens * (14 * a.hidden_size + 4 * widest) + (1 << 30)
+        scratch = max((delta_scratch_bytes(l.mixer, tokens) for l in a.layers), default=0)
+        return tokens * (14 * a.hidden_size + 4 * widest) + scratch + (1 << 30)
 
     # ----------------------------------------------------------------- forward
     def forward(self, input_ids: torch.Tensor, positions: torch.Tensor, meta, kv_pool,

@@ -202,6 +202,12 @@ def conv_state_update(conv_state: torch.Tensor, x: torch.Tensor, heads: int, kv_
         conv_state[slot] = torch.cat([old, x[q0:q0 + n].float()], 0)[-k:]
 
 
+def gated_delta_work_bytes(tokens: int, heads: int) -> int:
+    """The most scratch that :func:`gated_delta` allocates for a step of ``tokens`` rows: 3 KiB per head and chunk of 16 rows, a last part of
+    one with every sequence. Steps of fewer than 9 rows per sequence have no chunks."""
+    return 3072 * heads * (tokens // 16 + tokens // 9)
+
+
 def gated_delta(qkv32: torch.Tensor, bg: torch.Tensor, gate: torch.Tensor, norm_w: torch.Tensor, eps: float,
                 state: torch.Tensor, heads: int, kv_heads: int, dim: int, vdim: int, rag: Ragged,
                 z: Optional[torch.Tensor] = None, z_bias: Optional[torch.Tensor] = None,
