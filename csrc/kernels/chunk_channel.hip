@@ -15,8 +15,8 @@
 // Bound by instruction issue of a consuming and a helping wave per SIMD. 16 heads of 64 x 128 (us, token by token / in chunks): 16 x 1024 tokens 372 / 140, one
 // sequence of 1024 319 / 132, 32 x 300 ragged 151 / 82, 1 x 64 of 32 heads 24 / 13. Distance from 64 bits 0.86 - 0.95 of that token by token.
 //
-// An infinite key, value or state makes the rows from its token on and the state NaN, where token by token some of them may stay infinite;
-// earlier rows and other sequences are as they are.
+// The parts of an infinity are NaN. A wave that finds results or state of its columns not finite goes through the portion once more, token by
+// token from the state as it was, and puts what that gives in the place of what is not finite: infinities stay what they are.
 #include "chunk_channel.h"
 #include "chunk_parts.h"
 #include "lane_reduce.h"
@@ -54,7 +54,7 @@ template <int D> struct Rows {
       z[t] = *at_bytes<uint32_at2>(zb + row0 * zstride, 2 * (row * (uint32_t)zstride + d2));
     }
   }
-  __device__ __forceinline__ float decay(float x) const {   // exp(-softplus(-x) / tau), softplus_of<true> with its logarithm ahead of the choice
+  static __device__ __forceinline__ float decay(float x, float inv_tau) {   // exp(-softplus(-x) / tau), softplus_of<true> with its logarithm ahead of the choice
     const float e = exp_of<true>(-fabsf(x));
     float l = 0.6931471805599453f * __builtin_amdgcn_logf(1.0f + e);
     asm volatile("" : "+v"(l));
@@ -68,7 +68,7 @@ template <int D> struct Rows {
     for (int t = 0; t < 4; ++t) {
       const bool in = t0 + t <= last;
       asm volatile("" : "+v"(k[t]), "+v"(q[t]), "+v"(z[t]));   // (converted here, not where they are loaded and would be waited for)
-      float gx = decay(__uint_as_float(z[t] << 16) + bias0), gy = decay(__uint_as_float(z[t] & 0xffff0000u) + bias1);
+      float gx = decay(__uint_as_float(z[t] << 16) + bias0, inv_tau), gy = decay(__uint_as_float(z[t] & 0xffff0000u) + bias1, inv_tau);
       asm volatile("" : "+v"(gx), "+v"(gy));
       const uint32_t kw = in ? k[t] : 0u, qw = in ? q[t] : 0u;
       ko[t] = make_float2(__uint_as_float(kw << 16), __uint_as_float(kw & 0xffff0000u));
@@ -77,6 +77,37 @@ template <int D> struct Rows {
     }
   }
 };
+
+__device__ __forceinline__ bool finite(float x) { return fabsf(x) < INFINITY; }
+
+// A wave's 32 columns of a portion token by token, S [D, 32] (LDS) their state; a lane has one column and half of the channels. o: row 0's
+// results, state: what the chunks left, both replaced where they are not finite. (Loops that are not unrolled: a rare way is not to cost the
+// kernel registers.)
+template <int D, int V>
+__device__ __forceinline__ void token_by_token(const GatedLinearArgs& a, int q0, int L, int h, float* S, float* o, float* state) {
+  const int lane = threadIdx.x & 63, half = lane >> 5, v0 = (threadIdx.x >> 6) * 32 + (lane & 31);
+  const bf16_t* x = reinterpret_cast<const bf16_t*>(a.x) + (int64_t)q0 * a.xstride;
+  const bf16_t* z = reinterpret_cast<const bf16_t*>(a.z) + (int64_t)q0 * a.zstride + h * D;
+  const int g = h / (a.heads / a.groups) * D;
+  float* const own = S + (lane & 31);
+#pragma unroll 1
+  for (int t = 0; t < L; ++t, x += a.xstride, z += a.zstride) {
+    const float v = bf2f(x[a.voff + h * V + v0]);
+    float y = 0.f;
+#pragma unroll 1
+    for (int d = half * (D / 2); d < (half + 1) * (D / 2); ++d) {
+      const float s = fmaf(own[32 * d], Rows<D>::decay(bf2f(z[d]) + a.z_bias[h * D + d], a.inv_tau), bf2f(x[a.koff + g + d]) * v);
+      own[32 * d] = s;
+      y = fmaf(s, bf2f(x[a.qoff + g + d]), y);
+    }
+    y = xor32_sum(y) * a.qscale;
+    float* const at = o + (int64_t)t * a.heads * V + v0;
+    if (half == 0 && !finite(*at)) *at = y;
+  }
+#pragma unroll 1
+  for (int d = half * (D / 2); d < (half + 1) * (D / 2); ++d)
+    if (!finite(state[d * V + v0])) state[d * V + v0] = own[32 * d];
+}
 
 // LDS of a workgroup, in bytes
 template <int D> struct Lds {
@@ -272,6 +303,7 @@ __global__ void __launch_bounds__(2 * V + 4 * D, 1) chunk_channel_kernel(GatedLi
         const float y = st[so + (16 * t + e) * V + 16 * c];
         S[t][c][e] = fresh ? 0.f : y;   // (a new sequence reads its slot but not its content)
       }
+  float odd_sum = 0.f;   // 0 as long as all results are finite
   __syncthreads();
   __syncthreads();
   for (int n = 0; n < nch; ++n) {
@@ -363,6 +395,7 @@ __global__ void __launch_bounds__(2 * V + 4 * D, 1) chunk_channel_kernel(GatedLi
       for (int e = 0; e < 4; ++e) {
         o[c][e] = (qs[c][e] + ql[c][e]) * a.qscale;
         if (odd) o[c][e] = 4 * lg + e >= first[c] ? __builtin_nanf("") : o[c][e];
+        odd_sum = fmaf(o[c][e], 0.f, odd_sum);
       }
     if (whole) {
 #pragma unroll
@@ -415,11 +448,28 @@ __global__ void __launch_bounds__(2 * V + 4 * D, 1) chunk_channel_kernel(GatedLi
 #pragma unroll
     for (int c = 0; c < NB; ++c)
 #pragma unroll
+      for (int e = 0; e < 4; ++e) odd_sum = fmaf(S[t][c][e], 0.f, odd_sum);
+  const bool again = __ballot(odd_sum != 0.f) != 0;
+  float* const was = reinterpret_cast<float*>(sm) + wave * (D * 16 * NB);   // the state's columns as they were (nothing else is in LDS any more)
+  if (again) {
+#pragma unroll 1
+    for (int i = lane; i < D * 16 * NB; i += 64) was[i] = fresh ? 0.f : st[i / (16 * NB) * V + 16 * NB * wave + i % (16 * NB)];
+    __threadfence();
+  }
+#pragma unroll
+  for (int t = 0; t < ND; ++t)
+#pragma unroll
+    for (int c = 0; c < NB; ++c)
+#pragma unroll
       for (int e = 0; e < 4; ++e) st[so + (16 * t + e) * V + 16 * c] = S[t][c][e];
+  if (again) {
+    __threadfence();
+    token_by_token<D, V>(a, q0, L, h, was, a.out + ((int64_t)q0 * H + h) * V, st);
+  }
 }
 
 template <int D, int V> hipError_t launch_one(const GatedLinearArgs& a, RaggedRows r, hipStream_t s) {
-  constexpr size_t smem = Lds<D>::total;
+  constexpr size_t smem = Lds<D>::total > 4 * D * V ? Lds<D>::total : 4 * D * V;   // (the chunks', then the whole state where it is gone through again)
   static_assert(smem <= 160 * 1024, "LDS of a compute unit");
   const auto fn = chunk_channel_kernel<D, V>;
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);

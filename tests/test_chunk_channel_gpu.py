@@ -79,3 +79,39 @@ def test_later_tokens_do_not_reach_earlier_rows(cuda, what):
     assert not torch.isfinite(got[at:80, 5]).any()
     slot = int(args[4][1])
     assert torch.equal(st[[i for i in range(4) if i != slot]], ws[[i for i in range(4) if i != slot]]) and not torch.isfinite(st[slot, 0, :, 5]).all()
+
+
+@pytest.mark.parametrize("what", ["k", "q", "v", "state", "both", "nan", "overflow"])
+@pytest.mark.parametrize("H,G,D,V,pad", [(2, 2, 64, 128, 0), (3, 1, 64, 64, 1), (2, 1, 64, 256, 0), (2, 1, 128, 128, 3), (2, 2, 128, 64, 0)])
+def test_infinities_are_what_they_are_token_by_token(cuda, H, G, D, V, pad, what):
+    """Rows and states are infinite, of the right sign, or NaN exactly where the recurrence itself makes them so; all others are as near as ever."""
+    torch.manual_seed(D + V)
+    args = _inputs([40, 33, 41], [3, 0, 7], H, G, D, V, pad)
+    x, z, _, state, slots, _, _ = args
+    k0, v0 = G * D, 2 * G * D
+    if what in ("k", "both"):
+        x[50, k0 + 5] = float("inf")
+    if what == "q":
+        x[47, 3] = float("-inf")
+        x[60, D - 1] = float("inf")
+    if what in ("v", "both"):
+        x[90, v0 + V // 2 + 1] = float("-inf")
+    if what == "state":
+        state[slots[0], 0, 7, 9], state[slots[1], H - 1, 1, 2] = float("inf"), float("nan")   # (the second sequence is new: its slot is not read)
+    if what == "nan":
+        x[70, k0] = float("nan")
+        z[100, 1] = float("nan")
+    if what == "overflow":
+        state[slots[0], H - 1, :, 40] = 3e38
+        z[:40], x[:40, : k0] = 5.0, 4.0
+    want, ws = _exact(args, H, G, D, V)
+    want, ws = (torch.where(t.abs() > 3.4028235e38, t.sign() * float("inf"), t) for t in (want, ws))
+    got, st = _run(cuda, args, H, G, D, V)
+    if what == "state":
+        assert torch.isnan(st[slots[1]]).sum() == 0
+    assert not torch.isfinite(want).all()
+    for g, w in ((got.double(), want), (st[slots.long()].double(), ws[slots.long()])):
+        assert torch.equal(torch.isnan(g), torch.isnan(w)) and torch.equal(torch.isposinf(g), torch.isposinf(w)) and torch.equal(torch.isneginf(g), torch.isneginf(w))
+        keep = torch.isfinite(w)
+        small = keep & (w.abs() < 1e30)
+        assert (g[small] - w[small]).abs().max() <= 1e-5 * w[small].abs().max() + 1e-5 * w[small].square().mean().sqrt()
