@@ -481,36 +481,37 @@ std::string latent_attn(Tensor out, Tensor q_lat, Tensor q, int64_t rot_off, Ten
   a.chunk = 0;
   Tensor ws_o, ws_ml;
   if (die::latent_attn_uses_mfma(a)) {
-    // few row tiles (decode steps): split the keys over workgroups until about 256 are in flight. The key range
-    // is bounded by the window, else by the block table's width (a prompt step's: its longest context; under a captured graph: the model length;
-    // splits beyond a sequence's keys exit at once)
-    const int64_t rows_wg = max_q * H <= 32 ? 32 : 128;
-    const int64_t tiles = S * ((max_q * H + rows_wg - 1) / rows_wg);
+    // the key range is bounded by the window, else by the block table's width (a prompt step's: its longest context; under a captured graph: the
+    // model length; splits beyond a sequence's keys exit at once)
+    const int64_t cus = at::cuda::getCurrentDeviceProperties()->multiProcessorCount;
     int64_t bound = block_tables.size(1) * cache.size(1);
     if (window > 0) bound = std::min<int64_t>(bound, window + max_q);
-    int64_t ns = std::min<int64_t>({(int64_t)16, 512 / std::max<int64_t>(1, tiles), (bound + 63) / 64});
     if (die::latent_attn_decodes(a)) {
       // one workgroup per compute unit: twice as many write twice the partial results (32 sequences of 750 - 1500 keys, 16 heads 12.2 + 4.7 us, 14.3 + 5.9)
-      ns = std::min<int64_t>({(int64_t)16, at::cuda::getCurrentDeviceProperties()->multiProcessorCount / std::max<int64_t>(1, S * ((H + 15) / 16)), (bound + 127) / 128});
-    } else if (ns > 1 && a.impl == 0 && die::latent_attn_fits_rows(a)) {
-      const int64_t seen = window > 0 ? std::min<int64_t>(bound, window + (H + 63) / H + 31) : bound;   // of a tile of 64 rows
-      const int64_t most = ns;
-      // (times fitted to 524 random steps of rank 256 + 32 in 1 to 16 splits)
-      ns = best_splits({0.9, 1.16, 2.2, 13.9, 3.25, 1.3}, most, bound, seen, S * ((max_q * H + 63) / 64), tiles,
-                       at::cuda::getCurrentDeviceProperties()->multiProcessorCount, T * H * rank * 4);
-      a.fine = ns < most;   // (a split rounds relative to its own largest weight)
-    }
-    if (ns > 1) {
-      a.chunk = (int)((((bound + ns - 1) / ns) + 31) / 32 * 32);
-      a.nsplit = die::latent_attn_decodes(a) ? (int)ns : (int)((bound + a.chunk - 1) / a.chunk);
-      if (a.nsplit > 1) {
-        ws_o = at::empty({a.nsplit, H * T, rank}, q_lat.options().dtype(at::kFloat));
-        ws_ml = at::empty({a.nsplit, H * T, 2}, q_lat.options().dtype(at::kFloat));
-        a.ws_o = ws_o.data_ptr<float>();
-        a.ws_ml = ws_ml.data_ptr<float>();
-      } else {
-        a.nsplit = 1;
+      const int64_t ns = std::min<int64_t>({(int64_t)16, cus / std::max<int64_t>(1, S * ((H + 15) / 16)), (bound + 127) / 128});
+      a.nsplit = (int)std::max<int64_t>(1, ns);
+    } else {
+      // few row tiles: until about 512 workgroups are in flight, or less where that is estimated to be faster
+      const int64_t rows_wg = max_q * H <= 32 ? 32 : 128;
+      const int64_t tiles = S * ((max_q * H + rows_wg - 1) / rows_wg);
+      int64_t ns = std::min<int64_t>({(int64_t)16, 512 / std::max<int64_t>(1, tiles), (bound + 63) / 64});
+      if (ns > 1 && a.impl == 0 && die::latent_attn_fits_rows(a)) {
+        const int64_t seen = window > 0 ? std::min<int64_t>(bound, window + (H + 63) / H + 31) : bound;   // of a tile of 64 rows
+        const int64_t most = ns;
+        // (times fitted to 524 random steps of rank 256 + 32 in 1 to 16 splits)
+        ns = best_splits({0.9, 1.16, 2.2, 13.9, 3.25, 1.3}, most, bound, seen, S * ((max_q * H + 63) / 64), tiles, cus, T * H * rank * 4);
+        a.fine = ns < most;   // (a split rounds relative to its own largest weight)
       }
+      if (ns > 1) {
+        a.chunk = (int)((((bound + ns - 1) / ns) + 31) / 32 * 32);
+        a.nsplit = (int)((bound + a.chunk - 1) / a.chunk);
+      }
+    }
+    if (a.nsplit > 1) {
+      ws_o = at::empty({a.nsplit, H * T, rank}, q_lat.options().dtype(at::kFloat));
+      ws_ml = at::empty({a.nsplit, H * T, 2}, q_lat.options().dtype(at::kFloat));
+      a.ws_o = ws_o.data_ptr<float>();
+      a.ws_ml = ws_ml.data_ptr<float>();
     }
   }
   HIP_OK(die::launch_latent_attn(a, cur_stream()));

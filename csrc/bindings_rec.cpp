@@ -5,6 +5,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 
+#include "kernels/chunk_channel.h"
 #include "kernels/rec_launchers.h"
 
 using at::Tensor;
@@ -191,7 +192,8 @@ void exp_gate_scan(Tensor abe, Tensor x, int64_t ioff, int64_t foff, Tensor i_bi
                                    ragged(T, positions, cu_q, state_slots), cur_stream()));
 }
 
-void gated_linear_attn(Tensor out, OptTensor nq, Tensor x, int64_t qoff, int64_t koff, int64_t voff, OptTensor ab,
+// returns whether the step went through the chunks of decays per channel
+bool gated_linear_attn(Tensor out, OptTensor nq, Tensor x, int64_t qoff, int64_t koff, int64_t voff, OptTensor ab,
                        Tensor state, OptTensor n_state, int64_t heads, int64_t groups, int64_t dim, int64_t vdim,
                        double qscale, Tensor positions, OptTensor cu_q, Tensor state_slots, OptTensor z,
                        OptTensor z_bias, double inv_tau) {
@@ -253,7 +255,9 @@ void gated_linear_attn(Tensor out, OptTensor nq, Tensor x, int64_t qoff, int64_t
   a.dim = (int)dim;
   a.vdim = (int)vdim;
   a.qscale = (float)qscale;
-  HIP_OK(die::launch_gated_linear_attn(a, ragged(T, positions, cu_q, state_slots), cur_stream()));
+  const die::RaggedRows rag = ragged(T, positions, cu_q, state_slots);
+  HIP_OK(die::launch_gated_linear_attn(a, rag, cur_stream()));
+  return die::chunk_channel_fits(a, rag.total_rows, rag.num_seqs);
 }
 
 void head_norm_gate(Tensor out, Tensor o, OptTensor nq, OptTensor abe, Tensor g, Tensor w, int64_t heads, int64_t vdim,

@@ -442,23 +442,21 @@ const char* sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, O
   int64_t bound = block_tables.size(1) * cache.size(1);
   if (window > 0) bound = std::min<int64_t>(bound, window + max_q);
   if (seg > 0) bound = std::min<int64_t>(bound, seg + max_q);
-  int64_t ns = 1;
   if (die::sink_attn_uses_decode(a)) {
     // decode steps: a workgroup per (sequence, key/value head, split), which take trips of 128 keys in turn. Two workgroups per compute unit hold
     // enough loads in flight; more splits write and merge more partial results (32 sequences of 1000 - 2000 keys, 4 groups of 128 + 128: 16
     // splits 32.0 us, 4 27.6; 64 of 8 groups 42, one split and no merge 33). A little more than one or two workgroups per compute unit would leave
     // most of them waiting for a few: those are cut finer (40 sequences of 8 groups in 1 / 2 / 5 splits 50.2 / 52.3 / 47.7, 68 in 1 / 3 54.7 / 50.8).
     const int64_t wgs = std::max<int64_t>(1, S * kv_heads), cus = at::cuda::getCurrentDeviceProperties()->multiProcessorCount;
-    ns = wgs > cus && 3 * wgs <= 4 * cus ? 5 : wgs > 2 * cus && 3 * wgs <= 7 * cus ? 3 : std::max<int64_t>(1, 2 * cus / wgs);
-    ns = std::min<int64_t>({(int64_t)128, ns, (bound + 127) / 128});
-    a.nsplit = (int)ns;
+    int64_t ns = wgs > cus && 3 * wgs <= 4 * cus ? 5 : wgs > 2 * cus && 3 * wgs <= 7 * cus ? 3 : std::max<int64_t>(1, 2 * cus / wgs);
+    a.nsplit = (int)std::max<int64_t>(1, std::min<int64_t>({(int64_t)128, ns, (bound + 127) / 128}));
   } else if (die::sink_attn_uses_mfma(a)) {
     // few row tiles: split the keys over workgroups until about 2048 are in flight, or less where that is estimated to be faster (a gate
     // is applied to the merged fp32 rows, without splits to rounded ones: such steps keep their splits)
     const int64_t qpg = heads / kv_heads, rows = max_q * qpg;
     const int64_t rows_wg = rows <= 32 ? 32 : 128;
     const int64_t tiles = S * kv_heads * ((rows + rows_wg - 1) / rows_wg);
-    ns = std::min<int64_t>({(int64_t)16, 2048 / std::max<int64_t>(1, tiles), (bound + 63) / 64});
+    int64_t ns = std::min<int64_t>({(int64_t)16, 2048 / std::max<int64_t>(1, tiles), (bound + 63) / 64});
     if (ns > 1 && a.impl == 0 && !gate.has_value() && die::sink_attn_fits_rows(a)) {
       const bool broad = vdim > 128, shaped = a.softcap > 0.f || a.slopes != nullptr || a.bias != nullptr;
       // (fitted to the times of 1978 random steps, six kinds of scores, in 1 to 16 splits)
@@ -472,18 +470,16 @@ const char* sink_attn(Tensor out, Tensor q, Tensor cache, Tensor block_tables, O
                        T * heads * vdim * 4);
       a.fine = ns < most;   // (a split rounds relative to its own largest weight: fewer of them were up to 5 % further from 64 bits)
     }
-    if (ns > 1) a.chunk = (int)((((bound + ns - 1) / ns) + 31) / 32 * 32);
-  }
-  if (ns > 1) {
-    if (a.chunk > 0) a.nsplit = (int)((bound + a.chunk - 1) / a.chunk);
-    if (a.nsplit > 1) {
-      ws_o = at::empty({a.nsplit, T * heads, vdim}, q.options().dtype(at::kFloat));
-      ws_ml = at::empty({a.nsplit, T * heads, 2}, q.options().dtype(at::kFloat));
-      a.ws_o = ws_o.data_ptr<float>();
-      a.ws_ml = ws_ml.data_ptr<float>();
-    } else {
-      a.nsplit = 1;
+    if (ns > 1) {
+      a.chunk = (int)((((bound + ns - 1) / ns) + 31) / 32 * 32);
+      a.nsplit = (int)((bound + a.chunk - 1) / a.chunk);
     }
+  }
+  if (a.nsplit > 1) {
+    ws_o = at::empty({a.nsplit, T * heads, vdim}, q.options().dtype(at::kFloat));
+    ws_ml = at::empty({a.nsplit, T * heads, 2}, q.options().dtype(at::kFloat));
+    a.ws_o = ws_o.data_ptr<float>();
+    a.ws_ml = ws_ml.data_ptr<float>();
   }
   a.gate = nullptr;
   a.gstride = 0;

@@ -114,9 +114,10 @@ struct LatentAttnArgs {
   float scale;
   LatentShape sh;
   bool f32;
-  // split keys (matrix-core kernel only): nsplit > 1 workgroups per row tile take `chunk` keys each and write
-  // unnormalised partial sums to ws_o [nsplit, H * T, rank] and (running max in log2 units, sum) to
-  // ws_ml [nsplit, H * T, 2]; a merge kernel then writes `out`
+  // split keys (matrix cores only): nsplit > 1 workgroups per row tile share its keys and write unnormalised partial sums to
+  // ws_o [nsplit, H * T, rank] and (running max in log2 units, sum) to ws_ml [nsplit, H * T, 2]; a merge kernel then writes
+  // `out`. Decode steps (latent_attn_decodes) deal tiles of keys out in turn, to any nsplit >= 1, and do not read `chunk`; in
+  // the other kernels a workgroup takes `chunk` neighbouring keys and nsplit * chunk covers them all
   float* ws_o;
   float* ws_ml;
   int nsplit, chunk;

@@ -162,9 +162,10 @@ struct SinkAttnArgs {
   bool f32;
   int impl;               // 0: the decode-step kernel or matrix cores where they apply, else FMA; 1: FMA;
                           // 2: matrix cores or fail
-  // split keys (matrix-core kernel only): nsplit > 1 workgroups per row tile take `chunk` keys each and write
-  // unnormalised partial sums to ws_o [nsplit, T * H, vdim] and (running max in log2 units, sum) to
-  // ws_ml [nsplit, T * H, 2]; a merge kernel then writes `out`
+  // split keys (decode steps and matrix cores): nsplit > 1 workgroups per row tile share its keys and write unnormalised partial
+  // sums to ws_o [nsplit, T * H, vdim] and (running max in log2 units, sum) to ws_ml [nsplit, T * H, 2]; a merge kernel then
+  // writes `out`. The decode-step kernel (sink_attn_uses_decode) deals trips of 128 keys out in turn, to any nsplit >= 1, and
+  // does not read `chunk`; in the others a workgroup takes `chunk` neighbouring keys and nsplit * chunk covers them all
   float* ws_o;
   float* ws_ml;
   int nsplit, chunk;

@@ -2,7 +2,8 @@
 
 Both sides hold the same bf16 inputs. The kernel's decays come from the hardware's exponential and logarithm, some 2^-22 of an exponent of
 at most 1 per token; over a few hundred tokens a state's terms are off by 1e-5 of their size at most, and results by as much of their root
-mean square. A dropped or doubled token moves them by 1e-2 and more."""
+mean square. Over L tokens the roundings of the decays themselves and of the state, 2^-24 of a term each, add up to L 2^-24 at most. A dropped
+or doubled token moves them by 1e-2 and more."""
 
 import pytest
 import torch
@@ -21,6 +22,24 @@ def _inputs(lens, past, H, G, D, V, pad=0):
     state, slots = torch.randn(S + 1, H, D, V) * 0.3, torch.randperm(S + 1)[:S].int()
     pos = torch.cat([torch.arange(n) + p for n, p in zip(lens, past)])
     return x, z, zb, state, slots, pos, torch.tensor([0] + lens).cumsum(0).int()
+
+
+class _Recorded:
+    """The kernels, with what gated_linear_attn says of the way it took."""
+
+    def __init__(self, kern, said):
+        self.kern, self.said = kern, said
+
+    def __getattr__(self, name):
+        f = getattr(self.kern, name)
+        return (lambda *a: self.said.append(f(*a))) if name == "gated_linear_attn" else f
+
+
+@pytest.fixture
+def said(monkeypatch):
+    out, kern = [], rec._kern
+    monkeypatch.setattr(rec, "_kern", lambda: _Recorded(kern(), out))
+    return out
 
 
 def _run(cuda, args, H, G, D, V, scale=0.3, tau=16.0):
@@ -50,18 +69,21 @@ def _exact(args, H, G, D, V, scale=0.3, tau=16.0):
 
 
 @pytest.mark.parametrize("H,G,D,V,pad", [(4, 4, 64, 128, 0), (3, 1, 64, 64, 1), (2, 2, 64, 256, 3), (2, 1, 128, 128, 0), (4, 2, 128, 64, 1)])
-@pytest.mark.parametrize("lens,past", [([16], [0]), ([17, 1, 64, 33], [0, 4, 9, 0]), ([48, 15, 130], [2, 0, 0])])
-def test_portions(cuda, H, G, D, V, pad, lens, past):
+@pytest.mark.parametrize("lens,past", [([17], [0]), ([17, 1, 64, 33], [0, 4, 9, 0]), ([48, 15, 130], [2, 0, 0]), ([16], [0]), ([1000, 3], [0, 5])])
+def test_portions(cuda, said, H, G, D, V, pad, lens, past):
+    """(An average of 16 rows of 64 x 64 goes token by token.)"""
     torch.manual_seed(sum(lens) + D + V)
     args = _inputs(lens, past, H, G, D, V, pad)
     want, ws = _exact(args, H, G, D, V)
     got, st = _run(cuda, args, H, G, D, V)
-    assert (got.double() - want).abs().max() <= 1e-5 * want.square().mean().sqrt() + 1e-5 * want.abs().max()
-    assert (st.double() - ws).abs().max() <= 1e-5 * ws.abs().max()
+    assert said == [lens != [16] or (D, V) != (64, 64)]
+    tol = 1e-5 if max(lens) < 160 else 1e-5 + max(lens) * 2.0 ** -24
+    assert (got.double() - want).abs().max() <= tol * want.square().mean().sqrt() + tol * want.abs().max()
+    assert (st.double() - ws).abs().max() <= tol * ws.abs().max()
 
 
 @pytest.mark.parametrize("what", ["k", "v", "z"])
-def test_later_tokens_do_not_reach_earlier_rows(cuda, what):
+def test_later_tokens_do_not_reach_earlier_rows(cuda, said, what):
     """An infinite key or value or a NaN decay changes its own row and the later ones of its sequence, no others."""
     torch.manual_seed(3)
     H, D, V, at = 2, 64, 128, 60
@@ -72,6 +94,7 @@ def test_later_tokens_do_not_reach_earlier_rows(cuda, what):
     else:
         args[0][at, H * D + 5 if what == "k" else 2 * H * D + 5] = float("inf")
     got, st = _run(cuda, args, H, H, D, V)
+    assert said == [True, True]
     keep = torch.ones(121, dtype=torch.bool)
     keep[at:80] = False
     assert torch.equal(got[keep], want[keep])
@@ -83,7 +106,7 @@ def test_later_tokens_do_not_reach_earlier_rows(cuda, what):
 
 @pytest.mark.parametrize("what", ["k", "q", "v", "state", "both", "nan", "overflow"])
 @pytest.mark.parametrize("H,G,D,V,pad", [(2, 2, 64, 128, 0), (3, 1, 64, 64, 1), (2, 1, 64, 256, 0), (2, 1, 128, 128, 3), (2, 2, 128, 64, 0)])
-def test_infinities_are_what_they_are_token_by_token(cuda, H, G, D, V, pad, what):
+def test_infinities_are_what_they_are_token_by_token(cuda, said, H, G, D, V, pad, what):
     """Rows and states are infinite, of the right sign, or NaN exactly where the recurrence itself makes them so; all others are as near as ever."""
     torch.manual_seed(D + V)
     args = _inputs([40, 33, 41], [3, 0, 7], H, G, D, V, pad)
@@ -107,6 +130,7 @@ def test_infinities_are_what_they_are_token_by_token(cuda, H, G, D, V, pad, what
     want, ws = _exact(args, H, G, D, V)
     want, ws = (torch.where(t.abs() > 3.4028235e38, t.sign() * float("inf"), t) for t in (want, ws))
     got, st = _run(cuda, args, H, G, D, V)
+    assert said == [True]
     if what == "state":
         assert torch.isnan(st[slots[1]]).sum() == 0
     assert not torch.isfinite(want).all()
