@@ -487,7 +487,8 @@ std::string latent_attn(Tensor out, Tensor q_lat, Tensor q, int64_t rot_off, Ten
     int64_t bound = block_tables.size(1) * cache.size(1);
     if (window > 0) bound = std::min<int64_t>(bound, window + max_q);
     if (die::latent_attn_decodes(a)) {
-      // one workgroup per compute unit: twice as many write twice the partial results (32 sequences of 750 - 1500 keys, 16 heads 12.2 + 4.7 us, 14.3 + 5.9)
+      // one workgroup per compute unit: twice as many write twice the partial results (32 sequences of 750 - 1500 keys, 16 heads 12.2 + 4.7 us, 14.3 + 5.9).
+      // 16 at most, as the kernels before (one sequence of 16 heads then has 16 of them: 2000 / 8000 / 32000 keys 48 / 118 / 385 -> 20 / 25 / 43 us)
       const int64_t ns = std::min<int64_t>({(int64_t)16, cus / std::max<int64_t>(1, S * ((H + 15) / 16)), (bound + 127) / 128});
       a.nsplit = (int)std::max<int64_t>(1, ns);
     } else {

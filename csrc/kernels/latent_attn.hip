@@ -700,7 +700,10 @@ inline bool decode_fits(const LatentAttnArgs& a) {
 }
 // Two bf16 parts of the weights for more than 32 heads: such steps went through latent_attn_wide_kernel or FINE splits, which have them, and in one
 // part were up to 10 % further from 64 bits (in two, 40, 64 and 128 heads, 1.0001 of those kernels; 2 - 8 % of the time). Up to 32 heads the
-// kernels before had one part, and more splits: 0.988 of their distance in one.
+// kernels before had one part, and more splits: 0.988 of their distance in one. Workgroups of 16 heads read the same rows each, where
+// latent_attn_wide_kernel read a tile once for 64 rows, and are faster all the same (rank 256 + 32, with the merge, kernels before / this, us):
+// 64 heads 1 x 500 keys 29.0 / 16.2, 1 x 32000 257 / 47, 32 x 500 29.9 / 19.7, 32 x 2000 65 / 32, 64 x 4000 183 / 64; 128 heads 29.2 / 15.9, 262 / 48,
+// 29.9 / 18.7, 79 / 42, 212 / 99.
 template <int NDB, int NROT> hipError_t launch_decode(const LatentAttnArgs& a, hipStream_t s) {
   const auto fn = a.heads > 32 ? latent_attn_decode_kernel<NDB, NROT, true> : latent_attn_decode_kernel<NDB, NROT, false>;
   constexpr int smem = DecodeTile<NDB, NROT>::total;

@@ -170,9 +170,10 @@ __global__ void __launch_bounds__(1024) moe_align_few_kernel(int* __restrict__ o
   }
 }
 
-// More pairs: one workgroup per expert; the same, and a pair's place in `sorted` ascends within its expert. Every workgroup reads all ids, counts those of lower experts and of its own, and writes its own rows, whose places are
-// neighbours: the one workgroup was bound by its scattered stores and by LDS atomics. This is bound by the first reading of the ids, which
-// no L2 holds, and by a CU's instructions, five per id and wave. us, few / this: 32764 pairs of 16 experts 24.0 / 9.0, 8192 of 8 6.9 / 5.3,
+// More pairs: one workgroup per expert; the same, and a pair's place in `sorted` ascends within its expert. Every workgroup reads all
+// ids, counts those of lower experts and of its own, and writes its own rows, whose places are neighbours: the one workgroup was bound by
+// its scattered stores and by LDS atomics. This is bound by the first reading of the ids, which no L2 holds, and by a CU's instructions,
+// five per id and wave. us, few / this: 32764 pairs of 16 experts 24.0 / 9.0, 8192 of 8 6.9 / 5.3,
 // 5040 of 32 6.8 / 5.6, 4160 of 8 5.6 / 5.5, 1172 of 10 2.6 / 3.8 (lines of results that several XCDs share); with a launch's 5 us, 1024 of
 // 256 7.7 / 6.1, 1536 of 160 7.1 / 6.1, 2048 of 64 6.5 / 6.1, 3072 of 16 6.6 / 6.2.
 // U: ids per lane that stay in registers for the second pass.

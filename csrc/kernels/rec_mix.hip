@@ -9,8 +9,8 @@
 //   selective_scan            S[c, :] <- exp(d A[c, :]) S[c, :] + d x B; y = S[c, :] . C + D x; y * silu(z): a
 //                             channel's states in the registers of 1 - 4 lanes for the whole step (9 - 16 states: selective_scan.hip)
 //   exp_gate_scan             log-space input / forget gates under a running maximum: a wave-wide scan over tokens
-//   gated_linear_attn         S <- a S + b k v^T, o = S^T q (prompt portions: chunk_rec.hip, chunk_channel.hip): one workgroup per (sequence, head, block of columns), the
-//                             state in registers (four columns per group of 4 - 16 lanes); the normaliser n <- a n + b k with its
+//   gated_linear_attn         S <- a S + b k v^T, o = S^T q (prompt portions: chunk_rec.hip, chunk_channel.hip): one
+//                             workgroup per (sequence, head, block of columns), the state in registers (four columns per group of 4 - 16 lanes); the normaliser n <- a n + b k with its
 //                             read-out n . q rides on the first wave; optionally a decay per row of S,
 //                             sigmoid(z)^(1/tau), computed while a trip is staged
 //   head_norm_gate            (o / (max(|n . q|, floor) + 1e-6), optional,) per-head RMS norm, weight, sigmoid or SiLU gate

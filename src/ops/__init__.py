@@ -848,7 +848,10 @@ def moe_apply(x: torch.Tensor, w13: torch.Tensor, w2: torch.Tensor, w: torch.Ten
     x = x.contiguous()
     # rows of the extra groups are never computed: zero them so that weight 0 x row stays 0
     ys = (torch.zeros if groups > e else torch.empty)(t * k, hdim, dtype=x.dtype, device=x.device)
-    # (eight experts of 4096 x 14336, us, sorted / unsorted: 1 token 153 / 130, 8 tokens 466 / 436, 32 tokens 479 / 442)
+    # (us, sorted / unsorted, 1, 8 and 32 tokens, two choices: eight experts of 4096 x 14336 129 393 456 / 120 382 433, 4096 x 4096 48 124 144 /
+    # 41 118 131, 2048 x 2048 22.6 46 56 / 20.0 40 44, 512 x 1024 14.1 18.3 20.2 / 12.1 13.8 15.6; 16 of 4096 x 2048 30.6 110 151 / 30.9 107 143;
+    # six of 64 of 2048 x 1024 30 88 170 / 29 80 144; four of 32 of 1024 x 512 15.4 28 38 / 15.0 26 31, at 2 tokens 16.8 / 17.2, the one of 54
+    # such steps that is slower by 2 %)
     if t <= MOE_DECODE_MAX_T and decode_experts(kern, x, w13, w2, ids, k, t, MOE_SILU, ys=ys) is not None:
         if residual is not None:
             kern.moe_combine_residual(ssp, residual, ys, _NO_ROWS(x.device), w)

@@ -221,6 +221,9 @@ DECODE_EXPERTS_MAX_T = 128   # tokens of a decode step whose experts stream thro
 # decode products / grouped, 65, 96 and 128 tokens: scaled mixture of 8 experts of 2048 x 2048 60 62 67 / 52 53 52, weighted one 57 58 62 / 52 53 53,
 # 16 of 2048 x 1024 46 47 52 / 45 45 45; 80 and 128 tokens of 32 of 1024 x 1024 54 56 / 46 47, 32 of 2048 x 2048 158 161 / 155 161; but 8 of 2048 x
 # 1024 29.2 32.8 / 29.9 30.5, 8 of 1024 x 1024 20 24 / 24 25, 32 of 512 x 256 14 14 / 18 18, 32 of 4096 x 2048 (65, 96 and 128) 202 209 215 / 221 222 223.
+# Beside the lines (scaled, 65 and 128 tokens): below 2^25 weights 14 of 2048 x 1024 51 51 / 46 46, 8 of 2048 x 1792 48 53 / 47 47, 20 of 1024 x 1024
+# 47 47 / 45 45; above 2^22 of a matrix 16 of 2048 x 2304 100 101 / 103 101, 16 of 2560 x 2048 108 109 / 113 112, 32 of it 185 190 / 188 197, but 8 of 3072 x
+# 2048 72 77 / 67 69: no step is more than 1.2 % slower for them (40 of 1024 x 1024, 65 tokens, 70.2 / 71.0), some would still gain.
 GROUPED_EXPERTS_MIN_T, GROUPED_MIN_WEIGHTS, GROUPED_MAX_MATRIX = 65, 1 << 25, 1 << 22
 
 
