@@ -6,20 +6,22 @@
 // through the sorted order on the way, so there is no gather pass. A unit is the W or the x rows of a stage of 64 K (whole 128-byte
 // lines); five units fit, so that while one stage is read the next and half of the one behind it are on their way, and while a tile's
 // results are formed and stored the first units of the next tile. The LDS image is lane-linear; 16-byte pieces are XOR-ed by row,
-// which makes the 32x32x16 fragment reads (32 rows, one piece per lane) conflict-free.
+// which makes the fragment reads (16 or 32 rows, one piece per lane) conflict-free.
 //
-// The waves are two groups, one wave of each per SIMD, half a stage apart: while one group's 16 matrix instructions run, the other
+// The waves are two groups, one wave of each per SIMD, half a stage apart: while one group's 32 matrix instructions run, the other
 // reads its next fragments and issues its fetches, and a barrier exchanges them. (Both waves of a SIMD reading and multiplying at their
 // own pace left the matrix cores waiting for fragments: a stage took 2500 - 2900 cycles, now 2000 - 2500 of 2048.) The activation runs
 // on the fp32 accumulators (a wave holds gate and up of the same columns), which takes two passes over [rows, 2 ff] out, and rounds
 // once where the separate passes rounded twice.
 //
-// What holds it up at many rows: LDS, which per stage reads 192 KB and takes 64 KB in (2048 cycles, as long as the products), and the
-// clock, which the products pull down to 1.6 - 1.8 GHz. (One wave per SIMD with 128 x 128 products reads a third less and ran 4096 x
-// 14336 up to 5 % faster, 2048-wide experts up to 15 % slower, as nothing runs beside its epilogues.) At few rows it is the weights' rate from
-// HBM. Each product alone, before (a barrier per stage, one tile per workgroup) -> now, us: 4096 tokens, two of 8 experts of 4096 x 14336:
-// 1880 -> 1700 and 1050 -> 920; 1000 of them 637 -> 569 and 357 -> 290; 8191 tokens, four of 16 experts of 2048 x 1024: 174 -> 140 and 172 -> 144;
-// 450 of them 38 -> 25 and 26 -> 19; 3000 tokens, four of 32 experts of 4096 x 2048: 252 -> 210 and 290 -> 223.
+// What holds it up at many rows is power: under the products the clock falls to 1.6 - 1.8 GHz. So the tiles are 16x16x32 products: at the power limit
+// a wave of 64 x 128 results runs 1.85 - 1.88 PFLOP/s with them from LDS on normal values and 1.60 - 1.64 with 32x32x16 (without the limit, on zeros, both are the
+// same), the rows of x gone through there and back so that each product shares an operand with the one before it (1.88 against 1.83 - 1.85). The fetches
+// into LDS take most of the rest: without them this kernel reaches 1.70 PFLOP/s instead of 1.33, with all of them from L2 1.45. (Waves of 128 x 128 results, one
+// per SIMD, read a third less LDS; as a kernel they ran 7 - 20 % slower, as nothing runs beside its epilogues.) At few rows it is the weights' rate from HBM.
+// Each product alone, 32x32x16 -> 16x16x32, us: 4096 tokens, two of 8 experts of 4096 x 14336: 1894 -> 1597 and 976 -> 860; 1000 of them 681 -> 612 and
+// 322 -> 303; 8191 tokens, four of 16 experts of 2048 x 1024: 144 -> 125 and 151 -> 132; 3000 tokens, four of 32 experts of 4096 x 2048: 208 -> 184 and 227 ->
+// 212; 1500 tokens, two of 8 gated experts of 2048 x 2048: 60 -> 54 and 35 -> 33.
 #include <math.h>
 
 #include <algorithm>
@@ -166,8 +168,15 @@ struct Plan {
   }
 };
 
-// A lane's results of 32 TN weight rows: z(n, i) is register i of the n-th 32-row tile (weight rows 8 g + 4 hi + 0 .. 3 of it for i = 4 g ..).
-// Lanes 32 apart exchange halves of neighbouring g, so that each stores 8 columns at `op`, its own 8 hi columns on.
+// The activation on one value of a result column (with a gate: its gate and up sums).
+template <int ACT> __device__ __forceinline__ float activated(float g, float u, const MoeGemmArgs& a) {
+  if constexpr (ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU) return moe_gate<ACT>(g, u, a.limit, a.alpha);
+  if constexpr (ACT == MOE_ACT_RELU2) return fmaxf(g, 0.f) * fmaxf(g, 0.f);
+  return g;
+}
+
+// A lane's results of 32 TN weight rows by 32x32 products: z(n, i) is register i of the n-th 32-row tile (weight rows 8 g + 4 hi + 0 .. 3 of it for
+// i = 4 g ..). Lanes 32 apart exchange halves of neighbouring g, so that each stores 8 columns at `op`, its own 8 hi columns on.
 template <int ACT, class Z> __device__ __forceinline__ void store_row(Z z, uint16_t* op, bool in, const MoeGemmArgs& a) {
   constexpr bool GATED = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU;
 #pragma unroll
@@ -179,19 +188,32 @@ template <int ACT, class Z> __device__ __forceinline__ void store_row(Z z, uint1
       for (int q = 0; q < 2; ++q) {
         float y[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if constexpr (GATED)
-            y[i] = moe_gate<ACT>(z(n, 4 * (g + q) + i), z(TN / 2 + n, 4 * (g + q) + i), a.limit, a.alpha);
-          else
-            y[i] = z(n, 4 * (g + q) + i);
-          if constexpr (ACT == MOE_ACT_RELU2) y[i] = fmaxf(y[i], 0.f) * fmaxf(y[i], 0.f);
-        }
+        for (int i = 0; i < 4; ++i) y[i] = activated<ACT>(z(n, 4 * (g + q) + i), GATED ? z(TN / 2 + n, 4 * (g + q) + i) : 0.f, a);
         p[q][0] = pack2(y[0], y[1]), p[q][1] = pack2(y[2], y[3]);
       }
       const auto u = __builtin_amdgcn_permlane32_swap(p[0][0], p[1][0], false, false);
       const auto v = __builtin_amdgcn_permlane32_swap(p[0][1], p[1][1], false, false);
       if (in) *reinterpret_cast<uint4*>(op + 32 * n + 8 * g) = make_uint4(u[0], v[0], u[1], v[1]);
     }
+}
+// The same by 16x16 products: z(n, i) is register i of the n-th 16-row tile (weight rows 4 (lane / 16) + i of it). Lanes 16 apart exchange their
+// columns of neighbouring tiles; each stores 8 columns at `op`, its own 16 (lane / 16 % 2) + 8 (lane / 32) columns on.
+template <int ACT, class Z> __device__ __forceinline__ void store_row16(Z z, uint16_t* op, bool in, const MoeGemmArgs& a) {
+  constexpr bool GATED = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU;
+#pragma unroll
+  for (int n = 0; n < (GATED ? TN : 2 * TN); n += 2) {
+    uint32_t p[2][2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      float y[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[i] = activated<ACT>(z(n + q, i), GATED ? z(TN + n + q, i) : 0.f, a);
+      p[q][0] = pack2(y[0], y[1]), p[q][1] = pack2(y[2], y[3]);
+    }
+    const auto u = __builtin_amdgcn_permlane16_swap(p[0][0], p[1][0], false, false);
+    const auto v = __builtin_amdgcn_permlane16_swap(p[0][1], p[1][1], false, false);
+    if (in) *reinterpret_cast<uint4*>(op + 16 * n) = make_uint4(u[0], v[0], u[1], v[1]);
+  }
 }
 
 template <int ACT, bool TURN>
@@ -200,7 +222,7 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
   constexpr bool GATED = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU;
   constexpr int NO = GATED ? BN / 2 : BN;           // output columns of a tile
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wn = wave % WN, wm = wave / WN, fr = lane & 31, hi = lane >> 5;
+  const int wn = wave % WN, wm = wave / WN, fr = lane & 15, lg = lane >> 4;
   const int nst = a.K / BK;
 
   const Plan plan(a, a.ncols / NO, lane);
@@ -256,9 +278,9 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
     issue_x(0, 1, (u.M + 63) / 64);
     if (nst > 1) issue_w(1, 2);
   };
-  int lo[BK / 16];   // a fragment of 32 rows: the lane's place at step kk
+  int lo[BK / 32];   // a fragment of 16 rows: the lane's place at step kk
 #pragma unroll
-  for (int kk = 0; kk < BK / 16; ++kk) lo[kk] = fr * ROWB + 16 * ((2 * kk + hi) ^ swz(fr));
+  for (int kk = 0; kk < BK / 32; ++kk) lo[kk] = fr * ROWB + 16 * ((4 * kk + lg) ^ swz(fr));
 
   rows_of(t);
   begin(t);
@@ -268,31 +290,29 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
     if (more) rows_of(next);
     const int nx = (t.M + 63) / 64, mc = ((t.M + 31) / 32 + 1 - wm) / 2;   // 64-row pieces of x that are fetched; the wave's 32-row pieces
     auto run = [&](auto mc_) {
-    constexpr int MC = decltype(mc_)::value, MX = MC > 0 ? MC : 1;
-    f32x16_t acc[TN][MX] = {};
-    bf16x8_t wf[2][TN], xf[2][MX];
+    constexpr int MC = decltype(mc_)::value, MT = 2 * MC, MX = MT > 0 ? MT : 1, NT = 2 * TN;   // 16-row tiles of x, of W
+    f32x4_t acc[NT][MX] = {};
+    bf16x8_t wf[NT], xf[MX];
     auto products = [&] {
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-      for (int k = 0; k < 2; ++k)
+      for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int m = 0; m < MC; ++m)
-#pragma unroll
-          for (int n = 0; n < TN; ++n) acc[n][m] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[k][n], xf[k][m], acc[n][m], 0, 0, 0);
+        for (int i = 0; i < NT; ++i) {   // (there and back: one operand stays at every product)
+          const int n = m & 1 ? NT - 1 - i : i;
+          acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[n], xf[m], acc[n][m], 0, 0, 0);
+        }
       __builtin_amdgcn_s_setprio(0);
     };
       auto load = [&](int ws, int xs, auto half) {   // fragments of half a stage
         const char* wp = smem + ws * UNIT + 32 * TN * wn * ROWB;
         const char* xp = smem + xs * UNIT + 32 * wm * ROWB;
+        const int l = lo[decltype(half)::value];
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          const int l = lo[2 * decltype(half)::value + k];
+        for (int n = 0; n < NT; ++n) wf[n] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(wp + 16 * n * ROWB + l));
 #pragma unroll
-          for (int n = 0; n < TN; ++n) wf[k][n] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(wp + 32 * n * ROWB + l));
-#pragma unroll
-          for (int m = 0; m < MC; ++m)
-            xf[k][m] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(xp + 64 * m * ROWB + l));
-        }
+        for (int m = 0; m < MT; ++m)
+          xf[m] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(xp + (64 * (m / 2) + 16 * (m % 2)) * ROWB + l));
       };
       wait_vm<0>();
       barrier();
@@ -341,11 +361,11 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
 
     // ---- results: x row in the lane, weight rows in the registers
 #pragma unroll
-    for (int m = 0; m < MC; ++m) {
-      const int row = 32 * (2 * m + wm) + fr, rr = t.r0 + min(row, t.M - 1);
+    for (int m = 0; m < MT; ++m) {
+      const int row = 32 * (2 * (m / 2) + wm) + 16 * (m % 2) + fr, rr = t.r0 + min(row, t.M - 1);
       const float sc = a.scale != nullptr ? a.scale[a.sorted != nullptr ? a.sorted[rr] : rr] : 1.0f;
-      uint16_t* op = a.out + (int64_t)rr * a.ncols + t.n0 * NO + (GATED ? 16 : 32) * TN * wn + 8 * hi;
-      store_row<ACT>([&](int n, int i) __attribute__((always_inline)) { return acc[n][m][i] * sc; }, op, row < t.M, a);
+      uint16_t* op = a.out + (int64_t)rr * a.ncols + t.n0 * NO + (GATED ? 16 : 32) * TN * wn + 16 * (lg & 1) + 8 * (lg >> 1);
+      store_row16<ACT>([&](int n, int i) __attribute__((always_inline)) { return acc[n][m][i] * sc; }, op, row < t.M, a);
     }
     };
     if (mc == 4) run(IntC<4>{});
