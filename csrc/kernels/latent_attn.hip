@@ -768,9 +768,9 @@ template <int ROWS> __device__ __forceinline__ bool tile_of(const LatentAttnArgs
 // pieces lies in LDS as the DMA writes it, without gaps; the pieces of a row are exchanged (XOR) so that 16 consecutive rows' reads
 // of one piece fall on all banks, and so do the transposed reads of 8 rows by two pieces (the number is rotated for those: by the plain
 // row number pairs of rows shared banks, a quarter of the kernel's cycles).
-// Bound by LDS reads (34 KB per wave and tile at 128 bytes a cycle: 120 us of the 246 below). 16 sequences of 1024 rows, 16 heads,
+// Bound by the latency of its LDS reads (see latent_attn_two_kernel, which takes larger steps). 16 sequences of 1024 rows, 16 heads,
 // rank 256 + 32: 32 rows per wave, one wave per SIMD, tiles through registers, looked up piece by piece behind divisions: 518 us;
-// the same with DMA and the next tile's scores under the softmax 370; this 246 (585 TFLOP/s; 250 with the queries
+// the same with DMA and the next tile's scores under the softmax 370; this 246 (250 with the queries
 // loaded behind the first tile, where 24 - 100 rows of 20 and more sequences took 3 % longer too).
 template <int NDB, int NROT> struct RqTile {
   static constexpr int KCH = 4 * NDB + 2 * NROT, NPF = (MKT * KCH + 255) / 256, BYTES = NPF * 4096;
@@ -1007,6 +1007,317 @@ __global__ void __launch_bounds__(256, 3) latent_attn_mfma_rq_kernel(LatentAttnA
     const int64_t to = (int64_t)__shfl((int)orow, row, 64) * R + 8 * (lane % PR);
     const uint4 w = *reinterpret_cast<const uint4*>(os + row * Z::OP + 16 * (lane % PR));
     if (wrow + row < nrows) *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(a.out) + to) = w;
+  }
+}
+
+// The same with two groups of 16 rows per wave, each fragment that is read from LDS serving both, and the next ones read ahead of a step's products (with
+// one group and three waves per SIMD there are no registers for that, and every pair of products waited for its reads: a wave and tile took 6300
+// cycles for 410 instructions). Sums take 128 registers at rank 256; of the queries' 72 the first NQL steps' lie in LDS, so that two waves fit on a SIMD and two workgroups
+// of 128 rows on a CU. The scale enters with the exponential's argument (a positive one). What bounds it: vector instructions, 49 % of the cycles (80 to 210 of a wave and
+// tile rescale and exponentiate), beside products, 32 %, and LDS reads that the two waves of a SIMD don't hide; 16 sequences of 1024 rows, 16 heads, rank 256 + 32:
+// 257 -> 213 us. (The next tile's fetch kept apart from the transposed reads, which the compiler has wait for it, or waves in products first: 1 - 3 % slower.)
+template <int NDB, int NROT> struct TwoTile : RqTile<NDB, NROT> {
+  static_assert(NDB == 8, "below rank 256 three waves of one group are faster");
+  using Z = RqTile<NDB, NROT>;
+  static constexpr int ROWS = 128, NK = NDB + NROT / 2;         // rows of a workgroup; 32-wide steps of a row
+  static constexpr int NQL = NROT == 0 ? 5 : 4, QB = 2048 * NQL;   // steps whose query fragments lie in LDS, a wave's bytes of them
+  static constexpr int ALL = 2 * Z::BYTES + 4 * QB + 4 * Z::TABLE, LDS = ALL > 64 * Z::OP ? ALL : 64 * Z::OP;
+  static_assert(2 * LDS <= 160 * 1024, "two workgroups per compute unit");
+};
+template <int NDB, int NROT>
+__global__ void __launch_bounds__(256, 2) latent_attn_two_kernel(LatentAttnArgs a, uint32_t bs_mul, int bs_shift) {
+  using Z = TwoTile<NDB, NROT>;
+  constexpr int KCH = Z::KCH, NPF = Z::NPF, NLAT = NDB, NK = Z::NK, NQL = Z::NQL;   // 32-wide steps of a row: latent, in all
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];   // two tiles, query fragments, block-table entries; at the end the results
+  int s, row0;
+  if (!tile_of<Z::ROWS>(a, s, row0)) return;
+  const int lane = threadIdx.x & 63, tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int H = a.heads;
+  constexpr int R = 32 * NDB, Dk = R + 16 * NROT;
+  const int q0 = a.cu_q ? a.cu_q[s] : s;
+  const int nq = a.cu_q ? a.cu_q[s + 1] - q0 : 1;
+  const int nrows = nq * H;
+  const int ctx = a.ctx_lens[s];
+  const int last_row = min(row0 + Z::ROWS, nrows) - 1;
+  const int p_first = (int)a.positions[q0 + row0 / H], p_last = (int)a.positions[q0 + last_row / H];
+  const int jlo = a.window > 0 ? max(0, p_first - a.window + 1) : 0;
+  const int jhi = min(p_last, ctx - 1);
+  const bf16_t* cache = reinterpret_cast<const bf16_t*>(a.cache);
+  const int li = lane & 15, lg = lane >> 4;
+
+  const int wrow = row0 + wave * 32;
+  const bool wave_live = wrow < nrows, all_rows = wrow + 31 < nrows;
+  const int pw_min = wave_live ? (int)a.positions[q0 + wrow / H] : 0;
+  const int pw_max = wave_live ? (int)a.positions[q0 + min(wrow + 31, nrows - 1) / H] : 0;
+  // this lane's query fragments of either group: 32-wide step k of row li, columns 32 k + 8 lg .. + 8; an odd NROT leaves 16 columns, of which the lane
+  // has 4. The first NQL steps go to LDS. (Rows beyond the last repeat the first; every load is unconditional, so that all are in flight together, and
+  // beside the table's.)
+  int prow[2];
+  uint32_t orow[2];
+  float sink[2];
+  bf16x8_t qf[2][NK > 0 ? NK : 1];
+  short4_t qt[2] = {};
+  constexpr int E = NROT % 2 == 0 ? 8 : 4, NS = (NROT + 1) / 2;
+  bf16_t qr[2][NS > 0 ? NS : 1][E];
+  float fr[NS > 0 ? NS : 1][E / 2];
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const int myrow = wrow + 16 * g + li;
+    const bool rok = myrow < nrows;
+    const int64_t tq = rok ? q0 + myrow / H : q0;
+    const int hq = rok ? myrow % H : 0;
+    orow[g] = (uint32_t)((int64_t)hq * a.total_q + tq);
+    prow[g] = rok ? (int)a.positions[tq] : -1;
+    sink[g] = a.sink != nullptr ? a.sink[hq] : 0.f;
+    const bf16_t* qlat = reinterpret_cast<const bf16_t*>(a.q_lat) + (int64_t)orow[g] * R;
+#pragma unroll
+    for (int k = 0; k < NLAT; ++k) qf[g][k] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(qlat + 32 * k + 8 * lg));
+    if constexpr (NROT > 0) {
+      const bf16_t* qp = reinterpret_cast<const bf16_t*>(a.q_rot) + tq * a.q_stride + (int64_t)hq * a.q_hstride + E * lg;
+#pragma unroll
+      for (int k = 0; k < NS; ++k)
+#pragma unroll
+        for (int e = 0; e < E; ++e) qr[g][k][e] = qp[32 * k + e];
+    }
+  }
+  if constexpr (NROT > 0) {
+#pragma unroll
+    for (int k = 0; k < NS; ++k)
+#pragma unroll
+      for (int i = 0; i < E / 2; ++i)
+        fr[k][i] = a.sh.rot_pairs > 0 ? a.sh.inv_freq[min(16 * k + E / 2 * lg + i, a.sh.rot_pairs - 1)] : 0.f;
+  }
+
+  // Block-table entries of the workgroup's keys in LDS (TABLE at a time), so that a tile's loads depend on LDS reads alone
+  const int* bt = a.block_tables + (int64_t)s * a.bt_stride;
+  int* btl = reinterpret_cast<int*>(smem_raw + 2 * Z::BYTES + 4 * Z::QB);
+  char* const ql = smem_raw + 2 * Z::BYTES + wave * Z::QB + 16 * lane;   // the wave's query fragments
+  auto block_of = [&](int j) { return a.block_size == 1 ? j : (int)(__umulhi((uint32_t)j, bs_mul) >> bs_shift); };
+  const int b_hi = block_of(max(jhi, 0));
+  int b_lo = block_of(jlo);
+  auto stage_table = [&]() {
+    for (int u = tid; u < Z::TABLE && b_lo + u <= b_hi; u += 256) btl[u] = bt[b_lo + u];
+    __syncthreads();
+  };
+  stage_table();
+  // tile rows by DMA: piece u of this thread is 16 bytes of key krow[u] (beyond the tile: of key 31, into the slack)
+  int krow[NPF], pcol[NPF];
+#pragma unroll
+  for (int u = 0; u < NPF; ++u) {
+    const int idx = tid + 256 * u, row = min(idx / KCH, MKT - 1);
+    krow[u] = row;
+    pcol[u] = 8 * (idx < MKT * KCH ? (idx - row * KCH) ^ Z::swz(row) : 0);
+  }
+  auto fetch = [&](const bf16_t* src, char* to, int j0) __attribute__((always_inline)) {   // (keys beyond the last repeat it)
+    if (block_of(min(j0 + MKT - 1, jhi)) >= b_lo + Z::TABLE) {
+      __syncthreads();
+      b_lo = block_of(j0);
+      stage_table();
+    }
+    uint32_t row[NPF];   // (as many cache rows as a device holds)
+#pragma unroll
+    for (int u = 0; u < NPF; ++u) {
+      const int j = min(j0 + krow[u], jhi), jb = block_of(j);
+      row[u] = (uint32_t)btl[jb - b_lo] * (uint32_t)a.block_size + (uint32_t)(j - jb * a.block_size);
+    }
+    __builtin_amdgcn_sched_barrier(0);   // (all lookups, then the loads: they would go in turns, each waited for)
+#pragma unroll
+    for (int u = 0; u < NPF; ++u) {
+      __builtin_amdgcn_global_load_lds((global_cvoid*)(src + ((uint64_t)row[u] * Dk + pcol[u])), (lds_void*)(to + (256 * u + 64 * wave) * 16), 16, 0, 0);
+    }
+  };
+  const int nt = jhi < jlo ? 0 : (jhi - jlo) / MKT + 1;
+  if (nt > 0) fetch(cache, smem_raw, jlo);
+
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    if constexpr (NROT > 0) {
+#pragma unroll
+      for (int k = 0; k < NS; ++k) {
+        float f[8] = {};
+#pragma unroll
+        for (int i = 0; i < E / 2; ++i) {
+          const float u = bf2f(qr[g][k][2 * i]), w = bf2f(qr[g][k][2 * i + 1]);
+          float sn, cs;
+          __sincosf((float)prow[g] * fr[k][i], &sn, &cs);
+          const bool turned = 16 * k + E / 2 * lg + i < a.sh.rot_pairs;
+          f[2 * i] = turned ? u * cs - w * sn : u;
+          f[2 * i + 1] = turned ? w * cs + u * sn : w;
+        }
+        const uint4 w = pack8(f);
+        if constexpr (E == 8)
+          qf[g][NLAT + k] = __builtin_bit_cast(bf16x8_t, w);
+        else
+          qt[g] = __builtin_bit_cast(short4_t, make_uint2(w.x, w.y));
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < NQL; ++k) *reinterpret_cast<uint4*>(ql + 1024 * (2 * k + g)) = __builtin_bit_cast(uint4, qf[g][k]);
+  }
+  // (a wave reads the fragments that it wrote)
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+
+  constexpr float LOG2E = 1.4426950408889634f;
+  const float sl2 = a.scale * LOG2E;
+  float m[2], l[2];   // (l: the sum of this lane's keys)
+  f32x4_t o[2][2 * NDB];
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const bool has_sink = a.sink != nullptr && wrow + 16 * g + li < nrows;
+    m[g] = has_sink ? sink[g] * LOG2E : -1e30f;
+    l[g] = has_sink && lg == 0 ? 1.0f : 0.0f;
+#pragma unroll
+    for (int db = 0; db < 2 * NDB; ++db) o[g][db] = f32x4_t{};
+  }
+  // K fragments: key li of 16, piece 4 k + lg; V fragments: keys 4 lg .. of either 16 (the order in which the weights lie in
+  // registers), columns 16 db ..
+  // (the number that is XOR-ed is below G: a piece G and more on is an offset)
+  constexpr int KB = Z::G < 4 ? 1 : Z::G / 4, VB = Z::G / 2;
+  const int ksw = Z::swz(li), vrow = 4 * lg + (li >> 2), vsw = Z::swz(vrow);
+  uint32_t kat[KB], vat[VB];
+#pragma unroll
+  for (int u = 0; u < KB; ++u) kat[u] = 16 * li * KCH + 16 * ((4 * u + lg) ^ ksw);
+#pragma unroll
+  for (int u = 0; u < VB; ++u) vat[u] = 16 * vrow * KCH + 8 * (li & 1) + 16 * ((2 * u + (li >> 1 & 1)) ^ vsw);   // (rows r and r + 16 are exchanged alike)
+  // The queries are here. (Without this the compiler waits for them in the loop, behind the next tile's DMA and so for that too.)
+  __builtin_amdgcn_s_waitcnt(15 << 8 | 7 << 4);
+  // Tile i at `ks`, the next one's fetch to `to`. (Two places that share nothing: said so, since the compiler would have the transposed reads wait for the
+  // fetch, 5 % of the time.)
+  auto tile = [&](const bf16_t* src, char* to, const char* ks, int i) __attribute__((always_inline)) {
+    const int j0 = jlo + i * MKT;
+    // tile i is in LDS for every wave, and every wave has left the other buffer
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(7 << 4);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (i + 1 < nt) fetch(src, to, j0 + MKT);
+    if (!wave_live) return;
+    f32x4_t sc[2][2] = {};   // [group][16 keys]
+    // fragments of the next step of the row ahead of a step's products; each serves both groups
+    bf16x8_t kf[2][2], qs[2][2];
+    auto read_k = [&](int k) __attribute__((always_inline)) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        kf[k & 1][t] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(ks + kat[k % KB] + 256 * KCH * t + 64 * (k - k % KB)));
+      if (k < NQL) {
+#pragma unroll
+        for (int g = 0; g < 2; ++g) qs[k & 1][g] = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(ql + 1024 * (2 * k + g)));
+      }
+    };
+    read_k(0);
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+      if (k + 1 < NK) read_k(k + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+          sc[g][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[k & 1][t], k < NQL ? qs[k & 1][g] : qf[g][k], sc[g][t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (NROT % 2 != 0)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const uint2 w = *reinterpret_cast<const uint2*>(ks + 16 * li * KCH + 256 * KCH * t + 16 * ((4 * NK + (lg >> 1)) ^ ksw) + 8 * (lg & 1));
+#pragma unroll
+        for (int g = 0; g < 2; ++g) sc[g][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(short4_t, w), qt[g], sc[g][t], 0, 0, 0);
+      }
+    // V fragments VG column blocks ahead, the first ones beside the softmax
+    constexpr int VG = 2, NV = 2 * NDB / VG;
+    bf16x8_t vf[2][VG];
+    auto read_v = [&](int g) __attribute__((always_inline)) {
+#pragma unroll
+      for (int d = 0; d < VG; ++d) {
+        const int db = VG * g + d;
+        const char* at = ks + vat[db % VB] + 32 * (db - db % VB);
+        const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)at);
+        const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(at + 256 * KCH));
+        vf[g & 1][d] = __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+      }
+    };
+    read_v(0);
+    __builtin_amdgcn_sched_barrier(0);
+    // interior tiles (every key visible to every row of the wave) skip the per-score mask
+    const bool inner = all_rows && j0 + MKT - 1 <= min(pw_min, jhi) && (a.window <= 0 || pw_max - j0 < a.window);
+    if (!inner) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int j = j0 + 16 * t + 4 * lg + e;   // (rows beyond the last: position -1)
+            const bool valid = j <= jhi && j <= prow[g] && (a.window <= 0 || prow[g] - j < a.window);
+            sc[g][t][e] = valid ? sc[g][t][e] : -INFINITY;
+          }
+    }
+    bf16x8_t pf[2];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mx = fmaxf(mx, sc[g][t][e]);
+      const float mn = fmaxf(m[g], xor16_max(xor32_max(mx)) * sl2);
+      float alpha = __builtin_amdgcn_exp2f(m[g] - mn);
+      float sum = 0.f;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          sc[g][t][e] = __builtin_amdgcn_exp2f(fmaf(sc[g][t][e], sl2, -mn));
+          sum += sc[g][t][e];
+        }
+      l[g] = l[g] * alpha + sum;
+      m[g] = mn;
+      pf[g] = __builtin_bit_cast(bf16x8_t, make_uint4(pack2(sc[g][0][0], sc[g][0][1]), pack2(sc[g][0][2], sc[g][0][3]), pack2(sc[g][1][0], sc[g][1][1]),
+                                                      pack2(sc[g][1][2], sc[g][1][3])));
+      if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {   // wave-uniform
+        asm volatile("" : "+v"(alpha));                        // (not multiplied ahead of the condition)
+#pragma unroll
+        for (int db = 0; db < 2 * NDB; ++db)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[g][db][e] *= alpha;
+      }
+    }
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      if (v + 1 < NV) read_v(v + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int d = 0; d < VG; ++d)
+#pragma unroll
+        for (int g = 0; g < 2; ++g) o[g][VG * v + d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[v & 1][d], pf[g], o[g][VG * v + d], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  for (int i = 0; i < nt; ++i) tile(cache, smem_raw + (~i & 1) * Z::BYTES, smem_raw + (i & 1) * Z::BYTES, i);
+  // results through LDS (tiles and table are done with), 16 rows at a time, so that whole rows are written 16 bytes a lane
+  __syncthreads();
+  char* os = smem_raw + wave * 16 * Z::OP;
+  constexpr int PR = R / 8, RPI = 64 / PR;   // pieces of a row, rows of an instruction
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const float sum = xor16_sum(xor32_sum(l[g])), inv = sum > 0.f ? 1.0f / sum : 0.f;
+#pragma unroll
+    for (int db = 0; db < 2 * NDB; ++db)
+      *reinterpret_cast<uint2*>(os + li * Z::OP + 32 * db + 8 * lg) =
+          make_uint2(pack2(o[g][db][0] * inv, o[g][db][1] * inv), pack2(o[g][db][2] * inv, o[g][db][3] * inv));
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int u = 0; u < 16 / RPI; ++u) {
+      const int row = RPI * u + lane / PR;
+      const int64_t to = (int64_t)__shfl((int)orow[g], row, 64) * R + 8 * (lane % PR);
+      const uint4 w = *reinterpret_cast<const uint4*>(os + row * Z::OP + 16 * (lane % PR));
+      if (wrow + 16 * g + row < nrows) *reinterpret_cast<uint4*>(reinterpret_cast<bf16_t*>(a.out) + to) = w;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // (the rows are read before the other group's replace them)
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -1257,6 +1568,17 @@ template <int NDB, int NROT> hipError_t launch_wide(const LatentAttnArgs& a, hip
   hipLaunchKernelGGL(fn, grid, dim3(256), lds, s, a, bs_mul, log - 1);
   return hipGetLastError();
 }
+template <int NDB, int NROT> hipError_t launch_two(const LatentAttnArgs& a, hipStream_t s) {
+  int log = 1;
+  while ((int64_t)1 << log < a.block_size) ++log;
+  const uint32_t bs_mul = a.block_size == 1 ? 0 : (uint32_t)(((uint64_t)1 << (31 + log)) / a.block_size + 1);
+  constexpr int ROWS = TwoTile<NDB, NROT>::ROWS, lds = TwoTile<NDB, NROT>::LDS;
+  auto* fn = latent_attn_two_kernel<NDB, NROT>;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3((unsigned)(((int64_t)a.max_q * a.heads + ROWS - 1) / ROWS), (unsigned)a.num_seqs), dim3(256), lds, s, a, bs_mul, log - 1);
+  return hipGetLastError();
+}
 template <int NDB, int NROT> hipError_t launch_mfma_rq(const LatentAttnArgs& a, hipStream_t s) {
   // floor(j / block_size) = (j * bs_mul) >> (32 + bs_shift) for 31-bit j
   int log = 1;
@@ -1283,8 +1605,23 @@ inline bool wide_takes(const LatentAttnArgs& a) {
   const int64_t wgs = ((int64_t)a.max_q * a.heads + 63) / 64 * a.num_seqs, keys = (int64_t)a.bt_cols * a.block_size;
   return wgs <= 2 * (int64_t)num_cus() && keys > 64 && a.scale > 0.f;
 }
+// Two groups of 16 rows per wave: where there is more than one turn of its workgroups (two per CU), and enough keys that starting them, which takes
+// longer, doesn't count; in one turn where all sequences have the same rows and see many keys (with others the longest ends alone). One group / two, rank
+// 256 + 32, us: 16 x 1024 rows of 16 heads 257 / 213; 8 of 786 - 1000 101 / 89; 32 of 125 - 250, 32 heads 73 / 65; 16 of 200 - 400, 32 heads 67 / 63; 6 x 300 behind
+// 300, 32 heads, window 512 63 / 47; 8 x 500 behind 300 73 / 61; 4 x 1000 70 / 66. Not: 4 of 889 - 1000 70 / 74; 32 x 200 39 / 42; 32 of 50 - 100 behind 150 - 300
+// 33 / 37; 24 x 100 19 / 19. Without a rotary part, or with one of 64 (13 registers in scratch), the gain is 2 - 10 % smaller: twice the work.
+inline bool two_takes(const LatentAttnArgs& a) {
+  const int64_t cus = num_cus(), wgs = (int64_t)a.total_q * a.heads / 128, keys = (int64_t)a.bt_cols * a.block_size - a.max_q / 2;
+  const int64_t seen = a.window > 0 ? std::min<int64_t>(keys, a.window) : keys;   // by a row, about
+  if (a.sh.rank != 256 || !(a.scale > 0.f) || seen < 1) return false;
+  if (wgs > 2 * cus && wgs * seen >= (a.sh.rot_dim == 16 || a.sh.rot_dim == 32 ? 680 : 1360) * cus) return true;
+  return (int64_t)a.max_q * a.num_seqs == a.total_q && 4 * wgs > 5 * cus && seen >= 400;
+}
 template <int NDB, int NROT> hipError_t launch_rows(const LatentAttnArgs& a, hipStream_t s) {
-  return wide_takes(a) ? launch_wide<NDB, NROT>(a, s) : launch_mfma_rq<NDB, NROT>(a, s);
+  if (wide_takes(a)) return launch_wide<NDB, NROT>(a, s);
+  if constexpr (NDB == 8)
+    if (two_takes(a)) return launch_two<NDB, NROT>(a, s);
+  return launch_mfma_rq<NDB, NROT>(a, s);
 }
 template <int NDB> hipError_t launch_mfma_rq_rot(const LatentAttnArgs& a, hipStream_t s) {
   switch (a.sh.rot_dim) {
@@ -1364,6 +1701,7 @@ const char* latent_attn_kernel(const LatentAttnArgs& a) {
   if (decode_fits(a)) return "decode";
   const char* form = latent_attn_form(a);
   if (form[0] == 'r' && wide_takes(a)) return "wide";
+  if (form[0] == 'r' && two_takes(a)) return "two rows";
   return form[0] == 's' && a.fine ? "fine split" : form;
 }
 

@@ -136,7 +136,7 @@ bool latent_attn_fits_rows(const LatentAttnArgs& a);
 // the kernel that launch_latent_attn runs: "rows" (matrix cores, queries in registers), "tiles" (queries in LDS), "split" (the same,
 // keys split and merged), "fma"
 const char* latent_attn_form(const LatentAttnArgs& a);
-// its kernel: "wide" for the rows of few tiles, "fine split" for weights in two parts, else the form
+// its kernel: "wide" for the rows of few tiles, "two rows" for those of many behind many keys, "fine split" for weights in two parts, else the form
 const char* latent_attn_kernel(const LatentAttnArgs& a);
 
 }  // namespace die

@@ -99,6 +99,36 @@ def test_row_table_is_filled_again(cuda, rank, rot, heads, bs, lens, past, kerne
     assert ((got.float() - want).norm() / want.norm()).item() < 2 ** -7
 
 
+@pytest.mark.parametrize("rot,heads,bs,window,lens,past,kernel", [
+    (32, 32, 16, 0, (520, 511, 497, 520, 33, 519, 520, 512, 520), 0, "two rows"), (16, 31, 24, 300, (600, 590, 1, 600, 600, 130, 600), 200, "two rows"),
+    (0, 33, 7, 0, (700, 655, 700, 690, 129), 300, "two rows"), (64, 32, 1, 0, (650,) * 5, 1000, "two rows"), (32, 16, 1, 0, (1400, 1400), 0, "two rows"),
+    (32, 32, 16, 0, (250, 130) * 4, 0, "rows")])
+def test_two_groups_of_rows(cuda, rot, heads, bs, window, lens, past, kernel):
+    """Two groups of 16 rows per wave: remainders of the workgroups' 128 rows and of key tiles, windows, every rotary width, the table filled again."""
+    from src.ops import mix
+
+    rank = 256
+    torch.manual_seed(rot + heads + bs)
+    S, T, need = len(lens), sum(lens), -(-(max(lens) + past) // bs)
+    cache = torch.randn(1 + 2 * need, bs, rank + rot, device=cuda).to(torch.bfloat16)
+    bt = torch.randint(0, 1 + 2 * need, (S, need), device=cuda, dtype=torch.int32)
+    cu = torch.tensor([0, *lens], device=cuda).cumsum(0).int()
+    pos = torch.cat([torch.arange(n) + past for n in lens]).to(cuda)
+    ctx = torch.tensor([n + past for n in lens], device=cuda, dtype=torch.int32)
+    q_lat, q = torch.randn(heads, T, rank, device=cuda).to(torch.bfloat16), torch.randn(T, heads * (rot + 6), device=cuda).to(torch.bfloat16)
+    inv, sink, scale = ops.rope_inv_freq(10000.0, max(rot, 2), cuda)[: rot // 2], torch.randn(heads, device=cuda) + 1, 0.08
+    got = torch.empty_like(q_lat)
+    tail = (cache, bt, cu, ctx, pos, sink, max(lens), window, scale, rot, inv)
+    assert mix._kern().latent_attn_named(got, q_lat, q, 6, *tail, 0) == kernel
+    want = ops.latent_attn(q_lat, q, 6, *tail, impl=1).float()
+    e = 0.0
+    if rot:
+        e = scale * 2 ** -9 * float(q.view(T, heads, -1)[..., 6:].float().norm(dim=-1).max() * cache[..., rank:].float().norm(dim=-1).max())
+    top = float(cache[..., :rank].float().abs().max())
+    assert ((got.float() - want).abs() <= (2 ** -9 + 2 * e * 2.71828 ** (2 * e)) * top + 2 ** -7 * want.abs()).all()
+    assert ((got.float() - want).norm() / want.norm()).item() < 2 ** -7
+
+
 def test_results_at_any_8_bytes(cuda):
     """Results that start at no multiple of 16 bytes go to the kernel that writes 8 at a time: the bits that it writes anywhere."""
     from src.ops import mix
