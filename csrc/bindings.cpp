@@ -128,6 +128,63 @@ void rms_row_scale(Tensor rs, Tensor resid, Tensor x, double eps) {
                                    cur_stream()));
 }
 
+// the same after resid += slab.sum(0), slab [sk, T, hidden] fp32
+void rms_row_scale_slab(Tensor rs, Tensor resid, Tensor slab, double eps) {
+  CHK_CUDA(resid);
+  CHK_BF16(resid);
+  check_rows(resid, "resid");
+  CHK_DTYPE(rs, at::kFloat);
+  CHK_CONTIG(rs);
+  CHK_DTYPE(slab, at::kFloat);
+  CHK_CONTIG(slab);
+  TORCH_CHECK(rs.device() == resid.device() && slab.device() == resid.device() && rs.numel() >= resid.size(0), "rs [T] fp32");
+  TORCH_CHECK(slab.dim() == 3 && slab.size(0) >= 1 && slab.size(1) == resid.size(0) && slab.size(2) == resid.size(1), "slab [sk, T, hidden]");
+  TORCH_CHECK(resid.size(1) <= 8192, "hidden <= 8192");
+  HIP_OK(die::launch_rms_row_scale(rs.data_ptr<float>(), bf(resid), nullptr, (int)resid.size(0), (int)resid.size(1), resid.stride(0), 0,
+                                   (float)eps, cur_stream(), slab.data_ptr<float>(), (int)slab.size(0)));
+}
+
+// One dense product x [M, K] w [N, K]^T of a prompt step (bf16; moe_gemm.hip): into fp32 slabs y [sk, M, N], whose sum it is, or, with
+// w = [gate; up] and bf16 y [M, N / 2], silu(scale gate) scale up with a factor per row. tile_rows: 0, or the tiles to take.
+void dense_gemm(Tensor y, Tensor x, Tensor w, std::optional<Tensor> scale, int64_t tile_rows) {
+  CHK_CUDA(x);
+  CHK_BF16(x);
+  check_rows(x, "x");
+  CHK_BF16(w);
+  CHK_CONTIG(w);
+  CHK_CONTIG(y);
+  const bool slab = y.scalar_type() == at::kFloat;
+  TORCH_CHECK(w.dim() == 2 && w.size(1) == x.size(1) && w.device() == x.device() && y.device() == x.device(), "dense_gemm: w [N, K] of x's device");
+  TORCH_CHECK(y.dim() == (slab ? 3 : 2) && y.size(slab ? 1 : 0) == x.size(0) && y.size(-1) * (slab ? 1 : 2) == w.size(0) && (!slab || y.size(0) >= 1),
+              "dense_gemm: y [sk, M, N] fp32 or [M, N / 2] bf16");
+  die::MoeGemmArgs a{};
+  if (slab) {
+    TORCH_CHECK(!scale.has_value() && x.size(1) % (64 * y.size(0)) == 0, "dense_gemm: slabs of K / sk, a multiple of 64, and no scale");
+    a.slab = y.data_ptr<float>();
+  } else {
+    CHK_BF16(y);
+    a.out = static_cast<uint16_t*>(y.data_ptr());
+  }
+  if (scale.has_value()) {
+    CHK_DTYPE(*scale, at::kFloat);
+    CHK_CONTIG(*scale);
+    TORCH_CHECK(scale->numel() >= x.size(0) && scale->device() == x.device(), "dense_gemm: scale [M] fp32");
+    a.scale = scale->data_ptr<float>();
+  }
+  a.x = static_cast<const uint16_t*>(x.data_ptr());
+  a.ldx = x.stride(0);
+  a.w = static_cast<const uint16_t*>(w.data_ptr());
+  a.topk = 1;
+  a.act = slab ? die::MOE_ACT_NONE : die::MOE_ACT_SILU;
+  a.experts = slab ? (int)y.size(0) : 1;
+  a.rows = (int)x.size(0);
+  a.ncols = (int)y.size(-1);
+  a.K = (int)x.size(1);
+  a.tile_rows = (int)tile_rows;
+  TORCH_CHECK(die::moe_gemm_takes(a), "dense_gemm: sizes");
+  HIP_OK(die::launch_dense_gemm(a, cur_stream()));
+}
+
 void check_cache(const Tensor& c, int64_t hkv, int64_t head_dim, const char* name) {
   CHK_CUDA(c);
   CHK_BF16(c);
@@ -875,7 +932,8 @@ void fused_add_rms_norm_slab(Tensor out, Tensor slab, Tensor residual, Tensor w,
 }
 
 void rope_and_cache_slab(Tensor q_out, Tensor slab, Tensor positions, Tensor cos_sin, Tensor slot_mapping,
-                         Tensor k_cache, Tensor v_cache, int64_t hq, int64_t hkv, int64_t head_dim) {
+                         Tensor k_cache, Tensor v_cache, int64_t hq, int64_t hkv, int64_t head_dim,
+                         std::optional<Tensor> row_scale) {
   CHK_CUDA(slab);
   CHK_DTYPE(slab, at::kFloat);
   CHK_CONTIG(slab);
@@ -891,10 +949,16 @@ void rope_and_cache_slab(Tensor q_out, Tensor slab, Tensor positions, Tensor cos
   TORCH_CHECK(positions.numel() >= T && slot_mapping.numel() >= T, "positions/slots too short");
   check_cache(k_cache, hkv, head_dim, "k_cache");
   check_cache(v_cache, hkv, head_dim, "v_cache");
+  if (row_scale.has_value()) {
+    CHK_DTYPE(*row_scale, at::kFloat);
+    CHK_CONTIG(*row_scale);
+    TORCH_CHECK(row_scale->numel() >= T && row_scale->device() == slab.device(), "row_scale [T] fp32");
+  }
   HIP_OK(die::launch_rope_and_cache_slab(bf(q_out), slab.data_ptr<float>(), (int)slab.size(0),
                                           positions.data_ptr<int64_t>(), cos_sin.data_ptr<float>(),
                                           slot_mapping.data_ptr<int64_t>(), bf(k_cache), bf(v_cache), (int)T,
-                                          (int)hq, (int)hkv, (int)head_dim, (int)k_cache.size(2), cur_stream()));
+                                          (int)hq, (int)hkv, (int)head_dim, (int)k_cache.size(2), cur_stream(),
+                                          row_scale.has_value() ? row_scale->data_ptr<float>() : nullptr));
 }
 
 // ---- one-shot all-reduce over IPC-mapped peer buffers (src/parallel/custom_allreduce.py)
@@ -1089,7 +1153,11 @@ PYBIND11_MODULE(_C, m) {
   m.def("gemm_decode_grouped", &gemm_decode_grouped);
   m.def("gemm_decode_ids", &gemm_decode_ids);
   m.def("fused_add_rms_norm_slab", &fused_add_rms_norm_slab);
-  m.def("rope_and_cache_slab", &rope_and_cache_slab);
+  m.def("rope_and_cache_slab", &rope_and_cache_slab, py::arg("q_out"), py::arg("slab"), py::arg("positions"), py::arg("cos_sin"),
+        py::arg("slot_mapping"), py::arg("k_cache"), py::arg("v_cache"), py::arg("hq"), py::arg("hkv"), py::arg("head_dim"),
+        py::arg("row_scale") = py::none());
+  m.def("rms_row_scale_slab", &rms_row_scale_slab);
+  m.def("dense_gemm", &dense_gemm, py::arg("y"), py::arg("x"), py::arg("w"), py::arg("scale") = py::none(), py::arg("tile_rows") = 0);
   m.def("car_alloc", &car_alloc, py::arg("bytes"), py::arg("uncached") = true);
   m.def("car_tensor", &car_tensor);
   m.def("car_copy_to", &car_copy_to);

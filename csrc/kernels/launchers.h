@@ -25,8 +25,9 @@ hipError_t launch_silu_and_mul_views(bf16_t* out, int64_t ostride, const bf16_t*
                                      const float* row_scale = nullptr, int per = 0);
 // prefill RMSNorm as a row scale: resid += x (x optional; bf16, in place) and rs[row] = rsqrt(mean(resid^2) + eps)
 // of the rounded residual. Any number of rows; grid = rows
+// (with `slab`, the sum of fp32 split-K slabs [sk][rows][hidden] is added instead of x)
 hipError_t launch_rms_row_scale(float* rs, bf16_t* resid, const bf16_t* x, int rows, int hidden, int64_t rstride,
-                                int64_t xstride, float eps, hipStream_t s);
+                                int64_t xstride, float eps, hipStream_t s, const float* slab = nullptr, int sk = 0);
 
 hipError_t launch_rope_and_cache(bf16_t* qkv, int64_t qkv_stride, const int64_t* positions, const float* cos_sin,
                                  const int64_t* slot_mapping, bf16_t* k_cache, bf16_t* v_cache, int num_tokens,
@@ -185,7 +186,7 @@ hipError_t launch_fused_add_rms_norm_slab(bf16_t* out, const float* slab, int sk
 hipError_t launch_rope_and_cache_slab(bf16_t* q_out, const float* slab, int sk, const int64_t* positions,
                                       const float* cos_sin, const int64_t* slot_mapping, bf16_t* k_cache,
                                       bf16_t* v_cache, int num_tokens, int hq, int hkv, int head_dim, int block_size,
-                                      hipStream_t s);
+                                      hipStream_t s, const float* row_scale = nullptr);
 
 // one-shot all-reduce over IPC-mapped peer buffers (allreduce.hip)
 hipError_t launch_custom_all_reduce(const bf16_t* in, bf16_t* out, int64_t n, int rank, int world,

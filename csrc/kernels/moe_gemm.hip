@@ -74,6 +74,12 @@ __device__ __forceinline__ int scan64(int x, int lane) {
   return x + (lane >= 16 ? a : 0) + (lane >= 32 ? b : 0) + (lane >= 48 ? c : 0);
 }
 
+// the first row of expert i <= experts (without offsets every part has all rows, from 0 on); the rows of it
+__device__ __forceinline__ int first_row(const MoeGemmArgs& a, int i) { return a.offsets != nullptr ? a.offsets[min(i, a.experts)] : 0; }
+__device__ __forceinline__ int end_row(const MoeGemmArgs& a, int i) {
+  return a.offsets != nullptr ? a.offsets[min(i + 1, a.experts)] : i < a.experts ? a.rows : 0;
+}
+
 struct Tile {
   int e, n0, r0, M;   // expert, first output column, first of M rows
   int turn;           // the stage of K that it starts with
@@ -85,6 +91,7 @@ struct Tile {
 // half of the CUs idle (16 of 2048 x 1024, 256 rows: 33.0 / 34.6).
 __device__ __forceinline__ int first_stage(int n, int nst) { return (int)((uint64_t)((uint32_t)n * 2654435769u) * (uint32_t)nst >> 32); }
 __device__ __forceinline__ int stage_of(int s, int turn, int nst) { return s + turn >= nst ? s + turn - nst : s + turn; }
+__device__ __forceinline__ int stages(const MoeGemmArgs& a) { return a.slab != nullptr ? a.K / (BK * a.experts) : a.K / BK; }   // of a tile
 // The tiles of the launch, found from the offsets by every wave (lane i looks at experts i, i + 64, ...). Tiles of an expert are as even
 // as 32-row pieces allow, at most R rows. XCD i (blocks i, i + 8, ...) takes the i-th eighth of the list, whose neighbours share
 // weights or x rows; its CUs take turns. What is left for less than a turn of all of them is cut into `parts` by rows.
@@ -102,7 +109,7 @@ struct Plan {
     constexpr int NH = 5;   // heights 256, 224, .. 128: lanes 4 i + log2(parts)
     int n = 1, filled = 0;  // tiles of the lane's height; rows in whole 32-row pieces
     for (int b = 0; b < a.experts; b += 64) {
-      const int m = a.offsets[min(b + lane + 1, a.experts)] - a.offsets[min(b + lane, a.experts)];
+      const int m = end_row(a, b + lane) - first_row(a, b + lane);
       filled += 32 * __builtin_amdgcn_readlane(scan64((m + 31) / 32, lane), 63);
 #pragma unroll
       for (int i = 0; i < NH; ++i) {
@@ -141,7 +148,7 @@ struct Plan {
       int o0, o1, before, b = 0;
       uint64_t beyond;
       for (;; b += 64) {
-        o0 = a.offsets[min(b + lane, a.experts)], o1 = a.offsets[min(b + lane + 1, a.experts)];
+        o0 = first_row(a, b + lane), o1 = end_row(a, b + lane);
         const int own = (o1 - o0 + R - 1) / R * NT, upto = scan64(own, lane);
         beyond = __builtin_amdgcn_ballot_w64(upto > tile);
         before = upto - own;
@@ -160,7 +167,7 @@ struct Plan {
       tile -= g * gs * NT;
       const int h = (rows / 32 + cut - 1) / cut * 32, m0 = (g * gs + tile % gm) * rows + part * h;
       t.n0 = tile / gm;
-      t.turn = mts == 1 ? first_stage(t.e * NT + t.n0, a.K / BK) : 0;   // (used where the launch asks for it)
+      t.turn = mts == 1 ? first_stage(t.e * NT + t.n0, stages(a)) : 0;   // (used where the launch asks for it)
       t.M = min(min(t.M - m0, rows - part * h), h);
       t.r0 += m0;
       if (t.M > 0) return true;
@@ -216,14 +223,14 @@ template <int ACT, class Z> __device__ __forceinline__ void store_row16(Z z, uin
   }
 }
 
-template <int ACT, bool TURN>
+template <int ACT, bool TURN, bool SLAB = false>
 __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   constexpr bool GATED = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU;
   constexpr int NO = GATED ? BN / 2 : BN;           // output columns of a tile
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wn = wave % WN, wm = wave / WN, fr = lane & 15, lg = lane >> 4;
-  const int nst = a.K / BK;
+  const int nst = SLAB ? a.K / (BK * a.experts) : a.K / BK;
 
   const Plan plan(a, a.ncols / NO, lane);
   int job = (int)(blockIdx.x >> 3);
@@ -232,7 +239,7 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
 
   // ---- the wave's pieces of a unit: 8 rows each, 16-byte chunk c of row r at place c ^ swz(r)
   auto swz = [](int r) { return r >> 1 & 7; };
-  const char *wbase, *xbase = reinterpret_cast<const char*>(a.x);
+  const char *wbase, *xbase;
   uint32_t woff[PC], xoff[PC];
   int xr[PC];
   auto rows_of = [&](const Tile& u) {   // the x rows of the wave's pieces
@@ -246,7 +253,9 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
   int turn = 0;
   auto offsets_of = [&](const Tile& u) {
     turn = TURN ? u.turn : 0;
-    wbase = reinterpret_cast<const char*>(a.w) + (int64_t)u.e * (GATED ? 2 : 1) * a.ncols * a.K * 2;
+    const int64_t part = SLAB ? (int64_t)u.e * nst * ROWB : 0;   // of a row
+    wbase = reinterpret_cast<const char*>(a.w) + (SLAB ? part : (int64_t)u.e * (GATED ? 2 : 1) * a.ncols * a.K * 2);
+    xbase = reinterpret_cast<const char*>(a.x) + part;
 #pragma unroll
     for (int p = 0; p < PC; ++p) {
       const int r = 8 * (wave + NW * p) + lane / 8, col = 16 * (lane % 8 ^ swz(r));
@@ -363,6 +372,14 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       const int row = 32 * (2 * (m / 2) + wm) + 16 * (m % 2) + fr, rr = t.r0 + min(row, t.M - 1);
+      if constexpr (SLAB) {
+        float* sp = a.slab + ((int64_t)t.e * a.rows + rr) * a.ncols + t.n0 * NO + 32 * TN * wn + 4 * lg;
+        if (row < t.M) {
+#pragma unroll
+          for (int n = 0; n < NT; ++n) *reinterpret_cast<f32x4_t*>(sp + 16 * n) = acc[n][m];
+        }
+        continue;
+      }
       const float sc = a.scale != nullptr ? a.scale[a.sorted != nullptr ? a.sorted[rr] : rr] : 1.0f;
       uint16_t* op = a.out + (int64_t)rr * a.ncols + t.n0 * NO + (GATED ? 16 : 32) * TN * wn + 16 * (lg & 1) + 8 * (lg >> 1);
       store_row16<ACT>([&](int n, int i) __attribute__((always_inline)) { return acc[n][m][i] * sc; }, op, row < t.M, a);
@@ -400,18 +417,18 @@ constexpr int FN = 32 * TN, FUNIT = FN * ROWB;   // weight rows of a tile, bytes
 
 constexpr int FEW_LDS = 160 * 1024;
 
-template <int ACT, int NB>
+template <int ACT, int NB, bool SLAB = false>
 __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_few_kernel(MoeGemmArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   constexpr bool GATED = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU;
   constexpr int NO = (GATED ? FN / 2 : FN) * NB;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 31, hi = lane >> 5;
-  const int nst = a.K / BK, NT = a.ncols / NO;
+  const int nst = SLAB ? a.K / (BK * a.experts) : a.K / BK, NT = a.ncols / NO;
 
   // ---- the workgroup's tile: XCD i (blocks i, i + 8, ..) takes the i-th eighth of the list, whose neighbours share x rows or weights
   int total = 0;
   for (int b = 0; b < a.experts; b += 64) {
-    const int m = a.offsets[min(b + lane + 1, a.experts)] - a.offsets[min(b + lane, a.experts)];
+    const int m = end_row(a, b + lane) - first_row(a, b + lane);
     total += __builtin_amdgcn_readlane(scan64((m + BM - 1) / BM * NT, lane), 63);
   }
   const int per = (total + 7) / 8;
@@ -419,7 +436,7 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_few_kernel(MoeGemmArgs a)
   if ((int)(blockIdx.x >> 3) >= per || tile >= total) return;
   Tile t;
   for (int b = 0;; b += 64) {
-    const int o0 = a.offsets[min(b + lane, a.experts)], o1 = a.offsets[min(b + lane + 1, a.experts)];
+    const int o0 = first_row(a, b + lane), o1 = end_row(a, b + lane);
     const int own = (o1 - o0 + BM - 1) / BM * NT, upto = scan64(own, lane);
     const uint64_t beyond = __builtin_amdgcn_ballot_w64(upto > tile);
     if (beyond == 0) {   // (there is one: tile < total)
@@ -449,11 +466,11 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_few_kernel(MoeGemmArgs a)
     constexpr int MT = 2 * MX / MW, KS = BK / 16 / KG;   // 32-row tiles and 16-K steps of a wave
     const int wm = wave % MW, wn = wave / MW % NB, kg = wave / (MW * NB);
     // ---- the wave's pieces of a stage: 8 rows each, 16-byte chunk c of row r at place c ^ (r >> 1 & 7)
-    const int r8 = 8 * wave + lane / 8, col = 16 * (lane % 8 ^ (r8 >> 1 & 7));
+    const int r8 = 8 * wave + lane / 8, col = 16 * (lane % 8 ^ (r8 >> 1 & 7)) + (SLAB ? t.e * nst * ROWB : 0);
     const char* wp[NB];
 #pragma unroll
     for (int b = 0; b < NB; ++b)
-      wp[b] = reinterpret_cast<const char*>(a.w) + ((int64_t)t.e * (GATED ? 2 : 1) * a.ncols + t.n0 * NO + b * (NO / NB) +
+      wp[b] = reinterpret_cast<const char*>(a.w) + ((SLAB ? 0 : (int64_t)t.e * (GATED ? 2 : 1) * a.ncols) + t.n0 * NO + b * (NO / NB) +
                                                      (GATED ? (r8 & 32 ? a.ncols : 0) + r8 % 32 : r8)) * a.K * 2 + col;
     const char* xp[MX];
 #pragma unroll
@@ -538,6 +555,17 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_few_kernel(MoeGemmArgs a)
 #pragma unroll
           for (int i = 0; i < 16; ++i) acc[n][m][i] += sums[place(g, m, n, i)];
       const int row = 32 * (wm + MW * m) + fr, rr = t.r0 + min(row, t.M - 1);
+      if constexpr (SLAB) {   // (register 4 g + i: weight row 8 g + 4 hi + i)
+        float* sp = a.slab + ((int64_t)t.e * a.rows + rr) * a.ncols + t.n0 * NO + wn * FN + 4 * hi;
+        if (row < t.M) {
+#pragma unroll
+          for (int n = 0; n < TN; ++n)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+              *reinterpret_cast<f32x4_t*>(sp + 32 * n + 8 * g) = f32x4_t{acc[n][m][4 * g], acc[n][m][4 * g + 1], acc[n][m][4 * g + 2], acc[n][m][4 * g + 3]};
+        }
+        continue;
+      }
       const float sc = a.scale != nullptr ? a.scale[a.sorted != nullptr ? a.sorted[rr] : rr] : 1.0f;
       uint16_t* op = a.out + (int64_t)rr * a.ncols + t.n0 * NO + wn * (NO / NB) + 8 * hi;
       store_row<ACT>([&](int n, int i) __attribute__((always_inline)) { return acc[n][m][i] * sc; }, op, row < t.M, a);
@@ -559,13 +587,22 @@ inline int few_tiles(const MoeGemmArgs& a) {
   return a.rows <= (tiles <= 2 * a.cus ? 144 : 40) * (int64_t)a.experts ? ROWS_128 : ROWS_WHOLE;
 }
 
-template <int ACT, int NB> hipError_t launch_few(const MoeGemmArgs& a, hipStream_t s) {
-  auto* fn = moe_gemm_few_kernel<ACT, NB>;
+template <int ACT, int NB, bool SLAB = false> hipError_t launch_few(const MoeGemmArgs& a, hipStream_t s) {
+  auto* fn = moe_gemm_few_kernel<ACT, NB, SLAB>;
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, FEW_LDS);
   if (e != hipSuccess) return e;
   constexpr int NO = (ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU ? FN / 2 : FN) * NB;
-  const int64_t tiles = ((int64_t)std::min(a.experts, a.rows) + a.rows / BM) * (a.ncols / NO);   // at most
+  const int64_t mts = a.offsets == nullptr ? a.experts * (int64_t)((a.rows + BM - 1) / BM) : std::min(a.experts, a.rows) + a.rows / BM;   // at most
+  const int64_t tiles = mts * (a.ncols / NO);
   hipLaunchKernelGGL(fn, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(64 * NW), FEW_LDS, s, a);
+  return hipGetLastError();
+}
+
+template <int ACT, bool SLAB> hipError_t launch_whole(const MoeGemmArgs& a, bool turn, hipStream_t s) {
+  auto* fn = turn ? moe_gemm_kernel<ACT, true, SLAB> : moe_gemm_kernel<ACT, false, SLAB>;
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, NU * UNIT);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(fn, dim3(8 * std::max(a.cus / 8, 1)), dim3(64 * NW), NU * UNIT, s, a);
   return hipGetLastError();
 }
 
@@ -577,11 +614,14 @@ template <int ACT> hipError_t launch_act(MoeGemmArgs a, hipStream_t s) {
   // (at most one row tile per expert on average: the places cost 0.6 % where they are all the first, 8 of 4096 x 14336, 1024 rows each)
   constexpr int NO = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU ? BN / 2 : BN;
   const bool turn = a.rows <= (int64_t)BM * a.experts && 2 * (int64_t)a.experts * (a.ncols / NO) >= a.cus;
-  auto* fn = turn ? moe_gemm_kernel<ACT, true> : moe_gemm_kernel<ACT, false>;
-  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, NU * UNIT);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(fn, dim3(8 * std::max(a.cus / 8, 1)), dim3(64 * NW), NU * UNIT, s, a);
-  return hipGetLastError();
+  return launch_whole<ACT, false>(a, turn, s);
+}
+
+template <int ACT, bool SLAB> hipError_t launch_dense(const MoeGemmArgs& a, hipStream_t s) {
+  const bool one = a.rows <= BM;
+  if (a.tile_rows == ROWS_64) return launch_few<ACT, 1, SLAB>(a, s);
+  if (a.tile_rows == ROWS_128) return launch_few<ACT, 2, SLAB>(a, s);
+  return launch_whole<ACT, SLAB>(a, one, s);
 }
 
 }  // namespace
@@ -606,6 +646,21 @@ hipError_t launch_moe_gemm(const MoeGemmArgs& a, hipStream_t s) {
     case MOE_ACT_RELU2: return launch_act<MOE_ACT_RELU2>(a, s);
     default: return hipErrorInvalidValue;
   }
+}
+
+// Dense products of prompt steps of a few row tiles by the same kernels. 4096 weight rows are 16 - 32 tiles a row tile, so the parts of K are what fills the
+// chip: they go as the "experts" of one set of rows, each into an fp32 slab, which the pass behind the product (norm statistics, RoPE) sums. At 4096 x 14336
+// weights 129 rows take 34 us and 3.5 TB/s (34 with 7 parts, 38 with 4 of 64-row tiles), 442 55 (0.94 PFLOP/s), where the library's 64 x 64 and 64 x 128 tiles
+// take 55 and 86; the bound is the fetch of the tiles into LDS (10 TB/s). A gate and up product has tiles enough, and its activation on the sums saves
+// [rows, 2 ff] out and back: 442 rows of 4096 x 28672 105 -> 96. Which steps take it: prompt_slab_parts, prompt_silu_tiles in src/ops.
+hipError_t launch_dense_gemm(MoeGemmArgs a, hipStream_t s) {
+  if (a.rows == 0) return hipSuccess;
+  const bool slab = a.slab != nullptr;
+  if (a.rows < 0 || a.experts < 1 || a.topk != 1 || a.offsets != nullptr || a.sorted != nullptr || !moe_gemm_takes(a)) return hipErrorInvalidValue;
+  if (slab ? a.act != MOE_ACT_NONE || a.K % (BK * a.experts) != 0 : a.experts != 1 || a.act != MOE_ACT_SILU) return hipErrorInvalidValue;
+  if (a.tile_rows != 0 && a.tile_rows != ROWS_64 && a.tile_rows != ROWS_128 && (a.tile_rows < 128 || a.tile_rows > 256 || a.tile_rows % 32 != 0)) return hipErrorInvalidValue;
+  a.cus = num_cus();
+  return slab ? launch_dense<MOE_ACT_NONE, true>(a, s) : launch_dense<MOE_ACT_SILU, false>(a, s);
 }
 
 }  // namespace die

@@ -352,26 +352,46 @@ hipError_t launch_silu_and_mul(bf16_t* out, const bf16_t* in, int rows, int inte
 }
 
 // ----------------------------------------------------------------------------
-// Prefill RMSNorm as a row scale (the norm weight folded into Wqkv / Wgate_up): resid += x (optional, bf16,
-// in place) and rs[row] = rsqrt(mean(resid^2) + eps) of the rounded residual. The consumers apply rs to the
+// Prefill RMSNorm as a row scale (the norm weight folded into Wqkv / Wgate_up): resid += x (optional: bf16 rows, or the sum of
+// fp32 split-K slabs [sk][rows][hidden]; in place) and rs[row] = rsqrt(mean(resid^2) + eps) of the rounded residual. The consumers apply rs to the
 // projection's output rows (RoPE / KV write, the attention's Q load, SiLU * up), so no normalised copy of
 // the residual is written: 2 (3 with the add) x hidden x 2 bytes per row instead of 3 (4).
 // One workgroup per row; NC 16-byte chunks per thread, every load of the row in flight before the first use.
-template <int NC, bool ADD>
+template <int NC, int ADD>
 __global__ void __launch_bounds__(256) rms_row_scale_kernel(float* __restrict__ rs, bf16_t* __restrict__ resid,
                                                             const bf16_t* __restrict__ x, int hidden, int64_t rstride,
-                                                            int64_t xstride, float eps) {
+                                                            int64_t xstride, float eps,
+                                                            const float* __restrict__ slab, int sk) {
   __shared__ float red[4];
   const int64_t row = blockIdx.x;
   uint4* r = reinterpret_cast<uint4*>(resid + row * rstride);
-  const uint4* src = ADD ? reinterpret_cast<const uint4*>(x + row * xstride) : nullptr;
+  const uint4* src = ADD == 1 ? reinterpret_cast<const uint4*>(x + row * xstride) : nullptr;
   const int nchunk = hidden >> 3;
   uint4 rv[NC], xv[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     const int idx = min((int)threadIdx.x + c * 256, nchunk - 1);  // clamped, masked below
     rv[c] = r[idx];
-    if (ADD) xv[c] = src[idx];
+    if (ADD == 1) xv[c] = src[idx];
+  }
+  float4 sum[NC][2];
+  if (ADD == 2) {
+    const float4* p = reinterpret_cast<const float4*>(slab + row * hidden);
+    const int64_t step = (int64_t)gridDim.x * hidden / 4;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      const int idx = min((int)threadIdx.x + c * 256, nchunk - 1);
+      sum[c][0] = p[2 * idx], sum[c][1] = p[2 * idx + 1];
+    }
+#pragma unroll 4
+    for (int k = 1; k < sk; ++k)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        const int idx = min((int)threadIdx.x + c * 256, nchunk - 1);
+        const float4 u = p[k * step + 2 * idx], v = p[k * step + 2 * idx + 1];
+        sum[c][0].x += u.x, sum[c][0].y += u.y, sum[c][0].z += u.z, sum[c][0].w += u.w;
+        sum[c][1].x += v.x, sum[c][1].y += v.y, sum[c][1].z += v.z, sum[c][1].w += v.w;
+      }
   }
   float ss = 0.f;
 #pragma unroll
@@ -380,9 +400,14 @@ __global__ void __launch_bounds__(256) rms_row_scale_kernel(float* __restrict__ 
     if (idx < nchunk) {
       float a[8];
       unpack8(rv[c], a);
-      if (ADD) {
+      if (ADD != 0) {
         float b[8];
-        unpack8(xv[c], b);
+        if (ADD == 1) {
+          unpack8(xv[c], b);
+        } else {
+          const float4 u = sum[c][0], v = sum[c][1];
+          b[0] = u.x, b[1] = u.y, b[2] = u.z, b[3] = u.w, b[4] = v.x, b[5] = v.y, b[6] = v.z, b[7] = v.w;
+        }
 #pragma unroll
         for (int j = 0; j < 8; ++j) a[j] += b[j];
         const uint4 p = pack8(a);
@@ -401,19 +426,22 @@ __global__ void __launch_bounds__(256) rms_row_scale_kernel(float* __restrict__ 
 }
 
 hipError_t launch_rms_row_scale(float* rs, bf16_t* resid, const bf16_t* x, int rows, int hidden, int64_t rstride,
-                                int64_t xstride, float eps, hipStream_t s) {
+                                int64_t xstride, float eps, hipStream_t s, const float* slab, int sk) {
   if (rows == 0) return hipSuccess;
   if (hidden % 8) return hipErrorInvalidValue;
   const int nc = (hidden / 8 + 255) / 256;
   dim3 grid(rows), block(256);
 #define RR_CASE(N)                                                                                             \
   case N:                                                                                                     \
-    if (x != nullptr)                                                                                         \
-      hipLaunchKernelGGL((rms_row_scale_kernel<N, true>), grid, block, 0, s, rs, resid, x, hidden, rstride,     \
-                         xstride, eps);                                                                       \
+    if (slab != nullptr)                                                                                      \
+      hipLaunchKernelGGL((rms_row_scale_kernel<N, 2>), grid, block, 0, s, rs, resid, x, hidden, rstride,        \
+                         xstride, eps, slab, sk);                                                             \
+    else if (x != nullptr)                                                                                    \
+      hipLaunchKernelGGL((rms_row_scale_kernel<N, 1>), grid, block, 0, s, rs, resid, x, hidden, rstride,        \
+                         xstride, eps, slab, sk);                                                             \
     else                                                                                                      \
-      hipLaunchKernelGGL((rms_row_scale_kernel<N, false>), grid, block, 0, s, rs, resid, x, hidden, rstride,    \
-                         xstride, eps);                                                                       \
+      hipLaunchKernelGGL((rms_row_scale_kernel<N, 0>), grid, block, 0, s, rs, resid, x, hidden, rstride,        \
+                         xstride, eps, slab, sk);                                                             \
     break;
   switch (nc) {
     RR_CASE(1)

@@ -103,7 +103,7 @@ hipError_t launch_rope_and_cache(bf16_t* qkv, int64_t qkv_stride, const int64_t*
 }
 
 // Same op fed by fp32 split-K slabs [sk][T][(hq+2hkv)*D] of the decode QKV
-// GEMM: the slabs are summed here, q is written (bf16) to q_out [T][hq*D].
+// GEMM: the slabs are summed here (and scaled by the token's row_scale, if there is one), q is written (bf16) to q_out [T][hq*D].
 template <int D>
 __global__ void __launch_bounds__(256) rope_cache_slab_kernel(bf16_t* __restrict__ q_out,
                                                               const float* __restrict__ slab, int sk,
@@ -112,7 +112,7 @@ __global__ void __launch_bounds__(256) rope_cache_slab_kernel(bf16_t* __restrict
                                                               const int64_t* __restrict__ slot_mapping,
                                                               bf16_t* __restrict__ k_cache,
                                                               bf16_t* __restrict__ v_cache, int T, int hq, int hkv,
-                                                              int block_size) {
+                                                              int block_size, const float* __restrict__ row_scale) {
   constexpr int HALF = D / 2;
   constexpr int RC = HALF / 8;
   constexpr int VC = D / 8;
@@ -123,6 +123,7 @@ __global__ void __launch_bounds__(256) rope_cache_slab_kernel(bf16_t* __restrict
   const int64_t pos = positions[tok];
   const int64_t slot = slot_mapping ? slot_mapping[tok] : -1;
   const float* cs = cos_sin + pos * D;
+  const float rsc = row_scale != nullptr ? row_scale[tok] : 1.0f;
   const int n_rot = (hq + hkv) * RC;
   const int n_items = n_rot + hkv * VC;
   auto sum8 = [&](int off, float* v) {
@@ -134,6 +135,8 @@ __global__ void __launch_bounds__(256) rope_cache_slab_kernel(bf16_t* __restrict
       v[0] += a.x; v[1] += a.y; v[2] += a.z; v[3] += a.w;
       v[4] += b.x; v[5] += b.y; v[6] += b.z; v[7] += b.w;
     }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] *= rsc;
   };
   for (int it = threadIdx.x; it < n_items; it += blockDim.x) {
     if (it < n_rot) {
@@ -176,17 +179,17 @@ __global__ void __launch_bounds__(256) rope_cache_slab_kernel(bf16_t* __restrict
 hipError_t launch_rope_and_cache_slab(bf16_t* q_out, const float* slab, int sk, const int64_t* positions,
                                       const float* cos_sin, const int64_t* slot_mapping, bf16_t* k_cache,
                                       bf16_t* v_cache, int num_tokens, int hq, int hkv, int head_dim, int block_size,
-                                      hipStream_t s) {
+                                      hipStream_t s, const float* row_scale) {
   if (num_tokens == 0) return hipSuccess;
   dim3 grid(num_tokens), block(256);
   switch (head_dim) {
     case 64:
       hipLaunchKernelGGL(rope_cache_slab_kernel<64>, grid, block, 0, s, q_out, slab, sk, positions, cos_sin,
-                         slot_mapping, k_cache, v_cache, num_tokens, hq, hkv, block_size);
+                         slot_mapping, k_cache, v_cache, num_tokens, hq, hkv, block_size, row_scale);
       break;
     case 128:
       hipLaunchKernelGGL(rope_cache_slab_kernel<128>, grid, block, 0, s, q_out, slab, sk, positions, cos_sin,
-                         slot_mapping, k_cache, v_cache, num_tokens, hq, hkv, block_size);
+                         slot_mapping, k_cache, v_cache, num_tokens, hq, hkv, block_size, row_scale);
       break;
     default:
       return hipErrorInvalidValue;

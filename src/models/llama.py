@@ -434,11 +434,14 @@ class CausalLM:
         # one GPU (no all-reduce between a projection and its residual add): o and down add into the residual in
         # the GEMM epilogue, and the norm pass only reads the residual for its statistics
         gemm_resid = self.prefill_gemm_residual and not self.tp.enabled and not a.is_moe
+        # steps of few row tiles take o and down as fp32 split-K slabs instead, which the norm pass adds
         rs = ops.rms_row_scale(residual, None, eps)
-        h = None
+        h = slab = None
         last = len(self.layers) - 1
         for li, lw in enumerate(self.layers):
-            if li > 0:
+            if slab is not None:
+                rs = ops.rms_row_scale_slab(residual, slab, eps, out=rs)
+            elif li > 0:
                 rs = ops.rms_row_scale(residual, h, eps, out=rs)
             if li == last and meta.keep_rows is not None:
                 return self._last_layer_kept_rows(lw, residual, residual, positions, meta, kv_pool, rs=rs)
@@ -446,10 +449,16 @@ class CausalLM:
             if meta.kv_hook is not None:
                 meta.kv_hook(li)
             if gemm_resid:
-                ops.linear_residual(residual, attn, lw.o)
-                rs2 = ops.rms_row_scale(residual, None, eps)
-                act = ops.silu_and_mul(ops.linear(residual, lw.gate_up), row_scale=rs2)
-                ops.linear_residual(residual, act, lw.down)
+                slab = ops.prompt_slab(attn, lw.o)
+                if slab is None:
+                    ops.linear_residual(residual, attn, lw.o)
+                    rs2 = ops.rms_row_scale(residual, None, eps)
+                else:
+                    rs2 = ops.rms_row_scale_slab(residual, slab, eps)
+                act = ops.prompt_silu_mul(residual, lw.gate_up, rs2)
+                slab = ops.prompt_slab(act, lw.down)
+                if slab is None:
+                    ops.linear_residual(residual, act, lw.down)
                 continue
             o = self.tp.all_reduce(ops.linear(attn, lw.o))
             if a.is_moe:
@@ -459,6 +468,8 @@ class CausalLM:
                 rs2 = ops.rms_row_scale(residual, o, eps)
                 act = ops.silu_and_mul(ops.linear(residual, lw.gate_up), row_scale=rs2)
                 h = self.tp.all_reduce(ops.linear(act, lw.down))
+        if slab is not None:
+            return ops.fused_add_rms_norm_slab(slab, residual, self.norm, eps)
         if h is None:
             return ops.rms_norm(residual, self.norm, eps)
         return ops.fused_add_rms_norm(h, residual, self.norm, eps)
@@ -477,11 +488,8 @@ class CausalLM:
         li = len(self.layers) - 1
         keep = meta.keep_rows
         n = keep.numel()
-        qkv = ops.linear(x, lw.qkv)
         k_cache, v_cache = kv_pool[li, 0], kv_pool[li, 1]
-        fuse_q = qkv.is_cuda
-        ops.rope_and_cache(qkv, positions, self.cos_sin, meta.slot_mapping, k_cache, v_cache, hq, hkv, d,
-                           rot_q=not fuse_q, row_scale=rs)
+        qkv, fuse_q, rs = self._project_qkv(lw, x, positions, meta, k_cache, v_cache, rs)
         if meta.kv_hook is not None:
             meta.kv_hook(li)
         if n == 0:
@@ -500,18 +508,30 @@ class CausalLM:
         h = self.tp.all_reduce(self._mlp(lw, x2))
         return ops.fused_add_rms_norm(h, res, self.norm, eps)
 
+    def _project_qkv(self, lw: LayerWeights, x: torch.Tensor, positions: torch.Tensor, meta: AttnMetadata, k_cache: torch.Tensor,
+                     v_cache: torch.Tensor, rs: Optional[torch.Tensor]):
+        """The qkv projection, k and v into the cache: (rows that start with q, whether the attention has to rotate q, the scale that it has to
+        apply to q). Prefill on the GPU leaves q to the attention kernel's load (no q round trip through HBM), except in steps of few rows,
+        whose projection comes as split-K slabs that the RoPE kernel sums."""
+        d, hq, hkv = self.head_dim, self.hq, self.hkv
+        slab = ops.prompt_slab(x, lw.qkv, residual=False) if rs is not None else None
+        if slab is not None:
+            q = ops.rope_and_cache_slab(slab, positions, self.cos_sin, meta.slot_mapping, k_cache, v_cache, hq, hkv, d, row_scale=rs)
+            return q, False, None
+        qkv = ops.linear(x, lw.qkv)
+        fuse_q = meta.is_prefill and qkv.is_cuda
+        ops.rope_and_cache(qkv, positions, self.cos_sin, meta.slot_mapping, k_cache, v_cache, hq, hkv, d,
+                           rot_q=not fuse_q, row_scale=rs)
+        return qkv, fuse_q, rs
+
     def _attention(self, li: int, lw: LayerWeights, x: torch.Tensor, positions: torch.Tensor, meta: AttnMetadata,
                    kv_pool: torch.Tensor, rs: Optional[torch.Tensor] = None) -> torch.Tensor:
         """qkv projection, RoPE + paged KV write, paged attention (prefill or decode) -> [T, hq*d].
         rs (GPU prefill): x is the raw residual and rs its per-token RMSNorm scale, applied to k / v in the
         KV write and to q in the attention's Q load."""
         d, hq, hkv = self.head_dim, self.hq, self.hkv
-        qkv = ops.linear(x, lw.qkv)
         k_cache, v_cache = kv_pool[li, 0], kv_pool[li, 1]
-        # prefill on the GPU: q's RoPE happens in the attention kernel's Q load (no q round trip through HBM)
-        fuse_q = meta.is_prefill and qkv.is_cuda
-        ops.rope_and_cache(qkv, positions, self.cos_sin, meta.slot_mapping, k_cache, v_cache, hq, hkv, d,
-                           rot_q=not fuse_q, row_scale=rs)
+        qkv, fuse_q, rs = self._project_qkv(lw, x, positions, meta, k_cache, v_cache, rs)
         q = qkv[:, : hq * d]
         if meta.is_prefill:
             return ops.attn_prefill(q, k_cache, v_cache, meta.block_tables, meta.cu_q, meta.ctx_lens,

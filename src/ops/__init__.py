@@ -8,6 +8,7 @@ which lets the engine's control flow run in CPU-only tests.
 
 from __future__ import annotations
 
+import functools
 import os
 from typing import Optional
 
@@ -115,6 +116,14 @@ def rms_row_scale(resid: torch.Tensor, x: Optional[torch.Tensor], eps: float,
         out.copy_(torch.rsqrt(resid.float().pow(2).mean(-1) + eps))
         return out
     _kern().rms_row_scale(out, resid, x if x is not None else _empty(resid.device), float(eps))
+    return out
+
+
+def rms_row_scale_slab(resid: torch.Tensor, slab: torch.Tensor, eps: float, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """:func:`rms_row_scale` after resid += slab.sum(0), the split-K slabs [sk, T, hidden] of :func:`prompt_slab` (fp32 sums, one rounding)."""
+    if out is None:
+        out = torch.empty(resid.shape[0], dtype=torch.float32, device=resid.device)
+    _kern().rms_row_scale_slab(out, resid, slab, float(eps))
     return out
 
 
@@ -700,6 +709,76 @@ def linear_residual(resid: torch.Tensor, x: torch.Tensor, w: torch.Tensor) -> to
     return resid.addmm_(x, w.t())
 
 
+def _dense_gemm_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether csrc/kernels/moe_gemm.hip takes x @ w^T as one dense product of a prompt step."""
+    return (x.is_cuda and x.shape[0] > DECODE_GEMM_MAX_M and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous()
+            and w.shape[0] % 256 == 0 and x.shape[1] % 64 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and max(2 * w.numel(), x.shape[0] * x.stride(0)) < 1 << 31)
+
+
+@functools.lru_cache(maxsize=None)
+def _num_cus(device: int) -> int:
+    return torch.cuda.get_device_properties(device).multi_processor_count
+
+
+def slab_parts(m: int, n: int, k: int, cus: int):
+    """(parts of K, tile code) of :func:`prompt_slab`: tiles of 128 weight rows by all of up to 256 rows, above that of 256 by up to 256, and as
+    many parts of K as leave no compute unit two of them (at most 8, whole stages of 64; 16 of 1024 x 1024: 14.5 us instead of 11.9)."""
+    tiles, code = (n // 128, 96) if m <= 256 else (n // 256 * -(-m // 256), 0)
+    return max(d for d in range(1, 9) if d == 1 or (k % (64 * d) == 0 and tiles * d <= cus)), code
+
+
+def prompt_slab_parts(m: int, n: int, k: int, cus: int, residual: bool):
+    """:func:`slab_parts` where slabs are faster than the library's product, else None. us, the library / slabs, each with its consumer (the
+    library's tiles of few rows and 4096 columns or so leave compute units idle; slabs cost 8 sk m n bytes beside 2 m n k operations, so the line
+    goes with k):
+      4096 x 14336   129 rows 57 / 40, 256 65 / 49, 400 84 / 63, 768 110 / 88, 1024 135 / 113, 1500 171 / 151, 2048 206 / 200 (2300: one part, 241 / 246)
+      8192 x 28672   129 307 / 121, 400 300 / 185, 1024 384 / 365          8192 x 8192   256 83 / 55, 512 83 / 82, 700 101 / 95, 1024 121 / 127
+      4096 x 4096    129 35 / 25, 200 34 / 26, 256 26 / 29, 300 30 / 32, 512 34 / 35
+      qkv 6144 x 4096  129 43 / 29, 192 36 / 31, 256 43 / 34, 300 32 / 38   10240 x 8192, two parts   129 56 / 63, 256 92 / 80"""
+    sk, code = slab_parts(m, n, k, cus)
+    most = (224 if k < 8192 else 768 if k < 12288 else 1 << 31) if residual else 256
+    return None if m > most or sk < (2 if residual else 4) else (sk, code)
+
+
+def prompt_slab(x: torch.Tensor, w: torch.Tensor, residual: bool = True) -> Optional[torch.Tensor]:
+    """fp32 split-K slabs [sk, M, N] of x @ w^T for a prompt step of more than 128 rows, for a consumer that sums them (rms_row_scale_slab;
+    residual=False: rope_and_cache_slab), or None where the library product is the faster one."""
+    if not _dense_gemm_ok(x, w):
+        return None
+    m, k, n = x.shape[0], x.shape[1], w.shape[0]
+    plan = prompt_slab_parts(m, n, k, _num_cus(x.device.index), residual)
+    if plan is None:
+        return None
+    slab = torch.empty(plan[0], m, n, dtype=torch.float32, device=x.device)
+    _kern().dense_gemm(slab, x, w, None, plan[1])
+    return slab
+
+
+def prompt_silu_tiles(m: int, inter: int, k: int, cus: int) -> Optional[int]:
+    """Tile code of :func:`prompt_silu_mul`'s own product, or None for the library's. us, the library's with silu_and_mul / tiles of 256 weight
+    rows / of 128:
+      28672 x 4096   129 rows 61 / 65 / 58, 161 66 / 68 / 59, 200 72 / 75 / 77, 256 76 / 78 / 79, 257 80 / 78 / 109, 512 107 / 105, 768 171 / 167,
+                     1200 268 / 253, 2048 394 / 381, 3000 582 / 563, 4096 706 / 724, 8192 1418 / 1430
+      57344 x 8192   129 201 / 189 / 242, 256 224 / 245, 400 386 / 370, 700 576 / 555, 1024 780 / 732, 2048 1357 / 1370
+    One row tile leaves CUs idle or reads x for every 128 weight rows: to 168 rows tiles of 128 that fill the chip once, then the library to 256."""
+    if m <= 168:
+        return 96 if inter // 64 <= cus else 0
+    return None if m <= 256 or m > (3072 if inter * k <= 1 << 26 else 1536) else 0
+
+
+def prompt_silu_mul(x: torch.Tensor, w_gate_up: torch.Tensor, row_scale: torch.Tensor) -> torch.Tensor:
+    """silu(s x @ gate^T) * (s x @ up^T) of a prompt step, s the rows' scale (:func:`rms_row_scale`), w_gate_up = [gate; up]: one product with
+    the activation on its fp32 sums (rounded once), or the library's and :func:`silu_and_mul`."""
+    m, inter = x.shape[0], w_gate_up.shape[0] // 2
+    code = prompt_silu_tiles(m, inter, x.shape[1], _num_cus(x.device.index)) if _dense_gemm_ok(x, w_gate_up) else None
+    if code is None:
+        return silu_and_mul(linear(x, w_gate_up), row_scale=row_scale)
+    out = torch.empty(m, inter, dtype=x.dtype, device=x.device)
+    _kern().dense_gemm(out, x, w_gate_up, row_scale, code)
+    return out
+
+
 def linear_tiled(x: torch.Tensor, w: torch.Tensor, wr: int, kc: int) -> torch.Tensor:
     """y = x @ w^T (bf16, decode sizes) with w packed by gd_pack_weights for the (wr, kc) tile."""
     return gemm_decode(x, w, 0 | 32, wr, 1, kc=kc)
@@ -746,13 +825,14 @@ def fused_add_rms_norm_slab(slab: torch.Tensor, residual: torch.Tensor, w: torch
 
 
 def rope_and_cache_slab(slab, positions, cos_sin, slot_mapping, k_cache, v_cache, hq: int, hkv: int,
-                        head_dim: int, q_out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """Sum the QKV split-K slabs, rotate q/k, write k/v into the paged cache;
-    returns q [T, hq*D] (bf16)."""
+                        head_dim: int, q_out: Optional[torch.Tensor] = None,
+                        row_scale: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Sum the QKV split-K slabs (times the token's row_scale [T], if given), rotate q/k, write k/v into the paged
+    cache; returns q [T, hq*D] (bf16)."""
     t = slab.shape[1]
     if q_out is None:
         q_out = torch.empty(t, hq * head_dim, dtype=torch.bfloat16, device=slab.device)
-    _kern().rope_and_cache_slab(q_out, slab, positions, cos_sin, slot_mapping, k_cache, v_cache, hq, hkv, head_dim)
+    _kern().rope_and_cache_slab(q_out, slab, positions, cos_sin, slot_mapping, k_cache, v_cache, hq, hkv, head_dim, row_scale)
     return q_out
 
 
