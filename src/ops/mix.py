@@ -210,10 +210,11 @@ _MOE_ACT = {ACT_SILU: MOE_SILU, ACT_CLAMPED: MOE_CLAMPED, ACT_GELU_TANH: MOE_GEL
 
 
 # Rows per expert and elements of an expert's matrix from which a library GEMM pair per expert, behind a host read of the offsets,
-# is faster than the grouped product (eight experts, us, library / grouped; 4096 x 14336: 1024 rows 3131 / 2907, 1280 rows 3663 / 3470,
-# 1500 rows 3910 / 3799, 2048 rows 5332 / 5469, 4096 rows 10262 / 10633; smaller experts never: 4096 x 4096, 2048 rows 1745 / 1609,
-# 4096 rows 3491 / 3145; 4096 x 2048, 8192 rows 3378 / 3200; 2048 x 2048, 4096 rows 1088 / 906)
-GROUPED_MAX_ROWS, GROUPED_ANY_ROWS_SIZE = 1792, 1 << 25
+# is taken instead of the grouped product. The whole layer, us, library / grouped: eight experts of 4096 x 14336, 1792 rows each 4732 / 4005, 2048 rows
+# 5421 / 4725, 3000 rows 7015 / 6609, 4096 rows 9575 / 8828, 8192 rows 18045 / 17817; eight of 6144 x 16384, 3000 rows 14343 / 11084, 8192 rows 29954 /
+# 29456; sixteen of 4096 x 8192, 2048 rows 6219 / 5281, 8192 rows 21028 / 20437; four of 8192 x 8192, 10000 rows 12032 / 12257, 12288 rows 14209 / 15207. Smaller
+# experts keep the grouped one at any rows.
+GROUPED_MAX_ROWS, GROUPED_ANY_ROWS_SIZE = 8704, 1 << 25
 
 
 DECODE_EXPERTS_MAX_T = 128   # tokens of a decode step whose experts stream through the decode products
