@@ -39,15 +39,17 @@ namespace die {
 
 using namespace attn;
 
-// grid = (q tiles, num_seqs, hkv); block = 64 NW (NW waves, 32 query rows each); dynamic LDS =
-// 2 * NS * KV_TILE. NS: 32-key sub-tiles per pipeline stage (one barrier and one round of global loads
+// grid = (q tiles, num_seqs, hkv); block = 64 NW KG (NW waves, 32 query rows each, KG times); dynamic LDS =
+// 2 * NS * KV_TILE * KG. NS: 32-key sub-tiles per pipeline stage (one barrier and one round of global loads
 // per stage): NS = 2 halves the barriers and doubles the bytes in flight per round.
 // NW: every key / value byte staged into LDS is used by NW x 32 query rows, so L2 -> LDS traffic per
 // FLOP falls as 1 / NW. At NW = 4 (two workgroups per CU) the staging skeleton alone — loads, LDS
 // writes, barriers, no math — took 423 of 931 us at 4 x 4,096 (about 10 TB/s of L2 reads); NW = 8 (one
 // 512-thread workgroup per CU, the same 8 waves) halves that traffic.
-template <int G, int NS, int NW>
-__global__ void __launch_bounds__(64 * NW, 8 / NW) attn_prefill_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
+// KG: groups of NW waves that take the stages in turn, each with a ring of its own; their sums meet at the end. For steps of few row tiles, whose chain of
+// stages (1.5 - 2.5 us each 64 keys) is all that runs.
+template <int G, int NS, int NW, int KG = 1>
+__global__ void __launch_bounds__(64 * NW * KG, 8 / (NW * KG)) attn_prefill_kernel(bf16_t* __restrict__ out, const bf16_t* __restrict__ q,
                                                            int64_t q_stride, const bf16_t* __restrict__ k_cache,
                                                            const bf16_t* __restrict__ v_cache,
                                                            const int* __restrict__ block_tables, int bt_stride,
@@ -58,7 +60,9 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) attn_prefill_kernel(bf16_t* _
                                                            const float* __restrict__ q_scale) {
   constexpr int TPW = 32 / G;   // tokens per wave
   constexpr int TPB = NW * TPW;  // tokens per workgroup
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+  extern __shared__ __attribute__((aligned(16))) char smem_all[];
+  const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / (64 * NW)) : 0;
+  char* const smem = smem_all + kg * (2 * NS * KV_TILE);   // the group's ring
   // XCD-aware order: workgroups are dealt round-robin over the 8 XCDs (hardware id mod 8), so the
   // q tiles of one (sequence, kv head), which all stream the same K/V, would each land on a different
   // L2. Remap (bijectively) so that every XCD gets a contiguous run of logical ids: a group's tiles
@@ -73,7 +77,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) attn_prefill_kernel(bf16_t* _
   if (t0 >= qlen) return;
   const int ctx = ctx_lens[seq];
   const int pos0 = ctx - qlen;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5;
+  const int tid = threadIdx.x - kg * (64 * NW), lane = tid & 63, wave = tid >> 6, h = lane >> 5;
   const int row = lane & 31;
   const int tok = t0 + wave * TPW + row / G;
   const int head = kvh * G + row % G;
@@ -81,7 +85,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) attn_prefill_kernel(bf16_t* _
   const int kv_len_row = min(ctx, pos0 + min(tok, qlen - 1) + 1);
   const int kv_end = min(ctx, pos0 + min(t0 + TPB, qlen));
   constexpr int ST = NS * KT;  // keys per stage
-  const int ntiles = (kv_end + ST - 1) / ST;
+  const int ntiles = (kv_end + ST * KG - 1) / (ST * KG);   // a group's; its stage kt is the workgroup's stage kt KG + kg
   const int wave_last_tok = min(t0 + wave * TPW + TPW, qlen) - 1;
   const int wave_kv_end = pos0 + wave_last_tok + 1;
   // the wave's first row sees keys [0, pos0 + first token + 1); tiles below that need no causal mask
@@ -127,12 +131,12 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) attn_prefill_kernel(bf16_t* _
   u32x4_t kA[NP], vA[NP], kB[NP], vB[NP];
   auto load_one = [&](int kt, auto I, u32x4_t* kreg, u32x4_t* vreg) __attribute__((always_inline)) {
     constexpr int i = decltype(I)::value;
-    const int key = kt * ST + kr + RPP * i;
+    const int key = (kt * KG + kg) * ST + kr + RPP * i;
     // a wave stages 4 consecutive keys (4-aligned, block_size is a multiple of 16), all in one block: the
     // block id is wave-uniform, read by a scalar load instead of a per-lane dependent load. Keys past
     // kv_end re-read row kv_end - 1 of the same block: finite values the causal mask zeroes, and no
     // branch, so the wait counter stays exact with two sets in flight.
-    const int kb = __builtin_amdgcn_readfirstlane(min(kt * ST + RPP * i + (kr & ~3), kv_end - 1) / block_size);
+    const int kb = __builtin_amdgcn_readfirstlane(min((kt * KG + kg) * ST + RPP * i + (kr & ~3), kv_end - 1) / block_size);
     const int64_t blk = bt[kb];
     const int64_t roff = ((blk * hkv + kvh) * block_size + min(key, kv_end - 1) % block_size) * D + c * 8;
     kreg[i] = *reinterpret_cast<const u32x4_t*>(k_cache + roff);
@@ -151,7 +155,7 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) attn_prefill_kernel(bf16_t* _
   auto compute = [&](int kt, int cur) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < NS; ++j) {
-      const int kb0 = kt * ST + j * KT;
+      const int kb0 = (kt * KG + kg) * ST + j * KT;
       if (kb0 < wave_kv_end) {  // wave-uniform: sub-tile not entirely in this wave's causal future
         const char* kl = smem + (cur * NS + j) * KV_TILE;
         f32x16_t s = qk_lds(kl, qf, lane);
@@ -189,6 +193,33 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) attn_prefill_kernel(bf16_t* _
   }
 #undef LOAD_STAGE
 #undef STORE_STAGE
+  if constexpr (KG > 1) {   // the groups' sums meet behind the first group's rows of results (the loop's last barrier freed the rings)
+    constexpr int PER = 66 * 64;   // floats of a wave
+    float* const sums = reinterpret_cast<float*>(smem_all + NW * 32 * 272) + lane;
+    if (kg > 0) {
+      float* to = sums + ((kg - 1) * NW + wave) * PER;
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) to[(16 * db + r) * 64] = st.o[db][r];
+      to[64 * 64] = st.m;
+      to[65 * 64] = st.l;
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int g = 1; g < KG; ++g) {   // (the first group has seen the first key, so its maximum is finite)
+      const float* from = sums + ((g - 1) * NW + wave) * PER;
+      const float m2 = from[64 * 64], mn = fmaxf(st.m, m2);
+      const float f1 = __builtin_amdgcn_exp2f(st.m - mn), f2 = __builtin_amdgcn_exp2f(m2 - mn);
+      st.l = st.l * f1 + from[65 * 64] * f2;
+      st.m = mn;
+#pragma unroll
+      for (int db = 0; db < 4; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) st.o[db][r] = st.o[db][r] * f1 + from[(16 * db + r) * 64] * f2;
+    }
+  }
 
   // Epilogue: O staged through LDS and stored as whole rows. Stored straight from the MFMA layout, every
   // 8-byte lane store touched 32 rows (32 partial lines per instruction) and the store tail cost ~45 us
@@ -764,18 +795,28 @@ hipError_t launch_attn_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, c
   // for short ones, where more, shorter q tiles fill the chip (64 x 256: 119 vs 132 us; 32 x 512 within 1.5 %:
   // profiles/r5_prefill_attn_nw_ns.jsonl)
   const bool short_q = max_q_len <= 256;
-  const int NWr = short_q ? 4 : 8, NSr = short_q ? 1 : 2;
+  // Where row tiles leave compute units idle, or next to that behind many keys, the chain of a tile's stages is what takes the time, and two groups of 4
+  // waves share it. One group / two, us, 32 heads in 8 groups: 1 x 200 11.7 / 11.4, 1 x 300 16.5 / 13.9, 1 x 442 20.8 / 16.8, 1 x 1000 37.9 / 29.3, 1 x 300
+  // behind 1500 60.9 / 43.6, 2 x 500 23.2 / 18.9; up to two tiles per CU 1 x 1500 53 / 40, 1 x 2048 71 / 60, 2 x 1000 40 / 38, but 3 x 500 27 / 32, 4 x 512 26 / 34;
+  // of few keys 4 x 128 9.7 / 10.3, 1 x 129 9.5 / 10.1; beyond, 1 x 4096 160 / 197. (Four groups of 2 waves 1 x 1000 34, two of them 31.)
+  const int tpb4 = 4 * (32 / (G > 32 ? 32 : G));
+  const int64_t tiles4 = (int64_t)((max_q_len + tpb4 - 1) / tpb4) * num_seqs * hkv, cus = num_cus();
+  const bool two = (tiles4 <= cus && max_q_len >= 200) || (tiles4 <= 2 * cus && max_q_len >= 1000);
+  const int NWr = short_q || two ? 4 : 8, NSr = short_q || two ? 1 : 2, KGr = two ? 2 : 1;
   const int tpb = NWr * (32 / (G > 32 ? 32 : G));
-  dim3 grid((max_q_len + tpb - 1) / tpb, num_seqs, hkv), block(64 * NWr);
-  const size_t lds = std::max<size_t>(2 * NSr * KV_TILE, (size_t)NWr * 32 * 272);  // ring / O staging
-#define PF_CASE2(GG, NS_, NW_)                                                                                 \
-  if (G == GG && NSr == NS_ && NWr == NW_) {                                                                  \
-    hipLaunchKernelGGL((attn_prefill_kernel<GG, NS_, NW_>), grid, block, lds, s, out, q, q_stride, k_cache,    \
+  dim3 grid((max_q_len + tpb - 1) / tpb, num_seqs, hkv), block(64 * NWr * KGr);
+  const size_t lds = std::max<size_t>(2 * NSr * KV_TILE * KGr, (size_t)NWr * 32 * 272 + (KGr - 1) * NWr * 66 * 256);  // rings / O staging, the groups' sums
+#define PF_CASE3(GG, NS_, NW_, KG_)                                                                                 \
+  if (G == GG && NSr == NS_ && NWr == NW_ && KGr == KG_) {                                                                  \
+    auto* fn = attn_prefill_kernel<GG, NS_, NW_, KG_>;                                                          \
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
+    if (e != hipSuccess) return e;                                                                              \
+    hipLaunchKernelGGL(fn, grid, block, lds, s, out, q, q_stride, k_cache,    \
                        v_cache, block_tables, bt_stride, cu_q, ctx_lens, hq, hkv, block_size, sl2, cos_sin, n_pos, \
                        q_scale);                                                                               \
     return hipGetLastError();                                                                                  \
   }
-#define PF_CASE(GG) PF_CASE2(GG, 2, 8) PF_CASE2(GG, 1, 4)
+#define PF_CASE(GG) PF_CASE3(GG, 2, 8, 1) PF_CASE3(GG, 1, 4, 1) PF_CASE3(GG, 1, 4, 2)
   PF_CASE(1)
   PF_CASE(2)
   PF_CASE(4)
@@ -784,7 +825,7 @@ hipError_t launch_attn_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, c
   PF_CASE(32)
   return hipErrorInvalidValue;
 #undef PF_CASE
-#undef PF_CASE2
+#undef PF_CASE3
 }
 
 static long long* g_attn_ts = nullptr;

@@ -1,0 +1,37 @@
+"""Prompt attention in two groups of waves per workgroup (attention.hip, steps of few row tiles) against fp32 attention.
+
+Weights and results are rounded to bf16 once each (2^-9 of each value, at random): the 2-norm of the difference is within 2^-8 of that of the result, and
+no value is further off than 2^-6 of the rows' largest scale."""
+
+import math
+
+import pytest
+import torch
+
+from src import ops
+from src.ops import reference as ref
+
+pytestmark = pytest.mark.gpu
+
+
+# new tokens and lengths: one stage for the first group alone, odd and even numbers of stages, a row of one key beside long ones, keys before the step
+@pytest.mark.parametrize("qlens,ctxs", [([200], [200]), ([257], [257]), ([1, 320, 33], [1, 320, 33]), ([288, 5], [1000, 37]), ([1000], [1000]), ([1025], [1537])])
+@pytest.mark.parametrize("hkv,g", [(8, 4), (4, 1), (1, 8), (1, 32)])
+def test_groups(qlens, ctxs, hkv, g):
+    hq, t, blocks = hkv * g, sum(qlens), [(c + 15) // 16 for c in ctxs]
+    rng = torch.Generator(device="cuda").manual_seed(0)
+    kc, vc = (torch.randn(sum(blocks), hkv, 16, 128, generator=rng, device="cuda").bfloat16() for _ in range(2))
+    q = torch.randn(t, hq * 128, generator=rng, device="cuda").bfloat16()
+    perm = torch.randperm(sum(blocks), generator=rng, device="cuda").int()
+    bt = torch.zeros(len(qlens), max(blocks), dtype=torch.int32, device="cuda")
+    at = 0
+    for i, n in enumerate(blocks):
+        bt[i, :n] = perm[at: at + n]
+        at += n
+    cu = torch.tensor([0] + qlens).cumsum(0).int().cuda()
+    ctx = torch.tensor(ctxs, dtype=torch.int32, device="cuda")
+    scale = 1 / math.sqrt(128)
+    out = ops.attn_prefill(q, kc, vc, bt, cu, ctx, max(qlens), hq, hkv, scale).float()
+    want = ref.attention(q, kc, vc, bt, cu, ctx, hq, hkv, scale).reshape(t, -1).float()
+    assert float((out - want).norm() / want.norm()) < 2.0 ** -8
+    assert float((out - want).abs().max() / want.abs().max()) < 2.0 ** -6
