@@ -761,10 +761,11 @@ def prompt_silu_tiles(m: int, inter: int, k: int, cus: int) -> Optional[int]:
       28672 x 4096   129 rows 61 / 65 / 58, 161 66 / 68 / 59, 200 72 / 75 / 77, 256 76 / 78 / 79, 257 80 / 78 / 109, 512 107 / 105, 768 171 / 167,
                      1200 268 / 253, 2048 394 / 381, 3000 582 / 563, 4096 706 / 724, 8192 1418 / 1430
       57344 x 8192   129 201 / 189 / 242, 256 224 / 245, 400 386 / 370, 700 576 / 555, 1024 780 / 732, 2048 1357 / 1370
-    One row tile leaves CUs idle or reads x for every 128 weight rows: to 168 rows tiles of 128 that fill the chip once, then the library to 256."""
-    if m <= 168:
-        return 96 if inter // 64 <= cus else 0
-    return None if m <= 256 or m > (3072 if inter * k <= 1 << 26 else 1536) else 0
+    One row tile leaves CUs idle with tiles of 256: up to 256 rows tiles of 128 where these fill the chip once. (Between 169 and 256 rows the product
+    alone is as fast as the library's two launches; a whole step of four Llama layers is faster with it: 192 rows 915 / 883, 224 947 / 930, 256 969 / 951.)"""
+    if m <= 256 and inter // 64 <= cus:
+        return 96
+    return None if 168 < m <= 256 or m > (3072 if inter * k <= 1 << 26 else 1536) else 0
 
 
 def prompt_silu_mul(x: torch.Tensor, w_gate_up: torch.Tensor, row_scale: torch.Tensor) -> torch.Tensor:
