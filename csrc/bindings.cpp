@@ -961,6 +961,59 @@ void rope_and_cache_slab(Tensor q_out, Tensor slab, Tensor positions, Tensor cos
                                           row_scale.has_value() ? row_scale->data_ptr<float>() : nullptr));
 }
 
+// queries [n, q_width], residuals [n, H], block tables, context lengths, offsets 0 .. n and (with rs) scales of the rows `keep` of a prompt step
+std::vector<Tensor> keep_rows(Tensor keep, Tensor cu_q, Tensor block_tables, Tensor ctx_lens, Tensor q, int64_t q_width, Tensor resid,
+                              std::optional<Tensor> rs) {
+  CHK_CUDA(q);
+  CHK_BF16(q);
+  CHK_BF16(resid);
+  check_rows(q, "q");
+  check_rows(resid, "resid");
+  CHK_DTYPE(keep, at::kLong);
+  CHK_CONTIG(keep);
+  for (const Tensor& t : {cu_q, block_tables, ctx_lens}) CHK_DTYPE(t, at::kInt);
+  CHK_CONTIG(cu_q);
+  CHK_CONTIG(ctx_lens);
+  for (const Tensor& t : {keep, cu_q, block_tables, ctx_lens, resid}) TORCH_CHECK(t.device() == q.device(), "keep_rows: one device");
+  const int64_t n = keep.numel(), S = ctx_lens.numel();
+  TORCH_CHECK(S >= 1 && cu_q.numel() == S + 1 && block_tables.dim() == 2 && block_tables.size(0) == S && block_tables.stride(1) == 1,
+              "keep_rows: cu_q [S + 1], block_tables [S, W], ctx_lens [S]");
+  TORCH_CHECK(q.size(0) == resid.size(0) && q.size(0) >= 1 && q_width >= 1 && q_width <= q.size(1), "keep_rows: q and resid rows");
+  die::KeepRowsArgs a{};
+  const auto i32 = ctx_lens.options();
+  std::vector<Tensor> out = {at::empty({n, q_width}, q.options()), at::empty({n, resid.size(1)}, resid.options()),
+                             at::empty({n, block_tables.size(1)}, i32), at::empty({n}, i32), at::empty({n + 1}, i32)};
+  a.q_out = bf(out[0]);
+  a.resid_out = bf(out[1]);
+  a.bt_out = out[2].data_ptr<int>();
+  a.ctx_out = out[3].data_ptr<int>();
+  a.cu_out = out[4].data_ptr<int>();
+  if (rs.has_value()) {
+    CHK_DTYPE(*rs, at::kFloat);
+    CHK_CONTIG(*rs);
+    TORCH_CHECK(rs->device() == q.device() && rs->numel() >= q.size(0), "keep_rows: rs [T] fp32");
+    out.push_back(at::empty({n}, rs->options()));
+    a.rs = rs->data_ptr<float>();
+    a.rs_out = out[5].data_ptr<float>();
+  }
+  a.keep = keep.data_ptr<int64_t>();
+  a.cu_q = cu_q.data_ptr<int>();
+  a.block_tables = block_tables.data_ptr<int>();
+  a.ctx_lens = ctx_lens.data_ptr<int>();
+  a.q = bf(q);
+  a.resid = bf(resid);
+  a.q_stride = q.stride(0);
+  a.r_stride = resid.stride(0);
+  a.bt_stride = block_tables.stride(0);
+  a.rows = (int)q.size(0);
+  a.num_seqs = (int)S;
+  a.q_width = (int)q_width;
+  a.hidden = (int)resid.size(1);
+  a.bt_width = (int)block_tables.size(1);
+  HIP_OK(die::launch_keep_rows(a, (int)n, cur_stream()));
+  return out;
+}
+
 // ---- one-shot all-reduce over IPC-mapped peer buffers (src/parallel/custom_allreduce.py)
 int64_t car_alloc(int64_t bytes, bool uncached) {
   TORCH_CHECK(bytes > 0 && bytes % 256 == 0, "car_alloc: bytes must be a positive multiple of 256");
@@ -1157,6 +1210,7 @@ PYBIND11_MODULE(_C, m) {
         py::arg("slot_mapping"), py::arg("k_cache"), py::arg("v_cache"), py::arg("hq"), py::arg("hkv"), py::arg("head_dim"),
         py::arg("row_scale") = py::none());
   m.def("rms_row_scale_slab", &rms_row_scale_slab);
+  m.def("keep_rows", &keep_rows);
   m.def("dense_gemm", &dense_gemm, py::arg("y"), py::arg("x"), py::arg("w"), py::arg("scale") = py::none(), py::arg("tile_rows") = 0);
   m.def("car_alloc", &car_alloc, py::arg("bytes"), py::arg("uncached") = true);
   m.def("car_tensor", &car_tensor);

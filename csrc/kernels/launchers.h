@@ -188,6 +188,26 @@ hipError_t launch_rope_and_cache_slab(bf16_t* q_out, const float* slab, int sk, 
                                       bf16_t* v_cache, int num_tokens, int hq, int hkv, int head_dim, int block_size,
                                       hipStream_t s, const float* row_scale = nullptr);
 
+// the kept rows of a prompt step's last layer (rope_cache.hip): queries, residuals, block tables, context lengths, offsets 0 .. n, scales
+struct KeepRowsArgs {
+  bf16_t* q_out;            // [n, q_width]
+  bf16_t* resid_out;        // [n, hidden]
+  int* bt_out;              // [n, bt_width]
+  int* ctx_out;             // [n]
+  int* cu_out;              // [n + 1]
+  float* rs_out;            // [n], with rs
+  const int64_t* keep;      // [n] rows
+  const int* cu_q;          // [num_seqs + 1]
+  const int* block_tables;  // [num_seqs, bt_width], rows bt_stride apart
+  const int* ctx_lens;      // [num_seqs]
+  const bf16_t* q;          // rows of q_width and more, q_stride apart; all rows at 16-byte addresses
+  const bf16_t* resid;
+  const float* rs;          // [rows] or nullptr
+  int64_t q_stride, r_stride, bt_stride;
+  int rows, num_seqs, q_width, hidden, bt_width;
+};
+hipError_t launch_keep_rows(const KeepRowsArgs& a, int n, hipStream_t s);
+
 // one-shot all-reduce over IPC-mapped peer buffers (allreduce.hip)
 hipError_t launch_custom_all_reduce(const bf16_t* in, bf16_t* out, int64_t n, int rank, int world,
                                     const CarPeers& peers, uint32_t* ctl, int64_t cap_elems, int blocks,

@@ -198,6 +198,44 @@ hipError_t launch_rope_and_cache_slab(bf16_t* q_out, const float* slab, int sk, 
 }
 
 // ----------------------------------------------------------------------------
+// The rows of a prompt step that its last layer goes on with, and what the attention of one query per row needs: kept row i of sequence s (the
+// last with cu_q[s] <= keep[i]) -> its query and residual, s's block table and context length, offsets 0 .. n, and its norm scale. One workgroup
+// per kept row. Bound by its launch; as eight launches (gathers, a search, a range) it took some 30 us more in steps of 8 and 13 sequences (8 x 100 rows of
+// four Llama layers 1495 -> 1463), 3 - 7 in those of one.
+__global__ void __launch_bounds__(256) keep_rows_kernel(KeepRowsArgs a) {
+  __shared__ int before[4];
+  const int i = blockIdx.x, tid = threadIdx.x;
+  const int64_t row = min(max(a.keep[i], (int64_t)0), (int64_t)a.rows - 1);
+  int cnt = 0;
+  for (int j = tid; j < a.num_seqs; j += 256) cnt += a.cu_q[j + 1] <= row ? 1 : 0;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
+  if ((tid & 63) == 0) before[tid >> 6] = cnt;
+  const uint4* q = reinterpret_cast<const uint4*>(a.q + row * a.q_stride);
+  const uint4* r = reinterpret_cast<const uint4*>(a.resid + row * a.r_stride);
+  uint4* qo = reinterpret_cast<uint4*>(a.q_out) + (int64_t)i * (a.q_width / 8);
+  uint4* ro = reinterpret_cast<uint4*>(a.resid_out) + (int64_t)i * (a.hidden / 8);
+  for (int c = tid; c < a.q_width / 8; c += 256) qo[c] = q[c];
+  for (int c = tid; c < a.hidden / 8; c += 256) ro[c] = r[c];
+  __syncthreads();
+  const int s = min(before[0] + before[1] + before[2] + before[3], a.num_seqs - 1);
+  for (int c = tid; c < a.bt_width; c += 256) a.bt_out[(int64_t)i * a.bt_width + c] = a.block_tables[s * a.bt_stride + c];
+  if (tid == 0) {
+    a.ctx_out[i] = a.ctx_lens[s];
+    a.cu_out[i + 1] = i + 1;
+    if (i == 0) a.cu_out[0] = 0;
+    if (a.rs != nullptr) a.rs_out[i] = a.rs[row];
+  }
+}
+
+hipError_t launch_keep_rows(const KeepRowsArgs& a, int n, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  if (n < 0 || a.rows < 1 || a.num_seqs < 1 || a.q_width % 8 || a.hidden % 8 || a.q_stride % 8 || a.r_stride % 8) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(keep_rows_kernel, dim3(n), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
+// ----------------------------------------------------------------------------
 // Block movers. `slab` = elements of one (layer, kv, block) = hkv*block_size*D.
 // The pool is viewed as [planes = layers*2][num_blocks][slab].
 

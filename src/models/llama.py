@@ -494,15 +494,8 @@ class CausalLM:
             meta.kv_hook(li)
         if n == 0:
             return residual[:0]
-        # the sequence of each kept row (rows of sequence i: [cu_q[i], cu_q[i + 1]))
-        seq = torch.searchsorted(meta.cu_q[1:].to(torch.int64), keep, right=True)
-        q = qkv.index_select(0, keep)[:, : hq * d].contiguous()
-        cu1 = torch.arange(n + 1, dtype=torch.int32, device=q.device)
-        attn = ops.attn_prefill(q, k_cache, v_cache, meta.block_tables.index_select(0, seq),
-                                cu1, meta.ctx_lens.index_select(0, seq), 1, hq, hkv, self.scale,
-                                cos_sin=self.cos_sin if fuse_q else None,
-                                q_scale=rs.index_select(0, keep) if rs is not None else None)
-        res = residual.index_select(0, keep)
+        q, res, tables, ctx, cu1, qs = ops.keep_rows(keep, meta.cu_q, meta.block_tables, meta.ctx_lens, qkv, hq * d, residual, rs)
+        attn = ops.attn_prefill(q, k_cache, v_cache, tables, cu1, ctx, 1, hq, hkv, self.scale, cos_sin=self.cos_sin if fuse_q else None, q_scale=qs)
         o = self.tp.all_reduce(ops.linear(attn, lw.o))
         x2 = ops.fused_add_rms_norm(o, res, lw.ln2, eps)
         h = self.tp.all_reduce(self._mlp(lw, x2))

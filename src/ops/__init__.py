@@ -837,6 +837,26 @@ def rope_and_cache_slab(slab, positions, cos_sin, slot_mapping, k_cache, v_cache
     return q_out
 
 
+def keep_rows(keep: torch.Tensor, cu_q: torch.Tensor, block_tables: torch.Tensor, ctx_lens: torch.Tensor, q: torch.Tensor, q_width: int,
+              resid: torch.Tensor, rs: Optional[torch.Tensor] = None):
+    """What a prompt step's last layer goes on with for its rows ``keep`` (int64): their queries q[keep, :q_width] and residuals, the block table and
+    context length of each one's sequence (rows cu_q[i] .. cu_q[i + 1] are sequence i's), offsets 0 .. n (int32) and the rows' scales rs (or None).
+    One launch on the GPU."""
+    rows = (q, resid)
+    ints = (cu_q, block_tables, ctx_lens)
+    if (q.is_cuda and native_available() and all(t.dtype == torch.bfloat16 and t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
+                                                 for t in rows)
+            and all(t.dtype == torch.int32 for t in ints) and keep.dtype == torch.int64 and keep.is_contiguous() and cu_q.is_contiguous()
+            and ctx_lens.is_contiguous() and block_tables.stride(1) == 1 and cu_q.numel() == ctx_lens.numel() + 1 == block_tables.shape[0] + 1
+            and q.shape[0] == resid.shape[0] > 0 and q_width % 8 == resid.shape[1] % 8 == 0 and keep.numel() > 0):
+        out = _kern().keep_rows(keep, cu_q, block_tables, ctx_lens, q, q_width, resid, rs)
+        return tuple(out) if rs is not None else (*out, None)
+    seq = torch.searchsorted(cu_q[1:].to(torch.int64), keep, right=True)
+    return (q.index_select(0, keep)[:, :q_width].contiguous(), resid.index_select(0, keep), block_tables.index_select(0, seq),
+            ctx_lens.index_select(0, seq), torch.arange(keep.numel() + 1, dtype=torch.int32, device=q.device),
+            rs.index_select(0, keep) if rs is not None else None)
+
+
 def topk_softmax(gating: torch.Tensor, k: int, renorm: bool = True):
     if not gating.is_cuda:
         return ref.topk_softmax(gating, k, renorm)

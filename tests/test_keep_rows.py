@@ -1,0 +1,40 @@
+"""The rows that a prompt step's last layer goes on with, in one launch against the same gathers (copies: equal to the bit)."""
+
+import pytest
+import torch
+
+from src import ops
+
+
+def _step(dev, lens, width=24, hidden=40, extra=16, blocks=5):
+    g = torch.Generator().manual_seed(0)
+    t, s = sum(lens), len(lens)
+    cu = torch.tensor([0] + lens).cumsum(0).int()
+    wide = torch.randn(t, width + extra, generator=g).bfloat16()
+    tables = torch.randint(0, 99, (s, blocks + 3), generator=g, dtype=torch.int32)
+    args = [cu, tables, torch.randint(1, 99, (s,), generator=g, dtype=torch.int32), wide, torch.randn(t, hidden, generator=g).bfloat16(), torch.rand(t, generator=g)]
+    cu, tables, ctx, wide, resid, rs = (a.to(dev) for a in args)
+    return cu, tables[:, :blocks], ctx, wide, width, resid, rs
+
+
+def _want(keep, cu, tables, ctx, q, width, resid, rs):
+    seq = [next(i for i in range(len(cu) - 1) if int(cu[i + 1]) > int(k)) for k in keep]
+    return q[keep, :width], resid[keep], tables[seq], ctx[seq], torch.arange(len(keep) + 1, dtype=torch.int32), rs[keep] if rs is not None else None
+
+
+# one sequence, empty ones between, more sequences than a workgroup has threads; first, inner and last rows; with and without scales
+@pytest.mark.parametrize("lens", [[7], [1, 0, 0, 5, 3, 0], [2] * 600])
+@pytest.mark.parametrize("scaled", [True, False])
+@pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_rows(dev, lens, scaled):
+    cu, tables, ctx, q, width, resid, rs = _step(dev, lens)
+    rs = rs if scaled else None
+    ends = [int(e) - 1 for e, n in zip(cu[1:], lens) if n > 0]
+    for keep in (ends, [0], list(range(sum(lens)))[::3][::-1]):
+        at = torch.tensor(keep, dtype=torch.int64)
+        got = ops.keep_rows(at.to(dev), cu, tables, ctx, q, width, resid, rs)
+        want = _want(at, cu.cpu(), tables.cpu(), ctx.cpu(), q.cpu(), width, resid.cpu(), rs.cpu() if scaled else None)
+        for a, b in zip(got, want):
+            assert (a is None) == (b is None)
+            if a is not None:
+                assert a.dtype == b.dtype and a.is_contiguous() and torch.equal(a.cpu(), b)
