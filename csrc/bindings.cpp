@@ -963,7 +963,7 @@ void rope_and_cache_slab(Tensor q_out, Tensor slab, Tensor positions, Tensor cos
 
 // queries [n, q_width], residuals [n, H], block tables, context lengths, offsets 0 .. n and (with rs) scales of the rows `keep` of a prompt step
 std::vector<Tensor> keep_rows(Tensor keep, Tensor cu_q, Tensor block_tables, Tensor ctx_lens, Tensor q, int64_t q_width, Tensor resid,
-                              std::optional<Tensor> rs) {
+                              std::optional<Tensor> rs, std::optional<Tensor> cos_sin) {
   CHK_CUDA(q);
   CHK_BF16(q);
   CHK_BF16(resid);
@@ -995,6 +995,14 @@ std::vector<Tensor> keep_rows(Tensor keep, Tensor cu_q, Tensor block_tables, Ten
     out.push_back(at::empty({n}, rs->options()));
     a.rs = rs->data_ptr<float>();
     a.rs_out = out[5].data_ptr<float>();
+  }
+  if (cos_sin.has_value()) {
+    CHK_DTYPE(*cos_sin, at::kFloat);
+    CHK_CONTIG(*cos_sin);
+    TORCH_CHECK(cos_sin->device() == q.device() && cos_sin->dim() == 2 && cos_sin->size(0) >= 1 && cos_sin->size(1) == 128 && q_width % 128 == 0,
+                "keep_rows: cos_sin [positions, 128], heads of 128");
+    a.cos_sin = cos_sin->data_ptr<float>();
+    a.n_pos = (int)cos_sin->size(0);
   }
   a.keep = keep.data_ptr<int64_t>();
   a.cu_q = cu_q.data_ptr<int>();
@@ -1210,7 +1218,8 @@ PYBIND11_MODULE(_C, m) {
         py::arg("slot_mapping"), py::arg("k_cache"), py::arg("v_cache"), py::arg("hq"), py::arg("hkv"), py::arg("head_dim"),
         py::arg("row_scale") = py::none());
   m.def("rms_row_scale_slab", &rms_row_scale_slab);
-  m.def("keep_rows", &keep_rows);
+  m.def("keep_rows", &keep_rows, py::arg("keep"), py::arg("cu_q"), py::arg("block_tables"), py::arg("ctx_lens"), py::arg("q"), py::arg("q_width"),
+        py::arg("resid"), py::arg("rs"), py::arg("cos_sin") = py::none());
   m.def("dense_gemm", &dense_gemm, py::arg("y"), py::arg("x"), py::arg("w"), py::arg("scale") = py::none(), py::arg("tile_rows") = 0);
   m.def("car_alloc", &car_alloc, py::arg("bytes"), py::arg("uncached") = true);
   m.def("car_tensor", &car_tensor);

@@ -205,6 +205,8 @@ struct KeepRowsArgs {
   const float* rs;          // [rows] or nullptr
   int64_t q_stride, r_stride, bt_stride;
   int rows, num_seqs, q_width, hidden, bt_width;
+  const float* cos_sin;     // nullptr: queries as they are; [n_pos, 128]: heads of 128 turned at ctx - 1 and scaled by rs
+  int n_pos;
 };
 hipError_t launch_keep_rows(const KeepRowsArgs& a, int n, hipStream_t s);
 

@@ -215,10 +215,29 @@ __global__ void __launch_bounds__(256) keep_rows_kernel(KeepRowsArgs a) {
   const uint4* r = reinterpret_cast<const uint4*>(a.resid + row * a.r_stride);
   uint4* qo = reinterpret_cast<uint4*>(a.q_out) + (int64_t)i * (a.q_width / 8);
   uint4* ro = reinterpret_cast<uint4*>(a.resid_out) + (int64_t)i * (a.hidden / 8);
-  for (int c = tid; c < a.q_width / 8; c += 256) qo[c] = q[c];
+  if (a.cos_sin == nullptr)
+    for (int c = tid; c < a.q_width / 8; c += 256) qo[c] = q[c];
   for (int c = tid; c < a.hidden / 8; c += 256) ro[c] = r[c];
   __syncthreads();
   const int s = min(before[0] + before[1] + before[2] + before[3], a.num_seqs - 1);
+  if (a.cos_sin != nullptr) {   // heads of 128, turned at their sequence's last position and scaled (as the prompt attention does on loading them)
+    const float* cs = a.cos_sin + (int64_t)min(max(a.ctx_lens[s] - 1, 0), a.n_pos - 1) * 128;
+    const float scale = a.rs != nullptr ? a.rs[row] : 1.0f;
+    for (int it = tid; it < a.q_width / 16; it += 256) {
+      const int at = it / 8 * 16 + it % 8, d = it % 8 * 8;   // this chunk and the one 64 columns on
+      float x[8], y[8], xo[8], yo[8];
+      unpack8(q[at], x);
+      unpack8(q[at + 8], y);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float co = cs[d + j] * scale, si = cs[64 + d + j] * scale;
+        xo[j] = x[j] * co - y[j] * si;
+        yo[j] = y[j] * co + x[j] * si;
+      }
+      qo[at] = pack8(xo);
+      qo[at + 8] = pack8(yo);
+    }
+  }
   for (int c = tid; c < a.bt_width; c += 256) a.bt_out[(int64_t)i * a.bt_width + c] = a.block_tables[s * a.bt_stride + c];
   if (tid == 0) {
     a.ctx_out[i] = a.ctx_lens[s];
@@ -231,6 +250,7 @@ __global__ void __launch_bounds__(256) keep_rows_kernel(KeepRowsArgs a) {
 hipError_t launch_keep_rows(const KeepRowsArgs& a, int n, hipStream_t s) {
   if (n == 0) return hipSuccess;
   if (n < 0 || a.rows < 1 || a.num_seqs < 1 || a.q_width % 8 || a.hidden % 8 || a.q_stride % 8 || a.r_stride % 8) return hipErrorInvalidValue;
+  if (a.cos_sin != nullptr && (a.q_width % 128 || a.n_pos < 1)) return hipErrorInvalidValue;
   hipLaunchKernelGGL(keep_rows_kernel, dim3(n), dim3(256), 0, s, a);
   return hipGetLastError();
 }

@@ -838,10 +838,11 @@ def rope_and_cache_slab(slab, positions, cos_sin, slot_mapping, k_cache, v_cache
 
 
 def keep_rows(keep: torch.Tensor, cu_q: torch.Tensor, block_tables: torch.Tensor, ctx_lens: torch.Tensor, q: torch.Tensor, q_width: int,
-              resid: torch.Tensor, rs: Optional[torch.Tensor] = None):
+              resid: torch.Tensor, rs: Optional[torch.Tensor] = None, cos_sin: Optional[torch.Tensor] = None):
     """What a prompt step's last layer goes on with for its rows ``keep`` (int64): their queries q[keep, :q_width] and residuals, the block table and
     context length of each one's sequence (rows cu_q[i] .. cu_q[i + 1] are sequence i's), offsets 0 .. n (int32) and the rows' scales rs (or None).
-    One launch on the GPU."""
+    cos_sin ([max_pos, 128] fp32): the queries, heads of 128, come turned at their sequence's last position and scaled by rs, which is then not
+    returned. One launch on the GPU."""
     rows = (q, resid)
     ints = (cu_q, block_tables, ctx_lens)
     if (q.is_cuda and native_available() and all(t.dtype == torch.bfloat16 and t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
@@ -849,12 +850,18 @@ def keep_rows(keep: torch.Tensor, cu_q: torch.Tensor, block_tables: torch.Tensor
             and all(t.dtype == torch.int32 for t in ints) and keep.dtype == torch.int64 and keep.is_contiguous() and cu_q.is_contiguous()
             and ctx_lens.is_contiguous() and block_tables.stride(1) == 1 and cu_q.numel() == ctx_lens.numel() + 1 == block_tables.shape[0] + 1
             and q.shape[0] == resid.shape[0] > 0 and q_width % 8 == resid.shape[1] % 8 == 0 and keep.numel() > 0):
-        out = _kern().keep_rows(keep, cu_q, block_tables, ctx_lens, q, q_width, resid, rs)
-        return tuple(out) if rs is not None else (*out, None)
+        out = _kern().keep_rows(keep, cu_q, block_tables, ctx_lens, q, q_width, resid, rs, cos_sin)
+        return (*out[:5], out[5] if rs is not None and cos_sin is None else None)
     seq = torch.searchsorted(cu_q[1:].to(torch.int64), keep, right=True)
-    return (q.index_select(0, keep)[:, :q_width].contiguous(), resid.index_select(0, keep), block_tables.index_select(0, seq),
-            ctx_lens.index_select(0, seq), torch.arange(keep.numel() + 1, dtype=torch.int32, device=q.device),
-            rs.index_select(0, keep) if rs is not None else None)
+    q, ctx = q.index_select(0, keep)[:, :q_width].contiguous(), ctx_lens.index_select(0, seq)
+    scale = rs.index_select(0, keep) if rs is not None else None
+    if cos_sin is not None:
+        cs = cos_sin[(ctx.long() - 1).clamp(0, cos_sin.shape[0] - 1)][:, None, :] * (scale[:, None, None] if scale is not None else 1.0)
+        a, b = q.float().view(len(ctx), -1, 2, 64).unbind(2)
+        q = torch.cat([a * cs[..., :64] - b * cs[..., 64:], b * cs[..., :64] + a * cs[..., 64:]], -1).view_as(q).to(q.dtype)
+        scale = None
+    return (q, resid.index_select(0, keep), block_tables.index_select(0, seq), ctx,
+            torch.arange(keep.numel() + 1, dtype=torch.int32, device=q.device), scale)
 
 
 def topk_softmax(gating: torch.Tensor, k: int, renorm: bool = True):

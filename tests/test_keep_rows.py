@@ -38,3 +38,18 @@ def test_rows(dev, lens, scaled):
             assert (a is None) == (b is None)
             if a is not None:
                 assert a.dtype == b.dtype and a.is_contiguous() and torch.equal(a.cpu(), b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scaled", [True, False])
+def test_turned_queries(scaled):
+    """Heads of 128 turned at their sequence's last position and scaled, against the plain form in torch: the same fp32 terms, rounded to bf16 once
+    (2^-8 of the pair covers a sum next to a tie)."""
+    cu, tables, ctx, q, width, resid, rs = _step("cuda", [3, 1, 0, 9], width=384)
+    cs = torch.randn(60, 128, generator=torch.Generator().manual_seed(1)).cuda()   # (fewer positions than the longest context: the last one)
+    keep = torch.tensor([2, 3, 12], device="cuda")
+    got = ops.keep_rows(keep, cu, tables, ctx, q, width, resid, rs if scaled else None, cos_sin=cs)
+    want = ops.keep_rows(keep.cpu(), cu.cpu(), tables.cpu(), ctx.cpu(), q.cpu(), width, resid.cpu(), rs.cpu() if scaled else None, cos_sin=cs.cpu())
+    assert got[5] is None and want[5] is None and all(torch.equal(a.cpu(), b) for a, b in zip(got[1:5], want[1:5]))
+    a, b = got[0].float().cpu().view(3, 3, 2, 64), want[0].float().view(3, 3, 2, 64)
+    assert bool(((a - b).abs() <= 2.0 ** -8 * b.norm(dim=2, keepdim=True)).all())
