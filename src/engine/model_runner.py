@@ -244,7 +244,7 @@ class ModelRunner:
     def idle_tick(self) -> None:
         """Called by the engine loop while it has no work (TP runners send heartbeats)."""
 
-    def _sync_step(self, kind: int, a: int = 0, b: int = 0, c: int = 0, d: int = 0) -> None:
+    def _sync_step(self, kind: int, a: int = 0, b: int = 0, c: int = 0, d: int = 0, max_ctx: int = 0) -> None:
         """Hook for tensor parallelism: rank 0 publishes the step to followers
         (see :class:`src.parallel.tp_runner.TPModelRunner`). No-op at TP=1."""
 
@@ -271,9 +271,9 @@ class ModelRunner:
             nl[:nd] = nl[done]
         greedy = self._fill_sampling([chunks[i].seq for i in done], nd) if nd else True
         self._h2d(t, n, with_cu=True)
-        max_q = max(c.length for c in chunks)
-        self._sync_step(self.KIND_PREFILL, t, n, max_q, nd)
-        ids = self._exec_prefill(t, n, max_q, nd, greedy, kv_hook=kv_hook, max_ctx=max(c.start + c.length for c in chunks))
+        max_q, max_ctx = max(c.length for c in chunks), max(c.start + c.length for c in chunks)
+        self._sync_step(self.KIND_PREFILL, t, n, max_q, nd, max_ctx)
+        ids = self._exec_prefill(t, n, max_q, nd, greedy, kv_hook=kv_hook, max_ctx=max_ctx)
         res: List[Optional[int]] = [None] * n
         if nd:
             vals = self._to_host(ids, nd)

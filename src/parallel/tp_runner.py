@@ -7,8 +7,9 @@ are the same on every rank, so one block table serves the whole group).
 
 Step protocol (two messages per step):
 
-1. an 8-word header ``[kind, a, b, c, d, payload words, 0, 0]`` broadcast on the
-   host (gloo) group — followers read it without any GPU round trip;
+1. an 8-word header ``[kind, a, b, c, d, payload words, longest context, 0]`` broadcast on
+   the host (gloo) group — followers read it without any GPU round trip (the longest context of
+   a prompt step chooses and sizes its kernels, on every rank alike);
 2. ONE int64 payload with every input of the step packed back to back (token
    ids, positions, slots, context lengths, block-table rows, cu_q, last-token
    indices), built in pinned memory on rank 0, copied up once and broadcast over
@@ -163,7 +164,7 @@ class TPModelRunner(ModelRunner):
     def _bcast(self, t: torch.Tensor) -> None:
         self.tp.broadcast(t, src=0)
 
-    def _sync_step(self, kind: int, a: int = 0, b: int = 0, c: int = 0, d: int = 0) -> None:
+    def _sync_step(self, kind: int, a: int = 0, b: int = 0, c: int = 0, d: int = 0, max_ctx: int = 0) -> None:
         """Leader: header on the host group, then the packed payload (the leader's own device buffers
         were already filled by the runner's H2D copies, so it does not unpack)."""
         if not self.tp.enabled:
@@ -176,7 +177,7 @@ class TPModelRunner(ModelRunner):
             d = b if self._samp_dirty else 0
             self._samp_dirty = False
         nw = self._pack(kind, a, b, d)
-        self.h_hdr.copy_(torch.tensor([kind, a, b, c, d, nw, 0, 0], dtype=torch.int64))
+        self.h_hdr.copy_(torch.tensor([kind, a, b, c, d, nw, max_ctx, 0], dtype=torch.int64))
         self.tp.broadcast_host(self.h_hdr)
         if nw:
             self.d_pkt[:nw].copy_(self.h_pkts[self._pkt_par][:nw], non_blocking=self.is_cuda)
@@ -209,7 +210,7 @@ class TPModelRunner(ModelRunner):
         assert self.tp.rank != 0
         while True:
             self.tp.broadcast_host(self.h_hdr)
-            kind, a, b, c, d, nw = (int(x) for x in self.h_hdr.tolist()[:6])
+            kind, a, b, c, d, nw, max_ctx = (int(x) for x in self.h_hdr.tolist()[:7])
             if kind == self.KIND_STOP:
                 return
             if kind == self.KIND_HEARTBEAT:
@@ -218,7 +219,7 @@ class TPModelRunner(ModelRunner):
                 self._bcast(self.d_pkt[:nw])
                 self._unpack(kind, a, b, d)
             if kind == self.KIND_PREFILL:
-                self._exec_prefill(a, b, c, d, True)
+                self._exec_prefill(a, b, c, d, True, max_ctx=max_ctx)
             elif kind == self.KIND_WINDOW:
                 pad, k = b, c
                 self._pre_embed(pad)

@@ -81,6 +81,42 @@ def test_tp2_matches_tp1(preset, moe_parallel, sp):
     assert got == expect
 
 
+def _prompt_bounds_worker(rank, port, q):
+    os.environ.update(MASTER_ADDR="127.0.0.1", MASTER_PORT=str(port))
+    dist.init_process_group("gloo", rank=rank, world_size=2)
+    try:
+        obj = build_tp_engine("llama-tiny", TPContext(rank=rank, world_size=2), "cpu", cfg=_cfg(), max_model_len=256, capture=False,
+                              dtype=torch.float32, full_init=True, seed=3)
+        runner, seen = (obj.runner if rank == 0 else obj), []
+        forward = runner.model.forward
+        runner.model.forward = lambda ids, pos, meta, pool: seen.append((meta.max_q_len, meta.max_ctx, int(meta.ctx_lens.max()))
+                                                                        if meta.is_prefill else None) or forward(ids, pos, meta, pool)
+        if rank == 0:
+            obj.eos_token_id = None
+            obj.generate(PROMPTS, SamplingParams(max_tokens=2))
+            runner.stop_followers()
+        else:
+            runner.follower_loop()
+        q.put((rank, [x for x in seen if x is not None]))
+    finally:
+        dist.destroy_process_group()
+
+
+def test_prompt_steps_longest_context_on_every_rank():
+    """A prompt step's longest context chooses and sizes its kernels: the followers' is the leader's, also of portions behind earlier ones
+    (67 tokens in steps of 48)."""
+    ctx = mp.get_context("spawn")
+    q, port = ctx.Queue(), _free_port()
+    procs = [ctx.Process(target=_prompt_bounds_worker, args=(r, port, q)) for r in range(2)]
+    for p in procs:
+        p.start()
+    got = dict(q.get(timeout=120) for _ in range(2))
+    for p in procs:
+        p.join(60)
+        assert p.exitcode == 0
+    assert got[0] == got[1] and all(bound == most for _, bound, most in got[0]) and any(most > new for new, _, most in got[0])
+
+
 def test_fused_exchange_residency_rule_at_70b_tp8_shapes():
     """The exchange fused into the row-parallel decode GEMM (custom_allreduce.fused_exchange_ok, VERDICT r5 weak 5 /
     ADVICE r5): on an 8-GPU node (one rank per GPU, 256 CUs) the 70B TP=8 shard's o / down at 32 rows (wr = 32:
