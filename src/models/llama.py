@@ -481,9 +481,9 @@ class CausalLM:
         still projected and written to the cache (later steps attend to them), but the query, attention, o, MLP
         and final norm run for one row per sampled sequence — the other rows' last-layer outputs would be
         discarded (a 16,384-token prefill of 32 prompts keeps 32 rows: ~1/32 of a layer's GEMM work for the
-        sampled rows instead of a whole layer). The kept rows are each sequence's last token, so the attention is
-        a 1-query-per-sequence prefill attention over the full context. rs: x is the raw residual and rs its
-        RMSNorm row scales (:meth:`_forward_prefill_row_scale`)."""
+        sampled rows instead of a whole layer). The kept rows are each sequence's last token, so the attention has
+        one query per sequence over the full context: the decode kernel's behind many keys, else the prompt
+        kernel's. rs: x is the raw residual and rs its RMSNorm row scales (:meth:`_forward_prefill_row_scale`)."""
         eps, d, hq, hkv = self.arch.rms_eps, self.head_dim, self.hq, self.hkv
         li = len(self.layers) - 1
         keep = meta.keep_rows
@@ -496,7 +496,7 @@ class CausalLM:
             return residual[:0]
         # One query per sequence: behind many keys by the decode kernel, which splits them, where the prompt kernel goes through them in one chain. us,
         # prompt / decode kernel: 1 sequence of 300 keys 13.5 / 14.4, 512 19.5 / 14.6, 1000 35 / 15, 2000 66 / 15; 32 of 512 20.9 / 16.4, of 1000 37 / 25
-        split = qkv.is_cuda and max(meta.max_q_len, meta.max_ctx) >= 400 and n * hkv <= 256
+        split = qkv.is_cuda and max(meta.max_q_len, meta.max_ctx) >= 400 and n * hkv <= 256 and ops.decode_attn_merges(hq, hkv, k_cache.shape[2])
         q, res, tables, ctx, cu1, qs = ops.keep_rows(keep, meta.cu_q, meta.block_tables, meta.ctx_lens, qkv, hq * d, residual, rs,
                                                      cos_sin=self.cos_sin if fuse_q and split else None)
         if split:

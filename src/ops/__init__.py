@@ -163,6 +163,12 @@ def decode_partials(max_ctx: int) -> int:
     return int(_kern().decode_partials(max_ctx))
 
 
+def decode_attn_merges(hq: int, hkv: int, block_size: int) -> bool:
+    """Whether :func:`attn_decode` runs the kernel that merges its splits itself (launch_attn_decode in attention.hip). Other block sizes and groups of 16
+    heads take two launches of an older one; groups of 32 it refuses, which :func:`attn_prefill` takes."""
+    return hq % hkv == 0 and hq // hkv in (1, 2, 4, 8) and block_size == 16
+
+
 def attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, max_ctx: int, hq: int, hkv: int, scale: float,
                 part_o: Optional[torch.Tensor] = None, part_ml: Optional[torch.Tensor] = None,
                 out: Optional[torch.Tensor] = None, counters: Optional[torch.Tensor] = None,
