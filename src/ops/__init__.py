@@ -741,10 +741,16 @@ def prompt_slab_parts(m: int, n: int, k: int, cus: int, residual: bool):
       4096 x 14336   129 rows 57 / 40, 256 65 / 49, 400 84 / 63, 768 110 / 88, 1024 135 / 113, 1500 171 / 151, 2048 206 / 200 (2300: one part, 241 / 246)
       8192 x 28672   129 307 / 121, 400 300 / 185, 1024 384 / 365          8192 x 8192   256 83 / 55, 512 83 / 82, 700 101 / 95, 1024 121 / 127
       4096 x 4096    129 35 / 25, 200 34 / 26, 256 26 / 29, 300 30 / 32, 512 34 / 35
-      qkv 6144 x 4096  129 43 / 29, 192 36 / 31, 256 43 / 34, 300 32 / 38   10240 x 8192, two parts   129 56 / 63, 256 92 / 80"""
+      qkv 6144 x 4096  129 42 / 30, 160 32 / 32, 192 38 / 33, 256 45 / 36, 300 32 / 38   10240 x 8192, two parts   129 56 / 63, 256 92 / 80
+          5120 x 8192  129 36 / 42, 160 55 / 44, 256 78 / 51        4608 x 3072  129 22 / 25, 160 28 / 26, 256 36 / 30
+    A qkv product of fewer columns (small models, shards) is the library's: 3840 x 5120 129 31 / 29, 256 32 / 35; 3072 x 4096 129 20 / 27, 256 27 / 30; 2560 x 8192
+    129 28 / 31, 256 38 / 37; 1536 x 4096 17 / 24 and 20 / 30; 1280 x 8192 25 / 29 and 31 / 36; 1536 x 1024 14 / 19 and 14 / 25; and so is one of little K: 6144 x 2048 24 / 24,
+    160 rows 21 / 26, 256 28 / 28."""
     sk, code = slab_parts(m, n, k, cus)
-    most = (224 if k < 8192 else 768 if k < 12288 else 1 << 31) if residual else 256
-    return None if m > most or sk < (2 if residual else 4) else (sk, code)
+    if residual:
+        most = 224 if k < 8192 else 768 if k < 12288 else 1 << 31
+        return None if m > most or sk < 2 else (sk, code)
+    return (sk, code) if sk >= 4 and m <= 256 and k >= 2560 and (n >= 6144 or (n >= 4608 and m >= 160)) else None
 
 
 def prompt_slab(x: torch.Tensor, w: torch.Tensor, residual: bool = True) -> Optional[torch.Tensor]:

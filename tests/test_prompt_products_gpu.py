@@ -86,7 +86,7 @@ def test_rope_of_scaled_slabs():
 @pytest.mark.parametrize("rows", [129, 200, 257, 600])
 @pytest.mark.parametrize("keep", [False, True])
 def test_steps_of_few_row_tiles(monkeypatch, rows, keep):
-    """A prompt step through slabs and the gate on sums against the library's products: one bf16 rounding apart per product."""
+    """A prompt step with every product by slabs and the gate on sums against the library's products: one bf16 rounding apart per product."""
     from src.models.llama import AttnMetadata, CausalLM
     from src.models.presets import get_preset
 
@@ -100,7 +100,10 @@ def test_steps_of_few_row_tiles(monkeypatch, rows, keep):
     slots = torch.cat([pos[: rows - 100], nb * 16 + pos[rows - 100:]])
     got = []
     for own in (True, False):
-        if not own:
+        if own:   # (the rules leave products of these widths to the library)
+            monkeypatch.setattr(ops, "prompt_slab_parts", lambda mm, n, k, cus, residual: ops.slab_parts(mm, n, k, cus))
+            monkeypatch.setattr(ops, "prompt_silu_tiles", lambda mm, *a: 96 if mm <= 256 else 0)
+        else:
             monkeypatch.setattr(ops, "_dense_gemm_ok", lambda x, w: False)
         pool = torch.zeros(m.arch.num_layers, 2, 2 * nb, m.hkv, 16, 128, dtype=m.dtype, device="cuda")
         meta = AttnMetadata(True, slots, tables, torch.tensor([rows - 100, 100], dtype=torch.int32, device="cuda"), cu, max(rows - 100, 100),
@@ -111,12 +114,24 @@ def test_steps_of_few_row_tiles(monkeypatch, rows, keep):
 
 
 def test_parts_of_k():
-    """Parts are whole stages of K, one workgroup per compute unit at most, and none where the library is taken."""
+    """Parts are whole stages of K, one workgroup per compute unit at most."""
     for m in (129, 224, 256, 257, 512, 1000, 2048, 5000):
         for n, k in ((4096, 4096), (4096, 14336), (6144, 4096), (8192, 28672), (1024, 2048), (256, 64), (768, 192)):
             sk, code = ops.slab_parts(m, n, k, 256)
             assert 1 <= sk <= 8 and k % (64 * sk) == 0 and (sk == 1 or (n // 128 if code == 96 else n // 256 * -(-m // 256)) * sk <= 256)
-            for residual in (True, False):
-                assert ops.prompt_slab_parts(m, n, k, 256, residual) in (None, (sk, code))
     x, w = torch.zeros(300, 64, dtype=torch.bfloat16), torch.zeros(256, 64, dtype=torch.bfloat16)
     assert ops.prompt_slab(x, w) is None   # (not on a device)
+
+
+@pytest.mark.parametrize("n,k,residual,own,library", [
+    # qkv: either side of the lines in rows, columns and K; small models and shards
+    (6144, 4096, False, {129: 4, 256: 4}, [257, 300]), (5120, 8192, False, {160: 4, 256: 4}, [129, 159, 257]), (4608, 3072, False, {160: 6, 256: 6}, [129, 300]),
+    (6144, 2560, False, {129: 5, 256: 5}, [300]), (6144, 2048, False, {}, [129, 160, 256]), (3840, 5120, False, {}, [129, 256]), (3072, 4096, False, {}, [129, 256]),
+    (1536, 1024, False, {}, [129, 256]), (1536, 4096, False, {}, [129, 256]), (1280, 8192, False, {}, [129, 256]), (10240, 8192, False, {}, [129, 256]),
+    # o and down
+    (4096, 14336, True, {129: 8, 256: 8, 257: 8, 1024: 4, 2048: 2}, [2300]), (4096, 11008, True, {192: 4, 768: 4}, [769])])
+def test_choice_of_slabs(n, k, residual, own, library):
+    """The parts that are taken, and where the library is, on a device of 256 compute units."""
+    for m, sk in own.items():
+        assert ops.prompt_slab_parts(m, n, k, 256, residual) == (sk, 96 if m <= 256 else 0)
+    assert all(ops.prompt_slab_parts(m, n, k, 256, residual) is None for m in library)
