@@ -743,13 +743,17 @@ def prompt_slab_parts(m: int, n: int, k: int, cus: int, residual: bool):
       4096 x 4096    129 35 / 25, 200 34 / 26, 256 26 / 29, 300 30 / 32, 512 34 / 35
       qkv 6144 x 4096  129 42 / 30, 160 32 / 32, 192 38 / 33, 256 45 / 36, 300 32 / 38   10240 x 8192, two parts   129 56 / 63, 256 92 / 80
           5120 x 8192  129 36 / 42, 160 55 / 44, 256 78 / 51        4608 x 3072  129 22 / 25, 160 28 / 26, 256 36 / 30
+    In whole steps, us a layer that slabs take more than the library: 4096 x 4096 160 rows -6, 192 -8, 224 +1; 5120 x 5120 160 -6, 224 -10. Where the parts leave
+    compute units idle too: 2048 x 2048 129 0, 192 +1, 224 +2; 2560 x 4096 129 - 192 +2; 4096 x 11008 (half of them) 192 -30, 224 and 256 +3, 300 -6.
     A qkv product of fewer columns (small models, shards) is the library's: 3840 x 5120 129 31 / 29, 256 32 / 35; 3072 x 4096 129 20 / 27, 256 27 / 30; 2560 x 8192
     129 28 / 31, 256 38 / 37; 1536 x 4096 17 / 24 and 20 / 30; 1280 x 8192 25 / 29 and 31 / 36; 1536 x 1024 14 / 19 and 14 / 25; and so is one of little K: 6144 x 2048 24 / 24,
     160 rows 21 / 26, 256 28 / 28."""
     sk, code = slab_parts(m, n, k, cus)
     if residual:
-        most = 224 if k < 8192 else 768 if k < 12288 else 1 << 31
-        return None if m > most or sk < 2 else (sk, code)
+        most = 192 if k < 5120 else 224 if k < 8192 else 768 if k < 12288 else 1 << 31
+        wgs = sk * (n // 128 if m <= 256 else n // 256 * -(-m // 256))
+        few = 4 * wgs < 3 * cus if k < 5120 else 192 < m <= 256 and 2 * wgs <= cus
+        return None if m > most or sk < 2 or few else (sk, code)
     return (sk, code) if sk >= 4 and m <= 256 and k >= 2560 and (n >= 6144 or (n >= 4608 and m >= 160)) else None
 
 

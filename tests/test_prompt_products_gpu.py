@@ -129,7 +129,10 @@ def test_parts_of_k():
     (6144, 2560, False, {129: 5, 256: 5}, [300]), (6144, 2048, False, {}, [129, 160, 256]), (3840, 5120, False, {}, [129, 256]), (3072, 4096, False, {}, [129, 256]),
     (1536, 1024, False, {}, [129, 256]), (1536, 4096, False, {}, [129, 256]), (1280, 8192, False, {}, [129, 256]), (10240, 8192, False, {}, [129, 256]),
     # o and down
-    (4096, 14336, True, {129: 8, 256: 8, 257: 8, 1024: 4, 2048: 2}, [2300]), (4096, 11008, True, {192: 4, 768: 4}, [769])])
+    (4096, 14336, True, {129: 8, 256: 8, 257: 8, 1024: 4, 2048: 2}, [2300]), (4096, 11008, True, {192: 4, 257: 4, 768: 4}, [193, 256, 769]),
+    (2560, 9728, True, {129: 8, 256: 8, 768: 8}, [769]), (2048, 5632, True, {129: 8, 192: 8}, [193, 256, 257]), (5120, 5120, True, {129: 5, 224: 5}, [225, 300]),
+    (4096, 4096, True, {129: 8, 192: 8}, [193, 224, 300]), (3072, 3072, True, {129: 8, 192: 8}, [193, 256]), (2560, 4096, True, {}, [129, 192, 224, 300]),
+    (2048, 2048, True, {}, [129, 192, 224]), (1024, 1024, True, {}, [129, 224])])
 def test_choice_of_slabs(n, k, residual, own, library):
     """The parts that are taken, and where the library is, on a device of 256 compute units."""
     for m, sk in own.items():
