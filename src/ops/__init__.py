@@ -777,11 +777,18 @@ def prompt_silu_tiles(m: int, inter: int, k: int, cus: int) -> Optional[int]:
       28672 x 4096   129 rows 61 / 65 / 58, 161 66 / 68 / 59, 200 72 / 75 / 77, 256 76 / 78 / 79, 257 80 / 78 / 109, 512 107 / 105, 768 171 / 167,
                      1200 268 / 253, 2048 394 / 381, 3000 582 / 563, 4096 706 / 724, 8192 1418 / 1430
       57344 x 8192   129 201 / 189 / 242, 256 224 / 245, 400 386 / 370, 700 576 / 555, 1024 780 / 732, 2048 1357 / 1370
-    One row tile leaves CUs idle with tiles of 256: up to 256 rows tiles of 128 where these fill the chip once. (Between 169 and 256 rows the product
-    alone is as fast as the library's two launches; a whole step of four Llama layers is faster with it: 192 rows 915 / 883, 224 947 / 930, 256 969 / 951.)"""
+    Up to 256 rows tiles of 128 where these fill the chip once and not twice. (Between 169 and 256 rows the product alone is as fast as the library's two launches;
+    a whole step of four Llama layers is faster with it: 192 rows 915 / 883, 224 947 / 930, 256 969 / 951.) Where tiles are few, compute units idle: whole
+    steps, us a layer that the own product takes more than the library's. Tiles of 128, inter x k: 2048 x 1024 129 rows +4, 256 +8; 4096 x 2048 +9, +8; 8192 x 2048 0,
+    +4 (192 rows 0); 9728 x 2560 -4, 0; 8192 x 3072 +6, +8; 11008 x 4096 -2, +3 (192 rows -5); 14336 x 4096 -4, -2; 13824 x 5120 0, +4 (224 rows +10). Tiles
+    of 256, inter x k and how many: 2048 x 1024 32 +4, 64 +2, 96 and 160 +1; 4096 x 2048 64 +4, 96 +2, 128 0, 192 -2; 8192 x 2048 128 +1, 256 -6, 640 -19; 8192 x 3072 128 0, 256 -7; a
+    little more than one turn of all compute units 11008 x 4096 258 +10, 5632 x 2048 264 +2, but 9728 x 2560 304 -11."""
     if m <= 256 and inter // 64 <= cus:
-        return 96
-    return None if 168 < m <= 256 or m > (3072 if inter * k <= 1 << 26 else 1536) else 0
+        return 96 if k <= 4096 and 16 * (inter // 64) >= (9 if m <= 192 else 14) * cus else None
+    tiles = inter // 128 * -(-m // 256)
+    if 168 < m <= 256 or m > (3072 if inter * k <= 1 << 26 else 1536):
+        return None
+    return 0 if k >= 2048 and 16 * tiles >= 9 * cus and not 8 * cus < 8 * tiles <= 9 * cus else None
 
 
 def prompt_silu_mul(x: torch.Tensor, w_gate_up: torch.Tensor, row_scale: torch.Tensor) -> torch.Tensor:

@@ -138,3 +138,13 @@ def test_choice_of_slabs(n, k, residual, own, library):
     for m, sk in own.items():
         assert ops.prompt_slab_parts(m, n, k, 256, residual) == (sk, 96 if m <= 256 else 0)
     assert all(ops.prompt_slab_parts(m, n, k, 256, residual) is None for m in library)
+
+
+@pytest.mark.parametrize("inter,k,own,library", [
+    (14336, 4096, {129: 96, 256: 96, 257: 0, 600: 0, 3072: 0}, [3073]), (11008, 4096, {129: 96, 192: 96, 257: 0, 769: 0}, [193, 256, 513, 768]),
+    (9728, 2560, {129: 96, 192: 96, 257: 0}, [193, 256]), (8192, 2048, {513: 0, 2500: 0}, [129, 256, 257, 512]), (13824, 5120, {257: 0, 1000: 0}, [129, 160, 256, 1537]),
+    (28672, 8192, {129: 0, 168: 0, 257: 0, 1536: 0}, [169, 256, 1537]), (4096, 2048, {1281: 0, 2500: 0}, [129, 256, 300, 1000, 1024]), (2048, 1024, {}, [129, 160, 256, 300, 1500, 2500])])
+def test_choice_of_gate_tiles(inter, k, own, library):
+    """Tiles of the gate and up product, and where the library's is taken, on a device of 256 compute units."""
+    assert {m: ops.prompt_silu_tiles(m, inter, k, 256) for m in own} == own
+    assert all(ops.prompt_silu_tiles(m, inter, k, 256) is None for m in library)
