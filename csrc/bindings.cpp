@@ -2,6 +2,8 @@
 // validates device/dtype/shape up front and throws on mismatch — a wrong shape
 // never reaches a kernel (a faulting kernel can take down every GPU on the
 // host) — then launches on the current HIP stream (graph-capture safe).
+#include <algorithm>
+#include <climits>
 #include <cstdlib>
 
 #include <torch/extension.h>
@@ -216,7 +218,7 @@ void rope_and_cache(Tensor qkv, Tensor positions, Tensor cos_sin, Tensor slot_ma
 
 void attn_prefill(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor block_tables, Tensor cu_q,
                   Tensor ctx_lens, int64_t max_q_len, int64_t hq, int64_t hkv, double scale, Tensor cos_sin,
-                  Tensor q_scale) {
+                  Tensor q_scale, int64_t max_ctx) {
   CHK_CUDA(q);
   CHK_BF16(q);
   CHK_BF16(out);
@@ -248,7 +250,7 @@ void attn_prefill(Tensor out, Tensor q, Tensor k_cache, Tensor v_cache, Tensor b
                                    ctx_lens.data_ptr<int>(), (int)nseq, (int)max_q_len, (int)hq, (int)hkv, (int)D,
                                    (int)k_cache.size(2), (float)scale, cur_stream(),
                                    rot ? cos_sin.data_ptr<float>() : nullptr, rot ? (int)cos_sin.size(0) : 0,
-                                   opt_row_scale(q_scale, q.size(0), q, "attn_prefill")));
+                                   opt_row_scale(q_scale, q.size(0), q, "attn_prefill"), (int)std::clamp<int64_t>(max_ctx, 0, INT_MAX)));
 }
 
 // counters: int32 [>= num_seqs * hkv], zero before first use (the kernel re-arms them); an empty tensor
@@ -1175,6 +1177,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("silu_and_mul_views", &silu_and_mul_views);
   m.def("rope_and_cache", &rope_and_cache);
   m.def("attn_prefill", &attn_prefill);
+  m.def("attn_prefill_groups", &die::attn_prefill_groups);
   m.def("attn_decode", &attn_decode);
   m.def("attn_decode_fused", &attn_decode_fused);
   m.def("decode_partials", &decode_partials);

@@ -779,11 +779,29 @@ __global__ void __launch_bounds__(128) attn_decode_reduce_kernel(bf16_t* __restr
   out[((int64_t)seq * hq + head) * D + d] = f2bf(np > 0 ? acc / L : 0.f);
 }
 
+// Groups of 4 waves that share a row tile's keys. Where row tiles leave compute units idle the chain of a tile's stages is what takes the time, and two
+// groups share it (one workgroup per CU). One group / two, us, 32 heads in 8 key heads unless said: 1 x 200 12.0 / 11.5, 1 x 300 16.5 / 13.9, 1 x 450 21.3 / 17.1, 1 x 1000 39.0 / 29.6,
+// 1 x 450 behind 1500 67 / 48, 2 x 500 23.8 / 19.3; of few keys 1 x 129 9.5 / 10.1 and, with one query head per key head, 1 x 256 15.1 / 15.4 (with two 1 x 200 11.8 / 12.2).
+// Beyond one turn of the compute units it depends on which tiles share one. An XCD has a run of the list of tiles, each (sequence, key head)'s longest first. Up to a
+// ninth turn the last ones start behind short ones where an XCD has not much less than a whole list of them, and where not all are long for the keys before the step: 4 lists
+// 1 x 2100 72 / 61 (behind 1050 105 / 105), 8 1 x 1040 40 / 31 (behind 520 57 / 42, 2080 103 / 103), 24 1 x 1500 56 / 41, but 36 1 x 1000 42 / 49, 2 of 376 tiles 101 / 115 and one 97 / 125. Up
+// to two turns whole lists go to XCDs: 8 of them 1 x 1500 54 / 40, 1 x 2048 72 / 62 (behind 512 89 / 82, 1024 106 / 105, 4096 211 / 235), 8 heads per key head 1 x 1000 40 / 38 (behind 250
+// 49 / 49); 16 of them with many stages 1 x 4096 136 / 115, 2 x 2000 72 / 65, few 2 x 1000 40 / 38 but behind 128 45 / 46; others not: 12 lists 3 x 1300 49 / 68, 32
+// 1 x 2048 76 / 93, 64 4 x 1000 44 / 61, 4 1 x 4096 138 / 147. (Four groups of 2 waves 1 x 1000 34, two of them 31.)
+int attn_prefill_groups(int max_q_len, int num_seqs, int hq, int hkv, int64_t keys, int cus) {
+  const int G = hq / hkv, rows = 4 * (32 / (G > 32 ? 32 : G));
+  const int64_t lists = (int64_t)num_seqs * hkv, tiles = (max_q_len + rows - 1) / rows * lists;
+  if (tiles <= cus) return max_q_len >= 200 && keys >= (G >= 4 ? 200 : G == 2 ? 256 : 288) ? 2 : 1;
+  if (max_q_len < 1000) return 1;
+  if (8 * tiles <= 9 * (int64_t)cus) return lists >= 4 && lists <= 32 && 2 * keys <= 3 * (int64_t)max_q_len ? 2 : 1;
+  return tiles <= 2 * (int64_t)cus && 4 * keys <= 5 * (int64_t)max_q_len && (lists == 8 || (lists == 16 && max_q_len >= 1500)) ? 2 : 1;
+}
+
 hipError_t launch_attn_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, const bf16_t* k_cache,
                                const bf16_t* v_cache, const int* block_tables, int bt_stride, const int* cu_q,
                                const int* ctx_lens, int num_seqs, int max_q_len, int hq, int hkv, int head_dim,
                                int block_size, float scale, hipStream_t s, const float* cos_sin, int n_pos,
-                               const float* q_scale) {
+                               const float* q_scale, int max_ctx) {
   if (num_seqs == 0 || max_q_len == 0) return hipSuccess;
   if (cos_sin != nullptr && n_pos < 1) return hipErrorInvalidValue;
   if (q_scale != nullptr && cos_sin == nullptr) return hipErrorInvalidValue;  // applied with the rotation
@@ -795,13 +813,7 @@ hipError_t launch_attn_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, c
   // for short ones, where more, shorter q tiles fill the chip (64 x 256: 119 vs 132 us; 32 x 512 within 1.5 %:
   // profiles/r5_prefill_attn_nw_ns.jsonl)
   const bool short_q = max_q_len <= 256;
-  // Where row tiles leave compute units idle, or next to that behind many keys, the chain of a tile's stages is what takes the time, and two groups of 4
-  // waves share it. One group / two, us, 32 heads in 8 groups: 1 x 200 11.7 / 11.4, 1 x 300 16.5 / 13.9, 1 x 442 20.8 / 16.8, 1 x 1000 37.9 / 29.3, 1 x 300
-  // behind 1500 60.9 / 43.6, 2 x 500 23.2 / 18.9; up to two tiles per CU 1 x 1500 53 / 40, 1 x 2048 71 / 60, 2 x 1000 40 / 38, but 3 x 500 27 / 32, 4 x 512 26 / 34;
-  // of few keys 4 x 128 9.7 / 10.3, 1 x 129 9.5 / 10.1; beyond, 1 x 4096 160 / 197. (Four groups of 2 waves 1 x 1000 34, two of them 31.)
-  const int tpb4 = 4 * (32 / (G > 32 ? 32 : G));
-  const int64_t tiles4 = (int64_t)((max_q_len + tpb4 - 1) / tpb4) * num_seqs * hkv, cus = num_cus();
-  const bool two = (tiles4 <= cus && max_q_len >= 200) || (tiles4 <= 2 * cus && max_q_len >= 1000);
+  const bool two = attn_prefill_groups(max_q_len, num_seqs, hq, hkv, max_ctx > 0 ? std::min<int64_t>(max_ctx, (int64_t)bt_stride * block_size) : (int64_t)bt_stride * block_size, num_cus()) == 2;
   const int NWr = short_q || two ? 4 : 8, NSr = short_q || two ? 1 : 2, KGr = two ? 2 : 1;
   const int tpb = NWr * (32 / (G > 32 ? 32 : G));
   dim3 grid((max_q_len + tpb - 1) / tpb, num_seqs, hkv), block(64 * NWr * KGr);

@@ -45,7 +45,9 @@ hipError_t launch_attn_prefill(bf16_t* out, const bf16_t* q, int64_t q_stride, c
                                const bf16_t* v_cache, const int* block_tables, int bt_stride, const int* cu_q,
                                const int* ctx_lens, int num_seqs, int max_q_len, int hq, int hkv, int head_dim,
                                int block_size, float scale, hipStream_t s, const float* cos_sin = nullptr,
-                               int n_pos = 0, const float* q_scale = nullptr);
+                               int n_pos = 0, const float* q_scale = nullptr, int max_ctx = 0);
+// groups of waves over a row tile's keys that it takes: 1 or 2 (keys: of the longest sequence, or more; max_ctx > 0 above says how many that are)
+int attn_prefill_groups(int max_q_len, int num_seqs, int hq, int hkv, int64_t keys, int cus);
 // Fused decode-attention prologue (attention.hip, attn_decode_v3_kernel<G, true>).
 struct AttnDecodeFuse {
   const float* slab = nullptr;      // qkv projection split-K slabs [sk][M][width] fp32

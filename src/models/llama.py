@@ -537,7 +537,7 @@ class CausalLM:
         if meta.is_prefill:
             return ops.attn_prefill(q, k_cache, v_cache, meta.block_tables, meta.cu_q, meta.ctx_lens,
                                     meta.max_q_len, hq, hkv, self.scale, cos_sin=self.cos_sin if fuse_q else None,
-                                    q_scale=rs)
+                                    q_scale=rs, max_ctx=meta.max_ctx)
         return ops.attn_decode(q, k_cache, v_cache, meta.block_tables, meta.ctx_lens, meta.max_ctx, hq, hkv,
                                self.scale, part_o=meta.part_o, part_ml=meta.part_ml, counters=meta.attn_cnt)
 
@@ -598,7 +598,7 @@ class CausalLM:
                                         k_cache, v_cache, hq, hkv, d)
             if meta.is_prefill:
                 attn = ops.attn_prefill(q, k_cache, v_cache, meta.block_tables, meta.cu_q, meta.ctx_lens,
-                                        meta.max_q_len, hq, hkv, self.scale)
+                                        meta.max_q_len, hq, hkv, self.scale, max_ctx=meta.max_ctx)
             else:
                 attn = ops.attn_decode(q, k_cache, v_cache, meta.block_tables, meta.ctx_lens, meta.max_ctx, hq,
                                        hkv, self.scale, part_o=meta.part_o, part_ml=meta.part_ml,

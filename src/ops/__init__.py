@@ -143,10 +143,12 @@ def rope_and_cache(qkv, positions, cos_sin, slot_mapping, k_cache, v_cache, hq: 
 
 def attn_prefill(q, k_cache, v_cache, block_tables, cu_q, ctx_lens, max_q_len: int, hq: int, hkv: int,
                  scale: float, out: Optional[torch.Tensor] = None, cos_sin: Optional[torch.Tensor] = None,
-                 q_scale: Optional[torch.Tensor] = None) -> torch.Tensor:
+                 q_scale: Optional[torch.Tensor] = None, max_ctx: int = 0) -> torch.Tensor:
     """Causal paged prefill attention. cos_sin ([max_pos, 128] fp32): q is NOT yet rotated, the kernel
     applies RoPE to each Q row as it loads it (token positions ctx - q_len + i). q_scale (fp32 [T], with
-    cos_sin): each Q row is also scaled by its token's RMSNorm scale (:func:`rms_row_scale`)."""
+    cos_sin): each Q row is also scaled by its token's RMSNorm scale (:func:`rms_row_scale`). max_ctx: the longest
+    context, where it is known (0: as many keys as the tables hold); it chooses how waves share the keys, which changes no more than
+    the order of sums."""
     if not q.is_cuda:
         assert cos_sin is None and q_scale is None, "the CPU reference path takes a rotated q"
         return ref.attention(q, k_cache, v_cache, block_tables, cu_q, ctx_lens, hq, hkv, scale).reshape(q.shape[0], -1)
@@ -155,7 +157,7 @@ def attn_prefill(q, k_cache, v_cache, block_tables, cu_q, ctx_lens, max_q_len: i
     assert q_scale is None or cos_sin is not None, "the Q row scale is applied with the rotation"
     e = _empty(q.device)
     _kern().attn_prefill(out, q, k_cache, v_cache, block_tables, cu_q, ctx_lens, max_q_len, hq, hkv, scale,
-                         cos_sin if cos_sin is not None else e, q_scale if q_scale is not None else e)
+                         cos_sin if cos_sin is not None else e, q_scale if q_scale is not None else e, max_ctx)
     return out
 
 
