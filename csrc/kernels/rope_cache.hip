@@ -200,12 +200,15 @@ hipError_t launch_rope_and_cache_slab(bf16_t* q_out, const float* slab, int sk, 
 // ----------------------------------------------------------------------------
 // The rows of a prompt step that its last layer goes on with, and what the attention of one query per row needs: kept row i of sequence s (the
 // last with cu_q[s] <= keep[i]) -> its query and residual, s's block table and context length, offsets 0 .. n, and its norm scale. One workgroup
-// per kept row. Bound by its launch; as eight launches (gathers, a search, a range) it took some 30 us more in steps of 8 and 13 sequences (8 x 100 rows of
+// per kept row. A row outside the step is read nowhere: its query, residual and scale are NaN, so that what is made of them can't pass for a
+// result. Bound by its launch; as eight launches (gathers, a search, a range) it took some 30 us more in steps of 8 and 13 sequences (8 x 100 rows of
 // four Llama layers 1495 -> 1463), 3 - 7 in those of one.
 __global__ void __launch_bounds__(256) keep_rows_kernel(KeepRowsArgs a) {
   __shared__ int before[4];
   const int i = blockIdx.x, tid = threadIdx.x;
-  const int64_t row = min(max(a.keep[i], (int64_t)0), (int64_t)a.rows - 1);
+  const int64_t kept = a.keep[i], row = min(max(kept, (int64_t)0), (int64_t)a.rows - 1);
+  const bool inside = kept == row;
+  const uint4 nans = make_uint4(0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u);
   int cnt = 0;
   for (int j = tid; j < a.num_seqs; j += 256) cnt += a.cu_q[j + 1] <= row ? 1 : 0;
 #pragma unroll
@@ -216,13 +219,13 @@ __global__ void __launch_bounds__(256) keep_rows_kernel(KeepRowsArgs a) {
   uint4* qo = reinterpret_cast<uint4*>(a.q_out) + (int64_t)i * (a.q_width / 8);
   uint4* ro = reinterpret_cast<uint4*>(a.resid_out) + (int64_t)i * (a.hidden / 8);
   if (a.cos_sin == nullptr)
-    for (int c = tid; c < a.q_width / 8; c += 256) qo[c] = q[c];
-  for (int c = tid; c < a.hidden / 8; c += 256) ro[c] = r[c];
+    for (int c = tid; c < a.q_width / 8; c += 256) qo[c] = inside ? q[c] : nans;
+  for (int c = tid; c < a.hidden / 8; c += 256) ro[c] = inside ? r[c] : nans;
   __syncthreads();
   const int s = min(before[0] + before[1] + before[2] + before[3], a.num_seqs - 1);
   if (a.cos_sin != nullptr) {   // heads of 128, turned at their sequence's last position and scaled (as the prompt attention does on loading them)
     const float* cs = a.cos_sin + (int64_t)min(max(a.ctx_lens[s] - 1, 0), a.n_pos - 1) * 128;
-    const float scale = a.rs != nullptr ? a.rs[row] : 1.0f;
+    const float scale = !inside ? NAN : a.rs != nullptr ? a.rs[row] : 1.0f;
     for (int it = tid; it < a.q_width / 16; it += 256) {
       const int at = it / 8 * 16 + it % 8, d = it % 8 * 8;   // this chunk and the one 64 columns on
       float x[8], y[8], xo[8], yo[8];
@@ -243,7 +246,7 @@ __global__ void __launch_bounds__(256) keep_rows_kernel(KeepRowsArgs a) {
     a.ctx_out[i] = a.ctx_lens[s];
     a.cu_out[i + 1] = i + 1;
     if (i == 0) a.cu_out[0] = 0;
-    if (a.rs != nullptr) a.rs_out[i] = a.rs[row];
+    if (a.rs != nullptr) a.rs_out[i] = inside ? a.rs[row] : NAN;
   }
 }
 

@@ -867,7 +867,7 @@ def keep_rows(keep: torch.Tensor, cu_q: torch.Tensor, block_tables: torch.Tensor
     """What a prompt step's last layer goes on with for its rows ``keep`` (int64): their queries q[keep, :q_width] and residuals, the block table and
     context length of each one's sequence (rows cu_q[i] .. cu_q[i + 1] are sequence i's), offsets 0 .. n (int32) and the rows' scales rs (or None).
     cos_sin ([max_pos, 128] fp32): the queries, heads of 128, come turned at their sequence's last position and scaled by rs, which is then not
-    returned. One launch on the GPU."""
+    returned. A row outside the step raises on the CPU; on the GPU, in one launch, its query, residual and scale come as NaN."""
     rows = (q, resid)
     ints = (cu_q, block_tables, ctx_lens)
     if (q.is_cuda and native_available() and all(t.dtype == torch.bfloat16 and t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0

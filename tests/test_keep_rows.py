@@ -53,3 +53,23 @@ def test_turned_queries(scaled):
     assert got[5] is None and want[5] is None and all(torch.equal(a.cpu(), b) for a, b in zip(got[1:5], want[1:5]))
     a, b = got[0].float().cpu().view(3, 3, 2, 64), want[0].float().view(3, 3, 2, 64)
     assert bool(((a - b).abs() <= 2.0 ** -8 * b.norm(dim=2, keepdim=True)).all())
+
+
+@pytest.mark.parametrize("scaled", [True, False])
+@pytest.mark.parametrize("turned", [True, False])
+@pytest.mark.parametrize("dev", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_rows_outside_the_step(dev, scaled, turned):
+    """Refused on the CPU; NaN on the GPU, never another row's values, beside rows that are as ever."""
+    cu, tables, ctx, q, width, resid, rs = _step(dev, [3, 1, 0, 9], width=384)
+    args = (cu, tables, ctx, q, width, resid, rs if scaled else None, torch.ones(60, 128, device=dev) if turned else None)
+    keep = torch.tensor([-1, 13, 12, 2 ** 40], device=dev)
+    if dev == "cpu":
+        for at in (keep[:1], keep[1:2], keep[3:]):
+            with pytest.raises((IndexError, RuntimeError)):
+                ops.keep_rows(at, *args)
+        return
+    got, inner = ops.keep_rows(keep, *args), ops.keep_rows(keep[2:3], *args)
+    for a, b in zip(got[:2] + got[5:], inner[:2] + inner[5:]):
+        if a is not None:
+            assert bool(a[[0, 1, 3]].isnan().all()) and torch.equal(a[2:3], b) and not bool(b.isnan().any())
+    assert torch.equal(got[4].cpu(), torch.arange(5, dtype=torch.int32)) and torch.equal(got[3][2:3], inner[3]) and torch.equal(got[2][2:3], inner[2])
