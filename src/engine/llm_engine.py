@@ -23,6 +23,7 @@ from typing import Callable, Dict, List, Optional
 
 import torch
 
+from src import ops
 from src.config import EngineConfig
 from src.engine.block_manager import KVBlockManager
 from src.engine.model_runner import KVPool, ModelRunner
@@ -53,6 +54,8 @@ def plan_kv_blocks(arch: ArchConfig, model: CausalLM, cfg: EngineConfig, device:
     # activations of one prefill step (qkv, attn, gate_up, act, residual ...) + logits + slack
     act = t * (3 * h + (model.hq + 2 * model.hkv) * arch.head_dim + 3 * inter) * 2
     act += cfg.max_num_seqs * arch.vocab_size * 4 + (2 << 30)
+    # a layer's down, qkv and o in parts of K, the kept rows' splits
+    act += 3 * ops.PROMPT_SLAB_BYTES + ops.KEPT_PARTIALS_BYTES
     budget = min(free - act, cfg.gpu_memory_fraction * total - (total - free) - act)
     return max(16, int(budget // per_block))
 

@@ -494,14 +494,13 @@ class CausalLM:
             meta.kv_hook(li)
         if n == 0:
             return residual[:0]
-        # One query per sequence: behind many keys by the decode kernel, which splits them, where the prompt kernel goes through them in one chain. us,
-        # prompt / decode kernel: 1 sequence of 300 keys 13.5 / 14.4, 512 19.5 / 14.6, 1000 35 / 15, 2000 66 / 15; 32 of 512 20.9 / 16.4, of 1000 37 / 25
-        split = qkv.is_cuda and max(meta.max_q_len, meta.max_ctx) >= 400 and n * hkv <= 256 and ops.decode_attn_merges(hq, hkv, k_cache.shape[2])
+        keys = meta.block_tables.shape[1] * k_cache.shape[2]
+        keys = min(meta.max_ctx or keys, keys)
+        split = qkv.is_cuda and ops.kept_rows_split(n, hq, hkv, k_cache.shape[2], max(meta.max_q_len, meta.max_ctx), keys)
         q, res, tables, ctx, cu1, qs = ops.keep_rows(keep, meta.cu_q, meta.block_tables, meta.ctx_lens, qkv, hq * d, residual, rs,
                                                      cos_sin=self.cos_sin if fuse_q and split else None)
         if split:
-            room = tables.shape[1] * k_cache.shape[2]
-            attn = ops.attn_decode(q, k_cache, v_cache, tables, ctx, min(meta.max_ctx or room, room), hq, hkv, self.scale)
+            attn = ops.attn_decode(q, k_cache, v_cache, tables, ctx, keys, hq, hkv, self.scale)
         else:
             attn = ops.attn_prefill(q, k_cache, v_cache, tables, cu1, ctx, 1, hq, hkv, self.scale, cos_sin=self.cos_sin if fuse_q else None, q_scale=qs)
         o = self.tp.all_reduce(ops.linear(attn, lw.o))

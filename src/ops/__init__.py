@@ -171,6 +171,19 @@ def decode_attn_merges(hq: int, hkv: int, block_size: int) -> bool:
     return hq % hkv == 0 and hq // hkv in (1, 2, 4, 8) and block_size == 16
 
 
+KEPT_PARTIALS_BYTES = 128 << 20   # most that the splits of a prompt step's kept rows may take
+
+
+def kept_rows_split(n: int, hq: int, hkv: int, block_size: int, seen: int, keys: int) -> bool:
+    """Whether the attention of n kept rows of a prompt step, one query per sequence, goes to :func:`attn_decode`, which splits the keys, where
+    :func:`attn_prefill` goes through them in one chain: ``seen`` keys or more of the longest sequence, which has ``keys`` at most. us with
+    :func:`keep_rows`, prompt / decode kernel, 32 heads in 8 groups: 1 sequence of 400 keys 21.5 / 13.0, 1000 40 / 13, 2000 71 / 15, 8000 258 / 28; 32 of 400 24 / 20, of 1000 44 / 30, of
+    2000 77 / 52; 1, 2 and 8 heads per group alike. The partial sums, 520 bytes per row, head and 128 keys, are bounded: many sequences with one of
+    100 k keys among them, or unknown contexts in tables as wide as that, keep the prompt kernel."""
+    return (seen >= 400 and n * hkv <= 256 and decode_attn_merges(hq, hkv, block_size)
+            and n * hq * -(-keys // 128) * 520 <= KEPT_PARTIALS_BYTES)
+
+
 def attn_decode(q, k_cache, v_cache, block_tables, ctx_lens, max_ctx: int, hq: int, hkv: int, scale: float,
                 part_o: Optional[torch.Tensor] = None, part_ml: Optional[torch.Tensor] = None,
                 out: Optional[torch.Tensor] = None, counters: Optional[torch.Tensor] = None,
@@ -727,6 +740,9 @@ def _dense_gemm_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
 @functools.lru_cache(maxsize=None)
 def _num_cus(device: int) -> int:
     return torch.cuda.get_device_properties(device).multi_processor_count
+
+
+PROMPT_SLAB_BYTES = 64 << 20   # most that the slabs of one product take: 256 tiles of 256 x 256 sums
 
 
 def slab_parts(m: int, n: int, k: int, cus: int):

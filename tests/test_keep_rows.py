@@ -73,3 +73,35 @@ def test_rows_outside_the_step(dev, scaled, turned):
         if a is not None:
             assert bool(a[[0, 1, 3]].isnan().all()) and torch.equal(a[2:3], b) and not bool(b.isnan().any())
     assert torch.equal(got[4].cpu(), torch.arange(5, dtype=torch.int32)) and torch.equal(got[3][2:3], inner[3]) and torch.equal(got[2][2:3], inner[2])
+
+
+@pytest.mark.parametrize("n,hq,hkv,bs,seen,keys,split", [
+    (1, 32, 8, 16, 400, 400, True), (1, 32, 8, 16, 399, 399, False), (32, 32, 8, 16, 512, 2048, True), (33, 32, 8, 16, 512, 512, False), (1, 32, 1, 16, 1000, 1000, False),
+    (1, 16, 1, 16, 1000, 1000, False), (1, 32, 8, 32, 1000, 1000, False),
+    # partial sums of 520 bytes per row, head and 128 keys: 128 MiB of them, and one part more
+    (32, 32, 8, 16, 32256, 32256, True), (32, 32, 8, 16, 32257, 32257, False), (32, 32, 8, 16, 512, 131072, False), (1, 32, 8, 16, 512, 131072, True)])
+def test_choice_of_split_keys(n, hq, hkv, bs, seen, keys, split):
+    assert ops.kept_rows_split(n, hq, hkv, bs, seen, keys) is split
+
+
+def test_scratch_of_prompt_steps_is_counted(monkeypatch):
+    """The cache leaves room for a layer's slabs and the kept rows' splits, beside the slack for the rest."""
+    from types import SimpleNamespace
+
+    from src.config import EngineConfig
+    from src.engine.llm_engine import plan_kv_blocks
+    from src.engine.model_runner import KVPool
+    from src.models.presets import get_preset
+
+    free, arch = 1 << 36, get_preset("llama3-8b")
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda dev: (free, free))
+    cfg = EngineConfig(max_num_seqs=32, max_num_batched_tokens=4096, gpu_memory_fraction=1.0)
+    blocks = plan_kv_blocks(arch, SimpleNamespace(hq=32, hkv=8, inter=14336), cfg, torch.device("cuda"))
+    left = free - blocks * KVPool.bytes_per_block(arch.num_layers, 8, cfg.block_size, 128)
+    rows = 4096 * (3 * 4096 + 48 * 128 + 3 * 14336) * 2 + 32 * arch.vocab_size * 4
+    assert left - rows - (2 << 30) >= 3 * ops.PROMPT_SLAB_BYTES + ops.KEPT_PARTIALS_BYTES
+    for m in (129, 256, 257, 1024, 2048):
+        for n, k in ((4096, 14336), (8192, 28672), (6144, 4096), (5120, 5120)):
+            for residual in (True, False):
+                plan = ops.prompt_slab_parts(m, n, k, 256, residual)
+                assert plan is None or plan[0] * m * n * 4 <= ops.PROMPT_SLAB_BYTES
