@@ -496,7 +496,7 @@ class CausalLM:
             return residual[:0]
         keys = meta.block_tables.shape[1] * k_cache.shape[2]
         keys = min(meta.max_ctx or keys, keys)
-        split = qkv.is_cuda and ops.kept_rows_split(n, hq, hkv, k_cache.shape[2], max(meta.max_q_len, meta.max_ctx), keys)
+        split = qkv.is_cuda and ops.kept_rows_split(n, hq, hkv, k_cache.shape[2], x.shape[0], max(meta.max_q_len, meta.max_ctx), keys)
         q, res, tables, ctx, cu1, qs = ops.keep_rows(keep, meta.cu_q, meta.block_tables, meta.ctx_lens, qkv, hq * d, residual, rs,
                                                      cos_sin=self.cos_sin if fuse_q and split else None)
         if split:

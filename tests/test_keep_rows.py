@@ -75,13 +75,15 @@ def test_rows_outside_the_step(dev, scaled, turned):
     assert torch.equal(got[4].cpu(), torch.arange(5, dtype=torch.int32)) and torch.equal(got[3][2:3], inner[3]) and torch.equal(got[2][2:3], inner[2])
 
 
-@pytest.mark.parametrize("n,hq,hkv,bs,seen,keys,split", [
-    (1, 32, 8, 16, 400, 400, True), (1, 32, 8, 16, 399, 399, False), (32, 32, 8, 16, 512, 2048, True), (33, 32, 8, 16, 512, 512, False), (1, 32, 1, 16, 1000, 1000, False),
-    (1, 16, 1, 16, 1000, 1000, False), (1, 32, 8, 32, 1000, 1000, False),
+@pytest.mark.parametrize("n,hq,hkv,bs,rows,seen,keys,split", [
+    (1, 32, 8, 16, 400, 400, 400, True), (1, 32, 8, 16, 399, 399, 399, False), (33, 32, 8, 16, 1000, 512, 512, False), (1, 32, 1, 16, 1000, 1000, 1000, False),
+    (1, 16, 1, 16, 1000, 1000, 1000, False), (1, 32, 8, 32, 1000, 1000, 1000, False),
+    # rows against the longest context
+    (8, 32, 8, 16, 4096, 512, 2048, True), (9, 32, 8, 16, 4097, 512, 512, False), (32, 32, 8, 16, 16384, 512, 512, False), (32, 32, 8, 16, 3200, 1100, 1104, True),
     # partial sums of 520 bytes per row, head and 128 keys: 128 MiB of them, and one part more
-    (32, 32, 8, 16, 32256, 32256, True), (32, 32, 8, 16, 32257, 32257, False), (32, 32, 8, 16, 512, 131072, False), (1, 32, 8, 16, 512, 131072, True)])
-def test_choice_of_split_keys(n, hq, hkv, bs, seen, keys, split):
-    assert ops.kept_rows_split(n, hq, hkv, bs, seen, keys) is split
+    (32, 32, 8, 16, 600, 32256, 32256, True), (32, 32, 8, 16, 600, 32257, 32257, False), (32, 32, 8, 16, 600, 512, 131072, False), (1, 32, 8, 16, 600, 512, 131072, True)])
+def test_choice_of_split_keys(n, hq, hkv, bs, rows, seen, keys, split):
+    assert ops.kept_rows_split(n, hq, hkv, bs, rows, seen, keys) is split
 
 
 def test_scratch_of_prompt_steps_is_counted(monkeypatch):
