@@ -74,10 +74,13 @@ __device__ __forceinline__ int scan64(int x, int lane) {
   return x + (lane >= 16 ? a : 0) + (lane >= 32 ? b : 0) + (lane >= 48 ? c : 0);
 }
 
-// the first row of expert i <= experts (without offsets every part has all rows, from 0 on); the rows of it
-__device__ __forceinline__ int first_row(const MoeGemmArgs& a, int i) { return a.offsets != nullptr ? a.offsets[min(i, a.experts)] : 0; }
-__device__ __forceinline__ int end_row(const MoeGemmArgs& a, int i) {
-  return a.offsets != nullptr ? a.offsets[min(i + 1, a.experts)] : i < a.experts ? a.rows : 0;
+// What a launch goes through: rows of experts by offsets; one product's rows; one product's, with a part of K in the place of an expert. (Known to the compiler, so that an
+// expert's two offsets are loaded together: behind a test of the pointer they were loaded one after the other, per tile.)
+constexpr int OF_EXPERTS = 0, OF_ONE = 1, OF_PARTS = 2;
+// the first row of expert i <= experts, and the one behind its last
+template <int OF> __device__ __forceinline__ int first_row(const MoeGemmArgs& a, int i) { return OF == OF_EXPERTS ? a.offsets[min(i, a.experts)] : 0; }
+template <int OF> __device__ __forceinline__ int end_row(const MoeGemmArgs& a, int i) {
+  return OF == OF_EXPERTS ? a.offsets[min(i + 1, a.experts)] : i < a.experts ? a.rows : 0;
 }
 
 struct Tile {
@@ -91,7 +94,7 @@ struct Tile {
 // half of the CUs idle (16 of 2048 x 1024, 256 rows: 33.0 / 34.6).
 __device__ __forceinline__ int first_stage(int n, int nst) { return (int)((uint64_t)((uint32_t)n * 2654435769u) * (uint32_t)nst >> 32); }
 __device__ __forceinline__ int stage_of(int s, int turn, int nst) { return s + turn >= nst ? s + turn - nst : s + turn; }
-__device__ __forceinline__ int stages(const MoeGemmArgs& a) { return a.slab != nullptr ? a.K / (BK * a.experts) : a.K / BK; }   // of a tile
+template <int OF> __device__ __forceinline__ int stages(const MoeGemmArgs& a) { return OF == OF_PARTS ? a.K / (BK * a.experts) : a.K / BK; }   // of a tile
 // The tiles of the launch, found from the offsets by every wave (lane i looks at experts i, i + 64, ...). Tiles of an expert are as even
 // as 32-row pieces allow, at most R rows. XCD i (blocks i, i + 8, ...) takes the i-th eighth of the list, whose neighbours share
 // weights or x rows; its CUs take turns. What is left for less than a turn of all of them is cut into `parts` by rows.
@@ -100,7 +103,7 @@ __device__ __forceinline__ int stages(const MoeGemmArgs& a) { return a.slab != n
 // 64 26); of the whole, 0.7 go with the turns of the CU that has most and 0.3 with the mean of all, as CUs that rest leave the others a
 // higher clock. Over 43 products (200 - 16000 tokens of 5 expert sizes, random routing) that is within 1.8 % of the best R and parts on average;
 // the same R without parts 4.9 %, 256 rows without parts 14 %. (Candidates are weighed by a lane each: one after the other they took 5 us.)
-struct Plan {
+template <int OF> struct Plan {
   int R = 0, per = 0, count = 0, full = 0, parts = 1;   // count: tiles of the own XCD
   int NT, cpx;
   const MoeGemmArgs& a;
@@ -109,7 +112,7 @@ struct Plan {
     constexpr int NH = 5;   // heights 256, 224, .. 128: lanes 4 i + log2(parts)
     int n = 1, filled = 0;  // tiles of the lane's height; rows in whole 32-row pieces
     for (int b = 0; b < a.experts; b += 64) {
-      const int m = end_row(a, b + lane) - first_row(a, b + lane);
+      const int m = end_row<OF>(a, b + lane) - first_row<OF>(a, b + lane);
       filled += 32 * __builtin_amdgcn_readlane(scan64((m + 31) / 32, lane), 63);
 #pragma unroll
       for (int i = 0; i < NH; ++i) {
@@ -148,7 +151,7 @@ struct Plan {
       int o0, o1, before, b = 0;
       uint64_t beyond;
       for (;; b += 64) {
-        o0 = first_row(a, b + lane), o1 = end_row(a, b + lane);
+        o0 = first_row<OF>(a, b + lane), o1 = end_row<OF>(a, b + lane);
         const int own = (o1 - o0 + R - 1) / R * NT, upto = scan64(own, lane);
         beyond = __builtin_amdgcn_ballot_w64(upto > tile);
         before = upto - own;
@@ -167,7 +170,7 @@ struct Plan {
       tile -= g * gs * NT;
       const int h = (rows / 32 + cut - 1) / cut * 32, m0 = (g * gs + tile % gm) * rows + part * h;
       t.n0 = tile / gm;
-      t.turn = mts == 1 ? first_stage(t.e * NT + t.n0, stages(a)) : 0;   // (used where the launch asks for it)
+      t.turn = mts == 1 ? first_stage(t.e * NT + t.n0, stages<OF>(a)) : 0;   // (used where the launch asks for it)
       t.M = min(min(t.M - m0, rows - part * h), h);
       t.r0 += m0;
       if (t.M > 0) return true;
@@ -223,16 +226,17 @@ template <int ACT, class Z> __device__ __forceinline__ void store_row16(Z z, uin
   }
 }
 
-template <int ACT, bool TURN, bool SLAB = false>
+template <int ACT, bool TURN, int OF = OF_EXPERTS>
 __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   constexpr bool GATED = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU;
   constexpr int NO = GATED ? BN / 2 : BN;           // output columns of a tile
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wn = wave % WN, wm = wave / WN, fr = lane & 15, lg = lane >> 4;
-  const int nst = SLAB ? a.K / (BK * a.experts) : a.K / BK;
+  constexpr bool SLAB = OF == OF_PARTS;
+  const int nst = stages<OF>(a);
 
-  const Plan plan(a, a.ncols / NO, lane);
+  const Plan<OF> plan(a, a.ncols / NO, lane);
   int job = (int)(blockIdx.x >> 3);
   Tile t, next;
   if (!plan.find(job, t)) return;
@@ -417,18 +421,19 @@ constexpr int FN = 32 * TN, FUNIT = FN * ROWB;   // weight rows of a tile, bytes
 
 constexpr int FEW_LDS = 160 * 1024;
 
-template <int ACT, int NB, bool SLAB = false>
+template <int ACT, int NB, int OF = OF_EXPERTS>
 __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_few_kernel(MoeGemmArgs a) {
   extern __shared__ __attribute__((aligned(1024))) char smem[];
   constexpr bool GATED = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU;
   constexpr int NO = (GATED ? FN / 2 : FN) * NB;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 31, hi = lane >> 5;
-  const int nst = SLAB ? a.K / (BK * a.experts) : a.K / BK, NT = a.ncols / NO;
+  constexpr bool SLAB = OF == OF_PARTS;
+  const int nst = stages<OF>(a), NT = a.ncols / NO;
 
   // ---- the workgroup's tile: XCD i (blocks i, i + 8, ..) takes the i-th eighth of the list, whose neighbours share x rows or weights
   int total = 0;
   for (int b = 0; b < a.experts; b += 64) {
-    const int m = end_row(a, b + lane) - first_row(a, b + lane);
+    const int m = end_row<OF>(a, b + lane) - first_row<OF>(a, b + lane);
     total += __builtin_amdgcn_readlane(scan64((m + BM - 1) / BM * NT, lane), 63);
   }
   const int per = (total + 7) / 8;
@@ -436,7 +441,7 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_few_kernel(MoeGemmArgs a)
   if ((int)(blockIdx.x >> 3) >= per || tile >= total) return;
   Tile t;
   for (int b = 0;; b += 64) {
-    const int o0 = first_row(a, b + lane), o1 = end_row(a, b + lane);
+    const int o0 = first_row<OF>(a, b + lane), o1 = end_row<OF>(a, b + lane);
     const int own = (o1 - o0 + BM - 1) / BM * NT, upto = scan64(own, lane);
     const uint64_t beyond = __builtin_amdgcn_ballot_w64(upto > tile);
     if (beyond == 0) {   // (there is one: tile < total)
@@ -587,19 +592,19 @@ inline int few_tiles(const MoeGemmArgs& a) {
   return a.rows <= (tiles <= 2 * a.cus ? 144 : 40) * (int64_t)a.experts ? ROWS_128 : ROWS_WHOLE;
 }
 
-template <int ACT, int NB, bool SLAB = false> hipError_t launch_few(const MoeGemmArgs& a, hipStream_t s) {
-  auto* fn = moe_gemm_few_kernel<ACT, NB, SLAB>;
+template <int ACT, int NB, int OF = OF_EXPERTS> hipError_t launch_few(const MoeGemmArgs& a, hipStream_t s) {
+  auto* fn = moe_gemm_few_kernel<ACT, NB, OF>;
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, FEW_LDS);
   if (e != hipSuccess) return e;
   constexpr int NO = (ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU ? FN / 2 : FN) * NB;
-  const int64_t mts = a.offsets == nullptr ? a.experts * (int64_t)((a.rows + BM - 1) / BM) : std::min(a.experts, a.rows) + a.rows / BM;   // at most
+  const int64_t mts = OF != OF_EXPERTS ? a.experts * (int64_t)((a.rows + BM - 1) / BM) : std::min(a.experts, a.rows) + a.rows / BM;   // at most
   const int64_t tiles = mts * (a.ncols / NO);
   hipLaunchKernelGGL(fn, dim3((unsigned)(8 * ((tiles + 7) / 8))), dim3(64 * NW), FEW_LDS, s, a);
   return hipGetLastError();
 }
 
-template <int ACT, bool SLAB> hipError_t launch_whole(const MoeGemmArgs& a, bool turn, hipStream_t s) {
-  auto* fn = turn ? moe_gemm_kernel<ACT, true, SLAB> : moe_gemm_kernel<ACT, false, SLAB>;
+template <int ACT, int OF> hipError_t launch_whole(const MoeGemmArgs& a, bool turn, hipStream_t s) {
+  auto* fn = turn ? moe_gemm_kernel<ACT, true, OF> : moe_gemm_kernel<ACT, false, OF>;
   const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize, NU * UNIT);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(fn, dim3(8 * std::max(a.cus / 8, 1)), dim3(64 * NW), NU * UNIT, s, a);
@@ -614,14 +619,14 @@ template <int ACT> hipError_t launch_act(MoeGemmArgs a, hipStream_t s) {
   // (at most one row tile per expert on average: the places cost 0.6 % where they are all the first, 8 of 4096 x 14336, 1024 rows each)
   constexpr int NO = ACT >= MOE_ACT_SILU && ACT <= MOE_ACT_GELU ? BN / 2 : BN;
   const bool turn = a.rows <= (int64_t)BM * a.experts && 2 * (int64_t)a.experts * (a.ncols / NO) >= a.cus;
-  return launch_whole<ACT, false>(a, turn, s);
+  return launch_whole<ACT, OF_EXPERTS>(a, turn, s);
 }
 
-template <int ACT, bool SLAB> hipError_t launch_dense(const MoeGemmArgs& a, hipStream_t s) {
+template <int ACT, int OF> hipError_t launch_dense(const MoeGemmArgs& a, hipStream_t s) {
   const bool one = a.rows <= BM;
-  if (a.tile_rows == ROWS_64) return launch_few<ACT, 1, SLAB>(a, s);
-  if (a.tile_rows == ROWS_128) return launch_few<ACT, 2, SLAB>(a, s);
-  return launch_whole<ACT, SLAB>(a, one, s);
+  if (a.tile_rows == ROWS_64) return launch_few<ACT, 1, OF>(a, s);
+  if (a.tile_rows == ROWS_128) return launch_few<ACT, 2, OF>(a, s);
+  return launch_whole<ACT, OF>(a, one, s);
 }
 
 }  // namespace
@@ -660,7 +665,7 @@ hipError_t launch_dense_gemm(MoeGemmArgs a, hipStream_t s) {
   if (slab ? a.act != MOE_ACT_NONE || a.K % (BK * a.experts) != 0 : a.experts != 1 || a.act != MOE_ACT_SILU) return hipErrorInvalidValue;
   if (a.tile_rows != 0 && a.tile_rows != ROWS_64 && a.tile_rows != ROWS_128 && (a.tile_rows < 128 || a.tile_rows > 256 || a.tile_rows % 32 != 0)) return hipErrorInvalidValue;
   a.cus = num_cus();
-  return slab ? launch_dense<MOE_ACT_NONE, true>(a, s) : launch_dense<MOE_ACT_SILU, false>(a, s);
+  return slab ? launch_dense<MOE_ACT_NONE, OF_PARTS>(a, s) : launch_dense<MOE_ACT_SILU, OF_ONE>(a, s);
 }
 
 }  // namespace die
