@@ -415,7 +415,7 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_kernel(MoeGemmArgs a) {
 //   32 of 4096 x 2048, 1024                        102 107 115 125 134 / 109 126 141 163 177   / 100 108 112 132 147
 //   8 gated of 4096 x 14336, 3584                  352 361 373 402 429 / 363 452 495 575 614   / 323 361 379 457 485
 // So steps of up to a tile of 64 per CU take these up to 192 rows per expert on average (27 of 32 us; from 257 rows they are two tiles), of up to two
-// those of 128 rows up to 144; larger ones up to 40. (Two workgroups per CU, each with half the LDS and tiles of 64 by up to 128 rows: 15 17 19 27 for
+// those of 128 rows up to 144; larger ones up to 60 - 80 (few_tiles). (Two workgroups per CU, each with half the LDS and tiles of 64 by up to 128 rows: 15 17 19 27 for
 // the third, 55 61 68 108 for the fifth.)
 constexpr int FN = 32 * TN, FUNIT = FN * ROWB;   // weight rows of a tile, bytes of 64 rows of a stage
 
@@ -583,13 +583,15 @@ __global__ void __launch_bounds__(64 * NW, 2) moe_gemm_few_kernel(MoeGemmArgs a)
   else run(IntC<4>{});
 }
 
-// `tile_rows` of the tiles of 64 and 128 weight rows; what a step takes
+// `tile_rows` of the tiles of 64 and 128 weight rows; what a step takes. Beyond two turns of tiles of 64 those of 128 are faster where experts have few rows, up to four turns a few
+// more (whole tiles / 128, layers of 8 experts, gated, on cold weights, us: width 4096 x 14336, 50 rows each 521 / 505, 75 551 / 559; 4096 x 4096, 50 174 / 167, 62 179 / 174, 75 185 / 182,
+// 112 193 / 193; 32 of 4096 x 2048, 87 254 / 256).
 enum { ROWS_WHOLE = 0, ROWS_64 = 64, ROWS_128 = 96 };
 inline int few_tiles(const MoeGemmArgs& a) {
   const int no = a.act >= MOE_ACT_SILU && a.act <= MOE_ACT_GELU ? FN / 2 : FN;
   const int64_t tiles = (int64_t)std::min(a.experts, a.rows) * (a.ncols / no);   // of experts of up to 256 rows
   if (tiles <= a.cus && a.rows <= 192 * (int64_t)a.experts) return ROWS_64;
-  return a.rows <= (tiles <= 2 * a.cus ? 144 : 40) * (int64_t)a.experts ? ROWS_128 : ROWS_WHOLE;
+  return a.rows <= (tiles <= 2 * a.cus ? 144 : tiles <= 4 * a.cus ? 80 : 60) * (int64_t)a.experts ? ROWS_128 : ROWS_WHOLE;
 }
 
 template <int ACT, int NB, int OF = OF_EXPERTS> hipError_t launch_few(const MoeGemmArgs& a, hipStream_t s) {

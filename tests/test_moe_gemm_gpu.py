@@ -251,3 +251,19 @@ def test_tiles_that_start_within_k(cuda, tile, K, ncols, act):
     want = _want(x, w, offsets, idx, 2, act, scale, 1.5, 1.7)
     tol = 2.0 ** -8 * (want.abs() + want.square().mean(1, keepdim=True).sqrt())
     assert ((out.cpu().double() - want).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("experts,rows,tile", [(16, 40, 96), (16, 80, 96), (16, 81, 256), (32, 60, 96), (32, 61, 256)])
+def test_tiles_of_few_rows(cuda, experts, rows, tile):
+    """What a step of up to four turns of tiles of 64 weight rows (on 256 compute units), and one of more, takes on either side of its line: the bits of those
+    tiles and not of the others, whose sums run in another order."""
+    counts = [rows - 7, rows + 7] * (experts // 2)
+    x, w, offsets, idx, scale = _case(counts, 512, 4096, False, 2)
+    dev = [t.to(cuda) for t in (x, w, offsets, idx)]
+    out = {}
+    for code in (0, 96, 256):
+        out[code] = torch.full((sum(counts), 4096), float("nan"), dtype=torch.bfloat16, device=cuda)
+        assert mix._kern().moe_gemm(out[code], *dev, 2, None, mix.MOE_NONE, 1.5, 1.7, code)
+    assert torch.equal(out[0], out[tile]) and not torch.equal(out[0], out[96 + 256 - tile])
+    rel = ((out[96].float() - out[256].float()).norm() / out[256].float().norm()).item()
+    assert rel < 2.0 ** -9   # (rounded to another bf16 now and then)
