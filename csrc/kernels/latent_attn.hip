@@ -1015,7 +1015,7 @@ __global__ void __launch_bounds__(256, 3) latent_attn_mfma_rq_kernel(LatentAttnA
 // cycles for 410 instructions). Sums take 128 registers at rank 256; of the queries' 72 the first NQL steps' lie in LDS, so that two waves fit on a SIMD and two workgroups
 // of 128 rows on a CU. The scale enters with the exponential's argument (a positive one). What bounds it: vector instructions, 49 % of the cycles (80 to 210 of a wave and
 // tile rescale and exponentiate), beside products, 32 %, and LDS reads that the two waves of a SIMD don't hide; 16 sequences of 1024 rows, 16 heads, rank 256 + 32:
-// 257 -> 213 us. (The next tile's fetch kept apart from the transposed reads, which the compiler has wait for it, or waves in products first: 1 - 3 % slower.)
+// 243 -> 193 us in the step (by the profiler, median of 12 passes, 272 -> 214). (The next tile's fetch kept apart from the transposed reads, which the compiler has wait for it, or waves in products first: 1 - 3 % slower.)
 template <int NDB, int NROT> struct TwoTile : RqTile<NDB, NROT> {
   static_assert(NDB == 8, "below rank 256 three waves of one group are faster");
   using Z = RqTile<NDB, NROT>;
@@ -1183,8 +1183,7 @@ __global__ void __launch_bounds__(256, 2) latent_attn_two_kernel(LatentAttnArgs 
   for (int u = 0; u < VB; ++u) vat[u] = 16 * vrow * KCH + 8 * (li & 1) + 16 * ((2 * u + (li >> 1 & 1)) ^ vsw);   // (rows r and r + 16 are exchanged alike)
   // The queries are here. (Without this the compiler waits for them in the loop, behind the next tile's DMA and so for that too.)
   __builtin_amdgcn_s_waitcnt(15 << 8 | 7 << 4);
-  // Tile i at `ks`, the next one's fetch to `to`. (Two places that share nothing: said so, since the compiler would have the transposed reads wait for the
-  // fetch, 5 % of the time.)
+  // Tile i at `ks`, the next one's fetch to `to`
   auto tile = [&](const bf16_t* src, char* to, const char* ks, int i) __attribute__((always_inline)) {
     const int j0 = jlo + i * MKT;
     // tile i is in LDS for every wave, and every wave has left the other buffer
@@ -1607,9 +1606,10 @@ inline bool wide_takes(const LatentAttnArgs& a) {
 }
 // Two groups of 16 rows per wave: where there is more than one turn of its workgroups (two per CU), and enough keys that starting them, which takes
 // longer, doesn't count; in one turn where all sequences have the same rows and see many keys (with others the longest ends alone). One group / two, rank
-// 256 + 32, us: 16 x 1024 rows of 16 heads 257 / 213; 8 of 786 - 1000 101 / 89; 32 of 125 - 250, 32 heads 73 / 65; 16 of 200 - 400, 32 heads 67 / 63; 6 x 300 behind
+// 256 + 32, us: 16 x 1024 rows of 16 heads 243 / 193 (the step; the others launched alone, back to back); 8 of 786 - 1000 101 / 89; 32 of 125 - 250, 32 heads 73 / 65; 16 of 200 - 400, 32 heads 67 / 63; 6 x 300 behind
 // 300, 32 heads, window 512 63 / 47; 8 x 500 behind 300 73 / 61; 4 x 1000 70 / 66. Not: 4 of 889 - 1000 70 / 74; 32 x 200 39 / 42; 32 of 50 - 100 behind 150 - 300
-// 33 / 37; 24 x 100 19 / 19. Without a rotary part, or with one of 64 (13 registers in scratch), the gain is 2 - 10 % smaller: twice the work.
+// 33 / 37; 24 x 100 19 / 19. (58 random steps that it takes: 0.88 of the time, one slower by more than 1 %, 18 of up to 243 rows of 12 heads in tables ten times as wide 27 / 29, as
+// the tables' width stands for the keys.) Without a rotary part, or with one of 64 (13 registers in scratch), the gain is 2 - 10 % smaller: twice the work.
 inline bool two_takes(const LatentAttnArgs& a) {
   const int64_t cus = num_cus(), wgs = (int64_t)a.total_q * a.heads / 128, keys = (int64_t)a.bt_cols * a.block_size - a.max_q / 2;
   const int64_t seen = a.window > 0 ? std::min<int64_t>(keys, a.window) : keys;   // by a row, about

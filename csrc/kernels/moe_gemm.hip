@@ -17,11 +17,11 @@
 // What holds it up at many rows is power: under the products the clock falls to 1.6 - 1.8 GHz. So the tiles are 16x16x32 products: at the power limit
 // a wave of 64 x 128 results runs 1.85 - 1.88 PFLOP/s with them from LDS on normal values and 1.60 - 1.64 with 32x32x16 (without the limit, on zeros, both are the
 // same), the rows of x gone through there and back so that each product shares an operand with the one before it (1.88 against 1.83 - 1.85). The fetches
-// into LDS take most of the rest: without them this kernel reaches 1.70 PFLOP/s instead of 1.33, with all of them from L2 1.45. (Waves of 128 x 128 results, one
+// into LDS take most of the rest: a copy of this kernel without them ran 1.28 times as fast, one with all of them from L2 1.09 times. (Waves of 128 x 128 results, one
 // per SIMD, read a third less LDS; as a kernel they ran 7 - 20 % slower, as nothing runs beside its epilogues.) At few rows it is the weights' rate from HBM.
-// Each product alone, 32x32x16 -> 16x16x32, us: 4096 tokens, two of 8 experts of 4096 x 14336: 1894 -> 1597 and 976 -> 860; 1000 of them 681 -> 612 and
-// 322 -> 303; 8191 tokens, four of 16 experts of 2048 x 1024: 144 -> 125 and 151 -> 132; 3000 tokens, four of 32 experts of 4096 x 2048: 208 -> 184 and 227 ->
-// 212; 1500 tokens, two of 8 gated experts of 2048 x 2048: 60 -> 54 and 35 -> 33.
+// Each product alone, back to back over three sets of rows and weights, 32x32x16 -> 16x16x32, us: 8 gated experts of 4096 x 14336, two of them, 3000 tokens 1371 -> 1192 (1.18 PFLOP/s)
+// and 665 -> 590, 1075 tokens 644 -> 588 and 300 -> 279; four of 16 of 2048 x 1024, 8000 tokens 151 -> 137 and 149 -> 139; four of 32 of 4096 x 2048, 3000 tokens 223 -> 205 and 217 -> 208; two of 8
+// gated ones of 2048 x 2048, 1500 tokens 66 -> 65 and 41 -> 41. (By the profiler, whose passes run at lower and lower clocks, the median of 12 at 4096 tokens 1925 -> 1685 and 995 -> 898.)
 #include <math.h>
 
 #include <algorithm>
