@@ -789,6 +789,7 @@ __global__ void __launch_bounds__(128) attn_decode_reduce_kernel(bf16_t* __restr
 // 49 / 49); 16 of them with many stages 1 x 4096 136 / 115, 2 x 2000 72 / 65, few 2 x 1000 40 / 38 but behind 128 45 / 46; others not: 12 lists 3 x 1300 49 / 68, 32
 // 1 x 2048 76 / 93, 64 4 x 1000 44 / 61, 4 1 x 4096 138 / 147. (Four groups of 2 waves 1 x 1000 34, two of them 31.)
 int attn_prefill_groups(int max_q_len, int num_seqs, int hq, int hkv, int64_t keys, int cus) {
+  if (hkv < 1 || hq < hkv) return 1;
   const int G = hq / hkv, rows = 4 * (32 / (G > 32 ? 32 : G));
   const int64_t lists = (int64_t)num_seqs * hkv, tiles = (max_q_len + rows - 1) / rows * lists;
   if (tiles <= cus) return max_q_len >= 200 && keys >= (G >= 4 ? 200 : G == 2 ? 256 : 288) ? 2 : 1;

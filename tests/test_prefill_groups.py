@@ -18,3 +18,7 @@ _C = pytest.importorskip("src._C")
     (16, 1, 1, 3000, 3000, 1), (32, 1, 1, 2048, 2048, 1), (32, 2, 2, 1000, 1000, 1), (64, 2, 1, 1000, 1000, 1), (32, 8, 64, 512, 512, 1)])
 def test_groups(hq, hkv, seqs, rows, keys, groups):
     assert _C.attn_prefill_groups(rows, seqs, hq, hkv, keys, 256) == groups
+
+
+def test_heads_that_make_no_groups():
+    assert [_C.attn_prefill_groups(300, 1, hq, hkv, 300, 256) for hq, hkv in ((8, 0), (1, 2), (0, 0))] == [1, 1, 1]

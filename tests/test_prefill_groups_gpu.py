@@ -14,9 +14,25 @@ from src.ops import reference as ref
 pytestmark = pytest.mark.gpu
 
 
-# new tokens and lengths: one stage for the first group alone, odd and even numbers of stages, a row of one key beside long ones, keys before the step
-@pytest.mark.parametrize("qlens,ctxs", [([200], [200]), ([257], [257]), ([1, 320, 33], [1, 320, 33]), ([288, 5], [1000, 37]), ([1000], [1000]), ([1025], [1537])])
-@pytest.mark.parametrize("hkv,g", [(8, 4), (4, 1), (1, 8), (1, 32)])
+# new tokens and lengths: one stage for the first group alone, odd and even numbers of stages, a row of one key beside long ones, keys before the step, more than one turn of
+# row tiles with 8 key heads
+CASES = [([200], [200]), ([257], [257]), ([1, 320, 33], [1, 320, 33]), ([288, 5], [1000, 37]), ([1000], [1000]), ([1025], [1537]), ([1040], [1040]), ([1500], [1500])]
+HEADS = [(8, 4), (4, 1), (1, 8), (1, 32)]
+
+
+def _groups(qlens, ctxs, hkv, g):
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    return ops._kern().attn_prefill_groups(max(qlens), len(qlens), hkv * g, hkv, (max(ctxs) + 15) // 16 * 16, cus)
+
+
+def test_cases_take_two_groups():
+    """All with several heads per key head but the one behind many keys beyond a turn; from 288 keys on with one."""
+    taken = {h: [c for c in CASES if _groups(*c, *h) == 2] for h in HEADS}
+    assert taken[8, 4] == CASES[:5] + CASES[6:] and taken[4, 1] == CASES[2:] and taken[1, 8] == CASES and taken[1, 32] == CASES[:5]
+
+
+@pytest.mark.parametrize("qlens,ctxs", CASES)
+@pytest.mark.parametrize("hkv,g", HEADS)
 def test_groups(qlens, ctxs, hkv, g):
     hq, t, blocks = hkv * g, sum(qlens), [(c + 15) // 16 for c in ctxs]
     rng = torch.Generator(device="cuda").manual_seed(0)
